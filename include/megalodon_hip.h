@@ -688,6 +688,54 @@ int mega_split_bf16(const void* src, int dtype, int64_t n, void* hi, void* lo, v
 int mega_bench_stream_copy(const void* a, const void* b, void* out, int64_t bytes,
                            int workgroups, int nontemporal, void* stream);
 
+/* ------------------------------------------------------------------------
+ * One new token per sequence through a whole block, continuing a cache: the
+ * cache branch of moving_average_gated_attention.py:283-348 at sequence length
+ * one followed by normalized_feedforward_network.py:74-90 (SwiGLU, no dropout).
+ * All activations, weights and cached tensors in `dtype` (MEGA_BF16 / MEGA_F16)
+ * unless a type is given; stored norm weights are gamma - 1.  `x`, `y` (B, D).
+ * `k_cache` (B, >= length + 1, heads, S / heads) and `v_cache` (B, >= length + 1,
+ * heads, E / heads) with `k_stride` / `v_stride` elements between sequences hold
+ * `length` keys and values; the new ones are written behind them.  The query
+ * sees all length + 1 keys.  p (D, N) float32, q and gamma_hat (D, N) complex64 are
+ * the coefficients of complex_exponential_moving_average.py:100-117, h (B, D, N)
+ * complex64 the carried state.  `freqs`: S / heads / 2 complex64 factors of the
+ * token's position inside its chunk, or NULL.  rms_weight, ln_weight, ln_bias and the
+ * projections' biases may be NULL.  No synchronisation, no allocation.
+ * ---------------------------------------------------------------------- */
+typedef struct mega_block_decode_args {
+  int dtype;
+  int64_t B, D, S, E, F, heads, G, N; /* sequences, model, q/k, value, FFN widths, heads, norm groups, modes */
+  int64_t length, k_stride, v_stride;
+  float tsn_eps, rms_eps, z_eps, ln_eps;
+  const void* x;
+  const int64_t* prev_count;          /* (B) */
+  const void *prev_mean, *prev_var;   /* (B, G) */
+  const void *tsn_weight, *tsn_bias;  /* (D) */
+  const float *p, *q, *gamma_hat;
+  const void* omega;                  /* (D) */
+  const float* h_in;
+  const void* rms_weight;
+  const void *wz, *bz, *wr, *br, *wh1, *bh1, *wv, *bv, *wh2;
+  const void *qk_gamma, *qk_beta;     /* (2, S) */
+  const float* freqs;
+  const void *ln_weight, *ln_bias, *fc1, *fc2, *fc3;
+  void *k_cache, *v_cache;
+  void* y;
+  int64_t* count;
+  void *mean, *var;
+  float* h_out;
+  void* workspace;                    /* mega_block_decode_workspace_bytes, 256-byte aligned */
+} mega_block_decode_args;
+
+/* 1 if the step kernels take these sizes: B <= 32, N = 16, widths multiples of 32,
+ * groups of a multiple of 32 features, q/k head width 64, 128 or 256, value head width a
+ * power of two from 64 to 2048. */
+int mega_block_decode_supported(int dtype, int64_t B, int64_t D, int64_t S, int64_t E, int64_t F,
+                                int64_t heads, int64_t G, int64_t N);
+int64_t mega_block_decode_workspace_bytes(const mega_block_decode_args* args);
+int mega_block_decode(const mega_block_decode_args* args, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

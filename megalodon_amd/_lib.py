@@ -44,6 +44,23 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The C++ host extension (csrc/host); raises loudly when it has not been built."""
+    global _host
+    if _host is None:
+        load()
+        import torch  # noqa: F401  (its libraries have to be in the process first)
+        try:
+            from . import _host as ext
+        except ImportError as e:
+            raise RuntimeError(f"megalodon_amd._host is not built ({e}): build it with `python -m megalodon_amd._build`")
+        _host = ext
+    return _host
+
+
 def check(code: int, what: str) -> None:
     if code != 0:
         msg = load().mega_last_error().decode("utf-8", "replace")

@@ -19,6 +19,7 @@ from torch.nn import Parameter
 
 from .. import extension as megalodon_ops
 from ..fused_ops import memory_efficient_dropout, qk_norm_rotary, silu_mul, transpose_last2
+from .block_decode import decode_step
 from .chunk_attention import _InnerAttention
 from .complex_exponential_moving_average import MultiHeadComplexEMA
 from .linear import Linear, linear_group
@@ -149,6 +150,11 @@ class MegaBlock(nn.Module):
             norm_eps=norm_eps, rescale=rescale, init_std=init_std)
 
     def forward(self, x: Tensor, freqs_cis: Optional[Tensor] = None, mask: Optional[Tensor] = None, cache=None):
+        if (cache is not None and x.dim() == 3 and x.shape[1] == 1 and mask is None and not self.training
+                and not torch.is_grad_enabled()):
+            step = decode_step(self, x, freqs_cis, cache)
+            if step is not None:
+                return step
         y, cache = self.mega(x, freqs_cis, mask, cache)
         out = self.nffn(y, x)
         return out, cache

@@ -1,0 +1,101 @@
+"""The fused one-token step of a block (csrc/block_decode.hip) against the same step taken operator by
+operator, at the edges of what the kernels take: token tiles (1, 16, 17, 32 sequences), head
+widths, lengths of one key, one run and many runs of keys.  Tolerance: the 16-bit bar, 2e-2."""
+import pytest
+import torch
+
+from conftest import rel_err
+from megalodon_amd import _lib
+from megalodon_amd.modules import MegaBlock, RotaryEmbedding
+from megalodon_amd.modules.block_decode import decode_step
+
+pytestmark = pytest.mark.gpu
+
+
+def _block(D, S, E, F, heads, groups, chunk, dtype=torch.bfloat16, affine=True):
+    torch.manual_seed(3)
+    blk = MegaBlock(model_dim=D, z_dim=S, value_dim=E, num_heads=heads, cema_ndim=16, chunk_size=chunk,
+                    ffn_hidden_dim=F, norm_num_groups=groups, init_std=0.05, norm_affine=affine).cuda().to(dtype).eval()
+    with torch.no_grad():
+        for name, p in blk.named_parameters():
+            if p.abs().max() == 0:
+                p.normal_(0, 0.1)
+    return blk
+
+
+def _prompt(blk, B, n, D, S, E, heads, dtype, rotary):
+    empty = ((torch.empty(B, 0, heads, S // heads, dtype=dtype, device="cuda"),
+              torch.empty(B, 0, heads, E // heads, dtype=dtype, device="cuda"), 0), (None, None, None), None)
+    x = torch.randn(B, n, D, generator=torch.Generator().manual_seed(n)).to(dtype).cuda()
+    return blk(x, rotary.get_freqs_cis(0, n), None, empty)[1]
+
+
+@pytest.mark.parametrize("B,n,D,S,E,F,heads,groups,dtype,affine", [
+    (1, 1, 256, 128, 512, 512, 2, 2, torch.bfloat16, True),       # one cached key, 64-wide heads
+    (16, 40, 1024, 256, 2048, 2752, 1, 8, torch.bfloat16, True),  # a full token tile, 2048-wide values
+    (17, 513, 256, 512, 128, 96, 2, 8, torch.bfloat16, True),     # two token tiles, narrow values, many runs
+    (32, 7, 512, 256, 1024, 320, 2, 2, torch.float16, True),
+    (3, 1000, 384, 384, 768, 416, 3, 3, torch.bfloat16, False),   # no affine norms, reductions that do not divide by eight waves
+])
+def test_step_matches_operators(B, n, D, S, E, F, heads, groups, dtype, affine):
+    chunk = 1024
+    blk = _block(D, S, E, F, heads, groups, chunk, dtype, affine)
+    rotary = RotaryEmbedding(S // heads, chunk).cuda()
+    with torch.no_grad():
+        cache = _prompt(blk, B, n, D, S, E, heads, dtype, rotary)
+        for t in range(3):
+            x = torch.randn(B, 1, D, generator=torch.Generator().manual_seed(t)).to(dtype).cuda()
+            freqs = rotary.get_freqs_cis(n + t, n + t + 1) if t != 1 else None
+            before = [c.clone() for c in (*cache[0][:2], *cache[1], cache[2])]
+            y, wanted = blk.mega(x, freqs, None, cache)
+            y = blk.nffn(y, x)
+            got = decode_step(blk, x, freqs, cache)
+            assert got is not None
+            for a, b in zip(before, (*cache[0][:2], *cache[1], cache[2])):
+                assert torch.equal(a, b)  # the cache that was handed in is what it was
+            assert rel_err(got[0], y) <= 2e-2
+            assert got[1][0][2] == wanted[0][2] == n + t + 1
+            assert torch.equal(got[1][1][0], wanted[1][0])
+            for a, b in ((got[1][0][0], wanted[0][0]), (got[1][0][1], wanted[0][1]), (got[1][1][1], wanted[1][1]),
+                         (got[1][1][2], wanted[1][2])):
+                assert a.shape == b.shape and a.dtype == b.dtype and rel_err(a, b) <= 2e-2
+            assert got[1][2].dtype == wanted[2].dtype and rel_err(got[1][2], wanted[2]) <= 2e-2
+            cache = got[1]
+
+
+def test_last_token_of_a_chunk_empties_the_cache():
+    blk = _block(256, 128, 512, 512, 2, 2, 64)
+    rotary = RotaryEmbedding(64, 64).cuda()
+    with torch.no_grad():
+        cache = _prompt(blk, 2, 63, 256, 128, 512, 2, torch.bfloat16, rotary)
+        x = torch.randn(2, 1, 256, generator=torch.Generator().manual_seed(1)).bfloat16().cuda()
+        y, cache = decode_step(blk, x, rotary.get_freqs_cis(63, 64), cache)
+        assert cache[0][0].shape[1] == 0 and cache[0][1].shape[1] == 0 and cache[0][2] == 0
+        assert decode_step(blk, x, rotary.get_freqs_cis(0, 1), cache) is None  # the next chunk's first token: operators
+
+
+def test_cache_storage_is_shared_only_while_nobody_else_holds_it():
+    """Tokens are appended in place; two continuations of one cache do not touch each other."""
+    blk = _block(256, 128, 512, 512, 2, 2, 512)
+    rotary = RotaryEmbedding(64, 512).cuda()
+    with torch.no_grad():
+        cache = _prompt(blk, 2, 30, 256, 128, 512, 2, torch.bfloat16, rotary)
+        xs = [torch.randn(2, 1, 256, generator=torch.Generator().manual_seed(s)).bfloat16().cuda() for s in range(2)]
+        freqs = rotary.get_freqs_cis(30, 31)
+        where = cache[0][0].data_ptr()
+        _, first = decode_step(blk, xs[0], freqs, cache)
+        assert first[0][0].data_ptr() == where           # room behind the prompt
+        kept = first[0][0].clone(), first[0][1].clone()
+        _, second = decode_step(blk, xs[1], freqs, cache)
+        assert second[0][0].data_ptr() != where          # the first continuation is alive
+        assert torch.equal(first[0][0], kept[0]) and torch.equal(first[0][1], kept[1])
+        slice_of_first = first[0][1][:, -1:]
+        del first
+        _, third = decode_step(blk, xs[1], freqs, cache)
+        assert third[0][0].data_ptr() != where           # a view of it still is
+        assert torch.equal(slice_of_first, kept[1][:, -1:])
+        del slice_of_first
+        _, fourth = decode_step(blk, xs[1], freqs, cache)
+        assert fourth[0][0].data_ptr() == where
+        assert torch.equal(fourth[0][1], third[0][1])
+    assert _lib.host() is not None
