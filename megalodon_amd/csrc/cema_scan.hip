@@ -105,14 +105,50 @@ __device__ __forceinline__ float opaque_one() {
   return one;
 }
 
+// Rows that do not start on 16-byte boundaries (a length that is no multiple of 8, or an odd storage
+// offset): the same 16-byte accesses, which this part takes at any element's address, except
+// for the piece that straddles the end of the row, which goes element by element.
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+__device__ __forceinline__ u32x4 load_tail16(const uint16_t* src, int n) {
+  uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    if (e < n) w[e >> 1] |= static_cast<uint32_t>(src[e]) << (16 * (e & 1));
+  return u32x4{w[0], w[1], w[2], w[3]};
+}
+// steps elem .. elem + 7 of a row of L 16-bit steps, zero behind its end
+template <bool ANY>
+__device__ __forceinline__ u32x4 load8_16(const uint16_t* row, int64_t elem, bool on, int64_t L) {
+  const uint16_t* src = row + elem;
+  if (!ANY) return on && elem + 8 <= L ? *reinterpret_cast<const u32x4*>(src) : u32x4{0u, 0u, 0u, 0u};
+  u32x4 v = {0u, 0u, 0u, 0u};
+  if (on && elem + 8 <= L) v = *reinterpret_cast<const u32x4_any*>(src);
+  else if (on && elem < L) v = load_tail16(src, static_cast<int>(L - elem));
+  return v;
+}
+template <bool ANY>
+__device__ __forceinline__ void store8_16(uint16_t* row, int64_t elem, int64_t L, uint4 v) {
+  uint16_t* dst = row + elem;
+  if (elem + 8 <= L) {
+    if (ANY) *reinterpret_cast<u32x4_any*>(dst) = u32x4{v.x, v.y, v.z, v.w};
+    else *reinterpret_cast<uint4*>(dst) = v;
+  } else if (ANY && elem < L) {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (elem + e < L) dst[e] = static_cast<uint16_t>(w[e >> 1] >> (16 * (e & 1)));
+  }
+}
+
 // Eight consecutive steps of a row as a matrix operand: XP bf16 pieces whose sum
 // is the data exactly (bf16: the data itself; fp16: two pieces).
 template <int DT> struct XOp;
 template <> struct XOp<MEGA_BF16> {
   static constexpr int XP = 1;
   u32x4 pc[1];
-  __device__ __forceinline__ void load(const void* row, int64_t elem, bool on) {
-    pc[0] = on ? *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(row) + elem) : u32x4{0u, 0u, 0u, 0u};
+  template <bool ANY>
+  __device__ __forceinline__ void load(const void* row, int64_t elem, bool on, int64_t L) {
+    pc[0] = load8_16<ANY>(static_cast<const uint16_t*>(row), elem, on, L);
   }
   __device__ __forceinline__ void values(float* v) const {
     unpack8<MEGA_BF16>(make_uint4(pc[0][0], pc[0][1], pc[0][2], pc[0][3]), v);
@@ -121,11 +157,11 @@ template <> struct XOp<MEGA_BF16> {
 template <> struct XOp<MEGA_F16> {
   static constexpr int XP = 2;
   u32x4 pc[2];
-  __device__ __forceinline__ void load(const void* row, int64_t elem, bool on) {
+  template <bool ANY>
+  __device__ __forceinline__ void load(const void* row, int64_t elem, bool on, int64_t L) {
     float v[8];
-    uint4 raw = make_uint4(0u, 0u, 0u, 0u);
-    if (on) raw = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(row) + elem);
-    unpack8<MEGA_F16>(raw, v);
+    const u32x4 raw = load8_16<ANY>(static_cast<const uint16_t*>(row), elem, on, L);
+    unpack8<MEGA_F16>(make_uint4(raw[0], raw[1], raw[2], raw[3]), v);
     split8(v, pc[0], pc[1]);
   }
   __device__ __forceinline__ void values(float* v) const {
@@ -142,9 +178,11 @@ template <> struct XOp<MEGA_F16> {
 template <> struct XOp<MEGA_F32> {
   static constexpr int XP = 2;
   u32x4 pc[2];
-  __device__ __forceinline__ void load(const void* row, int64_t elem, bool on) {
+  template <bool ANY>
+  __device__ __forceinline__ void load(const void* row, int64_t elem, bool on, int64_t L) {
+    static_assert(!ANY, "float32 rows are aligned");
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
-    if (on) {
+    if (on && elem + 8 <= L) {
       const float4* src = reinterpret_cast<const float4*>(static_cast<const float*>(row) + elem);
       a = src[0];
       b = src[1];
@@ -191,7 +229,7 @@ static_assert(sizeof(cf) * 16 * (kT + 2) <= sizeof(float) * (kWaves * 32 + 1) * 
 // and waits for its own LDS operations can read what its other lanes wrote.
 __device__ __forceinline__ void wave_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-template <int DT, int NT>
+template <int DT, int NT, bool ANY>
 __global__ __launch_bounds__(kThreads, NT == 1 ? 3 : 2) void cema_scan_fwd_kernel(
     const void* __restrict__ x, void* __restrict__ y, const float* __restrict__ p,
     const cf* __restrict__ log_q, const cf* __restrict__ gamma, const float* __restrict__ omega,
@@ -219,7 +257,7 @@ __global__ __launch_bounds__(kThreads, NT == 1 ? 3 : 2) void cema_scan_fwd_kerne
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const int64_t elem = chunk * kT + 16 * s + 8 * g;
-        t[ctl][s].load(xrow, elem, row < rows && elem + 8 <= L);
+        t[ctl][s].template load<ANY>(xrow, elem, row < rows, L);
       }
     }
   };
@@ -481,8 +519,7 @@ __global__ __launch_bounds__(kThreads, NT == 1 ? 3 : 2) void cema_scan_fwd_kerne
                 }
               } else {
                 const uint4 oct = octet_of<DT>(acc, pr);
-                const int64_t elem = chunk * kT + 16 * (2 * it + pr) + 8 * g;
-                if (elem + 8 <= L) *reinterpret_cast<uint4*>(yrow + elem) = oct;
+                store8_16<ANY>(yrow, chunk * kT + 16 * (2 * it + pr) + 8 * g, L, oct);
               }
             }
           }
@@ -527,19 +564,19 @@ __global__ __launch_bounds__(kThreads, NT == 1 ? 3 : 2) void cema_scan_fwd_kerne
     for (int64_t seg0 = 0; seg0 < C; seg0 += NC) item(row, seg0);
 }
 
-template <int DT, int NT>
+template <int DT, int NT, bool ANY>
 int launch_fwd(const void* x, void* y, const float* p, const cf* log_q, const cf* gamma,
                const float* omega, const cf* h0, cf* h_last, int64_t B, int64_t D, int64_t N,
                int64_t L, hipStream_t stream) {
   const size_t lds = sizeof(FwdSmem<NT>);
-  MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cema_scan_fwd_kernel<DT, NT>),
+  MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cema_scan_fwd_kernel<DT, NT, ANY>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
   int dev = 0, cus = 0;
   MEGA_CHECK_HIP(hipGetDevice(&dev));
   MEGA_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   const int64_t rows = B * D, slots = (NT == 1 ? 3 : 2) * static_cast<int64_t>(cus);  // workgroups that fit a compute unit
   const unsigned grid = static_cast<unsigned>(rows < slots ? rows : slots);
-  cema_scan_fwd_kernel<DT, NT><<<dim3(grid), kThreads, lds, stream>>>(
+  cema_scan_fwd_kernel<DT, NT, ANY><<<dim3(grid), kThreads, lds, stream>>>(
       x, y, p, log_q, gamma, omega, h0, h_last, rows, static_cast<int>(D), static_cast<int>(N), L);
   MEGA_CHECK_LAUNCH();
   return MEGA_OK;
@@ -614,7 +651,7 @@ __device__ __forceinline__ void rstep(cf& h, cf& hd, cf g, cf gd, cf m, cf md) {
 // DX32: dx is written in float32 (or, with a null pointer, not at all) instead of the rows'
 // own type -- for callers that add up the backward of several bfloat16 pieces of one tensor;
 // DX32 == 2 adds to what dx holds instead of overwriting it.
-template <int DT, int DX32>
+template <int DT, int DX32, bool ANY>
 __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
     const void* __restrict__ dy, const void* __restrict__ x, void* __restrict__ dx,
     const float* __restrict__ p, const cf* __restrict__ log_q, const cf* __restrict__ gamma,
@@ -647,7 +684,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const int64_t elem = chunk * kT + 16 * s + 8 * g;
-      dn[s].load(dyrow, elem, row < rows && elem + 8 <= L);
+      dn[s].template load<ANY>(dyrow, elem, row < rows, L);
     }
   };
   auto load_x = [&](int64_t row, int64_t seg0) {
@@ -657,7 +694,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const int64_t elem = chunk * kT + 16 * s + 8 * g;
-      xb[s].load(xrow, elem, row < rows && elem + 8 <= L);
+      xb[s].template load<ANY>(xrow, elem, row < rows, L);
     }
   };
   struct RowParams {
@@ -1115,7 +1152,8 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
               const int64_t elem = chunk * kT + 16 * (2 * jt + pr) + 8 * h + 4 * g;
-              if (dx != nullptr && elem + 4 <= L) {
+              // (rows of any length: element by element -- the float32 sum of pieces is not the hot path)
+              if (!ANY && dx != nullptr && elem + 4 <= L) {
                 float4 v = make_float4(acc[8 * pr + 4 * h], acc[8 * pr + 4 * h + 1], acc[8 * pr + 4 * h + 2],
                                        acc[8 * pr + 4 * h + 3]);
                 if constexpr (DX32 == 2) {
@@ -1123,12 +1161,15 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
                   v = make_float4(v.x + o.x, v.y + o.y, v.z + o.z, v.w + o.w);
                 }
                 *reinterpret_cast<float4*>(dxrow + elem) = v;
+              } else if (ANY && dx != nullptr) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                  if (elem + e < L) dxrow[elem + e] = acc[8 * pr + 4 * h + e] + (DX32 == 2 ? static_cast<float>(dxrow[elem + e]) : 0.f);
               }
             }
           } else {
             const uint4 oct = octet_of<DT>(acc, pr);
-            const int64_t elem = chunk * kT + 16 * (2 * jt + pr) + 8 * g;
-            if (elem + 8 <= L) *reinterpret_cast<uint4*>(dxrow + elem) = oct;
+            store8_16<ANY>(dxrow, chunk * kT + 16 * (2 * jt + pr) + 8 * g, L, oct);
           }
         }
       }
@@ -1182,19 +1223,19 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
 #undef MEGA_LANE_IDS
 }
 
-template <int DX32>
+template <int DX32, bool ANY>
 int launch_bwd(const void* dy, const void* x, void* dx, const float* p, const cf* log_q,
                const cf* gamma, const float* omega, const cf* h0, float* dp, cf* dq, cf* dgamma, float* domega,
                cf* dh0, int64_t B, int64_t D, int64_t N, int64_t L, hipStream_t stream) {
   const int lds = static_cast<int>(sizeof(BwdSmem));
-  MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cema_scan_bwd_kernel<MEGA_BF16, DX32>),
+  MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cema_scan_bwd_kernel<MEGA_BF16, DX32, ANY>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds));
   int dev = 0, cus = 0;
   MEGA_CHECK_HIP(hipGetDevice(&dev));
   MEGA_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   const int64_t rows = B * D, slots = 2 * static_cast<int64_t>(cus);  // two workgroups fit a compute unit
   const unsigned grid = static_cast<unsigned>(rows < slots ? rows : slots);
-  cema_scan_bwd_kernel<MEGA_BF16, DX32><<<dim3(grid), kThreads, lds, stream>>>(
+  cema_scan_bwd_kernel<MEGA_BF16, DX32, ANY><<<dim3(grid), kThreads, lds, stream>>>(
       dy, x, dx, p, log_q, gamma, omega, h0, dp, dq, dgamma, domega, dh0, rows, static_cast<int>(D),
       static_cast<int>(N), L);
   MEGA_CHECK_LAUNCH();
@@ -1207,7 +1248,8 @@ int launch_bwd(const void* dy, const void* x, void* dx, const float* p, const cf
 using namespace mega;
 
 extern "C" int mega_cema_scan_supported(int dtype, int64_t N, int64_t L) {
-  return valid_dtype(dtype) && N >= 1 && N <= 16 && L >= 8 && L % 8 == 0;
+  // float32 rows of other lengths stay with the convolution, whose float32 transforms are the finer of the two
+  return valid_dtype(dtype) && N >= 1 && N <= 16 && L >= 1 && (dtype != MEGA_F32 || L % 8 == 0);
 }
 
 extern "C" int mega_cema_scan_fwd(const void* x, int dtype, const float* p, const float* log_q,
@@ -1220,10 +1262,10 @@ extern "C" int mega_cema_scan_fwd(const void* x, int dtype, const float* p, cons
   MEGA_CHECK_ARG(B * D <= 0x7fffffff, "%s: too many rows", who);
   if (!mega_cema_scan_supported(dtype, N, L))
     return set_error(MEGA_ERR_UNSUPPORTED,
-                     "%s: needs N <= 16 and L a multiple of 8 (dtype %d, N %lld, L %lld)",
+                     "%s: needs N <= 16 and, for float32 rows, L a multiple of 8 (dtype %d, N %lld, L %lld)",
                      who, dtype, (long long)N, (long long)L);
-  MEGA_CHECK_ARG(reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0,
-                 "%s: x and y must be 16-byte aligned", who);
+  const bool any = L % 8 != 0 || reinterpret_cast<uintptr_t>(x) % 16 != 0 || reinterpret_cast<uintptr_t>(y) % 16 != 0;
+  MEGA_CHECK_ARG(!any || dtype != MEGA_F32, "%s: float32 rows must be 16-byte aligned", who);
   if (B == 0 || D == 0) return MEGA_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const cf* lq = reinterpret_cast<const cf*>(log_q);
@@ -1231,13 +1273,16 @@ extern "C" int mega_cema_scan_fwd(const void* x, int dtype, const float* p, cons
   const cf* h0c = reinterpret_cast<const cf*>(h0);
   cf* hl = reinterpret_cast<cf*>(h_last);
   // one chunk tile per wave (segments of 128 chunks) measured 5 % faster than two for bfloat16 rows as well
-  if (dtype == MEGA_BF16) return launch_fwd<MEGA_BF16, 1>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s);
-  if (dtype == MEGA_F32) return launch_fwd<MEGA_F32, 1>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s);
-  return launch_fwd<MEGA_F16, 1>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s);
+  if (dtype == MEGA_F32) return launch_fwd<MEGA_F32, 1, false>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s);
+  if (dtype == MEGA_BF16)
+    return any ? launch_fwd<MEGA_BF16, 1, true>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s)
+               : launch_fwd<MEGA_BF16, 1, false>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s);
+  return any ? launch_fwd<MEGA_F16, 1, true>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s)
+             : launch_fwd<MEGA_F16, 1, false>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s);
 }
 
 extern "C" int mega_cema_scan_bwd_supported(int dtype, int64_t N, int64_t L) {
-  return dtype == MEGA_BF16 && N >= 1 && N <= 16 && L >= 8 && L % 8 == 0;
+  return dtype == MEGA_BF16 && N >= 1 && N <= 16 && L >= 1;
 }
 
 extern "C" int mega_cema_scan_bwd_state(const void* dy, const void* x, int dtype, const float* p,
@@ -1251,13 +1296,13 @@ extern "C" int mega_cema_scan_bwd_state(const void* dy, const void* x, int dtype
   MEGA_CHECK_ARG(B * D <= 0x7fffffff, "%s: too many rows", who);
   if (!mega_cema_scan_bwd_supported(dtype, N, L))
     return set_error(MEGA_ERR_UNSUPPORTED,
-                     "%s: needs bfloat16 rows, N <= 16 and L a multiple of 8 (dtype %d, N %lld, L %lld)", who,
+                     "%s: needs bfloat16 rows and N <= 16 (dtype %d, N %lld, L %lld)", who,
                      dtype, (long long)N, (long long)L);
   const auto al = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
-  MEGA_CHECK_ARG(al(dy) && al(x) && al(dx), "%s: dy, x and dx must be 16-byte aligned", who);
+  const bool any = L % 8 != 0 || !al(dy) || !al(x) || !al(dx);
   if (B == 0 || D == 0) return MEGA_OK;
   MEGA_CHECK_ARG(dh0 == nullptr || h0 != nullptr, "%s: dh0 without h0", who);
-  return launch_bwd<0>(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma),
+  return (any ? launch_bwd<0, true> : launch_bwd<0, false>)(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma),
                            omega, reinterpret_cast<const cf*>(h0), dp, reinterpret_cast<cf*>(dq),
                            reinterpret_cast<cf*>(dgamma), domega, reinterpret_cast<cf*>(dh0), B, D, N, L,
                            static_cast<hipStream_t>(stream));
@@ -1280,18 +1325,18 @@ extern "C" int mega_cema_scan_bwd_wide(const void* dy, const void* x, const floa
   MEGA_CHECK_ARG(B >= 0 && D >= 0 && L >= 0, "%s: negative size", who);
   MEGA_CHECK_ARG(B * D <= 0x7fffffff, "%s: too many rows", who);
   if (!mega_cema_scan_bwd_supported(MEGA_BF16, N, L))
-    return set_error(MEGA_ERR_UNSUPPORTED, "%s: needs N <= 16 and L a multiple of 8 (N %lld, L %lld)", who,
+    return set_error(MEGA_ERR_UNSUPPORTED, "%s: needs N <= 16 (N %lld, L %lld)", who,
                      (long long)N, (long long)L);
   const auto al = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
-  MEGA_CHECK_ARG(al(dy) && al(x) && al(dx), "%s: dy, x and dx must be 16-byte aligned", who);
+  const bool any = L % 8 != 0 || !al(dy) || !al(x) || !al(dx);
   if (B == 0 || D == 0) return MEGA_OK;
   MEGA_CHECK_ARG(dh0 == nullptr || h0 != nullptr, "%s: dh0 without h0", who);
   if (accumulate_dx && dx != nullptr)
-    return launch_bwd<2>(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma),
+    return (any ? launch_bwd<2, true> : launch_bwd<2, false>)(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma),
                          omega, reinterpret_cast<const cf*>(h0), dp, reinterpret_cast<cf*>(dq),
                          reinterpret_cast<cf*>(dgamma), domega, reinterpret_cast<cf*>(dh0), B, D, N, L,
                          static_cast<hipStream_t>(stream));
-  return launch_bwd<1>(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma),
+  return (any ? launch_bwd<1, true> : launch_bwd<1, false>)(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma),
                        omega, reinterpret_cast<const cf*>(h0), dp, reinterpret_cast<cf*>(dq),
                        reinterpret_cast<cf*>(dgamma), domega, reinterpret_cast<cf*>(dh0), B, D, N, L,
                        static_cast<hipStream_t>(stream));

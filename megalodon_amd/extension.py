@@ -630,6 +630,8 @@ def cema_scan_supported(x: torch.Tensor, ndim: int) -> bool:
     on the GPU, at most 32 modes (16 per launch), a length that is a multiple of 8."""
     if not x.is_cuda or x.dim() != 3 or x.dtype not in (torch.bfloat16, torch.float16, torch.float32) or ndim > 32:
         return False
+    if x.shape[-1] % 8 != 0:
+        return False
     fn = _lib.load().mega_cema_scan_supported
     return bool(fn(_lib.i32(_lib.dtype_code(x.dtype)), _lib.i64(min(ndim, 16)), _lib.i64(x.shape[-1])))
 
@@ -646,6 +648,8 @@ def cema_scan_fwd(x: torch.Tensor, p: torch.Tensor, log_q: torch.Tensor, gamma: 
     dev = _require_cuda(x, p, log_q, gamma, omega, h0)
     B, D, L = x.shape
     N = p.shape[1]
+    if L % 8 != 0:
+        raise RuntimeError(f"cema_scan_fwd: the row length must be a multiple of 8 (got {L})")
     xc = x.contiguous()
     if xc.data_ptr() % 16 != 0:
         xc = xc.clone(memory_format=torch.contiguous_format)
@@ -677,6 +681,8 @@ def cema_scan_bwd_supported(x: torch.Tensor, ndim: int) -> bool:
     pieces: 16 significant bits, what the forward takes of float32 rows as well);
     otherwise as the forward."""
     if not x.is_cuda or x.dim() != 3 or x.dtype not in (torch.bfloat16, torch.float16, torch.float32) or ndim > 32:
+        return False
+    if x.shape[-1] % 8 != 0:
         return False
     fn = _lib.load().mega_cema_scan_bwd_supported
     return bool(fn(_lib.i32(_lib.dtype_code(torch.bfloat16)), _lib.i64(min(ndim, 16)), _lib.i64(x.shape[-1])))
@@ -736,6 +742,8 @@ def cema_scan_bwd(y_grad: torch.Tensor, x: torch.Tensor, p: torch.Tensor, log_q:
     N = p.shape[1]
     if y_grad.shape != x.shape or y_grad.dtype != x.dtype:
         raise RuntimeError("cema_scan_bwd: y_grad must match x in shape and dtype")
+    if L % 8 != 0:
+        raise RuntimeError(f"cema_scan_bwd: the row length must be a multiple of 8 (got {L})")
     pc = p.reshape(D, N).contiguous().float()
     lq, gm = _as_c64(log_q, "log_q").reshape(D, N), _as_c64(gamma, "gamma").reshape(D, N)
     wc = None if omega is None else omega.reshape(-1).contiguous().float()
@@ -825,6 +833,7 @@ def timestep_norm_status(device=None) -> None:
             ws = _tsn_ws_cache.get((idx, stream, backward))
             if ws is not None:
                 _lib.call("mega_group_timestep_norm_status", _lib.ptr(ws), _lib.stream_ptr(dev))
+
 
 
 def _mask_bytes(padding_mask):
