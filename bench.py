@@ -347,16 +347,10 @@ def cema_leg(torch, dev, steps, warmup, copy_calibration):
 
     for _ in range(warmup):
         step()
-    log = {"mega_cema_scan_fwd": [], "mega_cema_scan_bwd_state": [], "mega_cema_coeffs_fwd": [], "mega_cema_coeffs_bwd": []}
-    _lib.set_event_log(log)
     dt = timed(steps)
-    _lib.set_event_log(None)
-    avg = {k: (sum(a.elapsed_time(b) for a, b in v) / max(1, len(v))) for k, v in log.items()}
     E = B * D * L
     # the two recurrence kernels launched back to back on the layer's own operands, device events
-    # around the run: the launch duration without the host's time to issue it (inside a step the
-    # device is idle when the first event of a call is recorded, so `kernels_ms` above holds the
-    # 10-25 us the host takes to launch as well)
+    # around the run: the launch duration without the host's time to issue it
     from megalodon_amd import extension as ops
     n_k = 20 if steps >= 5 else max(1, steps)
     with torch.no_grad():
@@ -365,6 +359,11 @@ def cema_leg(torch, dev, steps, warmup, copy_calibration):
         xd = x.detach()
         ms_f = dev_ms(torch, lambda: ops.cema_scan_fwd(xd, cp, clq, cgm, layer.omega), n_k, warm=min(3, n_k))
         ms_b = dev_ms(torch, lambda: ops.cema_scan_bwd(dy, xd, cp, clq, cgm, layer.omega), n_k, warm=min(3, n_k))
+        raw = [getattr(layer, n_).float() for n_ in ("alpha", "delta", "theta", "gamma")]
+        zp, zq = torch.zeros_like(cp), torch.zeros_like(cgm)
+        avg = {"mega_cema_scan_fwd": ms_f, "mega_cema_scan_bwd_state": ms_b,
+               "mega_cema_coeffs_fwd": dev_ms(torch, lambda: ops.cema_coeffs_fwd(*raw), n_k, warm=min(3, n_k)),
+               "mega_cema_coeffs_bwd": dev_ms(torch, lambda: ops.cema_coeffs_bwd(zp, zq, zq, *raw[:3]), n_k, warm=min(3, n_k))}
     res = {"ms_per_step": dt * 1e3, "tokens_per_s": B * L / dt,
            "GBps_on_10E": 10 * E / dt / 1e9, "frac_hbm_on_10E": 10 * E / dt / 1e9 / HBM_PEAK_GBS,
            "kernels_ms": avg,
@@ -489,16 +488,10 @@ def cema_leg(torch, dev, steps, warmup, copy_calibration):
 
     for _ in range(warmup):
         step()
-    log = {"mega_cema_scan_fwd": [], "mega_cema_scan_bwd_state": [], "mega_cema_coeffs_fwd": [], "mega_cema_coeffs_bwd": []}
-    _lib.set_event_log(log)
     dt = timed(steps)
-    _lib.set_event_log(None)
-    avg = {k: (sum(a.elapsed_time(b) for a, b in v) / max(1, len(v))) for k, v in log.items()}
     E = B * D * L
     # the two recurrence kernels launched back to back on the layer's own operands, device events
-    # around the run: the launch duration without the host's time to issue it (inside a step the
-    # device is idle when the first event of a call is recorded, so `kernels_ms` above holds the
-    # 10-25 us the host takes to launch as well)
+    # around the run: the launch duration without the host's time to issue it
     from megalodon_amd import extension as ops
     n_k = 20 if steps >= 5 else max(1, steps)
     with torch.no_grad():
@@ -507,6 +500,11 @@ def cema_leg(torch, dev, steps, warmup, copy_calibration):
         xd = x.detach()
         ms_f = dev_ms(torch, lambda: ops.cema_scan_fwd(xd, cp, clq, cgm, layer.omega), n_k, warm=min(3, n_k))
         ms_b = dev_ms(torch, lambda: ops.cema_scan_bwd(dy, xd, cp, clq, cgm, layer.omega), n_k, warm=min(3, n_k))
+        raw = [getattr(layer, n_).float() for n_ in ("alpha", "delta", "theta", "gamma")]
+        zp, zq = torch.zeros_like(cp), torch.zeros_like(cgm)
+        avg = {"mega_cema_scan_fwd": ms_f, "mega_cema_scan_bwd_state": ms_b,
+               "mega_cema_coeffs_fwd": dev_ms(torch, lambda: ops.cema_coeffs_fwd(*raw), n_k, warm=min(3, n_k)),
+               "mega_cema_coeffs_bwd": dev_ms(torch, lambda: ops.cema_coeffs_bwd(zp, zq, zq, *raw[:3]), n_k, warm=min(3, n_k))}
     res = {"ms_per_step": dt * 1e3, "tokens_per_s": B * L / dt,
            "GBps_on_10E": 10 * E / dt / 1e9, "frac_hbm_on_10E": 10 * E / dt / 1e9 / HBM_PEAK_GBS,
            "kernels_ms": avg,

@@ -688,6 +688,39 @@ int mega_split_bf16(const void* src, int dtype, int64_t n, void* hi, void* lo, v
 int mega_bench_stream_copy(const void* a, const void* b, void* out, int64_t bytes,
                            int workgroups, int nontemporal, void* stream);
 
+/* mega_cema_coeffs_fwd / _bwd on parameters of element type `dtype` (as a layer cast to bfloat16 holds
+ * them), the gradients in that type too; arithmetic float32.  The incoming gradients are `sets` stacks
+ * (sets, D, N), added up here -- one per sequence, as the recurrence's backward leaves them;
+ * dskip (sets, D) likewise gives domega (D) (both NULL: left out). */
+int mega_cema_layer_coeffs_fwd(int dtype, const void* alpha, const void* delta, const void* theta,
+                               const void* gamma, int64_t D, int64_t N, float* p, float* log_q,
+                               float* gamma_hat, void* stream);
+int mega_cema_layer_coeffs_bwd(int dtype, const float* dp, const float* dq, const float* dgamma_hat,
+                               const float* dskip, int64_t sets, const void* alpha,
+                               const void* delta, const void* theta, int64_t D, int64_t N,
+                               void* dalpha, void* ddelta, void* dtheta, void* dgamma,
+                               void* domega, void* stream);
+
+/* mega_group_timestep_norm_fwd_tl / _bwd_tl as the layer calls them
+ * (modules/timestep_norm.py:106-131): `weight` is the stored gamma - 1 (its gradient is gamma's), and with
+ * `shared_prior` the previous statistics are the layer's prior, one row for every sequence:
+ * prev_count one int64, prev_mean (G), prev_var (G) the logarithm of the variance.  In the backward
+ * dmean and dvar may be NULL (zero); with `shared_prior` dprev_mean and dprev_var are still per sequence, those of
+ * mean and variance. */
+int mega_timestep_norm_layer_fwd(const void* x, int dtype, const int64_t* prev_count,
+                                 const void* prev_mean, const void* prev_var, int shared_prior,
+                                 const void* weight, const void* bias, const uint8_t* padding_mask,
+                                 int64_t B, int64_t L, int64_t D, int64_t G, double eps, void* y,
+                                 int64_t* count, void* mean, void* var, float* cummean,
+                                 float* cumrstd, void* workspace, void* stream);
+int mega_timestep_norm_layer_bwd(const void* dy, const void* dmean, const void* dvar, const void* x,
+                                 int dtype, const void* prev_mean, int shared_prior,
+                                 const int64_t* count, const float* cummean, const float* cumrstd,
+                                 const void* weight, const uint8_t* padding_mask, int64_t B,
+                                 int64_t L, int64_t D, int64_t G, void* dx, void* dprev_mean,
+                                 void* dprev_var, void* dweight, void* dbias, void* workspace,
+                                 void* stream);
+
 /* ------------------------------------------------------------------------
  * One new token per sequence through a whole block, continuing a cache: the
  * cache branch of moving_average_gated_attention.py:283-348 at sequence length

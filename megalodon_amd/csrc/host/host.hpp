@@ -42,5 +42,6 @@ inline int code_of(at::ScalarType t) {
 }
 
 void bind_decode(py::module_& m);
+void bind_ops(py::module_& m);
 
 }  // namespace mega_host

@@ -3,4 +3,5 @@
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   mega_host::bind_decode(m);
+  mega_host::bind_ops(m);
 }

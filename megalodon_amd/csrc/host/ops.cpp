@@ -1,0 +1,573 @@
+// The differentiable operators of a block as C++ autograd nodes: check, allocate, launch -- and the
+// same in the backward, on the autograd engine's thread, without the interpreter.  A Python node
+// costs 10-15 us per direction, more than most of these kernels run for at ordinary sizes.
+#include "host.hpp"
+
+#include <torch/csrc/autograd/custom_function.h>
+
+#include <map>
+#include <mutex>
+#include <tuple>
+#include <vector>
+
+namespace mega_host {
+namespace {
+
+using torch::autograd::AutogradContext;
+using torch::autograd::Function;
+using torch::autograd::variable_list;
+using Optional = std::optional<Tensor>;
+
+int kernel_code(const Tensor& t) {
+  const int code = code_of(t.scalar_type());
+  if (code < 0) fail("unsupported dtype " + std::string(c10::toString(t.scalar_type())) + " (float32, bfloat16, float16 are supported)");
+  return code;
+}
+void need_gpu(std::initializer_list<const Tensor*> ts) {
+  const Tensor* first = nullptr;
+  for (const Tensor* t : ts) {
+    if (t == nullptr || !t->defined()) continue;
+    require(t->is_cuda(), "megalodon_amd ops need GPU (HIP) tensors; there is no CPU fallback");
+    if (first == nullptr) first = t;
+    require(t->device() == first->device(), "all tensors must be on the same device");
+  }
+}
+const Tensor* maybe(const Optional& t) { return t.has_value() ? &*t : nullptr; }
+void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+float* fptr(const Tensor& t) { return static_cast<float*>(ptr(t)); }
+Tensor some(const Optional& t) { return t.has_value() ? t->contiguous() : Tensor(); }
+Tensor bytes(int64_t n, const Tensor& like) { return at::empty({n}, like.options().dtype(at::kByte)); }
+Tensor floats(at::IntArrayRef shape, const Tensor& like) { return at::empty(shape, like.options().dtype(at::kFloat)); }
+bool wants_grad(std::initializer_list<const Tensor*> ts) {
+  if (!at::GradMode::is_enabled()) return false;
+  for (const Tensor* t : ts)
+    if (t != nullptr && t->defined() && t->requires_grad()) return true;
+  return false;
+}
+
+// ---- x.transpose(-2, -1).contiguous() ------------------------------------------------
+Tensor transpose_raw(const Tensor& x) {
+  need_gpu({&x});
+  require(x.dim() >= 2, "transpose_last2: x needs at least two dimensions");
+  const int code = kernel_code(x);
+  c10::DeviceGuard guard(x.device());
+  const Tensor xc = x.contiguous();
+  const int64_t R = xc.size(-2), C = xc.size(-1);
+  auto shape = xc.sizes().vec();
+  std::swap(shape[shape.size() - 1], shape[shape.size() - 2]);
+  Tensor out = at::empty(shape, xc.options());
+  check(mega_transpose(xc.data_ptr(), code, R * C > 0 ? xc.numel() / (R * C) : 0, R, C, out.data_ptr(), stream_of(x)), "mega_transpose");
+  return out;
+}
+struct TransposeFn : Function<TransposeFn> {
+  static Tensor forward(AutogradContext*, const Tensor& x) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    return transpose_raw(x);
+  }
+  static variable_list backward(AutogradContext*, variable_list g) { return {transpose_raw(g[0])}; }
+};
+Tensor transpose_last2(const Tensor& x) { return wants_grad({&x}) ? TransposeFn::apply(x) : transpose_raw(x); }
+
+// ---- silu(a) b ------------------------------------------------------------------------
+Tensor silu_mul_raw(const Tensor& a, const Tensor& b) {
+  need_gpu({&a, &b});
+  require(a.sizes() == b.sizes() && a.scalar_type() == b.scalar_type(), "silu_mul: a and b must have the same shape and dtype");
+  const int code = kernel_code(a);
+  c10::DeviceGuard guard(a.device());
+  const Tensor ac = a.contiguous(), bc = b.contiguous();
+  Tensor out = at::empty_like(ac);
+  check(mega_silu_mul_fwd(ac.data_ptr(), bc.data_ptr(), code, ac.numel(), out.data_ptr(), stream_of(a)), "mega_silu_mul_fwd");
+  return out;
+}
+struct SiluMulFn : Function<SiluMulFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& a, const Tensor& b) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    ctx->save_for_backward({a, b});
+    return silu_mul_raw(a, b);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const auto saved = ctx->get_saved_variables();
+    const Tensor a = saved[0].contiguous(), b = saved[1].contiguous(), go = g[0].contiguous();
+    c10::DeviceGuard guard(a.device());
+    Tensor da = at::empty_like(a), db = at::empty_like(b);
+    check(mega_silu_mul_bwd(go.data_ptr(), a.data_ptr(), b.data_ptr(), kernel_code(a), a.numel(), da.data_ptr(), db.data_ptr(), stream_of(a)), "mega_silu_mul_bwd");
+    return {da, db};
+  }
+};
+Tensor silu_mul(const Tensor& a, const Tensor& b) { return wants_grad({&a, &b}) ? SiluMulFn::apply(a, b) : silu_mul_raw(a, b); }
+
+// ---- LayerNorm / RMSNorm over the last axis, stored weight gamma - 1 ------------------------
+std::tuple<Tensor, Tensor, Tensor> layer_norm_raw(const Tensor& x, const Optional& weight, const Optional& bias, double eps, bool rms) {
+  need_gpu({&x});
+  const int64_t D = x.size(-1);
+  for (const Optional* t : {&weight, &bias})
+    if (t->has_value())
+      require((*t)->dim() == 1 && (*t)->size(0) == D && (*t)->scalar_type() == x.scalar_type() && (*t)->device() == x.device(),
+              "layer_norm: weight and bias must have the last axis' length, x's dtype and x's device");
+  const int code = kernel_code(x);
+  c10::DeviceGuard guard(x.device());
+  const Tensor xc = x.contiguous(), w = some(weight), b = rms ? Tensor() : some(bias);
+  const int64_t rows = D > 0 ? xc.numel() / D : 0;
+  Tensor y = at::empty_like(xc), mean = rms ? Tensor() : floats({rows}, x), rstd = floats({rows}, x);
+  check(mega_layer_norm_fwd(xc.data_ptr(), ptr(w), ptr(b), code, rows, D, eps, rms, y.data_ptr(), fptr(mean), fptr(rstd), stream_of(x)), "mega_layer_norm_fwd");
+  return {y, mean, rstd};
+}
+struct LayerNormFn : Function<LayerNormFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Optional& weight, const Optional& bias, double eps, bool rms) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    auto [y, mean, rstd] = layer_norm_raw(x, weight, bias, eps, rms);
+    ctx->save_for_backward({x, weight.value_or(Tensor()), mean, rstd});
+    ctx->saved_data["rms"] = rms;
+    ctx->saved_data["bias"] = bias.has_value();
+    return y;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const auto saved = ctx->get_saved_variables();
+    const bool rms = ctx->saved_data["rms"].toBool(), has_bias = ctx->saved_data["bias"].toBool();
+    const Tensor x = saved[0].contiguous(), weight = saved[1].defined() ? saved[1].contiguous() : Tensor(), go = g[0].contiguous();
+    require(go.scalar_type() == x.scalar_type(), "layer_norm_bwd: y_grad and x must have the same shape and dtype");
+    c10::DeviceGuard guard(x.device());
+    const int64_t D = x.size(-1), rows = D > 0 ? x.numel() / D : 0;
+    Tensor dx = at::empty_like(x), dw, db, ws;
+    if (weight.defined()) {
+      dw = at::empty_like(weight);
+      ws = bytes(mega_layer_norm_workspace_bytes(rows, D), x);
+    }
+    if (has_bias && !rms && weight.defined()) db = at::empty_like(weight);
+    if (rows == 0) {
+      if (dw.defined()) dw.zero_();
+      if (db.defined()) db.zero_();
+    } else {
+      check(mega_layer_norm_bwd(go.data_ptr(), x.data_ptr(), ptr(weight), fptr(saved[2]), fptr(saved[3]), kernel_code(x), rows, D, rms, dx.data_ptr(), ptr(dw), ptr(db), ptr(ws), stream_of(x)), "mega_layer_norm_bwd");
+    }
+    return {dx, dw, db, Tensor(), Tensor()};
+  }
+};
+Tensor layer_norm_plus_one(const Tensor& x, const Optional& weight, const Optional& bias, double eps, bool rms) {
+  if (wants_grad({&x, maybe(weight), maybe(bias)})) return LayerNormFn::apply(x, weight, bias, eps, rms);
+  return std::get<0>(layer_norm_raw(x, weight, bias, eps, rms));
+}
+
+// ---- z -> (q, k): per-head RMSNorm, two affine maps, rotary -----------------------------------
+Tensor real_freqs(const Optional& freqs, int64_t head_dim, const Tensor& z) {
+  if (!freqs.has_value()) return Tensor();
+  require(freqs->dim() == 2 && freqs->size(1) == head_dim / 2 && freqs->is_complex(), "qk_norm_rotary: freqs_cis must be complex (positions, head_dim / 2)");
+  return freqs->to(z.device(), at::kComplexFloat).contiguous();
+}
+std::tuple<Tensor, Tensor, Tensor> qk_raw(const Tensor& z, const Tensor& gamma, const Tensor& beta, const Tensor& fr, int64_t head_dim, double eps) {
+  need_gpu({&z, &gamma, &beta});
+  require(z.dim() == 3 && gamma.dim() == 2 && gamma.size(0) == 2 && gamma.size(1) == z.size(2) && beta.sizes() == gamma.sizes(), "qk_norm_rotary: z must be (B, L, S), gamma and beta (2, S)");
+  const int code = kernel_code(z);
+  const Tensor zc = z.contiguous(), gc = gamma.contiguous(), bc = beta.contiguous();
+  const int64_t B = z.size(0), L = z.size(1), S = z.size(2);
+  Tensor q = at::empty_like(zc), k = at::empty_like(zc), rstd = floats({B * L, S / head_dim}, z);
+  check(mega_qk_norm_rotary_fwd(zc.data_ptr(), gc.data_ptr(), bc.data_ptr(), fptr(fr), code, B * L, L, fr.defined() ? fr.size(0) : 1, S, head_dim, eps, q.data_ptr(), k.data_ptr(), fptr(rstd), stream_of(z)), "mega_qk_norm_rotary_fwd");
+  return {q, k, rstd};
+}
+struct QkFn : Function<QkFn> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& z, const Tensor& gamma, const Tensor& beta, const Optional& freqs, int64_t head_dim, double eps) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor fr = freqs.value_or(Tensor());
+    auto [q, k, rstd] = qk_raw(z, gamma, beta, fr, head_dim, eps);
+    ctx->save_for_backward({z, gamma, rstd, fr});
+    ctx->saved_data["head_dim"] = head_dim;
+    return {q, k};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const auto saved = ctx->get_saved_variables();
+    const Tensor z = saved[0].contiguous(), gamma = saved[1].contiguous(), dq = g[0].contiguous(), dk = g[1].contiguous();
+    const Tensor& fr = saved[3];
+    c10::DeviceGuard guard(z.device());
+    const int64_t B = z.size(0), L = z.size(1), S = z.size(2);
+    Tensor dz = at::empty_like(z), dgamma = at::empty_like(gamma), dbeta = at::empty_like(gamma), ws = bytes(mega_qk_norm_rotary_workspace_bytes(S), z);
+    check(mega_qk_norm_rotary_bwd(dq.data_ptr(), dk.data_ptr(), z.data_ptr(), gamma.data_ptr(), fptr(saved[2]), fptr(fr), kernel_code(z), B * L, L, fr.defined() ? fr.size(0) : 1, S, ctx->saved_data["head_dim"].toInt(), dz.data_ptr(), dgamma.data_ptr(), dbeta.data_ptr(), ws.data_ptr(), stream_of(z)), "mega_qk_norm_rotary_bwd");
+    return {dz, dgamma, dbeta, Tensor(), Tensor(), Tensor()};
+  }
+};
+std::tuple<Tensor, Tensor> qk_norm_rotary(const Tensor& z, const Tensor& gamma, const Tensor& beta, const Optional& freqs, int64_t head_dim, double eps) {
+  c10::OptionalDeviceGuard guard;
+  if (z.is_cuda()) guard.reset_device(z.device());
+  const Tensor fr = real_freqs(freqs, head_dim, z);
+  if (wants_grad({&z, &gamma, &beta})) {
+    auto qk = QkFn::apply(z, gamma, beta, fr.defined() ? Optional(fr) : Optional(), head_dim, eps);
+    return {qk[0], qk[1]};
+  }
+  auto [q, k, rstd] = qk_raw(z, gamma, beta, fr, head_dim, eps);
+  return {q, k};
+}
+
+// ---- TimestepNorm, the layer's call -------------------------------------------------------------
+// The last workspace of every (device, stream, direction) is kept for its status word
+// (timestep_norm_status); the launches themselves take a fresh one each, so calls of
+// different threads never share one.
+std::mutex last_mutex;
+std::map<std::tuple<int, void*, bool>, Tensor> last_workspace;
+Tensor tsn_workspace(const Tensor& x, int64_t groups, bool backward) {
+  Tensor ws = bytes(mega_group_timestep_norm_workspace_bytes(x.size(0), x.size(1), x.size(2), groups, backward), x);
+  std::lock_guard<std::mutex> lock(last_mutex);
+  last_workspace[{x.device().index(), stream_of(x), backward}] = ws;
+  return ws;
+}
+std::vector<Tensor> tsn_last_workspaces(int device, uintptr_t stream) {
+  std::lock_guard<std::mutex> lock(last_mutex);
+  std::vector<Tensor> out;
+  for (const bool backward : {false, true}) {
+    auto it = last_workspace.find({device, reinterpret_cast<void*>(stream), backward});
+    if (it != last_workspace.end()) out.push_back(it->second);
+  }
+  return out;
+}
+struct TsnOut {
+  Tensor y, count, mean, var, cummean, cumrstd;
+};
+TsnOut tsn_raw(const Tensor& x, const Tensor& count0, const Tensor& mean0, const Tensor& var0, bool shared, const Tensor& weight, const Tensor& bias, const Optional& mask, int64_t groups, double eps) {
+  const int64_t B = x.size(0), L = x.size(1), D = x.size(2);
+  TsnOut o;
+  o.y = at::empty_like(x);
+  o.count = at::empty({B}, x.options().dtype(at::kLong));
+  o.mean = at::empty({B, groups}, x.options());
+  o.var = at::empty({B, groups}, x.options());
+  o.cummean = floats({B, groups, L}, x);
+  o.cumrstd = floats({B, groups, L}, x);
+  const Tensor m = some(mask), ws = tsn_workspace(x, groups, false);
+  check(mega_timestep_norm_layer_fwd(x.data_ptr(), kernel_code(x), count0.data_ptr<int64_t>(), mean0.data_ptr(), var0.data_ptr(), shared, weight.data_ptr(), bias.data_ptr(), static_cast<const uint8_t*>(ptr(m)), B, L, D, groups, eps, o.y.data_ptr(), o.count.data_ptr<int64_t>(), o.mean.data_ptr(), o.var.data_ptr(), fptr(o.cummean), fptr(o.cumrstd), ws.data_ptr(), stream_of(x)), "mega_timestep_norm_layer_fwd");
+  return o;
+}
+struct TsnFn : Function<TsnFn> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& count0, const Tensor& mean0, const Tensor& var0, bool shared, const Tensor& weight, const Tensor& bias, const Optional& mask, int64_t groups, double eps) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor xc = x.contiguous();
+    TsnOut o = tsn_raw(xc, count0, mean0, var0, shared, weight, bias, mask, groups, eps);
+    ctx->save_for_backward({xc, mean0, o.count, o.cummean, o.cumrstd, weight, mask.value_or(Tensor())});
+    ctx->saved_data["groups"] = groups;
+    ctx->saved_data["shared"] = shared;
+    ctx->mark_non_differentiable({o.count});
+    ctx->set_materialize_grads(false);
+    return {o.y, o.count, o.mean, o.var};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &mean0 = saved[1], &weight = saved[5];
+    c10::DeviceGuard guard(x.device());
+    const int64_t B = x.size(0), L = x.size(1), D = x.size(2), groups = ctx->saved_data["groups"].toInt();
+    const bool shared = ctx->saved_data["shared"].toBool();
+    const Tensor dy = g[0].defined() ? g[0].contiguous() : at::zeros_like(x);
+    const Tensor dm = g[2].defined() ? g[2].contiguous() : Tensor(), dv = g[3].defined() ? g[3].contiguous() : Tensor();
+    const Tensor mask = saved[6].defined() ? saved[6].contiguous() : Tensor();
+    require(dy.scalar_type() == x.scalar_type(), "timestep_norm: y_grad must have x's dtype");
+    Tensor dx = at::empty_like(x), dpm = at::empty({B, groups}, x.options()), dpv = at::empty({B, groups}, x.options()), dw = at::empty_like(weight), db = at::empty_like(weight);
+    const Tensor ws = tsn_workspace(x, groups, true);
+    check(mega_timestep_norm_layer_bwd(dy.data_ptr(), ptr(dm), ptr(dv), x.data_ptr(), kernel_code(x), mean0.data_ptr(), shared, saved[2].data_ptr<int64_t>(), fptr(saved[3]), fptr(saved[4]), weight.data_ptr(), static_cast<const uint8_t*>(ptr(mask)), B, L, D, groups, dx.data_ptr(), dpm.data_ptr(), dpv.data_ptr(), dw.data_ptr(), db.data_ptr(), ws.data_ptr(), stream_of(x)), "mega_timestep_norm_layer_bwd");
+    if (shared) dpm = dpv = Tensor();  // the prior is no parameter here
+    return {dx, Tensor(), dpm, dpv, Tensor(), dw, db, Tensor(), Tensor(), Tensor()};
+  }
+};
+// (y, count, mean, var), or None where the layer has to prepare its operands itself (other element
+// types of weights or statistics, a prior that is trained)
+py::object timestep_norm_layer(const Tensor& x, const Optional& prev_count, const Optional& prev_mean, const Optional& prev_var, const Tensor& prior_count, const Tensor& prior_mean, const Tensor& prior_logv, const Tensor& weight, const Tensor& bias, const Optional& mask, int64_t groups, double eps) {
+  const bool shared = !prev_count.has_value();
+  if (!x.is_cuda() || x.dim() != 3 || code_of(x.scalar_type()) < 0 || x.size(0) < 1 || x.size(1) < 1) return py::none();
+  if (prev_mean.has_value() == shared || prev_var.has_value() == shared) return py::none();
+  const Tensor &count = shared ? prior_count : *prev_count, &mean = shared ? prior_mean : *prev_mean, &var = shared ? prior_logv : *prev_var;
+  if (shared && at::GradMode::is_enabled() && (mean.requires_grad() || var.requires_grad())) return py::none();
+  const int64_t B = x.size(0), D = x.size(2);
+  const auto is = [&](const Tensor& t, at::ScalarType type, int64_t n) { return t.scalar_type() == type && t.device() == x.device() && t.numel() == n && t.is_contiguous(); };
+  if (!is(weight, x.scalar_type(), D) || !is(bias, x.scalar_type(), D) || !is(count, at::kLong, shared ? 1 : B) || !is(mean, x.scalar_type(), shared ? groups : B * groups) || !is(var, x.scalar_type(), shared ? groups : B * groups)) return py::none();
+  if (mask.has_value()) {
+    if (mask->scalar_type() != at::kBool) fail("padding_mask must be a bool tensor");
+    if (mask->device() != x.device() || mask->numel() != B * x.size(1)) return py::none();
+  }
+  c10::DeviceGuard guard(x.device());
+  if (wants_grad({&x, &mean, &var, &weight, &bias})) {
+    auto o = TsnFn::apply(x, count, mean, var, shared, weight, bias, mask, groups, eps);
+    return py::make_tuple(o[0], o[1], o[2], o[3]);
+  }
+  TsnOut o = tsn_raw(x.contiguous(), count, mean, var, shared, weight, bias, mask, groups, eps);
+  return py::make_tuple(o.y, o.count, o.mean, o.var);
+}
+
+// ---- the EMA layer without a carried state ------------------------------------------------------
+// Coefficients in one float32 buffer (p, log q, gamma_hat), then the recurrence.
+Tensor cema_coeffs(const Tensor& alpha, const Tensor& delta, const Tensor& theta, const Tensor& gamma, int64_t D, int64_t N) {
+  Tensor c = floats({5 * D * N}, alpha);
+  float* p = c.data_ptr<float>();
+  check(mega_cema_layer_coeffs_fwd(kernel_code(alpha), alpha.data_ptr(), delta.data_ptr(), theta.data_ptr(), gamma.data_ptr(), D, N, p, p + D * N, p + 3 * D * N, stream_of(alpha)), "mega_cema_layer_coeffs_fwd");
+  return c;
+}
+Tensor scan_raw(const Tensor& x, const float* p, const float* log_q, const float* gamma_hat, const float* omega, const float* h0, float* h_last, int64_t N) {
+  Tensor y = at::empty_like(x);
+  check(mega_cema_scan_fwd(x.data_ptr(), kernel_code(x), p, log_q, gamma_hat, omega, h0, x.size(0), x.size(1), N, x.size(2), y.data_ptr(), h_last, stream_of(x)), "mega_cema_scan_fwd");
+  return y;
+}
+// float32 (contiguous) form of the skip weight
+Tensor as_float(const Tensor& t) { return t.to(at::kFloat).contiguous(); }
+// rows as the recurrence kernels take them: float32 ones on 16-byte boundaries
+Tensor rows_of(const Tensor& x) {
+  Tensor c = x.contiguous();
+  if (c.scalar_type() == at::kFloat && reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 != 0) c = c.clone(at::MemoryFormat::Contiguous);
+  return c;
+}
+std::tuple<Tensor, Tensor> split(const Tensor& t) {
+  const int64_t n = t.numel();
+  if (n % 8 != 0 || reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0) {
+    Tensor hi = t.to(at::kBFloat16);
+    return {hi, (t.to(at::kFloat) - hi.to(at::kFloat)).to(at::kBFloat16)};
+  }
+  Tensor hi = at::empty(t.sizes(), t.options().dtype(at::kBFloat16)), lo = at::empty_like(hi);
+  check(mega_split_bf16(t.data_ptr(), kernel_code(t), n, hi.data_ptr(), lo.data_ptr(), stream_of(t)), "mega_split_bf16");
+  return {hi, lo};
+}
+struct CemaFn : Function<CemaFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& alpha, const Tensor& delta, const Tensor& theta, const Tensor& gamma, const Tensor& omega) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const int64_t D = x.size(1), N = alpha.size(1);
+    const Tensor xc = rows_of(x), w = as_float(omega), c = cema_coeffs(alpha, delta, theta, gamma, D, N);
+    const float* p = c.data_ptr<float>();
+    Tensor y = scan_raw(xc, p, p + D * N, p + 3 * D * N, fptr(w), nullptr, nullptr, N);
+    ctx->save_for_backward({xc, alpha, delta, theta, gamma, omega, c, w});
+    return y;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &alpha = saved[1], &delta = saved[2], &theta = saved[3], &gamma = saved[4], &omega = saved[5], &c = saved[6], &w = saved[7];
+    require(g[0].sizes() == x.sizes() && g[0].scalar_type() == x.scalar_type(), "cema: y_grad must match x in shape and dtype");
+    c10::DeviceGuard guard(x.device());
+    const Tensor dy = rows_of(g[0]);
+    const int64_t B = x.size(0), D = x.size(1), L = x.size(2), N = alpha.size(1), DN = D * N;
+    const float *p = c.data_ptr<float>(), *lq = p + DN, *gh = p + 3 * DN;
+    void* s = stream_of(x);
+    // per-row gradients of the launches, stacked: (dp, dq, dgamma_hat, domega); the coefficients'
+    // backward adds the stack up
+    const int64_t sets = x.scalar_type() == at::kBFloat16 ? B : 3 * B;
+    const Tensor stack = floats({sets * (5 * DN + D)}, x);
+    float *dp = stack.data_ptr<float>(), *dq = dp + sets * DN, *dg = dq + 2 * sets * DN, *dw = dg + 2 * sets * DN;
+    Tensor dx;
+    if (x.scalar_type() == at::kBFloat16) {
+      dx = at::empty_like(x);
+      check(mega_cema_scan_bwd(dy.data_ptr(), x.data_ptr(), MEGA_BF16, p, lq, gh, fptr(w), B, D, N, L, dx.data_ptr(), dp, dq, dg, dw, s), "mega_cema_scan_bwd");
+    } else {
+      // linear in dy and, for the parameter gradients, in x: the bfloat16 pieces (dy_hi, x_hi), (dy_lo, x_hi),
+      // (dy_hi, x_lo); dx is linear in dy alone and is added up in float32
+      auto [g_hi, g_lo] = split(dy);
+      auto [x_hi, x_lo] = split(x);
+      Tensor dx32 = floats(x.sizes(), x);
+      const Tensor* pairs[3][2] = {{&g_hi, &x_hi}, {&g_lo, &x_hi}, {&g_hi, &x_lo}};
+      for (int i = 0; i < 3; ++i)
+        check(mega_cema_scan_bwd_wide(pairs[i][0]->data_ptr(), pairs[i][1]->data_ptr(), p, lq, gh, fptr(w), nullptr, B, D, N, L, i < 2 ? fptr(dx32) : nullptr, i == 1, dp + i * B * DN, dq + 2 * i * B * DN, dg + 2 * i * B * DN, dw + i * B * D, nullptr, s), "mega_cema_scan_bwd_wide");
+      dx = dx32.to(x.scalar_type());
+    }
+    Tensor da = at::empty_like(alpha), dd = at::empty_like(delta), dt = at::empty_like(theta), dga = at::empty_like(gamma), dom = at::empty_like(omega);
+    check(mega_cema_layer_coeffs_bwd(kernel_code(alpha), dp, dq, dg, dw, sets, alpha.data_ptr(), delta.data_ptr(), theta.data_ptr(), D, N, da.data_ptr(), dd.data_ptr(), dt.data_ptr(), dga.data_ptr(), dom.data_ptr(), s), "mega_cema_layer_coeffs_bwd");
+    return {dx, da, dd, dt, dga, dom};
+  }
+};
+// rows of this shape and type run on the recurrence kernels in one launch per piece
+bool cema_takes(const Tensor& x, int64_t N) {
+  return x.is_cuda() && x.dim() == 3 && N >= 1 && N <= 16 && code_of(x.scalar_type()) >= 0 && x.size(2) >= 1 && (x.scalar_type() != at::kFloat || x.size(2) % 8 == 0) && x.size(0) * x.size(1) <= 0x7fffffff;
+}
+py::object cema(const Tensor& x, const Tensor& alpha, const Tensor& delta, const Tensor& theta, const Tensor& gamma, const Tensor& omega) {
+  if (alpha.dim() != 3 || !cema_takes(x, alpha.size(1))) return py::none();
+  const int64_t D = x.size(1), N = alpha.size(1);
+  const auto is = [&](const Tensor& t, int64_t n) { return t.scalar_type() == alpha.scalar_type() && t.device() == x.device() && t.numel() == n && t.is_contiguous(); };
+  if (code_of(alpha.scalar_type()) < 0 || !is(alpha, D * N) || !is(delta, D * N) || !is(theta, D) || !is(gamma, 2 * D * N) || !is(omega, D)) return py::none();
+  c10::DeviceGuard guard(x.device());
+  if (wants_grad({&x, &alpha, &delta, &theta, &gamma, &omega})) return py::cast(CemaFn::apply(x, alpha, delta, theta, gamma, omega));
+  const Tensor xc = rows_of(x), w = as_float(omega), c = cema_coeffs(alpha, delta, theta, gamma, D, N);
+  const float* p = c.data_ptr<float>();
+  return py::cast(scan_raw(xc, p, p + D * N, p + 3 * D * N, fptr(w), nullptr, nullptr, N));
+}
+// with a carried state and / or the last state wanted, without gradients; p, log_q, gamma_hat float32 / complex64
+py::object cema_state(const Tensor& x, const Tensor& p, const Tensor& log_q, const Tensor& gamma_hat, const Tensor& omega, const Optional& h0, bool last) {
+  const int64_t N = p.size(1);
+  if (!cema_takes(x, N)) return py::none();
+  const int64_t B = x.size(0), D = x.size(1);
+  if (h0.has_value()) require(h0->scalar_type() == at::kComplexFloat && h0->numel() == B * D * N && h0->device() == x.device(), "cema: the carried state must be complex64 (B, D, N)");
+  c10::DeviceGuard guard(x.device());
+  const Tensor xc = rows_of(x), w = as_float(omega), h = some(h0);
+  Tensor h_last;
+  if (last) h_last = at::empty({B, D, N}, x.options().dtype(at::kComplexFloat));
+  Tensor y = scan_raw(xc, p.data_ptr<float>(), fptr(log_q), fptr(gamma_hat), fptr(w), fptr(h), fptr(h_last), N);
+  return py::make_tuple(y, last ? py::cast(h_last) : py::object(py::none()));
+}
+
+// ---- attention ------------------------------------------------------------------------------------
+struct AttnDims {
+  int64_t B, L1, L2, NH, H1, H2;
+};
+AttnDims attn_dims(const Tensor& q, const Tensor& k, const Tensor& v) {
+  need_gpu({&q, &k, &v});
+  require(q.dim() == 4 && k.dim() == 4 && v.dim() == 4, "q, k, v must be (B, L, N, H)");
+  const AttnDims d{q.size(0), q.size(1), k.size(1), q.size(2), q.size(3), v.size(3)};
+  require(k.size(0) == d.B && k.size(2) == d.NH && k.size(3) == d.H1 && v.size(0) == d.B && v.size(1) == d.L2 && v.size(2) == d.NH, "attention: inconsistent shapes");
+  require(q.scalar_type() == k.scalar_type() && q.scalar_type() == v.scalar_type(), "q, k, v must share one dtype");
+  return d;
+}
+std::tuple<Tensor, Tensor> attention_raw(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bool causal) {
+  const AttnDims d = attn_dims(q, k, v);
+  const int code = kernel_code(q);
+  Tensor y = at::empty({d.B, d.L1, d.NH, d.H2}, v.options()), w = at::empty({d.B, d.NH, d.L1, d.L2}, v.options());
+  const Tensor ws = bytes(mega_attention_workspace_bytes(d.B, d.L1, d.L2, d.NH, d.H1, d.H2, 0) * (code == MEGA_F32 ? 2 : 1), q);
+  // w goes to the backward and nowhere else: 2 leaves the zeros right of the diagonal block unwritten
+  check(mega_attention_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), code, d.B, d.L1, d.L2, d.NH, d.H1, d.H2, scale, causal ? 2 : 0, y.data_ptr(), w.data_ptr(), ws.data_ptr(), stream_of(q)), "mega_attention_fwd");
+  return {y, w};
+}
+struct AttentionFn : Function<AttentionFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, double scale, bool causal) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor qc = q.contiguous(), kc = k.contiguous(), vc = v.contiguous();
+    auto [y, w] = attention_raw(qc, kc, vc, scale, causal);
+    ctx->save_for_backward({qc, kc, vc, w});
+    ctx->saved_data["scale"] = scale;
+    ctx->saved_data["causal"] = causal;
+    return y;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &w = saved[3];
+    const AttnDims d = attn_dims(q, k, v);
+    c10::DeviceGuard guard(q.device());
+    const Tensor dy = g[0].contiguous();
+    Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
+    const int code = kernel_code(q);
+    const Tensor ws = bytes(mega_attention_workspace_bytes(d.B, d.L1, d.L2, d.NH, d.H1, d.H2, 1) * (code == MEGA_F32 ? 2 : 1), q);
+    check(mega_attention_bwd(dy.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), w.data_ptr(), code, d.B, d.L1, d.L2, d.NH, d.H1, d.H2, ctx->saved_data["scale"].toDouble(), ctx->saved_data["causal"].toBool(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), stream_of(q)), "mega_attention_bwd");
+    return {dq, dk, dv, Tensor(), Tensor()};
+  }
+};
+Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bool causal) {
+  attn_dims(q, k, v);
+  c10::DeviceGuard guard(q.device());
+  if (wants_grad({&q, &k, &v})) return AttentionFn::apply(q, k, v, scale, causal);
+  return std::get<0>(attention_raw(q.contiguous(), k.contiguous(), v.contiguous(), scale, causal));
+}
+
+// ---- linear layers --------------------------------------------------------------------------------
+// dW = g^T x, (out, in) from (tokens, out) and (tokens, in).  Both operands run across
+// the reduction axis (tokens) here, the slowest layout of the library GEMM on MI355X
+// (0.9-1.2 PFLOP/s at 32768 tokens against 1.5 for the forward's layout).  The attention
+// operator's product kernel takes exactly this layout (dV = P^T dY) and measured, at 32768
+// tokens, out x in = 11008 x 4096: 2.16 ms against 3.28 (3.16 with one operand transposed
+// first), 4096 x 11008: 2.22 / 3.13, 8192 x 4096: 1.54 / 1.87, 4096 x 4096: 0.78 / 0.92;
+// below one 256 x 256 tile per compute unit (1024 x 4096: 0.50 / 0.28 ms) the library stays.
+Tensor weight_grad(const Tensor& g, const Tensor& x) {
+  const int64_t tokens = g.size(0), n_out = g.size(1), n_in = x.size(1);
+  const int64_t tiles = ((n_out + 255) / 256) * ((n_in + 255) / 256);
+  // (operands of 2^30 elements and more leave the kernel's aligned path, whose offsets are 32-bit)
+  if (tokens >= 4096 && tokens % 32 == 0 && n_out % 8 == 0 && n_in % 8 == 0 && tiles >= 256 && tokens * std::max(n_out, n_in) < (1ll << 30)) {
+    const Tensor gc = g.contiguous(), xc = x.contiguous();
+    Tensor dw = at::empty({n_out, n_in}, x.options());
+    check(mega_linear_weight_grad(gc.data_ptr(), xc.data_ptr(), kernel_code(x), tokens, n_out, n_in, dw.data_ptr(), stream_of(x)), "mega_linear_weight_grad");
+    return dw;
+  }
+  return at::mm(g.t(), x);
+}
+Tensor flat(const Tensor& t) { return t.reshape({-1, t.size(-1)}); }
+// x W^T (+ bias), or x W^T + residual with the residual as the product's accumulator input
+Tensor linear_raw(const Tensor& x, const Tensor& weight, const Optional& bias, const Optional& residual) {
+  if (!residual.has_value()) return at::linear(x, weight, bias);
+  auto shape = x.sizes().vec();
+  shape.back() = weight.size(0);
+  return at::addmm(flat(*residual), flat(x), weight.t()).view(shape);
+}
+struct LinearFn : Function<LinearFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, const Optional& bias, const Optional& residual) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    ctx->save_for_backward({x, weight});
+    ctx->saved_data["bias"] = bias.has_value();
+    ctx->saved_data["residual"] = residual.has_value();
+    return linear_raw(x, weight, bias, residual);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &weight = saved[1];
+    const bool has_bias = ctx->saved_data["bias"].toBool(), has_residual = ctx->saved_data["residual"].toBool();
+    c10::DeviceGuard guard(x.device());
+    const Tensor g2 = flat(g[0]);
+    Tensor dx, dw, db, dr;
+    if (ctx->needs_input_grad(0)) dx = at::linear(g2, transpose_raw(weight)).view(x.sizes());  // rows along the reduction axis
+    if (ctx->needs_input_grad(1)) dw = weight_grad(g2, flat(x));
+    if (has_bias && ctx->needs_input_grad(2)) db = g2.sum(0);
+    if (has_residual && ctx->needs_input_grad(has_bias ? 3 : 2)) dr = g[0];
+    return {dx, dw, db, dr};
+  }
+};
+Tensor linear(const Tensor& x, const Tensor& weight, const Optional& bias, const Optional& residual) {
+  if (wants_grad({&x, &weight, maybe(bias), maybe(residual)})) return LinearFn::apply(x, weight, bias, residual);
+  return linear_raw(x, weight, bias, residual);
+}
+
+// several layers of one input: separate products forward, one accumulation of the input's gradient
+struct LinearGroupFn : Function<LinearGroupFn> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& x, at::TensorList params, std::vector<bool> has_bias) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    variable_list keep{x}, out;
+    size_t at_ = 0;
+    std::vector<int64_t> bias_flags;
+    for (const bool b : has_bias) {
+      const Tensor& w = params[at_++];
+      Optional bias;
+      if (b) bias = params[at_++];
+      keep.push_back(w);
+      bias_flags.push_back(b);
+      out.push_back(at::linear(x, w, bias));
+    }
+    ctx->save_for_backward(keep);
+    ctx->saved_data["bias"] = bias_flags;
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const auto saved = ctx->get_saved_variables();
+    const auto has_bias = ctx->saved_data["bias"].toIntVector();
+    const Tensor& x = saved[0];
+    c10::DeviceGuard guard(x.device());
+    const Tensor x2 = flat(x);
+    Tensor dx;
+    variable_list grads{Tensor()};
+    size_t edge = 1;
+    for (size_t i = 0; i < has_bias.size(); ++i) {
+      const Tensor& w = saved[1 + i];
+      const Tensor g2 = flat(g[i]);
+      if (ctx->needs_input_grad(0)) {
+        const Tensor wt = transpose_raw(w);  // (in, out), rows along the reduction axis
+        if (!dx.defined()) dx = at::linear(g2, wt);
+        else at::addmm_out(dx, dx, g2, wt.t());
+      }
+      grads.push_back(ctx->needs_input_grad(edge++) ? weight_grad(g2, x2) : Tensor());
+      if (has_bias[i]) grads.push_back(ctx->needs_input_grad(edge++) ? g2.sum(0) : Tensor());
+    }
+    grads[0] = dx.defined() ? dx.view(x.sizes()) : Tensor();
+    grads.push_back(Tensor());
+    return grads;
+  }
+};
+std::vector<Tensor> linear_group(const Tensor& x, const std::vector<Tensor>& params, const std::vector<bool>& has_bias) {
+  return LinearGroupFn::apply(x, at::TensorList(params), has_bias);
+}
+
+}  // namespace
+
+void bind_ops(py::module_& m) {
+  // a launch may wait for room in the stream's queue: not with the interpreter held
+  using free = py::call_guard<py::gil_scoped_release>;
+  m.def("transpose_last2", &transpose_last2, free());
+  m.def("silu_mul", &silu_mul, free());
+  m.def("layer_norm_plus_one", &layer_norm_plus_one, free());
+  m.def("qk_norm_rotary", &qk_norm_rotary, free());
+  m.def("timestep_norm_layer", &timestep_norm_layer);
+  m.def("tsn_last_workspaces", &tsn_last_workspaces);
+  m.def("cema", &cema);
+  m.def("cema_state", &cema_state);
+  m.def("attention", &attention, free());
+  m.def("linear", &linear, free());
+  m.def("linear_group", &linear_group, free());
+}
+
+}  // namespace mega_host

@@ -74,6 +74,11 @@ struct TsnParams {
   // element strides of cummean / cumrstd: (B, L, G) as the reference stores them, or (B, G, L)
   int64_t st_b, st_t, st_g;
   float eps;
+  // prior statistics: one row per sequence, or (the layer's learned prior) one for all of them, the
+  // variance then as its logarithm
+  int prev_row;     // elements between the sequences' rows of prev_mean / prev_var: G or 0
+  int prior_row;    // the same for prev_count, 1 or 0 (forward)
+  float gamma_plus; // 1 when `gamma` is the stored weight gamma - 1
 };
 
 __device__ __forceinline__ int64_t stat_index(const TsnParams& p, int b, int64_t t, int g) {
@@ -222,6 +227,23 @@ __device__ __forceinline__ float ldT(const void* p, int64_t i) {
 template <int DT>
 __device__ __forceinline__ void stT(void* p, int64_t i, float v) {
   Elem<DT>::store(static_cast<typename Elem<DT>::type*>(p) + i, v);
+}
+
+// prior statistics of a chain (see TsnParams)
+template <int DT>
+__device__ __forceinline__ Wel prior_of(const TsnParams& p, int b, int g) {
+  const int64_t at = static_cast<int64_t>(b) * p.prev_row + g;
+  const float v = ldT<DT>(p.prev_var, at);
+  return Wel{static_cast<float>(p.prev_count[b * p.prior_row]), ldT<DT>(p.prev_mean, at), p.prior_row ? v : expf(v)};
+}
+template <int DT>
+__device__ __forceinline__ float prior_mean(const TsnParams& p, int b, int g) {
+  return ldT<DT>(p.prev_mean, static_cast<int64_t>(b) * p.prev_row + g);
+}
+// gradients that arrive at the final statistics; nobody used them: zero
+template <int DT>
+__device__ __forceinline__ float incoming(const void* d, int64_t chain) {
+  return d != nullptr ? ldT<DT>(d, chain) : 0.f;
 }
 
 // Streamed accesses (store_streaming / load_once).  y (dx) is written once, in whole 128-byte lines, and read by another
@@ -417,8 +439,7 @@ __global__ __launch_bounds__(kThreads) void tsn_fwd_kernel(const TsnParams p) {
     btv = *reinterpret_cast<const uint4*>(static_cast<const typename Elem<DT>::type*>(p.beta) + g * p.Dg + col * VEC);
   }
   const int64_t chain64 = static_cast<int64_t>(b) * p.G + g;
-  const Wel prior{static_cast<float>(p.prev_count[b]), ldT<DT>(p.prev_mean, chain64),
-                  ldT<DT>(p.prev_var, chain64)};
+  const Wel prior = prior_of<DT>(p, b, g);
 #pragma unroll
   for (int q = 0; q < P; ++q) {
     const int r = q * RPP + wave * RPW + lane / LPR;
@@ -471,7 +492,7 @@ __global__ __launch_bounds__(kThreads) void tsn_fwd_kernel(const TsnParams p) {
     if (j == p.NT - 1 && lane == 63) {
       stT<DT>(p.mean, chain64, st.u);
       stT<DT>(p.var, chain64, st.v);
-      if (g == 0) p.count[b] = p.prev_count[b] + p.nbefore[b * (p.NT + 1) + p.NT];
+      if (g == 0) p.count[b] = p.prev_count[b * p.prior_row] + p.nbefore[b * (p.NT + 1) + p.NT];
     }
     // s_a/s_b reads retired before they are overwritten (LDS only: the stores
     // above need not have landed)
@@ -484,6 +505,8 @@ __global__ __launch_bounds__(kThreads) void tsn_fwd_kernel(const TsnParams p) {
 
   float gm[VEC], bt[VEC];
   Vec<DT>::unpack(gmv, gm);
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) gm[e] += p.gamma_plus;
   Vec<DT>::unpack(btv, bt);
 #pragma unroll
   for (int q = 0; q < P; ++q) {
@@ -562,8 +585,7 @@ void tsn_fwd_wave_kernel(const TsnParams p, int tiles) {
     btv = *reinterpret_cast<const uint4*>(static_cast<const typename Elem<DT>::type*>(p.beta) + g * p.Dg + col * VEC);
   }
   const int64_t chain64 = static_cast<int64_t>(b) * p.G + g;
-  const Wel prior{static_cast<float>(p.prev_count[b]), ldT<DT>(p.prev_mean, chain64),
-                  ldT<DT>(p.prev_var, chain64)};
+  const Wel prior = prior_of<DT>(p, b, g);
 #pragma unroll
   for (int q = 0; q < P; ++q) {
     const int r = q * RPW + lane / LPR;
@@ -623,7 +645,7 @@ void tsn_fwd_wave_kernel(const TsnParams p, int tiles) {
   if (j == p.NT - 1 && lane == 63) {
     stT<DT>(p.mean, chain64, st.u);
     stT<DT>(p.var, chain64, st.v);
-    if (g == 0) p.count[b] = p.prev_count[b] + p.nbefore[b * (p.NT + 1) + p.NT];
+    if (g == 0) p.count[b] = p.prev_count[b * p.prior_row] + p.nbefore[b * (p.NT + 1) + p.NT];
   }
   // the row moments were read before the scan (the shuffles above depend on
   // them); a wave runs in program order, so they can be overwritten now
@@ -637,6 +659,8 @@ void tsn_fwd_wave_kernel(const TsnParams p, int tiles) {
 
   float gm[VEC], bt[VEC];
   Vec<DT>::unpack(gmv, gm);
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) gm[e] += p.gamma_plus;
   Vec<DT>::unpack(btv, bt);
   typename Elem<DT>::type* yp = static_cast<typename Elem<DT>::type*>(p.y) + off0;
 #pragma unroll
@@ -662,8 +686,8 @@ __global__ __launch_bounds__(kWave) void tsn_fwd_serial_kernel(const TsnParams p
   const int b = chain / p.G, g = chain % p.G;
   const int lane = threadIdx.x;
   const float inv_dg = 1.f / static_cast<float>(p.Dg);
-  Wel st{static_cast<float>(p.prev_count[b]), ldT<DT>(p.prev_mean, chain), ldT<DT>(p.prev_var, chain)};
-  int64_t cnt = p.prev_count[b];
+  Wel st = prior_of<DT>(p, b, g);
+  int64_t cnt = p.prev_count[b * p.prior_row];
   for (int t = 0; t < p.L; ++t) {
     const int64_t row = (static_cast<int64_t>(b) * p.L + t) * p.D + g * p.Dg;
     const bool valid = p.mask == nullptr || p.mask[static_cast<int64_t>(b) * p.L + t] == 0;
@@ -688,7 +712,7 @@ __global__ __launch_bounds__(kWave) void tsn_fwd_serial_kernel(const TsnParams p
     }
     for (int i = lane; i < p.Dg; i += kWave) {
       const float xx = ldT<DT>(p.x, row + i);
-      const float o = valid ? (xx - st.u) * rstd * ldT<DT>(p.gamma, g * p.Dg + i) +
+      const float o = valid ? (xx - st.u) * rstd * (ldT<DT>(p.gamma, g * p.Dg + i) + p.gamma_plus) +
                                   ldT<DT>(p.beta, g * p.Dg + i)
                             : 0.f;
       stT<DT>(p.y, row + i, o);
@@ -827,9 +851,9 @@ void tsn_bwd_kernel(const TsnParams p) {
     gmv = *reinterpret_cast<const uint4*>(static_cast<const typename Elem<DT>::type*>(p.gamma) + g * p.Dg + col * VEC);
   const int64_t chain64 = static_cast<int64_t>(b) * p.G + g;
   // wave 0 only uses these; loading them in every wave keeps the code uniform
-  const float before_u = t0 == 0 ? ldT<DT>(p.prev_mean, chain64)
+  const float before_u = t0 == 0 ? prior_mean<DT>(p, b, g)
                                  : p.cummean_in[stat_index(p, b, t0 - 1, g)];
-  const State2 init{ldT<DT>(p.dmean, chain64), ldT<DT>(p.dvar, chain64)};
+  const State2 init{incoming<DT>(p.dmean, chain64), incoming<DT>(p.dvar, chain64)};
   const int* nb = p.nbefore + b * (p.NT + 1);
   const int64_t n0 = p.prev_count[b] - nb[p.NT];  // prior count
   const int nbj = nb[j];
@@ -848,6 +872,8 @@ void tsn_bwd_kernel(const TsnParams p) {
   __syncthreads();
   float gm[VEC];
   Vec<DT>::unpack(gmv, gm);
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) gm[e] += p.gamma_plus;
 
 #pragma unroll
   for (int q = 0; q < P; ++q) {
@@ -991,7 +1017,7 @@ __global__ __launch_bounds__(kWave) void tsn_bwd_serial_kernel(const TsnParams p
   const int b = chain / p.G, g = chain % p.G;
   const int lane = threadIdx.x;
   const float inv_dg = 1.f / static_cast<float>(p.Dg);
-  float ug = ldT<DT>(p.dmean, chain), vg = ldT<DT>(p.dvar, chain);
+  float ug = incoming<DT>(p.dmean, chain), vg = incoming<DT>(p.dvar, chain);
   int64_t m0 = p.prev_count[b];
   // per-(batch) partial sums live in part_g/part_b rows [b] (NT == 1 layout)
   for (int i = lane; i < p.Dg; i += kWave) {
@@ -1007,14 +1033,14 @@ __global__ __launch_bounds__(kWave) void tsn_bwd_serial_kernel(const TsnParams p
     }
     const int64_t so = stat_index(p, b, t, g);
     const float u = p.cummean_in[so], r = p.cumrstd_in[so];
-    const float prev_u = t == 0 ? ldT<DT>(p.prev_mean, chain) : p.cummean_in[so - p.st_t];
+    const float prev_u = t == 0 ? prior_mean<DT>(p, b, g) : p.cummean_in[so - p.st_t];
     const float c1 = static_cast<float>(m0 - 1) / static_cast<float>(m0);
     const float c2 = 1.f / static_cast<float>(m0);
     --m0;
     float sx = 0.f, sds = 0.f, sdb = 0.f;
     for (int i = lane; i < p.Dg; i += kWave) {
       const float xx = ldT<DT>(p.x, row + i), d = ldT<DT>(p.dy, row + i);
-      const float w = ldT<DT>(p.gamma, g * p.Dg + i);
+      const float w = ldT<DT>(p.gamma, g * p.Dg + i) + p.gamma_plus;
       sx += xx;
       sds += d * (xx - u) * w;
       sdb += d * w;
@@ -1027,7 +1053,7 @@ __global__ __launch_bounds__(kWave) void tsn_bwd_serial_kernel(const TsnParams p
     const float dvx = c2 * dvv;
     for (int i = lane; i < p.Dg; i += kWave) {
       const float xx = ldT<DT>(p.x, row + i), d = ldT<DT>(p.dy, row + i);
-      const float w = ldT<DT>(p.gamma, g * p.Dg + i);
+      const float w = ldT<DT>(p.gamma, g * p.Dg + i) + p.gamma_plus;
       stT<DT>(p.y, row + i, d * r * w + (dux + 2.f * dvx * (xx - ux)) * inv_dg);
       p.part_g[static_cast<int64_t>(b) * p.D + g * p.Dg + i] += d * (xx - u) * r;
       p.part_b[static_cast<int64_t>(b) * p.D + g * p.Dg + i] += d;
@@ -1261,7 +1287,7 @@ static int tsn_fwd_entry(bool time_last, const void* x, int dtype, const int64_t
                          const void* prev_mean, const void* prev_var, const void* gamma, const void* beta,
                          const uint8_t* padding_mask, int64_t B, int64_t L, int64_t D, int64_t G, double eps,
                          void* y, int64_t* count, void* mean, void* var, float* cummean, float* cumrstd,
-                         void* workspace, void* stream) {
+                         void* workspace, void* stream, bool plus_one = false, bool shared_prior = false) {
   MEGA_CHECK_ARG(valid_dtype(dtype), "mega_group_timestep_norm_fwd: bad dtype %d", dtype);
   int rc = check_dims("mega_group_timestep_norm_fwd", B, L, D, G);
   if (rc != MEGA_OK) return rc;
@@ -1275,6 +1301,7 @@ static int tsn_fwd_entry(bool time_last, const void* x, int dtype, const int64_t
   p.var = var; p.cummean = cummean; p.cumrstd = cumrstd;
   p.B = (int)B; p.L = (int)L; p.D = (int)D; p.G = (int)G; p.Dg = (int)(D / G);
   p.NT = (int)((L + kTL - 1) / kTL); p.eps = (float)eps;
+  p.prev_row = shared_prior ? 0 : p.G; p.prior_row = shared_prior ? 0 : 1; p.gamma_plus = plus_one ? 1.f : 0.f;
   set_stat_strides(p, time_last);
   hipStream_t s = static_cast<hipStream_t>(stream);
   MEGA_CHECK_ARG(L >= 1, "mega_group_timestep_norm_fwd: empty sequence");
@@ -1311,11 +1338,12 @@ static int tsn_bwd_entry(bool time_last, const void* dy, const void* dmean, cons
                          int dtype, const void* prev_mean, const int64_t* count, const float* cummean,
                          const float* cumrstd, const void* gamma, const uint8_t* padding_mask, int64_t B,
                          int64_t L, int64_t D, int64_t G, void* dx, void* dprev_mean, void* dprev_var,
-                         void* dgamma, void* dbeta, void* workspace, void* stream) {
+                         void* dgamma, void* dbeta, void* workspace, void* stream, bool plus_one = false,
+                         bool shared_prior = false) {
   MEGA_CHECK_ARG(valid_dtype(dtype), "mega_group_timestep_norm_bwd: bad dtype %d", dtype);
   int rc = check_dims("mega_group_timestep_norm_bwd", B, L, D, G);
   if (rc != MEGA_OK) return rc;
-  MEGA_CHECK_ARG(dy && dmean && dvar && x && prev_mean && count && cummean && cumrstd && gamma &&
+  MEGA_CHECK_ARG(dy && (plus_one || (dmean && dvar)) && x && prev_mean && count && cummean && cumrstd && gamma &&
                      dx && dprev_mean && dprev_var && dgamma && dbeta && workspace,
                  "mega_group_timestep_norm_bwd: null pointer");
   MEGA_CHECK_ARG(B >= 1 && L >= 1, "mega_group_timestep_norm_bwd: empty input");
@@ -1325,6 +1353,7 @@ static int tsn_bwd_entry(bool time_last, const void* dy, const void* dmean, cons
   p.cumrstd_in = cumrstd; p.y = dx; p.mean = dprev_mean; p.var = dprev_var;
   p.B = (int)B; p.L = (int)L; p.D = (int)D; p.G = (int)G; p.Dg = (int)(D / G);
   p.NT = (int)((L + kTL - 1) / kTL);
+  p.prev_row = shared_prior ? 0 : p.G; p.prior_row = 1; p.gamma_plus = plus_one ? 1.f : 0.f;
   set_stat_strides(p, time_last);
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (dtype) {
@@ -1356,6 +1385,26 @@ extern "C" int mega_group_timestep_norm_bwd_tl(const void* dy, const void* dmean
                                                void* workspace, void* stream) {
   return tsn_bwd_entry(true, dy, dmean, dvar, x, dtype, prev_mean, count, cummean, cumrstd, gamma, padding_mask,
                        B, L, D, G, dx, dprev_mean, dprev_var, dgamma, dbeta, workspace, stream);
+}
+
+extern "C" int mega_timestep_norm_layer_fwd(const void* x, int dtype, const int64_t* prev_count, const void* prev_mean,
+                                            const void* prev_var, int shared_prior, const void* weight,
+                                            const void* bias, const uint8_t* padding_mask, int64_t B, int64_t L,
+                                            int64_t D, int64_t G, double eps, void* y, int64_t* count, void* mean,
+                                            void* var, float* cummean, float* cumrstd, void* workspace,
+                                            void* stream) {
+  return tsn_fwd_entry(true, x, dtype, prev_count, prev_mean, prev_var, weight, bias, padding_mask, B, L, D, G, eps, y,
+                       count, mean, var, cummean, cumrstd, workspace, stream, true, shared_prior != 0);
+}
+
+extern "C" int mega_timestep_norm_layer_bwd(const void* dy, const void* dmean, const void* dvar, const void* x,
+                                            int dtype, const void* prev_mean, int shared_prior, const int64_t* count,
+                                            const float* cummean, const float* cumrstd, const void* weight,
+                                            const uint8_t* padding_mask, int64_t B, int64_t L, int64_t D, int64_t G,
+                                            void* dx, void* dprev_mean, void* dprev_var, void* dweight, void* dbias,
+                                            void* workspace, void* stream) {
+  return tsn_bwd_entry(true, dy, dmean, dvar, x, dtype, prev_mean, count, cummean, cumrstd, weight, padding_mask, B, L,
+                       D, G, dx, dprev_mean, dprev_var, dweight, dbias, workspace, stream, true, shared_prior != 0);
 }
 
 // Test hook: look-back poll limit (<= 0 restores the default) and a tile index

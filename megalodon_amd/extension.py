@@ -833,7 +833,8 @@ def timestep_norm_status(device=None) -> None:
             ws = _tsn_ws_cache.get((idx, stream, backward))
             if ws is not None:
                 _lib.call("mega_group_timestep_norm_status", _lib.ptr(ws), _lib.stream_ptr(dev))
-
+        for ws in _lib.host().tsn_last_workspaces(idx, stream):  # the layer's calls
+            _lib.call("mega_group_timestep_norm_status", _lib.ptr(ws), _lib.stream_ptr(dev))
 
 
 def _mask_bytes(padding_mask):

@@ -3,11 +3,11 @@
 `megalodon.distributed` look-ups: model-parallel world size is 1, so
 ``dim_per_partition == embed_dim`` and the theta permutation is drawn locally
 instead of being broadcast (:21-26).  On the GPU the layer runs as a chunked
-recurrence (fused_ops/cema_scan.py) wherever its kernels take the case --
-rows of a length that is a multiple of 8, at most 32 modes, with or without
-gradients, carried state and last state; MEGA_CEMA_FFT=1 in the environment
-keeps everything on the kernel-row + FFT-convolution operators that the
-remaining cases (other lengths) use."""
+recurrence (csrc/host/ops.cpp, fused_ops/cema_scan.py) wherever its kernels take
+the case -- at most 32 modes; 16-bit rows of any length and float32 rows of a
+length that is a multiple of 8; with or without gradients, carried state and
+last state; MEGA_CEMA_FFT=1 in the environment keeps everything on the
+kernel-row + FFT-convolution operators that the remaining cases use."""
 from typing import Optional, Tuple
 import math
 import os
@@ -15,6 +15,7 @@ import os
 import torch
 from torch import nn
 
+from .. import _lib
 from .. import extension as megalodon_ops
 from ..fused_ops import (cema_kernel, cema_scan, cema_scan_applicable, cema_scan_state, ema_hidden, ema_parameters,
                          fftconv_residual)
@@ -105,25 +106,33 @@ class MultiHeadComplexEMA(nn.Module):
             self._coeffs = None
             self._coeffs_kernel = None
         stateless = hx is None and not compute_last_state
-        needs_grad = torch.is_grad_enabled() and (x.requires_grad or any(t.requires_grad for t in self.parameters())
-                                                  or (hx is not None and hx.requires_grad))
         if self.alpha.is_cuda and os.environ.get("MEGA_CEMA_FFT") is None:
             # the layer as a chunked recurrence on the matrix cores (no kernel row, no
-            # transform, any length in one launch): bfloat16 / float16 rows with or without
-            # gradients, float32 rows and carried states where no gradient is wanted
-            if stateless and cema_scan_applicable(x, self.ndim, needs_grad):
+            # transform, any length in one launch)
+            if stateless:
+                out = _lib.host().cema(x, self.alpha, self.delta, self.theta, self.gamma, self.omega)
+                if out is not None:
+                    return out, None
+            needs_grad = torch.is_grad_enabled() and (
+                x.requires_grad or any(t.requires_grad for t in self.parameters())
+                or (hx is not None and hx.requires_grad))
+            if stateless and cema_scan_applicable(x, self.ndim, needs_grad):  # more than 16 modes, mixed parameter types
                 out = cema_scan(x, self.alpha.float(), self.delta.float(), self.theta.float(), self.gamma.float(),
                                 self.omega)
                 return out, None
+            if not stateless and not needs_grad:
+                # log q from the coefficient kernel, the one the stateless branch uses: a prefill
+                # and its carried continuation see the same decay rates
+                p, log_q, gamma = self._kernel_coeffs()
+                out = _lib.host().cema_state(x, p, log_q, gamma, self.omega, hx, compute_last_state)
+                if out is not None:
+                    return out
+                if cema_scan_applicable(x, self.ndim, False):
+                    return megalodon_ops.cema_scan_fwd(x, p, log_q, gamma, self.omega, hx, compute_last_state)
             if not stateless and needs_grad and cema_scan_applicable(x, self.ndim, True):
                 # carried state in, last state out, all differentiable (dh0 included)
                 return cema_scan_state(x, self.alpha.float(), self.delta.float(), self.theta.float(),
                                        self.gamma.float(), self.omega, hx, compute_last_state)
-            if not stateless and not needs_grad and cema_scan_applicable(x, self.ndim, False):
-                # log q from the coefficient kernel, the one the stateless branch uses: a prefill
-                # and its carried continuation see the same decay rates
-                p, log_q, gamma = self._kernel_coeffs()
-                return megalodon_ops.cema_scan_fwd(x, p, log_q, gamma, self.omega, hx, compute_last_state)
         if stateless and self.alpha.is_cuda:
             # no carried state: coefficients and kernel as one autograd node
             # (two launches per direction instead of the coefficient graph)
