@@ -688,6 +688,21 @@ int mega_split_bf16(const void* src, int dtype, int64_t n, void* hi, void* lo, v
 int mega_bench_stream_copy(const void* a, const void* b, void* out, int64_t bytes,
                            int workgroups, int nontemporal, void* stream);
 
+/* mega_attention_fwd / _bwd for a caller that hands the probabilities from the forward to the backward and
+ * nowhere else: their layout is the library's own, `saved` holds mega_attention_layer_saved_elements
+ * elements of the tensors' type (the backward's workspace as many again), and lengths off the kernels' slabs
+ * run on the same kernels as whole ones.  There 16-bit operands must be 16-byte aligned and
+ * scale positive. */
+int64_t mega_attention_layer_saved_elements(int dtype, int64_t B, int64_t L1, int64_t L2, int64_t NH,
+                                            int64_t H1, int64_t H2);
+int mega_attention_layer_fwd(const void* q, const void* k, const void* v, int dtype, int64_t B,
+                             int64_t L1, int64_t L2, int64_t NH, int64_t H1, int64_t H2,
+                             double scale, int causal, void* y, void* saved, void* stream);
+int mega_attention_layer_bwd(const void* dy, const void* q, const void* k, const void* v,
+                             const void* saved, int dtype, int64_t B, int64_t L1, int64_t L2,
+                             int64_t NH, int64_t H1, int64_t H2, double scale, int causal,
+                             void* dq, void* dk, void* dv, void* workspace, void* stream);
+
 /* mega_cema_coeffs_fwd / _bwd on parameters of element type `dtype` (as a layer cast to bfloat16 holds
  * them), the gradients in that type too; arithmetic float32.  The incoming gradients are `sets` stacks
  * (sets, D, N), added up here -- one per sequence, as the recurrence's backward leaves them;

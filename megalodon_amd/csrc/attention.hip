@@ -42,7 +42,8 @@ template <typename T>
 int softmax_wide_bwd(const T* y, T* dy, int64_t Z, int64_t L1, int64_t L2, int causal, hipStream_t s);
 // scores + softmax in one kernel (attention_scores.hip); -1: shape outside that kernel
 int attention_probs_fused(int dtype, const uint16_t* q, const uint16_t* k, uint16_t* w, int64_t B, int64_t L1,
-                          int64_t L2, int64_t NH, int64_t H1, float scale, int causal, int fill, hipStream_t s);
+                          int64_t L2, int64_t NH, int64_t H1, float scale, int causal, int fill, int64_t pitch,
+                          int64_t zrows, hipStream_t s);
 
 namespace {
 
@@ -113,6 +114,9 @@ struct GemmParams {
   int per_batch;           // work items per batch index
   int items;               // per_batch * batch
   int ta, tb;   // operand is k-major: element (m, k) at [k * ld + m]
+  int kvb;      // rows of k that a k-major B holds when K has been rounded up behind them (0: all K); A holds
+                // zeros there, so those rows of B may hold anything and the last real one stands in for them
+  int ms;       // rows of C to store when M has been rounded up (0: all M)
   int n_group;  // plain schedule: tiles numbered n fastest inside bands of n_group column tiles, then m,
                 // then band (0: one band) -- the 32 tiles an XCD works on at a time then share fewer
                 // distinct operand blocks (4 x 8 instead of 2 x 16 of a 16-column problem)
@@ -438,7 +442,8 @@ __device__ __forceinline__ void load_to_lds16(const void* base, uint32_t offset,
   asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_dst));
 }
 
-template <int DT, bool TA, bool TB>
+// RAG: p.kvb and p.ms are set (two k-major operands)
+template <int DT, bool TA, bool TB, bool RAG = false>
 __global__ __launch_bounds__(2 * kThreads) void gemm_dma_kernel(const GemmParams p) {
   extern __shared__ __align__(16) uint16_t smem[];
   constexpr int JN = 2, NL = 2, EP = 64 + 8;
@@ -513,14 +518,16 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_kernel(const GemmParams
   // of piece pc fetches what belongs at position l of the piece (addresses clamped into
   // the matrix, so every lane always loads)
   uint32_t offa[NL], offb[NL];
+  int rowb[NL];  // RAG: offb is the column part, the row is clamped per request
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
     const int pc = wave + 8 * i;
     const int krow = 2 * pc + (lane >> 5), cm = (lane & 31) ^ ((krow & 3) << 2);  // k-major piece
+    rowb[i] = kb + krow;
     const int row = 16 * pc + (lane >> 2), ck = (lane & 3) ^ ((lane >> 4) & 3);   // k-contiguous piece
     if (TA) offa[i] = static_cast<uint32_t>(((kb + krow) * p.lda + min(m0 + cm * 8, p.M - 8)) * 2);
     else offa[i] = static_cast<uint32_t>((static_cast<int64_t>(min(m0 + row, p.M - 1)) * p.lda + kb + ck * 8) * 2);
-    if (TB) offb[i] = static_cast<uint32_t>(((kb + krow) * p.ldb + min(n0 + cm * 8, p.N - 8)) * 2);
+    if (TB) offb[i] = static_cast<uint32_t>(((RAG ? 0 : kb + krow) * p.ldb + min(n0 + cm * 8, p.N - 8)) * 2);
     else offb[i] = static_cast<uint32_t>((static_cast<int64_t>(min(n0 + row, p.N - 1)) * p.ldb + kb + ck * 8) * 2);
   }
   const uint32_t stepa = static_cast<uint32_t>((TA ? p.lda : 1) * kSlab * 2);
@@ -531,8 +538,17 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_kernel(const GemmParams
   auto request_one = [&](int s, int stage, int n) {
     const uint32_t sc = static_cast<uint32_t>(min(s, nslab - 1));
     const uint32_t dst = lds_wave + static_cast<uint32_t>(stage * kDmaStage + (n >> 1) * 8 * 512 + (n & 1) * kDmaOperand) * 2;
-    if (n & 1) load_to_lds16(B, offb[n >> 1] + sc * stepb, dst);
-    else load_to_lds16(A, offa[n >> 1] + sc * stepa, dst);
+    if (n & 1) {
+      if constexpr (RAG) {
+        static_assert(TB, "rows of k");
+        const uint32_t row = static_cast<uint32_t>(min(rowb[n >> 1] + static_cast<int>(sc) * kSlab, p.kvb - 1));
+        load_to_lds16(B, offb[n >> 1] + row * static_cast<uint32_t>(p.ldb * 2), dst);
+      } else {
+        load_to_lds16(B, offb[n >> 1] + sc * stepb, dst);
+      }
+    } else {
+      load_to_lds16(A, offa[n >> 1] + sc * stepa, dst);
+    }
   };
   auto request = [&](int s, int stage) {
 #pragma unroll
@@ -672,7 +688,7 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_kernel(const GemmParams
     const int c = lane + kWave * i;
     const int row = c / (4 * JN), kc = (c % (4 * JN)) * 8;
     const int grow = m0 + wm * 128 + row, gcol = n0 + wn * (32 * JN) + kc;
-    if (grow < p.M && gcol < p.N) {
+    if (grow < (RAG ? p.ms : p.M) && gcol < p.N) {
       const u32x4 v = *reinterpret_cast<const u32x4*>(stage + row * EP + kc);
       uint16_t* dst = C + static_cast<int64_t>(grow) * p.ldc + gcol;
       if (vec_ok && gcol + 8 <= p.N) {
@@ -958,7 +974,8 @@ constexpr int kA64BBase = 3 * kA64Operand;          // the B buffers start behin
 constexpr size_t kA64Lds = sizeof(uint16_t) * (kA64BBase + kStages * kDmaOperand);
 static_assert(kA64Lds <= 160 * 1024 && sizeof(uint16_t) * 8 * 128 * (64 + 8) <= kA64Lds, "fits the LDS, holds the output tiles");
 
-template <int DT>
+// RAG: p.kvb is set
+template <int DT, bool RAG = false>
 __global__ __launch_bounds__(2 * kThreads) void gemm_dma_a64_kernel(const GemmParams p) {
   extern __shared__ __align__(16) uint16_t smem[];
   constexpr int JN = 2, EP = 64 + 8;
@@ -1036,6 +1053,7 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_a64_kernel(const GemmPa
   // 128 bytes each, the chunk at position c of row r holds k chunk c ^ ((r >> 1) & 7)); B: the
   // pieces w, w + 8 (2 rows of k, 512 bytes each).  Addresses are clamped into the matrix.
   uint32_t offa[4], offb[2];
+  int rowb[2];  // RAG: offb is the column part, the row is clamped per request
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int pc = wave + 8 * i;
@@ -1046,7 +1064,8 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_a64_kernel(const GemmPa
   for (int i = 0; i < 2; ++i) {
     const int pc = wave + 8 * i;
     const int krow = 2 * pc + (lane >> 5), cm = (lane & 31) ^ ((krow & 3) << 2);
-    offb[i] = static_cast<uint32_t>(((kb + krow) * p.ldb + min(n0 + cm * 8, p.N - 8)) * 2);
+    rowb[i] = kb + krow;
+    offb[i] = static_cast<uint32_t>(((RAG ? 0 : kb + krow) * p.ldb + min(n0 + cm * 8, p.N - 8)) * 2);
   }
   const uint32_t stepa = static_cast<uint32_t>(kSlab64 * 2);
   const uint32_t stepb = static_cast<uint32_t>(p.ldb * kSlab * 2);
@@ -1060,7 +1079,9 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_a64_kernel(const GemmPa
   };
   auto request_b = [&](int sb, int bb, int n) {
     const uint32_t sc = static_cast<uint32_t>(min(sb, nslab - 1));
-    load_to_lds16(B, offb[n] + sc * stepb, lds_wave + static_cast<uint32_t>(kA64BBase + bb * kDmaOperand + n * 8 * 512) * 2);
+    const uint32_t off = RAG ? offb[n] + static_cast<uint32_t>(min(rowb[n] + static_cast<int>(sc) * kSlab, p.kvb - 1)) * static_cast<uint32_t>(p.ldb * 2)
+                             : offb[n] + sc * stepb;
+    load_to_lds16(B, off, lds_wave + static_cast<uint32_t>(kA64BBase + bb * kDmaOperand + n * 8 * 512) * 2);
   };
 
   // fragment side: as in gemm_dma_kernel, k-step `set` of a 32-k step takes k = 16 g + 8 set + e
@@ -1341,15 +1362,18 @@ __global__ __launch_bounds__(kThreads) void softmax_bwd_kernel(const uint16_t* w
 
 template <int DT, int NCH>
 __global__ __launch_bounds__(kThreads) void softmax_bwd_vec_kernel(const uint16_t* w, uint16_t* dw,
-                                                                  int L1, int L2, int coff, int zfull) {
+                                                                  int L1, int L2, int coff, int zfull,
+                                                                  int zrows, int pitch) {
+  // rows of `pitch` >= L2 elements, zrows >= L1 of them per batch and head: what lies behind the keys and
+  // behind the queries is written as zeros
   const int lane = threadIdx.x % kWave;
   const int r = blockIdx.x * (kThreads / kWave) + threadIdx.x / kWave;
-  if (r >= L1) return;
-  const int64_t o = (static_cast<int64_t>(blockIdx.y) * L1 + r) * L2;
+  if (r >= zrows) return;
+  const int64_t o = (static_cast<int64_t>(blockIdx.y) * zrows + r) * pitch;
   const uint16_t* pw = w + o;
   uint16_t* pd = dw + o;
-  const int n = coff >= 0 ? min(r + 1 + coff, L2) : L2;
-  const int nz = (coff == 0 && !zfull) ? min(L2, (r / kTile + 1) * kTile) : L2;
+  const int n = r >= L1 ? 0 : coff >= 0 ? min(r + 1 + coff, L2) : L2;
+  const int nz = (coff == 0 && !zfull && r < L1) ? min(pitch, (r / kTile + 1) * kTile) : pitch;
   float pv[NCH][8], dv[NCH][8];
   float s = 0.f;
 #pragma unroll
@@ -1382,28 +1406,31 @@ __global__ __launch_bounds__(kThreads) void softmax_bwd_vec_kernel(const uint16_
 
 template <int DT>
 int launch_softmax(const uint16_t* p, uint16_t* x, int64_t Z, int64_t L1, int64_t L2, int causal,
-                   hipStream_t s, int zfull = 0, const DropKey* drop = nullptr) {
+                   hipStream_t s, int zfull = 0, const DropKey* drop = nullptr, int64_t zrows = 0,
+                   int64_t pitch = 0) {
   const int coff = causal ? static_cast<int>(L2 - L1) : -1;
   // p == nullptr: forward over x in place; else backward with probabilities p
   if (Z == 0 || L1 == 0 || L2 == 0) return MEGA_OK;
-  const dim3 grid((unsigned)((L1 + 3) / 4), (unsigned)Z);
-  const bool vec = L2 % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+  if (zrows == 0) zrows = L1, pitch = L2;  // (other layouts: backward, rows of at most 4096, pitch % 8 == 0)
+  const dim3 grid((unsigned)((zrows + 3) / 4), (unsigned)Z);
+  const bool vec = pitch % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(p) % 16 == 0;
   const DropKey dk = drop ? *drop : DropKey{};
 #define MEGA_SOFTMAX(NCH)                                                                        \
   if (p != nullptr)                                                                              \
-    softmax_bwd_vec_kernel<DT, NCH><<<grid, kThreads, 0, s>>>(p, x, (int)L1, (int)L2, coff, zfull); \
+    softmax_bwd_vec_kernel<DT, NCH><<<grid, kThreads, 0, s>>>(p, x, (int)L1, (int)L2, coff, zfull,   \
+                                                              (int)zrows, (int)pitch);             \
   else if (drop)                                                                                 \
     softmax_fwd_vec_kernel<DT, NCH, true><<<grid, kThreads, 0, s>>>(x, (int)L1, (int)L2, coff, zfull, dk); \
   else                                                                                           \
     softmax_fwd_vec_kernel<DT, NCH, false><<<grid, kThreads, 0, s>>>(x, (int)L1, (int)L2, coff, zfull, dk);
-  if (vec && L2 <= 512) {
+  if (vec && pitch <= 512) {
     MEGA_SOFTMAX(1)
-  } else if (vec && L2 <= 1024) {
+  } else if (vec && pitch <= 1024) {
     MEGA_SOFTMAX(2)
-  } else if (vec && L2 <= 2048) {
+  } else if (vec && pitch <= 2048) {
     MEGA_SOFTMAX(4)
-  } else if (vec && L2 <= 4096) {
+  } else if (vec && pitch <= 4096) {
     MEGA_SOFTMAX(8)
   } else if (p != nullptr) {
     softmax_bwd_kernel<DT><<<grid, kThreads, 0, s>>>(p, x, (int)L1, (int)L2, coff, zfull);
@@ -1428,7 +1455,9 @@ int launch_gemm_t(const GemmParams& p, int batch, hipStream_t s) {
                       (TB ? (p.N % 8 == 0 && p.N >= 8 && p.K * p.ldb < lim) : p.N * p.ldb < lim);
   const bool fast = fast_a && fast_b && p.K % kSlab == 0 && p.K >= kSlab;
   GemmParams q = p;
-  q.mt_count = (p.M + kTile - 1) / kTile;
+  if (!fast && p.kvb) q.K = p.kvb;  // the bounds-checked kernel takes the real sizes
+  if (!fast && p.ms) q.M = p.ms;
+  q.mt_count = (q.M + kTile - 1) / kTile;
   q.nt_count = (p.N + kTile - 1) / kTile;
   int64_t per_batch;
   if (p.tri_out) {
@@ -1467,10 +1496,23 @@ int launch_gemm_t(const GemmParams& p, int batch, hipStream_t s) {
     }
   }
   if constexpr (!TA && TB) {
-    if (fast && p.K % kSlab64 == 0) {
+    if (fast && p.K % kSlab64 == 0 && p.kvb) {
+      MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dma_a64_kernel<DT, true>),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)kA64Lds));
+      gemm_dma_a64_kernel<DT, true><<<grid, 2 * kThreads, kA64Lds, s>>>(q);
+      done = true;
+    } else if (fast && p.K % kSlab64 == 0) {
       MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dma_a64_kernel<DT>),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kA64Lds));
       gemm_dma_a64_kernel<DT><<<grid, 2 * kThreads, kA64Lds, s>>>(q);
+      done = true;
+    }
+  }
+  if constexpr (TA && TB) {
+    if (fast && p.kvb) {
+      MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dma_kernel<DT, TA, TB, true>),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDmaLds));
+      gemm_dma_kernel<DT, TA, TB, true><<<grid, 2 * kThreads, kDmaLds, s>>>(q);
       done = true;
     }
   }
@@ -1494,16 +1536,6 @@ int launch_gemm(const GemmParams& p, int batch, hipStream_t s) {
   return p.tb ? launch_gemm_t<DT, false, true>(p, batch, s) : launch_gemm_t<DT, false, false>(p, batch, s);
 }
 
-struct AttnWs {
-  int64_t dp, total;  // element offset of dP / dS, total bytes
-};
-AttnWs attn_ws(int64_t B, int64_t L1, int64_t L2, int64_t NH, int64_t H1, int64_t H2, bool bwd) {
-  AttnWs w;
-  w.dp = 0;
-  w.total = ((bwd ? B * NH * L1 * L2 : 0) + 8) * 2;
-  return w;
-}
-
 int check_attn(const char* who, int dtype, int64_t B, int64_t L1, int64_t L2, int64_t NH,
                int64_t H1, int64_t H2, int causal) {
   MEGA_CHECK_ARG(valid_dtype(dtype) || dtype == MEGA_F64, "%s: unknown dtype %d", who, dtype);
@@ -1516,15 +1548,31 @@ int check_attn(const char* who, int dtype, int64_t B, int64_t L1, int64_t L2, in
   return MEGA_OK;
 }
 
+// Layout of the probabilities and of dP: rows of `pitch` elements, `zrows` of them per (batch, head).
+struct PLayout {
+  int64_t zrows, pitch;
+};
+// What the layer's own calls use, where nobody else sees the probabilities: with L1 and L2 rounded up to
+// whole slabs (zeros behind the real rows and columns) every product runs on the kernels that send
+// slabs from memory straight into LDS; with rows of, say, 1021 elements none of the five could
+// (the bounds-checked kernel: 240 instead of 60 us for a 4 x 2 x 1021 x 1021 by 2048 product).
+PLayout layer_layout(int dtype, int64_t L1, int64_t L2, int64_t H1, int64_t H2) {
+  if (dtype != MEGA_BF16 && dtype != MEGA_F16) return {L1, L2};
+  if ((L1 % kSlab == 0 && L2 % kSlab64 == 0) || (H1 != 64 && H1 != 128 && H1 != 256) || H2 % 8 != 0) return {L1, L2};
+  const PLayout l{(L1 + kSlab - 1) / kSlab * kSlab, (L2 + kSlab64 - 1) / kSlab64 * kSlab64};
+  return l.pitch <= 4096 ? l : PLayout{L1, L2};  // the softmax backward holds a row in registers
+}
+
 template <int DT>
 int attn_fwd_impl(const uint16_t* q, const uint16_t* k, const uint16_t* v, int64_t B, int64_t L1,
                   int64_t L2, int64_t NH, int64_t H1, int64_t H2, float scale, int causal,
-                  uint16_t* y, uint16_t* w, uint16_t* ws, hipStream_t s, const DropKey* drop, int fill) {
-  (void)ws;
+                  uint16_t* y, uint16_t* w, hipStream_t s, const DropKey* drop, int fill, PLayout l) {
+  const bool rag = l.zrows != L1 || l.pitch != L2;
   const int Z = static_cast<int>(B * NH);
-  int rc = drop ? -1 : attention_probs_fused(DT, q, k, w, B, L1, L2, NH, H1, scale, causal, fill, s);
+  int rc = drop ? -1 : attention_probs_fused(DT, q, k, w, B, L1, L2, NH, H1, scale, causal, fill, l.pitch, l.zrows, s);
   if (rc > 0) return rc;
   if (rc < 0) {
+  MEGA_CHECK_ARG(!rag, "attention: operands must be 16-byte aligned and scale positive for lengths off the slab");
   // S = scale Q K^T  -> w
   GemmParams g{};
   g.A = q; g.B = k; g.C = w; g.M = (int)L1; g.N = (int)L2; g.K = (int)H1;
@@ -1538,9 +1586,9 @@ int attn_fwd_impl(const uint16_t* q, const uint16_t* k, const uint16_t* v, int64
   }
   // Y = P V: V[key][c] is the k-major B operand
   GemmParams o{};
-  o.A = w; o.B = v; o.C = y; o.M = (int)L1; o.N = (int)H2; o.K = (int)L2;
-  o.lda = L2; o.ldb = NH * H2; o.ldc = NH * H2; o.tb = 1;
-  o.sa0 = NH * L1 * L2; o.sa1 = L1 * L2; o.sb0 = L2 * NH * H2; o.sb1 = H2;
+  o.A = w; o.B = v; o.C = y; o.M = (int)L1; o.N = (int)H2; o.K = (int)l.pitch; o.kvb = rag ? (int)L2 : 0;
+  o.lda = l.pitch; o.ldb = NH * H2; o.ldc = NH * H2; o.tb = 1;
+  o.sa0 = NH * l.zrows * l.pitch; o.sa1 = l.zrows * l.pitch; o.sb0 = L2 * NH * H2; o.sb1 = H2;
   o.sc0 = L1 * NH * H2; o.sc1 = H2; o.nh = (int)NH; o.alpha = 1.f;
   o.tri_out = 0; o.k_mode = causal ? 1 : 0; o.off = causal ? (int)(L2 - L1) : 0;
   return launch_gemm<DT>(o, Z, s);
@@ -1550,40 +1598,40 @@ template <int DT>
 int attn_bwd_impl(const uint16_t* dy, const uint16_t* q, const uint16_t* k, const uint16_t* v,
                   const uint16_t* w, int64_t B, int64_t L1, int64_t L2, int64_t NH, int64_t H1,
                   int64_t H2, float scale, int causal, uint16_t* dq, uint16_t* dk, uint16_t* dv,
-                  uint16_t* ws, hipStream_t s) {
-  const AttnWs l = attn_ws(B, L1, L2, NH, H1, H2, true);
+                  uint16_t* dp, hipStream_t s, PLayout l) {
   const int Z = static_cast<int>(B * NH);
-  uint16_t* dp = ws + l.dp;
+  const bool rag = l.zrows != L1 || l.pitch != L2;
+  const int64_t sz0 = NH * l.zrows * l.pitch, sz1 = l.zrows * l.pitch;
   int rc;
   // dP = dY V^T
   GemmParams g{};
   g.A = dy; g.B = v; g.C = dp; g.M = (int)L1; g.N = (int)L2; g.K = (int)H2;
-  g.lda = NH * H2; g.ldb = NH * H2; g.ldc = L2;
+  g.lda = NH * H2; g.ldb = NH * H2; g.ldc = l.pitch;
   g.sa0 = L1 * NH * H2; g.sa1 = H2; g.sb0 = L2 * NH * H2; g.sb1 = H2;
-  g.sc0 = NH * L1 * L2; g.sc1 = L1 * L2; g.nh = (int)NH; g.alpha = 1.f;
+  g.sc0 = sz0; g.sc1 = sz1; g.nh = (int)NH; g.alpha = 1.f;
   g.tri_out = causal; g.k_mode = 0; g.off = causal ? (int)(L2 - L1) : 0;
   if ((rc = launch_gemm<DT>(g, Z, s)) != MEGA_OK) return rc;
   // dS = P o (dP - rowsum(P o dP)) in place
-  if ((rc = launch_softmax<DT>(w, dp, Z, L1, L2, causal, s)) != MEGA_OK) return rc;
+  if ((rc = launch_softmax<DT>(w, dp, Z, L1, L2, causal, s, 0, nullptr, l.zrows, l.pitch)) != MEGA_OK) return rc;
   // dQ = scale dS K: K[key][h] is the k-major B operand
   GemmParams a{};
-  a.A = dp; a.B = k; a.C = dq; a.M = (int)L1; a.N = (int)H1; a.K = (int)L2;
-  a.lda = L2; a.ldb = NH * H1; a.ldc = NH * H1; a.tb = 1;
-  a.sa0 = NH * L1 * L2; a.sa1 = L1 * L2; a.sb0 = L2 * NH * H1; a.sb1 = H1;
+  a.A = dp; a.B = k; a.C = dq; a.M = (int)L1; a.N = (int)H1; a.K = (int)l.pitch;
+  a.kvb = rag ? (int)L2 : 0; a.lda = l.pitch; a.ldb = NH * H1; a.ldc = NH * H1; a.tb = 1;
+  a.sa0 = sz0; a.sa1 = sz1; a.sb0 = L2 * NH * H1; a.sb1 = H1;
   a.sc0 = L1 * NH * H1; a.sc1 = H1; a.nh = (int)NH; a.alpha = scale; a.k_mode = causal ? 1 : 0; a.off = causal ? (int)(L2 - L1) : 0;
   if ((rc = launch_gemm<DT>(a, Z, s)) != MEGA_OK) return rc;
   // dK = scale dS^T Q: dS[q][key] and Q[q][h] are both k-major (k = q)
   GemmParams b{};
-  b.A = dp; b.B = q; b.C = dk; b.M = (int)L2; b.N = (int)H1; b.K = (int)L1;
-  b.lda = L2; b.ldb = NH * H1; b.ldc = NH * H1; b.ta = 1; b.tb = 1;
-  b.sa0 = NH * L1 * L2; b.sa1 = L1 * L2; b.sb0 = L1 * NH * H1; b.sb1 = H1;
+  b.A = dp; b.B = q; b.C = dk; b.M = (int)l.pitch; b.N = (int)H1; b.K = (int)l.zrows;
+  b.kvb = rag ? (int)L1 : 0; b.ms = rag ? (int)L2 : 0; b.lda = l.pitch; b.ldb = NH * H1; b.ldc = NH * H1; b.ta = 1; b.tb = 1;
+  b.sa0 = sz0; b.sa1 = sz1; b.sb0 = L1 * NH * H1; b.sb1 = H1;
   b.sc0 = L2 * NH * H1; b.sc1 = H1; b.nh = (int)NH; b.alpha = scale; b.k_mode = causal ? 2 : 0; b.off = causal ? (int)(L2 - L1) : 0;
   if ((rc = launch_gemm<DT>(b, Z, s)) != MEGA_OK) return rc;
   // dV = P^T dY: P[q][key] and dY[q][c] are both k-major (k = q)
   GemmParams c{};
-  c.A = w; c.B = dy; c.C = dv; c.M = (int)L2; c.N = (int)H2; c.K = (int)L1;
-  c.lda = L2; c.ldb = NH * H2; c.ldc = NH * H2; c.ta = 1; c.tb = 1;
-  c.sa0 = NH * L1 * L2; c.sa1 = L1 * L2; c.sb0 = L1 * NH * H2; c.sb1 = H2;
+  c.A = w; c.B = dy; c.C = dv; c.M = (int)l.pitch; c.N = (int)H2; c.K = (int)l.zrows;
+  c.kvb = rag ? (int)L1 : 0; c.ms = rag ? (int)L2 : 0; c.lda = l.pitch; c.ldb = NH * H2; c.ldc = NH * H2; c.ta = 1; c.tb = 1;
+  c.sa0 = sz0; c.sa1 = sz1; c.sb0 = L1 * NH * H2; c.sb1 = H2;
   c.sc0 = L2 * NH * H2; c.sc1 = H2; c.nh = (int)NH; c.alpha = 1.f; c.k_mode = causal ? 2 : 0; c.off = causal ? (int)(L2 - L1) : 0;
   return launch_gemm<DT>(c, Z, s);
 }
@@ -1596,7 +1644,7 @@ using namespace mega;
 extern "C" int64_t mega_attention_workspace_bytes(int64_t B, int64_t L1, int64_t L2, int64_t NH,
                                                   int64_t H1, int64_t H2, int backward) {
   if (B < 0 || L1 < 0 || L2 < 0 || NH < 1 || H1 < 1 || H2 < 1) return 16;
-  return attn_ws(B, L1, L2, NH, H1, H2, backward != 0).total;
+  return ((backward ? B * NH * L1 * L2 : 0) + 8) * 2;  // dP
 }
 
 // p in [0, 1]; p == 0 means no DropKey
@@ -1615,12 +1663,13 @@ static int make_dropkey(const char* who, double dropout, uint64_t seed, uint64_t
 static int attention_fwd_entry(const char* who, const void* q, const void* k, const void* v, int dtype,
                                int64_t B, int64_t L1, int64_t L2, int64_t NH, int64_t H1, int64_t H2,
                                double scale, int causal, const DropKey* drop, void* y, void* w,
-                               void* workspace, void* stream) {
+                               void* stream, bool layer = false) {
   int rc = check_attn(who, dtype, B, L1, L2, NH, H1, H2, causal);
   if (rc != MEGA_OK) return rc;
   if (B == 0 || L1 == 0) return MEGA_OK;
-  MEGA_CHECK_ARG(q && k && v && y && w && workspace, "%s: null pointer", who);
+  MEGA_CHECK_ARG(q && k && v && y && w, "%s: null pointer", who);
   MEGA_CHECK_ARG(L2 >= 1, "%s: no keys", who);
+  const PLayout l = layer ? layer_layout(dtype, L1, L2, H1, H2) : PLayout{L1, L2};
   hipStream_t s = static_cast<hipStream_t>(stream);
   // causal == 2: as 1, but w need only hold what mega_attention_bwd reads
   const int fill = causal == 2 ? 0 : 1;
@@ -1637,17 +1686,18 @@ static int attention_fwd_entry(const char* who, const void* q, const void* k, co
   auto m = [](void* p) { return static_cast<uint16_t*>(p); };
   if (dtype == MEGA_BF16)
     return attn_fwd_impl<MEGA_BF16>(u(q), u(k), u(v), B, L1, L2, NH, H1, H2, (float)scale, causal,
-                                    m(y), m(w), m(workspace), s, drop, fill);
+                                    m(y), m(w), s, drop, fill, l);
   return attn_fwd_impl<MEGA_F16>(u(q), u(k), u(v), B, L1, L2, NH, H1, H2, (float)scale, causal,
-                                 m(y), m(w), m(workspace), s, drop, fill);
+                                 m(y), m(w), s, drop, fill, l);
 }
 
 extern "C" int mega_attention_fwd(const void* q, const void* k, const void* v, int dtype, int64_t B,
                                   int64_t L1, int64_t L2, int64_t NH, int64_t H1, int64_t H2,
                                   double scale, int causal, void* y, void* w, void* workspace,
                                   void* stream) {
+  (void)workspace;
   return attention_fwd_entry("mega_attention_fwd", q, k, v, dtype, B, L1, L2, NH, H1, H2, scale,
-                             causal, nullptr, y, w, workspace, stream);
+                             causal, nullptr, y, w, stream);
 }
 
 extern "C" int mega_attention_dropkey_fwd(const void* q, const void* k, const void* v, int dtype,
@@ -1655,18 +1705,19 @@ extern "C" int mega_attention_dropkey_fwd(const void* q, const void* k, const vo
                                           int64_t H2, double scale, int causal, double dropout,
                                           uint64_t seed, uint64_t offset, void* y, void* w,
                                           void* workspace, void* stream) {
+  (void)workspace;
   DropKey dk;
   int rc = make_dropkey("mega_attention_dropkey_fwd", dropout, seed, offset,
                         B >= 0 && NH >= 0 && L1 >= 0 ? B * NH * L1 : 0, &dk);
   if (rc != MEGA_OK) return rc;
   return attention_fwd_entry("mega_attention_dropkey_fwd", q, k, v, dtype, B, L1, L2, NH, H1, H2,
-                             scale, causal, dropout > 0.0 ? &dk : nullptr, y, w, workspace, stream);
+                             scale, causal, dropout > 0.0 ? &dk : nullptr, y, w, stream);
 }
 
-extern "C" int mega_attention_bwd(const void* dy, const void* q, const void* k, const void* v,
-                                  const void* w, int dtype, int64_t B, int64_t L1, int64_t L2,
-                                  int64_t NH, int64_t H1, int64_t H2, double scale, int causal,
-                                  void* dq, void* dk, void* dv, void* workspace, void* stream) {
+static int attention_bwd_entry(const void* dy, const void* q, const void* k, const void* v,
+                               const void* w, int dtype, int64_t B, int64_t L1, int64_t L2,
+                               int64_t NH, int64_t H1, int64_t H2, double scale, int causal,
+                               void* dq, void* dk, void* dv, void* workspace, void* stream, bool layer) {
   int rc = check_attn("mega_attention_bwd", dtype, B, L1, L2, NH, H1, H2, causal);
   if (rc != MEGA_OK) return rc;
   if (B == 0) return MEGA_OK;
@@ -1687,13 +1738,44 @@ extern "C" int mega_attention_bwd(const void* dy, const void* q, const void* k, 
                                       static_cast<const double*>(w), B, L1, L2, NH, H1, H2, scale, causal,
                                       static_cast<double*>(dq), static_cast<double*>(dk), static_cast<double*>(dv),
                                       static_cast<double*>(workspace), s);
+  const PLayout l = layer ? layer_layout(dtype, L1, L2, H1, H2) : PLayout{L1, L2};
   auto u = [](const void* p) { return static_cast<const uint16_t*>(p); };
   auto m = [](void* p) { return static_cast<uint16_t*>(p); };
   if (dtype == MEGA_BF16)
     return attn_bwd_impl<MEGA_BF16>(u(dy), u(q), u(k), u(v), u(w), B, L1, L2, NH, H1, H2,
-                                    (float)scale, causal, m(dq), m(dk), m(dv), m(workspace), s);
+                                    (float)scale, causal, m(dq), m(dk), m(dv), m(workspace), s, l);
   return attn_bwd_impl<MEGA_F16>(u(dy), u(q), u(k), u(v), u(w), B, L1, L2, NH, H1, H2,
-                                 (float)scale, causal, m(dq), m(dk), m(dv), m(workspace), s);
+                                 (float)scale, causal, m(dq), m(dk), m(dv), m(workspace), s, l);
+}
+
+extern "C" int mega_attention_bwd(const void* dy, const void* q, const void* k, const void* v,
+                                  const void* w, int dtype, int64_t B, int64_t L1, int64_t L2,
+                                  int64_t NH, int64_t H1, int64_t H2, double scale, int causal,
+                                  void* dq, void* dk, void* dv, void* workspace, void* stream) {
+  return attention_bwd_entry(dy, q, k, v, w, dtype, B, L1, L2, NH, H1, H2, scale, causal, dq, dk, dv, workspace, stream,
+                             false);
+}
+
+extern "C" int64_t mega_attention_layer_saved_elements(int dtype, int64_t B, int64_t L1, int64_t L2, int64_t NH,
+                                                       int64_t H1, int64_t H2) {
+  if (B < 0 || L1 < 0 || L2 < 0 || NH < 1 || H1 < 1 || H2 < 1) return 0;
+  const PLayout l = layer_layout(dtype, L1, L2, H1, H2);
+  return B * NH * l.zrows * l.pitch;
+}
+
+extern "C" int mega_attention_layer_fwd(const void* q, const void* k, const void* v, int dtype, int64_t B, int64_t L1,
+                                        int64_t L2, int64_t NH, int64_t H1, int64_t H2, double scale, int causal,
+                                        void* y, void* saved, void* stream) {
+  return attention_fwd_entry("mega_attention_layer_fwd", q, k, v, dtype, B, L1, L2, NH, H1, H2, scale, causal ? 2 : 0,
+                             nullptr, y, saved, stream, true);
+}
+
+extern "C" int mega_attention_layer_bwd(const void* dy, const void* q, const void* k, const void* v, const void* saved,
+                                        int dtype, int64_t B, int64_t L1, int64_t L2, int64_t NH, int64_t H1,
+                                        int64_t H2, double scale, int causal, void* dq, void* dk, void* dv,
+                                        void* workspace, void* stream) {
+  return attention_bwd_entry(dy, q, k, v, saved, dtype, B, L1, L2, NH, H1, H2, scale, causal, dq, dk, dv, workspace,
+                             stream, true);
 }
 
 // ---- the weight gradient of a linear layer on the same product kernel ---------------

@@ -100,6 +100,8 @@ struct ProbsParams {
   int L1, L2, NH, Z, MT;
   int causal, off;
   int fill;  // also write zeros from the last tile to the end of every row
+  int pitch; // elements between rows of w: >= L2, a multiple of 8; columns behind L2 hold zeros
+  int zrows; // rows of w per (batch, head), L1 or more; those behind L1 are written as zeros
   float sl;  // scale * log2(e)
 };
 
@@ -206,7 +208,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_probs_kernel(const ProbsPara
   u32x4 fr[4][2];      // fragment sets: k-step ks of a slab lives in set ks % 4
   float m = -1e30f, l = 0.f;   // this lane's running maximum (raw score) and sum of exp
   float nm = 0.f;              // pass 1: -(block max) * sl; after it: -(max * sl + log2(sum)) of the whole row
-  uint16_t* wrow = p.w + (static_cast<int64_t>(z) * p.L1 + min(row, p.L1 - 1)) * p.L2;
+  uint16_t* wrow = p.w + (static_cast<int64_t>(z) * p.zrows + min(row, p.L1 - 1)) * p.pitch;
   const bool row_ok = row < p.L1;
 
   // The pass over one 32-key block of a finished tile (16 scores per lane, element i = key
@@ -267,7 +269,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_probs_kernel(const ProbsPara
           half_swap(py[2 * u], py[2 * u + 1]);
           const u32x4 o = {px[2 * u], py[2 * u], px[2 * u + 1], py[2 * u + 1]};
           const int col = c0 + x0 + 16 * u + 8 * h;
-          if (!MASK || (row_ok && col < p.L2)) *reinterpret_cast<u32x4*>(wrow + col) = o;
+          if (!MASK || (row_ok && col < p.pitch)) *reinterpret_cast<u32x4*>(wrow + col) = o;
         }
       }
     }
@@ -394,14 +396,22 @@ __global__ __launch_bounds__(64 * kWaves) void attn_probs_kernel(const ProbsPara
   {
     // zeros behind the last tile: to the end of the row with `fill`, else as far as the products that
     // read P in 256-row tiles go (the last key the 256-row block of this row block can see)
-    const int zend = (p.fill || !p.causal) ? p.L2 : min(p.L2, (m0 / 256 + 1) * 256 + p.off);
+    const int zend = (p.fill || !p.causal) ? p.pitch : min(p.pitch, (m0 / 256 + 1) * 256 + p.off);
     const u32x4 zero = {0u, 0u, 0u, 0u};
     if (nb * kKeys < zend) {
       for (int rr = 0; rr < 32 && r0 + rr < p.L1; ++rr) {
-        uint16_t* dst = p.w + (static_cast<int64_t>(z) * p.L1 + r0 + rr) * p.L2;
+        uint16_t* dst = p.w + (static_cast<int64_t>(z) * p.zrows + r0 + rr) * p.pitch;
         // whole lines, not read by this kernel: non-temporal (forward with full rows 1.312 -> 1.291 ms)
         for (int c = nb * kKeys + lane * 8; c < zend; c += 64 * 8) __builtin_nontemporal_store(zero, reinterpret_cast<u32x4*>(dst + c));
       }
+    }
+  }
+  // rows behind the last query (at most to the next multiple of 32: the wave that owns the last rows)
+  if (r0 < p.zrows && r0 + 32 > p.L1) {
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    for (int rr = max(r0, p.L1); rr < min(r0 + 32, p.zrows); ++rr) {
+      uint16_t* dst = p.w + (static_cast<int64_t>(z) * p.zrows + rr) * p.pitch;
+      for (int c = lane * 8; c < p.pitch; c += 64 * 8) *reinterpret_cast<u32x4*>(dst + c) = zero;
     }
   }
   // nothing may land in the LDS of a workgroup that has ended
@@ -422,18 +432,20 @@ int launch_probs(const ProbsParams& p, hipStream_t s) {
 
 }  // namespace
 
-// w = causal softmax of scale q k^T for 16-bit q (B, L1, NH, H1), k (B, L2, NH, H1), w (B, NH, L1, L2).
+// w = causal softmax of scale q k^T for 16-bit q (B, L1, NH, H1), k (B, L2, NH, H1), w (B, NH, zrows, pitch)
+// with zrows in L1 .. L1 rounded up to 32 and pitch >= L2.
 // Returns MEGA_OK, an error, or -1 when the shape is outside this kernel (the caller then runs the
-// product, softmax and zero fill as separate kernels): head widths other than 64, 128, 256, key
-// counts that are not a multiple of 8, operands that are not 16-byte aligned, scale <= 0.
+// product, softmax and zero fill as separate kernels): head widths other than 64, 128, 256, row
+// pitches that are not a multiple of 8, operands that are not 16-byte aligned, scale <= 0.
 // With `causal`, row r is written up to the end of the 64-key tile that holds the last key of the
 // row block (256 rows) it belongs to, with zeros behind its own last key; `fill` writes the zeros
 // up to the end of the row as well (always done when L2 > L1, where the backward products of the
 // operator read them).
 int attention_probs_fused(int dtype, const uint16_t* q, const uint16_t* k, uint16_t* w, int64_t B, int64_t L1,
-                          int64_t L2, int64_t NH, int64_t H1, float scale, int causal, int fill, hipStream_t s) {
+                          int64_t L2, int64_t NH, int64_t H1, float scale, int causal, int fill, int64_t pitch,
+                          int64_t zrows, hipStream_t s) {
   const auto a16 = [](const void* x) { return reinterpret_cast<uintptr_t>(x) % 16 == 0; };
-  if (!(H1 == 64 || H1 == 128 || H1 == 256) || L2 % 8 != 0 || !a16(q) || !a16(k) || !a16(w)) return -1;
+  if (!(H1 == 64 || H1 == 128 || H1 == 256) || pitch % 8 != 0 || !a16(q) || !a16(k) || !a16(w)) return -1;
   if (!(scale > 0.f) || !(scale < 1e30f)) return -1;
   const int64_t MT = (L1 + kRows - 1) / kRows;
   if (L2 * NH * H1 >= (1ll << 30) || B * NH * MT >= (1ll << 31) || L1 < 1 || L2 < 1) return -1;
@@ -442,6 +454,7 @@ int attention_probs_fused(int dtype, const uint16_t* q, const uint16_t* k, uint1
   p.L1 = (int)L1; p.L2 = (int)L2; p.NH = (int)NH; p.Z = (int)(B * NH); p.MT = (int)MT;
   p.causal = causal ? 1 : 0;
   p.off = causal ? (int)(L2 - L1) : 0;
+  p.pitch = (int)pitch; p.zrows = (int)zrows;
   p.fill = (causal && (fill || L2 > L1)) ? 1 : 0;
   p.sl = scale * 1.4426950408889634f;
 #define MEGA_PROBS(DT)                                   \

@@ -407,19 +407,23 @@ AttnDims attn_dims(const Tensor& q, const Tensor& k, const Tensor& v) {
   require(q.scalar_type() == k.scalar_type() && q.scalar_type() == v.scalar_type(), "q, k, v must share one dtype");
   return d;
 }
+// contiguous, on a 16-byte boundary
+Tensor attn_operand(const Tensor& t) {
+  Tensor c = t.contiguous();
+  return reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 == 0 ? c : c.clone(at::MemoryFormat::Contiguous);
+}
 std::tuple<Tensor, Tensor> attention_raw(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bool causal) {
   const AttnDims d = attn_dims(q, k, v);
   const int code = kernel_code(q);
-  Tensor y = at::empty({d.B, d.L1, d.NH, d.H2}, v.options()), w = at::empty({d.B, d.NH, d.L1, d.L2}, v.options());
-  const Tensor ws = bytes(mega_attention_workspace_bytes(d.B, d.L1, d.L2, d.NH, d.H1, d.H2, 0) * (code == MEGA_F32 ? 2 : 1), q);
-  // w goes to the backward and nowhere else: 2 leaves the zeros right of the diagonal block unwritten
-  check(mega_attention_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), code, d.B, d.L1, d.L2, d.NH, d.H1, d.H2, scale, causal ? 2 : 0, y.data_ptr(), w.data_ptr(), ws.data_ptr(), stream_of(q)), "mega_attention_fwd");
-  return {y, w};
+  Tensor y = at::empty({d.B, d.L1, d.NH, d.H2}, v.options());
+  Tensor saved = at::empty({mega_attention_layer_saved_elements(code, d.B, d.L1, d.L2, d.NH, d.H1, d.H2)}, v.options());
+  check(mega_attention_layer_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), code, d.B, d.L1, d.L2, d.NH, d.H1, d.H2, scale, causal, y.data_ptr(), saved.data_ptr(), stream_of(q)), "mega_attention_layer_fwd");
+  return {y, saved};
 }
 struct AttentionFn : Function<AttentionFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, double scale, bool causal) {
     at::AutoDispatchBelowADInplaceOrView below;
-    const Tensor qc = q.contiguous(), kc = k.contiguous(), vc = v.contiguous();
+    const Tensor qc = attn_operand(q), kc = attn_operand(k), vc = attn_operand(v);
     auto [y, w] = attention_raw(qc, kc, vc, scale, causal);
     ctx->save_for_backward({qc, kc, vc, w});
     ctx->saved_data["scale"] = scale;
@@ -432,11 +436,10 @@ struct AttentionFn : Function<AttentionFn> {
     const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &w = saved[3];
     const AttnDims d = attn_dims(q, k, v);
     c10::DeviceGuard guard(q.device());
-    const Tensor dy = g[0].contiguous();
+    const Tensor dy = attn_operand(g[0]);
     Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
-    const int code = kernel_code(q);
-    const Tensor ws = bytes(mega_attention_workspace_bytes(d.B, d.L1, d.L2, d.NH, d.H1, d.H2, 1) * (code == MEGA_F32 ? 2 : 1), q);
-    check(mega_attention_bwd(dy.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), w.data_ptr(), code, d.B, d.L1, d.L2, d.NH, d.H1, d.H2, ctx->saved_data["scale"].toDouble(), ctx->saved_data["causal"].toBool(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), stream_of(q)), "mega_attention_bwd");
+    const Tensor ws = at::empty_like(w);
+    check(mega_attention_layer_bwd(dy.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), w.data_ptr(), kernel_code(q), d.B, d.L1, d.L2, d.NH, d.H1, d.H2, ctx->saved_data["scale"].toDouble(), ctx->saved_data["causal"].toBool(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), stream_of(q)), "mega_attention_layer_bwd");
     return {dq, dk, dv, Tensor(), Tensor()};
   }
 };
@@ -444,7 +447,7 @@ Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, double scale
   attn_dims(q, k, v);
   c10::DeviceGuard guard(q.device());
   if (wants_grad({&q, &k, &v})) return AttentionFn::apply(q, k, v, scale, causal);
-  return std::get<0>(attention_raw(q.contiguous(), k.contiguous(), v.contiguous(), scale, causal));
+  return std::get<0>(attention_raw(attn_operand(q), attn_operand(k), attn_operand(v), scale, causal));
 }
 
 // ---- linear layers --------------------------------------------------------------------------------
