@@ -688,6 +688,16 @@ int mega_split_bf16(const void* src, int dtype, int64_t n, void* hi, void* lo, v
 int mega_bench_stream_copy(const void* a, const void* b, void* out, int64_t bytes,
                            int workgroups, int nontemporal, void* stream);
 
+/* mega_cema_scan_bwd / _wide for a caller that adds the parameter gradients up anyway (the layer): several
+ * rows of a channel share a workgroup and leave one set of gradients.  dp (sets, D, N), dq and dgamma
+ * likewise, domega (sets, D) with sets = mega_cema_layer_scan_sets(B, D, L).  bfloat16 dy and x; dx_mode 0: dx
+ * bfloat16; 1: float32, or not written when NULL; 2: added to float32 dx. */
+int64_t mega_cema_layer_scan_sets(int64_t B, int64_t D, int64_t L);
+int mega_cema_layer_scan_bwd(const void* dy, const void* x, const float* p, const float* log_q,
+                             const float* gamma, const float* omega, int64_t B, int64_t D,
+                             int64_t N, int64_t L, void* dx, int dx_mode, float* dp, float* dq,
+                             float* dgamma, float* domega, void* stream);
+
 /* mega_attention_fwd / _bwd for a caller that hands the probabilities from the forward to the backward and
  * nowhere else: their layout is the library's own, `saved` holds mega_attention_layer_saved_elements
  * elements of the tensors' type (the backward's workspace as many again), and lengths off the kernels' slabs

@@ -20,9 +20,13 @@
 // bf16 is exact, fp16 x is split into two exact bf16 pieces; the states are
 // float32 and split the same way; accumulation is float32.
 //
-// One workgroup of four waves owns a row; a segment of 128 NT chunks is
-// resident at a time: wave w holds chunk tiles NT w .. NT w + NT - 1 of it
-// (NT = 1 is what the entry point launches: 8192 steps per segment).
+// One workgroup of four waves owns a channel's rows: one of them, or, where the batch has several,
+// as many as still leave a workgroup for every slot of the chip.  Setting up the channel's parameter
+// matrices costs as much as half an item, and a row of 2048 steps fills one wave: rows are cut
+// into tiles of 32 chunks (2048 steps), the tiles of a channel's rows stand in one line, and a
+// workgroup takes four of them at a time, a tile per wave; the recurrence starts anew where a tile
+// is the first of its row.  (4 x 2048 rows of 5001 steps, forward and backward: 329 us with a row per
+// workgroup, 241 us so.)
 #include "common.hpp"
 #include "cema_pow.hpp"
 
@@ -207,9 +211,8 @@ __device__ __forceinline__ floatx16 mma_split(const u32x4* a, const u32x4* x, fl
 //   8..11  Q, (row tile it, k-step s2): rows i = 32 it + r, state columns m = 16 s2 + 8 g + e
 constexpr int kFwdBlocks = 12;
 
-template <int NT>
 struct FwdSmem {
-  static constexpr int NC = kWaves * NT * 32;  // chunks per segment
+  static constexpr int NC = kWaves * 32;       // chunks resident
   float klocal[kT];                            // k[0 .. 63] (+ omega at lag 0)
   float pn[16];
   cf gn[16];
@@ -225,55 +228,95 @@ struct FwdSmem {
 };
 static_assert(sizeof(cf) * 16 * (kT + 2) <= sizeof(float) * (kWaves * 32 + 1) * kHP, "the power table fits the state buffer");
 
+// The rows of a launch: groups of `nb` rows of one channel (d = group % D), each a line of tiles.
+struct Lines {
+  int B, D, nb, groups;  // groups = D ceil(B / nb)
+  int tpr;               // tiles per row
+  int64_t L, C;          // steps and chunks of a row
+  __device__ __forceinline__ int first_row(int group) const { return group / D * nb; }
+  __device__ __forceinline__ int tiles(int group) const { return min(nb, B - first_row(group)) * tpr; }
+};
+// A tile of a group's line: which row, where in it.  Stepping from one of a wave's tiles to the
+// next needs no division.
+struct Tile {
+  int64_t row;  // b D + d
+  int t;        // number in the line
+  int chunk0;   // first chunk inside the row
+  int nc;       // chunks of the row in it (0: no such tile)
+};
+__device__ __forceinline__ int tile_chunks(const Lines& ln, const Tile& w, int tiles) {
+  return w.t >= 0 && w.t < tiles ? min(static_cast<int>(ln.C) - w.chunk0, 32) : 0;
+}
+__device__ __forceinline__ Tile tile_at(const Lines& ln, int group, int t) {
+  Tile w;
+  const bool on = group < ln.groups;
+  const int b = t / ln.tpr;
+  w.row = on ? static_cast<int64_t>(ln.first_row(group) + b) * ln.D + group % ln.D : 0;
+  w.t = t;
+  w.chunk0 = (t - b * ln.tpr) * 32;
+  w.nc = on ? tile_chunks(ln, w, ln.tiles(group)) : 0;
+  return w;
+}
+__device__ __forceinline__ void tile_forward(const Lines& ln, Tile& w, int tiles) {
+  w.t += kWaves;
+  w.chunk0 += 32 * kWaves;
+  while (w.chunk0 >= 32 * ln.tpr) {
+    w.chunk0 -= 32 * ln.tpr;
+    w.row += ln.D;
+  }
+  w.nc = tile_chunks(ln, w, tiles);
+}
+__device__ __forceinline__ void tile_backward(const Lines& ln, Tile& w, int tiles) {
+  w.t -= kWaves;
+  w.chunk0 -= 32 * kWaves;
+  while (w.chunk0 < 0) {
+    w.chunk0 += 32 * ln.tpr;
+    w.row -= ln.D;
+  }
+  w.nc = tile_chunks(ln, w, tiles);
+}
+
 // LDS traffic of one wave is processed in order: a wave that has written rows
 // and waits for its own LDS operations can read what its other lanes wrote.
 __device__ __forceinline__ void wave_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-template <int DT, int NT, bool ANY>
-__global__ __launch_bounds__(kThreads, NT == 1 ? 3 : 2) void cema_scan_fwd_kernel(
+template <int DT, bool ANY>
+__global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
     const void* __restrict__ x, void* __restrict__ y, const float* __restrict__ p,
     const cf* __restrict__ log_q, const cf* __restrict__ gamma, const float* __restrict__ omega,
-    const cf* __restrict__ h0, cf* __restrict__ h_last, int64_t rows, int D, int N, int64_t L) {
-  using Smem = FwdSmem<NT>;
+    const cf* __restrict__ h0, cf* __restrict__ h_last, const Lines ln, int N) {
+  using Smem = FwdSmem;
   constexpr int NC = Smem::NC, CPS = NC / kSubs, XP = XOp<DT>::XP;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Smem& sm = *reinterpret_cast<Smem*>(smem_raw);
   cf (*qp)[kT + 2] = reinterpret_cast<cf(*)[kT + 2]>(sm.H);  // while a row is set up
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int64_t L = ln.L, C = ln.C;
   const int g = lane >> 5, r = lane & 31;
   // scan roles: mode sn; sub-segment sa = 4 wave + sl of CPS chunks, inside the wave's own tiles
   const int sn = tid & 15, sa = tid >> 4, sl = sa & 3;
-  const int64_t C = (L + kT - 1) / kT;
 
-  // The workgroup walks (row, segment) items: rows blockIdx.x, + gridDim.x, ...,
-  // the segments of a row in time order.  The x tiles of the next item and the
-  // parameters of the next row are requested ahead (two register sets for the
-  // tiles, swapped by taking the item body twice per loop turn).
-  auto load_tiles = [&](XOp<DT> (&t)[NT][4], int64_t row, int64_t seg0) {
-    const typename Elem<DT>::type* xrow = static_cast<const typename Elem<DT>::type*>(x) + row * L;
+  // The workgroup walks (group, four tiles) items: groups blockIdx.x, + gridDim.x, ..., the tiles
+  // of a group in line.  The x tile of the next item and the parameters of the next group are
+  // requested ahead.
+  auto load_tile = [&](XOp<DT> (&t)[4], const Tile& w) {
+    const typename Elem<DT>::type* xrow = static_cast<const typename Elem<DT>::type*>(x) + w.row * L;
 #pragma unroll
-    for (int ctl = 0; ctl < NT; ++ctl) {
-      const int64_t chunk = seg0 + (wave * NT + ctl) * 32 + r;
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const int64_t elem = chunk * kT + 16 * s + 8 * g;
-        t[ctl][s].template load<ANY>(xrow, elem, row < rows, L);
-      }
-    }
+    for (int s = 0; s < 4; ++s)
+      t[s].template load<ANY>(xrow, static_cast<int64_t>(w.chunk0 + r) * kT + 16 * s + 8 * g, w.nc > 0, L);
   };
   struct RowParams {
-    cf lq, gv, hv;
+    cf lq, gv;
     float pv, w;
   };
-  auto fetch_params = [&](int64_t row) {
-    RowParams rp{cf{0.f, 0.f}, cf{0.f, 0.f}, cf{0.f, 0.f}, 0.f, 0.f};
-    if (row < rows) {
-      const int d = static_cast<int>(row % D);
+  auto fetch_params = [&](int group) {
+    RowParams rp{cf{0.f, 0.f}, cf{0.f, 0.f}, 0.f, 0.f};
+    if (group < ln.groups) {
+      const int d = group % ln.D;
       if (sn < N) {
         rp.lq = log_q[d * N + sn];
         rp.gv = gamma[d * N + sn];
         rp.pv = p[d * N + sn];
-        if (h0 != nullptr && tid < 16) rp.hv = h0[row * N + sn];
       }
       if (omega != nullptr) rp.w = omega[d];
     }
@@ -286,7 +329,7 @@ __global__ __launch_bounds__(kThreads, NT == 1 ? 3 : 2) void cema_scan_fwd_kerne
 
   // tables, operand blocks and scan multipliers of a row's channel, from the
   // parameters fetched ahead; then the next row's parameters are requested
-  auto setup_row = [&](int64_t row) {
+  auto setup_row = [&](int group) {
     // the few powers that are evaluated directly (phase reduced in float64): 12 per mode;
     // everything else is a product of two of them and a short chain of multiplications
     cf direct{0.f, 0.f};
@@ -301,7 +344,6 @@ __global__ __launch_bounds__(kThreads, NT == 1 ? 3 : 2) void cema_scan_fwd_kerne
     if (tid < 16) {
       sm.pn[tid] = rp.pv;
       sm.gn[tid] = rp.gv;
-      sm.carry[0][tid] = rp.hv;
     }
     cur = 0;
     __syncthreads();
@@ -323,7 +365,7 @@ __global__ __launch_bounds__(kThreads, NT == 1 ? 3 : 2) void cema_scan_fwd_kerne
       qS = sm.pw[10][sn];
       qW = sm.pw[11][sn];
     }
-    const RowParams next_rp = fetch_params(row + gridDim.x);
+    const RowParams next_rp = fetch_params(group + static_cast<int>(gridDim.x));
     __syncthreads();
     for (int item = tid; item < kFwdBlocks * kWave; item += kThreads) {
       const int blk = item >> 6, ln = item & 63, rr = ln & 31, gg = ln >> 5;
@@ -369,36 +411,34 @@ __global__ __launch_bounds__(kThreads, NT == 1 ? 3 : 2) void cema_scan_fwd_kerne
     dst[1] = sm.aop[b][1][lane];
   };
 
-  // One (row, segment) item.  The item's x tiles were requested by the previous item (or
-  // the prologue); everything that reads them -- the local states and the K X part of the
-  // outputs -- comes first, then the same registers are reloaded with the next item's tiles
-  // while the scan and the state part of the outputs run.
-  XOp<DT> xb[NT][4];
-  auto item = [&](int64_t row, int64_t seg0) {
-    if (seg0 == 0) setup_row(row);
-    typename Elem<DT>::type* yrow = static_cast<typename Elem<DT>::type*>(y) + row * L;
-    const int nc = static_cast<int>(C - seg0 < NC ? C - seg0 : NC);
-    floatx16 yacc[NT][2];
+  // One item.  Its x tile was requested by the previous item (or the prologue); everything that
+  // reads it -- the local states and the K X part of the outputs -- comes first, then the
+  // same registers are reloaded with the next item's tile while the scan and the state part of
+  // the outputs run.
+  XOp<DT> xb[4];
+  Tile cur_tile = tile_at(ln, blockIdx.x, wave);  // this wave's tile of the item
+  auto item = [&](int group, int t0, int tiles) {
+    if (t0 == 0) setup_row(group);
+    const Tile w = cur_tile;
+    typename Elem<DT>::type* yrow = static_cast<typename Elem<DT>::type*>(y) + w.row * L;
+    const int c0 = wave * 32;
+    floatx16 yacc[2];
     // ---- local states S = P X, into this wave's own rows of the state buffer ----------
     {
       u32x4 P[4][2];
 #pragma unroll
       for (int s = 0; s < 4; ++s) load_block(s, P[s]);
+      if (w.nc > 0) {
+        floatx16 acc;
 #pragma unroll
-      for (int ctl = 0; ctl < NT; ++ctl) {
-        const int c0 = (wave * NT + ctl) * 32;
-        if (c0 < nc) {
-          floatx16 acc;
+        for (int i = 0; i < 16; ++i) acc[i] = 0.f;
 #pragma unroll
-          for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+        for (int s = 0; s < 4; ++s) acc = mma_split<XP>(P[s], xb[s].pc, acc);
+        float* dst = sm.H + (1 + c0 + r) * kHP + 4 * g;
 #pragma unroll
-          for (int s = 0; s < 4; ++s) acc = mma_split<XP>(P[s], xb[ctl][s].pc, acc);
-          float* dst = sm.H + (1 + c0 + r) * kHP + 4 * g;
-#pragma unroll
-          for (int qd = 0; qd < 4; ++qd)
-            *reinterpret_cast<float4*>(dst + 8 * qd) =
-                make_float4(acc[4 * qd], acc[4 * qd + 1], acc[4 * qd + 2], acc[4 * qd + 3]);
-        }
+        for (int qd = 0; qd < 4; ++qd)
+          *reinterpret_cast<float4*>(dst + 8 * qd) =
+              make_float4(acc[4 * qd], acc[4 * qd + 1], acc[4 * qd + 2], acc[4 * qd + 3]);
       }
     }
     // ---- the within-chunk part of the outputs, K X (omega x included: K carries omega on
@@ -408,29 +448,23 @@ __global__ __launch_bounds__(kThreads, NT == 1 ? 3 : 2) void cema_scan_fwd_kerne
 #pragma unroll
       for (int b = 0; b < 4; ++b) load_block(4 + b, K[b]);
 #pragma unroll
-      for (int ctl = 0; ctl < NT; ++ctl)
+      for (int it = 0; it < 2; ++it) {
 #pragma unroll
-        for (int it = 0; it < 2; ++it) {
+        for (int i = 0; i < 16; ++i) yacc[it][i] = 0.f;
+        if (w.nc > 0) {
 #pragma unroll
-          for (int i = 0; i < 16; ++i) yacc[ctl][it][i] = 0.f;
-          if ((wave * NT + ctl) * 32 < nc) {
-#pragma unroll
-            for (int s = 0; s < 2 + 2 * it; ++s)
-              yacc[ctl][it] = mma_split<XP>(K[1 + 2 * it - s], xb[ctl][s].pc, yacc[ctl][it]);
-          }
+          for (int s = 0; s < 2 + 2 * it; ++s) yacc[it] = mma_split<XP>(K[1 + 2 * it - s], xb[s].pc, yacc[it]);
         }
+      }
     }
     {
-      int64_t nrow = row, nseg = seg0 + NC;
-      if (nseg >= C) {
-        nrow = row + gridDim.x;
-        nseg = 0;
-      }
-      load_tiles(xb, nrow, nseg);
+      if (t0 + kWaves < tiles) tile_forward(ln, cur_tile, tiles);
+      else cur_tile = tile_at(ln, group + static_cast<int>(gridDim.x), wave);
+      load_tile(xb, cur_tile);
     }
     wave_sync();
-    // ---- scan over the chunks of the segment: a sub-segment per 16 lanes, the wave's four
-    //      sub-segments are its own chunks; one workgroup barrier hands over the waves' ends -----
+    // ---- scan over the chunks: a sub-segment per 16 lanes, the wave's four sub-segments are its
+    //      own chunks; one workgroup barrier hands over the waves' ends ---------------------------
     {
       float* col = sm.H + kHP + 2 * sn;  // state column n of row 1 + c
       float2 sv[CPS];                    // the sub-segment's local states, kept for the second pass
@@ -438,7 +472,7 @@ __global__ __launch_bounds__(kThreads, NT == 1 ? 3 : 2) void cema_scan_fwd_kerne
       for (int i = 0; i < CPS; ++i) {
         const int c = sa * CPS + i;
         const float2 s0 = *reinterpret_cast<const float2*>(col + c * kHP);  // read, then masked
-        sv[i] = c < nc ? s0 : make_float2(0.f, 0.f);
+        sv[i] = sl * CPS + i < w.nc ? s0 : make_float2(0.f, 0.f);
       }
       cf h{0.f, 0.f};
 #pragma unroll
@@ -453,11 +487,13 @@ __global__ __launch_bounds__(kThreads, NT == 1 ? 3 : 2) void cema_scan_fwd_kerne
       }
       lds_barrier();
       cf cin = sm.carry[cur][sn];
+      // through the tiles in front of this wave's, from the first one of its row if that is among the
+      // four (there the carried state enters)
+      const int k = w.chunk0 / 32, from = k <= wave ? wave - k : 0;
+      if (k <= wave) cin = h0 != nullptr && w.nc > 0 && sn < N ? h0[w.row * N + sn] : cf{0.f, 0.f};
 #pragma unroll
-      for (int w = 0; w < kWaves - 1; ++w) {
-        const cf e = sm.wave_end[par][w][sn];
-        if (w < wave) cin = cadd(cmul(qW, cin), e);
-      }
+      for (int v = 0; v < kWaves - 1; ++v)
+        if (v >= from && v < wave) cin = cadd(cmul(qW, cin), sm.wave_end[par][v][sn]);
       if (sa == kSubs - 1) sm.carry[cur ^ 1][sn] = cadd(cmul(qW, cin), sm.wave_end[par][kWaves - 1][sn]);
       if (sl == 0) *reinterpret_cast<float2*>(sm.wave_cin[wave] + 2 * sn) = make_float2(cin.x, cin.y);
 #pragma unroll
@@ -470,7 +506,7 @@ __global__ __launch_bounds__(kThreads, NT == 1 ? 3 : 2) void cema_scan_fwd_kerne
       for (int i = 0; i < CPS; ++i) {
         const int c = sa * CPS + i;
         h = cadd(cmul(qT, h), cf{sv[i].x, sv[i].y});
-        if (c < nc) *reinterpret_cast<float2*>(col + c * kHP) = make_float2(h.x, h.y);
+        if (sl * CPS + i < w.nc) *reinterpret_cast<float2*>(col + c * kHP) = make_float2(h.x, h.y);
       }
     }
     wave_sync();
@@ -479,48 +515,44 @@ __global__ __launch_bounds__(kThreads, NT == 1 ? 3 : 2) void cema_scan_fwd_kerne
       u32x4 Q[4][2];
 #pragma unroll
       for (int b = 0; b < 4; ++b) load_block(8 + b, Q[b]);
+      if (w.nc > 0) {
+        u32x4 hb[2][2];
+        // the state in front of chunk c0 + r: the previous row of the buffer, or, for the
+        // wave's first chunk, what the scan left in wave_cin
+        const float* hrow = r == 0 ? sm.wave_cin[wave] : sm.H + (c0 + r) * kHP;
 #pragma unroll
-      for (int ctl = 0; ctl < NT; ++ctl) {
-        const int c0 = (wave * NT + ctl) * 32;
-        if (c0 < nc) {
-          u32x4 hb[2][2];
-          // the state in front of chunk c0 + r: the previous row of the buffer, or, for the
-          // wave's first chunk, what the scan left in wave_cin
-          const float* hrow = (ctl == 0 && r == 0) ? sm.wave_cin[wave] : sm.H + (c0 + r) * kHP;
+        for (int s2 = 0; s2 < 2; ++s2) {
+          const float* src = hrow + 16 * s2 + 8 * g;
+          const float4 u = *reinterpret_cast<const float4*>(src);
+          const float4 u1 = *reinterpret_cast<const float4*>(src + 4);
+          const float v[8] = {u.x, u.y, u.z, u.w, u1.x, u1.y, u1.z, u1.w};
+          split8(v, hb[s2][0], hb[s2][1]);
+        }
+        const int64_t chunk = w.chunk0 + r;
+#pragma unroll
+        for (int it = 0; it < 2; ++it) {
+          floatx16 acc = yacc[it];
 #pragma unroll
           for (int s2 = 0; s2 < 2; ++s2) {
-            const float* src = hrow + 16 * s2 + 8 * g;
-            const float4 u = *reinterpret_cast<const float4*>(src);
-            const float4 w = *reinterpret_cast<const float4*>(src + 4);
-            const float v[8] = {u.x, u.y, u.z, u.w, w.x, w.y, w.z, w.w};
-            split8(v, hb[s2][0], hb[s2][1]);
+            acc = mfma_bf16(Q[2 * it + s2][0], hb[s2][0], acc);
+            acc = mfma_bf16(Q[2 * it + s2][1], hb[s2][0], acc);
+            acc = mfma_bf16(Q[2 * it + s2][0], hb[s2][1], acc);
           }
-          const int64_t chunk = seg0 + c0 + r;
 #pragma unroll
-          for (int it = 0; it < 2; ++it) {
-            floatx16 acc = yacc[ctl][it];
+          for (int pr = 0; pr < 2; ++pr) {
+            if constexpr (DT == MEGA_F32) {
+              // registers 8 pr + 4 h + e hold the steps 16 pr + 8 h + 4 g + e: two 16-byte stores
+              // per lane, no exchange between the halves of the wave
 #pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2) {
-              acc = mfma_bf16(Q[2 * it + s2][0], hb[s2][0], acc);
-              acc = mfma_bf16(Q[2 * it + s2][1], hb[s2][0], acc);
-              acc = mfma_bf16(Q[2 * it + s2][0], hb[s2][1], acc);
-            }
-#pragma unroll
-            for (int pr = 0; pr < 2; ++pr) {
-              if constexpr (DT == MEGA_F32) {
-                // registers 8 pr + 4 h + e hold the steps 16 pr + 8 h + 4 g + e: two 16-byte stores
-                // per lane, no exchange between the halves of the wave
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                  const int64_t elem = chunk * kT + 16 * (2 * it + pr) + 8 * h + 4 * g;
-                  if (elem + 4 <= L)
-                    *reinterpret_cast<float4*>(yrow + elem) = make_float4(acc[8 * pr + 4 * h], acc[8 * pr + 4 * h + 1],
-                                                                          acc[8 * pr + 4 * h + 2], acc[8 * pr + 4 * h + 3]);
-                }
-              } else {
-                const uint4 oct = octet_of<DT>(acc, pr);
-                store8_16<ANY>(yrow, chunk * kT + 16 * (2 * it + pr) + 8 * g, L, oct);
+              for (int h = 0; h < 2; ++h) {
+                const int64_t elem = chunk * kT + 16 * (2 * it + pr) + 8 * h + 4 * g;
+                if (elem + 4 <= L)
+                  *reinterpret_cast<float4*>(yrow + elem) = make_float4(acc[8 * pr + 4 * h], acc[8 * pr + 4 * h + 1],
+                                                                        acc[8 * pr + 4 * h + 2], acc[8 * pr + 4 * h + 3]);
               }
+            } else {
+              const uint4 oct = octet_of<DT>(acc, pr);
+              store8_16<ANY>(yrow, chunk * kT + 16 * (2 * it + pr) + 8 * g, L, oct);
             }
           }
         }
@@ -528,56 +560,76 @@ __global__ __launch_bounds__(kThreads, NT == 1 ? 3 : 2) void cema_scan_fwd_kerne
     }
     cur ^= 1;
     par ^= 1;
-    if (seg0 + NC >= C && h_last != nullptr) {
-      // the row's last segment: the state after step L - 1 (the last chunk may be partial)
-      lds_barrier();
-      if (tid < N) {
-        const typename Elem<DT>::type* xrow = static_cast<const typename Elem<DT>::type*>(x) + row * L;
-        const int rem = static_cast<int>(L - (C - 1) * kT);  // 1 .. 64 steps in the last chunk
-        const int cl = static_cast<int>(C - 1 - seg0);       // the last chunk inside this segment
-        cf h;
-        if (rem == kT) {
-          const float* lastrow = sm.H + (1 + cl) * kHP + 2 * tid;
-          h = cf{lastrow[0], lastrow[1]};
-        } else {
-          // H[C-2]: the row in front of the last chunk, or the wave's carried-in state
-          const float* prev = (cl % (NT * 32) == 0) ? sm.wave_cin[cl / (NT * 32)] + 2 * tid
-                                                    : sm.H + cl * kHP + 2 * tid;
-          // the recurrence itself over the last chunk's steps (the power table has made way for
-          // the states by now): h <- q h + p x
-          h = cf{prev[0], prev[1]};
-          const cf q1 = sm.pw[8][tid];
-          const float pp = sm.pn[tid];
-          for (int j = 0; j < rem; ++j) {
-            const float xv = Elem<DT>::load(xrow + (C - 1) * kT + j) * pp;
-            h = cmul(q1, h);
-            h.x += xv;
-          }
+    if (w.nc > 0 && w.chunk0 + 32 >= static_cast<int>(C) && h_last != nullptr && lane < N) {
+      // the state after step L - 1 (the row's last chunk may be partial), from this wave's own rows
+      const typename Elem<DT>::type* xrow = static_cast<const typename Elem<DT>::type*>(x) + w.row * L;
+      const int rem = static_cast<int>(L - (C - 1) * kT);  // 1 .. 64 steps in the last chunk
+      const int cl = w.nc - 1;                             // the last chunk inside the tile
+      cf h;
+      if (rem == kT) {
+        const float* lastrow = sm.H + (1 + c0 + cl) * kHP + 2 * lane;
+        h = cf{lastrow[0], lastrow[1]};
+      } else {
+        const float* prev = cl == 0 ? sm.wave_cin[wave] + 2 * lane : sm.H + (c0 + cl) * kHP + 2 * lane;
+        // the recurrence itself over the last chunk's steps (the power table has made way for
+        // the states by now): h <- q h + p x
+        h = cf{prev[0], prev[1]};
+        const cf q1 = sm.pw[8][lane];
+        const float pp = sm.pn[lane];
+        for (int j = 0; j < rem; ++j) {
+          const float xv = Elem<DT>::load(xrow + (C - 1) * kT + j) * pp;
+          h = cmul(q1, h);
+          h.x += xv;
         }
-        h_last[row * N + tid] = h;
       }
+      h_last[w.row * N + lane] = h;
     }
   };
 
-  load_tiles(xb, blockIdx.x, 0);
-  for (int64_t row = blockIdx.x; row < rows; row += gridDim.x)
-    for (int64_t seg0 = 0; seg0 < C; seg0 += NC) item(row, seg0);
+  load_tile(xb, cur_tile);
+  for (int group = blockIdx.x; group < ln.groups; group += static_cast<int>(gridDim.x)) {
+    const int tiles = ln.tiles(group);
+    for (int t0 = 0; t0 < tiles; t0 += kWaves) item(group, t0, tiles);
+  }
 }
 
-template <int DT, int NT, bool ANY>
+// How many rows of a channel a group takes: as many as leave `slots` groups, so that a small
+// launch still fills the chip.
+Lines make_lines(int64_t B, int64_t D, int64_t L, int64_t slots, bool single) {
+  Lines ln;
+  int64_t nb = single ? 1 : B * D / slots;
+  nb = nb < 1 ? 1 : (nb > B ? B : nb);
+  ln.B = static_cast<int>(B);
+  ln.D = static_cast<int>(D);
+  ln.nb = static_cast<int>(nb);
+  ln.groups = static_cast<int>(D * ((B + nb - 1) / nb));
+  ln.L = L;
+  ln.C = (L + kT - 1) / kT;
+  ln.tpr = static_cast<int>((ln.C + 31) / 32);
+  return ln;
+}
+int compute_units(int* cus) {
+  int dev = 0;
+  MEGA_CHECK_HIP(hipGetDevice(&dev));
+  MEGA_CHECK_HIP(hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev));
+  return MEGA_OK;
+}
+
+template <int DT, bool ANY>
 int launch_fwd(const void* x, void* y, const float* p, const cf* log_q, const cf* gamma,
                const float* omega, const cf* h0, cf* h_last, int64_t B, int64_t D, int64_t N,
                int64_t L, hipStream_t stream) {
-  const size_t lds = sizeof(FwdSmem<NT>);
-  MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cema_scan_fwd_kernel<DT, NT, ANY>),
+  const size_t lds = sizeof(FwdSmem);
+  MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cema_scan_fwd_kernel<DT, ANY>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-  int dev = 0, cus = 0;
-  MEGA_CHECK_HIP(hipGetDevice(&dev));
-  MEGA_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  const int64_t rows = B * D, slots = (NT == 1 ? 3 : 2) * static_cast<int64_t>(cus);  // workgroups that fit a compute unit
-  const unsigned grid = static_cast<unsigned>(rows < slots ? rows : slots);
-  cema_scan_fwd_kernel<DT, NT, ANY><<<dim3(grid), kThreads, lds, stream>>>(
-      x, y, p, log_q, gamma, omega, h0, h_last, rows, static_cast<int>(D), static_cast<int>(N), L);
+  int cus = 0;
+  const int rc = compute_units(&cus);
+  if (rc != MEGA_OK) return rc;
+  const int64_t slots = 3 * static_cast<int64_t>(cus);  // workgroups that fit the chip
+  const Lines ln = make_lines(B, D, L, slots, false);
+  const unsigned grid = static_cast<unsigned>(ln.groups < slots ? ln.groups : slots);
+  cema_scan_fwd_kernel<DT, ANY><<<dim3(grid), kThreads, lds, stream>>>(x, y, p, log_q, gamma, omega, h0, h_last, ln,
+                                                                       static_cast<int>(N));
   MEGA_CHECK_LAUNCH();
   return MEGA_OK;
 }
@@ -656,10 +708,10 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
     const void* __restrict__ dy, const void* __restrict__ x, void* __restrict__ dx,
     const float* __restrict__ p, const cf* __restrict__ log_q, const cf* __restrict__ gamma,
     const float* __restrict__ omega, const cf* __restrict__ h0, float* __restrict__ dp, cf* __restrict__ dq,
-    cf* __restrict__ dgamma, float* __restrict__ domega, cf* __restrict__ dh0, int64_t rows, int D, int N,
-    int64_t L) {
+    cf* __restrict__ dgamma, float* __restrict__ domega, cf* __restrict__ dh0, const Lines ln, int N) {
   static_assert(XOp<DT>::XP == 1, "the backward kernel takes bfloat16 rows");
-  constexpr int NC = kBwdNC, CPS = kBwdCPS;
+  constexpr int CPS = kBwdCPS;
+  const int64_t L = ln.L;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   BwdSmem& sm = *reinterpret_cast<BwdSmem*>(smem_raw);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -673,39 +725,33 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
   (void)stage
   cf (*qp)[kT + 2] = reinterpret_cast<cf(*)[kT + 2]>(sm.R);                 // setup and finish only
   cf (*ab)[2][16] = reinterpret_cast<cf(*)[2][16]>(sm.R + 2 * 16 * (kT + 2));  // finish only, behind the table
-  const int64_t C = (L + kT - 1) / kT;
-  const int64_t seg_last = (C - 1) / NC * NC;
+  // the last four tiles of a group's line, where its walk starts
+  auto tail_of = [&](int group) { return group < ln.groups ? (ln.tiles(group) - 1) / kWaves * kWaves : 0; };
 
   XOp<DT> db[4], xb[4], dn[4];  // dn: the next item's dy tile on its way
-  auto load_dy = [&](int64_t row, int64_t seg0) {
+  auto load_dy = [&](const Tile& w) {
     MEGA_LANE_IDS;
-    const uint16_t* dyrow = static_cast<const uint16_t*>(dy) + row * L;
-    const int64_t chunk = seg0 + wave * 32 + r;
+    const uint16_t* row = static_cast<const uint16_t*>(dy) + w.row * L;
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const int64_t elem = chunk * kT + 16 * s + 8 * g;
-      dn[s].template load<ANY>(dyrow, elem, row < rows, L);
-    }
+    for (int s = 0; s < 4; ++s)
+      dn[s].template load<ANY>(row, static_cast<int64_t>(w.chunk0 + r) * kT + 16 * s + 8 * g, w.nc > 0, L);
   };
-  auto load_x = [&](int64_t row, int64_t seg0) {
+  auto load_x = [&](const Tile& w) {
     MEGA_LANE_IDS;
-    const uint16_t* xrow = static_cast<const uint16_t*>(x) + row * L;
-    const int64_t chunk = seg0 + wave * 32 + r;
+    const uint16_t* row = static_cast<const uint16_t*>(x) + w.row * L;
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const int64_t elem = chunk * kT + 16 * s + 8 * g;
-      xb[s].template load<ANY>(xrow, elem, row < rows, L);
-    }
+    for (int s = 0; s < 4; ++s)
+      xb[s].template load<ANY>(row, static_cast<int64_t>(w.chunk0 + r) * kT + 16 * s + 8 * g, w.nc > 0, L);
   };
   struct RowParams {
     cf lq, gv;
     float pv, w;
   };
-  auto fetch_params = [&](int64_t row) {
+  auto fetch_params = [&](int group) {
     MEGA_LANE_IDS;
     RowParams rp{cf{0.f, 0.f}, cf{0.f, 0.f}, 0.f, 0.f};
-    if (row < rows) {
-      const int d = static_cast<int>(row % D);
+    if (group < ln.groups) {
+      const int d = group % ln.D;
       if (sn < N) {
         rp.lq = log_q[d * N + sn];
         rp.gv = gamma[d * N + sn];
@@ -730,7 +776,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
   floatx16 macc[3];      // M tiles (0,0), (1,0), (1,1) over this wave's chunks
   cf wacc[8], wdacc[8];  // W, W' of modes n = 4 qd + 2 g + b at index 2 qd + b, over this lane's chunks
 
-  auto setup_row = [&](int64_t row) {
+  auto setup_row = [&](int group) {
     MEGA_LANE_IDS;
     // powers evaluated directly (phase reduced in float64), 14 per mode: q^(4 k), q^(16 k)
     // (k < 4), q, q^64, q^(64 CPS), q^(64 CPS - 1), q^(256 CPS), q^(256 CPS - 1)
@@ -810,11 +856,11 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
 #pragma unroll
     for (int i = 0; i < 8; ++i) wacc[i] = wdacc[i] = cf{0.f, 0.f};
     __syncthreads();
-    rp = fetch_params(row + gridDim.x);
+    rp = fetch_params(group + static_cast<int>(gridDim.x));
   };
 
   // the row's reductions and its five gradient outputs
-  auto finish_row = [&](int64_t row) {
+  auto finish_row = [&](int64_t row) {  // the group's outputs; with a carried state a group is one row
     MEGA_LANE_IDS;
     // W, W': over the 32 lanes (chunks) of a half wave, then over the waves.  A lane holds 32
     // partial sums (8 modes x (W, W') x (re, im)) and each half of the wave its own 8 modes: the
@@ -956,7 +1002,8 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
     if (tid == 0) domega[row] = sm.dkin[0];
   };
 
-  auto item = [&](int64_t row, int64_t seg0) {
+  Tile cur_tile = tile_at(ln, blockIdx.x, tail_of(blockIdx.x) + wave);  // this wave's tile of the item
+  auto item = [&](int group, int t0, int tiles) {
     MEGA_LANE_IDS;
     // transposing read of the parked tile: row tile tt (32 time steps), k-step ks (16 chunks)
     const int tr_base = (8 * g + ((lane & 15) >> 2)) * kSP + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
@@ -965,19 +1012,20 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       const uint2 lo = lds_read_tr(q), hi = lds_read_tr(q + 4 * kSP);
       return u32x4{lo.x, lo.y, hi.x, hi.y};
     };
-    if (seg0 == seg_last) setup_row(row);
+    if (t0 + kWaves >= tiles) setup_row(group);
+    const Tile w = cur_tile;
     using dx_t = typename std::conditional<DX32 != 0, float, uint16_t>::type;
-    dx_t* dxrow = static_cast<dx_t*>(dx) + row * L;
-    const int nc = static_cast<int>(C - seg0 < NC ? C - seg0 : NC);
-    const int c0 = wave * 32;
-    const bool on = c0 < nc;
+    dx_t* dxrow = static_cast<dx_t*>(dx) + w.row * L;
+    const bool on = w.nc > 0;
     u32x4 xr[4];  // time-reversed x as an operand: steps 63 - (16 s + 8 g + e)
     // the next item of this workgroup: its x tile is requested as soon as this item's has been
     // consumed, its dy tile at the end of the item
-    int64_t nrow = row, nseg = seg0 - NC;
-    if (nseg < 0) {
-      nrow = row + gridDim.x;
-      nseg = seg_last;
+    Tile next = w;
+    if (t0 > 0) {
+      tile_backward(ln, next, tiles);
+    } else {
+      const int ng = group + static_cast<int>(gridDim.x);
+      next = tile_at(ln, ng, tail_of(ng) + wave);
     }
     if (on) {
       // ---- the wave's private tile: X parked first (it arrived an item ago), read back with
@@ -1015,7 +1063,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
         }
       wave_sync();  // the tile has been read: its place takes the wave's rows of (G, G')
     }
-    load_x(nrow, nseg);
+    load_x(next);
     if (on) {
       // ---- (G, G') = Pg DY, into this wave's own rows of the state buffer ----------------
 #pragma unroll
@@ -1037,7 +1085,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       }
     }
     wave_sync();
-    load_dy(nrow, nseg);
+    load_dy(next);
     // ---- reverse scan over the chunks of the segment; a wave's four sub-segments are its own
     //      chunks, one workgroup barrier hands over the waves' ends ---------------------------------
     {
@@ -1046,7 +1094,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
 #pragma unroll
       for (int i = 0; i < CPS; ++i) {
         const int c = sa * CPS + i;
-        const bool live = c < nc;
+        const bool live = sl * CPS + i < w.nc;
         const float2 a0 = *reinterpret_cast<const float2*>(col + c * kRP);
         const float2 b0 = *reinterpret_cast<const float2*>(col + c * kRP + 32);
         gv[i] = live ? a0 : make_float2(0.f, 0.f);
@@ -1073,11 +1121,13 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       }
       lds_barrier();
       cf h = sm.carry[cur][0][sn], hd = sm.carry[cur][1][sn];
+      // through the tiles behind this wave's, from the last one of its row if that is among the four
+      // (nothing comes from behind it)
+      const int k = ln.tpr - 1 - w.chunk0 / 32, from = wave + k < kWaves ? wave + k : kWaves - 1;
+      if (wave + k < kWaves) h = hd = cf{0.f, 0.f};
 #pragma unroll
-      for (int w = kWaves - 1; w >= 1; --w) {
-        const cf we = sm.wave_end[par][w][0][sn], wed = sm.wave_end[par][w][1][sn];
-        if (w > wave) rstep(h, hd, we, wed, qW, qWd);
-      }
+      for (int v = kWaves - 1; v >= 1; --v)
+        if (v > wave && v <= from) rstep(h, hd, sm.wave_end[par][v][0][sn], sm.wave_end[par][v][1][sn], qW, qWd);
       if (sa == 0) {
         // through wave 0's chunks too: the state at the start of the segment, the next item's carry
         cf ch = h, chd = hd;
@@ -1098,7 +1148,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       for (int i = CPS - 1; i >= 0; --i) {
         const int c = sa * CPS + i;
         rstep(h, hd, cf{gv[i].x, gv[i].y}, cf{gd[i].x, gd[i].y}, qT, qTd);
-        if (c < nc) {
+        if (sl * CPS + i < w.nc) {
           *reinterpret_cast<float2*>(col + c * kRP) = make_float2(h.x, h.y);
           *reinterpret_cast<float2*>(col + c * kRP + 32) = make_float2(hd.x, hd.y);
         }
@@ -1108,7 +1158,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
     if (on) {
       // (R, R')[c + 1]: the next row of the buffer, or, for the wave's last chunk, wave_cin;
       // chunks past the end of the row have X = 0 and DY = 0, their rows may hold anything
-      const bool live = c0 + r < nc;
+      const bool live = r < w.nc;
       const float* rnext = (r == 31) ? sm.wave_cin[wave] : myrows + (r + 1) * kRP;
       const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
       // the stores of dX go out first: they have the (X, X') products and the next item's
@@ -1119,13 +1169,13 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       for (int s2 = 0; s2 < 2; ++s2) {
         const float* src = rnext + 16 * s2 + 8 * g;
         const float4 u0 = *reinterpret_cast<const float4*>(src);
-        const float4 w0 = *reinterpret_cast<const float4*>(src + 4);
-        const float4 u = live ? u0 : zero4;
-        const float4 w = live ? w0 : zero4;
-        const float v[8] = {u.x, u.y, u.z, u.w, w.x, w.y, w.z, w.w};
+        const float4 u1 = *reinterpret_cast<const float4*>(src + 4);
+        const float4 ua = live ? u0 : zero4;
+        const float4 ub = live ? u1 : zero4;
+        const float v[8] = {ua.x, ua.y, ua.z, ua.w, ub.x, ub.y, ub.z, ub.w};
         split8(v, hb[s2][0], hb[s2][1]);
       }
-      const int64_t chunk = seg0 + c0 + r;
+      const int64_t chunk = w.chunk0 + r;
 #pragma unroll
       for (int jt = 0; jt < 2; ++jt) {
         floatx16 acc;
@@ -1209,35 +1259,48 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
     }
     cur ^= 1;
     par ^= 1;
-    if (seg0 == 0) finish_row(row);
+    if (t0 == 0) finish_row(group);
 #pragma unroll
     for (int s = 0; s < 4; ++s) db[s] = dn[s];
+    cur_tile = next;
   };
 
-  load_x(blockIdx.x, seg_last);
-  load_dy(blockIdx.x, seg_last);
+  load_x(cur_tile);
+  load_dy(cur_tile);
 #pragma unroll
   for (int s = 0; s < 4; ++s) db[s] = dn[s];
-  for (int64_t row = blockIdx.x; row < rows; row += gridDim.x)
-    for (int64_t seg0 = seg_last; seg0 >= 0; seg0 -= NC) item(row, seg0);
+  for (int group = blockIdx.x; group < ln.groups; group += static_cast<int>(gridDim.x)) {
+    const int tiles = ln.tiles(group);
+    for (int t0 = (tiles - 1) / kWaves * kWaves; t0 >= 0; t0 -= kWaves) item(group, t0, tiles);
+  }
 #undef MEGA_LANE_IDS
 }
 
+// Rows of a channel that the backward puts together (make_lines); a carried state's gradients are per row.
+int bwd_lines(int64_t B, int64_t D, int64_t L, bool single, Lines* ln, int64_t* slots) {
+  int cus = 0;
+  const int rc = compute_units(&cus);
+  if (rc != MEGA_OK) return rc;
+  *slots = 2 * static_cast<int64_t>(cus);  // two workgroups fit a compute unit
+  *ln = make_lines(B, D, L, *slots, single);
+  return MEGA_OK;
+}
+
+// single: gradients per row (B, D, N) as the operator returns them; else per group of rows
 template <int DX32, bool ANY>
 int launch_bwd(const void* dy, const void* x, void* dx, const float* p, const cf* log_q,
                const cf* gamma, const float* omega, const cf* h0, float* dp, cf* dq, cf* dgamma, float* domega,
-               cf* dh0, int64_t B, int64_t D, int64_t N, int64_t L, hipStream_t stream) {
+               cf* dh0, int64_t B, int64_t D, int64_t N, int64_t L, bool single, hipStream_t stream) {
   const int lds = static_cast<int>(sizeof(BwdSmem));
   MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cema_scan_bwd_kernel<MEGA_BF16, DX32, ANY>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-  int dev = 0, cus = 0;
-  MEGA_CHECK_HIP(hipGetDevice(&dev));
-  MEGA_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  const int64_t rows = B * D, slots = 2 * static_cast<int64_t>(cus);  // two workgroups fit a compute unit
-  const unsigned grid = static_cast<unsigned>(rows < slots ? rows : slots);
+  Lines ln;
+  int64_t slots = 0;
+  const int rc = bwd_lines(B, D, L, single || h0 != nullptr, &ln, &slots);
+  if (rc != MEGA_OK) return rc;
+  const unsigned grid = static_cast<unsigned>(ln.groups < slots ? ln.groups : slots);
   cema_scan_bwd_kernel<MEGA_BF16, DX32, ANY><<<dim3(grid), kThreads, lds, stream>>>(
-      dy, x, dx, p, log_q, gamma, omega, h0, dp, dq, dgamma, domega, dh0, rows, static_cast<int>(D),
-      static_cast<int>(N), L);
+      dy, x, dx, p, log_q, gamma, omega, h0, dp, dq, dgamma, domega, dh0, ln, static_cast<int>(N));
   MEGA_CHECK_LAUNCH();
   return MEGA_OK;
 }
@@ -1272,13 +1335,12 @@ extern "C" int mega_cema_scan_fwd(const void* x, int dtype, const float* p, cons
   const cf* gm = reinterpret_cast<const cf*>(gamma);
   const cf* h0c = reinterpret_cast<const cf*>(h0);
   cf* hl = reinterpret_cast<cf*>(h_last);
-  // one chunk tile per wave (segments of 128 chunks) measured 5 % faster than two for bfloat16 rows as well
-  if (dtype == MEGA_F32) return launch_fwd<MEGA_F32, 1, false>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s);
+  if (dtype == MEGA_F32) return launch_fwd<MEGA_F32, false>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s);
   if (dtype == MEGA_BF16)
-    return any ? launch_fwd<MEGA_BF16, 1, true>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s)
-               : launch_fwd<MEGA_BF16, 1, false>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s);
-  return any ? launch_fwd<MEGA_F16, 1, true>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s)
-             : launch_fwd<MEGA_F16, 1, false>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s);
+    return any ? launch_fwd<MEGA_BF16, true>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s)
+               : launch_fwd<MEGA_BF16, false>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s);
+  return any ? launch_fwd<MEGA_F16, true>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s)
+             : launch_fwd<MEGA_F16, false>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s);
 }
 
 extern "C" int mega_cema_scan_bwd_supported(int dtype, int64_t N, int64_t L) {
@@ -1304,7 +1366,7 @@ extern "C" int mega_cema_scan_bwd_state(const void* dy, const void* x, int dtype
   MEGA_CHECK_ARG(dh0 == nullptr || h0 != nullptr, "%s: dh0 without h0", who);
   return (any ? launch_bwd<0, true> : launch_bwd<0, false>)(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma),
                            omega, reinterpret_cast<const cf*>(h0), dp, reinterpret_cast<cf*>(dq),
-                           reinterpret_cast<cf*>(dgamma), domega, reinterpret_cast<cf*>(dh0), B, D, N, L,
+                           reinterpret_cast<cf*>(dgamma), domega, reinterpret_cast<cf*>(dh0), B, D, N, L, true,
                            static_cast<hipStream_t>(stream));
 }
 
@@ -1334,10 +1396,37 @@ extern "C" int mega_cema_scan_bwd_wide(const void* dy, const void* x, const floa
   if (accumulate_dx && dx != nullptr)
     return (any ? launch_bwd<2, true> : launch_bwd<2, false>)(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma),
                          omega, reinterpret_cast<const cf*>(h0), dp, reinterpret_cast<cf*>(dq),
-                         reinterpret_cast<cf*>(dgamma), domega, reinterpret_cast<cf*>(dh0), B, D, N, L,
+                         reinterpret_cast<cf*>(dgamma), domega, reinterpret_cast<cf*>(dh0), B, D, N, L, true,
                          static_cast<hipStream_t>(stream));
   return (any ? launch_bwd<1, true> : launch_bwd<1, false>)(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma),
                        omega, reinterpret_cast<const cf*>(h0), dp, reinterpret_cast<cf*>(dq),
-                       reinterpret_cast<cf*>(dgamma), domega, reinterpret_cast<cf*>(dh0), B, D, N, L,
+                       reinterpret_cast<cf*>(dgamma), domega, reinterpret_cast<cf*>(dh0), B, D, N, L, true,
                        static_cast<hipStream_t>(stream));
+}
+
+extern "C" int64_t mega_cema_layer_scan_sets(int64_t B, int64_t D, int64_t L) {
+  Lines ln;
+  int64_t slots = 0;
+  if (B < 1 || D < 1 || L < 1 || bwd_lines(B, D, L, false, &ln, &slots) != MEGA_OK) return 0;
+  return ln.groups / ln.D;
+}
+
+extern "C" int mega_cema_layer_scan_bwd(const void* dy, const void* x, const float* p, const float* log_q,
+                                        const float* gamma, const float* omega, int64_t B, int64_t D, int64_t N,
+                                        int64_t L, void* dx, int dx_mode, float* dp, float* dq, float* dgamma,
+                                        float* domega, void* stream) {
+  const char* who = "mega_cema_layer_scan_bwd";
+  MEGA_CHECK_ARG(dy && x && p && log_q && gamma && dp && dq && dgamma && domega, "%s: null pointer", who);
+  MEGA_CHECK_ARG(B >= 1 && D >= 1 && B * D <= 0x7fffffff, "%s: bad sizes", who);
+  MEGA_CHECK_ARG(dx_mode >= 0 && dx_mode <= 2 && (dx != nullptr || dx_mode == 1), "%s: bad dx", who);
+  if (!mega_cema_scan_bwd_supported(MEGA_BF16, N, L))
+    return set_error(MEGA_ERR_UNSUPPORTED, "%s: needs N <= 16 (N %lld, L %lld)", who, (long long)N, (long long)L);
+  const auto al = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
+  const bool any = L % 8 != 0 || !al(dy) || !al(x) || !al(dx);
+  auto go = dx_mode == 0   ? (any ? launch_bwd<0, true> : launch_bwd<0, false>)
+            : dx_mode == 1 ? (any ? launch_bwd<1, true> : launch_bwd<1, false>)
+                           : (any ? launch_bwd<2, true> : launch_bwd<2, false>);
+  return go(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma), omega, nullptr, dp,
+            reinterpret_cast<cf*>(dq), reinterpret_cast<cf*>(dgamma), domega, nullptr, B, D, N, L, false,
+            static_cast<hipStream_t>(stream));
 }

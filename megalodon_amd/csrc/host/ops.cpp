@@ -341,15 +341,15 @@ struct CemaFn : Function<CemaFn> {
     const int64_t B = x.size(0), D = x.size(1), L = x.size(2), N = alpha.size(1), DN = D * N;
     const float *p = c.data_ptr<float>(), *lq = p + DN, *gh = p + 3 * DN;
     void* s = stream_of(x);
-    // per-row gradients of the launches, stacked: (dp, dq, dgamma_hat, domega); the coefficients'
+    // gradients of the launches' groups of rows, stacked: (dp, dq, dgamma_hat, domega); the coefficients'
     // backward adds the stack up
-    const int64_t sets = x.scalar_type() == at::kBFloat16 ? B : 3 * B;
+    const int64_t per = mega_cema_layer_scan_sets(B, D, L), sets = x.scalar_type() == at::kBFloat16 ? per : 3 * per;
     const Tensor stack = floats({sets * (5 * DN + D)}, x);
     float *dp = stack.data_ptr<float>(), *dq = dp + sets * DN, *dg = dq + 2 * sets * DN, *dw = dg + 2 * sets * DN;
     Tensor dx;
     if (x.scalar_type() == at::kBFloat16) {
       dx = at::empty_like(x);
-      check(mega_cema_scan_bwd(dy.data_ptr(), x.data_ptr(), MEGA_BF16, p, lq, gh, fptr(w), B, D, N, L, dx.data_ptr(), dp, dq, dg, dw, s), "mega_cema_scan_bwd");
+      check(mega_cema_layer_scan_bwd(dy.data_ptr(), x.data_ptr(), p, lq, gh, fptr(w), B, D, N, L, dx.data_ptr(), 0, dp, dq, dg, dw, s), "mega_cema_layer_scan_bwd");
     } else {
       // linear in dy and, for the parameter gradients, in x: the bfloat16 pieces (dy_hi, x_hi), (dy_lo, x_hi),
       // (dy_hi, x_lo); dx is linear in dy alone and is added up in float32
@@ -358,7 +358,7 @@ struct CemaFn : Function<CemaFn> {
       Tensor dx32 = floats(x.sizes(), x);
       const Tensor* pairs[3][2] = {{&g_hi, &x_hi}, {&g_lo, &x_hi}, {&g_hi, &x_lo}};
       for (int i = 0; i < 3; ++i)
-        check(mega_cema_scan_bwd_wide(pairs[i][0]->data_ptr(), pairs[i][1]->data_ptr(), p, lq, gh, fptr(w), nullptr, B, D, N, L, i < 2 ? fptr(dx32) : nullptr, i == 1, dp + i * B * DN, dq + 2 * i * B * DN, dg + 2 * i * B * DN, dw + i * B * D, nullptr, s), "mega_cema_scan_bwd_wide");
+        check(mega_cema_layer_scan_bwd(pairs[i][0]->data_ptr(), pairs[i][1]->data_ptr(), p, lq, gh, fptr(w), B, D, N, L, i < 2 ? dx32.data_ptr() : nullptr, i == 1 ? 2 : 1, dp + i * per * DN, dq + 2 * i * per * DN, dg + 2 * i * per * DN, dw + i * per * D, s), "mega_cema_layer_scan_bwd");
       dx = dx32.to(x.scalar_type());
     }
     Tensor da = at::empty_like(alpha), dd = at::empty_like(delta), dt = at::empty_like(theta), dga = at::empty_like(gamma), dom = at::empty_like(omega);

@@ -19,9 +19,19 @@ def _rows(B, D, L, dtype, seed, offset):
     return v, t.copy_(v)
 
 
+class _picked:
+    """The parameters of some channels of a layer."""
+
+    def __init__(self, layer, pick):
+        for n in NAMES:
+            setattr(self, n, getattr(layer, n)[pick])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,D,L,offset", [(1, 2, 1, 0), (2, 3, 7, 0), (2, 2, 9, 1), (1, 3, 65, 0), (2, 3, 1021, 0),
-                                          (1, 2, 2047, 0), (1, 3, 4096, 3), (2, 2, 8193, 0), (1, 2, 20003, 5)])
+                                          (1, 2, 2047, 0), (1, 3, 4096, 3), (2, 2, 8193, 0), (1, 2, 20003, 5),
+                                          # several rows of a channel in one workgroup: two, two and one; five, of two tiles each
+                                          (5, 300, 130, 0), (5, 520, 2049, 1)])
 def test_layer_matches_oracle(B, D, L, offset, dtype):
     torch.manual_seed(L)
     layer = MultiHeadComplexEMA(D, 16).cuda().train()
@@ -30,26 +40,38 @@ def test_layer_matches_oracle(B, D, L, offset, dtype):
     x.requires_grad_(True)
     out, _ = layer(x)
     out.backward(dy)
+    grads = {n: getattr(layer, n).grad for n in NAMES}
+    dx = x.grad
+    if D > 64:  # every 50th channel is checked
+        pick = slice(0, None, 50)
+        out, dx, x0, dy0 = out[:, pick], dx[:, pick], x0[:, pick], dy0[:, pick]
+        grads = {n: g[pick] for n, g in grads.items()}
+        layer = _picked(layer, pick)
     pr = {n: getattr(layer, n).detach().cpu().double().requires_grad_(True) for n in NAMES}
     xo = x0.double().requires_grad_(True)
     p, q, g = ocema.calc_coeffs(pr["alpha"], pr["delta"], pr["theta"], pr["gamma"], 16)
     want = offt.fftconv_fwd(xo, ocema.ema_weight_fwd(p, q.log(), g, L)) + xo * pr["omega"]
     want.backward(dy0.double())
     assert out.dtype == dtype and rel_err(out, want.detach()) <= 2e-2
-    assert x.grad.dtype == dtype and rel_err(x.grad, xo.grad) <= 2e-2
+    assert dx.dtype == dtype and rel_err(dx, xo.grad) <= 2e-2
     for n in NAMES:
-        assert rel_err(getattr(layer, n).grad, pr[n].grad) <= 1e-4, n
+        assert rel_err(grads[n], pr[n].grad) <= 1e-4, n
 
 
-@pytest.mark.parametrize("L,offset", [(1, 0), (5, 0), (63, 1), (1531, 0), (8200, 1), (8201, 0)])
-def test_carried_and_last_state(L, offset):
-    B, D, N = 2, 3, 16
+@pytest.mark.parametrize("B,D,L,offset", [(2, 3, 1, 0), (2, 3, 5, 0), (2, 3, 63, 1), (2, 3, 1531, 0), (2, 3, 8200, 1),
+                                          (2, 3, 8201, 0), (5, 400, 70, 0), (7, 400, 2112, 0)])
+def test_carried_and_last_state(B, D, L, offset):
+    N = 16
     torch.manual_seed(L)
     layer = MultiHeadComplexEMA(D, N).cuda().eval()
     x0, x = _rows(B, D, L, torch.bfloat16, L, offset)
     h0 = torch.randn(B, D, N, dtype=torch.complex64, generator=torch.Generator().manual_seed(2))
     with torch.no_grad():
         out, last = layer(x, h0.cuda(), True)
+    if D > 64:  # every 50th channel is checked
+        pick = slice(0, None, 50)
+        out, last, x0, h0 = out[:, pick], last[:, pick], x0[:, pick], h0[:, pick]
+        layer = _picked(layer, pick)
     pr = {n: getattr(layer, n).detach().cpu().double() for n in NAMES}
     p, q, g = ocema.calc_coeffs(pr["alpha"], pr["delta"], pr["theta"], pr["gamma"], N)
     want = offt.fftconv_fwd(x0.double(), ocema.ema_weight_fwd(p, q.log(), g, L)) + x0.double() * pr["omega"]
