@@ -30,6 +30,7 @@
 #include "common.hpp"
 #include "cema_pow.hpp"
 
+#include <initializer_list>
 #include <type_traits>
 
 namespace mega {
@@ -109,38 +110,51 @@ __device__ __forceinline__ float opaque_one() {
   return one;
 }
 
-// Rows that do not start on 16-byte boundaries (a length that is no multiple of 8, or an odd storage
-// offset): the same 16-byte accesses, which this part takes at any element's address, except
-// for the piece that straddles the end of the row, which goes element by element.
+// How the rows of a launch lie in memory.
+//   kWhole   every row starts on a 16-byte boundary and its length is a multiple of 8
+//   kShifted rows of another length in a tensor that starts on one: a row is taken from the
+//            16-byte boundary at or in front of its start, the up to seven steps in front of it
+//            as zeros -- with no state before them the recurrence does not see them -- so that
+//            every access but those at the two ends is aligned
+//   kAny     a carried state, or a tensor that starts or ends off a boundary: the same 16-byte accesses at
+//            any element's address (which cost more: 4 x 2048 rows of 5001 steps forward and backward
+//            241 us so, 191 shifted, 169 for 5000 steps)
+enum { kWhole = 0, kShifted = 1, kAny = 2 };
 typedef u32x4 u32x4_any __attribute__((aligned(2)));
-__device__ __forceinline__ u32x4 load_tail16(const uint16_t* src, int n) {
-  uint32_t w[4] = {0u, 0u, 0u, 0u};
+// of the 16-bit steps elem .. elem + 7 those of lo .. hi - 1, zeros for the others
+__device__ __forceinline__ u32x4 keep_steps(u32x4 v, int elem, int lo, int hi) {
 #pragma unroll
   for (int e = 0; e < 8; ++e)
-    if (e < n) w[e >> 1] |= static_cast<uint32_t>(src[e]) << (16 * (e & 1));
-  return u32x4{w[0], w[1], w[2], w[3]};
-}
-// steps elem .. elem + 7 of a row of L 16-bit steps, zero behind its end
-template <bool ANY>
-__device__ __forceinline__ u32x4 load8_16(const uint16_t* row, int64_t elem, bool on, int64_t L) {
-  const uint16_t* src = row + elem;
-  if (!ANY) return on && elem + 8 <= L ? *reinterpret_cast<const u32x4*>(src) : u32x4{0u, 0u, 0u, 0u};
-  u32x4 v = {0u, 0u, 0u, 0u};
-  if (on && elem + 8 <= L) v = *reinterpret_cast<const u32x4_any*>(src);
-  else if (on && elem < L) v = load_tail16(src, static_cast<int>(L - elem));
+    if (elem + e < lo || elem + e >= hi) v[e >> 1] &= e & 1 ? 0x0000ffffu : 0xffff0000u;
   return v;
 }
-template <bool ANY>
-__device__ __forceinline__ void store8_16(uint16_t* row, int64_t elem, int64_t L, uint4 v) {
-  uint16_t* dst = row + elem;
-  if (elem + 8 <= L) {
-    if (ANY) *reinterpret_cast<u32x4_any*>(dst) = u32x4{v.x, v.y, v.z, v.w};
+// steps elem .. elem + 7 of a tile of which lo .. hi - 1 exist, zeros elsewhere
+template <int ROWS>
+__device__ __forceinline__ u32x4 load8_16(const uint16_t* tile, int elem, int lo, int hi) {
+  const uint16_t* src = tile + elem;
+  u32x4 v = {0u, 0u, 0u, 0u};
+  if (ROWS != kAny) {  // (kShifted: a piece with one of the steps is inside the tensor)
+    if (elem < hi) v = *reinterpret_cast<const u32x4*>(src);
+  } else if (elem + 8 <= hi) {
+    v = *reinterpret_cast<const u32x4_any*>(src);
+  } else if (elem < hi) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (elem + e < hi) v[e >> 1] |= static_cast<uint32_t>(src[e]) << (16 * (e & 1));
+  }
+  return v;
+}
+template <int ROWS>
+__device__ __forceinline__ void store8_16(uint16_t* tile, int elem, int lo, int hi, uint4 v) {
+  uint16_t* dst = tile + elem;
+  if ((ROWS != kShifted || elem >= lo) && elem + 8 <= hi) {
+    if (ROWS == kAny) *reinterpret_cast<u32x4_any*>(dst) = u32x4{v.x, v.y, v.z, v.w};
     else *reinterpret_cast<uint4*>(dst) = v;
-  } else if (ANY && elem < L) {
+  } else if (ROWS != kWhole && elem < hi) {
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
     for (int e = 0; e < 8; ++e)
-      if (elem + e < L) dst[e] = static_cast<uint16_t>(w[e >> 1] >> (16 * (e & 1)));
+      if (elem + e >= lo && elem + e < hi) dst[e] = static_cast<uint16_t>(w[e >> 1] >> (16 * (e & 1)));
   }
 }
 
@@ -150,10 +164,11 @@ template <int DT> struct XOp;
 template <> struct XOp<MEGA_BF16> {
   static constexpr int XP = 1;
   u32x4 pc[1];
-  template <bool ANY>
-  __device__ __forceinline__ void load(const void* row, int64_t elem, bool on, int64_t L) {
-    pc[0] = load8_16<ANY>(static_cast<const uint16_t*>(row), elem, on, L);
+  template <int ROWS>
+  __device__ __forceinline__ void load(const void* tile, int elem, int lo, int hi) {
+    pc[0] = load8_16<ROWS>(static_cast<const uint16_t*>(tile), elem, lo, hi);
   }
+  __device__ __forceinline__ void keep(int elem, int lo, int hi) { pc[0] = keep_steps(pc[0], elem, lo, hi); }
   __device__ __forceinline__ void values(float* v) const {
     unpack8<MEGA_BF16>(make_uint4(pc[0][0], pc[0][1], pc[0][2], pc[0][3]), v);
   }
@@ -161,12 +176,16 @@ template <> struct XOp<MEGA_BF16> {
 template <> struct XOp<MEGA_F16> {
   static constexpr int XP = 2;
   u32x4 pc[2];
-  template <bool ANY>
-  __device__ __forceinline__ void load(const void* row, int64_t elem, bool on, int64_t L) {
+  template <int ROWS>
+  __device__ __forceinline__ void load(const void* tile, int elem, int lo, int hi) {
     float v[8];
-    const u32x4 raw = load8_16<ANY>(static_cast<const uint16_t*>(row), elem, on, L);
+    const u32x4 raw = load8_16<ROWS>(static_cast<const uint16_t*>(tile), elem, lo, hi);
     unpack8<MEGA_F16>(make_uint4(raw[0], raw[1], raw[2], raw[3]), v);
     split8(v, pc[0], pc[1]);
+  }
+  __device__ __forceinline__ void keep(int elem, int lo, int hi) {
+    pc[0] = keep_steps(pc[0], elem, lo, hi);
+    pc[1] = keep_steps(pc[1], elem, lo, hi);
   }
   __device__ __forceinline__ void values(float* v) const {
     float a[8], b[8];
@@ -182,12 +201,13 @@ template <> struct XOp<MEGA_F16> {
 template <> struct XOp<MEGA_F32> {
   static constexpr int XP = 2;
   u32x4 pc[2];
-  template <bool ANY>
-  __device__ __forceinline__ void load(const void* row, int64_t elem, bool on, int64_t L) {
-    static_assert(!ANY, "float32 rows are aligned");
+  template <int ROWS>
+  __device__ __forceinline__ void load(const void* tile, int elem, int lo, int hi) {
+    static_assert(ROWS == kWhole, "float32 rows are aligned");
+    (void)lo;
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
-    if (on && elem + 8 <= L) {
-      const float4* src = reinterpret_cast<const float4*>(static_cast<const float*>(row) + elem);
+    if (elem < hi) {
+      const float4* src = reinterpret_cast<const float4*>(static_cast<const float*>(tile) + elem);
       a = src[0];
       b = src[1];
     }
@@ -232,21 +252,34 @@ static_assert(sizeof(cf) * 16 * (kT + 2) <= sizeof(float) * (kWaves * 32 + 1) * 
 struct Lines {
   int B, D, nb, groups;  // groups = D ceil(B / nb)
   int tpr;               // tiles per row
-  int64_t L, C;          // steps and chunks of a row
+  int64_t L;             // steps of a row
   __device__ __forceinline__ int first_row(int group) const { return group / D * nb; }
   __device__ __forceinline__ int tiles(int group) const { return min(nb, B - first_row(group)) * tpr; }
 };
 // A tile of a group's line: which row, where in it.  Stepping from one of a wave's tiles to the
-// next needs no division.
+// next needs no division; lanes address inside it by 32-bit offsets from a base that the wave shares
+// (4096 rows of 32768 steps forward and backward: 458 us with 64-bit offsets from the row, 446 so).
 struct Tile {
   int64_t row;  // b D + d
+  int64_t base; // element where the tile starts (kShifted: a row's first one, up to seven in front of the row)
+  int lo, hi;   // its steps lo .. hi - 1 exist (hi = 0: no such tile)
   int t;        // number in the line
   int chunk0;   // first chunk inside the row
-  int nc;       // chunks of the row in it (0: no such tile)
+  int nc;       // chunks of the row in it
+  // whether the tile's data have steps of another row among them (kShifted)
+  __device__ __forceinline__ bool cut() const { return lo > 0 || hi < 32 * kT; }
 };
-__device__ __forceinline__ int tile_chunks(const Lines& ln, const Tile& w, int tiles) {
-  return w.t >= 0 && w.t < tiles ? min(static_cast<int>(ln.C) - w.chunk0, 32) : 0;
+template <int ROWS>
+__device__ __forceinline__ void tile_row(const Lines& ln, Tile& w, int tiles) {
+  const int64_t start = w.row * ln.L;
+  const int front = ROWS == kShifted ? static_cast<int>(start & 7) : 0;
+  const int64_t behind = static_cast<int64_t>(w.chunk0) * kT - front;  // steps of the row in front of the tile
+  w.base = start + behind;
+  w.lo = ROWS == kShifted && w.chunk0 == 0 ? front : 0;
+  w.hi = w.t >= 0 && w.t < tiles ? static_cast<int>(max(int64_t{0}, min(ln.L - behind, int64_t{32 * kT}))) : 0;
+  w.nc = (w.hi + kT - 1) / kT;
 }
+template <int ROWS>
 __device__ __forceinline__ Tile tile_at(const Lines& ln, int group, int t) {
   Tile w;
   const bool on = group < ln.groups;
@@ -254,9 +287,10 @@ __device__ __forceinline__ Tile tile_at(const Lines& ln, int group, int t) {
   w.row = on ? static_cast<int64_t>(ln.first_row(group) + b) * ln.D + group % ln.D : 0;
   w.t = t;
   w.chunk0 = (t - b * ln.tpr) * 32;
-  w.nc = on ? tile_chunks(ln, w, ln.tiles(group)) : 0;
+  tile_row<ROWS>(ln, w, on ? ln.tiles(group) : 0);
   return w;
 }
+template <int ROWS>
 __device__ __forceinline__ void tile_forward(const Lines& ln, Tile& w, int tiles) {
   w.t += kWaves;
   w.chunk0 += 32 * kWaves;
@@ -264,8 +298,9 @@ __device__ __forceinline__ void tile_forward(const Lines& ln, Tile& w, int tiles
     w.chunk0 -= 32 * ln.tpr;
     w.row += ln.D;
   }
-  w.nc = tile_chunks(ln, w, tiles);
+  tile_row<ROWS>(ln, w, tiles);
 }
+template <int ROWS>
 __device__ __forceinline__ void tile_backward(const Lines& ln, Tile& w, int tiles) {
   w.t -= kWaves;
   w.chunk0 -= 32 * kWaves;
@@ -273,14 +308,14 @@ __device__ __forceinline__ void tile_backward(const Lines& ln, Tile& w, int tile
     w.chunk0 += 32 * ln.tpr;
     w.row -= ln.D;
   }
-  w.nc = tile_chunks(ln, w, tiles);
+  tile_row<ROWS>(ln, w, tiles);
 }
 
 // LDS traffic of one wave is processed in order: a wave that has written rows
 // and waits for its own LDS operations can read what its other lanes wrote.
 __device__ __forceinline__ void wave_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-template <int DT, bool ANY>
+template <int DT, int ROWS>
 __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
     const void* __restrict__ x, void* __restrict__ y, const float* __restrict__ p,
     const cf* __restrict__ log_q, const cf* __restrict__ gamma, const float* __restrict__ omega,
@@ -291,7 +326,6 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
   Smem& sm = *reinterpret_cast<Smem*>(smem_raw);
   cf (*qp)[kT + 2] = reinterpret_cast<cf(*)[kT + 2]>(sm.H);  // while a row is set up
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-  const int64_t L = ln.L, C = ln.C;
   const int g = lane >> 5, r = lane & 31;
   // scan roles: mode sn; sub-segment sa = 4 wave + sl of CPS chunks, inside the wave's own tiles
   const int sn = tid & 15, sa = tid >> 4, sl = sa & 3;
@@ -300,10 +334,10 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
   // of a group in line.  The x tile of the next item and the parameters of the next group are
   // requested ahead.
   auto load_tile = [&](XOp<DT> (&t)[4], const Tile& w) {
-    const typename Elem<DT>::type* xrow = static_cast<const typename Elem<DT>::type*>(x) + w.row * L;
+    const typename Elem<DT>::type* xrow = static_cast<const typename Elem<DT>::type*>(x) + w.base;
+    const int id = opaque(lane), at = (id & 31) * kT + 8 * (id >> 5);
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
-      t[s].template load<ANY>(xrow, static_cast<int64_t>(w.chunk0 + r) * kT + 16 * s + 8 * g, w.nc > 0, L);
+    for (int s = 0; s < 4; ++s) t[s].template load<ROWS>(xrow, at + 16 * s, w.lo, w.hi);
   };
   struct RowParams {
     cf lq, gv;
@@ -416,12 +450,18 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
   // same registers are reloaded with the next item's tile while the scan and the state part of
   // the outputs run.
   XOp<DT> xb[4];
-  Tile cur_tile = tile_at(ln, blockIdx.x, wave);  // this wave's tile of the item
+  Tile cur_tile = tile_at<ROWS>(ln, blockIdx.x, wave);  // this wave's tile of the item
   auto item = [&](int group, int t0, int tiles) {
     if (t0 == 0) setup_row(group);
     const Tile w = cur_tile;
-    typename Elem<DT>::type* yrow = static_cast<typename Elem<DT>::type*>(y) + w.row * L;
+    typename Elem<DT>::type* yrow = static_cast<typename Elem<DT>::type*>(y) + w.base;
     const int c0 = wave * 32;
+    if constexpr (ROWS == kShifted)
+      if (w.cut()) {
+        const int id = opaque(lane), at = (id & 31) * kT + 8 * (id >> 5);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) xb[s].keep(at + 16 * s, w.lo, w.hi);
+      }
     floatx16 yacc[2];
     // ---- local states S = P X, into this wave's own rows of the state buffer ----------
     {
@@ -458,8 +498,8 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
       }
     }
     {
-      if (t0 + kWaves < tiles) tile_forward(ln, cur_tile, tiles);
-      else cur_tile = tile_at(ln, group + static_cast<int>(gridDim.x), wave);
+      if (t0 + kWaves < tiles) tile_forward<ROWS>(ln, cur_tile, tiles);
+      else cur_tile = tile_at<ROWS>(ln, group + static_cast<int>(gridDim.x), wave);
       load_tile(xb, cur_tile);
     }
     wave_sync();
@@ -528,7 +568,7 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
           const float v[8] = {u.x, u.y, u.z, u.w, u1.x, u1.y, u1.z, u1.w};
           split8(v, hb[s2][0], hb[s2][1]);
         }
-        const int64_t chunk = w.chunk0 + r;
+        const int id = opaque(lane), at = (id & 31) * kT, ag = id >> 5;
 #pragma unroll
         for (int it = 0; it < 2; ++it) {
           floatx16 acc = yacc[it];
@@ -545,14 +585,14 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
               // per lane, no exchange between the halves of the wave
 #pragma unroll
               for (int h = 0; h < 2; ++h) {
-                const int64_t elem = chunk * kT + 16 * (2 * it + pr) + 8 * h + 4 * g;
-                if (elem + 4 <= L)
+                const int elem = at + 16 * (2 * it + pr) + 8 * h + 4 * ag;
+                if (elem < w.hi)
                   *reinterpret_cast<float4*>(yrow + elem) = make_float4(acc[8 * pr + 4 * h], acc[8 * pr + 4 * h + 1],
                                                                         acc[8 * pr + 4 * h + 2], acc[8 * pr + 4 * h + 3]);
               }
             } else {
               const uint4 oct = octet_of<DT>(acc, pr);
-              store8_16<ANY>(yrow, chunk * kT + 16 * (2 * it + pr) + 8 * g, L, oct);
+              store8_16<ROWS>(yrow, at + 16 * (2 * it + pr) + 8 * ag, w.lo, w.hi, oct);
             }
           }
         }
@@ -560,11 +600,11 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
     }
     cur ^= 1;
     par ^= 1;
-    if (w.nc > 0 && w.chunk0 + 32 >= static_cast<int>(C) && h_last != nullptr && lane < N) {
+    if (w.hi > 0 && w.base + w.hi == (w.row + 1) * ln.L && h_last != nullptr && lane < N) {
       // the state after step L - 1 (the row's last chunk may be partial), from this wave's own rows
-      const typename Elem<DT>::type* xrow = static_cast<const typename Elem<DT>::type*>(x) + w.row * L;
-      const int rem = static_cast<int>(L - (C - 1) * kT);  // 1 .. 64 steps in the last chunk
-      const int cl = w.nc - 1;                             // the last chunk inside the tile
+      const typename Elem<DT>::type* xrow = static_cast<const typename Elem<DT>::type*>(x) + w.base;
+      const int cl = w.nc - 1;           // the last chunk inside the tile
+      const int rem = w.hi - cl * kT;    // 1 .. 64 steps in it
       cf h;
       if (rem == kT) {
         const float* lastrow = sm.H + (1 + c0 + cl) * kHP + 2 * lane;
@@ -576,8 +616,8 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
         h = cf{prev[0], prev[1]};
         const cf q1 = sm.pw[8][lane];
         const float pp = sm.pn[lane];
-        for (int j = 0; j < rem; ++j) {
-          const float xv = Elem<DT>::load(xrow + (C - 1) * kT + j) * pp;
+        for (int j = cl == 0 ? w.lo : 0; j < rem; ++j) {
+          const float xv = Elem<DT>::load(xrow + cl * kT + j) * pp;
           h = cmul(q1, h);
           h.x += xv;
         }
@@ -595,7 +635,7 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
 
 // How many rows of a channel a group takes: as many as leave `slots` groups, so that a small
 // launch still fills the chip.
-Lines make_lines(int64_t B, int64_t D, int64_t L, int64_t slots, bool single) {
+Lines make_lines(int64_t B, int64_t D, int64_t L, int64_t slots, bool single, int rows) {
   Lines ln;
   int64_t nb = single ? 1 : B * D / slots;
   nb = nb < 1 ? 1 : (nb > B ? B : nb);
@@ -604,8 +644,8 @@ Lines make_lines(int64_t B, int64_t D, int64_t L, int64_t slots, bool single) {
   ln.nb = static_cast<int>(nb);
   ln.groups = static_cast<int>(D * ((B + nb - 1) / nb));
   ln.L = L;
-  ln.C = (L + kT - 1) / kT;
-  ln.tpr = static_cast<int>((ln.C + 31) / 32);
+  const int64_t chunks = (L + (rows == kShifted ? 7 : 0) + kT - 1) / kT;  // of a row with steps in front of it
+  ln.tpr = static_cast<int>((chunks + 31) / 32);
   return ln;
 }
 int compute_units(int* cus) {
@@ -615,20 +655,20 @@ int compute_units(int* cus) {
   return MEGA_OK;
 }
 
-template <int DT, bool ANY>
+template <int DT, int ROWS>
 int launch_fwd(const void* x, void* y, const float* p, const cf* log_q, const cf* gamma,
                const float* omega, const cf* h0, cf* h_last, int64_t B, int64_t D, int64_t N,
                int64_t L, hipStream_t stream) {
   const size_t lds = sizeof(FwdSmem);
-  MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cema_scan_fwd_kernel<DT, ANY>),
+  MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cema_scan_fwd_kernel<DT, ROWS>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
   int cus = 0;
   const int rc = compute_units(&cus);
   if (rc != MEGA_OK) return rc;
   const int64_t slots = 3 * static_cast<int64_t>(cus);  // workgroups that fit the chip
-  const Lines ln = make_lines(B, D, L, slots, false);
+  const Lines ln = make_lines(B, D, L, slots, false, ROWS);
   const unsigned grid = static_cast<unsigned>(ln.groups < slots ? ln.groups : slots);
-  cema_scan_fwd_kernel<DT, ANY><<<dim3(grid), kThreads, lds, stream>>>(x, y, p, log_q, gamma, omega, h0, h_last, ln,
+  cema_scan_fwd_kernel<DT, ROWS><<<dim3(grid), kThreads, lds, stream>>>(x, y, p, log_q, gamma, omega, h0, h_last, ln,
                                                                        static_cast<int>(N));
   MEGA_CHECK_LAUNCH();
   return MEGA_OK;
@@ -703,7 +743,7 @@ __device__ __forceinline__ void rstep(cf& h, cf& hd, cf g, cf gd, cf m, cf md) {
 // DX32: dx is written in float32 (or, with a null pointer, not at all) instead of the rows'
 // own type -- for callers that add up the backward of several bfloat16 pieces of one tensor;
 // DX32 == 2 adds to what dx holds instead of overwriting it.
-template <int DT, int DX32, bool ANY>
+template <int DT, int DX32, int ROWS>
 __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
     const void* __restrict__ dy, const void* __restrict__ x, void* __restrict__ dx,
     const float* __restrict__ p, const cf* __restrict__ log_q, const cf* __restrict__ gamma,
@@ -711,7 +751,6 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
     cf* __restrict__ dgamma, float* __restrict__ domega, cf* __restrict__ dh0, const Lines ln, int N) {
   static_assert(XOp<DT>::XP == 1, "the backward kernel takes bfloat16 rows");
   constexpr int CPS = kBwdCPS;
-  const int64_t L = ln.L;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   BwdSmem& sm = *reinterpret_cast<BwdSmem*>(smem_raw);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -731,17 +770,17 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
   XOp<DT> db[4], xb[4], dn[4];  // dn: the next item's dy tile on its way
   auto load_dy = [&](const Tile& w) {
     MEGA_LANE_IDS;
-    const uint16_t* row = static_cast<const uint16_t*>(dy) + w.row * L;
+    const uint16_t* row = static_cast<const uint16_t*>(dy) + w.base;
 #pragma unroll
     for (int s = 0; s < 4; ++s)
-      dn[s].template load<ANY>(row, static_cast<int64_t>(w.chunk0 + r) * kT + 16 * s + 8 * g, w.nc > 0, L);
+      dn[s].template load<ROWS>(row, r * kT + 16 * s + 8 * g, w.lo, w.hi);
   };
   auto load_x = [&](const Tile& w) {
     MEGA_LANE_IDS;
-    const uint16_t* row = static_cast<const uint16_t*>(x) + w.row * L;
+    const uint16_t* row = static_cast<const uint16_t*>(x) + w.base;
 #pragma unroll
     for (int s = 0; s < 4; ++s)
-      xb[s].template load<ANY>(row, static_cast<int64_t>(w.chunk0 + r) * kT + 16 * s + 8 * g, w.nc > 0, L);
+      xb[s].template load<ROWS>(row, r * kT + 16 * s + 8 * g, w.lo, w.hi);
   };
   struct RowParams {
     cf lq, gv;
@@ -1002,7 +1041,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
     if (tid == 0) domega[row] = sm.dkin[0];
   };
 
-  Tile cur_tile = tile_at(ln, blockIdx.x, tail_of(blockIdx.x) + wave);  // this wave's tile of the item
+  Tile cur_tile = tile_at<ROWS>(ln, blockIdx.x, tail_of(blockIdx.x) + wave);  // this wave's tile of the item
   auto item = [&](int group, int t0, int tiles) {
     MEGA_LANE_IDS;
     // transposing read of the parked tile: row tile tt (32 time steps), k-step ks (16 chunks)
@@ -1015,22 +1054,25 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
     if (t0 + kWaves >= tiles) setup_row(group);
     const Tile w = cur_tile;
     using dx_t = typename std::conditional<DX32 != 0, float, uint16_t>::type;
-    dx_t* dxrow = static_cast<dx_t*>(dx) + w.row * L;
+    dx_t* dxrow = static_cast<dx_t*>(dx) + w.base;
     const bool on = w.nc > 0;
     u32x4 xr[4];  // time-reversed x as an operand: steps 63 - (16 s + 8 g + e)
     // the next item of this workgroup: its x tile is requested as soon as this item's has been
     // consumed, its dy tile at the end of the item
     Tile next = w;
     if (t0 > 0) {
-      tile_backward(ln, next, tiles);
+      tile_backward<ROWS>(ln, next, tiles);
     } else {
       const int ng = group + static_cast<int>(gridDim.x);
-      next = tile_at(ln, ng, tail_of(ng) + wave);
+      next = tile_at<ROWS>(ln, ng, tail_of(ng) + wave);
     }
     if (on) {
       // ---- the wave's private tile: X parked first (it arrived an item ago), read back with
       //      chunks along k and time-reversed; then DY, whose loads were issued last ------------
       uint16_t* mine = stage + r * kSP + 8 * g;
+      if (ROWS == kShifted && w.cut())
+#pragma unroll
+        for (int s = 0; s < 4; ++s) xb[s].keep(r * kT + 16 * s + 8 * g, w.lo, w.hi);
 #pragma unroll
       for (int s = 0; s < 4; ++s) *reinterpret_cast<u32x4*>(mine + 16 * s) = xb[s].pc[0];
       wave_sync();
@@ -1046,6 +1088,9 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
         for (int e = 0; e < 4; ++e) xr[s][e] = __builtin_amdgcn_alignbit(v[3 - e], v[3 - e], 16);
       }
       wave_sync();
+      if (ROWS == kShifted && w.cut())
+#pragma unroll
+        for (int s = 0; s < 4; ++s) db[s].keep(r * kT + 16 * s + 8 * g, w.lo, w.hi);
 #pragma unroll
       for (int s = 0; s < 4; ++s) *reinterpret_cast<u32x4*>(mine + 16 * s) = db[s].pc[0];
       wave_sync();
@@ -1175,7 +1220,6 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
         const float v[8] = {ua.x, ua.y, ua.z, ua.w, ub.x, ub.y, ub.z, ub.w};
         split8(v, hb[s2][0], hb[s2][1]);
       }
-      const int64_t chunk = w.chunk0 + r;
 #pragma unroll
       for (int jt = 0; jt < 2; ++jt) {
         floatx16 acc;
@@ -1201,9 +1245,8 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
             // registers 8 pr + 4 h + e hold the steps 16 pr + 8 h + 4 g + e
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-              const int64_t elem = chunk * kT + 16 * (2 * jt + pr) + 8 * h + 4 * g;
-              // (rows of any length: element by element -- the float32 sum of pieces is not the hot path)
-              if (!ANY && dx != nullptr && elem + 4 <= L) {
+              const int elem = r * kT + 16 * (2 * jt + pr) + 8 * h + 4 * g;
+              if (dx != nullptr && ROWS != kAny && (ROWS == kWhole || elem >= w.lo) && elem + 4 <= w.hi) {
                 float4 v = make_float4(acc[8 * pr + 4 * h], acc[8 * pr + 4 * h + 1], acc[8 * pr + 4 * h + 2],
                                        acc[8 * pr + 4 * h + 3]);
                 if constexpr (DX32 == 2) {
@@ -1211,15 +1254,16 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
                   v = make_float4(v.x + o.x, v.y + o.y, v.z + o.z, v.w + o.w);
                 }
                 *reinterpret_cast<float4*>(dxrow + elem) = v;
-              } else if (ANY && dx != nullptr) {
+              } else if (ROWS != kWhole && dx != nullptr) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                  if (elem + e < L) dxrow[elem + e] = acc[8 * pr + 4 * h + e] + (DX32 == 2 ? static_cast<float>(dxrow[elem + e]) : 0.f);
+                  if (elem + e >= w.lo && elem + e < w.hi)
+                    dxrow[elem + e] = acc[8 * pr + 4 * h + e] + (DX32 == 2 ? static_cast<float>(dxrow[elem + e]) : 0.f);
               }
             }
           } else {
             const uint4 oct = octet_of<DT>(acc, pr);
-            store8_16<ANY>(dxrow, chunk * kT + 16 * (2 * jt + pr) + 8 * g, L, oct);
+            store8_16<ROWS>(dxrow, r * kT + 16 * (2 * jt + pr) + 8 * g, w.lo, w.hi, oct);
           }
         }
       }
@@ -1277,32 +1321,48 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
 }
 
 // Rows of a channel that the backward puts together (make_lines); a carried state's gradients are per row.
-int bwd_lines(int64_t B, int64_t D, int64_t L, bool single, Lines* ln, int64_t* slots) {
+int bwd_lines(int64_t B, int64_t D, int64_t L, bool single, int rows, Lines* ln, int64_t* slots) {
   int cus = 0;
   const int rc = compute_units(&cus);
   if (rc != MEGA_OK) return rc;
   *slots = 2 * static_cast<int64_t>(cus);  // two workgroups fit a compute unit
-  *ln = make_lines(B, D, L, *slots, single);
+  *ln = make_lines(B, D, L, *slots, single, rows);
   return MEGA_OK;
 }
 
 // single: gradients per row (B, D, N) as the operator returns them; else per group of rows
-template <int DX32, bool ANY>
+template <int DX32, int ROWS>
 int launch_bwd(const void* dy, const void* x, void* dx, const float* p, const cf* log_q,
                const cf* gamma, const float* omega, const cf* h0, float* dp, cf* dq, cf* dgamma, float* domega,
                cf* dh0, int64_t B, int64_t D, int64_t N, int64_t L, bool single, hipStream_t stream) {
   const int lds = static_cast<int>(sizeof(BwdSmem));
-  MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cema_scan_bwd_kernel<MEGA_BF16, DX32, ANY>),
+  MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cema_scan_bwd_kernel<MEGA_BF16, DX32, ROWS>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds));
   Lines ln;
   int64_t slots = 0;
-  const int rc = bwd_lines(B, D, L, single || h0 != nullptr, &ln, &slots);
+  const int rc = bwd_lines(B, D, L, single || h0 != nullptr, ROWS, &ln, &slots);
   if (rc != MEGA_OK) return rc;
   const unsigned grid = static_cast<unsigned>(ln.groups < slots ? ln.groups : slots);
-  cema_scan_bwd_kernel<MEGA_BF16, DX32, ANY><<<dim3(grid), kThreads, lds, stream>>>(
+  cema_scan_bwd_kernel<MEGA_BF16, DX32, ROWS><<<dim3(grid), kThreads, lds, stream>>>(
       dy, x, dx, p, log_q, gamma, omega, h0, dp, dq, dgamma, domega, dh0, ln, static_cast<int>(N));
   MEGA_CHECK_LAUNCH();
   return MEGA_OK;
+}
+
+using BwdLaunch = decltype(&launch_bwd<0, kWhole>);
+BwdLaunch bwd_for(int dx_mode, int rows) {
+  static const BwdLaunch table[3][3] = {{launch_bwd<0, kWhole>, launch_bwd<0, kShifted>, launch_bwd<0, kAny>},
+                                        {launch_bwd<1, kWhole>, launch_bwd<1, kShifted>, launch_bwd<1, kAny>},
+                                        {launch_bwd<2, kWhole>, launch_bwd<2, kShifted>, launch_bwd<2, kAny>}};
+  return table[dx_mode][rows];
+}
+
+// the layout of rows of length L in these tensors
+int rows_of(int64_t count, int64_t L, bool carried, std::initializer_list<const void*> tensors) {
+  for (const void* t : tensors)
+    if (reinterpret_cast<uintptr_t>(t) % 16 != 0) return kAny;
+  // (a tensor whose end is off a boundary too: the last row's aligned piece would reach past it)
+  return L % 8 == 0 ? kWhole : carried || count * L % 8 != 0 ? kAny : kShifted;
 }
 
 }  // namespace
@@ -1327,20 +1387,22 @@ extern "C" int mega_cema_scan_fwd(const void* x, int dtype, const float* p, cons
     return set_error(MEGA_ERR_UNSUPPORTED,
                      "%s: needs N <= 16 and, for float32 rows, L a multiple of 8 (dtype %d, N %lld, L %lld)",
                      who, dtype, (long long)N, (long long)L);
-  const bool any = L % 8 != 0 || reinterpret_cast<uintptr_t>(x) % 16 != 0 || reinterpret_cast<uintptr_t>(y) % 16 != 0;
-  MEGA_CHECK_ARG(!any || dtype != MEGA_F32, "%s: float32 rows must be 16-byte aligned", who);
+  const int rows = rows_of(B * D, L, h0 != nullptr, {x, y});
+  MEGA_CHECK_ARG(rows == kWhole || dtype != MEGA_F32, "%s: float32 rows must be 16-byte aligned", who);
   if (B == 0 || D == 0) return MEGA_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const cf* lq = reinterpret_cast<const cf*>(log_q);
   const cf* gm = reinterpret_cast<const cf*>(gamma);
   const cf* h0c = reinterpret_cast<const cf*>(h0);
   cf* hl = reinterpret_cast<cf*>(h_last);
-  if (dtype == MEGA_F32) return launch_fwd<MEGA_F32, false>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s);
-  if (dtype == MEGA_BF16)
-    return any ? launch_fwd<MEGA_BF16, true>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s)
-               : launch_fwd<MEGA_BF16, false>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s);
-  return any ? launch_fwd<MEGA_F16, true>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s)
-             : launch_fwd<MEGA_F16, false>(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s);
+  auto go = dtype == MEGA_F32     ? launch_fwd<MEGA_F32, kWhole>
+            : dtype == MEGA_BF16 ? (rows == kWhole     ? launch_fwd<MEGA_BF16, kWhole>
+                                    : rows == kShifted ? launch_fwd<MEGA_BF16, kShifted>
+                                                       : launch_fwd<MEGA_BF16, kAny>)
+                                 : (rows == kWhole     ? launch_fwd<MEGA_F16, kWhole>
+                                    : rows == kShifted ? launch_fwd<MEGA_F16, kShifted>
+                                                       : launch_fwd<MEGA_F16, kAny>);
+  return go(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s);
 }
 
 extern "C" int mega_cema_scan_bwd_supported(int dtype, int64_t N, int64_t L) {
@@ -1360,11 +1422,9 @@ extern "C" int mega_cema_scan_bwd_state(const void* dy, const void* x, int dtype
     return set_error(MEGA_ERR_UNSUPPORTED,
                      "%s: needs bfloat16 rows and N <= 16 (dtype %d, N %lld, L %lld)", who,
                      dtype, (long long)N, (long long)L);
-  const auto al = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
-  const bool any = L % 8 != 0 || !al(dy) || !al(x) || !al(dx);
   if (B == 0 || D == 0) return MEGA_OK;
   MEGA_CHECK_ARG(dh0 == nullptr || h0 != nullptr, "%s: dh0 without h0", who);
-  return (any ? launch_bwd<0, true> : launch_bwd<0, false>)(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma),
+  return bwd_for(0, rows_of(B * D, L, h0 != nullptr, {dy, x, dx}))(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma),
                            omega, reinterpret_cast<const cf*>(h0), dp, reinterpret_cast<cf*>(dq),
                            reinterpret_cast<cf*>(dgamma), domega, reinterpret_cast<cf*>(dh0), B, D, N, L, true,
                            static_cast<hipStream_t>(stream));
@@ -1389,16 +1449,14 @@ extern "C" int mega_cema_scan_bwd_wide(const void* dy, const void* x, const floa
   if (!mega_cema_scan_bwd_supported(MEGA_BF16, N, L))
     return set_error(MEGA_ERR_UNSUPPORTED, "%s: needs N <= 16 (N %lld, L %lld)", who,
                      (long long)N, (long long)L);
-  const auto al = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
-  const bool any = L % 8 != 0 || !al(dy) || !al(x) || !al(dx);
   if (B == 0 || D == 0) return MEGA_OK;
   MEGA_CHECK_ARG(dh0 == nullptr || h0 != nullptr, "%s: dh0 without h0", who);
   if (accumulate_dx && dx != nullptr)
-    return (any ? launch_bwd<2, true> : launch_bwd<2, false>)(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma),
+    return bwd_for(2, rows_of(B * D, L, h0 != nullptr, {dy, x, dx}))(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma),
                          omega, reinterpret_cast<const cf*>(h0), dp, reinterpret_cast<cf*>(dq),
                          reinterpret_cast<cf*>(dgamma), domega, reinterpret_cast<cf*>(dh0), B, D, N, L, true,
                          static_cast<hipStream_t>(stream));
-  return (any ? launch_bwd<1, true> : launch_bwd<1, false>)(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma),
+  return bwd_for(1, rows_of(B * D, L, h0 != nullptr, {dy, x, dx}))(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma),
                        omega, reinterpret_cast<const cf*>(h0), dp, reinterpret_cast<cf*>(dq),
                        reinterpret_cast<cf*>(dgamma), domega, reinterpret_cast<cf*>(dh0), B, D, N, L, true,
                        static_cast<hipStream_t>(stream));
@@ -1407,7 +1465,7 @@ extern "C" int mega_cema_scan_bwd_wide(const void* dy, const void* x, const floa
 extern "C" int64_t mega_cema_layer_scan_sets(int64_t B, int64_t D, int64_t L) {
   Lines ln;
   int64_t slots = 0;
-  if (B < 1 || D < 1 || L < 1 || bwd_lines(B, D, L, false, &ln, &slots) != MEGA_OK) return 0;
+  if (B < 1 || D < 1 || L < 1 || bwd_lines(B, D, L, false, kWhole, &ln, &slots) != MEGA_OK) return 0;
   return ln.groups / ln.D;
 }
 
@@ -1421,12 +1479,7 @@ extern "C" int mega_cema_layer_scan_bwd(const void* dy, const void* x, const flo
   MEGA_CHECK_ARG(dx_mode >= 0 && dx_mode <= 2 && (dx != nullptr || dx_mode == 1), "%s: bad dx", who);
   if (!mega_cema_scan_bwd_supported(MEGA_BF16, N, L))
     return set_error(MEGA_ERR_UNSUPPORTED, "%s: needs N <= 16 (N %lld, L %lld)", who, (long long)N, (long long)L);
-  const auto al = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
-  const bool any = L % 8 != 0 || !al(dy) || !al(x) || !al(dx);
-  auto go = dx_mode == 0   ? (any ? launch_bwd<0, true> : launch_bwd<0, false>)
-            : dx_mode == 1 ? (any ? launch_bwd<1, true> : launch_bwd<1, false>)
-                           : (any ? launch_bwd<2, true> : launch_bwd<2, false>);
-  return go(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma), omega, nullptr, dp,
+  return bwd_for(dx_mode, rows_of(B * D, L, false, {dy, x, dx}))(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma), omega, nullptr, dp,
             reinterpret_cast<cf*>(dq), reinterpret_cast<cf*>(dgamma), domega, nullptr, B, D, N, L, false,
             static_cast<hipStream_t>(stream));
 }

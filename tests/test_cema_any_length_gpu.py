@@ -30,6 +30,8 @@ class _picked:
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,D,L,offset", [(1, 2, 1, 0), (2, 3, 7, 0), (2, 2, 9, 1), (1, 3, 65, 0), (2, 3, 1021, 0),
                                           (1, 2, 2047, 0), (1, 3, 4096, 3), (2, 2, 8193, 0), (1, 2, 20003, 5),
+                                          # whole tensors of 16-byte pieces, rows taken from the boundary in front
+                                          (8, 1, 1, 0), (1, 8, 57, 0), (1, 8, 65, 0), (2, 8, 2043, 0), (1, 8, 20003, 0),
                                           # several rows of a channel in one workgroup: two, two and one; five, of two tiles each
                                           (5, 300, 130, 0), (5, 520, 2049, 1)])
 def test_layer_matches_oracle(B, D, L, offset, dtype):
