@@ -534,7 +534,7 @@ int mega_layer_norm_bwd(const void* dy, const void* x, const void* weight, const
  *   88-90,113-114).
  *   z, q, k (rows, S) of `dtype` (bfloat16 / float16), rows = batch * L; gamma,
  *   beta (2, S) of `dtype` as the module stores them; heads of Dh elements,
- *   Dh in {64, 128, 256, 512}, S in {512, 1024, 2048, 4096}.  `freqs`: (P, Dh/2)
+ *   Dh in {64, 128, 256, 512}, S a power of two from 64 to 4096.  `freqs`: (P, Dh/2)
  *   complex numbers as float32 pairs (cos, sin), or null for no rotary; row r
  *   uses position (r % L) % P (P = chunk length, or L for a shorter piece).
  *   rstd (rows, S / Dh) float32 is saved for the backward.  All buffers 16-byte

@@ -303,25 +303,41 @@ __global__ __launch_bounds__(kThreads) void norm_bwd_any_kernel(NormParams p, in
   }
 }
 
-// out[c] = sum over `groups` rows (`stride` floats apart) of part[., c], c < D:
-// 64 columns x 16 row slices per workgroup
+// out[c] = sum over `groups` rows (`stride` floats apart) of part[., c], c < D, for one or two
+// (part, out) pairs: 16 columns x 64 row slices per workgroup, so that the few columns of a norm
+// still occupy a workgroup per 64 bytes of a row and a thread has all its loads in flight.
+// (1024 rows of 4096 columns, two sums: PG_BEFORE with 64 columns x 16 slices and a launch each.)
+struct ColumnSums {
+  const float* part[2];
+  void* out[2];
+};
 template <int DT>
-__global__ __launch_bounds__(1024) void norm_param_grad_kernel(const float* part, int groups, int D,
-                                                              int stride, typename Elem<DT>::type* out) {
-  __shared__ float red[16][65];
-  const int cx = threadIdx.x % 64, sy = threadIdx.x / 64;
-  const int c = blockIdx.x * 64 + cx;
+__global__ __launch_bounds__(1024) void norm_param_grad_kernel(ColumnSums t, int groups, int D, int stride) {
+  __shared__ float red[16][17];
+  const int cx = threadIdx.x % 16, sy = threadIdx.x / 16, wave = threadIdx.x / kWave;
+  const int c = blockIdx.x * 16 + cx;
+  const float* part = t.part[blockIdx.y];
   float s = 0.f;
-  if (c < D)
-    for (int gidx = sy; gidx < groups; gidx += 16) s += part[static_cast<int64_t>(gidx) * stride + c];
-  red[sy][cx] = s;
-  __syncthreads();
-  if (sy == 0 && c < D) {
-    float t = 0.f;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) t += red[v][cx];
-    Elem<DT>::store(out + c, t);
+  if (c < D) {
+#pragma unroll 8
+    for (int gidx = sy; gidx < groups; gidx += 64) s += part[static_cast<int64_t>(gidx) * stride + c];
   }
+  s += __shfl_xor(s, 16);
+  s += __shfl_xor(s, 32);
+  if (threadIdx.x % kWave < 16) red[wave][cx] = s;
+  __syncthreads();
+  if (threadIdx.x < 16 && c < D) {
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) v += red[w][cx];
+    Elem<DT>::store(static_cast<typename Elem<DT>::type*>(t.out[blockIdx.y]) + c, v);
+  }
+}
+template <int DT>
+int launch_param_grad(const ColumnSums& t, int groups, int D, int stride, hipStream_t s) {
+  norm_param_grad_kernel<DT><<<dim3((D + 15) / 16, t.part[1] != nullptr ? 2 : 1), 1024, 0, s>>>(t, groups, D, stride);
+  MEGA_CHECK_LAUNCH();
+  return MEGA_OK;
 }
 
 
@@ -332,8 +348,9 @@ __global__ __launch_bounds__(1024) void norm_param_grad_kernel(const float* part
 // megalodon/modules/rotary_positional_embedding.py:53-77 on both: neighbouring
 // elements (2i, 2i+1) of a head are one complex number that is multiplied by
 // freqs[p][i], p = (row % L) % P the position inside the chunk.  One wavefront
-// holds a row of S = 512 * NCH elements, G = Dh / 8 lanes per head; z is read
-// once and q, k are written once.  The backward undoes the rotation with the
+// holds a row of S = 512 * NCH elements, or 512 / S rows of 64, 128 or 256 (one narrow head
+// each: left to the PyTorch expressions they are some 65 small launches per training step,
+// QK_NARROW), G = Dh / 8 lanes per head; z is read once and q, k are written once.  The backward undoes the rotation with the
 // conjugate factor, forms the gradients of the affine parameters as column
 // sums (per-workgroup partials, reduced in a fixed order afterwards) and the
 // RMSNorm gradient per head.
@@ -353,6 +370,14 @@ struct QkParams {
   float eps, inv_sqrt_dh;
 };
 
+// Where a lane's 16-byte pieces lie: lanes per row, the row among those of the wavefront.
+struct QkLane {
+  int lpr, slot, col;
+  __device__ __forceinline__ QkLane(int S, int lane)
+      : lpr(S < 512 ? S / 8 : kWave), slot(lane / lpr), col((lane - slot * lpr) * 8) {}
+  __device__ __forceinline__ int rows() const { return kWave / lpr; }
+};
+
 __device__ __forceinline__ void rotate8(float* u, const float4& f0, const float4& f1, bool conj) {
   const float c[4] = {f0.x, f0.z, f1.x, f1.z};
   const float sn[4] = {f0.y, f0.w, f1.y, f1.w};
@@ -369,29 +394,32 @@ template <int DT, int G, int NCH>
 __global__ __launch_bounds__(kThreads) void qk_fwd_kernel(QkParams p) {
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int heads = p.S / p.Dh;
+  const QkLane at(p.S, lane);
   const float inv_dh = 1.f / static_cast<float>(p.Dh);
   uint4 gq[NCH], gk[NCH], bq[NCH], bk[NCH];
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
-    const int c = (lane + kWave * i) * 8;
+    const int c = at.col + kWave * 8 * i;
     gq[i] = *reinterpret_cast<const uint4*>(p.gamma + c);
     gk[i] = *reinterpret_cast<const uint4*>(p.gamma + p.S + c);
     bq[i] = *reinterpret_cast<const uint4*>(p.beta + c);
     bk[i] = *reinterpret_cast<const uint4*>(p.beta + p.S + c);
   }
-  for (int64_t row = static_cast<int64_t>(blockIdx.x) * kWaves + wave; row < p.rows;
-       row += static_cast<int64_t>(gridDim.x) * kWaves) {
+  for (int64_t first = (static_cast<int64_t>(blockIdx.x) * kWaves + wave) * at.rows(); first < p.rows;
+       first += static_cast<int64_t>(gridDim.x) * kWaves * at.rows()) {
+    const bool on = first + at.slot < p.rows;  // the last wavefront's spare lanes take its first row
+    const int64_t row = on ? first + at.slot : first;
     const int pos = static_cast<int>(row % p.L) % p.P;
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
-      const int c = (lane + kWave * i) * 8;
+      const int c = at.col + kWave * 8 * i;
       float v[8], uq[8], uk[8], g[8], b[8];
       unpack8<DT>(*reinterpret_cast<const uint4*>(p.z + row * p.S + c), v);
       float ss = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
       const float r = rsqrtf(group_sum<G>(ss) * inv_dh + p.eps);
-      if (lane % G == 0) p.rstd[row * heads + c / p.Dh] = r;
+      if (on && lane % G == 0) p.rstd[row * heads + c / p.Dh] = r;
       opaque(gq[i]); opaque(bq[i]); opaque(gk[i]); opaque(bk[i]);
       unpack8<DT>(gq[i], g);
       unpack8<DT>(bq[i], b);
@@ -407,8 +435,10 @@ __global__ __launch_bounds__(kThreads) void qk_fwd_kernel(QkParams p) {
         rotate8(uq, f0, f1, false);
         rotate8(uk, f0, f1, false);
       }
-      *reinterpret_cast<uint4*>(p.q + row * p.S + c) = pack8<DT>(uq);
-      *reinterpret_cast<uint4*>(p.k + row * p.S + c) = pack8<DT>(uk);
+      if (on) {
+        *reinterpret_cast<uint4*>(p.q + row * p.S + c) = pack8<DT>(uq);
+        *reinterpret_cast<uint4*>(p.k + row * p.S + c) = pack8<DT>(uk);
+      }
     }
   }
 }
@@ -418,27 +448,34 @@ __global__ __launch_bounds__(kThreads) void qk_bwd_kernel(QkParams p) {
   extern __shared__ float acc[];  // 4 S floats
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int heads = p.S / p.Dh;
+  const QkLane at(p.S, lane);
   const float inv_dh = 1.f / static_cast<float>(p.Dh);
   uint4 gq[NCH], gk[NCH];
   float a_gq[NCH][8], a_gk[NCH][8], a_bq[NCH][8], a_bk[NCH][8];
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
-    const int c = (lane + kWave * i) * 8;
+    const int c = at.col + kWave * 8 * i;
     gq[i] = *reinterpret_cast<const uint4*>(p.gamma + c);
     gk[i] = *reinterpret_cast<const uint4*>(p.gamma + p.S + c);
 #pragma unroll
     for (int e = 0; e < 8; ++e) a_gq[i][e] = 0.f, a_gk[i][e] = 0.f, a_bq[i][e] = 0.f, a_bk[i][e] = 0.f;
   }
-  for (int64_t row = static_cast<int64_t>(blockIdx.x) * kWaves + wave; row < p.rows;
-       row += static_cast<int64_t>(gridDim.x) * kWaves) {
+  for (int64_t first = (static_cast<int64_t>(blockIdx.x) * kWaves + wave) * at.rows(); first < p.rows;
+       first += static_cast<int64_t>(gridDim.x) * kWaves * at.rows()) {
+    const bool on = first + at.slot < p.rows;  // the last wavefront's spare lanes take its first row
+    const int64_t row = on ? first + at.slot : first;
     const int pos = static_cast<int>(row % p.L) % p.P;
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
-      const int c = (lane + kWave * i) * 8;
+      const int c = at.col + kWave * 8 * i;
       float zn[8], dq[8], dk[8], g[8], dzn[8];
       unpack8<DT>(*reinterpret_cast<const uint4*>(p.z + row * p.S + c), zn);
       unpack8<DT>(*reinterpret_cast<const uint4*>(p.dq + row * p.S + c), dq);
       unpack8<DT>(*reinterpret_cast<const uint4*>(p.dk + row * p.S + c), dk);
+      if (!on) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dq[e] = dk[e] = 0.f;
+      }
       const float r = p.rstd[row * heads + c / p.Dh];
       if (p.freqs) {
         const float4* f = reinterpret_cast<const float4*>(p.freqs + (static_cast<int64_t>(pos) * p.Dh + c % p.Dh));
@@ -467,17 +504,27 @@ __global__ __launch_bounds__(kThreads) void qk_bwd_kernel(QkParams p) {
       s = group_sum<G>(s) * inv_dh;
 #pragma unroll
       for (int e = 0; e < 8; ++e) dzn[e] = r * (dzn[e] - zn[e] * s);
-      *reinterpret_cast<uint4*>(p.q + row * p.S + c) = pack8<DT>(dzn);
+      if (on) *reinterpret_cast<uint4*>(p.q + row * p.S + c) = pack8<DT>(dzn);
     }
   }
+  // the rows of a wavefront onto its first one's lanes
+  if constexpr (NCH == 1)
+    for (int off = at.lpr; off < kWave; off *= 2)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        a_gq[0][e] += __shfl_xor(a_gq[0][e], off);
+        a_gk[0][e] += __shfl_xor(a_gk[0][e], off);
+        a_bq[0][e] += __shfl_xor(a_bq[0][e], off);
+        a_bk[0][e] += __shfl_xor(a_bk[0][e], off);
+      }
   // column sums of this workgroup, wave by wave in a fixed order
   for (int w = 0; w < kWaves; ++w) {
-    if (wave == w) {
+    if (wave == w && at.slot == 0) {
 #pragma unroll
       for (int i = 0; i < NCH; ++i)
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const int c = (lane + kWave * i) * 8 + e;
+          const int c = at.col + kWave * 8 * i + e;
           const float vg0 = a_gq[i][e] * p.inv_sqrt_dh, vg1 = a_gk[i][e] * p.inv_sqrt_dh;
           if (w == 0) {
             acc[c] = vg0; acc[p.S + c] = vg1; acc[2 * p.S + c] = a_bq[i][e]; acc[3 * p.S + c] = a_bk[i][e];
@@ -494,7 +541,7 @@ __global__ __launch_bounds__(kThreads) void qk_bwd_kernel(QkParams p) {
 
 template <int DT, bool BWD>
 int launch_qk(const QkParams& p, int groups, hipStream_t s) {
-  const int G = p.Dh / 8, nch = p.S / 512;
+  const int G = p.Dh / 8, nch = p.S < 512 ? 1 : p.S / 512;
   const size_t lds = BWD ? static_cast<size_t>(4) * p.S * sizeof(float) : 0;
   bool hit = false;
 #define MEGA_QK(GG, NN)                                                      \
@@ -606,7 +653,6 @@ extern "C" int mega_layer_norm_fwd(const void* x, const void* weight, const void
 
 template <int DT, bool RMS>
 static int run_bwd(NormParams p, int dtype, void* dweight, void* dbias, float* ws, hipStream_t s) {
-  using T = typename Elem<DT>::type;
   const bool affine = dweight != nullptr;
   const Shape sh = vec_shape(dtype, p.D, p);
   const int rpg = sh.lpr ? kWaves * (kWave / sh.lpr) : kWaves;
@@ -631,15 +677,7 @@ static int run_bwd(NormParams p, int dtype, void* dweight, void* dbias, float* w
     norm_bwd_any_kernel<DT, RMS><<<groups, kThreads, affine ? active * stripe : 0, s>>>(p, active);
     MEGA_CHECK_LAUNCH();
   }
-  if (affine) {
-    const int blocks = (p.D + 63) / 64;
-    norm_param_grad_kernel<DT><<<blocks, 1024, 0, s>>>(p.part_w, groups, p.D, p.D, static_cast<T*>(dweight));
-    MEGA_CHECK_LAUNCH();
-    if (p.part_b) {
-      norm_param_grad_kernel<DT><<<blocks, 1024, 0, s>>>(p.part_b, groups, p.D, p.D, static_cast<T*>(dbias));
-      MEGA_CHECK_LAUNCH();
-    }
-  }
+  if (affine) return launch_param_grad<DT>({{p.part_w, p.part_b}, {dweight, dbias}}, groups, p.D, p.D, s);
   return MEGA_OK;
 }
 
@@ -675,9 +713,9 @@ static int check_qk(const char* who, int dtype, int64_t rows, int64_t L, int64_t
   MEGA_CHECK_ARG(rows >= 0 && (rows == 0 || L >= 1) && S >= 1 && Dh >= 1, "%s: bad sizes", who);
   MEGA_CHECK_ARG(!freqs || P >= 1, "%s: rotary factors without positions", who);
   if (!(Dh == 64 || Dh == 128 || Dh == 256 || Dh == 512) || S % Dh != 0 ||
-      !(S == 512 || S == 1024 || S == 2048 || S == 4096))
+      !(S == 64 || S == 128 || S == 256 || S == 512 || S == 1024 || S == 2048 || S == 4096))
     return set_error(MEGA_ERR_UNSUPPORTED,
-                     "%s: needs a head size of 64, 128, 256 or 512 and a width of 512, 1024, 2048 or 4096 "
+                     "%s: needs a head size of 64, 128, 256 or 512 and a width of 64 to 4096, a power of two "
                      "(got %lld, %lld)", who, (long long)Dh, (long long)S);
   return MEGA_OK;
 }
@@ -703,7 +741,8 @@ extern "C" int mega_qk_norm_rotary_fwd(const void* z, const void* gamma, const v
   p.q = static_cast<uint16_t*>(q); p.k = static_cast<uint16_t*>(k); p.rstd = rstd;
   p.rows = rows; p.L = (int)L; p.P = freqs ? (int)P : 1; p.S = (int)S; p.Dh = (int)Dh;
   p.eps = static_cast<float>(eps); p.inv_sqrt_dh = static_cast<float>(1.0 / sqrt(static_cast<double>(Dh)));
-  const int64_t g = (rows + kWaves - 1) / kWaves;
+  const int rpg = kWaves * static_cast<int>(S < 512 ? 512 / S : 1);
+  const int64_t g = (rows + rpg - 1) / rpg;
   const int groups = static_cast<int>(g > 16384 ? 16384 : g);
   hipStream_t s = static_cast<hipStream_t>(stream);
   return dtype == MEGA_BF16 ? launch_qk<MEGA_BF16, false>(p, groups, s) : launch_qk<MEGA_F16, false>(p, groups, s);
@@ -726,18 +765,12 @@ extern "C" int mega_qk_norm_rotary_bwd(const void* dq, const void* dk, const voi
   p.q = static_cast<uint16_t*>(dz); p.rstd = const_cast<float*>(rstd); p.part = static_cast<float*>(workspace);
   p.rows = rows; p.L = (int)L; p.P = freqs ? (int)P : 1; p.S = (int)S; p.Dh = (int)Dh;
   p.inv_sqrt_dh = static_cast<float>(1.0 / sqrt(static_cast<double>(Dh)));
-  const int groups = groups_for(rows, kWaves);
+  const int groups = groups_for(rows, kWaves * static_cast<int>(S < 512 ? 512 / S : 1));
   hipStream_t s = static_cast<hipStream_t>(stream);
   rc = dtype == MEGA_BF16 ? launch_qk<MEGA_BF16, true>(p, groups, s) : launch_qk<MEGA_F16, true>(p, groups, s);
   if (rc != MEGA_OK) return rc;
-  const int cols = 2 * static_cast<int>(S), blocks = (cols + 63) / 64;
-  if (dtype == MEGA_BF16) {
-    norm_param_grad_kernel<MEGA_BF16><<<blocks, 1024, 0, s>>>(p.part, groups, cols, 2 * cols, static_cast<uint16_t*>(dgamma));
-    norm_param_grad_kernel<MEGA_BF16><<<blocks, 1024, 0, s>>>(p.part + cols, groups, cols, 2 * cols, static_cast<uint16_t*>(dbeta));
-  } else {
-    norm_param_grad_kernel<MEGA_F16><<<blocks, 1024, 0, s>>>(p.part, groups, cols, 2 * cols, static_cast<uint16_t*>(dgamma));
-    norm_param_grad_kernel<MEGA_F16><<<blocks, 1024, 0, s>>>(p.part + cols, groups, cols, 2 * cols, static_cast<uint16_t*>(dbeta));
-  }
-  MEGA_CHECK_LAUNCH();
-  return MEGA_OK;
+  const int cols = 2 * static_cast<int>(S);
+  const ColumnSums sums{{p.part, p.part + cols}, {dgamma, dbeta}};
+  return dtype == MEGA_BF16 ? launch_param_grad<MEGA_BF16>(sums, groups, cols, 2 * cols, s)
+                            : launch_param_grad<MEGA_F16>(sums, groups, cols, 2 * cols, s);
 }

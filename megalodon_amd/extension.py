@@ -1257,7 +1257,7 @@ def layer_norm_bwd(y_grad: torch.Tensor, x: torch.Tensor, weight: Optional[torch
 def qk_norm_rotary_supported(z: torch.Tensor, gamma: torch.Tensor, head_dim: int) -> bool:
     """Shapes the fused z -> (q, k) kernel takes (include/megalodon_hip.h)."""
     return (z.is_cuda and z.dtype in (torch.bfloat16, torch.float16) and gamma.dtype == z.dtype
-            and head_dim in (64, 128, 256, 512) and z.shape[-1] in (512, 1024, 2048, 4096)
+            and head_dim in (64, 128, 256, 512) and z.shape[-1] in (64, 128, 256, 512, 1024, 2048, 4096)
             and z.shape[-1] % head_dim == 0 and z.dim() == 3)
 
 
