@@ -306,7 +306,7 @@ __global__ __launch_bounds__(kThreads) void norm_bwd_any_kernel(NormParams p, in
 // out[c] = sum over `groups` rows (`stride` floats apart) of part[., c], c < D, for one or two
 // (part, out) pairs: 16 columns x 64 row slices per workgroup, so that the few columns of a norm
 // still occupy a workgroup per 64 bytes of a row and a thread has all its loads in flight.
-// (1024 rows of 4096 columns, two sums: PG_BEFORE with 64 columns x 16 slices and a launch each.)
+// (1024 rows of 4096 columns, two sums: 20 us with 64 columns x 16 slices and a launch each, 4.3 so.)
 struct ColumnSums {
   const float* part[2];
   void* out[2];
@@ -350,7 +350,7 @@ int launch_param_grad(const ColumnSums& t, int groups, int D, int stride, hipStr
 // freqs[p][i], p = (row % L) % P the position inside the chunk.  One wavefront
 // holds a row of S = 512 * NCH elements, or 512 / S rows of 64, 128 or 256 (one narrow head
 // each: left to the PyTorch expressions they are some 65 small launches per training step,
-// QK_NARROW), G = Dh / 8 lanes per head; z is read once and q, k are written once.  The backward undoes the rotation with the
+// 0.5 ms of a block of 1024 channels on 2 x 2048 steps), G = Dh / 8 lanes per head; z is read once and q, k are written once.  The backward undoes the rotation with the
 // conjugate factor, forms the gradients of the affine parameters as column
 // sums (per-workgroup partials, reduced in a fixed order afterwards) and the
 // RMSNorm gradient per head.
