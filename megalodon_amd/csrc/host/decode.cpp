@@ -60,9 +60,15 @@ py::tuple views_of(const std::shared_ptr<KvBuffer>& buf, int64_t lo, int64_t hi)
   return py::make_tuple(k, v);
 }
 
-// (keys, values) of the old and the new tokens together, in storage with room for more
-py::tuple kv_append(const py::object& k_obj, const Tensor& v, const Tensor& k_new, const Tensor& v_new, int64_t chunk) {
+// (keys, values) of the old and the new tokens together, in storage with room for more; None for
+// operands that are not one batch of one type (the caller concatenates)
+py::object kv_append(const py::object& k_obj, const Tensor& v, const Tensor& k_new, const Tensor& v_new, int64_t chunk) {
   const Tensor k = k_obj.cast<Tensor>();
+  const auto joins = [](const Tensor& a, const Tensor& b) {
+    return a.dim() == 4 && b.dim() == 4 && a.size(0) == b.size(0) && a.sizes().slice(2) == b.sizes().slice(2) &&
+           a.scalar_type() == b.scalar_type() && a.device() == b.device() && !has_tangent(a) && !has_tangent(b);
+  };
+  if (!joins(k, k_new) || !joins(v, v_new) || k.size(1) != v.size(1) || k_new.size(1) != v_new.size(1)) return py::none();
   const int64_t n = k.size(1), more = k_new.size(1);
   auto buf = room_for(k_obj, k, v, more, chunk);
   buf->k.narrow(1, n, more).copy_(k_new);
@@ -88,6 +94,9 @@ py::object block_decode_step(const Tensor& x, const py::object& k_obj, const Ten
   if (dtype != MEGA_BF16 && dtype != MEGA_F16) return py::none();
   const auto dev = x.device();
   if (!x.is_cuda() || static_cast<int>(weights.size()) != kWeights) return py::none();
+  // a forward-mode tangent goes to the operators, which refuse it
+  for (const Tensor* t : {&x, &k, &v, &prev_mean, &prev_var, &hx})
+    if (has_tangent(*t)) return py::none();
   const auto aligned = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
   for (int i = 0; i < kWeights; ++i) {
     const Optional& w = weights[i];
@@ -96,7 +105,7 @@ py::object block_decode_step(const Tensor& x, const py::object& k_obj, const Ten
       if (may_lack) continue;
       return py::none();
     }
-    if (w->scalar_type() != type || w->device() != dev || !w->is_contiguous() || !aligned(*w)) return py::none();
+    if (has_tangent(*w) || w->scalar_type() != type || w->device() != dev || !w->is_contiguous() || !aligned(*w)) return py::none();
   }
   const int64_t B = x.size(0), D = x.size(2), S = weights[kWz]->size(0), E = weights[kWv]->size(0), F = weights[kFc1]->size(0),
                 N = p.size(1), n = k.size(1);

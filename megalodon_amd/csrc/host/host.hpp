@@ -41,6 +41,9 @@ inline int code_of(at::ScalarType t) {
   }
 }
 
+// whether a forward-mode derivative travels with the tensor
+inline bool has_tangent(const Tensor& t) { return t._fw_grad(/*level=*/0).defined(); }
+
 void bind_decode(py::module_& m);
 void bind_ops(py::module_& m);
 

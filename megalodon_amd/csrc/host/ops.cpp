@@ -38,10 +38,12 @@ float* fptr(const Tensor& t) { return static_cast<float*>(ptr(t)); }
 Tensor some(const Optional& t) { return t.has_value() ? t->contiguous() : Tensor(); }
 Tensor bytes(int64_t n, const Tensor& like) { return at::empty({n}, like.options().dtype(at::kByte)); }
 Tensor floats(at::IntArrayRef shape, const Tensor& like) { return at::empty(shape, like.options().dtype(at::kFloat)); }
+// whether the call has to go through its autograd node: a gradient is wanted, or an operand carries a
+// forward-mode tangent, which the node refuses (whatever the gradient mode) and a bare launch would drop
 bool wants_grad(std::initializer_list<const Tensor*> ts) {
-  if (!at::GradMode::is_enabled()) return false;
+  const bool on = at::GradMode::is_enabled();
   for (const Tensor* t : ts)
-    if (t != nullptr && t->defined() && t->requires_grad()) return true;
+    if (t != nullptr && t->defined() && ((on && t->requires_grad()) || has_tangent(*t))) return true;
   return false;
 }
 
@@ -128,6 +130,7 @@ struct LayerNormFn : Function<LayerNormFn> {
     const bool rms = ctx->saved_data["rms"].toBool(), has_bias = ctx->saved_data["bias"].toBool();
     const Tensor x = saved[0].contiguous(), weight = saved[1].defined() ? saved[1].contiguous() : Tensor(), go = g[0].contiguous();
     require(go.scalar_type() == x.scalar_type(), "layer_norm_bwd: y_grad and x must have the same shape and dtype");
+    const Tensor mean = saved[2].defined() ? saved[2].contiguous() : Tensor(), rstd = saved[3].contiguous();
     c10::DeviceGuard guard(x.device());
     const int64_t D = x.size(-1), rows = D > 0 ? x.numel() / D : 0;
     Tensor dx = at::empty_like(x), dw, db, ws;
@@ -140,7 +143,7 @@ struct LayerNormFn : Function<LayerNormFn> {
       if (dw.defined()) dw.zero_();
       if (db.defined()) db.zero_();
     } else {
-      check(mega_layer_norm_bwd(go.data_ptr(), x.data_ptr(), ptr(weight), fptr(saved[2]), fptr(saved[3]), kernel_code(x), rows, D, rms, dx.data_ptr(), ptr(dw), ptr(db), ptr(ws), stream_of(x)), "mega_layer_norm_bwd");
+      check(mega_layer_norm_bwd(go.data_ptr(), x.data_ptr(), ptr(weight), fptr(mean), fptr(rstd), kernel_code(x), rows, D, rms, dx.data_ptr(), ptr(dw), ptr(db), ptr(ws), stream_of(x)), "mega_layer_norm_bwd");
     }
     return {dx, dw, db, Tensor(), Tensor()};
   }
@@ -159,6 +162,7 @@ Tensor real_freqs(const Optional& freqs, int64_t head_dim, const Tensor& z) {
 std::tuple<Tensor, Tensor, Tensor> qk_raw(const Tensor& z, const Tensor& gamma, const Tensor& beta, const Tensor& fr, int64_t head_dim, double eps) {
   need_gpu({&z, &gamma, &beta});
   require(z.dim() == 3 && gamma.dim() == 2 && gamma.size(0) == 2 && gamma.size(1) == z.size(2) && beta.sizes() == gamma.sizes(), "qk_norm_rotary: z must be (B, L, S), gamma and beta (2, S)");
+  require(gamma.scalar_type() == z.scalar_type() && beta.scalar_type() == z.scalar_type(), "qk_norm_rotary: gamma and beta must have z's dtype");
   const int code = kernel_code(z);
   const Tensor zc = z.contiguous(), gc = gamma.contiguous(), bc = beta.contiguous();
   const int64_t B = z.size(0), L = z.size(1), S = z.size(2);
@@ -179,11 +183,11 @@ struct QkFn : Function<QkFn> {
     at::AutoDispatchBelowADInplaceOrView below;
     const auto saved = ctx->get_saved_variables();
     const Tensor z = saved[0].contiguous(), gamma = saved[1].contiguous(), dq = g[0].contiguous(), dk = g[1].contiguous();
-    const Tensor& fr = saved[3];
+    const Tensor fr = saved[3].defined() ? saved[3].contiguous() : Tensor(), rstd = saved[2].contiguous();
     c10::DeviceGuard guard(z.device());
     const int64_t B = z.size(0), L = z.size(1), S = z.size(2);
     Tensor dz = at::empty_like(z), dgamma = at::empty_like(gamma), dbeta = at::empty_like(gamma), ws = bytes(mega_qk_norm_rotary_workspace_bytes(S), z);
-    check(mega_qk_norm_rotary_bwd(dq.data_ptr(), dk.data_ptr(), z.data_ptr(), gamma.data_ptr(), fptr(saved[2]), fptr(fr), kernel_code(z), B * L, L, fr.defined() ? fr.size(0) : 1, S, ctx->saved_data["head_dim"].toInt(), dz.data_ptr(), dgamma.data_ptr(), dbeta.data_ptr(), ws.data_ptr(), stream_of(z)), "mega_qk_norm_rotary_bwd");
+    check(mega_qk_norm_rotary_bwd(dq.data_ptr(), dk.data_ptr(), z.data_ptr(), gamma.data_ptr(), fptr(rstd), fptr(fr), kernel_code(z), B * L, L, fr.defined() ? fr.size(0) : 1, S, ctx->saved_data["head_dim"].toInt(), dz.data_ptr(), dgamma.data_ptr(), dbeta.data_ptr(), ws.data_ptr(), stream_of(z)), "mega_qk_norm_rotary_bwd");
     return {dz, dgamma, dbeta, Tensor(), Tensor(), Tensor()};
   }
 };
@@ -203,8 +207,9 @@ std::tuple<Tensor, Tensor> qk_norm_rotary(const Tensor& z, const Tensor& gamma, 
 // The last workspace of every (device, stream, direction) is kept for its status word
 // (timestep_norm_status); the launches themselves take a fresh one each, so calls of
 // different threads never share one.
+// (never destroyed: at the process's end the allocator may be gone first)
 std::mutex last_mutex;
-std::map<std::tuple<int, void*, bool>, Tensor> last_workspace;
+auto& last_workspace = *new std::map<std::tuple<int, void*, bool>, Tensor>();
 Tensor tsn_workspace(const Tensor& x, int64_t groups, bool backward) {
   Tensor ws = bytes(mega_group_timestep_norm_workspace_bytes(x.size(0), x.size(1), x.size(2), groups, backward), x);
   std::lock_guard<std::mutex> lock(last_mutex);
@@ -251,7 +256,9 @@ struct TsnFn : Function<TsnFn> {
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     at::AutoDispatchBelowADInplaceOrView below;
     const auto saved = ctx->get_saved_variables();
-    const Tensor &x = saved[0], &mean0 = saved[1], &weight = saved[5];
+    // (saved-tensor hooks may hand back any layout)
+    const Tensor x = saved[0].contiguous(), mean0 = saved[1].contiguous(), count = saved[2].contiguous(),
+                 cummean = saved[3].contiguous(), cumrstd = saved[4].contiguous(), weight = saved[5].contiguous();
     c10::DeviceGuard guard(x.device());
     const int64_t B = x.size(0), L = x.size(1), D = x.size(2), groups = ctx->saved_data["groups"].toInt();
     const bool shared = ctx->saved_data["shared"].toBool();
@@ -261,7 +268,7 @@ struct TsnFn : Function<TsnFn> {
     require(dy.scalar_type() == x.scalar_type(), "timestep_norm: y_grad must have x's dtype");
     Tensor dx = at::empty_like(x), dpm = at::empty({B, groups}, x.options()), dpv = at::empty({B, groups}, x.options()), dw = at::empty_like(weight), db = at::empty_like(weight);
     const Tensor ws = tsn_workspace(x, groups, true);
-    check(mega_timestep_norm_layer_bwd(dy.data_ptr(), ptr(dm), ptr(dv), x.data_ptr(), kernel_code(x), mean0.data_ptr(), shared, saved[2].data_ptr<int64_t>(), fptr(saved[3]), fptr(saved[4]), weight.data_ptr(), static_cast<const uint8_t*>(ptr(mask)), B, L, D, groups, dx.data_ptr(), dpm.data_ptr(), dpv.data_ptr(), dw.data_ptr(), db.data_ptr(), ws.data_ptr(), stream_of(x)), "mega_timestep_norm_layer_bwd");
+    check(mega_timestep_norm_layer_bwd(dy.data_ptr(), ptr(dm), ptr(dv), x.data_ptr(), kernel_code(x), mean0.data_ptr(), shared, count.data_ptr<int64_t>(), fptr(cummean), fptr(cumrstd), weight.data_ptr(), static_cast<const uint8_t*>(ptr(mask)), B, L, D, groups, dx.data_ptr(), dpm.data_ptr(), dpv.data_ptr(), dw.data_ptr(), db.data_ptr(), ws.data_ptr(), stream_of(x)), "mega_timestep_norm_layer_bwd");
     if (shared) dpm = dpv = Tensor();  // the prior is no parameter here
     return {dx, Tensor(), dpm, dpv, Tensor(), dw, db, Tensor(), Tensor(), Tensor()};
   }
@@ -334,7 +341,7 @@ struct CemaFn : Function<CemaFn> {
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     at::AutoDispatchBelowADInplaceOrView below;
     const auto saved = ctx->get_saved_variables();
-    const Tensor &x = saved[0], &alpha = saved[1], &delta = saved[2], &theta = saved[3], &gamma = saved[4], &omega = saved[5], &c = saved[6], &w = saved[7];
+    const Tensor x = rows_of(saved[0]), alpha = saved[1].contiguous(), delta = saved[2].contiguous(), theta = saved[3].contiguous(), gamma = saved[4].contiguous(), omega = saved[5].contiguous(), c = saved[6].contiguous(), w = saved[7].contiguous();
     require(g[0].sizes() == x.sizes() && g[0].scalar_type() == x.scalar_type(), "cema: y_grad must match x in shape and dtype");
     c10::DeviceGuard guard(x.device());
     const Tensor dy = rows_of(g[0]);
@@ -433,7 +440,7 @@ struct AttentionFn : Function<AttentionFn> {
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     at::AutoDispatchBelowADInplaceOrView below;
     const auto saved = ctx->get_saved_variables();
-    const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &w = saved[3];
+    const Tensor q = attn_operand(saved[0]), k = attn_operand(saved[1]), v = attn_operand(saved[2]), w = attn_operand(saved[3]);
     const AttnDims d = attn_dims(q, k, v);
     c10::DeviceGuard guard(q.device());
     const Tensor dy = attn_operand(g[0]);

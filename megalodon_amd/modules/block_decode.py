@@ -7,6 +7,7 @@ from torch import Tensor
 from torch.nn.modules import module as nn_module
 
 from .. import _lib
+from ..fused_ops import swift_efficient_attention
 from .chunk_attention import _InnerAttention
 from .complex_exponential_moving_average import MultiHeadComplexEMA
 from .layer_norm import FusedLayerNorm, FusedRMSNorm
@@ -15,9 +16,14 @@ from .normalized_feedforward_network import NormalizedFeedForwardNetwork
 from .timestep_norm import TimestepNorm
 
 
+def _unheard(module) -> bool:
+    """Nobody listens to the module's forward or has put another in its place."""
+    return not module._forward_hooks and not module._forward_pre_hooks and "forward" not in module.__dict__
+
+
 def _plain(module, kind) -> bool:
-    """`module` is exactly a `kind` and nobody listens to its forward."""
-    return type(module) is kind and not module._forward_hooks and not module._forward_pre_hooks
+    """`module` is exactly a `kind` whose own forward runs."""
+    return type(module) is kind and _unheard(module)
 
 
 def decode_step(block, x: Tensor, freqs_cis: Optional[Tensor], cache):
@@ -36,12 +42,12 @@ def decode_step(block, x: Tensor, freqs_cis: Optional[Tensor], cache):
     tsn, cema, rms, znorm, attn = m["timenorm"], m["cema"], m["rmsnorm"], m["znorm"], m["inner_attention"]
     wz, wr, wh1, wv, wh2 = m["wz"], m["wr"], m["wh1"], m["wv"], m["wh2"]
     ln, fc1, fc2, fc3 = f["norm"], f["fc1"], f["fc2"], f["fc3"]
-    if (mega._forward_hooks or mega._forward_pre_hooks or nn_module._global_forward_hooks
+    if (not _unheard(mega) or nn_module._global_forward_hooks
             or nn_module._global_forward_pre_hooks or not _plain(nffn, NormalizedFeedForwardNetwork)
             or nffn._parameters.get("alpha") is not None or fc3 is None
             or not _plain(tsn, TimestepNorm) or not _plain(cema, MultiHeadComplexEMA)
             or not _plain(rms, FusedRMSNorm) or not _plain(znorm, FusedRMSNorm) or znorm.elementwise_affine
-            or not _plain(attn, _InnerAttention) or attn.attn_fn is None or not _plain(ln, FusedLayerNorm)
+            or not _plain(attn, _InnerAttention) or attn.attn_fn is not swift_efficient_attention or not _plain(ln, FusedLayerNorm)
             or any(not _plain(w, Linear) for w in (wz, wr, wh1, wv, wh2, fc1, fc2, fc3))
             or any(w._parameters["bias"] is not None for w in (wh2, fc1, fc2, fc3))):
         return None

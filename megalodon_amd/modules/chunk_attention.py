@@ -81,9 +81,12 @@ class _InnerAttention(nn.Module):
             old_k, old_v, old_len = cache
             total = old_len + new_len
             tail = total % self.chunk_size  # steps of the chunk still open after this call
+            joined = None
             if k.is_cuda and not torch.is_grad_enabled():
                 # behind the old ones, in storage with room for the tokens to come
-                all_k, all_v = _lib.host().kv_append(old_k, old_v, k, v, self.chunk_size)
+                joined = _lib.host().kv_append(old_k, old_v, k, v, self.chunk_size)
+            if joined is not None:
+                all_k, all_v = joined
                 carried = (all_k, all_v) if tail == total else (all_k[:, total - tail:], all_v[:, total - tail:])
                 if old_k.shape[1] > 0:
                     k, v = all_k, all_v

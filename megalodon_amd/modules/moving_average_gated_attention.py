@@ -151,7 +151,7 @@ class MegaBlock(nn.Module):
 
     def forward(self, x: Tensor, freqs_cis: Optional[Tensor] = None, mask: Optional[Tensor] = None, cache=None):
         if (cache is not None and x.dim() == 3 and x.shape[1] == 1 and mask is None and not self.training
-                and not torch.is_grad_enabled()):
+                and not torch.is_grad_enabled() and type(self.mega) is MovingAverageGatedAttention):
             step = decode_step(self, x, freqs_cis, cache)
             if step is not None:
                 return step

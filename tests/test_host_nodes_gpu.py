@@ -1,0 +1,107 @@
+"""What the C++ autograd nodes and the fused step owe to PyTorch's own machinery: forward-mode
+tangents are refused and not dropped, saved-tensor hooks may hand back any layout, and calls that
+the operator-by-operator path refuses or takes differently keep doing so."""
+import pytest
+import torch
+import torch.autograd.forward_ad as fwad
+
+from megalodon_amd import fused_ops as ops
+from megalodon_amd.modules import MegaBlock, MultiHeadComplexEMA, TimestepNorm
+from megalodon_amd.modules.block_decode import decode_step
+
+pytestmark = pytest.mark.gpu
+
+
+def _randn(*shape, dtype=torch.bfloat16):
+    return torch.randn(*shape, device="cuda").to(dtype)
+
+
+def _calls():
+    """name -> (function, operands); every operand may carry gradients or tangents."""
+    torch.manual_seed(0)
+    cema, tsn = MultiHeadComplexEMA(64, 4).cuda(), TimestepNorm(64, 4).cuda().bfloat16()
+    return {
+        "transpose_last2": (ops.transpose_last2, [_randn(2, 24, 64)]),
+        "silu_mul": (ops.silu_mul, [_randn(2, 24, 64), _randn(2, 24, 64)]),
+        "layer_norm": (ops.layer_norm_plus_one, [_randn(2, 24, 64), _randn(64), _randn(64)]),
+        "qk_norm_rotary": (lambda z, g, b: sum(ops.qk_norm_rotary(z, g, b, None, 64, 1e-5)),
+                           [_randn(2, 24, 128), _randn(2, 128), _randn(2, 128)]),
+        "attention": (ops.swift_efficient_attention, [_randn(2, 40, 2, 64), _randn(2, 40, 2, 64), _randn(2, 40, 2, 64)]),
+        "cema": (lambda x: cema(x)[0], [_randn(2, 64, 37)]),
+        "cema_f32": (lambda x: cema(x)[0], [_randn(2, 64, 40, dtype=torch.float32)]),
+        "timestep_norm": (lambda x: tsn(x)[0], [_randn(2, 37, 64)]),
+    }
+
+
+@pytest.mark.parametrize("grad_mode", [True, False])
+@pytest.mark.parametrize("name", [
+    "transpose_last2", "silu_mul", "layer_norm", "qk_norm_rotary", "attention", "cema", "cema_f32",
+                                  "timestep_norm"])
+def test_tangent_is_refused(name, grad_mode):
+    fn, args = _calls()[name]
+    with torch.set_grad_enabled(grad_mode), fwad.dual_level():
+        with pytest.raises(RuntimeError):
+            fn(fwad.make_dual(args[0], torch.ones_like(args[0])), *args[1:])
+
+
+def _scatter(t):
+    """The same values at an odd element offset and, where it has several axes, with other strides."""
+    if t.dim() < 2:
+        return torch.cat((t.new_zeros(1), t.reshape(-1)))[1:].view(t.shape)
+    turned = t.transpose(0, -1).contiguous()
+    return torch.cat((t.new_zeros(1), turned.reshape(-1)))[1:].view(turned.shape).transpose(0, -1)
+
+
+@pytest.mark.parametrize("name", ["transpose_last2", "silu_mul", "layer_norm", "qk_norm_rotary", "attention", "cema",
+                                  "cema_f32", "timestep_norm"])
+def test_saved_tensors_of_any_layout(name):
+    fn, args = _calls()[name]
+    grads = []
+    for unpack in (lambda t: t, _scatter):
+        leaves = [a.clone().requires_grad_(True) for a in args]
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            y = fn(*leaves)
+        y.backward(torch.ones_like(y))
+        grads.append([l.grad for l in leaves])
+    for a, b in zip(*grads):
+        # the same kernels on the same values; a misaligned operand may take the unvectorised flavour
+        assert (a.float() - b.float()).norm() <= 8e-3 * a.float().norm()
+
+
+def _decode_setup():
+    torch.manual_seed(1)
+    blk = MegaBlock(model_dim=256, z_dim=128, value_dim=512, num_heads=2, cema_ndim=16, chunk_size=64,
+                    ffn_hidden_dim=512, norm_num_groups=2).cuda().bfloat16().eval()
+    empty = ((_randn(2, 0, 2, 64), _randn(2, 0, 2, 256), 0), (None, None, None), None)
+    with torch.no_grad():
+        cache = blk(_randn(2, 9, 256), None, None, empty)[1]
+    return blk, cache
+
+
+def test_replaced_forward_is_called():
+    blk, cache = _decode_setup()
+    x = _randn(2, 1, 256)
+    with torch.no_grad():
+        assert decode_step(blk, x, None, cache) is not None
+        own, seen = blk.mega.wv.forward, []
+        blk.mega.wv.forward = lambda t: (seen.append(1), own(t))[1]
+        assert decode_step(blk, x, None, cache) is None
+        blk(x, None, None, cache)
+        assert seen
+        del blk.mega.wv.forward
+        blk.mega.inner_attention.attn_fn = lambda *a: ops.swift_efficient_attention(*a)
+        assert decode_step(blk, x, None, cache) is None
+
+
+def test_cache_of_another_batch_is_refused():
+    blk, cache = _decode_setup()
+    (k, v, n), norm, hx = cache
+    with torch.no_grad(), pytest.raises(RuntimeError):
+        blk.mega.inner_attention(_randn(1, 2, 128), _randn(1, 2, 128), _randn(1, 2, 512), None, None, (k, v, n))
+
+
+def test_tangent_in_a_step_is_refused():
+    blk, cache = _decode_setup()
+    x = _randn(2, 1, 256)
+    with torch.no_grad(), fwad.dual_level(), pytest.raises(RuntimeError):
+        blk(fwad.make_dual(x, torch.ones_like(x)), None, None, cache)
