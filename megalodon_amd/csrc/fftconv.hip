@@ -24,6 +24,15 @@ namespace {
 
 using namespace fftc;
 
+// Workgroups of a transform size that share a compute unit: the kernel's time is the latency of its
+// exchanges and barriers, so two waves per SIMD at every size, which is what the registers (32 complex
+// points per lane and operand: 219-256 of 256, none spilled) and the planes in LDS allow.  With one wave
+// per SIMD below M = 16384 (and 330 registers) and the loads in branches, forward / backward in
+// bfloat16 took 2 x 1024 rows of 3000: 152 / 348 us, now 51 / 138; of 8192: 226 / 479, now 95 / 198;
+// 1024 rows of 16384: 236 / 485, now 115 / 219; of 32768: 440 / 891, now 246 / 502 (the last by the loads alone).
+template <int LOGM>
+constexpr int kPerCu = 1 << (14 - LOGM);
+
 // ------------------------------ tables --------------------------------------
 constexpr int kMaxDevices = 16;
 constexpr int kMaxScratch = 4;  // scratch blocks per device and size before streams start taking turns
@@ -62,8 +71,8 @@ bool stream_is_capturing(hipStream_t stream) {
 // scratch slots live for the life of the process.  They are made on first use,
 // or ahead of time by mega_fftconv_prepare; making them allocates and, for the
 // tables, synchronises the stream once, so that call cannot be captured into a
-// graph.  Scratch is 2*M floats per resident workgroup (at most 2 workgroups
-// per CU).
+// graph.  Scratch is 2*M floats per resident workgroup (kPerCu of them per CU:
+// 34 MB at every size).
 template <int LOGM>
 int get_tables(hipStream_t stream, const c32** out, float** scratch, int* slots) {
   using C = Cfg<LOGM>;
@@ -75,8 +84,7 @@ int get_tables(hipStream_t stream, const c32** out, float** scratch, int* slots)
   if (slot == nullptr) {
     hipDeviceProp_t prop;
     MEGA_CHECK_HIP(hipGetDeviceProperties(&prop, dev));
-    const int per_cu = LOGM == 14 ? 1 : 2;
-    g_tables.slots[dev][LOGM - 11] = prop.multiProcessorCount * per_cu;
+    g_tables.slots[dev][LOGM - 11] = prop.multiProcessorCount * kPerCu<LOGM>;
     c32* p = nullptr;
     MEGA_CHECK_HIP(hipMalloc(reinterpret_cast<void**>(&p), sizeof(c32) * C::TABLE));
     std::vector<c32> host(C::TABLE);
@@ -185,34 +193,48 @@ template <> struct Pair<MEGA_F16> {
   }
 };
 
-// z[n] = s[2n] + i s[2n+1] of the zero-padded (optionally reversed) row.
+// The lane id, hidden from the optimiser: left alone it keeps the offsets of a row's 32 accesses in
+// registers from its load to its store, across both halves (with two waves per SIMD: 74 spilled).
+__device__ __forceinline__ int own_lane(int t) {
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
+// z[n] = s[2n] + i s[2n+1] of the zero-padded (optionally reversed) row.  Every lane reads inside the
+// row and takes zero for what lies behind it, so that the 32 loads stand in one piece without branches.
 // VEC: L is even and the row is pair-aligned, so (s[2n], s[2n+1]) is one access
 // addressed with a 32-bit offset from the wave-uniform row base.
 template <int LOGM, int DT, bool VEC>
 __device__ __forceinline__ void load_row(float* re, float* im, const void* row, int L, bool flip,
-                                         int t) {
+                                         int lane) {
   using C = Cfg<LOGM>;
+  const unsigned t = static_cast<unsigned>(own_lane(lane));
+  const unsigned count = VEC ? static_cast<unsigned>(L) >> 1 : static_cast<unsigned>(L), last = count - 1u;
+  const unsigned turn = flip ? ~0u : 0u, from = flip ? count : 0u;  // i or count - 1 - i
   if (VEC) {
     using P = typename Pair<DT>::type;
-    const unsigned half = static_cast<unsigned>(L) >> 1;
+    P raw[32];
 #pragma unroll
     for (int j = 0; j < 32; ++j) {
-      const unsigned n = static_cast<unsigned>(t) + C::T * j;
-      float lo = 0.f, hi = 0.f;
-      if (n < half)
-        Pair<DT>::unpack(gld<P>(row, (flip ? half - 1u - n : n) * static_cast<unsigned>(sizeof(P))), lo, hi);
-      re[j] = flip ? hi : lo;
-      im[j] = flip ? lo : hi;
+      const unsigned n = t + C::T * j;
+      raw[j] = gld<P>(row, (((n < last ? n : last) ^ turn) + from) * static_cast<unsigned>(sizeof(P)));
+    }
+#pragma unroll
+    for (int j = 0; j < 32; ++j) {
+      const bool in = t + C::T * j < count;
+      float lo, hi;
+      Pair<DT>::unpack(raw[j], lo, hi);
+      re[j] = in ? (flip ? hi : lo) : 0.f;
+      im[j] = in ? (flip ? lo : hi) : 0.f;
     }
   } else {
 #pragma unroll
     for (int j = 0; j < 32; ++j) {
-      const int m0 = 2 * (t + C::T * j), m1 = m0 + 1;
-      float a = 0.f, b = 0.f;
-      if (m0 < L) a = ld<DT>(row, flip ? L - 1 - m0 : m0);
-      if (m1 < L) b = ld<DT>(row, flip ? L - 1 - m1 : m1);
-      re[j] = a;
-      im[j] = b;
+      const unsigned m0 = 2u * (t + C::T * j), m1 = m0 + 1u;
+      const float a = ld<DT>(row, static_cast<int64_t>(((m0 < last ? m0 : last) ^ turn) + from));
+      const float b = ld<DT>(row, static_cast<int64_t>(((m1 < last ? m1 : last) ^ turn) + from));
+      re[j] = m0 < count ? a : 0.f;
+      im[j] = m1 < count ? b : 0.f;
     }
   }
 }
@@ -222,9 +244,10 @@ __device__ __forceinline__ void load_row(float* re, float* im, const void* row, 
 // value is out[m] + w * res[m] (res has the dtype and layout of the output row).
 template <int LOGM, int DT, bool VEC, bool ACC>
 __device__ __forceinline__ void store_row(const float* re, const float* im, void* row, int L,
-                                          bool flip, int t, const void* res = nullptr,
+                                          bool flip, int lane, const void* res = nullptr,
                                           float w = 0.f) {
   using C = Cfg<LOGM>;
+  const int t = own_lane(lane);
   if (VEC) {
     using P = typename Pair<DT>::type;
     const unsigned half = static_cast<unsigned>(L) >> 1;
@@ -355,12 +378,12 @@ __device__ __forceinline__ void conv_half(const void* arow, bool flip_a, const v
 // Persistent: workgroup g handles rows g, g + gridDim.x, ... and owns scratch
 // slot g (2*M floats).
 template <int LOGM, int DT, int MODE, bool VEC>
-__global__ __launch_bounds__(Cfg<LOGM>::T) void fftconv_kernel(
+__global__ __launch_bounds__(Cfg<LOGM>::T, 2) void fftconv_kernel(
     const void* __restrict__ a, const void* __restrict__ b, void* __restrict__ out, int rows,
     int D, int L, int flip, const c32* __restrict__ tab, float* __restrict__ scratch_all,
     const float* __restrict__ omega) {
   using C = Cfg<LOGM>;
-  extern __shared__ float lds[];
+  extern __shared__ __align__(16) float lds[];
   float* lre = lds;
   float* lim = lds + C::PLANE;
   const Tables tb = make_tables<LOGM>(tab);

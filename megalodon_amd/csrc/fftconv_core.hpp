@@ -45,8 +45,9 @@ namespace fftc {
 struct c32 {
   float x, y;
 };
-struct alignas(8) f2 {
-  float x, y;
+template <int V>
+struct alignas(4 * V) fvec {
+  float v[V];
 };
 
 // cos/sin of 2*pi*k/64
@@ -212,7 +213,11 @@ struct Cfg {
   static constexpr int R3 = M / 1024;       // radix of the third pass
   static constexpr int NSLOT = 16 / R3;     // residue pairs per lane
   static constexpr int LD1 = T + R3;        // row pitch of exchange 1 (floats)
-  static constexpr int LD2 = R3 + (R3 >= 4 ? 2 : 0);  // pitch of exchange 2
+  // Exchange 2: pitch of a residue's R3 values and how many of them one access moves.  Four at once
+  // need no padding (both directions then run over consecutive banks), which is also what lets four
+  // workgroups of M = 4096 share a compute unit's LDS; six apart in pairs, only three fit.
+  static constexpr int LD2 = R3 + (R3 >= 8 ? 2 : 0);
+  static constexpr int V2 = R3 == 4 ? 4 : 2;
   static constexpr int PLANE = (32 * LD1 > 1024 * LD2) ? 32 * LD1 : 1024 * LD2;
   static constexpr int TABLE = 4 * T + R3 + 96 + 2048;  // c32 entries
   static_assert(LOGM >= 11 && LOGM <= 14, "M must be 2048..16384");
@@ -410,15 +415,17 @@ MEGA_HD void x2_read(float* re, float* im, int t, const float* lre, const float*
     slot_residues<H>(t + C::T * u, c[0], c[1]);
 #pragma unroll
     for (int w = 0; w < 2; ++w) {
-      const f2* pr = reinterpret_cast<const f2*>(lre + c[w] * C::LD2);
-      const f2* pi = reinterpret_cast<const f2*>(lim + c[w] * C::LD2);
+      using V = fvec<C::V2>;
+      const V* pr = reinterpret_cast<const V*>(lre + c[w] * C::LD2);
+      const V* pi = reinterpret_cast<const V*>(lim + c[w] * C::LD2);
 #pragma unroll
-      for (int e = 0; e < C::R3 / 2; ++e) {
-        const f2 a = pr[e], b = pi[e];
-        re[sidx<LOGM>(u, w, 2 * e)] = a.x;
-        re[sidx<LOGM>(u, w, 2 * e + 1)] = a.y;
-        im[sidx<LOGM>(u, w, 2 * e)] = b.x;
-        im[sidx<LOGM>(u, w, 2 * e + 1)] = b.y;
+      for (int e = 0; e < C::R3 / C::V2; ++e) {
+        const V a = pr[e], b = pi[e];
+#pragma unroll
+        for (int i = 0; i < C::V2; ++i) {
+          re[sidx<LOGM>(u, w, C::V2 * e + i)] = a.v[i];
+          im[sidx<LOGM>(u, w, C::V2 * e + i)] = b.v[i];
+        }
       }
     }
   }
@@ -541,12 +548,19 @@ MEGA_HD void ix2_write(const float* re, const float* im, int t, float* lre, floa
     slot_residues<H>(t + C::T * u, c[0], c[1]);
 #pragma unroll
     for (int w = 0; w < 2; ++w) {
-      f2* pr = reinterpret_cast<f2*>(lre + c[w] * C::LD2);
-      f2* pi = reinterpret_cast<f2*>(lim + c[w] * C::LD2);
+      using V = fvec<C::V2>;
+      V* pr = reinterpret_cast<V*>(lre + c[w] * C::LD2);
+      V* pi = reinterpret_cast<V*>(lim + c[w] * C::LD2);
 #pragma unroll
-      for (int e = 0; e < C::R3 / 2; ++e) {
-        pr[e] = f2{re[sidx<LOGM>(u, w, 2 * e)], re[sidx<LOGM>(u, w, 2 * e + 1)]};
-        pi[e] = f2{im[sidx<LOGM>(u, w, 2 * e)], im[sidx<LOGM>(u, w, 2 * e + 1)]};
+      for (int e = 0; e < C::R3 / C::V2; ++e) {
+        V a, b;
+#pragma unroll
+        for (int i = 0; i < C::V2; ++i) {
+          a.v[i] = re[sidx<LOGM>(u, w, C::V2 * e + i)];
+          b.v[i] = im[sidx<LOGM>(u, w, C::V2 * e + i)];
+        }
+        pr[e] = a;
+        pi[e] = b;
       }
     }
   }

@@ -57,6 +57,24 @@ def _data(B, D, L, dtype, seed):
     return x, k, dy
 
 
+# more rows than workgroups are resident (256 CUs: 2048 at M = 2048, 1024 at M = 4096), even and odd
+MANY_ROWS = [(1, 2051, 2050), (1, 1027, 4099), (2, 520, 8192)]
+
+
+@pytest.mark.parametrize("B,D,L", MANY_ROWS)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_more_rows_than_workgroups(B, D, L, dtype):
+    x, k, dy = (t.cuda() for t in _data(B, D, L, dtype, L))
+    y = ops.fftconv_fwd(x, k)
+    dx, dk = ops.fftconv_bwd(dy, x, k, torch.float32)
+    spectrum = lambda t: torch.fft.rfft(t.double(), 2 * L)
+    xf, kf, gf = spectrum(x), spectrum(k), spectrum(dy)
+    back = lambda f: torch.fft.irfft(f, 2 * L)[..., :L]
+    assert rel_err(y, back(xf * kf)) <= TOL[dtype]
+    assert rel_err(dx, back(gf * kf.conj())) <= TOL[dtype]
+    assert rel_err(dk, back((gf * xf.conj()).sum(0))) <= 1e-4
+
+
 @pytest.mark.parametrize("B,D,L", SHAPES)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_fwd_matches_oracle(B, D, L, dtype, engine):
