@@ -85,6 +85,35 @@ def test_fwd_matches_oracle(B, D, L, dtype, engine):
     assert rel_err(y, want) <= TOL[dtype]
 
 
+# time-domain kernel: four outputs per thread up to 1024, eight above; a wave's share is 256 or 512
+@pytest.mark.parametrize("L", [3, 4, 5, 255, 256, 257, 1023, 1024, 1025, 1031, 1536, 1537, 2047])
+@pytest.mark.parametrize("B,D", [(1, 5), (3, 2)])
+def test_direct_sums_at_the_shares_edges(B, D, L):
+    """Bar: a chain of L multiply-adds in float32, L half units in the last place (2^-24 each)
+    of the sum of the terms' magnitudes, plus the store's own."""
+    x, k, dy = (t.cuda() for t in _data(B, D, L, torch.float32, 7 * L + B))
+    y = ops.fftconv_fwd(x, k)
+    dx, dk = ops.fftconv_bwd(dy, x, k, torch.float32)
+    lag = torch.arange(L, device="cuda")
+    lag = lag[:, None] - lag[None, :]
+    toeplitz = lambda t: torch.where(lag >= 0, t.double()[..., lag.clamp(min=0)], 0.0)   # [i, s] = t[i - s]
+    kt, xt = toeplitz(k), toeplitz(x)
+    for got, m, v, sums in ((y, kt, x, "dis,bds->bdi"), (dx, kt, dy, "dis,bdi->bds"), (dk, xt, dy, "bdis,bdi->ds")):
+        want = torch.einsum(sums, m, v.double())
+        size = torch.einsum(sums, m.abs(), v.double().abs())
+        assert bool(((got.double() - want).abs() <= (L * B + 1) * 2.0 ** -24 * size).all())
+
+
+def test_direct_sums_stay_causal_for_infinities():
+    L = 1500
+    x, k, _ = (t.cuda() for t in _data(1, 5, L, torch.float32, 1))
+    clean = ops.fftconv_fwd(x, k)
+    for at in (7, 512, 1030):
+        bad = x.clone()
+        bad[..., at] = float("inf")
+        assert torch.equal(ops.fftconv_fwd(bad, k)[..., :at], clean[..., :at])
+
+
 @pytest.mark.parametrize("B,D,L", SHAPES)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_bwd_matches_oracle(B, D, L, dtype, engine):
