@@ -523,6 +523,13 @@ int mega_layer_norm_bwd(const void* dy, const void* x, const void* weight, const
                         const float* rstd, int dtype, int64_t rows, int64_t D, int rms, void* dx,
                         void* dweight, void* dbias, void* workspace, void* stream);
 
+/* Column sums: out (cols) = sum over the rows of x (rows, cols), bfloat16 / float16, float32 inside, in a
+ * fixed order; out has x's type.  A linear layer's bias gradient.  MEGA_ERR_UNSUPPORTED for other
+ * types, rows that are no multiple of 8 long or x off the 16-byte boundaries.
+ *   `workspace`: mega_column_sums_workspace_bytes(rows, cols) bytes. */
+int64_t mega_column_sums_workspace_bytes(int64_t rows, int64_t cols);
+int mega_column_sums(const void* x, int dtype, int64_t rows, int64_t cols, void* out, void* workspace, void* stream);
+
 /* ------------------------------------------------------------------------
  * z -> (q, k): per-head RMSNorm, the two affine maps and the rotary product.
  *

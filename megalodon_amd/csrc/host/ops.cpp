@@ -478,6 +478,17 @@ Tensor weight_grad(const Tensor& g, const Tensor& x) {
   return at::mm(g.t(), x);
 }
 Tensor flat(const Tensor& t) { return t.reshape({-1, t.size(-1)}); }
+// the bias gradient: column sums of g (tokens, out)
+Tensor bias_grad(const Tensor& g) {
+  const int64_t rows = g.size(0), cols = g.size(1);
+  const bool taken = rows >= 1 && cols >= 1 && cols % 8 == 0 && cols <= (1 << 24) &&
+                     (g.scalar_type() == at::kBFloat16 || g.scalar_type() == at::kHalf) && g.is_contiguous() &&
+                     reinterpret_cast<uintptr_t>(g.data_ptr()) % 16 == 0;
+  if (!taken) return g.sum(0);
+  Tensor out = at::empty({cols}, g.options()), ws = bytes(mega_column_sums_workspace_bytes(rows, cols), g);
+  check(mega_column_sums(g.data_ptr(), kernel_code(g), rows, cols, out.data_ptr(), ws.data_ptr(), stream_of(g)), "mega_column_sums");
+  return out;
+}
 // x W^T (+ bias), or x W^T + residual with the residual as the product's accumulator input
 Tensor linear_raw(const Tensor& x, const Tensor& weight, const Optional& bias, const Optional& residual) {
   if (!residual.has_value()) return at::linear(x, weight, bias);
@@ -503,7 +514,7 @@ struct LinearFn : Function<LinearFn> {
     Tensor dx, dw, db, dr;
     if (ctx->needs_input_grad(0)) dx = at::linear(g2, transpose_raw(weight)).view(x.sizes());  // rows along the reduction axis
     if (ctx->needs_input_grad(1)) dw = weight_grad(g2, flat(x));
-    if (has_bias && ctx->needs_input_grad(2)) db = g2.sum(0);
+    if (has_bias && ctx->needs_input_grad(2)) db = bias_grad(g2);
     if (has_residual && ctx->needs_input_grad(has_bias ? 3 : 2)) dr = g[0];
     return {dx, dw, db, dr};
   }
@@ -551,7 +562,7 @@ struct LinearGroupFn : Function<LinearGroupFn> {
         else at::addmm_out(dx, dx, g2, wt.t());
       }
       grads.push_back(ctx->needs_input_grad(edge++) ? weight_grad(g2, x2) : Tensor());
-      if (has_bias[i]) grads.push_back(ctx->needs_input_grad(edge++) ? g2.sum(0) : Tensor());
+      if (has_bias[i]) grads.push_back(ctx->needs_input_grad(edge++) ? bias_grad(g2) : Tensor());
     }
     grads[0] = dx.defined() ? dx.view(x.sizes()) : Tensor();
     grads.push_back(Tensor());
