@@ -1,12 +1,12 @@
-"""`nn.Linear` whose input gradient is computed from a transposed copy of the weight.
+"""`nn.Linear` whose input gradient is computed, for large products, from a transposed copy of the weight.
 
 With model-parallel world size 1 the reference's Column/RowParallelLinear are
 `F.linear` (megalodon/modules/model_parallel/layers.py:222-235,321-341), whose
 backward forms `dx = dy @ W` with W (out, in) read along its rows.  On MI355X
 the library GEMM is 13-24 % faster when both operands run along the reduction
 axis (`dy @ Wt^T` with Wt = W^T contiguous, the same layout the forward
-`x @ W^T` uses), and the tiled transpose of W costs 15-30 us, so the backward
-makes that copy; the weight gradient of the large layers runs on the attention
+`x @ W^T` uses), and the tiled transpose of W costs 5-30 us, so the backward
+makes that copy where the product is large enough to win it back; the weight gradient of the large layers runs on the attention
 operator's product kernel.  The autograd nodes are C++ (csrc/host/ops.cpp).
 Values are those of `F.linear`; parameters keep the names and shapes of
 `nn.Linear`, so state dicts are interchangeable."""
