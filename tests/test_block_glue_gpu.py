@@ -6,6 +6,7 @@ import torch
 import torch.nn.functional as F
 
 from conftest import rel_err
+from megalodon_amd import _lib
 from megalodon_amd import extension as ops
 from megalodon_amd.fused_ops import silu_mul, transpose_last2
 
@@ -19,6 +20,8 @@ pytestmark = pytest.mark.gpu
     (3, 50, 77),        # ragged: element-wise path
     (2, 3, 8, 4096),    # leading dimensions fold into the batch; R far below a tile
     (1, 1, 1),
+    # pieces off the boundaries (256 tiles and more), sides at the edges of a tile; one tile fewer
+    (256, 64, 64), (256, 64, 65), (128, 129, 127), (64, 65, 509), (32, 1021, 73), (16, 257, 900), (51, 135, 301), (255, 100, 100),
 ])
 def test_transpose_is_a_bit_exact_move(shape, dtype):
     g = torch.Generator().manual_seed(sum(shape))
@@ -33,6 +36,12 @@ def test_transpose_of_views_and_unaligned_buffers():
     base = torch.randn(2 * 64 * 128 + 1, device="cuda").bfloat16()
     x = base[1:].view(2, 64, 128)                 # 2-byte aligned only
     assert torch.equal(ops.transpose_last2(x), x.transpose(1, 2).contiguous())
+    for z, rows, cols in ((300, 128, 64), (300, 67, 121)):     # bytes behind the matrices stay what they were
+        out = torch.full((z * rows * cols + 9,), 7.0, device="cuda").bfloat16()
+        y = torch.randn(z, rows, cols, device="cuda").bfloat16()
+        _lib.call("mega_transpose", _lib.ptr(y), _lib.i32(_lib.dtype_code(y.dtype)), _lib.i64(z), _lib.i64(rows),
+                  _lib.i64(cols), _lib.ptr(out[1:]), _lib.stream_ptr(y.device))
+        assert torch.equal(out[1:-8].view(z, cols, rows), y.transpose(1, 2)) and out[0] == 7 and bool((out[-8:] == 7).all())
     v = torch.randn(4, 128, 256, device="cuda").half()[:, :, ::2]   # strided input
     assert torch.equal(ops.transpose_last2(v), v.transpose(1, 2).contiguous())
     e = torch.empty(0, 8, 16, device="cuda", dtype=torch.bfloat16)
