@@ -759,10 +759,9 @@ int mega_timestep_norm_layer_bwd(const void* dy, const void* dmean, const void* 
  * one followed by normalized_feedforward_network.py:74-90 (SwiGLU, no dropout).
  * All activations, weights and cached tensors in `dtype` (MEGA_BF16 / MEGA_F16)
  * unless a type is given; stored norm weights are gamma - 1.  `x`, `y` (B, D).
- * `k_cache` (B, >= length + 1, heads, S / heads) and `v_cache` (B, >= length + 1,
- * heads, E / heads) with `k_stride` / `v_stride` elements between sequences hold
- * `length` keys and values; the new ones are written behind them.  The query
- * sees all length + 1 keys.  p (D, N) float32, q and gamma_hat (D, N) complex64 are
+ * `k_in` (B, length, heads, S / heads) and `v_in` (B, length, heads, E / heads) are the cached
+ * keys and values; `k_out` and `v_out` (the same with length + 1, other memory) receive
+ * them and the new ones behind them.  The query sees all length + 1 keys.  p (D, N) float32, q and gamma_hat (D, N) complex64 are
  * the coefficients of complex_exponential_moving_average.py:100-117, h (B, D, N)
  * complex64 the carried state.  `freqs`: S / heads / 2 complex64 factors of the
  * token's position inside its chunk, or NULL.  rms_weight, ln_weight, ln_bias and the
@@ -771,7 +770,7 @@ int mega_timestep_norm_layer_bwd(const void* dy, const void* dmean, const void* 
 typedef struct mega_block_decode_args {
   int dtype;
   int64_t B, D, S, E, F, heads, G, N; /* sequences, model, q/k, value, FFN widths, heads, norm groups, modes */
-  int64_t length, k_stride, v_stride;
+  int64_t length;
   float tsn_eps, rms_eps, z_eps, ln_eps;
   const void* x;
   const int64_t* prev_count;          /* (B) */
@@ -785,7 +784,8 @@ typedef struct mega_block_decode_args {
   const void *qk_gamma, *qk_beta;     /* (2, S) */
   const float* freqs;
   const void *ln_weight, *ln_bias, *fc1, *fc2, *fc3;
-  void *k_cache, *v_cache;
+  const void *k_in, *v_in;
+  void *k_out, *v_out;
   void* y;
   int64_t* count;
   void *mean, *var;

@@ -2,13 +2,14 @@
 // (the cache branch of megalodon/modules/moving_average_gated_attention.py:283-348
 // followed by normalized_feedforward_network.py:74-90, at sequence length one).
 //
-// The step is bound by reading the block's weights and the cached keys and
+// The step is bound by reading the block's weights once and moving the cached keys and
 // values once: at width 4096 the weights are 514 MB, and operator by operator a
 // step was 59 launches, 0.84 ms for one sequence and 4.1 ms for sixteen (1531 and
-// 3000 cached tokens).  Here it is seven launches, 0.145 and 0.31 ms, cut where a whole row is needed by everybody:
+// 3000 cached tokens).  Here it is seven launches, 0.151 and 0.50 ms, cut where a whole row is needed by everybody:
 //   1. step_kernel    TimestepNorm step, EMA state step, partial square sums of the row
-//   2. skinny_kernel  RMSNorm folded into z, r, h1; v = silu(...) straight into the cache
-//   3. attend_kernel  q, k (norm, affine maps, rotary), new key into the cache, one softmax part per split
+//   2. skinny_kernel  RMSNorm folded into z, r, h1; v = silu(...) straight into the new cache
+//   3. attend_kernel  q, k (norm, affine maps, rotary), one softmax part per split; the old keys and values
+//                     pass into the new cache as they are read, the new key joins them
 //   4. combine_kernel the parts put together, gate silu(r)
 //   5. skinny_kernel  wh2 + h1 + residual, partial moments of the row
 //   6. skinny_kernel  LayerNorm folded into fc1, fc3; silu(a) b
@@ -363,8 +364,11 @@ __global__ __launch_bounds__(NW * kWave, MT == 1 ? 4 : 2) void skinny_kernel(con
 // LPK neighbouring lanes), softmax over the run, and the run's weighted sum of values, each
 // thread owning eight of the value columns so that a value row is one contiguous read of
 // the workgroup.  The first value rows are requested before the scores are known.
-// The partial (max, sum, weighted values) go out in float32.  Sixteen sequences of 3000 keys,
-// four heads, 256 + 2048 wide: 885 MB in 135 us.
+// The partial (max, sum, weighted values) go out in float32.  Every old key and value is read by
+// exactly one workgroup, which writes it to its place in the new cache on the way: a cache that has been
+// handed out is never written again, and the one that continues it is contiguous.  (Appended in place to storage
+// with room the steps took 0.144 and 0.32 ms, but then a cache shares memory with the one it continues; with
+// stores that stay in the caches 0.156 and 0.52.)
 constexpr int kAttendThreads = 256;
 constexpr int kMaxKeys = 1024;  // keys of a run
 constexpr int kAhead = 8;       // value rows in flight per thread
@@ -372,9 +376,8 @@ constexpr int kAhead = 8;       // value rows in flight per thread
 struct AttendParams {
   const uint16_t *z, *gamma, *beta;  // (B, S); (2, S)
   const float* freqs;                // (zh / 2) complex, or null
-  uint16_t* k;                       // cache: key (b, t, head) at b * kb + (t * heads + head) * zh
-  const uint16_t* v;
-  int64_t kb, vb;
+  const uint16_t *k_old, *v_old;     // (B, total - 1, heads, zh | H2)
+  uint16_t *k, *v;                   // (B, total, heads, zh | H2); the last row of v is written already
   float* part;                       // (B * heads, splits, H2)
   float2* ml;                        // (B * heads, splits): max and sum
   int heads, H2, total, splits, per; // total keys with the new one; per = keys of a run
@@ -397,14 +400,16 @@ __global__ __launch_bounds__(kAttendThreads) void attend_kernel(const AttendPara
 
   // value rows: thread column c8 of key group kg
   const int cols = a.H2 >> 3, kgroups = kAttendThreads / cols, c8 = (tid % cols) * 8, kg = tid / cols;
-  const uint16_t* vp = a.v + b * a.vb + static_cast<int64_t>(h) * a.H2 + c8;
-  const int64_t vstep = static_cast<int64_t>(a.heads) * a.H2;
+  const int64_t vstep = static_cast<int64_t>(a.heads) * a.H2, vcol = static_cast<int64_t>(h) * a.H2 + c8;
+  const int old_hi = newest ? nk - 1 : nk;  // keys of the run that the old cache holds
+  const uint16_t* vp = a.v_old + (static_cast<int64_t>(b) * (a.total - 1) + k_lo) * vstep + vcol;
+  uint16_t* vq = a.v + (static_cast<int64_t>(b) * a.total + k_lo) * vstep + vcol;
   uint4 ahead[kAhead];
-  auto request = [&](int i0) {
+  auto request = [&](int i0) {  // rows past the run's end: the last one again, unused
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
-      const int j = i0 + i * kgroups;
-      ahead[i] = load_once(vp + static_cast<int64_t>(k_lo + (j < nk ? j : nk - 1)) * vstep);
+      const int j = i0 + i * kgroups, at = j < nk ? j : nk - 1;
+      ahead[i] = load_once((at < old_hi ? vp : vq) + at * vstep);
     }
   };
   request(kg);
@@ -445,25 +450,26 @@ __global__ __launch_bounds__(kAttendThreads) void attend_kernel(const AttendPara
       finish(a.gamma + S, a.beta + S, kn);
       const uint4 packed = pack8<DT>(kn);
       if (tid < LPK)
-        *reinterpret_cast<uint4*>(a.k + b * a.kb + static_cast<int64_t>(a.total - 1) * S + at) = packed;
+        *reinterpret_cast<uint4*>(a.k + (static_cast<int64_t>(b) * a.total + a.total - 1) * S + at) = packed;
       unpack8<DT>(packed, kn);
     }
   }
-  const uint16_t* kp = a.k + b * a.kb + static_cast<int64_t>(h) * zh + c;
-  const int old_hi = newest ? nk - 1 : nk;  // keys of the run that lie in the cache already
+  const uint16_t* kp = a.k_old + (static_cast<int64_t>(b) * (a.total - 1) + k_lo) * S + h * zh + c;
+  uint16_t* kq = a.k + (static_cast<int64_t>(b) * a.total + k_lo) * S + h * zh + c;
   constexpr int kU = 4;
   for (int j0 = wave * KPW + lane / LPK; j0 - lane / LPK < old_hi; j0 += 4 * KPW * kU) {
     uint4 raw[kU];
 #pragma unroll
     for (int i = 0; i < kU; ++i) {
       const int j = j0 + i * 4 * KPW;
-      raw[i] = old_hi > 0 ? load_once(kp + static_cast<int64_t>(k_lo + (j < old_hi ? j : old_hi - 1)) * S)
+      raw[i] = old_hi > 0 ? load_once(kp + static_cast<int64_t>(j < old_hi ? j : old_hi - 1) * S)
                           : make_uint4(0u, 0u, 0u, 0u);
     }
 #pragma unroll
     for (int i = 0; i < kU; ++i) {
       const int j = j0 + i * 4 * KPW;
       float kv[8], s = 0.f;
+      if (j < old_hi) store_streaming(kq + static_cast<int64_t>(j) * S, raw[i]);
       unpack8<DT>(raw[i], kv);
 #pragma unroll
       for (int e = 0; e < 8; ++e) s += q[e] * kv[e];
@@ -509,6 +515,7 @@ __global__ __launch_bounds__(kAttendThreads) void attend_kernel(const AttendPara
     for (int i = 0; i < kAhead; ++i) {
       const int j = j0 + i * kgroups;
       const float w = j < nk ? score[j] : 0.f;
+      if (j < old_hi) store_streaming(vq + j * vstep, now[i]);
       float vv[8];
       unpack8<DT>(now[i], vv);
 #pragma unroll
@@ -657,8 +664,8 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
   {
     SkinnyParams p{};
     // the wide layers first: the narrow one fills the gaps at the end
-    p.seg[0] = seg(a.wv, none, a.bv, at16(l.tsn), static_cast<uint16_t*>(a.v_cache) + a.length * a.E, a.v_stride, E,
-                   32, kNormNone, 1);
+    p.seg[0] = seg(a.wv, none, a.bv, at16(l.tsn), static_cast<uint16_t*>(a.v_out) + a.length * a.E,
+                   (a.length + 1) * a.E, E, 32, kNormNone, 1);
     p.seg[1] = seg(a.wr, none, a.br, at16(l.cema), at16(l.r), E, E, 32, kNormRms, 0);
     p.seg[2] = seg(a.wh1, none, a.bh1, at16(l.cema), at16(l.h1), D, D, 32, kNormRms, 0);
     p.seg[3] = seg(a.wz, none, a.bz, at16(l.cema), at16(l.z), S, S, 32, kNormRms, 0);
@@ -671,8 +678,8 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
   int splits, per;
   key_runs(static_cast<int64_t>(B) * H, a.length + 1, &splits, &per);
   {
-    AttendParams p{at16(l.z), u16(a.qk_gamma), u16(a.qk_beta), a.freqs, static_cast<uint16_t*>(a.k_cache),
-                   u16(a.v_cache), a.k_stride, a.v_stride, reinterpret_cast<float*>(ws + l.part),
+    AttendParams p{at16(l.z), u16(a.qk_gamma), u16(a.qk_beta), a.freqs, u16(a.k_in), u16(a.v_in),
+                   static_cast<uint16_t*>(a.k_out), static_cast<uint16_t*>(a.v_out), reinterpret_cast<float*>(ws + l.part),
                    reinterpret_cast<float2*>(ws + l.ml), H, H2, static_cast<int>(a.length + 1), splits, per, a.z_eps,
                    1.f / sqrtf(static_cast<float>(zh))};
     const dim3 grid(splits, B * H);
@@ -738,13 +745,11 @@ extern "C" int mega_block_decode(const mega_block_decode_args* a, void* stream) 
   if (!mega_block_decode_supported(a->dtype, a->B, a->D, a->S, a->E, a->F, a->heads, a->G, a->N))
     return set_error(MEGA_ERR_UNSUPPORTED, "%s: sizes outside what the step kernels take", who);
   MEGA_CHECK_ARG(a->length >= 1 && a->length < (1 << 24), "%s: length must be at least 1", who);
-  MEGA_CHECK_ARG(a->k_stride >= (a->length + 1) * a->S && a->v_stride >= (a->length + 1) * a->E,
-                 "%s: the cache has no room for the new token", who);
   for (const void* q : {a->x, a->prev_mean, a->prev_var, a->tsn_weight, a->tsn_bias, a->omega, a->wz, a->wr, a->wh1,
                         a->wv, a->wh2, a->qk_gamma, a->qk_beta, a->fc1, a->fc2, a->fc3,
                         static_cast<const void*>(a->p), static_cast<const void*>(a->q),
                         static_cast<const void*>(a->gamma_hat), static_cast<const void*>(a->h_in),
-                        static_cast<const void*>(a->k_cache), static_cast<const void*>(a->v_cache),
+                        a->k_in, a->v_in, static_cast<const void*>(a->k_out), static_cast<const void*>(a->v_out),
                         static_cast<const void*>(a->y), static_cast<const void*>(a->mean),
                         static_cast<const void*>(a->var), static_cast<const void*>(a->h_out),
                         static_cast<const void*>(a->workspace)})
@@ -754,10 +759,10 @@ extern "C" int mega_block_decode(const mega_block_decode_args* a, void* stream) 
                         a->ln_bias, a->qk_gamma, a->qk_beta, static_cast<const void*>(a->p),
                         static_cast<const void*>(a->q), static_cast<const void*>(a->gamma_hat),
                         static_cast<const void*>(a->h_in), static_cast<const void*>(a->h_out),
-                        static_cast<const void*>(a->k_cache), static_cast<const void*>(a->v_cache),
+                        a->k_in, a->v_in, static_cast<const void*>(a->k_out), static_cast<const void*>(a->v_out),
                         static_cast<const void*>(a->workspace)})
     MEGA_CHECK_ARG(reinterpret_cast<uintptr_t>(q) % 16 == 0, "%s: operands must be 16-byte aligned", who);
-  MEGA_CHECK_ARG(a->k_stride % 8 == 0 && a->v_stride % 8 == 0, "%s: cache strides must be multiples of 8", who);
+  MEGA_CHECK_ARG(a->k_in != a->k_out && a->v_in != a->v_out, "%s: the new cache must not be the old one", who);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (a->dtype == MEGA_BF16) return a->B <= 16 ? run<MEGA_BF16, 1>(*a, s) : run<MEGA_BF16, 2>(*a, s);
   return a->B <= 16 ? run<MEGA_F16, 1>(*a, s) : run<MEGA_F16, 2>(*a, s);

@@ -18,7 +18,6 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
-from .. import _lib
 from ..fused_ops import memory_efficient_dropout, swift_efficient_attention
 
 _FUSED = {"swift": swift_efficient_attention, "fused": swift_efficient_attention}
@@ -81,19 +80,8 @@ class _InnerAttention(nn.Module):
             old_k, old_v, old_len = cache
             total = old_len + new_len
             tail = total % self.chunk_size  # steps of the chunk still open after this call
-            joined = None
-            if k.is_cuda and not torch.is_grad_enabled():
-                # behind the old ones, in storage with room for the tokens to come
-                joined = _lib.host().kv_append(old_k, old_v, k, v, self.chunk_size)
-            if joined is not None:
-                all_k, all_v = joined
-                carried = (all_k, all_v) if tail == total else (all_k[:, total - tail:], all_v[:, total - tail:])
-                if old_k.shape[1] > 0:
-                    k, v = all_k, all_v
-            else:
-                k, v = torch.cat((old_k, k), dim=1), torch.cat((old_v, v), dim=1)
-                carried = (k.detach()[:, total - tail:], v.detach()[:, total - tail:])
-            carried = (*carried, tail)
+            k, v = torch.cat((old_k, k), dim=1), torch.cat((old_v, v), dim=1)
+            carried = (k.detach()[:, total - tail:], v.detach()[:, total - tail:], tail)
 
         q, k, v = self._chunks(q), self._chunks(k), self._chunks(v)
         if self.attn_fn is not None:

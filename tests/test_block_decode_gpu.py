@@ -1,11 +1,13 @@
 """The fused one-token step of a block (csrc/block_decode.hip) against the same step taken operator by
 operator, at the edges of what the kernels take: token tiles (1, 16, 17, 32 sequences), head
 widths, lengths of one key, one run and many runs of keys.  Tolerance: the 16-bit bar, 2e-2."""
+import copy
+import io
+
 import pytest
 import torch
 
 from conftest import rel_err
-from megalodon_amd import _lib
 from megalodon_amd.modules import MegaBlock, RotaryEmbedding
 from megalodon_amd.modules.block_decode import decode_step
 
@@ -74,28 +76,67 @@ def test_last_token_of_a_chunk_empties_the_cache():
         assert decode_step(blk, x, rotary.get_freqs_cis(0, 1), cache) is None  # the next chunk's first token: operators
 
 
-def test_cache_storage_is_shared_only_while_nobody_else_holds_it():
-    """Tokens are appended in place; two continuations of one cache do not touch each other."""
+def _tensors(cache):
+    return [*cache[0][:2], *cache[1], cache[2]]
+
+
+def test_continued_cache_shares_nothing_with_the_old_one():
+    """A cache is a value: continuing it, or writing to what came out, leaves it as it was; what comes out is
+    contiguous and can be copied, saved and continued in any gradient mode."""
     blk = _block(256, 128, 512, 512, 2, 2, 512)
     rotary = RotaryEmbedding(64, 512).cuda()
+    xs = [torch.randn(2, 1, 256, generator=torch.Generator().manual_seed(s)).bfloat16().cuda() for s in range(2)]
+    many = torch.randn(2, 5, 256, generator=torch.Generator().manual_seed(7)).bfloat16().cuda()
+    freqs = rotary.get_freqs_cis(30, 31)
     with torch.no_grad():
         cache = _prompt(blk, 2, 30, 256, 128, 512, 2, torch.bfloat16, rotary)
-        xs = [torch.randn(2, 1, 256, generator=torch.Generator().manual_seed(s)).bfloat16().cuda() for s in range(2)]
-        freqs = rotary.get_freqs_cis(30, 31)
-        where = cache[0][0].data_ptr()
+        before = [t.clone() for t in _tensors(cache)]
         _, first = decode_step(blk, xs[0], freqs, cache)
-        assert first[0][0].data_ptr() == where           # room behind the prompt
-        kept = first[0][0].clone(), first[0][1].clone()
+        kept = [t.clone() for t in _tensors(first)]
         _, second = decode_step(blk, xs[1], freqs, cache)
-        assert second[0][0].data_ptr() != where          # the first continuation is alive
-        assert torch.equal(first[0][0], kept[0]) and torch.equal(first[0][1], kept[1])
-        slice_of_first = first[0][1][:, -1:]
-        del first
-        _, third = decode_step(blk, xs[1], freqs, cache)
-        assert third[0][0].data_ptr() != where           # a view of it still is
-        assert torch.equal(slice_of_first, kept[1][:, -1:])
-        del slice_of_first
-        _, fourth = decode_step(blk, xs[1], freqs, cache)
-        assert fourth[0][0].data_ptr() == where
-        assert torch.equal(fourth[0][1], third[0][1])
-    assert _lib.host() is not None
+        _, longer = blk(many, rotary.get_freqs_cis(30, 35), None, cache)
+        for other in (second, longer):
+            storages = {t.untyped_storage().data_ptr() for t in _tensors(other)}
+            assert not storages & {t.untyped_storage().data_ptr() for t in _tensors(first) + _tensors(cache)}
+        assert all(torch.equal(a, b) for a, b in zip(_tensors(first), kept))
+        copied = copy.deepcopy(first)
+        saved = io.BytesIO()
+        torch.save(first, saved)
+        for c in (first, second, longer):
+            assert c[0][0].is_contiguous() and c[0][1].is_contiguous()
+            for t in _tensors(c):
+                t.zero_()
+        assert all(torch.equal(a, b) for a, b in zip(_tensors(cache), before))
+        saved.seek(0)
+        for c in (copied, torch.load(saved)):
+            assert all(torch.equal(a, b) for a, b in zip(_tensors(c), kept))
+    with torch.inference_mode():
+        inferred = _prompt(blk, 2, 30, 256, 128, 512, 2, torch.bfloat16, rotary)
+    with torch.no_grad():
+        for x, n in ((xs[0], 1), (many, 5)):
+            f = rotary.get_freqs_cis(30, 30 + n)
+            a, b = blk(x, f, None, inferred), blk(x, f, None, cache)
+            assert torch.equal(a[0], b[0]) and all(torch.equal(s, t) for s, t in zip(_tensors(a[1]), _tensors(b[1])))
+
+
+def test_two_streams_continue_one_cache():
+    """Two streams continue one cache at the same time, one of them dropping its result before it is done."""
+    blk = _block(256, 128, 512, 512, 2, 2, 512)
+    rotary = RotaryEmbedding(64, 512).cuda()
+    xs = [torch.randn(2, 1, 256, generator=torch.Generator().manual_seed(s)).bfloat16().cuda() for s in range(2)]
+    freqs = rotary.get_freqs_cis(300, 301)
+    with torch.no_grad():
+        cache = _prompt(blk, 2, 300, 256, 128, 512, 2, torch.bfloat16, rotary)
+        wanted = [decode_step(blk, x, freqs, cache) for x in xs]
+        streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+        torch.cuda.synchronize()
+        for _ in range(20):
+            got = []
+            for x, s in zip(xs, streams):
+                with torch.cuda.stream(s):
+                    y, c = decode_step(blk, x, freqs, cache)
+                    got.append((y, c[0][0][:, -1:].clone()))
+                    del c
+            torch.cuda.synchronize()
+            for (y, k), w in zip(got, wanted):
+                assert torch.equal(y, w[0]) and torch.equal(k, w[1][0][0][:, -1:])
