@@ -22,9 +22,11 @@ py::object block_decode_step(const Tensor& x, const Tensor& k, const Tensor& v, 
   if (dtype != MEGA_BF16 && dtype != MEGA_F16) return py::none();
   const auto dev = x.device();
   if (!x.is_cuda() || static_cast<int>(weights.size()) != kWeights) return py::none();
-  // a forward-mode tangent goes to the operators, which refuse it
-  for (const Tensor* t : {&x, &k, &v, &prev_mean, &prev_var, &hx})
-    if (has_tangent(*t)) return py::none();
+  // a forward-mode tangent goes to the operators, which refuse it, and so does a lazily conjugated or negated
+  // view, which they resolve
+  for (const Tensor* t : {&x, &k, &v, &prev_count, &prev_mean, &prev_var, &hx})
+    if (has_tangent(*t) || lazy(*t)) return py::none();
+  if (freqs.has_value() && lazy(*freqs)) return py::none();
   const auto aligned = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
   for (int i = 0; i < kWeights; ++i) {
     const Optional& w = weights[i];
@@ -33,7 +35,7 @@ py::object block_decode_step(const Tensor& x, const Tensor& k, const Tensor& v, 
       if (may_lack) continue;
       return py::none();
     }
-    if (has_tangent(*w) || w->scalar_type() != type || w->device() != dev || !w->is_contiguous() || !aligned(*w)) return py::none();
+    if (has_tangent(*w) || lazy(*w) || w->scalar_type() != type || w->device() != dev || !w->is_contiguous() || !aligned(*w)) return py::none();
   }
   const int64_t B = x.size(0), D = x.size(2), S = weights[kWz]->size(0), E = weights[kWv]->size(0), F = weights[kFc1]->size(0),
                 N = p.size(1), n = k.size(1);

@@ -41,6 +41,11 @@ inline int code_of(at::ScalarType t) {
   }
 }
 
+// what a tensor says is in its memory: a lazily conjugated or negated view keeps the sign in a bit that neither
+// contiguous() nor data_ptr() looks at
+inline bool lazy(const Tensor& t) { return t.is_conj() || t.is_neg(); }
+inline Tensor stored(const Tensor& t) { return lazy(t) ? t.resolve_conj().resolve_neg() : t; }
+
 // whether a forward-mode derivative travels with the tensor
 inline bool has_tangent(const Tensor& t) { return t._fw_grad(/*level=*/0).defined(); }
 

@@ -157,7 +157,7 @@ Tensor layer_norm_plus_one(const Tensor& x, const Optional& weight, const Option
 Tensor real_freqs(const Optional& freqs, int64_t head_dim, const Tensor& z) {
   if (!freqs.has_value()) return Tensor();
   require(freqs->dim() == 2 && freqs->size(1) == head_dim / 2 && freqs->is_complex(), "qk_norm_rotary: freqs_cis must be complex (positions, head_dim / 2)");
-  return freqs->to(z.device(), at::kComplexFloat).contiguous();
+  return stored(freqs->to(z.device(), at::kComplexFloat)).contiguous();
 }
 std::tuple<Tensor, Tensor, Tensor> qk_raw(const Tensor& z, const Tensor& gamma, const Tensor& beta, const Tensor& fr, int64_t head_dim, double eps) {
   need_gpu({&z, &gamma, &beta});
@@ -395,7 +395,7 @@ py::object cema_state(const Tensor& x, const Tensor& p, const Tensor& log_q, con
   const int64_t B = x.size(0), D = x.size(1);
   if (h0.has_value()) require(h0->scalar_type() == at::kComplexFloat && h0->numel() == B * D * N && h0->device() == x.device(), "cema: the carried state must be complex64 (B, D, N)");
   c10::DeviceGuard guard(x.device());
-  const Tensor xc = rows_of(x), w = as_float(omega), h = some(h0);
+  const Tensor xc = rows_of(x), w = as_float(omega), h = h0.has_value() ? stored(*h0).contiguous() : Tensor();
   Tensor h_last;
   if (last) h_last = at::empty({B, D, N}, x.options().dtype(at::kComplexFloat));
   Tensor y = scan_raw(xc, p.data_ptr<float>(), fptr(log_q), fptr(gamma_hat), fptr(w), fptr(h), fptr(h_last), N);

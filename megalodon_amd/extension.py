@@ -37,7 +37,7 @@ def _as_c64(t: torch.Tensor, name: str, wide: bool = False) -> torch.Tensor:
     want = torch.complex128 if wide else torch.complex64
     if t.dtype != want:
         raise RuntimeError(f"{name} must be {str(want)[6:]} (got {t.dtype})")
-    return t.contiguous()
+    return t.resolve_conj().contiguous()  # a conjugate view keeps its sign in a bit that the pointer does not show
 
 
 def _real_of(wide: bool) -> torch.dtype:
@@ -1266,7 +1266,7 @@ def _freqs_real(freqs_cis: Optional[torch.Tensor], head_dim: int, dev) -> Tuple[
         return None, 1
     if freqs_cis.dim() != 2 or freqs_cis.shape[1] != head_dim // 2 or not freqs_cis.is_complex():
         raise RuntimeError("qk_norm_rotary: freqs_cis must be complex (positions, head_dim / 2)")
-    fr = torch.view_as_real(freqs_cis.to(device=dev, dtype=torch.complex64)).contiguous()
+    fr = torch.view_as_real(freqs_cis.to(device=dev, dtype=torch.complex64).resolve_conj()).contiguous()
     return fr, freqs_cis.shape[0]
 
 
