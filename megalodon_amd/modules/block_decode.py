@@ -42,7 +42,8 @@ def decode_step(block, x: Tensor, freqs_cis: Optional[Tensor], cache):
     tsn, cema, rms, znorm, attn = m["timenorm"], m["cema"], m["rmsnorm"], m["znorm"], m["inner_attention"]
     wz, wr, wh1, wv, wh2 = m["wz"], m["wr"], m["wh1"], m["wv"], m["wh2"]
     ln, fc1, fc2, fc3 = f["norm"], f["fc1"], f["fc2"], f["fc3"]
-    if (not _unheard(mega) or nn_module._global_forward_hooks
+    # (a submodule that is in training mode by itself has its dropouts, which the step does not)
+    if (mega.training or nffn.training or attn.training or not _unheard(mega) or nn_module._global_forward_hooks
             or nn_module._global_forward_pre_hooks or not _plain(nffn, NormalizedFeedForwardNetwork)
             or nffn._parameters.get("alpha") is not None or fc3 is None
             or not _plain(tsn, TimestepNorm) or not _plain(cema, MultiHeadComplexEMA)

@@ -14,10 +14,10 @@ from megalodon_amd.modules.block_decode import decode_step
 pytestmark = pytest.mark.gpu
 
 
-def _block(D, S, E, F, heads, groups, chunk, dtype=torch.bfloat16, affine=True):
+def _block(D, S, E, F, heads, groups, chunk, dtype=torch.bfloat16, affine=True, **dropouts):
     torch.manual_seed(3)
     blk = MegaBlock(model_dim=D, z_dim=S, value_dim=E, num_heads=heads, cema_ndim=16, chunk_size=chunk,
-                    ffn_hidden_dim=F, norm_num_groups=groups, init_std=0.05, norm_affine=affine).cuda().to(dtype).eval()
+                    ffn_hidden_dim=F, norm_num_groups=groups, init_std=0.05, norm_affine=affine, **dropouts).cuda().to(dtype).eval()
     with torch.no_grad():
         for name, p in blk.named_parameters():
             if p.abs().max() == 0:
@@ -140,3 +140,20 @@ def test_two_streams_continue_one_cache():
             torch.cuda.synchronize()
             for (y, k), w in zip(got, wanted):
                 assert torch.equal(y, w[0]) and torch.equal(k, w[1][0][0][:, -1:])
+
+
+@pytest.mark.parametrize("part", ["mega", "mega.inner_attention", "nffn"])
+def test_submodule_in_training_mode_keeps_its_dropout(part):
+    """`block.eval()` and one submodule back in training mode, for instance for Monte Carlo dropout."""
+    blk = _block(256, 128, 512, 512, 2, 2, 512, dropout=0.5, attention_dropout=0.5, hidden_dropout=0.5)
+    rotary = RotaryEmbedding(64, 512).cuda()
+    x = torch.randn(2, 1, 256, generator=torch.Generator().manual_seed(1)).bfloat16().cuda()
+    with torch.no_grad():
+        cache = _prompt(blk, 2, 30, 256, 128, 512, 2, torch.bfloat16, rotary)
+        freqs = rotary.get_freqs_cis(30, 31)
+        a, b = (blk(x, freqs, None, cache)[0] for _ in range(2))
+        assert torch.equal(a, b)
+        blk.get_submodule(part).training = True
+        assert decode_step(blk, x, freqs, cache) is None
+        a, b = (blk(x, freqs, None, cache)[0] for _ in range(2))
+        assert not torch.equal(a, b)
