@@ -34,10 +34,11 @@ def decode_step(block, x: Tensor, freqs_cis: Optional[Tensor], cache):
     if cache_attn is None or hx is None or cache_norm[0] is None or cache_norm[1] is None or cache_norm[2] is None:
         return None
     keys, values, length = cache_attn
-    if length < 1 or keys.shape[1] != length or not x.is_cuda:
-        return None
     mods = block._modules
     mega, nffn = mods["mega"], mods["nffn"]
+    # (a cache is an unfinished chunk: what is longer is refused by the operators)
+    if length < 1 or length >= mega.chunk_size or keys.shape[1] != length or not x.is_cuda:
+        return None
     m, f = mega._modules, nffn._modules
     tsn, cema, rms, znorm, attn = m["timenorm"], m["cema"], m["rmsnorm"], m["znorm"], m["inner_attention"]
     wz, wr, wh1, wv, wh2 = m["wz"], m["wr"], m["wh1"], m["wv"], m["wh2"]

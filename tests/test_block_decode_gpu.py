@@ -157,3 +157,14 @@ def test_submodule_in_training_mode_keeps_its_dropout(part):
         assert decode_step(blk, x, freqs, cache) is None
         a, b = (blk(x, freqs, None, cache)[0] for _ in range(2))
         assert not torch.equal(a, b)
+
+
+def test_cache_of_a_whole_chunk_is_refused():
+    blk = _block(256, 128, 512, 512, 2, 2, 64)
+    rotary = RotaryEmbedding(64, 128).cuda()
+    x = torch.randn(2, 1, 256, generator=torch.Generator().manual_seed(1)).bfloat16().cuda()
+    with torch.no_grad():
+        attn, norm, h = _prompt(blk, 2, 63, 256, 128, 512, 2, torch.bfloat16, rotary)
+        keys, values = (torch.cat((t, t[:, :2]), dim=1) for t in attn[:2])
+        with pytest.raises(RuntimeError):
+            blk(x, rotary.get_freqs_cis(65, 66), None, ((keys, values, 65), norm, h))
