@@ -1,59 +1,62 @@
 // The one-token step of a block on a cache (csrc/block_decode.hip).
 #include "host.hpp"
 
+#include <tuple>
 #include <vector>
 
 namespace mega_host {
 namespace {
 
 using Optional = std::optional<Tensor>;
+// (out, ((keys, values, length), (count, mean, var), state))
+using Step = std::tuple<Tensor, std::tuple<std::tuple<Tensor, Tensor, int64_t>, std::tuple<Tensor, Tensor, Tensor>, Tensor>>;
 
 // The step, or None where the step kernels do not take the sizes, types or layouts (the caller then
 // goes operator by operator).  `weights` in the order of the enumeration below.
 enum { kTsnW, kTsnB, kOmega, kRmsW, kWz, kBz, kWr, kBr, kWh1, kBh1, kWv, kBv, kWh2, kGamma, kBeta, kLnW, kLnB, kFc1, kFc2, kFc3, kWeights };
 
-py::object block_decode_step(const Tensor& x, const Tensor& k, const Tensor& v, const Tensor& prev_count,
+std::optional<Step> block_decode_step(const Tensor& x, const Tensor& k, const Tensor& v, const Tensor& prev_count,
                              const Tensor& prev_mean, const Tensor& prev_var, const Tensor& hx, const Optional& freqs,
                              const std::vector<Optional>& weights, const Tensor& p, const Tensor& q, const Tensor& gamma_hat,
                              int64_t heads, int64_t groups, int64_t chunk, double tsn_eps, double rms_eps, double z_eps,
                              double ln_eps) {
   const auto type = x.scalar_type();
   const int dtype = code_of(type);
-  if (dtype != MEGA_BF16 && dtype != MEGA_F16) return py::none();
+  if (dtype != MEGA_BF16 && dtype != MEGA_F16) return std::nullopt;
   const auto dev = x.device();
-  if (!x.is_cuda() || static_cast<int>(weights.size()) != kWeights) return py::none();
+  if (!x.is_cuda() || static_cast<int>(weights.size()) != kWeights) return std::nullopt;
   // a forward-mode tangent goes to the operators, which refuse it, and so does a lazily conjugated or negated
   // view, which they resolve
   for (const Tensor* t : {&x, &k, &v, &prev_count, &prev_mean, &prev_var, &hx})
-    if (has_tangent(*t) || lazy(*t)) return py::none();
-  if (freqs.has_value() && lazy(*freqs)) return py::none();
+    if (has_tangent(*t) || lazy(*t)) return std::nullopt;
+  if (freqs.has_value() && lazy(*freqs)) return std::nullopt;
   const auto aligned = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
   for (int i = 0; i < kWeights; ++i) {
     const Optional& w = weights[i];
     const bool may_lack = i == kRmsW || i == kBz || i == kBr || i == kBh1 || i == kBv || i == kLnW || i == kLnB;
     if (!w.has_value()) {
       if (may_lack) continue;
-      return py::none();
+      return std::nullopt;
     }
-    if (has_tangent(*w) || lazy(*w) || w->scalar_type() != type || w->device() != dev || !w->is_contiguous() || !aligned(*w)) return py::none();
+    if (has_tangent(*w) || lazy(*w) || w->scalar_type() != type || w->device() != dev || !w->is_contiguous() || !aligned(*w)) return std::nullopt;
   }
   const int64_t B = x.size(0), D = x.size(2), S = weights[kWz]->size(0), E = weights[kWv]->size(0), F = weights[kFc1]->size(0),
                 N = p.size(1), n = k.size(1);
-  if (!mega_block_decode_supported(dtype, B, D, S, E, F, heads, groups, N)) return py::none();
+  if (!mega_block_decode_supported(dtype, B, D, S, E, F, heads, groups, N)) return std::nullopt;
   const auto is = [&](const Tensor& t, at::ScalarType ty, at::IntArrayRef shape) {
     return t.scalar_type() == ty && t.device() == dev && t.sizes() == shape && t.is_contiguous();
   };
   if (!is(prev_count, at::kLong, {B}) || !is(prev_mean, type, {B, groups}) || !is(prev_var, type, {B, groups}) ||
       !is(hx, at::kComplexFloat, {B, D, N}) || !aligned(hx) || !x.is_contiguous())
-    return py::none();
+    return std::nullopt;
   if (k.scalar_type() != type || v.scalar_type() != type || k.device() != dev || v.device() != dev ||
       k.sizes() != at::IntArrayRef({B, n, heads, S / heads}) || v.sizes() != at::IntArrayRef({B, n, heads, E / heads}) || n < 1)
-    return py::none();
+    return std::nullopt;
   if (p.scalar_type() != at::kFloat || q.scalar_type() != at::kComplexFloat || gamma_hat.scalar_type() != at::kComplexFloat ||
       p.numel() != D * N || q.numel() != D * N || gamma_hat.numel() != D * N || !p.is_contiguous() || !q.is_contiguous() ||
       !gamma_hat.is_contiguous() || !aligned(p) || !aligned(q) || !aligned(gamma_hat) || p.device() != dev)
-    return py::none();
-  if (freqs.has_value() && !is(*freqs, at::kComplexFloat, {1, S / heads / 2})) return py::none();
+    return std::nullopt;
+  if (freqs.has_value() && !is(*freqs, at::kComplexFloat, {1, S / heads / 2})) return std::nullopt;
 
   c10::DeviceGuard guard(dev);
   const auto rows = [&](const Tensor& t) {
@@ -91,14 +94,14 @@ py::object block_decode_step(const Tensor& x, const Tensor& k, const Tensor& v, 
   a.workspace = ws.data_ptr();
   check(mega_block_decode(&a, stream_of(x)), "mega_block_decode");
   const int64_t total = n + 1, tail = total % chunk;  // (0: the chunk is closed and its cache given up)
-  return py::make_tuple(y, py::make_tuple(py::make_tuple(k_out.narrow(1, total - tail, tail), v_out.narrow(1, total - tail, tail), tail),
-                                          py::make_tuple(count, mean, var), h));
+  return Step{y, {{k_out.narrow(1, total - tail, tail), v_out.narrow(1, total - tail, tail), tail}, {count, mean, var}, h}};
 }
 
 }  // namespace
 
 void bind_decode(py::module_& m) {
-  m.def("block_decode_step", &block_decode_step);
+  // a launch may wait for room in the stream's queue: not with the interpreter held
+  m.def("block_decode_step", &block_decode_step, py::call_guard<py::gil_scoped_release>());
 }
 
 }  // namespace mega_host

@@ -275,26 +275,26 @@ struct TsnFn : Function<TsnFn> {
 };
 // (y, count, mean, var), or None where the layer has to prepare its operands itself (other element
 // types of weights or statistics, a prior that is trained)
-py::object timestep_norm_layer(const Tensor& x, const Optional& prev_count, const Optional& prev_mean, const Optional& prev_var, const Tensor& prior_count, const Tensor& prior_mean, const Tensor& prior_logv, const Tensor& weight, const Tensor& bias, const Optional& mask, int64_t groups, double eps) {
+std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> timestep_norm_layer(const Tensor& x, const Optional& prev_count, const Optional& prev_mean, const Optional& prev_var, const Tensor& prior_count, const Tensor& prior_mean, const Tensor& prior_logv, const Tensor& weight, const Tensor& bias, const Optional& mask, int64_t groups, double eps) {
   const bool shared = !prev_count.has_value();
-  if (!x.is_cuda() || x.dim() != 3 || code_of(x.scalar_type()) < 0 || x.size(0) < 1 || x.size(1) < 1) return py::none();
-  if (prev_mean.has_value() == shared || prev_var.has_value() == shared) return py::none();
+  if (!x.is_cuda() || x.dim() != 3 || code_of(x.scalar_type()) < 0 || x.size(0) < 1 || x.size(1) < 1) return std::nullopt;
+  if (prev_mean.has_value() == shared || prev_var.has_value() == shared) return std::nullopt;
   const Tensor &count = shared ? prior_count : *prev_count, &mean = shared ? prior_mean : *prev_mean, &var = shared ? prior_logv : *prev_var;
-  if (shared && at::GradMode::is_enabled() && (mean.requires_grad() || var.requires_grad())) return py::none();
+  if (shared && at::GradMode::is_enabled() && (mean.requires_grad() || var.requires_grad())) return std::nullopt;
   const int64_t B = x.size(0), D = x.size(2);
   const auto is = [&](const Tensor& t, at::ScalarType type, int64_t n) { return t.scalar_type() == type && t.device() == x.device() && t.numel() == n && t.is_contiguous(); };
-  if (!is(weight, x.scalar_type(), D) || !is(bias, x.scalar_type(), D) || !is(count, at::kLong, shared ? 1 : B) || !is(mean, x.scalar_type(), shared ? groups : B * groups) || !is(var, x.scalar_type(), shared ? groups : B * groups)) return py::none();
+  if (!is(weight, x.scalar_type(), D) || !is(bias, x.scalar_type(), D) || !is(count, at::kLong, shared ? 1 : B) || !is(mean, x.scalar_type(), shared ? groups : B * groups) || !is(var, x.scalar_type(), shared ? groups : B * groups)) return std::nullopt;
   if (mask.has_value()) {
     if (mask->scalar_type() != at::kBool) fail("padding_mask must be a bool tensor");
-    if (mask->device() != x.device() || mask->numel() != B * x.size(1)) return py::none();
+    if (mask->device() != x.device() || mask->numel() != B * x.size(1)) return std::nullopt;
   }
   c10::DeviceGuard guard(x.device());
   if (wants_grad({&x, &mean, &var, &weight, &bias})) {
     auto o = TsnFn::apply(x, count, mean, var, shared, weight, bias, mask, groups, eps);
-    return py::make_tuple(o[0], o[1], o[2], o[3]);
+    return std::make_tuple(o[0], o[1], o[2], o[3]);
   }
   TsnOut o = tsn_raw(x.contiguous(), count, mean, var, shared, weight, bias, mask, groups, eps);
-  return py::make_tuple(o.y, o.count, o.mean, o.var);
+  return std::make_tuple(o.y, o.count, o.mean, o.var);
 }
 
 // ---- the EMA layer without a carried state ------------------------------------------------------
@@ -377,21 +377,21 @@ struct CemaFn : Function<CemaFn> {
 bool cema_takes(const Tensor& x, int64_t N) {
   return x.is_cuda() && x.dim() == 3 && N >= 1 && N <= 16 && code_of(x.scalar_type()) >= 0 && x.size(2) >= 1 && (x.scalar_type() != at::kFloat || x.size(2) % 8 == 0) && x.size(0) * x.size(1) <= 0x7fffffff;
 }
-py::object cema(const Tensor& x, const Tensor& alpha, const Tensor& delta, const Tensor& theta, const Tensor& gamma, const Tensor& omega) {
-  if (alpha.dim() != 3 || !cema_takes(x, alpha.size(1))) return py::none();
+Optional cema(const Tensor& x, const Tensor& alpha, const Tensor& delta, const Tensor& theta, const Tensor& gamma, const Tensor& omega) {
+  if (alpha.dim() != 3 || !cema_takes(x, alpha.size(1))) return std::nullopt;
   const int64_t D = x.size(1), N = alpha.size(1);
   const auto is = [&](const Tensor& t, int64_t n) { return t.scalar_type() == alpha.scalar_type() && t.device() == x.device() && t.numel() == n && t.is_contiguous(); };
-  if (code_of(alpha.scalar_type()) < 0 || !is(alpha, D * N) || !is(delta, D * N) || !is(theta, D) || !is(gamma, 2 * D * N) || !is(omega, D)) return py::none();
+  if (code_of(alpha.scalar_type()) < 0 || !is(alpha, D * N) || !is(delta, D * N) || !is(theta, D) || !is(gamma, 2 * D * N) || !is(omega, D)) return std::nullopt;
   c10::DeviceGuard guard(x.device());
-  if (wants_grad({&x, &alpha, &delta, &theta, &gamma, &omega})) return py::cast(CemaFn::apply(x, alpha, delta, theta, gamma, omega));
+  if (wants_grad({&x, &alpha, &delta, &theta, &gamma, &omega})) return CemaFn::apply(x, alpha, delta, theta, gamma, omega);
   const Tensor xc = rows_of(x), w = as_float(omega), c = cema_coeffs(alpha, delta, theta, gamma, D, N);
   const float* p = c.data_ptr<float>();
-  return py::cast(scan_raw(xc, p, p + D * N, p + 3 * D * N, fptr(w), nullptr, nullptr, N));
+  return scan_raw(xc, p, p + D * N, p + 3 * D * N, fptr(w), nullptr, nullptr, N);
 }
 // with a carried state and / or the last state wanted, without gradients; p, log_q, gamma_hat float32 / complex64
-py::object cema_state(const Tensor& x, const Tensor& p, const Tensor& log_q, const Tensor& gamma_hat, const Tensor& omega, const Optional& h0, bool last) {
+std::optional<std::tuple<Tensor, Optional>> cema_state(const Tensor& x, const Tensor& p, const Tensor& log_q, const Tensor& gamma_hat, const Tensor& omega, const Optional& h0, bool last) {
   const int64_t N = p.size(1);
-  if (!cema_takes(x, N)) return py::none();
+  if (!cema_takes(x, N)) return std::nullopt;
   const int64_t B = x.size(0), D = x.size(1);
   if (h0.has_value()) require(h0->scalar_type() == at::kComplexFloat && h0->numel() == B * D * N && h0->device() == x.device(), "cema: the carried state must be complex64 (B, D, N)");
   c10::DeviceGuard guard(x.device());
@@ -399,7 +399,7 @@ py::object cema_state(const Tensor& x, const Tensor& p, const Tensor& log_q, con
   Tensor h_last;
   if (last) h_last = at::empty({B, D, N}, x.options().dtype(at::kComplexFloat));
   Tensor y = scan_raw(xc, p.data_ptr<float>(), fptr(log_q), fptr(gamma_hat), fptr(w), fptr(h), fptr(h_last), N);
-  return py::make_tuple(y, last ? py::cast(h_last) : py::object(py::none()));
+  return std::make_tuple(y, last ? Optional(h_last) : std::nullopt);
 }
 
 // ---- attention ------------------------------------------------------------------------------------
@@ -589,10 +589,10 @@ void bind_ops(py::module_& m) {
   m.def("silu_mul", &silu_mul, free());
   m.def("layer_norm_plus_one", &layer_norm_plus_one, free());
   m.def("qk_norm_rotary", &qk_norm_rotary, free());
-  m.def("timestep_norm_layer", &timestep_norm_layer);
-  m.def("tsn_last_workspaces", &tsn_last_workspaces);
-  m.def("cema", &cema);
-  m.def("cema_state", &cema_state);
+  m.def("timestep_norm_layer", &timestep_norm_layer, free());
+  m.def("tsn_last_workspaces", &tsn_last_workspaces, free());
+  m.def("cema", &cema, free());
+  m.def("cema_state", &cema_state, free());
   m.def("attention", &attention, free());
   m.def("linear", &linear, free());
   m.def("linear_group", &linear_group, free());

@@ -120,26 +120,27 @@ def test_continued_cache_shares_nothing_with_the_old_one():
 
 
 def test_two_streams_continue_one_cache():
-    """Two streams continue one cache at the same time, one of them dropping its result before it is done."""
+    """One stream's continuation is dropped while its kernels still wait; the other's has to stay what it is."""
     blk = _block(256, 128, 512, 512, 2, 2, 512)
     rotary = RotaryEmbedding(64, 512).cuda()
     xs = [torch.randn(2, 1, 256, generator=torch.Generator().manual_seed(s)).bfloat16().cuda() for s in range(2)]
     freqs = rotary.get_freqs_cis(300, 301)
     with torch.no_grad():
         cache = _prompt(blk, 2, 300, 256, 128, 512, 2, torch.bfloat16, rotary)
+        before = [t.clone() for t in _tensors(cache)]
         wanted = [decode_step(blk, x, freqs, cache) for x in xs]
-        streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+        late, early = torch.cuda.Stream(), torch.cuda.Stream()
         torch.cuda.synchronize()
-        for _ in range(20):
-            got = []
-            for x, s in zip(xs, streams):
-                with torch.cuda.stream(s):
-                    y, c = decode_step(blk, x, freqs, cache)
-                    got.append((y, c[0][0][:, -1:].clone()))
-                    del c
+        for _ in range(3):
+            with torch.cuda.stream(late):
+                torch.cuda._sleep(10_000_000)
+                first = decode_step(blk, xs[0], freqs, cache)[0]
+            with torch.cuda.stream(early):
+                y, kept = decode_step(blk, xs[1], freqs, cache)
             torch.cuda.synchronize()
-            for (y, k), w in zip(got, wanted):
-                assert torch.equal(y, w[0]) and torch.equal(k, w[1][0][0][:, -1:])
+            assert torch.equal(first, wanted[0][0]) and torch.equal(y, wanted[1][0])
+            assert all(torch.equal(a, b) for a, b in zip(_tensors(kept), _tensors(wanted[1][1])))
+            assert all(torch.equal(a, b) for a, b in zip(_tensors(cache), before))
 
 
 @pytest.mark.parametrize("part", ["mega", "mega.inner_attention", "nffn"])
