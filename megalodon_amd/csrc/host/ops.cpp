@@ -503,6 +503,15 @@ Tensor linear_raw(const Tensor& x, const Tensor& weight, const Optional& bias, c
   shape.back() = weight.size(0);
   return at::addmm(flat(*residual), flat(x), weight.t()).view(shape);
 }
+// A layer's gradients (dx, dW, db) as recorded operations: under create_graph the backward is itself
+// differentiated, so nothing in it may go below autograd or to a kernel that autograd does not know.
+struct LinearGrads {
+  Tensor dx, dw, db;
+};
+LinearGrads linear_recorded(const Tensor& g, const Tensor& x, const Tensor& weight, bool dx, bool dw, bool db) {
+  const Tensor g2 = flat(g);
+  return {dx ? at::mm(g2, weight).view(x.sizes()) : Tensor(), dw ? at::mm(g2.t(), flat(x)) : Tensor(), db ? g2.sum(0) : Tensor()};
+}
 struct LinearFn : Function<LinearFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, const Optional& bias, const Optional& residual) {
     at::AutoDispatchBelowADInplaceOrView below;
@@ -512,11 +521,15 @@ struct LinearFn : Function<LinearFn> {
     return linear_raw(x, weight, bias, residual);
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
-    at::AutoDispatchBelowADInplaceOrView below;
     const auto saved = ctx->get_saved_variables();
     const Tensor &x = saved[0], &weight = saved[1];
     const bool has_bias = ctx->saved_data["bias"].toBool(), has_residual = ctx->saved_data["residual"].toBool();
     c10::DeviceGuard guard(x.device());
+    if (at::GradMode::is_enabled()) {
+      auto r = linear_recorded(g[0], x, weight, ctx->needs_input_grad(0), ctx->needs_input_grad(1), has_bias && ctx->needs_input_grad(2));
+      return {r.dx, r.dw, r.db, has_residual && ctx->needs_input_grad(has_bias ? 3 : 2) ? g[0] : Tensor()};
+    }
+    at::AutoDispatchBelowADInplaceOrView below;
     const Tensor g2 = flat(g[0]);
     Tensor dx, dw, db, dr;
     if (ctx->needs_input_grad(0)) dx = (turned(g2, weight) ? at::linear(g2, transpose_raw(weight)) : at::mm(g2, weight)).view(x.sizes());
@@ -551,15 +564,27 @@ struct LinearGroupFn : Function<LinearGroupFn> {
     return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
-    at::AutoDispatchBelowADInplaceOrView below;
     const auto saved = ctx->get_saved_variables();
     const auto has_bias = ctx->saved_data["bias"].toIntVector();
     const Tensor& x = saved[0];
     c10::DeviceGuard guard(x.device());
-    const Tensor x2 = flat(x);
     Tensor dx;
     variable_list grads{Tensor()};
     size_t edge = 1;
+    if (at::GradMode::is_enabled()) {
+      for (size_t i = 0; i < has_bias.size(); ++i) {
+        const bool dw = ctx->needs_input_grad(edge++), db = has_bias[i] && ctx->needs_input_grad(edge++);
+        auto r = linear_recorded(g[i], x, saved[1 + i], ctx->needs_input_grad(0), dw, db);
+        if (r.dx.defined()) dx = dx.defined() ? dx + r.dx : r.dx;
+        grads.push_back(r.dw);
+        if (has_bias[i]) grads.push_back(r.db);
+      }
+      grads[0] = dx;
+      grads.push_back(Tensor());
+      return grads;
+    }
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor x2 = flat(x);
     for (size_t i = 0; i < has_bias.size(); ++i) {
       const Tensor& w = saved[1 + i];
       const Tensor g2 = flat(g[i]);

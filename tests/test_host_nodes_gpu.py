@@ -8,6 +8,7 @@ import torch.autograd.forward_ad as fwad
 from megalodon_amd import fused_ops as ops
 from megalodon_amd.modules import MegaBlock, MultiHeadComplexEMA, TimestepNorm
 from megalodon_amd.modules.block_decode import decode_step
+from megalodon_amd.modules.linear import Linear, linear_group
 
 pytestmark = pytest.mark.gpu
 
@@ -105,3 +106,36 @@ def test_tangent_in_a_step_is_refused():
     x = _randn(2, 1, 256)
     with torch.no_grad(), fwad.dual_level(), pytest.raises(RuntimeError):
         blk(fwad.make_dual(x, torch.ones_like(x)), None, None, cache)
+
+
+@pytest.mark.parametrize("layers,bias,residual", [(1, True, False), (1, False, True), (3, True, False)])
+def test_linear_second_derivatives(layers, bias, residual):
+    """A gradient penalty: the gradients of |dy/dx|^2 (+ |dy/dW|^2) against those of float32 `F.linear`.  Each
+    product rounds to bfloat16 once per pass, 2^-8 of its size, and there are up to four in a row: 2e-2."""
+    torch.manual_seed(2)
+    mods = [Linear(64, 96, bias=bias).cuda().bfloat16() for _ in range(layers)]
+    x0, r0 = _randn(40, 64), _randn(40, 96) if residual else None
+    results = []
+    for native in (True, False):
+        kind = torch.bfloat16 if native else torch.float32
+        x = x0.to(kind).requires_grad_(True)
+        params = [p.detach().to(kind).requires_grad_(True) for m in mods for p in m.parameters()]
+        for m, at in zip(mods, range(0, len(params), 2 if bias else 1)):
+            m.weight = torch.nn.Parameter(params[at].detach())
+            m.bias = torch.nn.Parameter(params[at + 1].detach()) if bias else None
+        leaves = [x] + [p for m in mods for p in m.parameters()]
+        if not native:
+            ys = [torch.nn.functional.linear(x, m.weight, m.bias) for m in mods]
+        elif layers > 1:
+            ys = linear_group(x, mods)
+        else:
+            ys = [mods[0](x, residual=r0)] if residual else [mods[0](x)]
+        if residual and not native:
+            ys = [y + r0.float() for y in ys]
+        loss = sum((y.float() ** 2).mean() for y in ys)
+        first = torch.autograd.grad(loss, leaves, create_graph=True)
+        assert all(g.grad_fn is not None for g in first)
+        penalty = sum((g.float() ** 2).sum() for g in first)
+        results.append(torch.autograd.grad(penalty, leaves))
+    for a, b in zip(*results):
+        assert (a.float() - b).norm() <= 2e-2 * b.norm()
