@@ -195,7 +195,7 @@ std::tuple<Tensor, Tensor> qk_norm_rotary(const Tensor& z, const Tensor& gamma, 
   c10::OptionalDeviceGuard guard;
   if (z.is_cuda()) guard.reset_device(z.device());
   const Tensor fr = real_freqs(freqs, head_dim, z);
-  if (wants_grad({&z, &gamma, &beta})) {
+  if (wants_grad({&z, &gamma, &beta}) || (fr.defined() && has_tangent(fr))) {
     auto qk = QkFn::apply(z, gamma, beta, fr.defined() ? Optional(fr) : Optional(), head_dim, eps);
     return {qk[0], qk[1]};
   }

@@ -45,6 +45,13 @@ def test_tangent_is_refused(name, grad_mode):
             fn(fwad.make_dual(args[0], torch.ones_like(args[0])), *args[1:])
 
 
+def test_tangent_of_rotary_factors_is_refused():
+    z, gamma, beta = _randn(2, 24, 128), _randn(2, 128), _randn(2, 128)
+    f = torch.polar(torch.ones(24, 32), torch.rand(24, 32)).cuda()
+    with torch.no_grad(), fwad.dual_level(), pytest.raises(RuntimeError):
+        ops.qk_norm_rotary(z, gamma, beta, fwad.make_dual(f, torch.ones_like(f)), 64, 1e-5)
+
+
 def _scatter(t):
     """The same values at an odd element offset and, where it has several axes, with other strides."""
     if t.dim() < 2:
