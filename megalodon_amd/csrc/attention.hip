@@ -115,7 +115,7 @@ struct GemmParams {
   int items;               // per_batch * batch
   int ta, tb;   // operand is k-major: element (m, k) at [k * ld + m]
   int kvb;      // rows of k that a k-major B holds when K has been rounded up behind them (0: all K); A holds
-                // zeros there, so those rows of B may hold anything and the last real one stands in for them
+                // zeros there, and zeros stand in for those rows of B (0 times an infinity would be NaN)
   int ms;       // rows of C to store when M has been rounded up (0: all M)
   int n_group;  // plain schedule: tiles numbered n fastest inside bands of n_group column tiles, then m,
                 // then band (0: one band) -- the 32 tiles an XCD works on at a time then share fewer
@@ -441,6 +441,16 @@ constexpr size_t kDmaLds = sizeof(uint16_t) * (8 * 128 * (64 + 8) > kStages * kD
 __device__ __forceinline__ void load_to_lds16(const void* base, uint32_t offset, uint32_t lds_dst) {
   asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_dst));
 }
+// The same through a buffer descriptor: bytes at and behind its end arrive as zeros.
+__device__ __forceinline__ u32x4 buffer_of(const void* base, uint32_t bytes) {
+  const uint64_t a = reinterpret_cast<uint64_t>(base);
+  return u32x4{static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(a))),
+               static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(a >> 32) & 0xffff)),
+               static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(bytes))), 0x00020000u};
+}
+__device__ __forceinline__ void load_to_lds16(u32x4 buffer, uint32_t offset, uint32_t lds_dst) {
+  asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(offset), "s"(buffer), "s"(lds_dst));
+}
 
 // RAG: p.kvb and p.ms are set (two k-major operands)
 template <int DT, bool TA, bool TB, bool RAG = false>
@@ -518,34 +528,30 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_kernel(const GemmParams
   // of piece pc fetches what belongs at position l of the piece (addresses clamped into
   // the matrix, so every lane always loads)
   uint32_t offa[NL], offb[NL];
-  int rowb[NL];  // RAG: offb is the column part, the row is clamped per request
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
     const int pc = wave + 8 * i;
     const int krow = 2 * pc + (lane >> 5), cm = (lane & 31) ^ ((krow & 3) << 2);  // k-major piece
-    rowb[i] = kb + krow;
     const int row = 16 * pc + (lane >> 2), ck = (lane & 3) ^ ((lane >> 4) & 3);   // k-contiguous piece
     if (TA) offa[i] = static_cast<uint32_t>(((kb + krow) * p.lda + min(m0 + cm * 8, p.M - 8)) * 2);
     else offa[i] = static_cast<uint32_t>((static_cast<int64_t>(min(m0 + row, p.M - 1)) * p.lda + kb + ck * 8) * 2);
-    if (TB) offb[i] = static_cast<uint32_t>(((RAG ? 0 : kb + krow) * p.ldb + min(n0 + cm * 8, p.N - 8)) * 2);
+    if (TB) offb[i] = static_cast<uint32_t>(((kb + krow) * p.ldb + min(n0 + cm * 8, p.N - 8)) * 2);
     else offb[i] = static_cast<uint32_t>((static_cast<int64_t>(min(n0 + row, p.N - 1)) * p.ldb + kb + ck * 8) * 2);
   }
   const uint32_t stepa = static_cast<uint32_t>((TA ? p.lda : 1) * kSlab * 2);
   const uint32_t stepb = static_cast<uint32_t>((TB ? p.ldb : 1) * kSlab * 2);
   const uint32_t lds_wave = __builtin_amdgcn_readfirstlane(
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint16_t*)(smem))) + wave * 1024);
+  // RAG: B ends with row kvb - 1
+  const u32x4 bufb = RAG ? buffer_of(B, static_cast<uint32_t>(((p.kvb - 1) * p.ldb + p.N) * 2)) : u32x4{};
   // request number n of a slab: n = 0, 2 the two pieces of A, n = 1, 3 those of B
   auto request_one = [&](int s, int stage, int n) {
     const uint32_t sc = static_cast<uint32_t>(min(s, nslab - 1));
     const uint32_t dst = lds_wave + static_cast<uint32_t>(stage * kDmaStage + (n >> 1) * 8 * 512 + (n & 1) * kDmaOperand) * 2;
     if (n & 1) {
-      if constexpr (RAG) {
-        static_assert(TB, "rows of k");
-        const uint32_t row = static_cast<uint32_t>(min(rowb[n >> 1] + static_cast<int>(sc) * kSlab, p.kvb - 1));
-        load_to_lds16(B, offb[n >> 1] + row * static_cast<uint32_t>(p.ldb * 2), dst);
-      } else {
-        load_to_lds16(B, offb[n >> 1] + sc * stepb, dst);
-      }
+      static_assert(TB || !RAG, "rows of k");
+      if constexpr (RAG) load_to_lds16(bufb, offb[n >> 1] + sc * stepb, dst);
+      else load_to_lds16(B, offb[n >> 1] + sc * stepb, dst);
     } else {
       load_to_lds16(A, offa[n >> 1] + sc * stepa, dst);
     }
@@ -1053,7 +1059,6 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_a64_kernel(const GemmPa
   // 128 bytes each, the chunk at position c of row r holds k chunk c ^ ((r >> 1) & 7)); B: the
   // pieces w, w + 8 (2 rows of k, 512 bytes each).  Addresses are clamped into the matrix.
   uint32_t offa[4], offb[2];
-  int rowb[2];  // RAG: offb is the column part, the row is clamped per request
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int pc = wave + 8 * i;
@@ -1064,13 +1069,14 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_a64_kernel(const GemmPa
   for (int i = 0; i < 2; ++i) {
     const int pc = wave + 8 * i;
     const int krow = 2 * pc + (lane >> 5), cm = (lane & 31) ^ ((krow & 3) << 2);
-    rowb[i] = kb + krow;
-    offb[i] = static_cast<uint32_t>(((RAG ? 0 : kb + krow) * p.ldb + min(n0 + cm * 8, p.N - 8)) * 2);
+    offb[i] = static_cast<uint32_t>(((kb + krow) * p.ldb + min(n0 + cm * 8, p.N - 8)) * 2);
   }
   const uint32_t stepa = static_cast<uint32_t>(kSlab64 * 2);
   const uint32_t stepb = static_cast<uint32_t>(p.ldb * kSlab * 2);
   const uint32_t lds_wave = __builtin_amdgcn_readfirstlane(
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint16_t*)(smem))) + wave * 1024);
+  // RAG: B ends with row kvb - 1
+  const u32x4 bufb = RAG ? buffer_of(B, static_cast<uint32_t>(((p.kvb - 1) * p.ldb + p.N) * 2)) : u32x4{};
   // A slab ja into A buffer ab (4 requests), B slab s into B buffer bb (2 requests); slabs past the
   // end ask for the last one again, so that every step issues the same number of requests
   auto request_a = [&](int ja, int ab, int n) {
@@ -1079,9 +1085,9 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_a64_kernel(const GemmPa
   };
   auto request_b = [&](int sb, int bb, int n) {
     const uint32_t sc = static_cast<uint32_t>(min(sb, nslab - 1));
-    const uint32_t off = RAG ? offb[n] + static_cast<uint32_t>(min(rowb[n] + static_cast<int>(sc) * kSlab, p.kvb - 1)) * static_cast<uint32_t>(p.ldb * 2)
-                             : offb[n] + sc * stepb;
-    load_to_lds16(B, off, lds_wave + static_cast<uint32_t>(kA64BBase + bb * kDmaOperand + n * 8 * 512) * 2);
+    const uint32_t off = offb[n] + sc * stepb, dst = lds_wave + static_cast<uint32_t>(kA64BBase + bb * kDmaOperand + n * 8 * 512) * 2;
+    if constexpr (RAG) load_to_lds16(bufb, off, dst);
+    else load_to_lds16(B, off, dst);
   };
 
   // fragment side: as in gemm_dma_kernel, k-step `set` of a 32-k step takes k = 16 g + 8 set + e

@@ -1,7 +1,8 @@
 """Attention through autograd at lengths off the products' slabs (32 queries, 64 keys) and at their
 edges, where the probabilities are kept with rows and columns of zeros behind the real ones, against a
 float32 reference; values next to the last row are poisoned in the tensor behind to show that
-nothing of it is used.  Tolerance: the 16-bit bar, 2e-2."""
+nothing of it is used.  Infinities in the last real row reach what reads it, and nothing else.
+Tolerance: the 16-bit bar, 2e-2."""
 import pytest
 import torch
 
@@ -58,3 +59,33 @@ def test_forward_and_gradients(B, L1, L2, NH, H1, H2, causal, dtype):
         assert rel_err(got, ref) <= 2e-2 or (got.float().cpu() - ref).abs().max() <= 2e-2
     with torch.no_grad():
         assert torch.equal(swift_efficient_attention(qc, kc, vc, scale, 0.0, causal, True), y)
+
+
+@pytest.mark.parametrize("B,L,NH,H1,H2,causal,dtype", [
+    (1, 33, 2, 64, 64, True, torch.bfloat16),
+    (2, 77, 1, 128, 72, False, torch.float16),
+    (1, 300, 2, 256, 256, False, torch.bfloat16),
+    (1, 1021, 1, 64, 320, True, torch.bfloat16),
+])
+def test_infinite_last_rows(B, L, NH, H1, H2, causal, dtype):
+    """An infinite value row makes the outputs that see it infinite, an infinite row of the output's gradient the
+    value gradients; rows of zeros behind them must not turn that into NaN."""
+    g = torch.Generator().manual_seed(L)
+    q, k = (torch.randn(B, L, NH, H1, generator=g).to(dtype).cuda() for _ in range(2))
+    v, dy = (torch.randn(B, L, NH, H2, generator=g).to(dtype).cuda() for _ in range(2))
+    v_inf, dy_inf = v.clone(), dy.clone()
+    v_inf[:, -1] = float("inf")
+    dy_inf[:, -1] = float("inf")
+    scale = 0.1 * H1 ** -0.5  # every key has a probability that 16 bits hold
+    with torch.no_grad():
+        y = swift_efficient_attention(q, k, v_inf, scale, 0.0, causal, True)
+        finite = swift_efficient_attention(q, k, v, scale, 0.0, causal, True)
+    assert torch.isposinf(y[:, -1]).all()
+    if not causal:
+        assert torch.isposinf(y).all()
+    else:  # (rows that share a tile with the last one multiply it by a zero probability)
+        clear = (L - 1) // 256 * 256
+        assert torch.equal(y[:, :clear], finite[:, :clear])
+    leaves = [t.clone().requires_grad_(True) for t in (q, k, v)]
+    swift_efficient_attention(*leaves, scale, 0.0, causal, True).backward(dy_inf)
+    assert torch.isposinf(leaves[2].grad).all()
