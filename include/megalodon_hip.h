@@ -707,11 +707,11 @@ int mega_cema_layer_scan_bwd(const void* dy, const void* x, const float* p, cons
 
 /* mega_attention_fwd / _bwd for a caller that hands the probabilities from the forward to the backward and
  * nowhere else: their layout is the library's own, `saved` holds mega_attention_layer_saved_elements
- * elements of the tensors' type (the backward's workspace as many again), and lengths off the kernels' slabs
- * run on the same kernels as whole ones.  There 16-bit operands must be 16-byte aligned and
- * scale positive. */
+ * elements of the tensors' type (the backward's workspace as many again; sizes and scale as in the calls), and
+ * lengths off the kernels' slabs run on the same kernels as whole ones.  There 16-bit operands must be 16-byte
+ * aligned. */
 int64_t mega_attention_layer_saved_elements(int dtype, int64_t B, int64_t L1, int64_t L2, int64_t NH,
-                                            int64_t H1, int64_t H2);
+                                            int64_t H1, int64_t H2, double scale);
 int mega_attention_layer_fwd(const void* q, const void* k, const void* v, int dtype, int64_t B,
                              int64_t L1, int64_t L2, int64_t NH, int64_t H1, int64_t H2,
                              double scale, int causal, void* y, void* saved, void* stream);

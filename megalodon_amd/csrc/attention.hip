@@ -41,6 +41,7 @@ int softmax_wide_fwd(T* x, int64_t Z, int64_t L1, int64_t L2, int causal, const 
 template <typename T>
 int softmax_wide_bwd(const T* y, T* dy, int64_t Z, int64_t L1, int64_t L2, int causal, hipStream_t s);
 // scores + softmax in one kernel (attention_scores.hip); -1: shape outside that kernel
+bool attention_probs_takes(int dtype, int64_t B, int64_t L1, int64_t L2, int64_t NH, int64_t H1, float scale);
 int attention_probs_fused(int dtype, const uint16_t* q, const uint16_t* k, uint16_t* w, int64_t B, int64_t L1,
                           int64_t L2, int64_t NH, int64_t H1, float scale, int causal, int fill, int64_t pitch,
                           int64_t zrows, hipStream_t s);
@@ -1562,9 +1563,10 @@ struct PLayout {
 // whole slabs (zeros behind the real rows and columns) every product runs on the kernels that send
 // slabs from memory straight into LDS; with rows of, say, 1021 elements none of the five could
 // (the bounds-checked kernel: 240 instead of 60 us for a 4 x 2 x 1021 x 1021 by 2048 product).
-PLayout layer_layout(int dtype, int64_t L1, int64_t L2, int64_t H1, int64_t H2) {
-  if (dtype != MEGA_BF16 && dtype != MEGA_F16) return {L1, L2};
-  if ((L1 % kSlab == 0 && L2 % kSlab64 == 0) || (H1 != 64 && H1 != 128 && H1 != 256) || H2 % 8 != 0) return {L1, L2};
+PLayout layer_layout(int dtype, int64_t B, int64_t L1, int64_t L2, int64_t NH, int64_t H1, int64_t H2, double scale) {
+  if ((L1 % kSlab == 0 && L2 % kSlab64 == 0) || H2 % 8 != 0) return {L1, L2};
+  // the padded rows and columns are written by the scores kernel alone
+  if (!attention_probs_takes(dtype, B, L1, L2, NH, H1, static_cast<float>(scale))) return {L1, L2};
   const PLayout l{(L1 + kSlab - 1) / kSlab * kSlab, (L2 + kSlab64 - 1) / kSlab64 * kSlab64};
   return l.pitch <= 4096 ? l : PLayout{L1, L2};  // the softmax backward holds a row in registers
 }
@@ -1578,7 +1580,7 @@ int attn_fwd_impl(const uint16_t* q, const uint16_t* k, const uint16_t* v, int64
   int rc = drop ? -1 : attention_probs_fused(DT, q, k, w, B, L1, L2, NH, H1, scale, causal, fill, l.pitch, l.zrows, s);
   if (rc > 0) return rc;
   if (rc < 0) {
-  MEGA_CHECK_ARG(!rag, "attention: operands must be 16-byte aligned and scale positive for lengths off the slab");
+  MEGA_CHECK_ARG(!rag, "attention: operands must be 16-byte aligned for lengths off the slab");
   // S = scale Q K^T  -> w
   GemmParams g{};
   g.A = q; g.B = k; g.C = w; g.M = (int)L1; g.N = (int)L2; g.K = (int)H1;
@@ -1675,7 +1677,7 @@ static int attention_fwd_entry(const char* who, const void* q, const void* k, co
   if (B == 0 || L1 == 0) return MEGA_OK;
   MEGA_CHECK_ARG(q && k && v && y && w, "%s: null pointer", who);
   MEGA_CHECK_ARG(L2 >= 1, "%s: no keys", who);
-  const PLayout l = layer ? layer_layout(dtype, L1, L2, H1, H2) : PLayout{L1, L2};
+  const PLayout l = layer ? layer_layout(dtype, B, L1, L2, NH, H1, H2, scale) : PLayout{L1, L2};
   hipStream_t s = static_cast<hipStream_t>(stream);
   // causal == 2: as 1, but w need only hold what mega_attention_bwd reads
   const int fill = causal == 2 ? 0 : 1;
@@ -1744,7 +1746,7 @@ static int attention_bwd_entry(const void* dy, const void* q, const void* k, con
                                       static_cast<const double*>(w), B, L1, L2, NH, H1, H2, scale, causal,
                                       static_cast<double*>(dq), static_cast<double*>(dk), static_cast<double*>(dv),
                                       static_cast<double*>(workspace), s);
-  const PLayout l = layer ? layer_layout(dtype, L1, L2, H1, H2) : PLayout{L1, L2};
+  const PLayout l = layer ? layer_layout(dtype, B, L1, L2, NH, H1, H2, scale) : PLayout{L1, L2};
   auto u = [](const void* p) { return static_cast<const uint16_t*>(p); };
   auto m = [](void* p) { return static_cast<uint16_t*>(p); };
   if (dtype == MEGA_BF16)
@@ -1763,9 +1765,9 @@ extern "C" int mega_attention_bwd(const void* dy, const void* q, const void* k, 
 }
 
 extern "C" int64_t mega_attention_layer_saved_elements(int dtype, int64_t B, int64_t L1, int64_t L2, int64_t NH,
-                                                       int64_t H1, int64_t H2) {
+                                                       int64_t H1, int64_t H2, double scale) {
   if (B < 0 || L1 < 0 || L2 < 0 || NH < 1 || H1 < 1 || H2 < 1) return 0;
-  const PLayout l = layer_layout(dtype, L1, L2, H1, H2);
+  const PLayout l = layer_layout(dtype, B, L1, L2, NH, H1, H2, scale);
   return B * NH * l.zrows * l.pitch;
 }
 

@@ -432,11 +432,18 @@ int launch_probs(const ProbsParams& p, hipStream_t s) {
 
 }  // namespace
 
+// Whether attention_probs_fused takes these sizes and this scale, for operands on 16-byte boundaries.
+bool attention_probs_takes(int dtype, int64_t B, int64_t L1, int64_t L2, int64_t NH, int64_t H1, float scale) {
+  if ((dtype != MEGA_BF16 && dtype != MEGA_F16) || (H1 != 64 && H1 != 128 && H1 != 256)) return false;
+  if (!(scale > 0.f) || !(scale < 1e30f) || L1 < 1 || L2 < 1) return false;
+  return L2 * NH * H1 < (1ll << 30) && B * NH * ((L1 + kRows - 1) / kRows) < (1ll << 31);
+}
+
 // w = causal softmax of scale q k^T for 16-bit q (B, L1, NH, H1), k (B, L2, NH, H1), w (B, NH, zrows, pitch)
 // with zrows in L1 .. L1 rounded up to 32 and pitch >= L2.
 // Returns MEGA_OK, an error, or -1 when the shape is outside this kernel (the caller then runs the
-// product, softmax and zero fill as separate kernels): head widths other than 64, 128, 256, row
-// pitches that are not a multiple of 8, operands that are not 16-byte aligned, scale <= 0.
+// product, softmax and zero fill as separate kernels): what attention_probs_takes refuses, row
+// pitches that are not a multiple of 8, operands that are not 16-byte aligned.
 // With `causal`, row r is written up to the end of the 64-key tile that holds the last key of the
 // row block (256 rows) it belongs to, with zeros behind its own last key; `fill` writes the zeros
 // up to the end of the row as well (always done when L2 > L1, where the backward products of the
@@ -445,10 +452,8 @@ int attention_probs_fused(int dtype, const uint16_t* q, const uint16_t* k, uint1
                           int64_t L2, int64_t NH, int64_t H1, float scale, int causal, int fill, int64_t pitch,
                           int64_t zrows, hipStream_t s) {
   const auto a16 = [](const void* x) { return reinterpret_cast<uintptr_t>(x) % 16 == 0; };
-  if (!(H1 == 64 || H1 == 128 || H1 == 256) || pitch % 8 != 0 || !a16(q) || !a16(k) || !a16(w)) return -1;
-  if (!(scale > 0.f) || !(scale < 1e30f)) return -1;
+  if (!attention_probs_takes(dtype, B, L1, L2, NH, H1, scale) || pitch % 8 != 0 || !a16(q) || !a16(k) || !a16(w)) return -1;
   const int64_t MT = (L1 + kRows - 1) / kRows;
-  if (L2 * NH * H1 >= (1ll << 30) || B * NH * MT >= (1ll << 31) || L1 < 1 || L2 < 1) return -1;
   ProbsParams p{};
   p.q = q; p.k = k; p.w = w;
   p.L1 = (int)L1; p.L2 = (int)L2; p.NH = (int)NH; p.Z = (int)(B * NH); p.MT = (int)MT;

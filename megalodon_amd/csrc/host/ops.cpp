@@ -423,7 +423,7 @@ std::tuple<Tensor, Tensor> attention_raw(const Tensor& q, const Tensor& k, const
   const AttnDims d = attn_dims(q, k, v);
   const int code = kernel_code(q);
   Tensor y = at::empty({d.B, d.L1, d.NH, d.H2}, v.options());
-  Tensor saved = at::empty({mega_attention_layer_saved_elements(code, d.B, d.L1, d.L2, d.NH, d.H1, d.H2)}, v.options());
+  Tensor saved = at::empty({mega_attention_layer_saved_elements(code, d.B, d.L1, d.L2, d.NH, d.H1, d.H2, scale)}, v.options());
   check(mega_attention_layer_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), code, d.B, d.L1, d.L2, d.NH, d.H1, d.H2, scale, causal, y.data_ptr(), saved.data_ptr(), stream_of(q)), "mega_attention_layer_fwd");
   return {y, saved};
 }

@@ -41,3 +41,21 @@ def test_attention_rejects_an_unknown_causal_code():
               ctypes.c_double(1.0), ctypes.c_int(3), null, null, null, null)
     assert code == 1
     assert b"causal" in lib.mega_last_error()
+
+
+def test_attention_layer_pads_only_what_the_scores_kernel_writes():
+    """Rows and columns behind the real ones exist only where the kernel that writes them takes the call: the same
+    sizes and scales, or the forward would refuse what plain rows take."""
+    fn = _lib.load().mega_attention_layer_saved_elements
+    fn.restype = ctypes.c_int64
+    i64 = ctypes.c_int64
+
+    def saved(L, heads, width, scale, dtype=1):
+        return fn(ctypes.c_int(dtype), i64(1), i64(L), i64(L), i64(heads), i64(width), i64(64), ctypes.c_double(scale))
+
+    assert saved(1021, 2, 256, 1.0) == 2 * 1024 * 1024
+    for scale in (1e30, 3e38, 1e300, 0.0, -1.0, float("nan")):
+        assert saved(1021, 2, 256, scale) == 2 * 1021 * 1021
+    assert saved(1021, 5000, 256, 1.0) == 5000 * 1021 * 1021   # a batch entry of 2^30 elements and more
+    assert saved(1021, 2, 96, 1.0) == 2 * 1021 * 1021
+    assert saved(1021, 2, 256, 1.0, dtype=0) == 2 * 1021 * 1021

@@ -89,3 +89,22 @@ def test_infinite_last_rows(B, L, NH, H1, H2, causal, dtype):
     leaves = [t.clone().requires_grad_(True) for t in (q, k, v)]
     swift_efficient_attention(*leaves, scale, 0.0, causal, True).backward(dy_inf)
     assert torch.isposinf(leaves[2].grad).all()
+
+
+@pytest.mark.parametrize("L", [64, 77])
+def test_scale_beyond_the_scores_kernel(L):
+    """Scales from 1e30 take the separate product and softmax, at every length: a row picks its largest score."""
+    g = torch.Generator().manual_seed(L)
+    q, k, v, dy = (torch.randn(1, L, 2, 64, generator=g).bfloat16() for _ in range(4))
+    leaves = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    y = swift_efficient_attention(*leaves, 1e30, 0.0, True, True)
+    y.backward(dy.cuda())
+    s = torch.matmul(q.float().transpose(1, 2), k.float().permute(0, 2, 3, 1))
+    s = s.masked_fill(torch.ones(L, L).triu(1).bool(), float("-inf"))
+    top, at = s.topk(2, dim=-1) if L > 1 else (None, None)
+    clear = (top[..., 0] - top[..., 1]) > 2 ** -7 * top[..., 0].abs()  # apart after the scores' rounding
+    clear[..., 0] = True
+    want = torch.gather(v.float().transpose(1, 2), 2, at[..., :1].expand(-1, -1, -1, 64))
+    assert clear.float().mean() > 0.5
+    assert torch.equal(y.detach().float().cpu().transpose(1, 2)[clear], want[clear])
+    assert torch.isfinite(leaves[2].grad).all()
