@@ -438,9 +438,10 @@ constexpr size_t kDmaLds = sizeof(uint16_t) * (8 * 128 * (64 + 8) > kStages * kD
 // (lds_dst wave-uniform).  Written as assembly so that the compiler does not see a vector
 // memory instruction that writes LDS: it would put a wait for every request in flight in
 // front of the transposing LDS reads.  The waits for these requests are the explicit
-// `s_waitcnt vmcnt` below.  M0 is reserved: the compiler keeps nothing in it across statements.
+// `s_waitcnt vmcnt` below.  M0 is reserved: the compiler keeps nothing in it across statements.  A load to LDS
+// may follow a scalar write of M0 after one wait state, which the compiler does not add inside assembly.
 __device__ __forceinline__ void load_to_lds16(const void* base, uint32_t offset, uint32_t lds_dst) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_dst));
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_dst));
 }
 // The same through a buffer descriptor: bytes at and behind its end arrive as zeros.
 __device__ __forceinline__ u32x4 buffer_of(const void* base, uint32_t bytes) {
@@ -450,7 +451,7 @@ __device__ __forceinline__ u32x4 buffer_of(const void* base, uint32_t bytes) {
                static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(bytes))), 0x00020000u};
 }
 __device__ __forceinline__ void load_to_lds16(u32x4 buffer, uint32_t offset, uint32_t lds_dst) {
-  asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(offset), "s"(buffer), "s"(lds_dst));
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(offset), "s"(buffer), "s"(lds_dst));
 }
 
 // RAG: p.kvb and p.ms are set (two k-major operands)

@@ -83,9 +83,10 @@ __device__ __forceinline__ void half_swap(float& a, float& b) {
 // One request: lane l's 16 bytes at base + offset go to LDS bytes lds_dst + 16 l .. + 15
 // (lds_dst wave-uniform, in M0).  Assembly, so that the compiler does not see a vector memory
 // instruction that writes LDS (it would wait for every request in flight in front of each LDS
-// read); the waits for these requests are the explicit `s_waitcnt vmcnt` below.
+// read); the waits for these requests are the explicit `s_waitcnt vmcnt` below, the s_nop the wait state between
+// a scalar write of M0 and a load to LDS.
 __device__ __forceinline__ void load_to_lds16(const void* base, uint32_t offset, uint32_t lds_dst) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_dst));
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_dst));
 }
 
 constexpr int kWaves = 8;                    // waves of a workgroup (two per SIMD)
