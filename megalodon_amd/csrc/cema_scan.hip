@@ -16,7 +16,7 @@
 // (v_mfma_f32_32x32x16_bf16); a row of x is read from memory once, straight
 // into operand registers (a lane's 16-byte load is 8 consecutive steps of one
 // chunk), and y is written once from the accumulators.  Parameter matrices are
-// float32 values split into two bf16 pieces (hi + lo, 16 significant bits); x in
+// float32 values split into two bf16 pieces (hi + lo, 16 significant bits; some have a third, see kFine); x in
 // bf16 is exact, fp16 x is split into two exact bf16 pieces; the states are
 // float32 and split the same way; accumulation is float32.
 //
@@ -60,6 +60,15 @@ __device__ __forceinline__ void split8(const float* v, u32x4& hi, u32x4& lo) {
     hi[e] = h;
     lo[e] = pack_bf16x2(r0, r1);
   }
+}
+// ... and what is left of them behind that: 24 significant bits in three pieces
+__device__ __forceinline__ u32x4 split8_third(const float* v, u32x4 hi, u32x4 lo) {
+  u32x4 third;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    third[e] = pack_bf16x2((v[2 * e] - __uint_as_float(hi[e] << 16)) - __uint_as_float(lo[e] << 16),
+                           (v[2 * e + 1] - __uint_as_float(hi[e] & 0xffff0000u)) - __uint_as_float(lo[e] & 0xffff0000u));
+  return third;
 }
 __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -120,6 +129,17 @@ __device__ __forceinline__ float opaque_one() {
 //            any element's address (which cost more: 4 x 2048 rows of 5001 steps forward and backward
 //            241 us so, 191 shifted, 169 for 5000 steps)
 enum { kWhole = 0, kShifted = 1, kAny = 2 };
+// The lengths of the last two came to these kernels from a float32 convolution and keep its precision: the matrices
+// that make the states (P, Pg) have a third bf16 piece, products of two split factors keep their lo * lo term, and the
+// state after the last step is summed with powers that are evaluated directly.  Relative errors against 64 bits (2-norm,
+// the largest over 121 .. 32767 steps) at the layer's initial decays, the convolution's and these kernels' (two pieces):
+//   y, dx before rounding     4.0e-6, 4.0e-6     2.7e-6, 2.7e-6 (K has two pieces; 2.7e-6, 2.7e-6)
+//   state after the last step 2.6e-7             2.1e-7 (1.5e-6; of float16 rows 2.2e-6)
+//   dalpha, ddelta, dtheta    9.7e-7 1.2e-6 1.7e-6   3.4e-7 6.3e-7 1.4e-6 (5.3e-7 1.0e-6 1.8e-6; 3.0e-6 3.4e-6 4.0e-6)
+// With decays a hundred times slower the float32 coefficients bound every path: y 6.6e-5 both, 4.1e-6 and 4.4e-6
+// in rows of 121 steps, the only place where y and dx are further off than before (K again).  The third pieces cost 7 %:
+// 4 x 2048 rows of 5001 steps forward and backward 168 -> 180 us.
+template <int ROWS> constexpr bool kFine = ROWS != kWhole;
 typedef u32x4 u32x4_any __attribute__((aligned(2)));
 // of the 16-bit steps elem .. elem + 7 those of lo .. hi - 1, zeros for the others
 __device__ __forceinline__ u32x4 keep_steps(u32x4 v, int elem, int lo, int hi) {
@@ -216,12 +236,13 @@ template <> struct XOp<MEGA_F32> {
   }
 };
 
-// acc += (A_hi + A_lo) * x with the lo * lo term of a two-piece x left out
-template <int XP>
+// acc += (A_hi + A_lo) * x, without FINE the lo * lo term of a two-piece x left out
+template <int XP, bool FINE = false>
 __device__ __forceinline__ floatx16 mma_split(const u32x4* a, const u32x4* x, floatx16 acc) {
   acc = mfma_bf16(a[0], x[0], acc);
   acc = mfma_bf16(a[1], x[0], acc);
   if (XP == 2) acc = mfma_bf16(a[0], x[1], acc);
+  if (XP == 2 && FINE) acc = mfma_bf16(a[1], x[1], acc);
   return acc;
 }
 
@@ -247,6 +268,10 @@ struct FwdSmem {
   float H[(NC + 1) * kHP];
 };
 static_assert(sizeof(cf) * 16 * (kT + 2) <= sizeof(float) * (kWaves * 32 + 1) * kHP, "the power table fits the state buffer");
+struct FwdSmemFine : FwdSmem {
+  u32x4 third[4][kWave];  // third pieces of P
+};
+static_assert(3 * sizeof(FwdSmemFine) <= 160 * 1024, "three workgroups per compute unit");
 
 // The rows of a launch: groups of `nb` rows of one channel (d = group % D), each a line of tiles.
 struct Lines {
@@ -320,7 +345,8 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
     const void* __restrict__ x, void* __restrict__ y, const float* __restrict__ p,
     const cf* __restrict__ log_q, const cf* __restrict__ gamma, const float* __restrict__ omega,
     const cf* __restrict__ h0, cf* __restrict__ h_last, const Lines ln, int N) {
-  using Smem = FwdSmem;
+  constexpr bool FINE = kFine<ROWS>;
+  using Smem = typename std::conditional<FINE, FwdSmemFine, FwdSmem>::type;
   constexpr int NC = Smem::NC, CPS = NC / kSubs, XP = XOp<DT>::XP;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Smem& sm = *reinterpret_cast<Smem*>(smem_raw);
@@ -433,6 +459,8 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
       split8(v, hi, lo);
       sm.aop[blk][0][ln] = hi;
       sm.aop[blk][1][ln] = lo;
+      if constexpr (FINE)
+        if (blk < 4) sm.third[blk][ln] = split8_third(v, hi, lo);
     }
     __syncthreads();
     rp = next_rp;
@@ -473,7 +501,10 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[i] = 0.f;
 #pragma unroll
-        for (int s = 0; s < 4; ++s) acc = mma_split<XP>(P[s], xb[s].pc, acc);
+        for (int s = 0; s < 4; ++s) {
+          acc = mma_split<XP, FINE>(P[s], xb[s].pc, acc);
+          if constexpr (FINE) acc = mfma_bf16(sm.third[s][lane], xb[s].pc[0], acc);
+        }
         float* dst = sm.H + (1 + c0 + r) * kHP + 4 * g;
 #pragma unroll
         for (int qd = 0; qd < 4; ++qd)
@@ -493,7 +524,7 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
         for (int i = 0; i < 16; ++i) yacc[it][i] = 0.f;
         if (w.nc > 0) {
 #pragma unroll
-          for (int s = 0; s < 2 + 2 * it; ++s) yacc[it] = mma_split<XP>(K[1 + 2 * it - s], xb[s].pc, yacc[it]);
+          for (int s = 0; s < 2 + 2 * it; ++s) yacc[it] = mma_split<XP, FINE>(K[1 + 2 * it - s], xb[s].pc, yacc[it]);
         }
       }
     }
@@ -573,11 +604,7 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
         for (int it = 0; it < 2; ++it) {
           floatx16 acc = yacc[it];
 #pragma unroll
-          for (int s2 = 0; s2 < 2; ++s2) {
-            acc = mfma_bf16(Q[2 * it + s2][0], hb[s2][0], acc);
-            acc = mfma_bf16(Q[2 * it + s2][1], hb[s2][0], acc);
-            acc = mfma_bf16(Q[2 * it + s2][0], hb[s2][1], acc);
-          }
+          for (int s2 = 0; s2 < 2; ++s2) acc = mma_split<2, FINE>(Q[2 * it + s2], hb[s2], acc);
 #pragma unroll
           for (int pr = 0; pr < 2; ++pr) {
             if constexpr (DT == MEGA_F32) {
@@ -600,29 +627,58 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
     }
     cur ^= 1;
     par ^= 1;
-    if (w.hi > 0 && w.base + w.hi == (w.row + 1) * ln.L && h_last != nullptr && lane < N) {
+    if (w.hi > 0 && w.base + w.hi == (w.row + 1) * ln.L && h_last != nullptr && (FINE || lane < N)) {
       // the state after step L - 1 (the row's last chunk may be partial), from this wave's own rows
       const typename Elem<DT>::type* xrow = static_cast<const typename Elem<DT>::type*>(x) + w.base;
       const int cl = w.nc - 1;           // the last chunk inside the tile
       const int rem = w.hi - cl * kT;    // 1 .. 64 steps in it
-      cf h;
-      if (rem == kT) {
-        const float* lastrow = sm.H + (1 + c0 + cl) * kHP + 2 * lane;
-        h = cf{lastrow[0], lastrow[1]};
-      } else {
-        const float* prev = cl == 0 ? sm.wave_cin[wave] + 2 * lane : sm.H + (c0 + cl) * kHP + 2 * lane;
-        // the recurrence itself over the last chunk's steps (the power table has made way for
-        // the states by now): h <- q h + p x
-        h = cf{prev[0], prev[1]};
-        const cf q1 = sm.pw[8][lane];
-        const float pp = sm.pn[lane];
-        for (int j = cl == 0 ? w.lo : 0; j < rem; ++j) {
-          const float xv = Elem<DT>::load(xrow + cl * kT + j) * pp;
-          h = cmul(q1, h);
-          h.x += xv;
+      if constexpr (FINE) {
+        // q^rem h + p sum_e q^e x[rem - 1 - e], h the state in front of that chunk; lane (n, a) = (lane % 16, lane / 16) adds
+        // up the exponents 16 a .. 16 a + 15 of mode n.  (Step by step the rounding of q alone costs 1e-6 over a chunk.)
+        const int first = cl == 0 ? w.lo : 0, n = lane & 15, a = lane >> 4;
+        const cf q1 = sm.pw[8][n];
+        cf t{0.f, 0.f};
+#pragma unroll 1
+        for (int k = 0; k < 4; ++k) {
+          cf v{0.f, 0.f};
+#pragma unroll
+          for (int e = 3; e >= 0; --e) {
+            const int j = rem - 1 - (16 * a + 4 * k + e);
+            v = cmul(q1, v);
+            if (j >= first) v.x += Elem<DT>::load(xrow + cl * kT + j);
+          }
+          t = cadd(t, cmul(sm.pw[k][n], v));
         }
+        t = cmul(sm.pw[4 + a][n], t);
+        t.x += __shfl_xor(t.x, 16, 64);
+        t.y += __shfl_xor(t.y, 16, 64);
+        t.x += __shfl_xor(t.x, 32, 64);
+        t.y += __shfl_xor(t.y, 32, 64);
+        cf qr = rem == kT ? sm.pw[9][n] : cmul(sm.pw[(rem >> 2) & 3][n], sm.pw[4 + ((rem >> 4) & 3)][n]);
+        for (int e = rem & 3; e > 0; --e) qr = cmul(qr, q1);
+        const float* prev = cl == 0 ? sm.wave_cin[wave] + 2 * n : sm.H + (c0 + cl) * kHP + 2 * n;
+        const cf h = cmul(qr, cf{prev[0], prev[1]});
+        if (lane < N) h_last[w.row * N + lane] = cf{h.x + sm.pn[n] * t.x, h.y + sm.pn[n] * t.y};
+      } else {
+        cf h;
+        if (rem == kT) {
+          const float* lastrow = sm.H + (1 + c0 + cl) * kHP + 2 * lane;
+          h = cf{lastrow[0], lastrow[1]};
+        } else {
+          const float* prev = cl == 0 ? sm.wave_cin[wave] + 2 * lane : sm.H + (c0 + cl) * kHP + 2 * lane;
+          // the recurrence itself over the last chunk's steps (the power table has made way for
+          // the states by now): h <- q h + p x
+          h = cf{prev[0], prev[1]};
+          const cf q1 = sm.pw[8][lane];
+          const float pp = sm.pn[lane];
+          for (int j = 0; j < rem; ++j) {
+            const float xv = Elem<DT>::load(xrow + cl * kT + j) * pp;
+            h = cmul(q1, h);
+            h.x += xv;
+          }
+        }
+        h_last[w.row * N + lane] = h;
       }
-      h_last[w.row * N + lane] = h;
     }
   };
 
@@ -659,7 +715,7 @@ template <int DT, int ROWS>
 int launch_fwd(const void* x, void* y, const float* p, const cf* log_q, const cf* gamma,
                const float* omega, const cf* h0, cf* h_last, int64_t B, int64_t D, int64_t N,
                int64_t L, hipStream_t stream) {
-  const size_t lds = sizeof(FwdSmem);
+  const size_t lds = kFine<ROWS> ? sizeof(FwdSmemFine) : sizeof(FwdSmem);
   MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cema_scan_fwd_kernel<DT, ROWS>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
   int cus = 0;
@@ -722,15 +778,24 @@ struct BwdSmem {
   cf wave_end[2][kWaves][2][16];         // the same for each wave's four sub-segments, by item parity
   float wave_cin[kWaves][64];            // (R, R') behind each wave's last chunk
   cf carry[2][2][16];
-  float red[kWaves][2][32];
-  float dpart[kWaves][kT];
-  float dkin[kT];
+};
+// a row's reductions, in the place of a wave's own sub-segment ends
+struct BwdSums {
+  float red[2][32];
+  float dpart[kT];
+  float dkin[kT];                        // wave 0's
+};
+static_assert(sizeof(BwdSums) <= sizeof(cf) * 4 * 2 * 16, "a wave's sums fit its four sub-segments");
+struct BwdSmemFine : BwdSmem {
+  u32x4 third[4][kWave];                 // third pieces of Pg, first kind (the second kind's: in registers)
 };
 static_assert(sizeof(cf) * 16 * (kT + 2) + sizeof(cf) * 16 * 2 * 16 <= sizeof(float) * kBwdNC * kRP,
               "the power table and the final partial sums live in the state buffer");
 static_assert(32 * kSP * 2 <= 32 * kRP * 4 && 16 * kWave * 4 <= 32 * kRP * 4 && kWave * 33 <= 32 * kRP,
               "a wave's parked tile and one accumulator tile fit its own rows of the state buffer");
-static_assert(sizeof(BwdSmem) <= 80 * 1024, "two workgroups per compute unit");
+static_assert(sizeof(cf) * 16 * (kT + 2) + sizeof(u32x4) * 4 * kWave <= sizeof(float) * kBwdNC * kRP,
+              "the third pieces of the second kind pass through the state buffer, behind the power table");
+static_assert(sizeof(BwdSmemFine) <= 80 * 1024, "two workgroups per compute unit");
 
 // (h, h') <- (g, g') + [[m, 0], [md, m]] (h, h'): one step of the reverse scan, over a chunk
 // (m = q^64, md = 64 q^63), a sub-segment or a wave's chunks (the same form with larger powers)
@@ -752,7 +817,9 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
   static_assert(XOp<DT>::XP == 1, "the backward kernel takes bfloat16 rows");
   constexpr int CPS = kBwdCPS;
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  BwdSmem& sm = *reinterpret_cast<BwdSmem*>(smem_raw);
+  constexpr bool FINE = kFine<ROWS>;
+  using Smem = typename std::conditional<FINE, BwdSmemFine, BwdSmem>::type;
+  Smem& sm = *reinterpret_cast<Smem*>(smem_raw);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   // lane-derived indices, re-derived from an opaque thread id wherever a phase starts
 #define MEGA_LANE_IDS                                                          \
@@ -764,6 +831,9 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
   (void)stage
   cf (*qp)[kT + 2] = reinterpret_cast<cf(*)[kT + 2]>(sm.R);                 // setup and finish only
   cf (*ab)[2][16] = reinterpret_cast<cf(*)[2][16]>(sm.R + 2 * 16 * (kT + 2));  // finish only, behind the table
+  u32x4 (*passed)[kWave] = reinterpret_cast<u32x4(*)[kWave]>(sm.R + 2 * 16 * (kT + 2));  // setup only, the same place
+  auto sums = [&](int wv) -> BwdSums& { return *reinterpret_cast<BwdSums*>(&sm.sub_end[4 * wv][0][0]); };  // finish only
+  u32x4 third1[4];  // FINE: third pieces of Pg, second kind
   // the last four tiles of a group's line, where its walk starts
   auto tail_of = [&](int group) { return group < ln.groups ? (ln.tiles(group) - 1) / kWaves * kWaves : 0; };
 
@@ -887,6 +957,8 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       split8(v, hi, lo);
       sm.aop[blk][0][ln] = hi;
       sm.aop[blk][1][ln] = lo;
+      if constexpr (FINE)
+        if (blk < 8) (blk < 4 ? sm.third[blk] : passed[blk - 4])[ln] = split8_third(v, hi, lo);
     }
 #pragma unroll
     for (int t = 0; t < 3; ++t)
@@ -895,6 +967,11 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
 #pragma unroll
     for (int i = 0; i < 8; ++i) wacc[i] = wdacc[i] = cf{0.f, 0.f};
     __syncthreads();
+    if constexpr (FINE) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) third1[s] = passed[s][lane];
+      __syncthreads();  // every wave has its pieces: the buffer takes the parked tiles
+    }
     rp = fetch_params(group + static_cast<int>(gridDim.x));
   };
 
@@ -922,7 +999,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       float acc = 0.f;
 #pragma unroll
       for (int j = 0; j < 32; ++j) acc += part[j];
-      sm.red[wave][g][r] = acc;
+      sums(wave).red[g][r] = acc;
     }
     // dkin[l] = sum_j M[j + l][j]: each wave sums the diagonals of its own M, one 32 x 32 tile
     // at a time through its own rows of the state buffer ([i][j], pitch 33).  Lane (g, t) walks
@@ -958,10 +1035,10 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       const float cross_lo = lo[1] + __shfl_xor(lo[1], 32, 64);
       const float cross_hi = hi[1] + __shfl_xor(hi[1], 32, 64);
       // lag l <= 31: same[d = l] + cross[d = l - 32]; lag l >= 32: cross[d = l - 32]
-      sm.dpart[wave][lane] = g == 0 ? same + cross_hi : cross_lo;
+      sums(wave).dpart[lane] = g == 0 ? same + cross_hi : cross_lo;
     }
     __syncthreads();  // every wave is done with the state buffer: it takes the power table again
-    if (tid < kT) sm.dkin[tid] = (sm.dpart[0][tid] + sm.dpart[1][tid]) + (sm.dpart[2][tid] + sm.dpart[3][tid]);
+    if (tid < kT) sums(0).dkin[tid] = (sums(0).dpart[tid] + sums(1).dpart[tid]) + (sums(2).dpart[tid] + sums(3).dpart[tid]);
     {
       cf v = cmul(sm.pw[sa & 3][sn], sm.pw[4 + (sa >> 2)][sn]);
 #pragma unroll
@@ -977,7 +1054,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int l = 4 * sa + e;
-        const float dk = sm.dkin[l];
+        const float dk = sums(0).dkin[l];
         const cf v = qp[sn][l];
         ain.x = fmaf(dk, v.x, ain.x);
         ain.y = fmaf(dk, v.y, ain.y);
@@ -1003,10 +1080,11 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       const int hg = (n >> 1) & 1, idx = 2 * (n >> 2) + (n & 1);
       cf w{0.f, 0.f}, wd{0.f, 0.f};
       for (int wv = 0; wv < kWaves; ++wv) {
-        w.x += sm.red[wv][hg][4 * idx];
-        w.y += sm.red[wv][hg][4 * idx + 1];
-        wd.x += sm.red[wv][hg][4 * idx + 2];
-        wd.y += sm.red[wv][hg][4 * idx + 3];
+        const float* part = sums(wv).red[hg] + 4 * idx;
+        w.x += part[0];
+        w.y += part[1];
+        wd.x += part[2];
+        wd.y += part[3];
       }
       const cf qq = sm.pw[8][n];
       const cf A = cadd(ain, cmul(qq, w));
@@ -1038,7 +1116,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       dgamma[row * N + n] = dgv;
     }
     // the skip term sat on the diagonal of K, not in M: domega = sum dy x = dkin[0]
-    if (tid == 0) domega[row] = sm.dkin[0];
+    if (tid == 0) domega[row] = sums(0).dkin[0];
   };
 
   Tile cur_tile = tile_at<ROWS>(ln, blockIdx.x, tail_of(blockIdx.x) + wave);  // this wave's tile of the item
@@ -1121,6 +1199,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
           u32x4 a[2];
           load_block(kind * 4 + s, a, lane);
           acc = mma_split<1>(a, db[s].pc, acc);
+          if constexpr (FINE) acc = mfma_bf16(kind ? third1[s] : sm.third[s][lane], db[s].pc[0], acc);
         }
         float* dst = myrows + r * kRP + 32 * kind + 4 * g;
 #pragma unroll
@@ -1235,9 +1314,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
         for (int s2 = 0; s2 < 2; ++s2) {
           u32x4 a[2];
           load_block(12 + 2 * jt + s2, a, lane);
-          acc = mfma_bf16(a[0], hb[s2][0], acc);
-          acc = mfma_bf16(a[1], hb[s2][0], acc);
-          acc = mfma_bf16(a[0], hb[s2][1], acc);
+          acc = mma_split<2, FINE>(a, hb[s2], acc);
         }
 #pragma unroll
         for (int pr = 0; pr < 2; ++pr) {
@@ -1279,6 +1356,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
             u32x4 a[2];
             load_block(kind * 4 + s, a, lane);
             xacc[kind] = mma_split<1>(a, &xr[s], xacc[kind]);
+            if constexpr (FINE) xacc[kind] = mfma_bf16(kind ? third1[s] : sm.third[s][lane], xr[s], xacc[kind]);
           }
         }
 #pragma unroll
@@ -1335,7 +1413,7 @@ template <int DX32, int ROWS>
 int launch_bwd(const void* dy, const void* x, void* dx, const float* p, const cf* log_q,
                const cf* gamma, const float* omega, const cf* h0, float* dp, cf* dq, cf* dgamma, float* domega,
                cf* dh0, int64_t B, int64_t D, int64_t N, int64_t L, bool single, hipStream_t stream) {
-  const int lds = static_cast<int>(sizeof(BwdSmem));
+  const int lds = static_cast<int>(kFine<ROWS> ? sizeof(BwdSmemFine) : sizeof(BwdSmem));
   MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cema_scan_bwd_kernel<MEGA_BF16, DX32, ROWS>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds));
   Lines ln;

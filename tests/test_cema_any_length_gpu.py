@@ -99,3 +99,30 @@ def test_parameters_in_bfloat16():
     for n in NAMES:
         got = getattr(layer, n).grad
         assert got.dtype == torch.bfloat16 and rel_err(got, pr[n].grad) <= 2e-2, n
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,D,L", [(3, 64, 121), (2, 64, 201), (2, 64, 513), (2, 64, 777)])
+def test_float32_results_keep_float32_precision(B, D, L, dtype):
+    """The last state and the parameter gradients are float32 results: a float32 convolution has them to some four
+    units of 2^-24 in the 2-norm, rows and powers of 16 bits to twice that and more.  Bar: six."""
+    torch.manual_seed(L)
+    layer = MultiHeadComplexEMA(D, 16).cuda().train()
+    x0, x = _rows(B, D, L, dtype, L, 0)
+    dy0, dy = _rows(B, D, L, dtype, L + 1, 0)
+    x.requires_grad_(True)
+    layer(x)[0].backward(dy)
+    with torch.no_grad():
+        last = layer(x, None, True)[1]
+    pr = {n: getattr(layer, n).detach().cpu().double().requires_grad_(True) for n in NAMES}
+    p, q, g = ocema.calc_coeffs(pr["alpha"], pr["delta"], pr["theta"], pr["gamma"], 16)
+    want = offt.fftconv_fwd(x0.double(), ocema.ema_weight_fwd(p, q.log(), g, L)) + x0.double() * pr["omega"]
+    want.backward(dy0.double())
+
+    def err(got, ref):
+        got, ref = (torch.view_as_real(t) if t.is_complex() else t for t in (got.detach().cpu(), ref.detach()))
+        return ((got.double() - ref).norm() / ref.norm()).item()
+
+    errors = {n: err(getattr(layer, n).grad, pr[n].grad) for n in ("alpha", "gamma", "omega")}
+    errors["last"] = err(last, ocema.ema_hidden_fwd(x0, p, q.log(), None))
+    assert max(errors.values()) <= 6 * 2 ** -24, errors
