@@ -84,3 +84,37 @@ def mega_block_forward(p, x, *, num_heads, ndim, chunk_size, groups, eps=1e-5, s
     else:
         hid = F.silu(F.linear(n, p["nffn.fc1.weight"]))
     return F.linear(hid, p["nffn.fc2.weight"]) + x
+
+
+def mega_block_step(p, x, cache, *, num_heads, ndim, groups, eps=1e-5, freqs_cis=None):
+    """One new token x (B, 1, D) on `cache` = ((keys, values, n), (count, mean, var), h), the whole of it an
+    unfinished chunk (the cache branch of moving_average_gated_attention.py:283-348, SwiGLU network): (out, keys,
+    values, count, mean, var, h) in float64 / complex128."""
+    (keys, values, _), (count, mean, var), h = cache
+    x, keys, values = x.double(), keys.double(), values.double()
+    B, _, D = x.shape
+    tsn, count, mean, var, _, _ = otn.group_timestep_norm_closed_form_full(
+        x, count, mean, var, p["mega.timenorm.weight"] + 1.0, p["mega.timenorm.bias"], None, groups, eps)
+    pp, q, g = ocema.calc_coeffs(p["mega.cema.alpha"], p["mega.cema.delta"], p["mega.cema.theta"],
+                                 p["mega.cema.gamma"], ndim)
+    h = q.squeeze(-1) * h.to(torch.complex128) + pp.squeeze(-1) * tsn[:, 0].unsqueeze(-1)
+    cema = (g * h).sum(-1).real.unsqueeze(1) + tsn * p["mega.cema.omega"].reshape(-1)
+    mx = _rms(cema, p.get("mega.rmsnorm.weight"), eps)
+    lin = lambda name, t: F.linear(t, p[f"mega.{name}.weight"], p.get(f"mega.{name}.bias"))
+    z = lin("wz", mx)
+    zh = z.shape[-1] // num_heads
+    z = _rms(z.view(B, 1, num_heads, zh), None, eps).view(B, 1, -1).unsqueeze(2)
+    z = z * ((p["mega.gamma"] + 1.0) / math.sqrt(zh)) + p["mega.beta"]
+    qq, kk = (t.reshape(B, 1, num_heads, zh) for t in torch.unbind(z, dim=2))
+    if freqs_cis is not None:
+        qq, kk = rotary(qq, freqs_cis), rotary(kk, freqs_cis)
+    v = F.silu(lin("wv", tsn))
+    keys = torch.cat((keys, kk), dim=1)
+    values = torch.cat((values, v.view(B, 1, num_heads, -1)), dim=1)
+    y, _ = oattn.chunk_attention_fwd(qq, keys, values, 1.0, False)
+    attn = y.reshape(B, 1, -1) * F.silu(lin("wr", mx))
+    y1 = lin("wh1", mx) + lin("wh2", attn) + x
+    n = F.layer_norm(y1, (D,), None if "nffn.norm.weight" not in p else p["nffn.norm.weight"] + 1.0,
+                     p.get("nffn.norm.bias"), eps)
+    hid = F.silu(F.linear(n, p["nffn.fc1.weight"])) * F.linear(n, p["nffn.fc3.weight"])
+    return F.linear(hid, p["nffn.fc2.weight"]) + x, keys, values, count, mean, var, h

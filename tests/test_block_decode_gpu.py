@@ -1,4 +1,4 @@
-"""The fused one-token step of a block (csrc/block_decode.hip) against the same step taken operator by
+"""The fused one-token step of a block (csrc/block_decode.hip) against the same step in 64 bits and taken operator by
 operator, at the edges of what the kernels take: token tiles (1, 16, 17, 32 sequences), head
 widths, lengths of one key, one run and many runs of keys.  Tolerance: the 16-bit bar, 2e-2."""
 import copy
@@ -10,6 +10,7 @@ import torch
 from conftest import rel_err
 from megalodon_amd.modules import MegaBlock, RotaryEmbedding
 from megalodon_amd.modules.block_decode import decode_step
+from oracle import block as oblock
 
 pytestmark = pytest.mark.gpu
 
@@ -32,13 +33,16 @@ def _prompt(blk, B, n, D, S, E, heads, dtype, rotary):
     return blk(x, rotary.get_freqs_cis(0, n), None, empty)[1]
 
 
-@pytest.mark.parametrize("B,n,D,S,E,F,heads,groups,dtype,affine", [
+SIZES = pytest.mark.parametrize("B,n,D,S,E,F,heads,groups,dtype,affine", [
     (1, 1, 256, 128, 512, 512, 2, 2, torch.bfloat16, True),       # one cached key, 64-wide heads
     (16, 40, 1024, 256, 2048, 2752, 1, 8, torch.bfloat16, True),  # a full token tile, 2048-wide values
     (17, 513, 256, 512, 128, 96, 2, 8, torch.bfloat16, True),     # two token tiles, narrow values, many runs
     (32, 7, 512, 256, 1024, 320, 2, 2, torch.float16, True),
     (3, 1000, 384, 384, 768, 416, 3, 3, torch.bfloat16, False),   # no affine norms, reductions that do not divide by eight waves
 ])
+
+
+@SIZES
 def test_step_matches_operators(B, n, D, S, E, F, heads, groups, dtype, affine):
     chunk = 1024
     blk = _block(D, S, E, F, heads, groups, chunk, dtype, affine)
@@ -63,6 +67,44 @@ def test_step_matches_operators(B, n, D, S, E, F, heads, groups, dtype, affine):
                 assert a.shape == b.shape and a.dtype == b.dtype and rel_err(a, b) <= 2e-2
             assert got[1][2].dtype == wanted[2].dtype and rel_err(got[1][2], wanted[2]) <= 2e-2
             cache = got[1]
+
+
+def _err(got, want):
+    got, want = (torch.view_as_real(t.detach().cpu().resolve_conj()) if t.is_complex() else t.detach().cpu() for t in (got, want))
+    return ((got.double() - want.double()).norm() / want.double().norm()).item()
+
+
+@SIZES
+def test_step_against_float64(B, n, D, S, E, F, heads, groups, dtype, affine):
+    """The step and the operators from one cache, against the same step in 64 bits.  A rounding to bfloat16 is 2^-9 / sqrt(3)
+    = 1.1e-3 in the norm; up to five lie in front of keys, values and statistics, twelve in front of the output (normalised
+    row, EMA output, its norm, four projections' values, q, k, attention, gate, y1, its norm, hidden): 2.5e-3 and 3.9e-3
+    where nothing amplifies them.  Bars twice that.  And the step, which rounds in fewer places than the
+    operators, may not be further off than they are."""
+    chunk = 1024
+    blk = _block(D, S, E, F, heads, groups, chunk, dtype, affine)
+    rotary = RotaryEmbedding(S // heads, chunk).cuda()
+    p = {k: v.detach().double().cpu() for k, v in blk.named_parameters()}
+    with torch.no_grad():
+        cache = _prompt(blk, B, n, D, S, E, heads, dtype, rotary)
+        on_host = (tuple(t.cpu() for t in cache[0][:2]) + (n,), tuple(t.cpu() for t in cache[1]), cache[2].cpu())
+        x = torch.randn(B, 1, D, generator=torch.Generator().manual_seed(1)).to(dtype).cuda()
+        freqs = rotary.get_freqs_cis(n, n + 1)
+        want = oblock.mega_block_step(p, x.cpu(), on_host, num_heads=heads, ndim=16, groups=groups,
+                                      eps=blk.mega.timenorm.eps, freqs_cis=freqs.cpu())
+        y, after = blk.mega(x, freqs, None, cache)
+        operators = (blk.nffn(y, x), *_tensors(after))
+        y, after = decode_step(blk, x, freqs, cache)
+        step = (y, *_tensors(after))
+    for name, s, o, w in zip(("out", "keys", "values", "count", "mean", "var", "state"), step, operators, want):
+        if name == "count":
+            assert torch.equal(s.cpu(), w.to(s.dtype))
+            continue
+        if name in ("keys", "values"):  # the old rows are the cache's own
+            assert torch.equal(s[:, :-1].cpu().double(), w[:, :-1])
+            s, o, w = s[:, -1], o[:, -1], w[:, -1]
+        assert _err(s, w) <= (7.8e-3 if name == "out" else 5e-3), (name, _err(s, w))
+        assert _err(s, w) <= 1.1 * _err(o, w) + 2 ** -14, (name, _err(s, w), _err(o, w))
 
 
 def test_last_token_of_a_chunk_empties_the_cache():

@@ -208,3 +208,20 @@ def test_gradients_of_the_oracle_match_the_restatement():
     g2 = torch.autograd.grad((_restated_block(p, x, **CFG) * dy).sum(), [x] + [p[n] for n in names])
     for n, a, b in zip(["x"] + names, g1, g2):
         assert torch.allclose(a, b, atol=1e-9, rtol=1e-8), n
+
+
+def test_step_continues_the_whole_pass():
+    """The one-token oracle, fed token by token from the first on, gives the rows of the whole-sequence oracle."""
+    p, B, L, heads, ndim, groups = _params(), 2, CFG["chunk_size"], CFG["num_heads"], CFG["ndim"], CFG["groups"]
+    x = torch.randn(B, L, D, dtype=torch.float64, generator=torch.Generator().manual_seed(5))
+    freqs = torch.polar(torch.ones(L, Z // heads // 2), 6 * torch.rand(L, Z // heads // 2)).to(torch.complex128)
+    whole = ob.mega_block_forward(p, x, freqs_cis=freqs, **CFG)
+    cache = ((torch.empty(B, 0, heads, Z // heads), torch.empty(B, 0, heads, H // heads), 0),
+             (torch.zeros(B, dtype=torch.int64), torch.zeros(B, groups), torch.ones(B, groups)),
+             torch.zeros(B, D, ndim, dtype=torch.complex128))
+    for t in range(L):
+        out, k, v, count, mean, var, h = ob.mega_block_step(p, x[:, t:t + 1], cache, num_heads=heads, ndim=ndim,
+                                                            groups=groups, freqs_cis=freqs[t:t + 1])
+        assert (out - whole[:, t:t + 1]).abs().max() <= 1e-10
+        assert int(count[0]) == t + 1
+        cache = ((k, v, t + 1), (count, mean, var), h)
