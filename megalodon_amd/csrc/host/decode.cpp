@@ -25,6 +25,7 @@ std::optional<Step> block_decode_step(const Tensor& x, const Tensor& k, const Te
   if (dtype != MEGA_BF16 && dtype != MEGA_F16) return std::nullopt;
   const auto dev = x.device();
   if (!x.is_cuda() || static_cast<int>(weights.size()) != kWeights) return std::nullopt;
+  if (x.dim() != 3 || x.size(1) != 1 || k.dim() != 4 || p.dim() < 2 || heads < 1) return std::nullopt;
   // a forward-mode tangent goes to the operators, which refuse it, and so does a lazily conjugated or negated
   // view, which they resolve
   for (const Tensor* t : {&x, &k, &v, &prev_count, &prev_mean, &prev_var, &hx})
@@ -42,6 +43,10 @@ std::optional<Step> block_decode_step(const Tensor& x, const Tensor& k, const Te
   }
   const int64_t B = x.size(0), D = x.size(2), S = weights[kWz]->size(0), E = weights[kWv]->size(0), F = weights[kFc1]->size(0),
                 N = p.size(1), n = k.size(1);
+  const int64_t rows[kWeights] = {1, 1, 1, 1, S, 1, E, 1, D, 1, E, 1, D, 2, 2, 1, 1, F, D, F};
+  const int64_t cols[kWeights] = {D, D, D, D, D, S, D, E, D, D, D, E, E, S, S, D, D, D, F, D};
+  for (int i = 0; i < kWeights; ++i)  // (the operators refuse what does not fit)
+    if (weights[i].has_value() && (weights[i]->numel() != rows[i] * cols[i] || (rows[i] > 1 && weights[i]->size(-1) != cols[i]))) return std::nullopt;
   if (!mega_block_decode_supported(dtype, B, D, S, E, F, heads, groups, N)) return std::nullopt;
   const auto is = [&](const Tensor& t, at::ScalarType ty, at::IntArrayRef shape) {
     return t.scalar_type() == ty && t.device() == dev && t.sizes() == shape && t.is_contiguous();
@@ -59,11 +64,11 @@ std::optional<Step> block_decode_step(const Tensor& x, const Tensor& k, const Te
   if (freqs.has_value() && !is(*freqs, at::kComplexFloat, {1, S / heads / 2})) return std::nullopt;
 
   c10::DeviceGuard guard(dev);
-  const auto rows = [&](const Tensor& t) {
+  const auto dense = [&](const Tensor& t) {
     const Tensor c = t.contiguous();
     return aligned(c) ? c : c.clone(at::MemoryFormat::Contiguous);
   };
-  const Tensor k_in = rows(k), v_in = rows(v);
+  const Tensor k_in = dense(k), v_in = dense(v);
   // the cache that is handed back is the caller's own, as a concatenation would be: it shares nothing with
   // the old one, whatever streams, threads or later writes the two meet
   Tensor k_out = at::empty({B, n + 1, heads, S / heads}, x.options()), v_out = at::empty({B, n + 1, heads, E / heads}, x.options());

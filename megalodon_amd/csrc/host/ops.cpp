@@ -396,6 +396,7 @@ std::optional<std::tuple<Tensor, Optional>> cema_state(const Tensor& x, const Te
   const int64_t N = p.size(1);
   if (!cema_takes(x, N)) return std::nullopt;
   const int64_t B = x.size(0), D = x.size(1);
+  require(p.numel() == D * N && log_q.numel() == D * N && gamma_hat.numel() == D * N && omega.numel() == D, "cema: x and the parameters must have the same number of channels");
   if (h0.has_value()) require(h0->scalar_type() == at::kComplexFloat && h0->numel() == B * D * N && h0->device() == x.device(), "cema: the carried state must be complex64 (B, D, N)");
   c10::DeviceGuard guard(x.device());
   const Tensor xc = rows_of(x), w = as_float(omega), h = h0.has_value() ? stored(*h0).contiguous() : Tensor();

@@ -211,3 +211,21 @@ def test_cache_of_a_whole_chunk_is_refused():
         keys, values = (torch.cat((t, t[:, :2]), dim=1) for t in attn[:2])
         with pytest.raises(RuntimeError):
             blk(x, rotary.get_freqs_cis(65, 66), None, ((keys, values, 65), norm, h))
+
+
+@pytest.mark.parametrize("name,shape", [
+    ("mega.wr.weight", (480, 256)), ("mega.wr.bias", (480,)), ("mega.wh2.weight", (256, 480)), ("mega.wh1.weight", (128, 512)),
+    ("mega.gamma", (2, 64)), ("nffn.fc3.weight", (480, 256)), ("nffn.fc2.weight", (512, 256)), ("mega.rmsnorm.weight", (128,)),
+    ("mega.cema.omega", (128, 1)),
+])
+def test_weights_of_other_shapes_are_refused(name, shape):
+    """As the operators do; the step's kernels take the shapes from the block's first weights."""
+    blk = _block(256, 128, 512, 512, 2, 2, 64)
+    rotary = RotaryEmbedding(64, 64).cuda()
+    x = torch.randn(2, 1, 256, generator=torch.Generator().manual_seed(1)).bfloat16().cuda()
+    with torch.no_grad():
+        cache = _prompt(blk, 2, 9, 256, 128, 512, 2, torch.bfloat16, rotary)
+        owner, leaf = name.rsplit(".", 1)
+        setattr(blk.get_submodule(owner), leaf, torch.nn.Parameter(torch.zeros(shape, dtype=torch.bfloat16, device="cuda")))
+        with pytest.raises(RuntimeError):
+            decode_step(blk, x, rotary.get_freqs_cis(9, 10), cache) or blk(x, rotary.get_freqs_cis(9, 10), None, cache)

@@ -126,3 +126,14 @@ def test_float32_results_keep_float32_precision(B, D, L, dtype):
     errors = {n: err(getattr(layer, n).grad, pr[n].grad) for n in ("alpha", "gamma", "omega")}
     errors["last"] = err(last, ocema.ema_hidden_fwd(x0, p, q.log(), None))
     assert max(errors.values()) <= 6 * 2 ** -24, errors
+
+
+@pytest.mark.parametrize("channels", [32, 128])
+@pytest.mark.parametrize("L", [40, 41])
+def test_rows_of_another_width_are_refused(channels, L):
+    layer = MultiHeadComplexEMA(64, 16).cuda().eval()
+    x = torch.randn(2, channels, L, device="cuda").bfloat16()
+    with torch.no_grad(), pytest.raises(RuntimeError):
+        layer(x, None, True)
+    with torch.no_grad(), pytest.raises(RuntimeError):
+        layer(x, torch.zeros(2, channels, 16, dtype=torch.complex64, device="cuda"), False)
