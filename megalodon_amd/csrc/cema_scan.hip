@@ -70,6 +70,25 @@ __device__ __forceinline__ u32x4 split8_third(const float* v, u32x4 hi, u32x4 lo
                            (v[2 * e + 1] - __uint_as_float(hi[e] & 0xffff0000u)) - __uint_as_float(lo[e] & 0xffff0000u));
   return third;
 }
+// Third pieces of k[0 .. 63] for the Toeplitz blocks, whose lanes read eight consecutive lags each: one table of the
+// lags in the blocks' order, zeros at negative ones, and a second one that starts an element later, so that every
+// lane reads whole words.
+constexpr int kThirdLags = 96;
+typedef uint16_t ThirdTable[2][kThirdLags];
+template <bool DOWN>  // index i: lag 63 - i, else i - 31
+__device__ __forceinline__ void fill_thirds(ThirdTable& t, const float* k, int tid) {
+  if (tid < 2 * kThirdLags) {
+    const int i = tid < kThirdLags ? tid : tid - kThirdLags + 1, lag = DOWN ? kT - 1 - i : i - 31;
+    const float v = lag >= 0 && lag < kT ? k[lag] : 0.f;
+    const float r = v - __uint_as_float(pack_bf16x2(v, 0.f) << 16);
+    t[0][tid] = static_cast<uint16_t>(pack_bf16x2(r - __uint_as_float(pack_bf16x2(r, 0.f) << 16), 0.f));
+  }
+}
+// elements i .. i + 7
+__device__ __forceinline__ u32x4 read_thirds(const ThirdTable& t, int i) {
+  const uint32_t* w = reinterpret_cast<const uint32_t*>(t[i & 1]) + (i >> 1);
+  return u32x4{w[0], w[1], w[2], w[3]};
+}
 __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
@@ -129,16 +148,16 @@ __device__ __forceinline__ float opaque_one() {
 //            any element's address (which cost more: 4 x 2048 rows of 5001 steps forward and backward
 //            241 us so, 191 shifted, 169 for 5000 steps)
 enum { kWhole = 0, kShifted = 1, kAny = 2 };
-// The lengths of the last two came to these kernels from a float32 convolution and keep its precision: the matrices
-// that make the states (P, Pg) have a third bf16 piece, products of two split factors keep their lo * lo term, and the
-// state after the last step is summed with powers that are evaluated directly.  Relative errors against 64 bits (2-norm,
-// the largest over 121 .. 32767 steps) at the layer's initial decays, the convolution's and these kernels' (two pieces):
-//   y, dx before rounding     4.0e-6, 4.0e-6     2.7e-6, 2.7e-6 (K has two pieces; 2.7e-6, 2.7e-6)
-//   state after the last step 2.6e-7             2.1e-7 (1.5e-6; of float16 rows 2.2e-6)
-//   dalpha, ddelta, dtheta    9.7e-7 1.2e-6 1.7e-6   3.4e-7 6.3e-7 1.4e-6 (5.3e-7 1.0e-6 1.8e-6; 3.0e-6 3.4e-6 4.0e-6)
-// With decays a hundred times slower the float32 coefficients bound every path: y 6.6e-5 both, 4.1e-6 and 4.4e-6
-// in rows of 121 steps, the only place where y and dx are further off than before (K again).  The third pieces cost 7 %:
-// 4 x 2048 rows of 5001 steps forward and backward 168 -> 180 us.
+// The lengths of the last two came to these kernels from a float32 convolution and keep its precision: P, Pg and K have
+// a third bf16 piece, products of two split factors keep their lo * lo term, and the state after the last step is
+// summed with powers that are evaluated directly.  Relative errors against 64 bits (2-norm, the largest over 121 .. 32767
+// steps) at the layer's initial decays, the convolution's, these kernels' and in brackets two pieces':
+//   dx before rounding (y alike)  4.0e-6                   4.7e-7 (2.7e-6)
+//   state after the last step     2.6e-7                   2.1e-7 (1.5e-6; of float16 rows 2.2e-6)
+//   dalpha, ddelta, dtheta        9.7e-7, 1.2e-6, 1.7e-6   3.4e-7, 6.3e-7, 1.4e-6 (5.3e-7, 1.0e-6, 1.8e-6; 3.0e-6, 3.4e-6, 4.0e-6)
+// With decays ten and a hundred times slower, where the float32 coefficients bound every path: dx 4.8e-6 / 3.1e-6 and
+// 7.5e-5 both (3.3e-6 instead of 4.0e-6 in rows of 121 steps).  The pieces cost 13 %: 4 x 2048 rows of 5001 steps forward and
+// backward 177 -> 200 us on one box.
 template <int ROWS> constexpr bool kFine = ROWS != kWhole;
 typedef u32x4 u32x4_any __attribute__((aligned(2)));
 // of the 16-bit steps elem .. elem + 7 those of lo .. hi - 1, zeros for the others
@@ -270,6 +289,7 @@ struct FwdSmem {
 static_assert(sizeof(cf) * 16 * (kT + 2) <= sizeof(float) * (kWaves * 32 + 1) * kHP, "the power table fits the state buffer");
 struct FwdSmemFine : FwdSmem {
   u32x4 third[4][kWave];  // third pieces of P
+  alignas(4) ThirdTable kthird;
 };
 static_assert(3 * sizeof(FwdSmemFine) <= 160 * 1024, "three workgroups per compute unit");
 
@@ -462,6 +482,7 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
       if constexpr (FINE)
         if (blk < 4) sm.third[blk][ln] = split8_third(v, hi, lo);
     }
+    if constexpr (FINE) fill_thirds<true>(sm.kthird, sm.klocal, tid);
     __syncthreads();
     rp = next_rp;
   };
@@ -524,7 +545,12 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
         for (int i = 0; i < 16; ++i) yacc[it][i] = 0.f;
         if (w.nc > 0) {
 #pragma unroll
-          for (int s = 0; s < 2 + 2 * it; ++s) yacc[it] = mma_split<XP, FINE>(K[1 + 2 * it - s], xb[s].pc, yacc[it]);
+          for (int s = 0; s < 2 + 2 * it; ++s) {
+            const int b = 1 + 2 * it - s;
+            yacc[it] = mma_split<XP, FINE>(K[b], xb[s].pc, yacc[it]);
+            // (block b: lags 16 (b - 1) + r - 8 g - e)
+            if constexpr (FINE) yacc[it] = mfma_bf16(read_thirds(sm.kthird, kT - 1 - 16 * (b - 1) - r + 8 * g), xb[s].pc[0], yacc[it]);
+          }
         }
       }
     }
@@ -770,7 +796,6 @@ struct BwdSmem {
   // private tile for the parked dy / x data before they are written; between rows the buffer
   // holds the power table (setup) and the reduction scratch (finish).
   float R[kBwdNC * kRP];
-  float klocal[kT];
   float pn[16];
   cf gn[16];
   cf pw[14][16];                         // powers evaluated directly (see setup_row)
@@ -788,13 +813,14 @@ struct BwdSums {
 static_assert(sizeof(BwdSums) <= sizeof(cf) * 4 * 2 * 16, "a wave's sums fit its four sub-segments");
 struct BwdSmemFine : BwdSmem {
   u32x4 third[4][kWave];                 // third pieces of Pg, first kind (the second kind's: in registers)
+  alignas(4) ThirdTable kthird;
 };
 static_assert(sizeof(cf) * 16 * (kT + 2) + sizeof(cf) * 16 * 2 * 16 <= sizeof(float) * kBwdNC * kRP,
               "the power table and the final partial sums live in the state buffer");
 static_assert(32 * kSP * 2 <= 32 * kRP * 4 && 16 * kWave * 4 <= 32 * kRP * 4 && kWave * 33 <= 32 * kRP,
               "a wave's parked tile and one accumulator tile fit its own rows of the state buffer");
-static_assert(sizeof(cf) * 16 * (kT + 2) + sizeof(u32x4) * 4 * kWave <= sizeof(float) * kBwdNC * kRP,
-              "the third pieces of the second kind pass through the state buffer, behind the power table");
+static_assert(sizeof(cf) * 16 * (kT + 2) + sizeof(u32x4) * 4 * kWave + sizeof(float) * kT <= sizeof(float) * kBwdNC * kRP,
+              "the third pieces of the second kind pass through the state buffer, behind the power table, k behind them");
 static_assert(sizeof(BwdSmemFine) <= 80 * 1024, "two workgroups per compute unit");
 
 // (h, h') <- (g, g') + [[m, 0], [md, m]] (h, h'): one step of the reverse scan, over a chunk
@@ -832,6 +858,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
   cf (*qp)[kT + 2] = reinterpret_cast<cf(*)[kT + 2]>(sm.R);                 // setup and finish only
   cf (*ab)[2][16] = reinterpret_cast<cf(*)[2][16]>(sm.R + 2 * 16 * (kT + 2));  // finish only, behind the table
   u32x4 (*passed)[kWave] = reinterpret_cast<u32x4(*)[kWave]>(sm.R + 2 * 16 * (kT + 2));  // setup only, the same place
+  float* const klocal = sm.R + 2 * 16 * (kT + 2) + 4 * 4 * kWave;  // setup only: k[0 .. 63] (+ omega at lag 0)
   auto sums = [&](int wv) -> BwdSums& { return *reinterpret_cast<BwdSums*>(&sm.sub_end[4 * wv][0][0]); };  // finish only
   u32x4 third1[4];  // FINE: third pieces of Pg, second kind
   // the last four tiles of a group's line, where its walk starts
@@ -914,7 +941,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       for (int e = 0; e < 4; ++e) {
         qp[sn][4 * sa + e] = v;
         const float kl = group_sum<16>(c.x * v.x - c.y * v.y);
-        if (sn == 0) sm.klocal[4 * sa + e] = (sa == 0 && e == 0) ? kl + rp.w : kl;  // omega on the diagonal
+        if (sn == 0) klocal[4 * sa + e] = (sa == 0 && e == 0) ? kl + rp.w : kl;  // omega on the diagonal
         v = cmul(v, q1);
       }
       if (sa == 15) qp[sn][kT] = sm.pw[9][sn];
@@ -940,7 +967,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const int lag = o - rr + 8 * gg + e;
-          const float kv = sm.klocal[lag >= 0 ? lag : 0];  // read, then masked: no branch around the load
+          const float kv = klocal[lag >= 0 ? lag : 0];  // read, then masked: no branch around the load
           v[e] = lag >= 0 ? kv : 0.f;
         }
       } else {
@@ -960,6 +987,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       if constexpr (FINE)
         if (blk < 8) (blk < 4 ? sm.third[blk] : passed[blk - 4])[ln] = split8_third(v, hi, lo);
     }
+    if constexpr (FINE) fill_thirds<false>(sm.kthird, klocal, tid);
 #pragma unroll
     for (int t = 0; t < 3; ++t)
 #pragma unroll
@@ -1309,6 +1337,8 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
           u32x4 a[2];
           load_block(8 + s - 2 * jt, a, lane);
           acc = mma_split<1>(a, db[s].pc, acc);
+          // (block b: lags 16 b - r + 8 g + e)
+          if constexpr (FINE) acc = mfma_bf16(read_thirds(sm.kthird, 16 * (s - 2 * jt) - r + 8 * g + 31), db[s].pc[0], acc);
         }
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
