@@ -25,8 +25,8 @@
 // matrices costs as much as half an item, and a row of 2048 steps fills one wave: rows are cut
 // into tiles of 32 chunks (2048 steps), the tiles of a channel's rows stand in one line, and a
 // workgroup takes four of them at a time, a tile per wave; the recurrence starts anew where a tile
-// is the first of its row.  (4 x 2048 rows of 5001 steps, forward and backward: 329 us with a row per
-// workgroup, 241 us so.)
+// is the first of its row.  (4 x 2048 rows of 5000 steps, forward and backward: 254 us with a row per
+// workgroup, 161 us so; 4096 single rows of 32768 steps 419 and 420.)
 #include "common.hpp"
 #include "cema_pow.hpp"
 
@@ -146,7 +146,7 @@ __device__ __forceinline__ float opaque_one() {
 //            every access but those at the two ends is aligned
 //   kAny     a carried state, or a tensor that starts or ends off a boundary: the same 16-byte accesses at
 //            any element's address (which cost more: 4 x 2048 rows of 5001 steps forward and backward
-//            241 us so, 191 shifted, 169 for 5000 steps)
+//            258 us so, 190 shifted; 161 for 5000 steps, whole rows without third pieces)
 enum { kWhole = 0, kShifted = 1, kAny = 2 };
 // The lengths of the last two came to these kernels from a float32 convolution and keep its precision: P, Pg and K have
 // a third bf16 piece, products of two split factors keep their lo * lo term, and the state after the last step is
@@ -157,7 +157,7 @@ enum { kWhole = 0, kShifted = 1, kAny = 2 };
 //   dalpha, ddelta, dtheta        9.7e-7, 1.2e-6, 1.7e-6   3.4e-7, 6.3e-7, 1.4e-6 (5.3e-7, 1.0e-6, 1.8e-6; 3.0e-6, 3.4e-6, 4.0e-6)
 // With decays ten and a hundred times slower, where the float32 coefficients bound every path: dx 4.8e-6 / 3.1e-6 and
 // 7.5e-5 both (3.3e-6 instead of 4.0e-6 in rows of 121 steps).  The pieces cost 13 %: 4 x 2048 rows of 5001 steps forward and
-// backward 177 -> 200 us on one box.
+// backward 168 -> 190 us.
 template <int ROWS> constexpr bool kFine = ROWS != kWhole;
 typedef u32x4 u32x4_any __attribute__((aligned(2)));
 // of the 16-bit steps elem .. elem + 7 those of lo .. hi - 1, zeros for the others
@@ -302,8 +302,7 @@ struct Lines {
   __device__ __forceinline__ int tiles(int group) const { return min(nb, B - first_row(group)) * tpr; }
 };
 // A tile of a group's line: which row, where in it.  Stepping from one of a wave's tiles to the
-// next needs no division; lanes address inside it by 32-bit offsets from a base that the wave shares
-// (4096 rows of 32768 steps forward and backward: 458 us with 64-bit offsets from the row, 446 so).
+// next needs no division; lanes address inside it by 32-bit offsets from a base that the wave shares.
 struct Tile {
   int64_t row;  // b D + d
   int64_t base; // element where the tile starts (kShifted: a row's first one, up to seven in front of the row)
