@@ -503,6 +503,7 @@ bool turned(const Tensor& g, const Tensor& w) {
 // x W^T (+ bias), or x W^T + residual with the residual as the product's accumulator input
 Tensor linear_raw(const Tensor& x, const Tensor& weight, const Optional& bias, const Optional& residual) {
   if (!residual.has_value()) return at::linear(x, weight, bias);
+  require(x.dim() >= 1 && residual->dim() >= 1, "linear: x and residual need at least one dimension");
   auto shape = x.sizes().vec();
   shape.back() = weight.size(0);
   return at::addmm(flat(*residual), flat(x), weight.t()).view(shape);

@@ -146,3 +146,11 @@ def test_linear_second_derivatives(layers, bias, residual):
         results.append(torch.autograd.grad(penalty, leaves))
     for a, b in zip(*results):
         assert (a.float() - b).norm() <= 2e-2 * b.norm()
+
+
+def test_rows_without_dimensions_are_refused():
+    lin = Linear(64, 32, bias=False).cuda().bfloat16()
+    scalar = torch.zeros((), dtype=torch.bfloat16, device="cuda")
+    for x, r in ((scalar, scalar), (_randn(4, 64), scalar), (scalar, _randn(4, 32))):
+        with pytest.raises((RuntimeError, IndexError)):
+            lin(x, residual=r)
