@@ -229,3 +229,30 @@ def test_weights_of_other_shapes_are_refused(name, shape):
         setattr(blk.get_submodule(owner), leaf, torch.nn.Parameter(torch.zeros(shape, dtype=torch.bfloat16, device="cuda")))
         with pytest.raises(RuntimeError):
             decode_step(blk, x, rotary.get_freqs_cis(9, 10), cache) or blk(x, rotary.get_freqs_cis(9, 10), None, cache)
+
+
+def test_step_in_a_graph():
+    """A captured step replays on what its input tensors hold then, and leaves the cache that it reads alone."""
+    blk = _block(256, 128, 512, 512, 2, 2, 512)
+    rotary = RotaryEmbedding(64, 512).cuda()
+    xs = [torch.randn(2, 1, 256, generator=torch.Generator().manual_seed(s)).bfloat16().cuda() for s in range(4)]
+    freqs = rotary.get_freqs_cis(30, 31)
+    with torch.no_grad():
+        cache = _prompt(blk, 2, 30, 256, 128, 512, 2, torch.bfloat16, rotary)
+        before = [t.clone() for t in _tensors(cache)]
+        wanted = [decode_step(blk, x, freqs, cache) for x in xs]
+        x = xs[0].clone()
+        stream = torch.cuda.Stream()
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            decode_step(blk, x, freqs, cache)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            y, after = decode_step(blk, x, freqs, cache)
+        for source, (out, kept) in zip(xs, wanted):
+            x.copy_(source)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, out) and all(torch.equal(a, b) for a, b in zip(_tensors(after), _tensors(kept)))
+            assert all(torch.equal(a, b) for a, b in zip(_tensors(cache), before))
