@@ -618,11 +618,12 @@ int mega_group_sequence_norm_bwd(const void* dy, const void* x, const int64_t* c
  * which is the recurrence h[t] = q h[t-1] + p x[t], out[t] = Re sum_n gamma_n
  * h_n[t] + omega x[t] with h[-1] = hx.  The row is processed in chunks of 64
  * steps as matrix products on the matrix cores (bf16 operand pieces carrying
- * 16 significant bits, float32 states and accumulation); x is read once and
- * out written once.
- *   x, y (B, D, L) of `dtype` (MEGA_BF16, MEGA_F16 or MEGA_F32; float32 rows
- *   enter the products with their 16 leading bits, y is written in float32),
- *   16-byte aligned, any L % 8 == 0 (no upper limit); p (D, N) float32; log_q, gamma (D, N)
+ * 16 significant bits, 24 for the matrices that make states and for k in 16-bit rows whose
+ * length is no multiple of 8 or that start off a 16-byte boundary; float32 states and
+ * accumulation); x is read once and out written once.
+ *   x, y (B, D, L) of `dtype`: MEGA_BF16 or MEGA_F16, any L >= 1 and any alignment, or
+ *   MEGA_F32, 16-byte aligned with L % 8 == 0 (float32 rows enter the products with their 16
+ *   leading bits, y is written in float32); no upper limit of L; p (D, N) float32; log_q, gamma (D, N)
  *   complex64 as mega_ema_weight_fwd takes them, N <= 16; omega (D) float32 or
  *   null; h0 (B, D, N) complex64 or null (zero state); h_last (B, D, N)
  *   complex64 or null (not wanted).
@@ -638,8 +639,8 @@ int mega_cema_scan_fwd(const void* x, int dtype, const float* p, const float* lo
  * replaces the chain fftconv_bwd -> (dx, dk), ema_parameters_bwd(dk, ...) ->
  * (dp, dq, dgamma) and the two elementwise passes of the skip term
  *   (fused_ops/fftconv.py:53-75, csrc/ops/ema_parameters.cc:80-98,141-156);
- * dk is never formed.  dy, x, dx (B, D, L) bfloat16, 16-byte aligned,
- * L % 8 == 0; the parameter gradients come PER ROW, (B, D, N) -- dp float32,
+ * dk is never formed.  dy, x, dx (B, D, L) bfloat16, any L >= 1 and any alignment;
+ * the parameter gradients come PER ROW, (B, D, N) -- dp float32,
  * dq and dgamma complex64 in PyTorch's conjugate convention, as
  * mega_ema_weight_bwd returns them -- and domega (B, D) float32; the caller
  * sums over B.  mega_cema_scan_bwd_supported(dtype, N, L) tells whether a
