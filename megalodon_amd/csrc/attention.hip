@@ -49,6 +49,7 @@ int attention_probs_fused(int dtype, const uint16_t* q, const uint16_t* k, uint1
 namespace {
 
 constexpr int kTile = 256;     // workgroup tile (M and N)
+constexpr int kSmall = 128;    // the same where 256 leaves compute units idle
 constexpr int kSlab = 32;      // k elements staged per iteration
 // LDS slab layout: 16-byte chunks (8 k values of one row), chunk (c, row) at
 // index c * kChunkPitch + row.  A fragment read then has consecutive lanes on
@@ -114,6 +115,7 @@ struct GemmParams {
   int mt_count, nt_count;  // tiles along m and n
   int per_batch;           // work items per batch index
   int items;               // per_batch * batch
+  int snake;               // 128-wide tiles of unequal length: all of them run at once
   int ta, tb;   // operand is k-major: element (m, k) at [k * ld + m]
   int kvb;      // rows of k that a k-major B holds when K has been rounded up behind them (0: all K); A holds
                 // zeros there, and zeros stand in for those rows of B (0 times an infinity would be NaN)
@@ -454,13 +456,21 @@ __device__ __forceinline__ void load_to_lds16(u32x4 buffer, uint32_t offset, uin
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(offset), "s"(buffer), "s"(lds_dst));
 }
 
-// RAG: p.kvb and p.ms are set (two k-major operands)
-template <int DT, bool TA, bool TB, bool RAG = false>
-__global__ __launch_bounds__(2 * kThreads) void gemm_dma_kernel(const GemmParams p) {
+//
+// T: the workgroup's tile, 256 (2 x 4 waves of 128 x 64) or 128 (2 x 2 waves of 64 x 64, two workgroups per CU).
+// RAG: p.kvb and p.ms are set (B k-major)
+template <int DT, bool TA, bool TB, bool RAG = false, int T = kTile>
+__global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
   extern __shared__ __align__(16) uint16_t smem[];
   constexpr int JN = 2, NL = 2, EP = 64 + 8;
+  constexpr int IT = T / 64;                 // 32-row blocks of a wave
+  constexpr int NW = T / 32;                 // waves
+  constexpr int kOperand = T * kSlab;        // elements of an operand slab
+  constexpr int kStage = 2 * kOperand;
+  constexpr int CR = T / 8;                  // 16-byte chunks of a row of k
+  constexpr int KR = 64 / CR;                // rows of k in a 1 KB piece
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  const int wm = wave >> 2, wn = wave & 3;
+  const int wm = wave / (NW / 2), wn = wave % (NW / 2);
   // work items as in gemm_kernel
   const int G = static_cast<int>(gridDim.x), lin = static_cast<int>(blockIdx.x);
   int it_lo, it_hi, it_step;
@@ -474,20 +484,37 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_kernel(const GemmParams
     it_hi = p.items;
     it_step = G;
   }
+  if (T != kTile && p.snake) it_lo = lin, it_hi = p.items, it_step = G;  // one item per workgroup, in order
   for (int item = it_lo; item < it_hi; item += it_step) {
-  const int zz = item / p.per_batch;
+  int zz = item / p.per_batch;
   const int rem = item % p.per_batch;
   int nt, mt_first, mt_second = -1;
   if (p.tri_out) {
     int t = rem, m = 0;
     while (true) {
-      const int cnt = min(p.nt_count, (m * kTile + (kTile - 1) + p.off) / kTile + 1);
+      const int cnt = min(p.nt_count, (m * T + (T - 1) + p.off) / T + 1);
       if (t < cnt) break;
       t -= cnt;
       ++m;
     }
     mt_first = m;
     nt = t;
+  } else if (p.k_mode && T != kTile) {
+    // One tile per item, its length falling with its rank.  Where all of them run at once (snake), the two of a
+    // CU are a grid's half apart: the longer half of the row blocks, longest first, then the shorter half, shortest
+    // first.  Else long and short ones in turn, batch by batch.
+    int rank;
+    if (p.snake) {
+      const int layer = p.nt_count * (p.items / p.per_batch), pr = item / layer, h = (p.mt_count + 1) / 2;
+      zz = item % layer / p.nt_count;
+      nt = item % p.nt_count;
+      rank = pr >= h ? p.mt_count - 1 - (pr - h) : pr;
+    } else {
+      const int pr = rem / p.nt_count;
+      nt = rem % p.nt_count;
+      rank = (pr & 1) ? p.mt_count - 1 - (pr >> 1) : pr >> 1;
+    }
+    mt_first = p.k_mode == 1 ? p.mt_count - 1 - rank : rank;
   } else if (p.k_mode) {
     nt = rem % p.nt_count;
     const int pr = rem / p.nt_count;
@@ -512,15 +539,15 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_kernel(const GemmParams
   for (int half = 0; half < 2; ++half) {
   const int mt = half == 0 ? mt_first : mt_second;
   if (mt < 0) break;
-  const int m0 = mt * kTile, n0 = nt * kTile;
+  const int m0 = mt * T, n0 = nt * T;
   int kb = 0, ke = p.K;
-  if (p.k_mode == 1) ke = min(p.K, ((mt + 1) * kTile + p.off + kSlab - 1) / kSlab * kSlab);
-  if (p.k_mode == 2) kb = min(p.K, max(0, mt * kTile - p.off) / kSlab * kSlab);
+  if (p.k_mode == 1) ke = min(p.K, ((mt + 1) * T + p.off + kSlab - 1) / kSlab * kSlab);
+  if (p.k_mode == 2) kb = min(p.K, max(0, mt * T - p.off) / kSlab * kSlab);
   const int nslab = (ke - kb + kSlab - 1) / kSlab;
 
-  floatx16 acc[4][JN];
+  floatx16 acc[IT][JN];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < IT; ++i)
 #pragma unroll
     for (int j = 0; j < JN; ++j)
 #pragma unroll
@@ -532,8 +559,8 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_kernel(const GemmParams
   uint32_t offa[NL], offb[NL];
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
-    const int pc = wave + 8 * i;
-    const int krow = 2 * pc + (lane >> 5), cm = (lane & 31) ^ ((krow & 3) << 2);  // k-major piece
+    const int pc = wave + NW * i;
+    const int krow = KR * pc + lane / CR, cm = (lane % CR) ^ ((krow & 3) << 2);  // k-major piece
     const int row = 16 * pc + (lane >> 2), ck = (lane & 3) ^ ((lane >> 4) & 3);   // k-contiguous piece
     if (TA) offa[i] = static_cast<uint32_t>(((kb + krow) * p.lda + min(m0 + cm * 8, p.M - 8)) * 2);
     else offa[i] = static_cast<uint32_t>((static_cast<int64_t>(min(m0 + row, p.M - 1)) * p.lda + kb + ck * 8) * 2);
@@ -549,7 +576,7 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_kernel(const GemmParams
   // request number n of a slab: n = 0, 2 the two pieces of A, n = 1, 3 those of B
   auto request_one = [&](int s, int stage, int n) {
     const uint32_t sc = static_cast<uint32_t>(min(s, nslab - 1));
-    const uint32_t dst = lds_wave + static_cast<uint32_t>(stage * kDmaStage + (n >> 1) * 8 * 512 + (n & 1) * kDmaOperand) * 2;
+    const uint32_t dst = lds_wave + static_cast<uint32_t>(stage * kStage + (n >> 1) * NW * 512 + (n & 1) * kOperand) * 2;
     if (n & 1) {
       static_assert(TB || !RAG, "rows of k");
       if constexpr (RAG) load_to_lds16(bufb, offb[n >> 1] + sc * stepb, dst);
@@ -566,25 +593,25 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_kernel(const GemmParams
   // fragment side: k-step `set` of a slab takes k = 16 g + 8 set + e for lane half g
   const int g = lane >> 5, r = lane & 31;
   const int ta_a = (lane & 15) >> 2, ta_h = (lane >> 4) & 1, ta_b = lane & 3;
-  int fra[4], frb[JN];
+  int fra[IT], frb[JN];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if (TA) fra[i] = (16 * g + ta_a) * kTile + (((wm * 16 + 4 * i + 2 * ta_h + (ta_b >> 1)) ^ (ta_a << 2)) * 8) + 4 * (ta_b & 1);
-    else fra[i] = (wm * 128 + 32 * i + r) * kSlab + (((2 * g) ^ ((r >> 2) & 3)) * 8);
+  for (int i = 0; i < IT; ++i) {
+    if (TA) fra[i] = (16 * g + ta_a) * T + (((wm * 4 * IT + 4 * i + 2 * ta_h + (ta_b >> 1)) ^ (ta_a << 2)) * 8) + 4 * (ta_b & 1);
+    else fra[i] = (wm * 32 * IT + 32 * i + r) * kSlab + (((2 * g) ^ ((r >> 2) & 3)) * 8);
   }
 #pragma unroll
   for (int j = 0; j < JN; ++j) {
-    if (TB) frb[j] = kDmaOperand + (16 * g + ta_a) * kTile + (((wn * 8 + 4 * j + 2 * ta_h + (ta_b >> 1)) ^ (ta_a << 2)) * 8) + 4 * (ta_b & 1);
-    else frb[j] = kDmaOperand + (wn * 64 + 32 * j + r) * kSlab + (((2 * g) ^ ((r >> 2) & 3)) * 8);
+    if (TB) frb[j] = kOperand + (16 * g + ta_a) * T + (((wn * 8 + 4 * j + 2 * ta_h + (ta_b >> 1)) ^ (ta_a << 2)) * 8) + 4 * (ta_b & 1);
+    else frb[j] = kOperand + (wn * 64 + 32 * j + r) * kSlab + (((2 * g) ^ ((r >> 2) & 3)) * 8);
   }
-  u32x4 fa0[4], fb0[JN], fa1[4], fb1[JN];
+  u32x4 fa0[IT], fb0[JN], fa1[IT], fb1[JN];
   auto fread = [&](u32x4* fa, u32x4* fb, int set, int stage) {
-    const uint16_t* base = smem + stage * kDmaStage;
+    const uint16_t* base = smem + stage * kStage;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < IT; ++i) {
       if (TA) {
-        const uint16_t* q = base + fra[i] + set * 8 * kTile;
-        const uint2 lo = lds_read_tr(q), hi = lds_read_tr(q + 4 * kTile);
+        const uint16_t* q = base + fra[i] + set * 8 * T;
+        const uint2 lo = lds_read_tr(q), hi = lds_read_tr(q + 4 * T);
         fa[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
       } else {
         // chunk 2 g + set sits at position (2 g + set) ^ swizzle = ((2 g) ^ swizzle) ^ set
@@ -592,8 +619,8 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_kernel(const GemmParams
       }
       if (i < JN) {
         if (TB) {
-          const uint16_t* q = base + frb[i] + set * 8 * kTile;
-          const uint2 lo = lds_read_tr(q), hi = lds_read_tr(q + 4 * kTile);
+          const uint16_t* q = base + frb[i] + set * 8 * T;
+          const uint2 lo = lds_read_tr(q), hi = lds_read_tr(q + 4 * T);
           fb[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
         } else {
           fb[i] = *reinterpret_cast<const u32x4*>(base + (frb[i] ^ (set * 8)));
@@ -604,7 +631,7 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_kernel(const GemmParams
   // products lo .. hi - 1 of a k-step, numbered 2 i + j
   auto mma = [&](const u32x4* fa, const u32x4* fb, int lo, int hi) {
 #pragma unroll
-    for (int n = 0; n < 4 * JN; ++n)
+    for (int n = 0; n < IT * JN; ++n)
       if (n >= lo && n < hi) acc[n >> 1][n & 1] = Mma<DT>::run(fb[n & 1], fa[n >> 1], acc[n >> 1][n & 1]);
   };
 
@@ -615,29 +642,29 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_kernel(const GemmParams
   //   second half: read the first fragment set of slab cur + 1, request slab cur + 4 into
   //                the buffer slab cur has just left, 8 MFMAs on the second set.
 #define MEGA_SGB(mask, n) __builtin_amdgcn_sched_group_barrier(mask, n, 0)
-  constexpr int kFragReads = (TA ? 2 : 1) + (TB ? JN / 2 : (JN + 3) / 4);
+  constexpr int kFragReads = (TA ? 2 : 1) + (JN * (TB ? 2 : 1) + IT - 1) / IT;
 #define MEGA_DMA_STEP(R)                                                   \
   {                                                                        \
     const int cur = it + (R);                                              \
     fread(fa1, fb1, 1, (R));                                               \
-    mma(fa0, fb0, 0, 8);                                                   \
-    _Pragma("unroll") for (int sg = 0; sg < 4; ++sg) {                     \
+    mma(fa0, fb0, 0, IT * JN);                                             \
+    _Pragma("unroll") for (int sg = 0; sg < IT; ++sg) {                    \
       MEGA_SGB(0x008, 1);                                                  \
       MEGA_SGB(0x100, kFragReads);                                         \
     }                                                                      \
-    MEGA_SGB(0x008, 4 * JN - 4);                                           \
+    MEGA_SGB(0x008, IT * JN - IT);                                         \
     __builtin_amdgcn_sched_barrier(0);                                     \
     asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory"); \
     fread(fa0, fb0, 0, ((R) + 1) & 3);                                     \
-    mma(fa1, fb1, 0, 4);                                                   \
-    _Pragma("unroll") for (int sg = 0; sg < 4; ++sg) {                     \
+    mma(fa1, fb1, 0, IT);                                                  \
+    _Pragma("unroll") for (int sg = 0; sg < IT; ++sg) {                    \
       MEGA_SGB(0x008, 1);                                                  \
       MEGA_SGB(0x100, kFragReads);                                         \
     }                                                                      \
     __builtin_amdgcn_sched_barrier(0);                                     \
     _Pragma("unroll") for (int n = 0; n < 2 * NL; ++n) {                   \
       request_one(cur + kStages, (R), n);                                  \
-      mma(fa1, fb1, 4 + n, 5 + n);                                         \
+      mma(fa1, fb1, IT + n, IT + 1 + n);                                   \
       __builtin_amdgcn_sched_barrier(0);                                   \
     }                                                                      \
   }
@@ -664,10 +691,10 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_kernel(const GemmParams
 #undef MEGA_DMA_STEP
 #undef MEGA_SGB
 
-  // epilogue as in gemm_kernel: the wave's 128 x 64 tile through its own LDS region
-  uint16_t* stage = smem + wave * 128 * EP;
+  // epilogue as in gemm_kernel: the wave's tile through its own LDS region
+  uint16_t* stage = smem + wave * 32 * IT * EP;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < IT; ++i) {
 #pragma unroll
     for (int j = 0; j < JN; ++j) {
       const int row = i * 32 + (lane & 31);
@@ -692,10 +719,10 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_kernel(const GemmParams
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave reads back only its own region
   const bool vec_ok = (p.ldc % 8 == 0) && (reinterpret_cast<uintptr_t>(C) % 16 == 0);
 #pragma unroll 4
-  for (int i = 0; i < 8 * JN; ++i) {
+  for (int i = 0; i < 2 * IT * JN; ++i) {
     const int c = lane + kWave * i;
     const int row = c / (4 * JN), kc = (c % (4 * JN)) * 8;
-    const int grow = m0 + wm * 128 + row, gcol = n0 + wn * (32 * JN) + kc;
+    const int grow = m0 + wm * 32 * IT + row, gcol = n0 + wn * (32 * JN) + kc;
     if (grow < (RAG ? p.ms : p.M) && gcol < p.N) {
       const u32x4 v = *reinterpret_cast<const u32x4*>(stage + row * EP + kc);
       uint16_t* dst = C + static_cast<int64_t>(grow) * p.ldc + gcol;
@@ -732,12 +759,14 @@ constexpr int kDma64Operand = kTile * kSlab64;  // elements of an operand slab (
 constexpr int kDma64Stage = 2 * kDma64Operand;
 static_assert(sizeof(uint16_t) * 2 * kDma64Stage <= kDmaLds, "two slab buffers fit");
 
-template <int DT, bool TA, bool TB>
-__global__ __launch_bounds__(2 * kThreads) void gemm_dma64_kernel(const GemmParams p) {
+template <int DT, bool TA, bool TB, int T = kTile>
+__global__ __launch_bounds__(2 * T) void gemm_dma64_kernel(const GemmParams p) {
   extern __shared__ __align__(16) uint16_t smem[];
   constexpr int JN = 2, NL = 4, EP = 64 + 8;
+  constexpr int IT = T / 64, NW = T / 32, kOperand = T * kSlab64, kStage = 2 * kOperand;  // as in gemm_dma_kernel
+  static_assert(T == kTile || (!TA && !TB), "pieces of k rows are written for 256 columns");
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  const int wm = wave >> 2, wn = wave & 3;
+  const int wm = wave / (NW / 2), wn = wave % (NW / 2);
   const int G = static_cast<int>(gridDim.x), lin = static_cast<int>(blockIdx.x);
   int it_lo, it_hi, it_step;
   if (G % kXcds == 0) {
@@ -757,7 +786,7 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma64_kernel(const GemmPara
   if (p.tri_out) {
     int t = rem, m = 0;
     while (true) {
-      const int cnt = min(p.nt_count, (m * kTile + (kTile - 1) + p.off) / kTile + 1);
+      const int cnt = min(p.nt_count, (m * T + (T - 1) + p.off) / T + 1);
       if (t < cnt) break;
       t -= cnt;
       ++m;
@@ -768,7 +797,7 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma64_kernel(const GemmPara
     nt = rem % p.nt_count;
     const int pr = rem / p.nt_count;
     mt_first = p.mt_count - 1 - pr;
-    if (mt_first != pr) mt_second = pr;
+    if (T == kTile && mt_first != pr) mt_second = pr;
   } else {
     nt = rem % p.nt_count;
     mt_first = rem / p.nt_count;
@@ -780,17 +809,17 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma64_kernel(const GemmPara
   for (int half = 0; half < 2; ++half) {
   const int mt = half == 0 ? mt_first : mt_second;
   if (mt < 0) break;
-  const int m0 = mt * kTile, n0 = nt * kTile;
+  const int m0 = mt * T, n0 = nt * T;
   // k range as in gemm_kernel, widened to whole slabs of 64 (K % 64 == 0): what the wider range
   // adds are probabilities the softmax has written as zeros
   int kb = 0, ke = p.K;
-  if (p.k_mode == 1) ke = min(p.K, ((mt + 1) * kTile + p.off + kSlab64 - 1) / kSlab64 * kSlab64);
-  if (p.k_mode == 2) kb = min(p.K, max(0, mt * kTile - p.off) / kSlab64 * kSlab64);
+  if (p.k_mode == 1) ke = min(p.K, ((mt + 1) * T + p.off + kSlab64 - 1) / kSlab64 * kSlab64);
+  if (p.k_mode == 2) kb = min(p.K, max(0, mt * T - p.off) / kSlab64 * kSlab64);
   const int nslab = (ke - kb + kSlab64 - 1) / kSlab64;
 
-  floatx16 acc[4][JN];
+  floatx16 acc[IT][JN];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < IT; ++i)
 #pragma unroll
     for (int j = 0; j < JN; ++j)
 #pragma unroll
@@ -800,7 +829,7 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma64_kernel(const GemmPara
   uint32_t offa[NL], offb[NL];
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
-    const int pc = wave + 8 * i;
+    const int pc = wave + NW * i;
     const int krow = 2 * pc + (lane >> 5), cm = (lane & 31) ^ ((krow & 3) << 2);   // k-major piece: 2 rows of k
     const int row = 8 * pc + (lane >> 3), ck = (lane & 7) ^ ((row >> 1) & 7);      // k-contiguous piece: 8 rows
     if (TA) offa[i] = static_cast<uint32_t>(((kb + krow) * p.lda + min(m0 + cm * 8, p.M - 8)) * 2);
@@ -815,7 +844,7 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma64_kernel(const GemmPara
   // request number n of a slab: even n the pieces of A, odd n those of B
   auto request_one = [&](int s, int stage, int n) {
     const uint32_t sc = static_cast<uint32_t>(min(s, nslab - 1));
-    const uint32_t dst = lds_wave + static_cast<uint32_t>(stage * kDma64Stage + (n >> 1) * 8 * 512 + (n & 1) * kDma64Operand) * 2;
+    const uint32_t dst = lds_wave + static_cast<uint32_t>(stage * kStage + (n >> 1) * NW * 512 + (n & 1) * kOperand) * 2;
     if (n & 1) load_to_lds16(B, offb[n >> 1] + sc * stepb, dst);
     else load_to_lds16(A, offa[n >> 1] + sc * stepa, dst);
   };
@@ -827,23 +856,23 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma64_kernel(const GemmPara
   // fragment side: k-step `set` (0 .. 3) of a slab takes k = 16 set + 8 g + e for lane half g
   const int g = lane >> 5, r = lane & 31;
   const int ta_a = (lane & 15) >> 2, ta_h = (lane >> 4) & 1, ta_b = lane & 3;
-  int fra[4], frb[JN];
+  int fra[IT], frb[JN];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < IT; ++i) {
     if (TA) fra[i] = (8 * g + ta_a) * kTile + (((wm * 16 + 4 * i + 2 * ta_h + (ta_b >> 1)) ^ (ta_a << 2)) * 8) + 4 * (ta_b & 1);
-    else fra[i] = (wm * 128 + 32 * i + r) * kSlab64 + ((g ^ ((r >> 1) & 7)) * 8);
+    else fra[i] = (wm * 32 * IT + 32 * i + r) * kSlab64 + ((g ^ ((r >> 1) & 7)) * 8);
   }
 #pragma unroll
   for (int j = 0; j < JN; ++j) {
-    if (TB) frb[j] = kDma64Operand + (8 * g + ta_a) * kTile + (((wn * 8 + 4 * j + 2 * ta_h + (ta_b >> 1)) ^ (ta_a << 2)) * 8) + 4 * (ta_b & 1);
-    else frb[j] = kDma64Operand + (wn * 64 + 32 * j + r) * kSlab64 + ((g ^ ((r >> 1) & 7)) * 8);
+    if (TB) frb[j] = kOperand + (8 * g + ta_a) * kTile + (((wn * 8 + 4 * j + 2 * ta_h + (ta_b >> 1)) ^ (ta_a << 2)) * 8) + 4 * (ta_b & 1);
+    else frb[j] = kOperand + (wn * 64 + 32 * j + r) * kSlab64 + ((g ^ ((r >> 1) & 7)) * 8);
   }
-  u32x4 fa0[4], fb0[JN], fa1[4], fb1[JN];
+  u32x4 fa0[IT], fb0[JN], fa1[IT], fb1[JN];
   // fragments lo .. hi - 1 of a k-step: number i = row block i of A and, for i < JN, column block i of B
-  auto fread = [&](u32x4* fa, u32x4* fb, int set, int stage, int lo = 0, int hi = 4) {
-    const uint16_t* base = smem + stage * kDma64Stage;
+  auto fread = [&](u32x4* fa, u32x4* fb, int set, int stage, int lo = 0, int hi = T / 64) {
+    const uint16_t* base = smem + stage * kStage;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < IT; ++i) {
       if (i < lo || i >= hi) continue;
       if (TA) {
         const uint16_t* q = base + fra[i] + set * 16 * kTile;
@@ -866,7 +895,7 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma64_kernel(const GemmPara
   };
   auto mma = [&](const u32x4* fa, const u32x4* fb, int lo, int hi) {
 #pragma unroll
-    for (int n = 0; n < 4 * JN; ++n)
+    for (int n = 0; n < IT * JN; ++n)
       if (n >= lo && n < hi) acc[n >> 1][n & 1] = Mma<DT>::run(fb[n & 1], fa[n >> 1], acc[n >> 1][n & 1]);
   };
 
@@ -876,16 +905,16 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma64_kernel(const GemmPara
   // barrier; then the first fragments of the next slab, the requests for the slab after it into
   // the buffer just left (one per product), the last 8 products.
 #define MEGA_SGB(mask, n) __builtin_amdgcn_sched_group_barrier(mask, n, 0)
-  constexpr int kFragReads = (TA ? 2 : 1) + (TB ? JN / 2 : (JN + 3) / 4);
+  constexpr int kFragReads = (TA ? 2 : 1) + (JN * (TB ? 2 : 1) + IT - 1) / IT;
 #define MEGA_DMA64_KSTEP(FA, FB, NFA, NFB, SET, STAGE)                     \
   {                                                                        \
     fread(NFA, NFB, (SET) + 1, (STAGE));                                   \
-    mma(FA, FB, 0, 8);                                                     \
-    _Pragma("unroll") for (int sg = 0; sg < 4; ++sg) {                     \
+    mma(FA, FB, 0, IT * JN);                                               \
+    _Pragma("unroll") for (int sg = 0; sg < IT; ++sg) {                    \
       MEGA_SGB(0x008, 1);                                                  \
       MEGA_SGB(0x100, kFragReads);                                         \
     }                                                                      \
-    MEGA_SGB(0x008, 4);                                                    \
+    MEGA_SGB(0x008, IT * JN - IT);                                         \
     __builtin_amdgcn_sched_barrier(0);                                     \
   }
 #define MEGA_DMA64_STEP(R)                                                 \
@@ -896,7 +925,7 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma64_kernel(const GemmPara
     MEGA_DMA64_KSTEP(fa0, fb0, fa1, fb1, 2, (R))                           \
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); \
     _Pragma("unroll") for (int n = 0; n < 2 * NL; ++n) {                   \
-      if (n < 4) fread(fa0, fb0, 0, (R) ^ 1, n, n + 1);                    \
+      if (n < IT) fread(fa0, fb0, 0, (R) ^ 1, n, n + 1);                    \
       request_one(cur + 2, (R), n);                                        \
       mma(fa1, fb1, n, n + 1);                                             \
       __builtin_amdgcn_sched_barrier(0);                                   \
@@ -920,10 +949,10 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma64_kernel(const GemmPara
 #undef MEGA_DMA64_KSTEP
 #undef MEGA_SGB
 
-  // epilogue as in gemm_kernel: the wave's 128 x 64 tile through its own LDS region
-  uint16_t* stage = smem + wave * 128 * EP;
+  // epilogue as in gemm_kernel: the wave's tile through its own LDS region
+  uint16_t* stage = smem + wave * 32 * IT * EP;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < IT; ++i) {
 #pragma unroll
     for (int j = 0; j < JN; ++j) {
       const int row = i * 32 + (lane & 31);
@@ -948,10 +977,10 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma64_kernel(const GemmPara
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   const bool vec_ok = (p.ldc % 8 == 0) && (reinterpret_cast<uintptr_t>(C) % 16 == 0);
 #pragma unroll 4
-  for (int i = 0; i < 8 * JN; ++i) {
+  for (int i = 0; i < 2 * IT * JN; ++i) {
     const int c = lane + kWave * i;
     const int row = c / (4 * JN), kc = (c % (4 * JN)) * 8;
-    const int grow = m0 + wm * 128 + row, gcol = n0 + wn * (32 * JN) + kc;
+    const int grow = m0 + wm * 32 * IT + row, gcol = n0 + wn * (32 * JN) + kc;
     if (grow < p.M && gcol < p.N) {
       const u32x4 v = *reinterpret_cast<const u32x4*>(stage + row * EP + kc);
       uint16_t* dst = C + static_cast<int64_t>(grow) * p.ldc + gcol;
@@ -1453,6 +1482,67 @@ int launch_softmax(const uint16_t* p, uint16_t* x, int64_t Z, int64_t L1, int64_
 }
 
 // ------------------------------ host side --------------------------------------
+// One 128-wide tile per workgroup, two workgroups per CU; grids of whole rounds of the XCDs.
+template <int DT, bool TA, bool TB>
+int launch_small(const GemmParams& q, int cus, hipStream_t s) {
+  constexpr size_t lds = sizeof(uint16_t) * kStages * 2 * kSmall * kSlab;
+  static_assert(lds == sizeof(uint16_t) * 2 * 2 * kSmall * kSlab64 && lds >= sizeof(uint16_t) * 4 * 64 * (64 + 8), "two slabs of 64 k; holds the output tiles");
+  const dim3 grid(static_cast<unsigned>((q.items + kXcds - 1) / kXcds * kXcds));
+  // (two k-contiguous operands: whole cache lines pay where tiles share a CU, 2 x 1024 x 1024 by 2048 and a tile per CU
+  // 22 us with slabs of 64 against 18; 8 of them 28 / 35)
+  if constexpr (TB) {
+    if (q.kvb) {
+      gemm_dma_kernel<DT, TA, TB, true, kSmall><<<grid, 2 * kSmall, lds, s>>>(q);
+      MEGA_CHECK_LAUNCH();
+      return MEGA_OK;
+    }
+  }
+  if constexpr (!TA && !TB) {
+    if (q.K % kSlab64 == 0 && q.items > cus) {
+      gemm_dma64_kernel<DT, TA, TB, kSmall><<<grid, 2 * kSmall, lds, s>>>(q);
+      MEGA_CHECK_LAUNCH();
+      return MEGA_OK;
+    }
+  }
+  gemm_dma_kernel<DT, TA, TB, false, kSmall><<<grid, 2 * kSmall, lds, s>>>(q);
+  MEGA_CHECK_LAUNCH();
+  return MEGA_OK;
+}
+
+// Tiles and work items of a product in tiles of T: items in all, the k of the longest one and of all together.
+struct Tiling {
+  int mt, nt;
+  int64_t per_batch, items, longest, total;
+};
+Tiling tiling(const GemmParams& p, int batch, int T) {
+  Tiling t{(p.M + T - 1) / T, (p.N + T - 1) / T, 0, 0, p.K, 0};
+  // the k of row block mt
+  const auto kof = [&](int64_t mt) -> int64_t {
+    if (p.k_mode == 1) return std::min<int64_t>(p.K, (mt + 1) * T + p.off);
+    if (p.k_mode == 2) return p.K - std::min<int64_t>(p.K, std::max<int64_t>(0, mt * T - p.off));
+    return p.K;
+  };
+  if (p.tri_out) {
+    for (int m = 0; m < t.mt; ++m) t.per_batch += std::min<int64_t>(t.nt, (static_cast<int64_t>(m) * T + (T - 1) + p.off) / T + 1);
+    t.total = t.per_batch * p.K;
+  } else if (p.k_mode) {
+    const bool pairs = T == kTile;
+    t.per_batch = static_cast<int64_t>(t.nt) * (pairs ? (t.mt + 1) / 2 : t.mt);
+    t.longest = 0;
+    for (int m = 0; m < t.mt; ++m) {
+      const int other = t.mt - 1 - m;
+      t.longest = std::max(t.longest, kof(m) + (pairs && other != m ? kof(other) : 0));
+      t.total += t.nt * kof(m);
+    }
+  } else {
+    t.per_batch = static_cast<int64_t>(t.nt) * t.mt;
+    t.total = t.per_batch * p.K;
+  }
+  t.items = t.per_batch * batch;
+  t.total *= batch;
+  return t;
+}
+
 template <int DT, bool TA, bool TB>
 int launch_gemm_t(const GemmParams& p, int batch, hipStream_t s) {
   const auto a16 = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
@@ -1465,28 +1555,45 @@ int launch_gemm_t(const GemmParams& p, int batch, hipStream_t s) {
   GemmParams q = p;
   if (!fast && p.kvb) q.K = p.kvb;  // the bounds-checked kernel takes the real sizes
   if (!fast && p.ms) q.M = p.ms;
-  q.mt_count = (q.M + kTile - 1) / kTile;
-  q.nt_count = (p.N + kTile - 1) / kTile;
-  int64_t per_batch;
-  if (p.tri_out) {
-    per_batch = 0;
-    for (int m = 0; m < q.mt_count; ++m)
-      per_batch += std::min<int64_t>(q.nt_count, (static_cast<int64_t>(m) * kTile + (kTile - 1) + p.off) / kTile + 1);
-  } else if (p.k_mode) {
-    per_batch = static_cast<int64_t>(q.nt_count) * ((q.mt_count + 1) / 2);
-  } else {
-    per_batch = static_cast<int64_t>(q.nt_count) * q.mt_count;
-  }
-  const int64_t items = per_batch * batch;
-  MEGA_CHECK_ARG(items <= 0x7fffffff, "attention: too many tiles");
-  q.per_batch = static_cast<int>(per_batch);
-  q.items = static_cast<int>(items);
   int dev = 0, cus = 0;
   MEGA_CHECK_HIP(hipGetDevice(&dev));
   MEGA_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  Tiling t = tiling(q, batch, kTile);
+  bool small = false;
+  // Tiles of 128 where tiles of 256 leave too much of the chip idle.  A CU takes 0.21 us for 32 k of a tile of 128,
+  // alone or two at a time (0.42), and 0.5-0.6 us for a tile of 256: the costs below, in units of 0.21 us and 32 k.
+  // Tiles of unequal length spread over the CUs as they end.  Large / small in us: dQ of 2 x 1024 x 1024 by 256 29 / 10,
+  // of 32 36 / 26; P V of 8 x 1024 x 1024 by 2048 33 / 26, of 16 43 / 49, of 1 x 4096 x 4096 75 / 40, of 4 112 / 172; dP of
+  // 4 x 1531 x 1531 by 2048 75 / 28, of 16 x 1024 x 1024 45 / 52.
+  if constexpr (!TA || TB) {
+    if (fast) {
+      const Tiling u = tiling(q, batch, kSmall);
+      const double large_cost = 2.4 * static_cast<double>((t.items + cus - 1) / cus) * t.longest;
+      double small_cost = static_cast<double>(u.longest);
+      if (u.items > cus) {
+        // N <= 64: half of a small tile is idle and what counts is the reading of A, there in half cache lines
+        const double load = static_cast<double>(u.total) / cus * (!TA && p.N <= 64 ? 1.4 : 1.0);
+        small_cost = q.k_mode ? load + 0.5 * u.longest : 2.0 * static_cast<double>((u.items + 2 * cus - 1) / (2 * cus)) * u.longest;
+      }
+      small = small_cost < large_cost;
+      if (small) t = u;
+    }
+  }
+  MEGA_CHECK_ARG(t.items <= 0x7fffffff, "attention: too many tiles");
+  q.mt_count = t.mt;
+  q.nt_count = t.nt;
+  q.per_batch = static_cast<int>(t.per_batch);
+  q.items = static_cast<int>(t.items);
+  if constexpr (!TA || TB) {
+    if (small) {
+      q.snake = q.k_mode && t.items <= 2 * cus;
+      if (q.kvb && !q.ms) q.ms = q.M;
+      return launch_small<DT, TA, TB>(q, cus, s);
+    }
+  }
   // one workgroup per CU (its LDS and registers fill one); a multiple of the
   // XCD count whenever there are that many items
-  int64_t g = std::min<int64_t>(items, cus);
+  int64_t g = std::min<int64_t>(t.items, cus);
   if (g >= kXcds) g -= g % kXcds;
   const dim3 grid(static_cast<unsigned>(g));
   const size_t lds = kGemmLds;

@@ -420,8 +420,193 @@ __global__ __launch_bounds__(64 * kWaves) void attn_probs_kernel(const ProbsPara
 #undef MEGA_SGB
 }
 
+// ---- the same for few row blocks ---------------------------------------------------------------
+// Row blocks of 256 leave the chip idle at ordinary sizes (four heads and 1531 steps: 24 workgroups walk their keys
+// twice, 83 us).  Here a workgroup owns 32 query rows and its eight waves share out the keys, 32-key block
+// b to wave b % 8, so every wave holds all of its scores (KB blocks of 16 registers) at once: one pass, the row
+// maximum and the row sum combined over the waves through LDS (33 us).  A wave's keys are its own, so their
+// fragments come from memory straight into registers, a ring of RING fragments ahead of the products.
+// Rows of more than 256 KB keys (SEGMENTS) pass in pieces of that many keys: running maxima and sums, then the
+// probabilities of the last piece, whose scores are still there, and of the others from products formed again.
+// Every row block reads its keys from the L2 anew, which is what bounds full grids: those take the kernel above.
+template <int DT, int H1, int KB, bool SEGMENTS>
+__global__ __launch_bounds__(64 * kWaves) void attn_probs_short_kernel(const ProbsParams p) {
+  constexpr int QF = H1 / 16;
+  constexpr int RING = KB > 4 && QF > 8 ? 8 : QF;
+  constexpr int STEP = KB * kWaves;  // 32-key blocks of a piece
+  __shared__ float red[2][kWaves][32];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int r = lane & 31, h = lane >> 5;
+  const int idx = static_cast<int>(blockIdx.x);
+  const int mt = p.MT - 1 - idx / p.Z, z = idx % p.Z;  // long rows first
+  const int b = z / p.NH, hd = z % p.NH;
+  const int m0 = mt * 32, row = m0 + r;
+  const int ld = p.NH * H1;
+  const uint16_t* Q = p.q + static_cast<int64_t>(b) * p.L1 * ld + hd * H1;
+  const uint16_t* K = p.k + static_cast<int64_t>(b) * p.L2 * ld + hd * H1;
+
+  const int kend = p.causal ? min(p.L2, min(m0 + 32, p.L1) + p.off) : p.L2;
+  const int nblk = (kend + 31) / 32;
+  const int lim = p.causal ? min(row + p.off, p.L2 - 1) : p.L2 - 1;  // last key of this lane's row
+
+  // lane (r, h) holds k = 16 f + 8 h .. + 7 of fragment f, of its query row and of key r of a block
+  const uint16_t* kbase = K + 8 * h;
+  const auto key_row = [&](int blk) { return kbase + static_cast<int64_t>(min(32 * blk + r, p.L2 - 1)) * ld; };
+  u32x4 kf[RING], qf[QF];
+  {
+    const uint16_t* qr = Q + static_cast<int64_t>(min(row, p.L1 - 1)) * ld + 8 * h;
+#pragma unroll
+    for (int f = 0; f < QF; ++f) qf[f] = *reinterpret_cast<const u32x4*>(qr + 16 * f);
+  }
+  // scores of the piece that starts with block b0, masked: element e of accumulator i is key
+  // 32 (b0 + wave + 8 i) + 8 (e / 4) + 4 h + e % 4
+  floatx16 acc[KB];
+  const auto scores = [&](int b0) {
+    const uint16_t* first = key_row(b0 + wave);
+#pragma unroll
+    for (int f = 0; f < RING; ++f) kf[f] = *reinterpret_cast<const u32x4*>(first + 16 * f);
+#pragma unroll
+    for (int i = 0; i < KB; ++i) {
+      const int blk = b0 + wave + kWaves * i;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
+      if (blk < nblk) {
+        const uint16_t* here = key_row(blk);
+        const uint16_t* next = key_row(blk + kWaves);  // (clamped into the keys)
+#pragma unroll
+        for (int f = 0; f < QF; ++f) {
+          acc[i] = mma16<DT>(kf[f % RING], qf[f], acc[i]);
+          kf[f % RING] = *reinterpret_cast<const u32x4*>(f + RING < QF ? here + 16 * (f + RING) : next + 16 * (f + RING - QF));
+        }
+        const int x0 = 32 * blk + 4 * h;
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (x0 + 8 * (e >> 2) + (e & 3) > lim) acc[i][e] = -INFINITY;
+      }
+    }
+  };
+  const auto each = [&](int b0, auto&& f) {
+#pragma unroll
+    for (int i = 0; i < KB; ++i)
+      if (b0 + wave + kWaves * i < nblk) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][e] = f(acc[i][e]);
+      }
+  };
+  uint16_t* w = p.w + static_cast<int64_t>(z) * p.zrows * p.pitch;
+  uint16_t* wrow = w + static_cast<int64_t>(row) * p.pitch;
+  // probabilities of a piece from the accumulators, turned into 8 consecutive keys per lane
+  const auto store = [&](int b0) {
+#pragma unroll
+    for (int i = 0; i < KB; ++i) {
+      const int blk = b0 + wave + kWaves * i;
+      if (blk >= nblk) continue;
+      uint32_t px[4], py[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        px[g] = pack2<DT>(acc[i][4 * g], acc[i][4 * g + 1]);
+        py[g] = pack2<DT>(acc[i][4 * g + 2], acc[i][4 * g + 3]);
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        half_swap(px[2 * u], px[2 * u + 1]);
+        half_swap(py[2 * u], py[2 * u + 1]);
+        const u32x4 o = {px[2 * u], py[2 * u], px[2 * u + 1], py[2 * u + 1]};
+        const int col = 32 * blk + 16 * u + 8 * h;
+        if (row < p.L1 && col < p.pitch) *reinterpret_cast<u32x4*>(wrow + col) = o;
+      }
+    }
+  };
+
+  if constexpr (!SEGMENTS) {
+    scores(0);
+    float m = -INFINITY;
+    each(0, [&](float s) { return m = fmaxf(m, s), s; });
+    m = fmaxf(m, __shfl_xor(m, 32, 64));
+    if (h == 0) red[0][wave][r] = m;
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < kWaves; ++v) m = fmaxf(m, red[0][v][r]);
+    const float nm = -m * p.sl;
+    float l = 0.f;
+    each(0, [&](float s) {
+      s = __builtin_amdgcn_exp2f(fmaf(s, p.sl, nm));
+      l += s;
+      return s;
+    });
+    l += __shfl_xor(l, 32, 64);
+    if (h == 0) red[1][wave][r] = l;
+    __syncthreads();
+    l = 0.f;
+#pragma unroll
+    for (int v = 0; v < kWaves; ++v) l += red[1][v][r];
+    const float c = 1.f / l;
+    each(0, [&](float s) { return s * c; });
+    store(0);
+  } else {
+    float m = -INFINITY, l = 0.f;
+    int b0 = 0;
+    for (;; b0 += STEP) {
+      scores(b0);
+      float tm = m;
+      each(b0, [&](float s) { return tm = fmaxf(tm, s), s; });
+      const float base = tm == -INFINITY ? 0.f : tm;  // (no key of this lane's yet)
+      l *= __builtin_amdgcn_exp2f((m - base) * p.sl);
+      each(b0, [&](float s) { return l += __builtin_amdgcn_exp2f(fmaf(s, p.sl, -base * p.sl)), s; });
+      m = tm;
+      if (b0 + STEP >= nblk) break;
+    }
+    // the lane halves and the waves of a row
+    float M = fmaxf(m, __shfl_xor(m, 32, 64));
+    if (h == 0) red[0][wave][r] = M;
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < kWaves; ++v) M = fmaxf(M, red[0][v][r]);
+    l *= __builtin_amdgcn_exp2f((m - M) * p.sl);
+    l += __shfl_xor(l, 32, 64);
+    if (h == 0) red[1][wave][r] = l;
+    __syncthreads();
+    l = 0.f;
+#pragma unroll
+    for (int v = 0; v < kWaves; ++v) l += red[1][v][r];
+    const float nm = -M * p.sl - __builtin_amdgcn_logf(l);  // v_log_f32 is log2
+    for (;;) {
+      each(b0, [&](float s) { return __builtin_amdgcn_exp2f(fmaf(s, p.sl, nm)); });
+      store(b0);
+      if (b0 == 0) break;
+      b0 -= STEP;
+      scores(b0);
+    }
+  }
+
+  const int zend = (p.fill || !p.causal) ? p.pitch : min(p.pitch, (m0 / 256 + 1) * 256 + p.off);
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  // zeros behind the last block, as far as the products read P or to the end of the row; rows behind the last query
+  const int z0 = row < p.L1 ? nblk * 32 : 0, z1 = row < p.L1 ? zend : row < p.zrows ? p.pitch : 0;
+  for (int c8 = z0 + (wave * 2 + h) * 8; c8 < z1; c8 += 2 * kWaves * 8) *reinterpret_cast<u32x4*>(wrow + c8) = zero;
+}
+
+template <int DT, int H1>
+int launch_probs_short(ProbsParams p, hipStream_t s) {
+  p.MT = (p.L1 + 31) / 32;
+  const dim3 grid(static_cast<unsigned>(p.Z * p.MT));
+  if (p.L2 <= 4 * 32 * kWaves) attn_probs_short_kernel<DT, H1, 4, false><<<grid, 64 * kWaves, 0, s>>>(p);
+  else if (p.L2 <= 8 * 32 * kWaves) attn_probs_short_kernel<DT, H1, 8, false><<<grid, 64 * kWaves, 0, s>>>(p);
+  else attn_probs_short_kernel<DT, H1, 8, true><<<grid, 64 * kWaves, 0, s>>>(p);
+  MEGA_CHECK_LAUNCH();
+  return MEGA_OK;
+}
+
 template <int DT, int H1>
 int launch_probs(const ProbsParams& p, hipStream_t s) {
+  // Few row blocks, both kernels in us (us of this one / of the short-row kernel, head width 256): 1024 keys, 64 row
+  // blocks of 32 55 / 24, 512 56 / 37, 768 60 / 57, 1024 58 / 72; 2048 keys, 128 row blocks 99 / 41, 512 101 / 53, 768 103 / 83,
+  // 1024 104 / 106; 4096 keys, 128 185 / 98, 512 187 / 114, 1024 201 / 235.  Head width 64, 1500 keys, 752: 60 / 29.
+  int dev = 0, cus = 0;
+  MEGA_CHECK_HIP(hipGetDevice(&dev));
+  MEGA_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  if (static_cast<int64_t>(p.Z) * ((p.L1 + 31) / 32) <= 3 * cus) return launch_probs_short<DT, H1>(p, s);
   constexpr int KW = H1 >= 128 ? 128 : 64;
   const size_t lds = sizeof(uint16_t) * kRing * kKeys * KW;
   MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_probs_kernel<DT, H1>),
