@@ -120,6 +120,16 @@ struct GemmParams {
   int kvb;      // rows of k that a k-major B holds when K has been rounded up behind them (0: all K); A holds
                 // zeros there, and zeros stand in for those rows of B (0 times an infinity would be NaN)
   int ms;       // rows of C to store when M has been rounded up (0: all M)
+  // Linear layers (LIN): C = A B^T + bias + add, with up to three problems in one launch.  Side by side along n (two
+  // k-contiguous operands: layers of one input) they differ in B, C, ldc, bias and N; along m (two k-major operands: their
+  // weight gradients) in A, lda, C and M.  Tiles mt (nt) >= start[i] belong to problem i + 1.
+  const uint16_t* bias;    // N values or null
+  const uint16_t* add;     // summand of C's layout or null
+  const uint16_t* op[2];
+  uint16_t* out[2];
+  const uint16_t* bias_of[2];
+  int size[2], start[2];
+  int kva;      // as kvb, for a k-major A (LIN: rows behind it are not there; else they hold zeros)
   int n_group;  // plain schedule: tiles numbered n fastest inside bands of n_group column tiles, then m,
                 // then band (0: one band) -- the 32 tiles an XCD works on at a time then share fewer
                 // distinct operand blocks (4 x 8 instead of 2 x 16 of a 16-column problem)
@@ -414,6 +424,110 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(const GemmParams p) {
   }  // work item
 }
 
+// Four values of a 16-bit row as floats.
+template <int DT>
+__device__ __forceinline__ void load4(const uint16_t* q, float* v) {
+  const uint2 u = *reinterpret_cast<const uint2*>(q);
+  const uint32_t w[2] = {u.x, u.y};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint16_t b = static_cast<uint16_t>(w[e >> 1] >> (16 * (e & 1)));
+    v[e] = DT == MEGA_BF16 ? bf16_bits_to_float(b) : f16_bits_to_float(b);
+  }
+}
+
+// What a tile's item of work is in the end: its operands and its place.
+struct Tile {
+  const uint16_t *A, *B, *bias;
+  uint16_t* C;
+  int M, N, mt, nt;
+  int64_t lda, ldc;
+};
+// LIN: the problem that tile (mt, nt) of the launch belongs to, and its place there
+template <bool LIN, bool TA, bool TB>
+__device__ __forceinline__ Tile tile_of(const GemmParams& p, int z0, int z1, int mt, int nt) {
+  Tile t{p.A + z0 * p.sa0 + z1 * p.sa1, p.B + z0 * p.sb0 + z1 * p.sb1, nullptr, p.C + z0 * p.sc0 + z1 * p.sc1, p.M, p.N, mt, nt, p.lda, p.ldc};
+  if constexpr (LIN) {
+    t.bias = p.bias;
+    const int at = TA ? mt : nt;
+    const int i = at >= p.start[1] ? 2 : at >= p.start[0] ? 1 : 0;
+    if (i > 0) {
+      const uint16_t* op = i == 2 ? p.op[1] : p.op[0];
+      const int size = i == 2 ? p.size[1] : p.size[0], start = i == 2 ? p.start[1] : p.start[0];
+      t.C = i == 2 ? p.out[1] : p.out[0];
+      t.bias = i == 2 ? p.bias_of[1] : p.bias_of[0];
+      if constexpr (TA) t.A = op, t.lda = size, t.M = size, t.mt = mt - start;
+      else t.B = op, t.ldc = size, t.N = size, t.nt = nt - start;
+    }
+  }
+  return t;
+}
+
+// Epilogue of a wave: its 32 IT x 64 accumulators at row0, col0 of C through its own LDS region `stage` ([row][EP]) into
+// 16-byte row segments.  The products are issued as B-fragment x A-fragment, so a 32x32 MFMA tile holds C transposed:
+// lane l has row m = l % 32 and register r the column n = 8 (r / 4) + 4 (l / 32) + r % 4.
+template <int DT, int IT, bool LIN>
+__device__ __forceinline__ void store_tile(const floatx16 (&acc)[IT][2], const GemmParams& p, const Tile& t, int rows, int row0, int col0,
+                                           int lane, uint16_t* stage) {
+  constexpr int JN = 2, EP = 64 + 8;
+#pragma unroll
+  for (int i = 0; i < IT; ++i) {
+#pragma unroll
+    for (int j = 0; j < JN; ++j) {
+      const int row = i * 32 + (lane & 31);
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        const int col = j * 32 + 8 * q4 + 4 * (lane >> 5);
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = p.alpha * acc[i][j][4 * q4 + e];
+        if constexpr (LIN) {  // (N % 8 == 0: four columns are all inside or all outside)
+          float a[4];
+          if (t.bias != nullptr && col0 + col < t.N) {
+            load4<DT>(t.bias + col0 + col, a);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += a[e];
+          }
+          if (p.add != nullptr && row0 + row < rows && col0 + col < t.N) {
+            load4<DT>(p.add + static_cast<int64_t>(row0 + row) * t.ldc + col0 + col, a);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += a[e];
+          }
+        }
+        uint2 w;
+        if (DT == MEGA_BF16) {
+          w.x = pack_bf16x2(v[0], v[1]);
+          w.y = pack_bf16x2(v[2], v[3]);
+        } else {
+          w.x = static_cast<uint32_t>(float_to_f16_bits(v[0])) | (static_cast<uint32_t>(float_to_f16_bits(v[1])) << 16);
+          w.y = static_cast<uint32_t>(float_to_f16_bits(v[2])) | (static_cast<uint32_t>(float_to_f16_bits(v[3])) << 16);
+        }
+        *reinterpret_cast<uint2*>(stage + row * EP + col) = w;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave reads back only its own region
+  const bool vec_ok = (t.ldc % 8 == 0) && (reinterpret_cast<uintptr_t>(t.C) % 16 == 0);
+#pragma unroll 4
+  for (int i = 0; i < 4 * IT; ++i) {
+    const int c = lane + kWave * i;
+    const int row = c / (4 * JN), kc = (c % (4 * JN)) * 8;
+    const int grow = row0 + row, gcol = col0 + kc;
+    if (grow < rows && gcol < t.N) {
+      const u32x4 v = *reinterpret_cast<const u32x4*>(stage + row * EP + kc);
+      uint16_t* dst = t.C + static_cast<int64_t>(grow) * t.ldc + gcol;
+      if (vec_ok && gcol + 8 <= t.N) {
+        __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dst));  // whole lines, read by a later kernel
+      } else {
+        const uint16_t* e = reinterpret_cast<const uint16_t*>(&v);
+        for (int q = 0; q < 8; ++q)
+          if (gcol + q < t.N) dst[q] = e[q];
+      }
+    }
+  }
+}
+
 // ---- the same product with the operand slabs sent from memory straight into LDS ------
 // Eight waves of 128 x 64 as above, aligned operands only.  `global_load_lds_dwordx4`
 // writes the 64 lanes' 16-byte pieces to 1 KB of consecutive LDS (base in M0), so no slab
@@ -459,10 +573,10 @@ __device__ __forceinline__ void load_to_lds16(u32x4 buffer, uint32_t offset, uin
 //
 // T: the workgroup's tile, 256 (2 x 4 waves of 128 x 64) or 128 (2 x 2 waves of 64 x 64, two workgroups per CU).
 // RAG: p.kvb and p.ms are set (B k-major)
-template <int DT, bool TA, bool TB, bool RAG = false, int T = kTile>
+template <int DT, bool TA, bool TB, bool RAG = false, int T = kTile, bool LIN = false>
 __global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
   extern __shared__ __align__(16) uint16_t smem[];
-  constexpr int JN = 2, NL = 2, EP = 64 + 8;
+  constexpr int JN = 2, NL = 2;
   constexpr int IT = T / 64;                 // 32-row blocks of a wave
   constexpr int NW = T / 32;                 // waves
   constexpr int kOperand = T * kSlab;        // elements of an operand slab
@@ -533,13 +647,12 @@ __global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
     }
   }
   const int z0 = zz / p.nh, z1 = zz % p.nh;
-  const uint16_t* A = p.A + z0 * p.sa0 + z1 * p.sa1;
-  const uint16_t* B = p.B + z0 * p.sb0 + z1 * p.sb1;
-  uint16_t* C = p.C + z0 * p.sc0 + z1 * p.sc1;
   for (int half = 0; half < 2; ++half) {
-  const int mt = half == 0 ? mt_first : mt_second;
-  if (mt < 0) break;
-  const int m0 = mt * T, n0 = nt * T;
+  if (half == 1 && mt_second < 0) break;
+  const Tile t = tile_of<LIN, TA, TB>(p, z0, z1, half == 0 ? mt_first : mt_second, nt);
+  const int mt = t.mt;
+  const uint16_t *A = t.A, *B = t.B;
+  const int m0 = mt * T, n0 = t.nt * T;
   int kb = 0, ke = p.K;
   if (p.k_mode == 1) ke = min(p.K, ((mt + 1) * T + p.off + kSlab - 1) / kSlab * kSlab);
   if (p.k_mode == 2) kb = min(p.K, max(0, mt * T - p.off) / kSlab * kSlab);
@@ -562,17 +675,18 @@ __global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
     const int pc = wave + NW * i;
     const int krow = KR * pc + lane / CR, cm = (lane % CR) ^ ((krow & 3) << 2);  // k-major piece
     const int row = 16 * pc + (lane >> 2), ck = (lane & 3) ^ ((lane >> 4) & 3);   // k-contiguous piece
-    if (TA) offa[i] = static_cast<uint32_t>(((kb + krow) * p.lda + min(m0 + cm * 8, p.M - 8)) * 2);
-    else offa[i] = static_cast<uint32_t>((static_cast<int64_t>(min(m0 + row, p.M - 1)) * p.lda + kb + ck * 8) * 2);
-    if (TB) offb[i] = static_cast<uint32_t>(((kb + krow) * p.ldb + min(n0 + cm * 8, p.N - 8)) * 2);
-    else offb[i] = static_cast<uint32_t>((static_cast<int64_t>(min(n0 + row, p.N - 1)) * p.ldb + kb + ck * 8) * 2);
+    if (TA) offa[i] = static_cast<uint32_t>(((kb + krow) * t.lda + min(m0 + cm * 8, t.M - 8)) * 2);
+    else offa[i] = static_cast<uint32_t>((static_cast<int64_t>(min(m0 + row, t.M - 1)) * t.lda + kb + ck * 8) * 2);
+    if (TB) offb[i] = static_cast<uint32_t>(((kb + krow) * p.ldb + min(n0 + cm * 8, t.N - 8)) * 2);
+    else offb[i] = static_cast<uint32_t>((static_cast<int64_t>(min(n0 + row, t.N - 1)) * p.ldb + kb + ck * 8) * 2);
   }
-  const uint32_t stepa = static_cast<uint32_t>((TA ? p.lda : 1) * kSlab * 2);
+  const uint32_t stepa = static_cast<uint32_t>((TA ? t.lda : 1) * kSlab * 2);
   const uint32_t stepb = static_cast<uint32_t>((TB ? p.ldb : 1) * kSlab * 2);
   const uint32_t lds_wave = __builtin_amdgcn_readfirstlane(
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint16_t*)(smem))) + wave * 1024);
   // RAG: B ends with row kvb - 1
-  const u32x4 bufb = RAG ? buffer_of(B, static_cast<uint32_t>(((p.kvb - 1) * p.ldb + p.N) * 2)) : u32x4{};
+  const u32x4 bufb = RAG ? buffer_of(B, static_cast<uint32_t>(((p.kvb - 1) * p.ldb + t.N) * 2)) : u32x4{};
+  const u32x4 bufa = RAG && LIN && TA ? buffer_of(A, static_cast<uint32_t>(((p.kva - 1) * t.lda + t.M) * 2)) : u32x4{};
   // request number n of a slab: n = 0, 2 the two pieces of A, n = 1, 3 those of B
   auto request_one = [&](int s, int stage, int n) {
     const uint32_t sc = static_cast<uint32_t>(min(s, nslab - 1));
@@ -582,7 +696,8 @@ __global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
       if constexpr (RAG) load_to_lds16(bufb, offb[n >> 1] + sc * stepb, dst);
       else load_to_lds16(B, offb[n >> 1] + sc * stepb, dst);
     } else {
-      load_to_lds16(A, offa[n >> 1] + sc * stepa, dst);
+      if constexpr (RAG && LIN && TA) load_to_lds16(bufa, offa[n >> 1] + sc * stepa, dst);
+      else load_to_lds16(A, offa[n >> 1] + sc * stepa, dst);
     }
   };
   auto request = [&](int s, int stage) {
@@ -590,19 +705,22 @@ __global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
     for (int n = 0; n < 2 * NL; ++n) request_one(s, stage, n);
   };
 
-  // fragment side: k-step `set` of a slab takes k = 16 g + 8 set + e for lane half g
+  // fragment side: k-step `set` of a slab takes k = 16 g + 8 set + e for lane half g, with two k-contiguous operands
+  // k = 16 set + 8 g + e (the products of gemm_dma64_kernel in the same order: the same bits)
+  constexpr bool KC = !TA && !TB;
+  constexpr int kSetFlip = KC ? 16 : 8;
   const int g = lane >> 5, r = lane & 31;
   const int ta_a = (lane & 15) >> 2, ta_h = (lane >> 4) & 1, ta_b = lane & 3;
   int fra[IT], frb[JN];
 #pragma unroll
   for (int i = 0; i < IT; ++i) {
     if (TA) fra[i] = (16 * g + ta_a) * T + (((wm * 4 * IT + 4 * i + 2 * ta_h + (ta_b >> 1)) ^ (ta_a << 2)) * 8) + 4 * (ta_b & 1);
-    else fra[i] = (wm * 32 * IT + 32 * i + r) * kSlab + (((2 * g) ^ ((r >> 2) & 3)) * 8);
+    else fra[i] = (wm * 32 * IT + 32 * i + r) * kSlab + (((KC ? g : 2 * g) ^ ((r >> 2) & 3)) * 8);
   }
 #pragma unroll
   for (int j = 0; j < JN; ++j) {
     if (TB) frb[j] = kOperand + (16 * g + ta_a) * T + (((wn * 8 + 4 * j + 2 * ta_h + (ta_b >> 1)) ^ (ta_a << 2)) * 8) + 4 * (ta_b & 1);
-    else frb[j] = kOperand + (wn * 64 + 32 * j + r) * kSlab + (((2 * g) ^ ((r >> 2) & 3)) * 8);
+    else frb[j] = kOperand + (wn * 64 + 32 * j + r) * kSlab + (((KC ? g : 2 * g) ^ ((r >> 2) & 3)) * 8);
   }
   u32x4 fa0[IT], fb0[JN], fa1[IT], fb1[JN];
   auto fread = [&](u32x4* fa, u32x4* fb, int set, int stage) {
@@ -615,7 +733,7 @@ __global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
         fa[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
       } else {
         // chunk 2 g + set sits at position (2 g + set) ^ swizzle = ((2 g) ^ swizzle) ^ set
-        fa[i] = *reinterpret_cast<const u32x4*>(base + (fra[i] ^ (set * 8)));
+        fa[i] = *reinterpret_cast<const u32x4*>(base + (fra[i] ^ (set * kSetFlip)));
       }
       if (i < JN) {
         if (TB) {
@@ -623,7 +741,7 @@ __global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
           const uint2 lo = lds_read_tr(q), hi = lds_read_tr(q + 4 * T);
           fb[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
         } else {
-          fb[i] = *reinterpret_cast<const u32x4*>(base + (frb[i] ^ (set * 8)));
+          fb[i] = *reinterpret_cast<const u32x4*>(base + (frb[i] ^ (set * kSetFlip)));
         }
       }
     }
@@ -691,50 +809,7 @@ __global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
 #undef MEGA_DMA_STEP
 #undef MEGA_SGB
 
-  // epilogue as in gemm_kernel: the wave's tile through its own LDS region
-  uint16_t* stage = smem + wave * 32 * IT * EP;
-#pragma unroll
-  for (int i = 0; i < IT; ++i) {
-#pragma unroll
-    for (int j = 0; j < JN; ++j) {
-      const int row = i * 32 + (lane & 31);
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const int col = j * 32 + 8 * q4 + 4 * (lane >> 5);
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = p.alpha * acc[i][j][4 * q4 + e];
-        uint2 w;
-        if (DT == MEGA_BF16) {
-          w.x = pack_bf16x2(v[0], v[1]);
-          w.y = pack_bf16x2(v[2], v[3]);
-        } else {
-          w.x = static_cast<uint32_t>(float_to_f16_bits(v[0])) | (static_cast<uint32_t>(float_to_f16_bits(v[1])) << 16);
-          w.y = static_cast<uint32_t>(float_to_f16_bits(v[2])) | (static_cast<uint32_t>(float_to_f16_bits(v[3])) << 16);
-        }
-        *reinterpret_cast<uint2*>(stage + row * EP + col) = w;
-      }
-    }
-  }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave reads back only its own region
-  const bool vec_ok = (p.ldc % 8 == 0) && (reinterpret_cast<uintptr_t>(C) % 16 == 0);
-#pragma unroll 4
-  for (int i = 0; i < 2 * IT * JN; ++i) {
-    const int c = lane + kWave * i;
-    const int row = c / (4 * JN), kc = (c % (4 * JN)) * 8;
-    const int grow = m0 + wm * 32 * IT + row, gcol = n0 + wn * (32 * JN) + kc;
-    if (grow < (RAG ? p.ms : p.M) && gcol < p.N) {
-      const u32x4 v = *reinterpret_cast<const u32x4*>(stage + row * EP + kc);
-      uint16_t* dst = C + static_cast<int64_t>(grow) * p.ldc + gcol;
-      if (vec_ok && gcol + 8 <= p.N) {
-        __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dst));  // whole lines, read by a later kernel
-      } else {
-        const uint16_t* e = reinterpret_cast<const uint16_t*>(&v);
-        for (int q = 0; q < 8; ++q)
-          if (gcol + q < p.N) dst[q] = e[q];
-      }
-    }
-  }
+  store_tile<DT, IT, LIN>(acc, p, t, RAG && !LIN ? p.ms : t.M, m0 + wm * 32 * IT, n0 + wn * 64, lane, smem + wave * 32 * IT * (64 + 8));
   // the output regions overlap the slab buffers: every read of this tile's epilogue
   // retires before the next tile's first slab is requested
   lds_barrier();
@@ -759,10 +834,10 @@ constexpr int kDma64Operand = kTile * kSlab64;  // elements of an operand slab (
 constexpr int kDma64Stage = 2 * kDma64Operand;
 static_assert(sizeof(uint16_t) * 2 * kDma64Stage <= kDmaLds, "two slab buffers fit");
 
-template <int DT, bool TA, bool TB, int T = kTile>
+template <int DT, bool TA, bool TB, int T = kTile, bool LIN = false>
 __global__ __launch_bounds__(2 * T) void gemm_dma64_kernel(const GemmParams p) {
   extern __shared__ __align__(16) uint16_t smem[];
-  constexpr int JN = 2, NL = 4, EP = 64 + 8;
+  constexpr int JN = 2, NL = 4;
   constexpr int IT = T / 64, NW = T / 32, kOperand = T * kSlab64, kStage = 2 * kOperand;  // as in gemm_dma_kernel
   static_assert(T == kTile || (!TA && !TB), "pieces of k rows are written for 256 columns");
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
@@ -798,18 +873,22 @@ __global__ __launch_bounds__(2 * T) void gemm_dma64_kernel(const GemmParams p) {
     const int pr = rem / p.nt_count;
     mt_first = p.mt_count - 1 - pr;
     if (T == kTile && mt_first != pr) mt_second = pr;
+  } else if (p.n_group > 0) {  // as in gemm_dma_kernel
+    const int band = p.n_group * p.mt_count, b0 = rem / band, r2 = rem % band;
+    const int w = min(p.n_group, p.nt_count - b0 * p.n_group);
+    nt = b0 * p.n_group + r2 % w;
+    mt_first = r2 / w;
   } else {
     nt = rem % p.nt_count;
     mt_first = rem / p.nt_count;
   }
   const int z0 = zz / p.nh, z1 = zz % p.nh;
-  const uint16_t* A = p.A + z0 * p.sa0 + z1 * p.sa1;
-  const uint16_t* B = p.B + z0 * p.sb0 + z1 * p.sb1;
-  uint16_t* C = p.C + z0 * p.sc0 + z1 * p.sc1;
   for (int half = 0; half < 2; ++half) {
-  const int mt = half == 0 ? mt_first : mt_second;
-  if (mt < 0) break;
-  const int m0 = mt * T, n0 = nt * T;
+  if (half == 1 && mt_second < 0) break;
+  const Tile t = tile_of<LIN, TA, TB>(p, z0, z1, half == 0 ? mt_first : mt_second, nt);
+  const int mt = t.mt;
+  const uint16_t *A = t.A, *B = t.B;
+  const int m0 = mt * T, n0 = t.nt * T;
   // k range as in gemm_kernel, widened to whole slabs of 64 (K % 64 == 0): what the wider range
   // adds are probabilities the softmax has written as zeros
   int kb = 0, ke = p.K;
@@ -832,12 +911,12 @@ __global__ __launch_bounds__(2 * T) void gemm_dma64_kernel(const GemmParams p) {
     const int pc = wave + NW * i;
     const int krow = 2 * pc + (lane >> 5), cm = (lane & 31) ^ ((krow & 3) << 2);   // k-major piece: 2 rows of k
     const int row = 8 * pc + (lane >> 3), ck = (lane & 7) ^ ((row >> 1) & 7);      // k-contiguous piece: 8 rows
-    if (TA) offa[i] = static_cast<uint32_t>(((kb + krow) * p.lda + min(m0 + cm * 8, p.M - 8)) * 2);
-    else offa[i] = static_cast<uint32_t>((static_cast<int64_t>(min(m0 + row, p.M - 1)) * p.lda + kb + ck * 8) * 2);
-    if (TB) offb[i] = static_cast<uint32_t>(((kb + krow) * p.ldb + min(n0 + cm * 8, p.N - 8)) * 2);
-    else offb[i] = static_cast<uint32_t>((static_cast<int64_t>(min(n0 + row, p.N - 1)) * p.ldb + kb + ck * 8) * 2);
+    if (TA) offa[i] = static_cast<uint32_t>(((kb + krow) * t.lda + min(m0 + cm * 8, t.M - 8)) * 2);
+    else offa[i] = static_cast<uint32_t>((static_cast<int64_t>(min(m0 + row, t.M - 1)) * t.lda + kb + ck * 8) * 2);
+    if (TB) offb[i] = static_cast<uint32_t>(((kb + krow) * p.ldb + min(n0 + cm * 8, t.N - 8)) * 2);
+    else offb[i] = static_cast<uint32_t>((static_cast<int64_t>(min(n0 + row, t.N - 1)) * p.ldb + kb + ck * 8) * 2);
   }
-  const uint32_t stepa = static_cast<uint32_t>((TA ? p.lda : 1) * kSlab64 * 2);
+  const uint32_t stepa = static_cast<uint32_t>((TA ? t.lda : 1) * kSlab64 * 2);
   const uint32_t stepb = static_cast<uint32_t>((TB ? p.ldb : 1) * kSlab64 * 2);
   const uint32_t lds_wave = __builtin_amdgcn_readfirstlane(
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint16_t*)(smem))) + wave * 1024);
@@ -949,50 +1028,7 @@ __global__ __launch_bounds__(2 * T) void gemm_dma64_kernel(const GemmParams p) {
 #undef MEGA_DMA64_KSTEP
 #undef MEGA_SGB
 
-  // epilogue as in gemm_kernel: the wave's tile through its own LDS region
-  uint16_t* stage = smem + wave * 32 * IT * EP;
-#pragma unroll
-  for (int i = 0; i < IT; ++i) {
-#pragma unroll
-    for (int j = 0; j < JN; ++j) {
-      const int row = i * 32 + (lane & 31);
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const int col = j * 32 + 8 * q4 + 4 * (lane >> 5);
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = p.alpha * acc[i][j][4 * q4 + e];
-        uint2 w;
-        if (DT == MEGA_BF16) {
-          w.x = pack_bf16x2(v[0], v[1]);
-          w.y = pack_bf16x2(v[2], v[3]);
-        } else {
-          w.x = static_cast<uint32_t>(float_to_f16_bits(v[0])) | (static_cast<uint32_t>(float_to_f16_bits(v[1])) << 16);
-          w.y = static_cast<uint32_t>(float_to_f16_bits(v[2])) | (static_cast<uint32_t>(float_to_f16_bits(v[3])) << 16);
-        }
-        *reinterpret_cast<uint2*>(stage + row * EP + col) = w;
-      }
-    }
-  }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  const bool vec_ok = (p.ldc % 8 == 0) && (reinterpret_cast<uintptr_t>(C) % 16 == 0);
-#pragma unroll 4
-  for (int i = 0; i < 2 * IT * JN; ++i) {
-    const int c = lane + kWave * i;
-    const int row = c / (4 * JN), kc = (c % (4 * JN)) * 8;
-    const int grow = m0 + wm * 32 * IT + row, gcol = n0 + wn * (32 * JN) + kc;
-    if (grow < p.M && gcol < p.N) {
-      const u32x4 v = *reinterpret_cast<const u32x4*>(stage + row * EP + kc);
-      uint16_t* dst = C + static_cast<int64_t>(grow) * p.ldc + gcol;
-      if (vec_ok && gcol + 8 <= p.N) {
-        __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dst));  // whole lines, read by a later kernel
-      } else {
-        const uint16_t* e = reinterpret_cast<const uint16_t*>(&v);
-        for (int q = 0; q < 8; ++q)
-          if (gcol + q < p.N) dst[q] = e[q];
-      }
-    }
-  }
+  store_tile<DT, IT, LIN>(acc, p, t, t.M, m0 + wm * 32 * IT, n0 + wn * 64, lane, smem + wave * 32 * IT * (64 + 8));
   lds_barrier();
   }  // tile of the pair
   }  // work item
@@ -1012,10 +1048,10 @@ constexpr size_t kA64Lds = sizeof(uint16_t) * (kA64BBase + kStages * kDmaOperand
 static_assert(kA64Lds <= 160 * 1024 && sizeof(uint16_t) * 8 * 128 * (64 + 8) <= kA64Lds, "fits the LDS, holds the output tiles");
 
 // RAG: p.kvb is set
-template <int DT, bool RAG = false>
+template <int DT, bool RAG = false, bool LIN = false>
 __global__ __launch_bounds__(2 * kThreads) void gemm_dma_a64_kernel(const GemmParams p) {
   extern __shared__ __align__(16) uint16_t smem[];
-  constexpr int JN = 2, EP = 64 + 8;
+  constexpr int JN = 2;
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   const int wm = wave >> 2, wn = wave & 3;
   // work items as in gemm_kernel
@@ -1063,13 +1099,12 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_a64_kernel(const GemmPa
     }
   }
   const int z0 = zz / p.nh, z1 = zz % p.nh;
-  const uint16_t* A = p.A + z0 * p.sa0 + z1 * p.sa1;
-  const uint16_t* B = p.B + z0 * p.sb0 + z1 * p.sb1;
-  uint16_t* C = p.C + z0 * p.sc0 + z1 * p.sc1;
   for (int half = 0; half < 2; ++half) {
-  const int mt = half == 0 ? mt_first : mt_second;
-  if (mt < 0) break;
-  const int m0 = mt * kTile, n0 = nt * kTile;
+  if (half == 1 && mt_second < 0) break;
+  const Tile t = tile_of<LIN, false, true>(p, z0, z1, half == 0 ? mt_first : mt_second, nt);
+  const int mt = t.mt;
+  const uint16_t *A = t.A, *B = t.B;
+  const int m0 = mt * kTile, n0 = t.nt * kTile;
   // k range as in gemm_kernel, widened to whole slabs of 64 (K % 64 == 0): what the wider range
   // adds are probabilities the softmax has written as zeros
   int kb = 0, ke = p.K;
@@ -1094,20 +1129,20 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_a64_kernel(const GemmPa
   for (int i = 0; i < 4; ++i) {
     const int pc = wave + 8 * i;
     const int row = 8 * pc + (lane >> 3), ck = (lane & 7) ^ ((row >> 1) & 7);
-    offa[i] = static_cast<uint32_t>((static_cast<int64_t>(min(m0 + row, p.M - 1)) * p.lda + kb + ck * 8) * 2);
+    offa[i] = static_cast<uint32_t>((static_cast<int64_t>(min(m0 + row, t.M - 1)) * t.lda + kb + ck * 8) * 2);
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int pc = wave + 8 * i;
     const int krow = 2 * pc + (lane >> 5), cm = (lane & 31) ^ ((krow & 3) << 2);
-    offb[i] = static_cast<uint32_t>(((kb + krow) * p.ldb + min(n0 + cm * 8, p.N - 8)) * 2);
+    offb[i] = static_cast<uint32_t>(((kb + krow) * p.ldb + min(n0 + cm * 8, t.N - 8)) * 2);
   }
   const uint32_t stepa = static_cast<uint32_t>(kSlab64 * 2);
   const uint32_t stepb = static_cast<uint32_t>(p.ldb * kSlab * 2);
   const uint32_t lds_wave = __builtin_amdgcn_readfirstlane(
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint16_t*)(smem))) + wave * 1024);
   // RAG: B ends with row kvb - 1
-  const u32x4 bufb = RAG ? buffer_of(B, static_cast<uint32_t>(((p.kvb - 1) * p.ldb + p.N) * 2)) : u32x4{};
+  const u32x4 bufb = RAG ? buffer_of(B, static_cast<uint32_t>(((p.kvb - 1) * p.ldb + t.N) * 2)) : u32x4{};
   // A slab ja into A buffer ab (4 requests), B slab s into B buffer bb (2 requests); slabs past the
   // end ask for the last one again, so that every step issues the same number of requests
   auto request_a = [&](int ja, int ab, int n) {
@@ -1223,50 +1258,7 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_a64_kernel(const GemmPa
 #undef MEGA_A64_STEP
 #undef MEGA_SGB
 
-  // epilogue as in gemm_kernel: the wave's 128 x 64 tile through its own LDS region
-  uint16_t* stage = smem + wave * 128 * EP;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-#pragma unroll
-    for (int j = 0; j < JN; ++j) {
-      const int row = i * 32 + (lane & 31);
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const int col = j * 32 + 8 * q4 + 4 * (lane >> 5);
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = p.alpha * acc[i][j][4 * q4 + e];
-        uint2 w;
-        if (DT == MEGA_BF16) {
-          w.x = pack_bf16x2(v[0], v[1]);
-          w.y = pack_bf16x2(v[2], v[3]);
-        } else {
-          w.x = static_cast<uint32_t>(float_to_f16_bits(v[0])) | (static_cast<uint32_t>(float_to_f16_bits(v[1])) << 16);
-          w.y = static_cast<uint32_t>(float_to_f16_bits(v[2])) | (static_cast<uint32_t>(float_to_f16_bits(v[3])) << 16);
-        }
-        *reinterpret_cast<uint2*>(stage + row * EP + col) = w;
-      }
-    }
-  }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave reads back only its own region
-  const bool vec_ok = (p.ldc % 8 == 0) && (reinterpret_cast<uintptr_t>(C) % 16 == 0);
-#pragma unroll 4
-  for (int i = 0; i < 8 * JN; ++i) {
-    const int c = lane + kWave * i;
-    const int row = c / (4 * JN), kc = (c % (4 * JN)) * 8;
-    const int grow = m0 + wm * 128 + row, gcol = n0 + wn * (32 * JN) + kc;
-    if (grow < p.M && gcol < p.N) {
-      const u32x4 v = *reinterpret_cast<const u32x4*>(stage + row * EP + kc);
-      uint16_t* dst = C + static_cast<int64_t>(grow) * p.ldc + gcol;
-      if (vec_ok && gcol + 8 <= p.N) {
-        __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dst));  // whole lines, read by a later kernel
-      } else {
-        const uint16_t* e = reinterpret_cast<const uint16_t*>(&v);
-        for (int q = 0; q < 8; ++q)
-          if (gcol + q < p.N) dst[q] = e[q];
-      }
-    }
-  }
+  store_tile<DT, 4, LIN>(acc, p, t, t.M, m0 + wm * 32 * 4, n0 + wn * 64, lane, smem + wave * 32 * 4 * (64 + 8));
   // the output regions overlap the slab buffers: every read of this tile's epilogue
   // retires before the next tile's first slab is requested
   lds_barrier();
@@ -1591,11 +1583,8 @@ int launch_gemm_t(const GemmParams& p, int batch, hipStream_t s) {
       return launch_small<DT, TA, TB>(q, cus, s);
     }
   }
-  // one workgroup per CU (its LDS and registers fill one); a multiple of the
-  // XCD count whenever there are that many items
-  int64_t g = std::min<int64_t>(t.items, cus);
-  if (g >= kXcds) g -= g % kXcds;
-  const dim3 grid(static_cast<unsigned>(g));
+  // one workgroup per CU (its LDS and registers fill one), in whole rounds of the XCDs
+  const dim3 grid(static_cast<unsigned>(std::min<int64_t>((t.items + kXcds - 1) / kXcds, std::max(cus / kXcds, 1)) * kXcds));
   const size_t lds = kGemmLds;
   // Aligned operands: slabs from memory straight into LDS, eight waves of 128 x 64.  Products of
   // two k-contiguous operands (S = Q K^T, dP = dY V^T) take slabs of 64 k; one k-contiguous and
@@ -1892,6 +1881,231 @@ extern "C" int mega_attention_layer_bwd(const void* dy, const void* q, const voi
                                         void* workspace, void* stream) {
   return attention_bwd_entry(dy, q, k, v, saved, dtype, B, L1, L2, NH, H1, H2, scale, causal, dq, dk, dv, workspace,
                              stream, true);
+}
+
+// ---- linear layers on the same product kernels ---------------------------------------
+namespace mega {
+namespace {
+
+template <auto Kernel>
+int launch_tiles(const GemmParams& q, int grid, int threads, size_t lds, hipStream_t s) {
+  MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  Kernel<<<dim3(static_cast<unsigned>(grid)), threads, lds, s>>>(q);
+  MEGA_CHECK_LAUNCH();
+  return MEGA_OK;
+}
+
+enum { kForward, kInputGrad, kWeightGrad };
+
+// The tiles of the `count` problems of a launch (sizes along the axis they lie side by side on), in tiles of T.
+void lay_out(GemmParams& q, int kind, int count, const int64_t* sizes, int T) {
+  const auto tiles = [&](int64_t n) { return static_cast<int>((n + T - 1) / T); };
+  q.start[0] = q.start[1] = 0x7fffffff;
+  int along = tiles(sizes[0]);
+  for (int i = 1; i < count; ++i) {
+    q.start[i - 1] = along;
+    q.size[i - 1] = static_cast<int>(sizes[i]);
+    along += tiles(sizes[i]);
+  }
+  q.mt_count = kind == kWeightGrad ? along : tiles(q.M);
+  q.nt_count = kind == kForward ? along : tiles(q.N);
+  q.per_batch = q.items = q.mt_count * q.nt_count;
+}
+
+int compute_units(int* cus) {
+  int dev = 0;
+  MEGA_CHECK_HIP(hipGetDevice(&dev));
+  MEGA_CHECK_HIP(hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev));
+  return MEGA_OK;
+}
+
+// Time of a launch in us by what was measured (1000 to 32768 tokens, layers of 1024 to 11008).  A tile of 256 takes longer
+// for 32 k the more of the chip works (the clock falls: forward 0.45 us alone, 0.80 with every CU busy); tiles of 128 run
+// two to a CU, each pair as long as two one after the other; every round of tiles starts and ends in a few us.
+double estimate(const GemmParams& q, int kind, int T, int cus) {
+  const double slabs = (q.K + kSlab - 1) / kSlab, rounds = (q.items + cus - 1) / cus, load = q.items / (rounds * cus);
+  if (T == kTile) {
+    if (kind == kWeightGrad) return rounds * (slabs * (0.40 + 0.36 * load) + 1) + 2;
+    if (kind == kForward) return rounds * (slabs * (0.45 + 0.35 * load) + 5) + 3;
+    return rounds * (slabs * (0.42 + 0.37 * load) + 5) + 2;
+  }
+  if (kind == kWeightGrad) return rounds * slabs * 0.23 + 3;
+  if (kind == kForward) return rounds * (slabs * 0.255 + 1.3) + 3;
+  return rounds * (slabs * 0.27 + 1) + 3;
+}
+
+// Lays the tiles out in the size that is expected to be faster; its time.
+double plan(GemmParams& q, int kind, int count, const int64_t* sizes, int cus, bool* small) {
+  GemmParams l = q;
+  lay_out(l, kind, count, sizes, kTile);
+  lay_out(q, kind, count, sizes, kSmall);
+  const double tl = estimate(l, kind, kTile, cus), ts = estimate(q, kind, kSmall, cus);
+  *small = ts <= tl;
+  if (!*small) q = l;
+  return std::min(ts, tl);
+}
+
+// The part of a launch's problems that is problem i alone.
+GemmParams one_of(const GemmParams& q, int kind, int i, int64_t size) {
+  GemmParams o = q;
+  if (kind == kForward) {
+    if (i > 0) o.B = q.op[i - 1], o.C = q.out[i - 1], o.bias = q.bias_of[i - 1];
+    o.N = (int)size;
+    o.ldc = size;
+  } else {
+    if (i > 0) o.A = q.op[i - 1], o.C = q.out[i - 1];
+    o.M = (int)size;
+    o.lda = size;
+  }
+  return o;
+}
+// The time of `count` problems in one launch, or one launch after the other where that is shorter (*apart).
+double plan_group(const GemmParams& q, int kind, int count, const int64_t* sizes, int cus, bool* apart) {
+  GemmParams g = q;
+  bool small;
+  const double together = plan(g, kind, count, sizes, cus, &small);
+  *apart = false;
+  if (count == 1) return together;
+  double sum = 0;
+  for (int i = 0; i < count; ++i) {
+    GemmParams o = one_of(q, kind, i, sizes[i]);
+    sum += plan(o, kind, 1, sizes + i, cus, &small);
+  }
+  *apart = sum < 1.05 * together;  // (at equal rounds of tiles: 2 x 11008 x 4096, 32768 tokens, 4280 us apart, 4384 together)
+  return std::min(sum, together);
+}
+
+template <int DT>
+int launch_linear(GemmParams q, int kind, int count, const int64_t* sizes, hipStream_t s) {
+  q.nh = 1; q.alpha = 1.f; q.n_group = 8;
+  int cus = 0;
+  if (const int rc = compute_units(&cus); rc != MEGA_OK) return rc;
+  bool apart = false, small = false;
+  plan_group(q, kind, count, sizes, cus, &apart);
+  if (apart) {
+    for (int i = 0; i < count; ++i)
+      if (const int rc = launch_linear<DT>(one_of(q, kind, i, sizes[i]), kind, 1, sizes + i, s); rc != MEGA_OK) return rc;
+    return MEGA_OK;
+  }
+  plan(q, kind, count, sizes, cus, &small);
+  const size_t lds = small ? sizeof(uint16_t) * kStages * 2 * kSmall * kSlab : kDmaLds;
+  const int threads = small ? 2 * kSmall : 2 * kTile;
+  int grid = (q.items + kXcds - 1) / kXcds * kXcds;
+  if (!small) grid = std::min(grid, std::max(cus / kXcds, 1) * kXcds);
+  if (kind == kForward) {
+    if (!small) return launch_tiles<gemm_dma64_kernel<DT, false, false, kTile, true>>(q, grid, threads, lds, s);
+    if (q.items <= cus) return launch_tiles<gemm_dma_kernel<DT, false, false, false, kSmall, true>>(q, grid, threads, lds, s);
+    return launch_tiles<gemm_dma64_kernel<DT, false, false, kSmall, true>>(q, grid, threads, lds, s);
+  }
+  if (kind == kInputGrad) {
+    if (!small) return launch_tiles<gemm_dma_a64_kernel<DT, false, true>>(q, grid, threads, kA64Lds, s);
+    return launch_tiles<gemm_dma_kernel<DT, false, true, false, kSmall, true>>(q, grid, threads, lds, s);
+  }
+  const bool rag = q.K % kSlab != 0;
+  q.kva = q.kvb = q.K;
+  q.ms = q.M;
+  q.K = (q.K + kSlab - 1) / kSlab * kSlab;
+  if (rag) {
+    if (!small) return launch_tiles<gemm_dma_kernel<DT, true, true, true, kTile, true>>(q, grid, threads, lds, s);
+    return launch_tiles<gemm_dma_kernel<DT, true, true, true, kSmall, true>>(q, grid, threads, lds, s);
+  }
+  if (!small) return launch_tiles<gemm_dma_kernel<DT, true, true, false, kTile, true>>(q, grid, threads, lds, s);
+  return launch_tiles<gemm_dma_kernel<DT, true, true, false, kSmall, true>>(q, grid, threads, lds, s);
+}
+
+}  // namespace
+}  // namespace mega
+
+// (the contiguous reduction axis of forward and input gradient comes in slabs of 64)
+static int check_linear(const char* who, int kind, int dtype, int64_t tokens, int64_t n_in, int count, const int64_t* n_out) {
+  MEGA_CHECK_ARG(dtype == MEGA_BF16 || dtype == MEGA_F16, "%s: bfloat16 or float16 tensors", who);
+  MEGA_CHECK_ARG(count >= 1 && count <= 3 && n_out != nullptr, "%s: one to three layers", who);
+  const int64_t in = kind == kForward ? 64 : 8, out = kind == kInputGrad ? 64 : 8;
+  MEGA_CHECK_ARG(tokens >= 1 && n_in >= in && n_in % in == 0 && tokens < (1 << 30) / n_in, "%s: bad sizes", who);
+  for (int i = 0; i < count; ++i)
+    MEGA_CHECK_ARG(n_out[i] >= out && n_out[i] % out == 0 && tokens < (1 << 30) / n_out[i] && n_in < (1 << 30) / n_out[i], "%s: bad sizes", who);
+  return MEGA_OK;
+}
+static bool aligned16(const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; }
+
+// Whether the launch is expected to be faster than the library's products, one call a layer.
+extern "C" int mega_linear_takes(int kind, int dtype, int64_t tokens, int64_t n_in, int count, const int64_t* n_out) {
+  if (kind < kForward || kind > kWeightGrad || check_linear("mega_linear_takes", kind, dtype, tokens, n_in, count, n_out) != MEGA_OK) return 0;
+  int cus = 0;
+  if (compute_units(&cus) != MEGA_OK) return 0;
+  if (kind == kWeightGrad) {
+    // Both operands run across the reduction axis, the library's slowest layout: this kernel is ahead at every size (us,
+    // library / here): 4096 tokens, 256 + 2048 + 1024 x 1024 91 / 30, 2 x 2752 x 1024 85 / 58, 2 x 5504 x 2048 174 / 166, 11008 x 4096
+    // 380 / 281; 4084 tokens, 2048 x 5504 106 / 82; 1531, 4096 x 11008 174 / 122; 32768, 3328 x 1024 595 / 280, except a long
+    // reduction over few tiles, which the library cuts up.
+    int64_t tiles = 0;
+    for (int i = 0; i < count; ++i) tiles += (n_out[i] + kSmall - 1) / kSmall * ((n_in + kSmall - 1) / kSmall);
+    return tokens <= 4096 || 4 * tiles >= cus;
+  }
+  GemmParams q{};
+  bool apart;
+  q.M = (int)tokens; q.N = (int)(kind == kForward ? n_out[0] : n_in); q.K = (int)(kind == kForward ? n_in : n_out[0]);
+  const double here = plan_group(q, kind, kind == kForward ? count : 1, kind == kForward ? n_out : &n_in, cus, &apart);
+  // The library: at least 20 us a call (its host path), then what it reaches on products of so many terms, in PFLOP/s; widths
+  // off the multiples of 1024 cost it a quarter up to some 2^39.  Forward, us (library / here): 4096 tokens, 256 + 2048 + 1024 x
+  // 1024 60 / 33, 2 x 2752 x 1024 71 / 61, 2 x 5504 x 2048 181 / 165, 2 x 11008 x 4096 813 / 594, 4096 x 2048 51 / 61, 8192 x 4096
+  // 180 / 214; 1531 tokens, 2 x 11008 x 4096 262 / 283.  Input gradient: 2752 x 1024 32 / 24, 4096 x 2048 65 / 73.
+  double library = 0;
+  for (int i = 0; i < count; ++i) {
+    const double products = static_cast<double>(tokens) * n_in * n_out[i];
+    if (kind == kInputGrad && products > 0x1p35) return 0;  // goes through a transposed copy of W there
+    const double rate = kind == kInputGrad ? 1.1 : products > 0x1p39 ? 1.5 : products < 0x1p33 ? 1.0 : n_out[i] % 1024 == 0 ? 1.4 : 1.1;
+    library += std::max(20.0, 2e-9 * products / rate + (kind == kInputGrad ? 10 : 8));
+  }
+  return here <= library;
+}
+
+extern "C" int mega_linear_fwd(const void* x, const void* const* w, const void* const* bias, const void* add, int dtype,
+                               int64_t tokens, int64_t n_in, int count, const int64_t* n_out, void* const* y, void* stream) {
+  const int rc = check_linear("mega_linear_fwd", kForward, dtype, tokens, n_in, count, n_out);
+  if (rc != MEGA_OK) return rc;
+  MEGA_CHECK_ARG(w && y && aligned16(x) && x && aligned16(add) && (!add || count == 1), "mega_linear_fwd: null or misaligned pointer");
+  for (int i = 0; i < count; ++i)
+    MEGA_CHECK_ARG(w[i] && y[i] && aligned16(w[i]) && aligned16(y[i]) && (!bias || aligned16(bias[i])), "mega_linear_fwd: null or misaligned pointer");
+  const auto u = [](const void* q) { return static_cast<const uint16_t*>(q); };
+  GemmParams g{};
+  g.A = u(x); g.B = u(w[0]); g.C = static_cast<uint16_t*>(y[0]);
+  g.M = (int)tokens; g.N = (int)n_out[0]; g.K = (int)n_in;
+  g.lda = n_in; g.ldb = n_in; g.ldc = n_out[0];
+  g.bias = bias ? u(bias[0]) : nullptr; g.add = u(add);
+  for (int i = 1; i < count; ++i) g.op[i - 1] = u(w[i]), g.out[i - 1] = static_cast<uint16_t*>(y[i]), g.bias_of[i - 1] = bias ? u(bias[i]) : nullptr;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  return dtype == MEGA_BF16 ? launch_linear<MEGA_BF16>(g, kForward, count, n_out, s) : launch_linear<MEGA_F16>(g, kForward, count, n_out, s);
+}
+
+extern "C" int mega_linear_input_grad(const void* dy, const void* w, const void* add, int dtype, int64_t tokens, int64_t n_out,
+                                      int64_t n_in, void* dx, void* stream) {
+  const int rc = check_linear("mega_linear_input_grad", kInputGrad, dtype, tokens, n_in, 1, &n_out);
+  if (rc != MEGA_OK) return rc;
+  MEGA_CHECK_ARG(dy && w && dx && aligned16(dy) && aligned16(w) && aligned16(dx) && aligned16(add), "mega_linear_input_grad: null or misaligned pointer");
+  GemmParams g{};
+  g.A = static_cast<const uint16_t*>(dy); g.B = static_cast<const uint16_t*>(w); g.C = static_cast<uint16_t*>(dx);
+  g.M = (int)tokens; g.N = (int)n_in; g.K = (int)n_out;
+  g.lda = n_out; g.ldb = n_in; g.ldc = n_in; g.tb = 1;
+  g.add = static_cast<const uint16_t*>(add);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  return dtype == MEGA_BF16 ? launch_linear<MEGA_BF16>(g, kInputGrad, 1, &n_in, s) : launch_linear<MEGA_F16>(g, kInputGrad, 1, &n_in, s);
+}
+
+extern "C" int mega_linear_weight_grads(const void* const* dy, const void* x, int dtype, int64_t tokens, int64_t n_in, int count,
+                                        const int64_t* n_out, void* const* dw, void* stream) {
+  const int rc = check_linear("mega_linear_weight_grads", kWeightGrad, dtype, tokens, n_in, count, n_out);
+  if (rc != MEGA_OK) return rc;
+  MEGA_CHECK_ARG(dy && dw && x && aligned16(x), "mega_linear_weight_grads: null or misaligned pointer");
+  for (int i = 0; i < count; ++i) MEGA_CHECK_ARG(dy[i] && dw[i] && aligned16(dy[i]) && aligned16(dw[i]), "mega_linear_weight_grads: null or misaligned pointer");
+  const auto u = [](const void* q) { return static_cast<const uint16_t*>(q); };
+  GemmParams g{};
+  g.A = u(dy[0]); g.B = u(x); g.C = static_cast<uint16_t*>(dw[0]);
+  g.M = (int)n_out[0]; g.N = (int)n_in; g.K = (int)tokens;
+  g.lda = n_out[0]; g.ldb = n_in; g.ldc = n_in; g.ta = 1; g.tb = 1;
+  for (int i = 1; i < count; ++i) g.op[i - 1] = u(dy[i]), g.out[i - 1] = static_cast<uint16_t*>(dw[i]);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  return dtype == MEGA_BF16 ? launch_linear<MEGA_BF16>(g, kWeightGrad, count, n_out, s) : launch_linear<MEGA_F16>(g, kWeightGrad, count, n_out, s);
 }
 
 // ---- the weight gradient of a linear layer on the same product kernel ---------------

@@ -3,6 +3,7 @@
 // costs 10-15 us per direction, more than most of these kernels run for at ordinary sizes.
 #include "host.hpp"
 
+#include <ATen/autocast_mode.h>
 #include <torch/csrc/autograd/custom_function.h>
 
 #include <map>
@@ -462,24 +463,42 @@ Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, double scale
 }
 
 // ---- linear layers --------------------------------------------------------------------------------
-// dW = g^T x, (out, in) from (tokens, out) and (tokens, in).  Both operands run across
-// the reduction axis (tokens) here, the slowest layout of the library GEMM on MI355X
-// (0.9-1.2 PFLOP/s at 32768 tokens against 1.5 for the forward's layout).  The attention
-// operator's product kernel takes exactly this layout (dV = P^T dY) and measured, at 32768
-// tokens, out x in = 11008 x 4096: 2.16 ms against 3.28 (3.16 with one operand transposed
-// first), 4096 x 11008: 2.22 / 3.13, 8192 x 4096: 1.54 / 1.87, 4096 x 4096: 0.78 / 0.92;
-// below one 256 x 256 tile per compute unit (1024 x 4096: 0.50 / 0.28 ms) the library stays.
-Tensor weight_grad(const Tensor& g, const Tensor& x) {
-  const int64_t tokens = g.size(0), n_out = g.size(1), n_in = x.size(1);
-  const int64_t tiles = ((n_out + 255) / 256) * ((n_in + 255) / 256);
-  // (operands of 2^30 elements and more leave the kernel's aligned path, whose offsets are 32-bit)
-  if (tokens >= 4096 && tokens % 32 == 0 && n_out % 8 == 0 && n_in % 8 == 0 && tiles >= 256 && tokens * std::max(n_out, n_in) < (1ll << 30)) {
-    const Tensor gc = g.contiguous(), xc = x.contiguous();
-    Tensor dw = at::empty({n_out, n_in}, x.options());
-    check(mega_linear_weight_grad(gc.data_ptr(), xc.data_ptr(), kernel_code(x), tokens, n_out, n_in, dw.data_ptr(), stream_of(x)), "mega_linear_weight_grad");
-    return dw;
+// A matrix as the library's products take it: its own memory (no vmap wrapper), whole rows, 16-byte boundary.
+bool dense16(const Tensor& t) {
+  return t.has_storage() && t.is_contiguous() && !lazy(t) && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+}
+enum { kLinearForward, kLinearInputGrad, kLinearWeightGrad };
+// dW_i = g_i^T x, (out_i, in) from (tokens, out_i) and (tokens, in), for layers of one input in one launch.
+variable_list weight_grads(variable_list gs, const Tensor& x) {
+  const int64_t tokens = x.size(0), n_in = x.size(1);
+  const int code = code_of(x.scalar_type());
+  bool taken = !gs.empty() && gs.size() <= 3 && x.has_storage();
+  for (const Tensor& g : gs) taken = taken && g.has_storage() && g.scalar_type() == x.scalar_type() && g.size(0) == tokens;
+  std::vector<int64_t> n_out;
+  for (const Tensor& g : gs) n_out.push_back(g.size(1));
+  taken = taken && mega_linear_takes(kLinearWeightGrad, code, tokens, n_in, static_cast<int>(gs.size()), n_out.data());
+  variable_list dw;
+  if (taken) {
+    const Tensor xc = x.contiguous();
+    std::vector<const void*> from;
+    std::vector<void*> to;
+    taken = dense16(xc);
+    for (Tensor& g : gs) {
+      g = g.contiguous();
+      taken = taken && dense16(g);
+    }
+    if (taken) {
+      for (const Tensor& g : gs) {
+        dw.push_back(at::empty({g.size(1), n_in}, x.options()));
+        from.push_back(g.data_ptr());
+        to.push_back(dw.back().data_ptr());
+      }
+      check(mega_linear_weight_grads(from.data(), xc.data_ptr(), code, tokens, n_in, static_cast<int>(gs.size()), n_out.data(), to.data(), stream_of(x)), "mega_linear_weight_grads");
+      return dw;
+    }
   }
-  return at::mm(g.t(), x);
+  for (const Tensor& g : gs) dw.push_back(at::mm(g.t(), x));
+  return dw;
 }
 Tensor flat(const Tensor& t) { return t.reshape({-1, t.size(-1)}); }
 // the bias gradient: column sums of g (tokens, out)
@@ -500,8 +519,58 @@ Tensor bias_grad(const Tensor& g) {
 bool turned(const Tensor& g, const Tensor& w) {
   return static_cast<double>(g.size(0)) * w.size(0) * w.size(1) > static_cast<double>(1ll << 35);
 }
+// dx = g W, added to `sum` (in place) where there is one
+Tensor input_grad(const Tensor& g, const Tensor& w, const Tensor& sum) {
+  const int64_t tokens = g.size(0), n_out = g.size(1), n_in = w.size(1);
+  const int code = code_of(g.scalar_type());
+  if (w.scalar_type() == g.scalar_type() && w.size(0) == n_out && mega_linear_takes(kLinearInputGrad, code, tokens, n_in, 1, &n_out) &&
+      dense16(g) && dense16(w) && (!sum.defined() || dense16(sum))) {
+    const Tensor dx = sum.defined() ? sum : at::empty({tokens, n_in}, g.options());
+    check(mega_linear_input_grad(g.data_ptr(), w.data_ptr(), ptr(sum), code, tokens, n_out, n_in, dx.data_ptr(), stream_of(g)), "mega_linear_input_grad");
+    return dx;
+  }
+  if (!sum.defined()) return turned(g, w) ? at::linear(g, transpose_raw(w)) : at::mm(g, w);
+  const Tensor wt = turned(g, w) ? transpose_raw(w).t() : w;
+  Tensor dx = sum;
+  at::addmm_out(dx, sum, g, wt);
+  return dx;
+}
+// y_i = x W_i^T (+ bias_i), + residual with one layer, in one launch; nothing where the library's products are faster or
+// the operands are not what the launch takes
+std::optional<variable_list> products(const Tensor& x, const variable_list& w, const std::vector<Optional>& bias, const Optional& residual) {
+  const auto type = x.scalar_type();
+  if (!x.is_cuda() || x.dim() < 1 || (type != at::kBFloat16 && type != at::kHalf) || w.size() > 3 || at::autocast::is_autocast_enabled(at::kCUDA)) return std::nullopt;
+  const int64_t n_in = x.size(-1), tokens = n_in > 0 ? x.numel() / n_in : 0;
+  const auto fits = [&](const Tensor& t) { return t.scalar_type() == type && t.device() == x.device() && dense16(t); };
+  if (tokens < 1 || !fits(x)) return std::nullopt;
+  std::vector<int64_t> n_out;
+  for (size_t i = 0; i < w.size(); ++i) {
+    if (w[i].dim() != 2 || w[i].size(1) != n_in || !fits(w[i])) return std::nullopt;
+    if (bias[i].has_value() && (bias[i]->dim() != 1 || bias[i]->size(0) != w[i].size(0) || !fits(*bias[i]))) return std::nullopt;
+    n_out.push_back(w[i].size(0));
+  }
+  auto shape = x.sizes().vec();
+  shape.back() = n_out[0];
+  if (residual.has_value() && (w.size() != 1 || residual->sizes() != at::IntArrayRef(shape) || !fits(*residual))) return std::nullopt;
+  const int code = code_of(type), count = static_cast<int>(w.size());
+  if (!mega_linear_takes(kLinearForward, code, tokens, n_in, count, n_out.data())) return std::nullopt;
+  c10::DeviceGuard guard(x.device());
+  variable_list y;
+  std::vector<const void*> wp, bp;
+  std::vector<void*> yp;
+  for (size_t i = 0; i < w.size(); ++i) {
+    shape.back() = n_out[i];
+    y.push_back(at::empty(shape, x.options()));
+    wp.push_back(w[i].data_ptr());
+    bp.push_back(bias[i].has_value() ? bias[i]->data_ptr() : nullptr);
+    yp.push_back(y.back().data_ptr());
+  }
+  check(mega_linear_fwd(x.data_ptr(), wp.data(), bp.data(), residual.has_value() ? residual->data_ptr() : nullptr, code, tokens, n_in, count, n_out.data(), yp.data(), stream_of(x)), "mega_linear_fwd");
+  return y;
+}
 // x W^T (+ bias), or x W^T + residual with the residual as the product's accumulator input
 Tensor linear_raw(const Tensor& x, const Tensor& weight, const Optional& bias, const Optional& residual) {
+  if (auto y = products(x, {weight}, {bias}, residual); y.has_value()) return (*y)[0];
   if (!residual.has_value()) return at::linear(x, weight, bias);
   require(x.dim() >= 1 && residual->dim() >= 1, "linear: x and residual need at least one dimension");
   auto shape = x.sizes().vec();
@@ -537,8 +606,8 @@ struct LinearFn : Function<LinearFn> {
     at::AutoDispatchBelowADInplaceOrView below;
     const Tensor g2 = flat(g[0]);
     Tensor dx, dw, db, dr;
-    if (ctx->needs_input_grad(0)) dx = (turned(g2, weight) ? at::linear(g2, transpose_raw(weight)) : at::mm(g2, weight)).view(x.sizes());
-    if (ctx->needs_input_grad(1)) dw = weight_grad(g2, flat(x));
+    if (ctx->needs_input_grad(0)) dx = input_grad(g2, weight, Tensor()).view(x.sizes());
+    if (ctx->needs_input_grad(1)) dw = weight_grads({g2}, flat(x))[0];
     if (has_bias && ctx->needs_input_grad(2)) db = bias_grad(g2);
     if (has_residual && ctx->needs_input_grad(has_bias ? 3 : 2)) dr = g[0];
     return {dx, dw, db, dr};
@@ -553,17 +622,20 @@ Tensor linear(const Tensor& x, const Tensor& weight, const Optional& bias, const
 struct LinearGroupFn : Function<LinearGroupFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& x, at::TensorList params, std::vector<bool> has_bias) {
     at::AutoDispatchBelowADInplaceOrView below;
-    variable_list keep{x}, out;
+    variable_list keep{x}, weights;
+    std::vector<Optional> biases;
     size_t at_ = 0;
     std::vector<int64_t> bias_flags;
     for (const bool b : has_bias) {
-      const Tensor& w = params[at_++];
-      Optional bias;
-      if (b) bias = params[at_++];
-      keep.push_back(w);
+      weights.push_back(params[at_++]);
+      biases.push_back(b ? Optional(params[at_++]) : Optional());
+      keep.push_back(weights.back());
       bias_flags.push_back(b);
-      out.push_back(at::linear(x, w, bias));
     }
+    variable_list out;
+    if (auto y = products(x, weights, biases, Optional()); y.has_value()) out = *y;
+    else
+      for (size_t i = 0; i < weights.size(); ++i) out.push_back(linear_raw(x, weights[i], biases[i], Optional()));
     ctx->save_for_backward(keep);
     ctx->saved_data["bias"] = bias_flags;
     return out;
@@ -590,16 +662,24 @@ struct LinearGroupFn : Function<LinearGroupFn> {
     }
     at::AutoDispatchBelowADInplaceOrView below;
     const Tensor x2 = flat(x);
+    variable_list wanted;             // the gradients whose layers want a weight gradient,
+    std::vector<size_t> place;        // and where in `grads` it goes
     for (size_t i = 0; i < has_bias.size(); ++i) {
       const Tensor& w = saved[1 + i];
       const Tensor g2 = flat(g[i]);
-      if (ctx->needs_input_grad(0)) {
-        const Tensor wt = turned(g2, w) ? transpose_raw(w).t() : w;
-        if (!dx.defined()) dx = at::mm(g2, wt);
-        else at::addmm_out(dx, dx, g2, wt);
+      if (ctx->needs_input_grad(0)) dx = input_grad(g2, w, dx);
+      if (ctx->needs_input_grad(edge++)) {
+        wanted.push_back(g2);
+        place.push_back(grads.size());
       }
-      grads.push_back(ctx->needs_input_grad(edge++) ? weight_grad(g2, x2) : Tensor());
+      grads.push_back(Tensor());
       if (has_bias[i]) grads.push_back(ctx->needs_input_grad(edge++) ? bias_grad(g2) : Tensor());
+    }
+    if (wanted.size() <= 3) {
+      const variable_list dw = wanted.empty() ? variable_list() : weight_grads(wanted, x2);
+      for (size_t i = 0; i < dw.size(); ++i) grads[place[i]] = dw[i];
+    } else {
+      for (size_t i = 0; i < wanted.size(); ++i) grads[place[i]] = weight_grads({wanted[i]}, x2)[0];
     }
     grads[0] = dx.defined() ? dx.view(x.sizes()) : Tensor();
     grads.push_back(Tensor());

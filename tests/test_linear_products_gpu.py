@@ -1,0 +1,112 @@
+"""The linear layers' three products on the library's own kernels (`mega_linear_*`), one to three layers of one input in a
+launch, against float64: one row, edges of tiles of 128 and 256, tokens off the slabs of 32, layers narrower than a
+tile, sizes that take either tile.  A 16-bit result of a float32 accumulation: 2^-9 of each value (bfloat16, float16
+2^-12) from its one rounding, and as much again for sums of thousands of terms in float32."""
+import ctypes
+
+import pytest
+import torch
+
+from megalodon_amd import _lib
+from megalodon_amd.modules.linear import Linear, linear_group
+
+pytestmark = pytest.mark.gpu
+
+
+def _pointers(tensors):
+    return (ctypes.c_void_p * len(tensors))(*[0 if t is None else t.data_ptr() for t in tensors])
+
+
+def _poisoned(t):  # NaN behind the last element
+    buf = torch.full((t.numel() + 4096,), float("nan"), dtype=t.dtype, device="cuda")
+    return buf[:t.numel()].view(t.shape).copy_(t)
+
+
+def _close(got, want):
+    eps = 2.0 ** -8 if got.dtype == torch.bfloat16 else 2.0 ** -11
+    assert torch.isfinite(got.float()).all()
+    assert (got.double() - want).norm() <= eps * want.norm()
+
+
+@pytest.mark.parametrize("tokens,n_in,n_out,dtype", [
+    (1, 64, [64], torch.bfloat16),
+    (33, 64, [64, 128], torch.float16),
+    (127, 192, [192], torch.bfloat16),
+    (129, 128, [64, 320, 128], torch.bfloat16),
+    (256, 256, [256, 128, 64], torch.float16),
+    (257, 320, [192], torch.bfloat16),
+    (1021, 2048, [512, 4096, 2048], torch.bfloat16),   # tiles of 256 forward
+    (1021, 5504, [2048], torch.bfloat16),
+    (2048, 2048, [5504], torch.float16),
+    (4084, 1024, [2752, 2752], torch.bfloat16),
+    (4084, 2048, [512, 4096, 2048], torch.bfloat16),   # tiles of 256 for the weight gradients
+    (4100, 704, [2048, 64], torch.float16),
+])
+def test_products_match_float64(tokens, n_in, n_out, dtype):
+    g = torch.Generator("cuda").manual_seed(tokens + n_in)
+    rows = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x = _poisoned(rows(tokens, n_in).to(dtype))
+    w = [_poisoned((rows(o, n_in) / n_in ** 0.5).to(dtype)) for o in n_out]
+    bias = [rows(o).to(dtype) if i != 1 else None for i, o in enumerate(n_out)]
+    dy = [_poisoned(rows(tokens, o).to(dtype)) for o in n_out]
+    add, code, i64 = rows(tokens, n_out[0]).to(dtype), _lib.dtype_code(dtype), ctypes.c_int64
+    y = [torch.empty(tokens, o, dtype=dtype, device="cuda") for o in n_out]
+    dw = [torch.empty_like(t) for t in w]
+    outs, s = (i64 * len(n_out))(*n_out), _lib.stream_ptr(x.device)
+    call = lambda name, *a: _lib.call(name, *a, s)
+    call("mega_linear_fwd", _lib.ptr(x), _pointers(w), _pointers(bias), None, _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(len(w)), outs, _pointers(y))
+    call("mega_linear_weight_grads", _pointers(dy), _lib.ptr(x), _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(len(w)), outs, _pointers(dw))
+    x64, w64, dy64 = x.double(), [t.double() for t in w], [t.double() for t in dy]
+    for i in range(len(w)):
+        _close(y[i], x64 @ w64[i].t() + (0 if bias[i] is None else bias[i].double()))
+        _close(dw[i], dy64[i].t() @ x64)
+        # one layer alone gives the same bits as in the group
+        if len(w) > 1:
+            alone = torch.empty_like(y[i])
+            call("mega_linear_fwd", _lib.ptr(x), _pointers([w[i]]), _pointers([bias[i]]), None, _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(1), (i64 * 1)(n_out[i]), _pointers([alone]))
+            assert torch.equal(alone, y[i])
+    call("mega_linear_fwd", _lib.ptr(x), _pointers(w[:1]), None, _lib.ptr(add), _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(1), (i64 * 1)(n_out[0]), _pointers(y[:1]))
+    _close(y[0], x64 @ w64[0].t() + add.double())
+    dx = torch.empty_like(x)
+    for i in range(len(w)):  # added up in place
+        before = dx.double()
+        call("mega_linear_input_grad", _lib.ptr(dy[i]), _lib.ptr(w[i]), _lib.ptr(dx) if i else None, _lib.i32(code), i64(tokens), i64(n_out[i]), i64(n_in), _lib.ptr(dx))
+        _close(dx, dy64[i] @ w64[i] + (before if i else 0))
+
+
+def test_refused_sizes():
+    fn = _lib.load().mega_linear_takes
+    i64 = ctypes.c_int64
+    takes = lambda kind, tokens, n_in, *n_out: fn(kind, 1, i64(tokens), i64(n_in), len(n_out), (i64 * len(n_out))(*n_out))
+    assert takes(0, 100, 256, 256) and takes(1, 100, 256, 256) and takes(2, 100, 256, 72)
+    for kind, sizes in [(0, (100, 72, 64)), (1, (100, 64, 72)), (2, (100, 64, 77)), (2, (0, 64, 64)), (0, (1 << 24, 64, 64)),
+                        (0, (8, 64, 64, 64, 64, 64)), (3, (64, 64, 64))]:
+        assert not takes(kind, *sizes)
+
+
+@pytest.mark.parametrize("tokens,sizes", [(40, (128, 64)), (300, (192, 320))])
+def test_layers_whose_operands_need_the_general_path(tokens, sizes):
+    """Transposed and misaligned operands, broadcast residuals, more layers than a launch takes, a vmapped backward: as ever."""
+    torch.manual_seed(tokens)
+    n_in, n_out = sizes
+    layer = Linear(n_in, n_out, bias=False).cuda().bfloat16()
+    x = torch.randn(tokens, n_in, device="cuda").bfloat16()
+    want = x.double() @ layer.weight.double().t()
+    with torch.no_grad():
+        _close(layer(x.t().contiguous().t()), want)
+        shifted = torch.empty(tokens * n_in + 1, dtype=x.dtype, device="cuda")[1:].view(tokens, n_in).copy_(x)
+        _close(layer(shifted), want)
+        row = torch.randn(n_out, device="cuda").bfloat16()
+        _close(layer(x, residual=row.expand(tokens, n_out)), want + row.double())
+        with pytest.raises(RuntimeError):
+            layer(x[:, : n_in // 2])
+    leaf = x.clone().requires_grad_(True)
+    four = [Linear(n_in, n_out).cuda().bfloat16() for _ in range(4)]
+    ys = linear_group(leaf, four)
+    torch.autograd.backward(ys, [torch.ones_like(y) for y in ys])
+    _close(leaf.grad, sum(torch.ones(tokens, n_out, dtype=torch.float64, device="cuda") @ l.weight.double() for l in four))
+    y = layer(leaf)
+    many = torch.randn(3, tokens, n_out, device="cuda").bfloat16()
+    dx, dw = torch.autograd.grad(y, (leaf, layer.weight), many, is_grads_batched=True)
+    _close(dx, many.double() @ layer.weight.double())
+    _close(dw, torch.stack([g.double().t() @ x.double() for g in many]))
