@@ -650,6 +650,12 @@ int mega_group_sequence_norm_bwd(const void* dy, const void* x, const int64_t* c
  *   others return MEGA_ERR_UNSUPPORTED (use the kernel-row path then).
  * ---------------------------------------------------------------------- */
 int mega_cema_scan_supported(int dtype, int64_t N, int64_t L);
+/* The same from the layer's raw parameters of `param_dtype` (alpha, delta (D, N), theta (D), gamma (D, N, 2), omega (D);
+ * the coefficients are those of mega_cema_layer_coeffs_fwd): rows of which a workgroup takes no more than one item form them
+ * in the same launch, others in one of their own.  workspace: 5 D N floats. */
+int mega_cema_layer_fwd(const void* x, int dtype, int param_dtype, const void* alpha, const void* delta,
+                        const void* theta, const void* gamma, const void* omega, int64_t B, int64_t D,
+                        int64_t N, int64_t L, void* y, void* workspace, void* stream);
 int mega_cema_scan_fwd(const void* x, int dtype, const float* p, const float* log_q,
                        const float* gamma, const float* omega, const float* h0, int64_t B,
                        int64_t D, int64_t N, int64_t L, void* y, float* h_last, void* stream);

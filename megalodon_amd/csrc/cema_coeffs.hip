@@ -17,13 +17,12 @@
 //   dtheta = t (1 - t) (2 pi / N) sum_n n dphi_n
 //   dgamma = sqrt(1 / N) (Re dgamma_hat, Im dgamma_hat)
 #include "common.hpp"
+#include "cema_pow.hpp"
 
 namespace mega {
 namespace {
 
 constexpr int kThreads = 256;
-
-__device__ __forceinline__ float sigmoidf(float v) { return 1.f / (1.f + expf(-v)); }
 
 template <int DT>
 __global__ __launch_bounds__(kThreads) void cema_coeffs_fwd_kernel(
@@ -35,15 +34,12 @@ __global__ __launch_bounds__(kThreads) void cema_coeffs_fwd_kernel(
   const int64_t ch = i / N;
   const int n = static_cast<int>(i % N);
   using E = Elem<DT>;
-  const float a = sigmoidf(E::load(alpha + i)), d = sigmoidf(E::load(delta + i)), t = sigmoidf(E::load(theta + ch));
-  const float scale = sqrtf(1.f / static_cast<float>(N));
-  p[i] = a;
-  // log |q| = log(1 - a d) without forming 1 - a d: rounded to float32 that difference loses
-  // the decay rate's low bits when a d is small (6e-4 of it at a d = 1e-4)
-  log_q[2 * i] = log1pf(-a * d);
-  log_q[2 * i + 1] = static_cast<float>(n + 1) * (t * (6.283185307179586f / static_cast<float>(N)));
-  gamma_hat[2 * i] = E::load(gamma + 2 * i) * scale;
-  gamma_hat[2 * i + 1] = E::load(gamma + 2 * i + 1) * scale;
+  const CemaCoeffs c = cema_coeffs(E::load(alpha + i), E::load(delta + i), E::load(theta + ch), n, N);
+  p[i] = c.p;
+  log_q[2 * i] = c.log_rho;
+  log_q[2 * i + 1] = c.phi;
+  gamma_hat[2 * i] = E::load(gamma + 2 * i) * c.scale;
+  gamma_hat[2 * i + 1] = E::load(gamma + 2 * i + 1) * c.scale;
 }
 
 // One thread per (channel, mode); the sum over the modes of a channel runs
@@ -77,7 +73,7 @@ __global__ __launch_bounds__(kThreads) void cema_coeffs_bwd_kernel(
       hi += h.y;
       if (n == 0 && dskip != nullptr) gw += dskip[k * D + ch];
     }
-    const float a = sigmoidf(E::load(alpha + i)), d = sigmoidf(E::load(delta + i)), t = sigmoidf(E::load(theta + ch));
+    const float a = cema_sigmoid(E::load(alpha + i)), d = cema_sigmoid(E::load(delta + i)), t = cema_sigmoid(E::load(theta + ch));
     const float rho = 1.f - a * d;
     const float phi = static_cast<float>(n + 1) * (t * (6.283185307179586f / static_cast<float>(N)));
     float sn, cs;
@@ -97,7 +93,7 @@ __global__ __launch_bounds__(kThreads) void cema_coeffs_bwd_kernel(
   if (on && n == 0) {
     float s = 0.f;
     for (int k = 0; k < N; ++k) s += s_phi[local_ch * N + k];
-    const float t = sigmoidf(E::load(theta + ch));
+    const float t = cema_sigmoid(E::load(theta + ch));
     E::store(dtheta + ch, t * (1.f - t) * (6.283185307179586f / static_cast<float>(N)) * s);
   }
 }

@@ -22,4 +22,16 @@ __device__ __forceinline__ cf qpow(float a, float phi, int64_t j) {
   return {mag * c, mag * s};
 }
 
+// The coefficients of mode n (0-based) of N from a channel's raw parameters (see cema_coeffs.hip).
+struct CemaCoeffs {
+  float p, log_rho, phi, scale;
+};
+__device__ __forceinline__ float cema_sigmoid(float v) { return 1.f / (1.f + expf(-v)); }
+__device__ __forceinline__ CemaCoeffs cema_coeffs(float alpha, float delta, float theta, int n, int N) {
+  const float a = cema_sigmoid(alpha), d = cema_sigmoid(delta), t = cema_sigmoid(theta);
+  // log |q| = log(1 - a d) without forming 1 - a d: rounded to float32 that difference loses
+  // the decay rate's low bits when a d is small (6e-4 of it at a d = 1e-4)
+  return {a, log1pf(-a * d), static_cast<float>(n + 1) * (t * (6.283185307179586f / static_cast<float>(N))), sqrtf(1.f / static_cast<float>(N))};
+}
+
 }  // namespace mega

@@ -75,6 +75,16 @@ __device__ __forceinline__ u32x4 split8_third(const float* v, u32x4 hi, u32x4 lo
 // lane reads whole words.
 constexpr int kThirdLags = 96;
 typedef uint16_t ThirdTable[2][kThirdLags];
+// The first two pieces of the lags in such tables (in place of whole operand blocks).
+__device__ __forceinline__ void fill_pieces(ThirdTable& hi, ThirdTable& lo, const float* k, int tid) {
+  if (tid < 2 * kThirdLags) {
+    const int lag = kT - 1 - (tid < kThirdLags ? tid : tid - kThirdLags + 1);
+    const float v = lag >= 0 && lag < kT ? k[lag] : 0.f;
+    const uint32_t h = pack_bf16x2(v, 0.f);
+    hi[0][tid] = static_cast<uint16_t>(h);
+    lo[0][tid] = static_cast<uint16_t>(pack_bf16x2(v - __uint_as_float(h << 16), 0.f));
+  }
+}
 template <bool DOWN>  // index i: lag 63 - i, else i - 31
 __device__ __forceinline__ void fill_thirds(ThirdTable& t, const float* k, int tid) {
   if (tid < 2 * kThirdLags) {
@@ -271,27 +281,59 @@ __device__ __forceinline__ floatx16 mma_split(const u32x4* a, const u32x4* x, fl
 //   8..11  Q, (row tile it, k-step s2): rows i = 32 it + r, state columns m = 16 s2 + 8 g + e
 constexpr int kFwdBlocks = 12;
 
-struct FwdSmem {
+// ONE: a workgroup takes one item (at most four tiles) and ends.  Setting up its channel is a chain of short phases
+// with a barrier between them, so what counts is how many workgroups share a compute unit: without the blocks of K,
+// whose lags are read out of a table of 96 instead, four fit (128 registers a lane: nothing is loaded ahead).
+template <bool ONE>
+struct FwdSmemOf {
   static constexpr int NC = kWaves * 32;       // chunks resident
-  float klocal[kT];                            // k[0 .. 63] (+ omega at lag 0)
+  static constexpr int kBlocks = ONE ? 8 : kFwdBlocks;
+  union {
+    float klocal[kT];                          // k[0 .. 63] (+ omega at lag 0), while a row is set up
+    cf sub_end[kWaves * 3][16];                // local end state of each sub-segment but a wave's last
+  };
   float pn[16];
   cf gn[16];
-  cf sub_end[kSubs][16];                       // local end state of each sub-segment (4 per wave)
   cf wave_end[2][kWaves][16];                  // local end state of each wave's 4 sub-segments, by item parity
   float wave_cin[kWaves][32];                  // state in front of each wave's first chunk
   cf carry[2][16];
   cf pw[12][16];                               // q^(4 k), q^(16 k) (k < 4), q, q^64, q^(64 CPS), q^(256 CPS)
-  u32x4 aop[kFwdBlocks][2][kWave];
+  u32x4 aop[kBlocks][2][kWave];                // ONE: P, then Q
   // row 1 + c: state after chunk c of the segment; while a row is set up the buffer holds the
   // power table q_n^e, e = 0 .. 64 (16 x 66 complex), from which the operand blocks are built
   float H[(NC + 1) * kHP];
 };
-static_assert(sizeof(cf) * 16 * (kT + 2) <= sizeof(float) * (kWaves * 32 + 1) * kHP, "the power table fits the state buffer");
+struct FwdSmem : FwdSmemOf<false> {};
 struct FwdSmemFine : FwdSmem {
   u32x4 third[4][kWave];  // third pieces of P
   alignas(4) ThirdTable kthird;
 };
+struct FwdSmemOne : FwdSmemOf<true> {
+  cf lq[16];
+  alignas(4) ThirdTable kpiece[2];
+};
+struct FwdSmemOneFine : FwdSmemOne {
+  u32x4 third[4][kWave];
+  alignas(4) ThirdTable kthird;
+};
+static_assert(sizeof(cf) * 16 * (kT + 2) <= sizeof(float) * (kWaves * 32 + 1) * kHP, "the power table fits the state buffer");
 static_assert(3 * sizeof(FwdSmemFine) <= 160 * 1024, "three workgroups per compute unit");
+static_assert(4 * sizeof(FwdSmemOne) <= 160 * 1024 && 3 * sizeof(FwdSmemOneFine) <= 160 * 1024, "four (three) workgroups per compute unit");
+
+// The channels' coefficients: p, log q, gamma in float32, or, where `alpha` is not null, the layer's raw parameters of element type
+// `dtype`, turned into them as mega_cema_layer_coeffs_fwd does.
+struct Coeffs {
+  const float* p;
+  const cf *log_q, *gamma;
+  const float* omega;
+  const void *alpha, *delta, *theta, *raw_gamma, *raw_omega;
+  int dtype;
+};
+__device__ __forceinline__ float load_any(const void* base, int dtype, int64_t i) {
+  if (dtype == MEGA_F32) return static_cast<const float*>(base)[i];
+  const uint16_t v = static_cast<const uint16_t*>(base)[i];
+  return dtype == MEGA_BF16 ? bf16_bits_to_float(v) : f16_bits_to_float(v);
+}
 
 // The rows of a launch: groups of `nb` rows of one channel (d = group % D), each a line of tiles.
 struct Lines {
@@ -359,13 +401,13 @@ __device__ __forceinline__ void tile_backward(const Lines& ln, Tile& w, int tile
 // and waits for its own LDS operations can read what its other lanes wrote.
 __device__ __forceinline__ void wave_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-template <int DT, int ROWS>
-__global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
-    const void* __restrict__ x, void* __restrict__ y, const float* __restrict__ p,
-    const cf* __restrict__ log_q, const cf* __restrict__ gamma, const float* __restrict__ omega,
+template <int DT, int ROWS, bool ONE>
+__global__ __launch_bounds__(kThreads, ONE && !kFine<ROWS> ? 4 : 3) void cema_scan_fwd_kernel(
+    const void* __restrict__ x, void* __restrict__ y, const Coeffs co,
     const cf* __restrict__ h0, cf* __restrict__ h_last, const Lines ln, int N) {
   constexpr bool FINE = kFine<ROWS>;
-  using Smem = typename std::conditional<FINE, FwdSmemFine, FwdSmem>::type;
+  using Smem = typename std::conditional<ONE, typename std::conditional<FINE, FwdSmemOneFine, FwdSmemOne>::type,
+                                         typename std::conditional<FINE, FwdSmemFine, FwdSmem>::type>::type;
   constexpr int NC = Smem::NC, CPS = NC / kSubs, XP = XOp<DT>::XP;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Smem& sm = *reinterpret_cast<Smem*>(smem_raw);
@@ -392,12 +434,14 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
     RowParams rp{cf{0.f, 0.f}, cf{0.f, 0.f}, 0.f, 0.f};
     if (group < ln.groups) {
       const int d = group % ln.D;
-      if (sn < N) {
-        rp.lq = log_q[d * N + sn];
-        rp.gv = gamma[d * N + sn];
-        rp.pv = p[d * N + sn];
+      if (sn < N && co.p != nullptr) {
+        const int i = d * N + sn;
+        rp.lq = co.log_q[i];
+        rp.gv = co.gamma[i];
+        rp.pv = co.p[i];
       }
-      if (omega != nullptr) rp.w = omega[d];
+      if (co.raw_omega != nullptr) rp.w = load_any(co.raw_omega, co.dtype, d);
+      else if (co.omega != nullptr) rp.w = co.omega[d];
     }
     return rp;
   };
@@ -411,6 +455,25 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
   auto setup_row = [&](int group) {
     // the few powers that are evaluated directly (phase reduced in float64): 12 per mode;
     // everything else is a product of two of them and a short chain of multiplications
+    if constexpr (ONE) {
+      // one lane per mode forms or fetches its coefficients (238 vector instructions of 1100 when every lane did)
+      if (tid < 16) {
+        if (co.alpha != nullptr && tid < N) {
+          const int d = group % ln.D, i = d * N + tid;
+          const CemaCoeffs c = cema_coeffs(load_any(co.alpha, co.dtype, i), load_any(co.delta, co.dtype, i), load_any(co.theta, co.dtype, d), tid, N);
+          rp.lq = cf{c.log_rho, c.phi};
+          rp.gv = cf{load_any(co.raw_gamma, co.dtype, 2 * i) * c.scale, load_any(co.raw_gamma, co.dtype, 2 * i + 1) * c.scale};
+          rp.pv = c.p;
+        }
+        sm.lq[tid] = rp.lq;
+        sm.pn[tid] = rp.pv;
+        sm.gn[tid] = rp.gv;
+      }
+      __syncthreads();
+      rp.lq = sm.lq[sn];
+      rp.pv = sm.pn[sn];
+      rp.gv = sm.gn[sn];
+    }
     cf direct{0.f, 0.f};
     if (tid < 12 * 16 && sn < N) {
       const int k = tid >> 4;
@@ -418,9 +481,9 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
                           : (k < 8 ? 16 * (k - 4) : (k == 8 ? 1 : (k == 9 ? kT : (k == 10 ? kT * CPS : 4 * kT * CPS))));
       direct = qpow(rp.lq.x, rp.lq.y, e);
     }
-    __syncthreads();  // every wave is done with the previous row's tables and carried state
+    if constexpr (!ONE) __syncthreads();  // every wave is done with the previous row's tables and carried state
     if (tid < 12 * 16) sm.pw[tid >> 4][sn] = direct;
-    if (tid < 16) {
+    if (!ONE && tid < 16) {
       sm.pn[tid] = rp.pv;
       sm.gn[tid] = rp.gv;
     }
@@ -444,10 +507,11 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
       qS = sm.pw[10][sn];
       qW = sm.pw[11][sn];
     }
-    const RowParams next_rp = fetch_params(group + static_cast<int>(gridDim.x));
+    RowParams next_rp{};
+    if constexpr (!ONE) next_rp = fetch_params(group + static_cast<int>(gridDim.x));
     __syncthreads();
-    for (int item = tid; item < kFwdBlocks * kWave; item += kThreads) {
-      const int blk = item >> 6, ln = item & 63, rr = ln & 31, gg = ln >> 5;
+    for (int item = tid; item < Smem::kBlocks * kWave; item += kThreads) {
+      const int at = item >> 6, blk = ONE && at >= 4 ? at + 4 : at, ln = item & 63, rr = ln & 31, gg = ln >> 5;
       float v[8];
       if (blk < 4) {
         const int n = rr >> 1, part = rr & 1;
@@ -476,11 +540,12 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
       }
       u32x4 hi, lo;
       split8(v, hi, lo);
-      sm.aop[blk][0][ln] = hi;
-      sm.aop[blk][1][ln] = lo;
+      sm.aop[at][0][ln] = hi;
+      sm.aop[at][1][ln] = lo;
       if constexpr (FINE)
         if (blk < 4) sm.third[blk][ln] = split8_third(v, hi, lo);
     }
+    if constexpr (ONE) fill_pieces(sm.kpiece[0], sm.kpiece[1], sm.klocal, tid);
     if constexpr (FINE) fill_thirds<true>(sm.kthird, sm.klocal, tid);
     __syncthreads();
     rp = next_rp;
@@ -537,7 +602,14 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
     {
       u32x4 K[4][2];
 #pragma unroll
-      for (int b = 0; b < 4; ++b) load_block(4 + b, K[b]);
+      for (int b = 0; b < 4; ++b) {
+        if constexpr (ONE) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) K[b][h] = read_thirds(sm.kpiece[h], kT - 1 - 16 * (b - 1) - r + 8 * g);
+        } else {
+          load_block(4 + b, K[b]);
+        }
+      }
 #pragma unroll
       for (int it = 0; it < 2; ++it) {
 #pragma unroll
@@ -553,7 +625,7 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
         }
       }
     }
-    {
+    if constexpr (!ONE) {
       if (t0 + kWaves < tiles) tile_forward<ROWS>(ln, cur_tile, tiles);
       else cur_tile = tile_at<ROWS>(ln, group + static_cast<int>(gridDim.x), wave);
       load_tile(xb, cur_tile);
@@ -573,16 +645,16 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
       cf h{0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < CPS; ++i) h = cadd(cmul(qT, h), cf{sv[i].x, sv[i].y});
-      sm.sub_end[sa][sn] = h;
+      if (sl < 3) sm.sub_end[3 * wave + sl][sn] = h;
       wave_sync();
       if (sl == 3) {
-        cf e = sm.sub_end[sa - 3][sn];
-        e = cadd(cmul(qS, e), sm.sub_end[sa - 2][sn]);
-        e = cadd(cmul(qS, e), sm.sub_end[sa - 1][sn]);
+        cf e = sm.sub_end[3 * wave][sn];
+        e = cadd(cmul(qS, e), sm.sub_end[3 * wave + 1][sn]);
+        e = cadd(cmul(qS, e), sm.sub_end[3 * wave + 2][sn]);
         sm.wave_end[par][wave][sn] = cadd(cmul(qS, e), h);
       }
       lds_barrier();
-      cf cin = sm.carry[cur][sn];
+      cf cin = ONE ? cf{0.f, 0.f} : sm.carry[cur][sn];
       // through the tiles in front of this wave's, from the first one of its row if that is among the
       // four (there the carried state enters)
       const int k = w.chunk0 / 32, from = k <= wave ? wave - k : 0;
@@ -590,11 +662,11 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
 #pragma unroll
       for (int v = 0; v < kWaves - 1; ++v)
         if (v >= from && v < wave) cin = cadd(cmul(qW, cin), sm.wave_end[par][v][sn]);
-      if (sa == kSubs - 1) sm.carry[cur ^ 1][sn] = cadd(cmul(qW, cin), sm.wave_end[par][kWaves - 1][sn]);
+      if (!ONE && sa == kSubs - 1) sm.carry[cur ^ 1][sn] = cadd(cmul(qW, cin), sm.wave_end[par][kWaves - 1][sn]);
       if (sl == 0) *reinterpret_cast<float2*>(sm.wave_cin[wave] + 2 * sn) = make_float2(cin.x, cin.y);
 #pragma unroll
       for (int s = 0; s < 3; ++s) {
-        const cf e = sm.sub_end[4 * wave + s][sn];
+        const cf e = sm.sub_end[3 * wave + s][sn];
         if (s < sl) cin = cadd(cmul(qS, cin), e);
       }
       h = cin;
@@ -610,7 +682,7 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
     {
       u32x4 Q[4][2];
 #pragma unroll
-      for (int b = 0; b < 4; ++b) load_block(8 + b, Q[b]);
+      for (int b = 0; b < 4; ++b) load_block((ONE ? 4 : 8) + b, Q[b]);
       if (w.nc > 0) {
         u32x4 hb[2][2];
         // the state in front of chunk c0 + r: the previous row of the buffer, or, for the
@@ -708,6 +780,10 @@ __global__ __launch_bounds__(kThreads, 3) void cema_scan_fwd_kernel(
   };
 
   load_tile(xb, cur_tile);
+  if constexpr (ONE) {
+    item(blockIdx.x, 0, ln.tiles(blockIdx.x));
+    return;
+  }
   for (int group = blockIdx.x; group < ln.groups; group += static_cast<int>(gridDim.x)) {
     const int tiles = ln.tiles(group);
     for (int t0 = 0; t0 < tiles; t0 += kWaves) item(group, t0, tiles);
@@ -736,23 +812,37 @@ int compute_units(int* cus) {
   return MEGA_OK;
 }
 
-template <int DT, int ROWS>
-int launch_fwd(const void* x, void* y, const float* p, const cf* log_q, const cf* gamma,
-               const float* omega, const cf* h0, cf* h_last, int64_t B, int64_t D, int64_t N,
-               int64_t L, hipStream_t stream) {
-  const size_t lds = kFine<ROWS> ? sizeof(FwdSmemFine) : sizeof(FwdSmem);
-  MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cema_scan_fwd_kernel<DT, ROWS>),
+template <int DT, int ROWS, bool ONE>
+int launch_fwd_as(const void* x, void* y, const Coeffs& co, const cf* h0, cf* h_last, const Lines& ln, unsigned grid, int64_t N, hipStream_t stream) {
+  const size_t lds = ONE ? (kFine<ROWS> ? sizeof(FwdSmemOneFine) : sizeof(FwdSmemOne)) : (kFine<ROWS> ? sizeof(FwdSmemFine) : sizeof(FwdSmem));
+  MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cema_scan_fwd_kernel<DT, ROWS, ONE>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-  int cus = 0;
-  const int rc = compute_units(&cus);
-  if (rc != MEGA_OK) return rc;
-  const int64_t slots = 3 * static_cast<int64_t>(cus);  // workgroups that fit the chip
-  const Lines ln = make_lines(B, D, L, slots, false, ROWS);
-  const unsigned grid = static_cast<unsigned>(ln.groups < slots ? ln.groups : slots);
-  cema_scan_fwd_kernel<DT, ROWS><<<dim3(grid), kThreads, lds, stream>>>(x, y, p, log_q, gamma, omega, h0, h_last, ln,
-                                                                       static_cast<int>(N));
+  cema_scan_fwd_kernel<DT, ROWS, ONE><<<dim3(grid), kThreads, lds, stream>>>(x, y, co, h0, h_last, ln, static_cast<int>(N));
   MEGA_CHECK_LAUNCH();
   return MEGA_OK;
+}
+// Whether the groups hold no more than the four tiles of an item each: a workgroup per group then.
+int lines_of(int64_t B, int64_t D, int64_t L, int rows, Lines* ln, int64_t* slots, bool* one) {
+  int cus = 0;
+  if (const int rc = compute_units(&cus); rc != MEGA_OK) return rc;
+  *slots = (rows == kWhole ? 4 : 3) * static_cast<int64_t>(cus);  // workgroups that fit the chip
+  *ln = make_lines(B, D, L, *slots, false, rows);
+  *one = ln->nb * static_cast<int64_t>(ln->tpr) <= kWaves;
+  if (!*one) {
+    *slots = 3 * static_cast<int64_t>(cus);
+    *ln = make_lines(B, D, L, *slots, false, rows);
+  }
+  return MEGA_OK;
+}
+template <int DT, int ROWS>
+int launch_fwd(const void* x, void* y, const Coeffs& co, const cf* h0, cf* h_last, int64_t B, int64_t D, int64_t N,
+               int64_t L, hipStream_t stream) {
+  Lines ln;
+  int64_t slots = 0;
+  bool one = false;
+  if (const int rc = lines_of(B, D, L, ROWS, &ln, &slots, &one); rc != MEGA_OK) return rc;
+  if (one) return launch_fwd_as<DT, ROWS, true>(x, y, co, h0, h_last, ln, static_cast<unsigned>(ln.groups), N, stream);
+  return launch_fwd_as<DT, ROWS, false>(x, y, co, h0, h_last, ln, static_cast<unsigned>(ln.groups < slots ? ln.groups : slots), N, stream);
 }
 
 
@@ -1482,12 +1572,8 @@ extern "C" int mega_cema_scan_supported(int dtype, int64_t N, int64_t L) {
   return valid_dtype(dtype) && N >= 1 && N <= 16 && L >= 1 && (dtype != MEGA_F32 || L % 8 == 0);
 }
 
-extern "C" int mega_cema_scan_fwd(const void* x, int dtype, const float* p, const float* log_q,
-                                  const float* gamma, const float* omega, const float* h0,
-                                  int64_t B, int64_t D, int64_t N, int64_t L, void* y, float* h_last,
-                                  void* stream) {
-  const char* who = "mega_cema_scan_fwd";
-  MEGA_CHECK_ARG(x && p && log_q && gamma && y, "%s: null pointer", who);
+static int scan_fwd_entry(const char* who, const void* x, int dtype, const Coeffs& co, const float* h0, int64_t B, int64_t D,
+                          int64_t N, int64_t L, void* y, float* h_last, void* stream) {
   MEGA_CHECK_ARG(B >= 0 && D >= 0 && L >= 0, "%s: negative size", who);
   MEGA_CHECK_ARG(B * D <= 0x7fffffff, "%s: too many rows", who);
   if (!mega_cema_scan_supported(dtype, N, L))
@@ -1498,8 +1584,6 @@ extern "C" int mega_cema_scan_fwd(const void* x, int dtype, const float* p, cons
   MEGA_CHECK_ARG(rows == kWhole || dtype != MEGA_F32, "%s: float32 rows must be 16-byte aligned", who);
   if (B == 0 || D == 0) return MEGA_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const cf* lq = reinterpret_cast<const cf*>(log_q);
-  const cf* gm = reinterpret_cast<const cf*>(gamma);
   const cf* h0c = reinterpret_cast<const cf*>(h0);
   cf* hl = reinterpret_cast<cf*>(h_last);
   auto go = dtype == MEGA_F32     ? launch_fwd<MEGA_F32, kWhole>
@@ -1509,7 +1593,48 @@ extern "C" int mega_cema_scan_fwd(const void* x, int dtype, const float* p, cons
                                  : (rows == kWhole     ? launch_fwd<MEGA_F16, kWhole>
                                     : rows == kShifted ? launch_fwd<MEGA_F16, kShifted>
                                                        : launch_fwd<MEGA_F16, kAny>);
-  return go(x, y, p, lq, gm, omega, h0c, hl, B, D, N, L, s);
+  return go(x, y, co, h0c, hl, B, D, N, L, s);
+}
+
+extern "C" int mega_cema_scan_fwd(const void* x, int dtype, const float* p, const float* log_q,
+                                  const float* gamma, const float* omega, const float* h0, int64_t B,
+                                  int64_t D, int64_t N, int64_t L, void* y, float* h_last,
+                                  void* stream) {
+  const char* who = "mega_cema_scan_fwd";
+  MEGA_CHECK_ARG(x && p && log_q && gamma && y, "%s: null pointer", who);
+  Coeffs co{};
+  co.p = p;
+  co.log_q = reinterpret_cast<const cf*>(log_q);
+  co.gamma = reinterpret_cast<const cf*>(gamma);
+  co.omega = omega;
+  return scan_fwd_entry(who, x, dtype, co, h0, B, D, N, L, y, h_last, stream);
+}
+
+extern "C" int mega_cema_layer_fwd(const void* x, int dtype, int param_dtype, const void* alpha, const void* delta, const void* theta,
+                                   const void* gamma, const void* omega, int64_t B, int64_t D, int64_t N, int64_t L, void* y,
+                                   void* workspace, void* stream) {
+  const char* who = "mega_cema_layer_fwd";
+  MEGA_CHECK_ARG(x && alpha && delta && theta && gamma && omega && y && workspace, "%s: null pointer", who);
+  MEGA_CHECK_ARG(valid_dtype(param_dtype), "%s: unknown parameter dtype %d", who, param_dtype);
+  MEGA_CHECK_ARG(B >= 1 && D >= 1 && N >= 1 && N <= 16 && L >= 1 && B * D <= 0x7fffffff, "%s: bad sizes", who);
+  Coeffs co{};
+  co.dtype = param_dtype;
+  co.raw_omega = omega;
+  Lines ln;
+  int64_t slots = 0;
+  bool one = false;
+  if (const int rc = lines_of(B, D, L, rows_of(B * D, L, false, {x, y}), &ln, &slots, &one); rc != MEGA_OK) return rc;
+  if (one) {
+    co.alpha = alpha; co.delta = delta; co.theta = theta; co.raw_gamma = gamma;
+  } else {
+    float* w = static_cast<float*>(workspace);
+    const int rc = mega_cema_layer_coeffs_fwd(param_dtype, alpha, delta, theta, gamma, D, N, w, w + D * N, w + 3 * D * N, stream);
+    if (rc != MEGA_OK) return rc;
+    co.p = w;
+    co.log_q = reinterpret_cast<const cf*>(w + D * N);
+    co.gamma = reinterpret_cast<const cf*>(w + 3 * D * N);
+  }
+  return scan_fwd_entry(who, x, dtype, co, nullptr, B, D, N, L, y, nullptr, stream);
 }
 
 extern "C" int mega_cema_scan_bwd_supported(int dtype, int64_t N, int64_t L) {

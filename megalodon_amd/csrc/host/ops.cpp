@@ -388,9 +388,11 @@ Optional cema(const Tensor& x, const Tensor& alpha, const Tensor& delta, const T
   if (code_of(alpha.scalar_type()) < 0 || !is(alpha, D * N) || !is(delta, D * N) || !is(theta, D) || !is(gamma, 2 * D * N) || !is(omega, D)) return std::nullopt;
   c10::DeviceGuard guard(x.device());
   if (wants_grad({&x, &alpha, &delta, &theta, &gamma, &omega})) return CemaFn::apply(x, alpha, delta, theta, gamma, omega);
-  const Tensor xc = rows_of(x), w = as_float(omega), c = cema_coeffs(alpha, delta, theta, gamma, D, N);
-  const float* p = c.data_ptr<float>();
-  return scan_raw(xc, p, p + D * N, p + 3 * D * N, fptr(w), nullptr, nullptr, N);
+  const Tensor xc = rows_of(x), ws = floats({5 * D * N}, x);
+  Tensor y = at::empty_like(xc);
+  if (y.numel() == 0) return y;
+  check(mega_cema_layer_fwd(xc.data_ptr(), kernel_code(x), kernel_code(alpha), alpha.data_ptr(), delta.data_ptr(), theta.data_ptr(), gamma.data_ptr(), omega.data_ptr(), x.size(0), D, N, x.size(2), y.data_ptr(), ws.data_ptr(), stream_of(x)), "mega_cema_layer_fwd");
+  return y;
 }
 // with a carried state and / or the last state wanted, without gradients; p, log_q, gamma_hat float32 / complex64
 std::optional<std::tuple<Tensor, Optional>> cema_state(const Tensor& x, const Tensor& p, const Tensor& log_q, const Tensor& gamma_hat, const Tensor& omega, const Optional& h0, bool last) {
