@@ -148,7 +148,7 @@ int mega_cema_coeffs_bwd(const float* dp, const float* dq, const float* dgamma_h
  *   a stream gets a block of its own, so launches on different streams never
  *   share slots, up to four blocks; a fifth stream takes over the block that
  *   has been idle longest and waits on the device for the last launch that
- *   used it); they are kept until process exit (32 MiB per block at every
+ *   used it); they are kept until process exit (96 MiB per block at every
  *   size on 256 compute units).  mega_fftconv_prepare(L, stream) makes
  *   them ahead of time (it allocates and synchronises `stream` once; not
  *   capturable); after it, the convolution entry points on that stream only

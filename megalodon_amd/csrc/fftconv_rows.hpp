@@ -1,0 +1,566 @@
+// The transform path of the causal convolution: row kernels, their tables and scratch, one transform size to a
+// translation unit (fftconv_m11.hip .. fftconv_m14.hip: M = 2^11 .. 2^14 complex points).
+#pragma once
+
+#include "common.hpp"
+#include "fftconv_core.hpp"
+
+#include <algorithm>
+#include <mutex>
+#include <vector>
+
+namespace mega {
+
+// ------------------------------ tables --------------------------------------
+constexpr int kFftDevices = 16;
+constexpr int kFftScratch = 4;  // scratch blocks per device and size before streams start taking turns
+struct StreamScratch {
+  hipStream_t stream;  // the stream whose launches used the block last
+  float* ptr;
+  hipEvent_t done;     // recorded behind the last launch that used the block
+  uint64_t tick;       // when that was
+  bool pinned;         // used under stream capture: the graph's replays own the block from then on
+};
+struct TableCache {
+  fftc::c32* ptr[kFftDevices][4] = {};
+  int slots[kFftDevices][4] = {};
+  // Launches on different streams of a device may overlap, and a workgroup's
+  // slot is picked by its index alone, so a stream gets a block of its own --
+  // up to kFftScratch of them per device and size.  A further stream takes
+  // over the block that has been idle longest and first waits (on the device,
+  // through the block's event) for the last launch that used it.  Blocks used
+  // under stream capture are never handed on.
+  std::vector<StreamScratch> scratch[kFftDevices][4];
+  uint64_t tick = 0;
+  std::mutex mu;
+};
+extern TableCache fft_tables;  // fftconv.hip
+
+// Rows of a size, by the unit that has it: mode 0 and 1 as fftconv_kernel has them.
+template <int LOGM>
+int fftconv_rows(int dtype, int mode, const void* a, const void* b, void* out, int64_t B, int64_t D, int64_t L, int flip,
+                 const float* omega, hipStream_t stream);
+// Makes a size's tables and the stream's scratch block.
+template <int LOGM>
+int fftconv_tables(hipStream_t stream);
+
+namespace {
+// ------------------------------ row I/O --------------------------------------
+template <int DT>
+__device__ __forceinline__ float ld(const void* base, int64_t i) {
+  return Elem<DT>::load(static_cast<const typename Elem<DT>::type*>(base) + i);
+}
+template <int DT>
+__device__ __forceinline__ void st(void* base, int64_t i, float v) {
+  Elem<DT>::store(static_cast<typename Elem<DT>::type*>(base) + i, v);
+}
+}  // namespace
+
+#ifdef MEGA_FFTCONV_LOGM
+namespace {
+
+using namespace fftc;
+
+// Workgroups of a transform size that share a compute unit: the kernel's time is the latency of its
+// exchanges and barriers, so two waves per SIMD at every size, which is what the registers (32 complex
+// points per lane and operand: 219-256 of 256, none spilled) and the planes in LDS allow.  With one wave
+// per SIMD below M = 16384 (and 330 registers) and the loads in branches, forward / backward in
+// bfloat16 took 2 x 1024 rows of 3000: 152 / 348 us, now 51 / 138; of 8192: 226 / 479, now 95 / 198;
+// 1024 rows of 16384: 236 / 485, now 115 / 219; of 32768: 440 / 891, now 246 / 502 (the last by the loads alone).
+template <int LOGM>
+constexpr int kPerCu = 1 << (14 - LOGM);
+
+constexpr int kSlotParts = 3;  // parts of a workgroup's scratch slot, 2 M floats each, a part of all slots together
+
+
+bool stream_is_capturing(hipStream_t stream) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
+// Twiddle tables (one per device and transform size) and the per-workgroup
+// scratch slots live for the life of the process.  They are made on first use,
+// or ahead of time by mega_fftconv_prepare; making them allocates and, for the
+// tables, synchronises the stream once, so that call cannot be captured into a
+// graph.  Scratch is three parts of 2*M floats per resident workgroup (kPerCu of
+// them per CU: 101 MB at every size).
+template <int LOGM>
+int get_tables(hipStream_t stream, const c32** out, float** scratch, int* slots) {
+  using C = Cfg<LOGM>;
+  int dev = 0;
+  MEGA_CHECK_HIP(hipGetDevice(&dev));
+  MEGA_CHECK_ARG(dev >= 0 && dev < kFftDevices, "device index %d not supported", dev);
+  std::lock_guard<std::mutex> lock(fft_tables.mu);
+  c32*& slot = fft_tables.ptr[dev][LOGM - 11];
+  if (slot == nullptr) {
+    hipDeviceProp_t prop;
+    MEGA_CHECK_HIP(hipGetDeviceProperties(&prop, dev));
+    fft_tables.slots[dev][LOGM - 11] = prop.multiProcessorCount * kPerCu<LOGM>;
+    c32* p = nullptr;
+    MEGA_CHECK_HIP(hipMalloc(reinterpret_cast<void**>(&p), sizeof(c32) * C::TABLE));
+    std::vector<c32> host(C::TABLE);
+    fill_tables<LOGM>(host.data());
+    hipError_t e = hipMemcpyAsync(p, host.data(), sizeof(c32) * C::TABLE, hipMemcpyHostToDevice, stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(stream);
+    if (e != hipSuccess) {
+      (void)hipFree(p);
+      return set_error(MEGA_ERR_HIP, "fftconv table init failed: %s", hipGetErrorString(e));
+    }
+    slot = p;
+  }
+  const int nslots = fft_tables.slots[dev][LOGM - 11];
+  std::vector<StreamScratch>& blocks = fft_tables.scratch[dev][LOGM - 11];
+  StreamScratch* mine = nullptr;
+  int open_blocks = 0;
+  for (StreamScratch& s : blocks) {
+    if (s.stream == stream) mine = &s;
+    open_blocks += s.pinned ? 0 : 1;
+  }
+  const bool capturing = stream_is_capturing(stream);
+  if (mine == nullptr && open_blocks >= kFftScratch && !capturing) {
+    // take over the block that has been idle longest, behind its last launch
+    for (StreamScratch& s : blocks)
+      if (!s.pinned && (mine == nullptr || s.tick < mine->tick)) mine = &s;
+    MEGA_CHECK_HIP(hipStreamWaitEvent(stream, mine->done, 0));
+    mine->stream = stream;
+  }
+  if (mine == nullptr) {
+    float* sc = nullptr;
+    hipEvent_t ev = nullptr;
+    MEGA_CHECK_HIP(hipMalloc(reinterpret_cast<void**>(&sc), sizeof(float) * kSlotParts * 2 * C::M * nslots));
+    hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    if (e != hipSuccess) {
+      (void)hipFree(sc);
+      return set_error(MEGA_ERR_HIP, "fftconv scratch event: %s", hipGetErrorString(e));
+    }
+    blocks.push_back(StreamScratch{stream, sc, ev, 0, false});
+    mine = &blocks.back();
+  }
+  mine->tick = ++fft_tables.tick;
+  if (capturing) mine->pinned = true;
+  *out = slot;
+  *scratch = mine->ptr;
+  *slots = nslots;
+  return MEGA_OK;
+}
+
+// Marks the end of the launches that used `stream`'s scratch block, so that a
+// later take-over can order itself behind them.  Not recorded under capture
+// (the block is pinned there).
+template <int LOGM>
+int scratch_used(hipStream_t stream) {
+  int dev = 0;
+  MEGA_CHECK_HIP(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lock(fft_tables.mu);
+  for (StreamScratch& s : fft_tables.scratch[dev][LOGM - 11])
+    if (s.stream == stream && !s.pinned) MEGA_CHECK_HIP(hipEventRecord(s.done, stream));
+  return MEGA_OK;
+}
+
+// uniform base + 32-bit unsigned byte offset (scalar-base addressing form)
+template <typename V>
+__device__ __forceinline__ V gld(const void* base, unsigned byte_off) {
+  return *reinterpret_cast<const V*>(static_cast<const char*>(base) + byte_off);
+}
+template <typename V>
+__device__ __forceinline__ void gst(void* base, unsigned byte_off, V v) {
+  *reinterpret_cast<V*>(static_cast<char*>(base) + byte_off) = v;
+}
+
+// A pair of adjacent elements as one 32/64-bit access.
+template <int DT> struct Pair;
+template <> struct Pair<MEGA_F32> {
+  using type = float2;
+  static __device__ __forceinline__ void unpack(type v, float& lo, float& hi) { lo = v.x; hi = v.y; }
+  static __device__ __forceinline__ type pack(float lo, float hi) { return make_float2(lo, hi); }
+};
+template <> struct Pair<MEGA_BF16> {
+  using type = uint32_t;
+  static __device__ __forceinline__ void unpack(type v, float& lo, float& hi) {
+    lo = __uint_as_float(v << 16);
+    hi = __uint_as_float(v & 0xffff0000u);
+  }
+  static __device__ __forceinline__ type pack(float lo, float hi) { return pack_bf16x2(lo, hi); }
+};
+template <> struct Pair<MEGA_F16> {
+  using type = uint32_t;
+  static __device__ __forceinline__ void unpack(type v, float& lo, float& hi) {
+    lo = f16_bits_to_float(static_cast<uint16_t>(v & 0xffffu));
+    hi = f16_bits_to_float(static_cast<uint16_t>(v >> 16));
+  }
+  static __device__ __forceinline__ type pack(float lo, float hi) {
+    return static_cast<uint32_t>(float_to_f16_bits(lo)) |
+           (static_cast<uint32_t>(float_to_f16_bits(hi)) << 16);
+  }
+};
+
+// The lane id, hidden from the optimiser: left alone it keeps the offsets of a row's 32 accesses in
+// registers from its load to its store, across both halves (with two waves per SIMD: 74 spilled).
+__device__ __forceinline__ int own_lane(int t) {
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
+// z[n] = s[2n] + i s[2n+1] of the zero-padded (optionally reversed) row.  Every lane reads inside the
+// row and takes zero for what lies behind it, so that the 32 loads stand in one piece without branches.
+// VEC: L is even and the row is pair-aligned, so (s[2n], s[2n+1]) is one access
+// addressed with a 32-bit offset from the wave-uniform row base.
+template <int LOGM, int DT, bool VEC>
+__device__ __forceinline__ void load_row(float* re, float* im, const void* row, int L, bool flip,
+                                         int lane) {
+  using C = Cfg<LOGM>;
+  const unsigned t = static_cast<unsigned>(own_lane(lane));
+  const unsigned count = VEC ? static_cast<unsigned>(L) >> 1 : static_cast<unsigned>(L), last = count - 1u;
+  const unsigned turn = flip ? ~0u : 0u, from = flip ? count : 0u;  // i or count - 1 - i
+  if (VEC) {
+    using P = typename Pair<DT>::type;
+    P raw[32];
+#pragma unroll
+    for (int j = 0; j < 32; ++j) {
+      const unsigned n = t + C::T * j;
+      raw[j] = gld<P>(row, (((n < last ? n : last) ^ turn) + from) * static_cast<unsigned>(sizeof(P)));
+    }
+#pragma unroll
+    for (int j = 0; j < 32; ++j) {
+      const bool in = t + C::T * j < count;
+      float lo, hi;
+      Pair<DT>::unpack(raw[j], lo, hi);
+      re[j] = in ? (flip ? hi : lo) : 0.f;
+      im[j] = in ? (flip ? lo : hi) : 0.f;
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 32; ++j) {
+      const unsigned m0 = 2u * (t + C::T * j), m1 = m0 + 1u;
+      const float a = ld<DT>(row, static_cast<int64_t>(((m0 < last ? m0 : last) ^ turn) + from));
+      const float b = ld<DT>(row, static_cast<int64_t>(((m1 < last ? m1 : last) ^ turn) + from));
+      re[j] = m0 < count ? a : 0.f;
+      im[j] = m1 < count ? b : 0.f;
+    }
+  }
+}
+
+// out[2n] = re[j], out[2n+1] = im[j] for n = t + T j (reversed when flip);
+// ACC adds to what is there (fp32 rows only).  With `res` non-null the stored
+// value is out[m] + w * res[m] (res has the dtype and layout of the output row).
+template <int LOGM, int DT, bool VEC, bool ACC>
+__device__ __forceinline__ void store_row(const float* re, const float* im, void* row, int L,
+                                          bool flip, int lane, const void* res = nullptr,
+                                          float w = 0.f) {
+  using C = Cfg<LOGM>;
+  const int t = own_lane(lane);
+  if (VEC) {
+    using P = typename Pair<DT>::type;
+    const unsigned half = static_cast<unsigned>(L) >> 1;
+#pragma unroll
+    for (int j = 0; j < 32; ++j) {
+      const unsigned n = static_cast<unsigned>(t) + C::T * j;
+      if (n < half) {
+        float lo = flip ? im[j] : re[j], hi = flip ? re[j] : im[j];
+        const unsigned off = (flip ? half - 1u - n : n) * static_cast<unsigned>(sizeof(P));
+        if (ACC) {
+          float plo, phi;
+          Pair<DT>::unpack(gld<P>(row, off), plo, phi);
+          lo += plo;
+          hi += phi;
+        }
+        if (res != nullptr) {
+          float rlo, rhi;
+          Pair<DT>::unpack(gld<P>(res, off), rlo, rhi);
+          lo = fmaf(w, rlo, lo);
+          hi = fmaf(w, rhi, hi);
+        }
+        gst<P>(row, off, Pair<DT>::pack(lo, hi));
+      }
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 32; ++j) {
+      const int m0 = 2 * (t + C::T * j), m1 = m0 + 1;
+      if (m0 < L) {
+        const int o = flip ? L - 1 - m0 : m0;
+        const float r = res != nullptr ? w * ld<DT>(res, o) : 0.f;
+        st<DT>(row, o, (ACC ? ld<DT>(row, o) + re[j] : re[j]) + r);
+      }
+      if (m1 < L) {
+        const int o = flip ? L - 1 - m1 : m1;
+        const float r = res != nullptr ? w * ld<DT>(res, o) : 0.f;
+        st<DT>(row, o, (ACC ? ld<DT>(row, o) + im[j] : im[j]) + r);
+      }
+    }
+  }
+}
+
+// Hides the table base from common-subexpression elimination / loop hoisting:
+// twiddles are re-read from L1/L2 at each use instead of being kept live in
+// registers across transforms (which would spill).
+__device__ __forceinline__ Tables launder(Tables tb) {
+  asm volatile("" : "+s"(tb.kr), "+s"(tb.kbo), "+s"(tb.kbe), "+s"(tb.kbo2));
+  asm volatile("" : "+s"(tb.kp2), "+s"(tb.ki3), "+s"(tb.kre), "+s"(tb.kro), "+s"(tb.pw));
+  return tb;
+}
+
+template <int LOGM, int H>
+__device__ __forceinline__ void forward_half(float* re, float* im, int t, const Tables& tb0,
+                                             float* lre, float* lim) {
+  const Tables tb = launder(tb0);
+  fwd_pass1<LOGM, H>(re, im, t, tb);
+  __syncthreads();
+  x1_write<LOGM>(re, im, t, lre, lim);
+  __syncthreads();
+  x1_read<LOGM>(re, im, t, lre, lim);
+  fwd_pass2<LOGM>(re, im, t, tb);
+  __syncthreads();
+  x2_write<LOGM>(re, im, t, lre, lim);
+  __syncthreads();
+  x2_read<LOGM, H>(re, im, t, lre, lim);
+  fwd_pass3<LOGM>(re, im);
+}
+
+template <int LOGM, int H>
+__device__ __forceinline__ void inverse_half(float* re, float* im, int t, const Tables& tb0,
+                                             float* lre, float* lim) {
+  const Tables tb = launder(tb0);
+  inv_pass3<LOGM, H>(re, im, t, tb);
+  __syncthreads();
+  ix2_write<LOGM, H>(re, im, t, lre, lim);
+  __syncthreads();
+  ix2_read<LOGM>(re, im, t, lre, lim);
+  inv_pass2<LOGM, H>(re, im, t, tb);
+  __syncthreads();
+  ix1_write<LOGM>(re, im, t, lre, lim);
+  __syncthreads();
+  ix1_read<LOGM>(re, im, t, lre, lim);
+  inv_pass1<H>(re, im);
+}
+
+// The lane's 32 values as they stand in its registers, to and from a part of the workgroup's scratch slot (2 M floats a part).
+template <int LOGM>
+__device__ __forceinline__ void keep(float* part, const float* re, const float* im, int t) {
+  using C = Cfg<LOGM>;
+#pragma unroll
+  for (int j = 0; j < 32; ++j) {
+    gst<float>(part, (j * C::T + t) * 4u, re[j]);
+    gst<float>(part, (C::M + j * C::T + t) * 4u, im[j]);
+  }
+}
+template <int LOGM, bool ADD>
+__device__ __forceinline__ void fetch(const float* part, float* re, float* im, int t) {
+  using C = Cfg<LOGM>;
+#pragma unroll
+  for (int j = 0; j < 32; ++j) {
+    const float a = gld<float>(part, (j * C::T + t) * 4u), b = gld<float>(part, (C::M + j * C::T + t) * 4u);
+    re[j] = ADD ? re[j] + a : a;
+    im[j] = ADD ? im[j] + b : b;
+  }
+}
+
+// Back from a product of spectra.  Half 0 leaves its M outputs zy[t + T j] in `part`; half 1 adds them and has the
+// sum in (re, im), zy[t + T j] at register j.
+template <int LOGM, int H>
+__device__ __forceinline__ void outputs(float* re, float* im, int t, const Tables& tb, float* lre, float* lim, float* part) {
+  inverse_half<LOGM, H>(re, im, t, tb, lre, lim);
+  float ore[32], oim[32];
+#pragma unroll
+  for (int j = 0; j < 32; ++j) {
+    ore[j] = re[out_pos<H>(j)];
+    oim[j] = im[out_pos<H>(j)];
+  }
+  if (H == 0) keep<LOGM>(part, ore, oim, t);
+  else fetch<LOGM, true>(part, ore, oim, t);
+#pragma unroll
+  for (int j = 0; j < 32; ++j) {
+    re[j] = ore[j];
+    im[j] = oim[j];
+  }
+}
+
+// The rows of a channel that a workgroup takes: two at a time, which then share the transform of k (MODE 0) or the
+// inverse transform of dk, whose spectrum is summed over them (MODE 1).  The kernels' time is the transforms' arithmetic
+// (87 % of the vector issue slots), so what counts is their number: 2.5 per row instead of 3.  In MODE 0 k's spectrum then has
+// to stay in registers to the row's end: 8 to 12 of them spill, at M = 16384 72 and with odd lengths' loads 26, where the
+// rows go one by one (PAIR 1), as a channel's only row does.  One kernel for dx and dk, with dy's spectrum formed once (4
+// transforms per row), spills 54 to 139 registers and takes 269 us where these two take 168.
+// bfloat16, forward / backward in us: 2 x 1024 rows of 8192 97 / 194 -> 86 / 168, 4 x 1024 of 8190 181 / 385 -> 158 / 325; of
+// channels whose rows now share out the chip for dk too: 8 x 256 of 8192 89 / 377 -> 82 / 169, 8 x 512 of 3001 120 / 541 -> 119 / 271.
+struct Rows {
+  int B, D, L;
+  int nb, groups;  // group g: channel g % D, rows g / D nb ..
+  int part;        // floats from a part of a slot to its next
+};
+
+// spectrum of a row's half H; SCALED: times 1 / (4 N) (E, O halves and the inverse), as one factor of every product is
+template <int LOGM, int DT, bool VEC, int H, bool SCALED>
+__device__ __forceinline__ void spectrum(float* re, float* im, const void* row, int L, bool flip, int t, const Tables& tb,
+                                         float* lre, float* lim) {
+  load_row<LOGM, DT, VEC>(re, im, row, L, flip, t);
+  forward_half<LOGM, H>(re, im, t, tb, lre, lim);
+  if (SCALED) {
+    constexpr float scale = 1.0f / (8.0f * Cfg<LOGM>::M);
+#pragma unroll
+    for (int j = 0; j < 32; ++j) {
+      re[j] *= scale;
+      im[j] *= scale;
+    }
+  }
+}
+
+// MODE 0: out[b,d,:] = conv(a[b,d,:], k[d,:]) (+ omega[d] a[b,d,:] when omega is given); `flip` reverses a on load and the
+//         result on store (backward dx).  a, out have dtype DT; b is k, fp32.
+// MODE 1: out[d,:] = sum_b reverse(conv(reverse(a[b,d,:]), x[b,d,:])), fp32 (backward dk); b is x.  `flip`: a channel's rows are
+//         shared by several workgroups, whose sums stand in their slots.
+template <int LOGM, int DT, int MODE, bool VEC, int H, int PAIR>
+__device__ __forceinline__ void conv_half(const void* a, const void* b, void* out, const Rows& rows, int d, int b0, int n, bool add,
+                                          int flip, const Tables& tb, float* lre, float* lim, float* scratch, const float* omega) {
+  using C = Cfg<LOGM>;
+  const int64_t pitch = static_cast<int64_t>(rows.L) * (DT == MEGA_F32 ? 4 : 2);
+  float pre[32], pim[32];
+  const int count = PAIR == 1 ? 1 : n;
+  if (MODE == 0) {
+    const int t = own_lane(threadIdx.x) & (C::T - 1);  // (restores the range so that offsets stay 32-bit)
+    spectrum<LOGM, MEGA_F32, VEC, H, true>(pre, pim, static_cast<const float*>(b) + static_cast<int64_t>(d) * rows.L, rows.L, false, t, tb, lre, lim);
+  }
+#pragma unroll 1
+  for (int i = 0; i < count; ++i) {
+    const int t = own_lane(threadIdx.x) & (C::T - 1);
+    const int64_t row = static_cast<int64_t>(b0 + i) * rows.D + d;
+    const char* arow = static_cast<const char*>(a) + row * pitch;
+    float re[32], im[32];
+    if (MODE == 1) spectrum<LOGM, DT, VEC, H, true>(pre, pim, static_cast<const char*>(b) + row * pitch, rows.L, false, t, tb, lre, lim);
+    spectrum<LOGM, DT, VEC, H, false>(re, im, arow, rows.L, MODE == 1 || flip != 0, t, tb, lre, lim);
+    pointwise<LOGM, H>(re, im, pre, pim, t, launder(tb));
+    // the slot's parts: half 0's outputs; of the second row, or (MODE 1) the spectrum so far; a shared channel's sum
+    if (MODE == 1) {
+      if (i > 0) fetch<LOGM, true>(scratch + rows.part, re, im, t);
+      if (i + 1 < count) {
+        keep<LOGM>(scratch + rows.part, re, im, t);
+        continue;
+      }
+    }
+    outputs<LOGM, H>(re, im, t, tb, lre, lim, MODE == 0 ? scratch + i * rows.part : scratch);
+    if (H == 1 && MODE == 0)
+      store_row<LOGM, DT, VEC, false>(re, im, static_cast<char*>(out) + row * pitch, rows.L, flip != 0, t,
+                                      omega != nullptr ? arow : nullptr, omega != nullptr ? omega[d] : 0.f);
+    if (H == 1 && MODE == 1) {
+      float* sum = flip ? scratch + 2 * rows.part : static_cast<float*>(out) + static_cast<int64_t>(d) * rows.L;
+      if (add) store_row<LOGM, MEGA_F32, VEC, true>(re, im, sum, rows.L, true, t);
+      else store_row<LOGM, MEGA_F32, VEC, false>(re, im, sum, rows.L, true, t);
+    }
+  }
+}
+template <int LOGM, int DT, int MODE, bool VEC, int PAIR>
+__global__ __launch_bounds__(Cfg<LOGM>::T, 2) void fftconv_kernel(
+    const void* __restrict__ a, const void* __restrict__ b, void* __restrict__ out, const Rows rows, int flip,
+    const c32* __restrict__ tab, float* __restrict__ scratch_all, const float* __restrict__ omega) {
+  extern __shared__ __align__(16) float lds[];
+  float *lre = lds, *lim = lds + Cfg<LOGM>::PLANE;
+  const Tables tb = make_tables<LOGM>(tab);
+  float* scratch = scratch_all + blockIdx.x * 2 * Cfg<LOGM>::M;
+  for (int g = blockIdx.x; g < rows.groups; g += gridDim.x) {
+    const int d = g % rows.D, first = g / rows.D * rows.nb, end = min(rows.B, first + rows.nb);
+    for (int b0 = first; b0 < end; b0 += PAIR) {
+      const int n = min(PAIR, end - b0);
+      conv_half<LOGM, DT, MODE, VEC, 0, PAIR>(a, b, out, rows, d, b0, n, b0 > first, flip, tb, lre, lim, scratch, omega);
+      conv_half<LOGM, DT, MODE, VEC, 1, PAIR>(a, b, out, rows, d, b0, n, b0 > first, flip, tb, lre, lim, scratch, omega);
+    }
+  }
+}
+// dk of channels whose rows several workgroups took, from their slots in order
+__global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict__ scratch, float* __restrict__ dk, const Rows rows, int slot) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= static_cast<int64_t>(rows.D) * rows.L) return;
+  const int d = static_cast<int>(i / rows.L), m = static_cast<int>(i % rows.L);
+  float sum = 0.f;
+  for (int g = d; g < rows.groups; g += rows.D) sum += scratch[2 * static_cast<int64_t>(rows.part) + static_cast<int64_t>(g) * slot + m];
+  dk[i] = sum;
+}
+
+// How a launch shares out its rows: the rows of a channel that a group takes are chosen for the shortest line of
+// transforms, in halves of one, that a workgroup slot gets (5 for a pair of rows, 3 for a row alone).  `bound`: a channel's sum
+// stands in its groups' slots, so that there may be no more groups than slots, unless a group has the channel to itself.
+Rows make_rows(int64_t B, int64_t D, int64_t L, int slots, int part, int pair, bool bound) {
+  int64_t best = B, least = -1;
+  for (int64_t nb = 1; nb <= B; ++nb) {
+    const int64_t groups = D * ((B + nb - 1) / nb);
+    if (bound && nb < B && groups > slots) continue;
+    const int64_t cost = (groups + slots - 1) / slots * (pair == 2 ? nb / 2 * 5 + nb % 2 * 3 : nb * 3);
+    if (least < 0 || cost < least) best = nb, least = cost;
+  }
+  return Rows{static_cast<int>(B), static_cast<int>(D), static_cast<int>(L), static_cast<int>(best), static_cast<int>(D * ((B + best - 1) / best)), part};
+}
+
+template <int LOGM, int DT, int MODE, bool VEC, int PAIR>
+int launch_rows(const void* a, const void* b, void* out, const Rows& rows, int flip, const float* omega, const c32* tab, float* scratch,
+                int slots, hipStream_t stream) {
+  const size_t lds_bytes = sizeof(float) * 2 * Cfg<LOGM>::PLANE;
+  MEGA_CHECK_HIP(hipFuncSetAttribute(
+      reinterpret_cast<const void*>(&fftconv_kernel<LOGM, DT, MODE, VEC, PAIR>),
+      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
+  fftconv_kernel<LOGM, DT, MODE, VEC, PAIR><<<dim3(static_cast<unsigned>(std::min(rows.groups, slots))), Cfg<LOGM>::T, lds_bytes, stream>>>(
+      a, b, out, rows, flip, tab, scratch, omega);
+  MEGA_CHECK_LAUNCH();
+  return MEGA_OK;
+}
+
+template <int LOGM, int DT, int MODE, bool VEC>
+int launch_fft_v(const void* a, const void* b, void* out, int64_t B, int64_t D, int64_t L, int flip, const float* omega, hipStream_t stream) {
+  using C = Cfg<LOGM>;
+  const c32* tab = nullptr;
+  float* scratch = nullptr;
+  int slots = 0;
+  int rc = get_tables<LOGM>(stream, &tab, &scratch, &slots);
+  if (rc != MEGA_OK) return rc;
+  MEGA_CHECK_ARG(B * D <= 0x7fffffff, "fftconv: too many rows");
+  constexpr int kMost = MODE == 0 && (LOGM == 14 || !VEC) ? 1 : 2;
+  const Rows rows = make_rows(B, D, L, slots, slots * 2 * C::M, kMost, MODE == 1);
+  const bool split = MODE == 1 && rows.nb < B;
+  const int how = MODE == 1 ? split : flip;
+  if (kMost == 1 || rows.nb == 1) rc = launch_rows<LOGM, DT, MODE, VEC, 1>(a, b, out, rows, how, omega, tab, scratch, slots, stream);
+  else rc = launch_rows<LOGM, DT, MODE, VEC, kMost>(a, b, out, rows, how, omega, tab, scratch, slots, stream);
+  if (rc != MEGA_OK) return rc;
+  if (split) {
+    split_sum_kernel<<<dim3(static_cast<unsigned>((D * L + 255) / 256)), 256, 0, stream>>>(scratch, static_cast<float*>(out), rows, 2 * C::M);
+    MEGA_CHECK_LAUNCH();
+  }
+  return scratch_used<LOGM>(stream);
+}
+
+template <int LOGM, int DT, int MODE>
+int launch_fft(const void* a, const void* b, void* out, int64_t B, int64_t D, int64_t L, int flip,
+               const float* omega, hipStream_t stream) {
+  const auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 8 == 0; };
+  const bool vec = (L % 2 == 0) && al(a) && al(b) && al(out);
+  return vec ? launch_fft_v<LOGM, DT, MODE, true>(a, b, out, B, D, L, flip, omega, stream)
+             : launch_fft_v<LOGM, DT, MODE, false>(a, b, out, B, D, L, flip, omega, stream);
+}
+
+}  // namespace
+
+template <int LOGM>
+int fftconv_rows(int dtype, int mode, const void* a, const void* b, void* out, int64_t B, int64_t D, int64_t L, int flip,
+                 const float* omega, hipStream_t stream) {
+  switch (2 * dtype + mode) {
+    case 2 * MEGA_F32: return launch_fft<LOGM, MEGA_F32, 0>(a, b, out, B, D, L, flip, omega, stream);
+    case 2 * MEGA_F32 + 1: return launch_fft<LOGM, MEGA_F32, 1>(a, b, out, B, D, L, flip, omega, stream);
+    case 2 * MEGA_BF16: return launch_fft<LOGM, MEGA_BF16, 0>(a, b, out, B, D, L, flip, omega, stream);
+    case 2 * MEGA_BF16 + 1: return launch_fft<LOGM, MEGA_BF16, 1>(a, b, out, B, D, L, flip, omega, stream);
+    case 2 * MEGA_F16: return launch_fft<LOGM, MEGA_F16, 0>(a, b, out, B, D, L, flip, omega, stream);
+    default: return launch_fft<LOGM, MEGA_F16, 1>(a, b, out, B, D, L, flip, omega, stream);
+  }
+}
+template <int LOGM>
+int fftconv_tables(hipStream_t stream) {
+  const c32* tab = nullptr;
+  float* scratch = nullptr;
+  int slots = 0;
+  return get_tables<LOGM>(stream, &tab, &scratch, &slots);
+}
+template int fftconv_rows<MEGA_FFTCONV_LOGM>(int, int, const void*, const void*, void*, int64_t, int64_t, int64_t, int, const float*, hipStream_t);
+template int fftconv_tables<MEGA_FFTCONV_LOGM>(hipStream_t);
+#endif  // MEGA_FFTCONV_LOGM
+
+}  // namespace mega
