@@ -70,6 +70,31 @@ __device__ __forceinline__ u32x4 split8_third(const float* v, u32x4 hi, u32x4 lo
                            (v[2 * e + 1] - __uint_as_float(hi[e] & 0xffff0000u)) - __uint_as_float(lo[e] & 0xffff0000u));
   return third;
 }
+// The operand blocks of a channel's powers are written by the threads that form the powers, thread (n, a) those of mode n
+// with four exponents.  Four columns 4 quad .. 4 quad + 3 of row m of four blocks (rows m, k-steps of 16 columns):
+template <bool THIRD>
+__device__ __forceinline__ void put_columns(u32x4 (*blocks)[2][kWave], u32x4 (*third)[kWave], int m, int quad, const float* v) {
+  const int blk = quad >> 2, ln = m + 32 * ((quad >> 1) & 1), half = quad & 1;
+  uint2 hi, lo, rest;
+  uint32_t *const h = &hi.x, *const l = &lo.x, *const t = &rest.x;
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    h[e] = pack_bf16x2(v[2 * e], v[2 * e + 1]);
+    const float r0 = v[2 * e] - __uint_as_float(h[e] << 16), r1 = v[2 * e + 1] - __uint_as_float(h[e] & 0xffff0000u);
+    l[e] = pack_bf16x2(r0, r1);
+    if (THIRD) t[e] = pack_bf16x2(r0 - __uint_as_float(l[e] << 16), r1 - __uint_as_float(l[e] & 0xffff0000u));
+  }
+  reinterpret_cast<uint2*>(&blocks[blk][0][ln])[half] = hi;
+  reinterpret_cast<uint2*>(&blocks[blk][1][ln])[half] = lo;
+  if (THIRD) reinterpret_cast<uint2*>(&third[blk][ln])[half] = rest;
+}
+// ... and the columns 2 n, 2 n + 1 of row i of four blocks (row tile of 32, k-step of 16 columns)
+__device__ __forceinline__ void put_pair(u32x4 (*blocks)[2][kWave], int n, int i, float a, float b) {
+  const int blk = 2 * (i >> 5) + (n >> 3), ln = (i & 31) + 32 * ((n >> 2) & 1);
+  const uint32_t h = pack_bf16x2(a, b);
+  reinterpret_cast<uint32_t*>(&blocks[blk][0][ln])[n & 3] = h;
+  reinterpret_cast<uint32_t*>(&blocks[blk][1][ln])[n & 3] = pack_bf16x2(a - __uint_as_float(h << 16), b - __uint_as_float(h & 0xffff0000u));
+}
 // Third pieces of k[0 .. 63] for the Toeplitz blocks, whose lanes read eight consecutive lags each: one table of the
 // lags in the blocks' order, zeros at negative ones, and a second one that starts an element later, so that every
 // lane reads whole words.
@@ -283,24 +308,27 @@ constexpr int kFwdBlocks = 12;
 
 // ONE: a workgroup takes one item (at most four tiles) and ends.  Setting up its channel is a chain of short phases
 // with a barrier between them, so what counts is how many workgroups share a compute unit: without the blocks of K,
-// whose lags are read out of a table of 96 instead, four fit (128 registers a lane: nothing is loaded ahead).
+// whose lags are read out of a table of 96 instead, four fit (128 registers a lane: nothing is loaded ahead).  Half of the
+// rest is the issue of vector instructions, 500 a wave: the threads that form the powers write the operand blocks of P and
+// Q themselves (no table between), and a wave without a tile does nothing but its share of the set-up.  Rows of 2048
+// float32 steps of 1024 channels: 15.8 us three to a compute unit with a launch for the coefficients, 11.2 four, 9.9 so;
+// 4096 channels of 1531 bfloat16 steps with their last state 51 -> 34, of 2048 31 -> 25, of 4088 54 -> 35.
 template <bool ONE>
 struct FwdSmemOf {
   static constexpr int NC = kWaves * 32;       // chunks resident
-  static constexpr int kBlocks = ONE ? 8 : kFwdBlocks;
+  static constexpr int kBlocks = ONE ? 8 : kFwdBlocks, kQ = kBlocks - 4;
   union {
     float klocal[kT];                          // k[0 .. 63] (+ omega at lag 0), while a row is set up
     cf sub_end[kWaves * 3][16];                // local end state of each sub-segment but a wave's last
   };
   float pn[16];
   cf gn[16];
-  cf wave_end[2][kWaves][16];                  // local end state of each wave's 4 sub-segments, by item parity
+  cf wave_end[ONE ? 1 : 2][kWaves][16];        // local end state of each wave's 4 sub-segments, by item parity
   float wave_cin[kWaves][32];                  // state in front of each wave's first chunk
   cf carry[2][16];
   cf pw[12][16];                               // q^(4 k), q^(16 k) (k < 4), q, q^64, q^(64 CPS), q^(256 CPS)
   u32x4 aop[kBlocks][2][kWave];                // ONE: P, then Q
-  // row 1 + c: state after chunk c of the segment; while a row is set up the buffer holds the
-  // power table q_n^e, e = 0 .. 64 (16 x 66 complex), from which the operand blocks are built
+  // row 1 + c: state after chunk c of the segment
   float H[(NC + 1) * kHP];
 };
 struct FwdSmem : FwdSmemOf<false> {};
@@ -313,12 +341,11 @@ struct FwdSmemOne : FwdSmemOf<true> {
   alignas(4) ThirdTable kpiece[2];
 };
 struct FwdSmemOneFine : FwdSmemOne {
-  u32x4 third[4][kWave];
-  alignas(4) ThirdTable kthird;
+  alignas(4) ThirdTable kthird;  // (third pieces of P: in registers)
 };
-static_assert(sizeof(cf) * 16 * (kT + 2) <= sizeof(float) * (kWaves * 32 + 1) * kHP, "the power table fits the state buffer");
+static_assert(sizeof(u32x4) * 4 * kWave <= sizeof(float) * (kWaves * 32 + 1) * kHP, "the third pieces of P pass through the state buffer");
 static_assert(3 * sizeof(FwdSmemFine) <= 160 * 1024, "three workgroups per compute unit");
-static_assert(4 * sizeof(FwdSmemOne) <= 160 * 1024 && 3 * sizeof(FwdSmemOneFine) <= 160 * 1024, "four (three) workgroups per compute unit");
+static_assert(4 * sizeof(FwdSmemOneFine) <= 160 * 1024, "four workgroups per compute unit");
 
 // The channels' coefficients: p, log q, gamma in float32, or, where `alpha` is not null, the layer's raw parameters of element type
 // `dtype`, turned into them as mega_cema_layer_coeffs_fwd does.
@@ -402,7 +429,7 @@ __device__ __forceinline__ void tile_backward(const Lines& ln, Tile& w, int tile
 __device__ __forceinline__ void wave_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 template <int DT, int ROWS, bool ONE>
-__global__ __launch_bounds__(kThreads, ONE && !kFine<ROWS> ? 4 : 3) void cema_scan_fwd_kernel(
+__global__ __launch_bounds__(kThreads, ONE ? 4 : 3) void cema_scan_fwd_kernel(
     const void* __restrict__ x, void* __restrict__ y, const Coeffs co,
     const cf* __restrict__ h0, cf* __restrict__ h_last, const Lines ln, int N) {
   constexpr bool FINE = kFine<ROWS>;
@@ -411,7 +438,6 @@ __global__ __launch_bounds__(kThreads, ONE && !kFine<ROWS> ? 4 : 3) void cema_sc
   constexpr int NC = Smem::NC, CPS = NC / kSubs, XP = XOp<DT>::XP;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Smem& sm = *reinterpret_cast<Smem*>(smem_raw);
-  cf (*qp)[kT + 2] = reinterpret_cast<cf(*)[kT + 2]>(sm.H);  // while a row is set up
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int g = lane >> 5, r = lane & 31;
   // scan roles: mode sn; sub-segment sa = 4 wave + sl of CPS chunks, inside the wave's own tiles
@@ -446,6 +472,8 @@ __global__ __launch_bounds__(kThreads, ONE && !kFine<ROWS> ? 4 : 3) void cema_sc
     return rp;
   };
 
+  u32x4 (*passed)[kWave] = reinterpret_cast<u32x4(*)[kWave]>(sm.H);  // ONE and FINE, setup only: third pieces of P
+  u32x4 third_p[4];
   cf qT{0.f, 0.f}, qS{0.f, 0.f}, qW{0.f, 0.f};
   int cur = 0, par = 0;
   RowParams rp = fetch_params(blockIdx.x);
@@ -490,19 +518,35 @@ __global__ __launch_bounds__(kThreads, ONE && !kFine<ROWS> ? 4 : 3) void cema_sc
     cur = 0;
     __syncthreads();
     {
-      // q^(4 sa + e), e < 4, and this mode's share of k at those lags, summed over the
-      // 16 modes (the 16 lanes of a row): the skip term omega x rides on k[0]
-      cf v = cmul(sm.pw[sa & 3][sn], sm.pw[4 + (sa >> 2)][sn]);
+      // q^(4 sa + e), e < 4, and this mode's share of k at those lags, summed over the 16 modes (the 16 lanes of a row):
+      // the skip term omega x rides on k[0].  They are this thread's columns of P, and with q^(4 sa + 4) its rows of Q.
+      cf v[5];
+      v[0] = cmul(sm.pw[sa & 3][sn], sm.pw[4 + (sa >> 2)][sn]);
+      v[4] = sa == 15 ? sm.pw[9][sn] : cmul(sm.pw[(sa + 1) & 3][sn], sm.pw[4 + (((sa + 1) >> 2) & 3)][sn]);
       const cf q1 = sm.pw[8][sn];
       const cf c{rp.pv * rp.gv.x, rp.pv * rp.gv.y};
+      const int id = opaque(tid), n = id & 15, quad = id >> 4;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        qp[sn][4 * sa + e] = v;
-        const float kl = group_sum<16>(c.x * v.x - c.y * v.y);
+        if (e > 0) v[e] = cmul(v[e - 1], q1);
+        const float kl = group_sum<16>(c.x * v[e].x - c.y * v[e].y);
         if (sn == 0) sm.klocal[4 * sa + e] = (sa == 0 && e == 0) ? kl + rp.w : kl;
-        v = cmul(v, q1);
       }
-      if (sa == 15) qp[sn][kT] = sm.pw[9][sn];
+      u32x4 (*third)[kWave] = nullptr;
+      if constexpr (FINE && ONE) third = passed;
+      else if constexpr (FINE) third = sm.third;
+#pragma unroll
+      for (int part = 0; part < 2; ++part) {  // step j has the exponent 63 - j
+        float pv[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pv[e] = rp.pv * (part ? v[3 - e].y : v[3 - e].x);
+        put_columns<FINE>(sm.aop, third, 2 * n + part, 15 - quad, pv);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const cf w = cmul(rp.gv, v[e + 1]);
+        put_pair(sm.aop + Smem::kQ, n, 4 * quad + e, w.x, -w.y);
+      }
       qT = sm.pw[9][sn];
       qS = sm.pw[10][sn];
       qW = sm.pw[11][sn];
@@ -510,43 +554,25 @@ __global__ __launch_bounds__(kThreads, ONE && !kFine<ROWS> ? 4 : 3) void cema_sc
     RowParams next_rp{};
     if constexpr (!ONE) next_rp = fetch_params(group + static_cast<int>(gridDim.x));
     __syncthreads();
-    for (int item = tid; item < Smem::kBlocks * kWave; item += kThreads) {
-      const int at = item >> 6, blk = ONE && at >= 4 ? at + 4 : at, ln = item & 63, rr = ln & 31, gg = ln >> 5;
+    if constexpr (!ONE) {
+      const int b = wave, id = opaque(lane), rr = id & 31, gg = id >> 5, o = 16 * (b - 1);
       float v[8];
-      if (blk < 4) {
-        const int n = rr >> 1, part = rr & 1;
-        const float pp = sm.pn[n];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const cf w = qp[n][kT - 1 - (16 * blk + 8 * gg + e)];
-          v[e] = pp * (part ? w.y : w.x);
-        }
-      } else if (blk < 8) {
-        const int o = 16 * (blk - 5);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int lag = o + rr - 8 * gg - e;
-          const float kv = sm.klocal[lag >= 0 ? lag : 0];  // read, then masked: no branch around the load
-          v[e] = lag >= 0 ? kv : 0.f;
-        }
-      } else {
-        const int it = (blk - 8) >> 1, s2 = (blk - 8) & 1, i = 32 * it + rr;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int m = 16 * s2 + 8 * gg + e, n = m >> 1;
-          const cf w = cmul(sm.gn[n], qp[n][i + 1]);
-          v[e] = (m & 1) ? -w.y : w.x;
-        }
+      for (int e = 0; e < 8; ++e) {
+        const int lag = o + rr - 8 * gg - e;
+        const float kv = sm.klocal[lag >= 0 ? lag : 0];  // read, then masked: no branch around the load
+        v[e] = lag >= 0 ? kv : 0.f;
       }
       u32x4 hi, lo;
       split8(v, hi, lo);
-      sm.aop[at][0][ln] = hi;
-      sm.aop[at][1][ln] = lo;
-      if constexpr (FINE)
-        if (blk < 4) sm.third[blk][ln] = split8_third(v, hi, lo);
+      sm.aop[4 + b][0][lane] = hi;
+      sm.aop[4 + b][1][lane] = lo;
     }
     if constexpr (ONE) fill_pieces(sm.kpiece[0], sm.kpiece[1], sm.klocal, tid);
     if constexpr (FINE) fill_thirds<true>(sm.kthird, sm.klocal, tid);
+    if constexpr (FINE && ONE)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) third_p[s] = passed[s][lane];
     __syncthreads();
     rp = next_rp;
   };
@@ -575,20 +601,28 @@ __global__ __launch_bounds__(kThreads, ONE && !kFine<ROWS> ? 4 : 3) void cema_sc
 #pragma unroll
         for (int s = 0; s < 4; ++s) xb[s].keep(at + 16 * s, w.lo, w.hi);
       }
+    // a wave behind the line's end only keeps the barriers (of several items it is the last that has any: not worth the registers)
+    const bool on = w.nc > 0, runs = !ONE || on, ends = on && h_last != nullptr && w.base + w.hi == (w.row + 1) * ln.L;
+    const int cl = w.nc - 1, rem = w.hi - cl * kT;  // the tile's last chunk, 1 .. 64 steps in it
+    // those steps, for the state after them: a lane each
+    auto load_end = [&] { return ends && lane < rem ? Elem<DT>::load(static_cast<const typename Elem<DT>::type*>(x) + w.base + cl * kT + lane) : 0.f; };
+    float x_end = 0.f;
+    if constexpr (ONE) x_end = load_end();
     floatx16 yacc[2];
     // ---- local states S = P X, into this wave's own rows of the state buffer ----------
-    {
+    if (runs) {
       u32x4 P[4][2];
 #pragma unroll
       for (int s = 0; s < 4; ++s) load_block(s, P[s]);
-      if (w.nc > 0) {
+      if (on) {
         floatx16 acc;
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[i] = 0.f;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
           acc = mma_split<XP, FINE>(P[s], xb[s].pc, acc);
-          if constexpr (FINE) acc = mfma_bf16(sm.third[s][lane], xb[s].pc[0], acc);
+          if constexpr (FINE && ONE) acc = mfma_bf16(third_p[s], xb[s].pc[0], acc);
+          else if constexpr (FINE) acc = mfma_bf16(sm.third[s][lane], xb[s].pc[0], acc);
         }
         float* dst = sm.H + (1 + c0 + r) * kHP + 4 * g;
 #pragma unroll
@@ -599,7 +633,7 @@ __global__ __launch_bounds__(kThreads, ONE && !kFine<ROWS> ? 4 : 3) void cema_sc
     }
     // ---- the within-chunk part of the outputs, K X (omega x included: K carries omega on
     //      its diagonal); the accumulators wait for the state part ------------------------
-    {
+    if (runs) {
       u32x4 K[4][2];
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
@@ -614,7 +648,7 @@ __global__ __launch_bounds__(kThreads, ONE && !kFine<ROWS> ? 4 : 3) void cema_sc
       for (int it = 0; it < 2; ++it) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) yacc[it][i] = 0.f;
-        if (w.nc > 0) {
+        if (on) {
 #pragma unroll
           for (int s = 0; s < 2 + 2 * it; ++s) {
             const int b = 1 + 2 * it - s;
@@ -633,16 +667,16 @@ __global__ __launch_bounds__(kThreads, ONE && !kFine<ROWS> ? 4 : 3) void cema_sc
     wave_sync();
     // ---- scan over the chunks: a sub-segment per 16 lanes, the wave's four sub-segments are its
     //      own chunks; one workgroup barrier hands over the waves' ends ---------------------------
-    {
-      float* col = sm.H + kHP + 2 * sn;  // state column n of row 1 + c
-      float2 sv[CPS];                    // the sub-segment's local states, kept for the second pass
+    float* const col = sm.H + kHP + 2 * sn;  // state column n of row 1 + c
+    float2 sv[CPS];                          // the sub-segment's local states, kept for the second pass
+    cf h{0.f, 0.f};
+    if (runs) {
 #pragma unroll
       for (int i = 0; i < CPS; ++i) {
         const int c = sa * CPS + i;
         const float2 s0 = *reinterpret_cast<const float2*>(col + c * kHP);  // read, then masked
         sv[i] = sl * CPS + i < w.nc ? s0 : make_float2(0.f, 0.f);
       }
-      cf h{0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < CPS; ++i) h = cadd(cmul(qT, h), cf{sv[i].x, sv[i].y});
       if (sl < 3) sm.sub_end[3 * wave + sl][sn] = h;
@@ -653,7 +687,9 @@ __global__ __launch_bounds__(kThreads, ONE && !kFine<ROWS> ? 4 : 3) void cema_sc
         e = cadd(cmul(qS, e), sm.sub_end[3 * wave + 2][sn]);
         sm.wave_end[par][wave][sn] = cadd(cmul(qS, e), h);
       }
-      lds_barrier();
+    }
+    lds_barrier();
+    if (runs) {
       cf cin = ONE ? cf{0.f, 0.f} : sm.carry[cur][sn];
       // through the tiles in front of this wave's, from the first one of its row if that is among the
       // four (there the carried state enters)
@@ -679,11 +715,11 @@ __global__ __launch_bounds__(kThreads, ONE && !kFine<ROWS> ? 4 : 3) void cema_sc
     }
     wave_sync();
     // ---- the state part of the outputs, Q H[c-1], and the stores ------------------------------
-    {
+    if (runs) {
       u32x4 Q[4][2];
 #pragma unroll
-      for (int b = 0; b < 4; ++b) load_block((ONE ? 4 : 8) + b, Q[b]);
-      if (w.nc > 0) {
+      for (int b = 0; b < 4; ++b) load_block(Smem::kQ + b, Q[b]);
+      if (on) {
         u32x4 hb[2][2];
         // the state in front of chunk c0 + r: the previous row of the buffer, or, for the
         // wave's first chunk, what the scan left in wave_cin
@@ -724,25 +760,24 @@ __global__ __launch_bounds__(kThreads, ONE && !kFine<ROWS> ? 4 : 3) void cema_sc
     }
     cur ^= 1;
     par ^= 1;
-    if (w.hi > 0 && w.base + w.hi == (w.row + 1) * ln.L && h_last != nullptr && (FINE || lane < N)) {
+    if (ends) {  // (every lane: they pass each other the steps)
       // the state after step L - 1 (the row's last chunk may be partial), from this wave's own rows
-      const typename Elem<DT>::type* xrow = static_cast<const typename Elem<DT>::type*>(x) + w.base;
-      const int cl = w.nc - 1;           // the last chunk inside the tile
-      const int rem = w.hi - cl * kT;    // 1 .. 64 steps in it
+      if constexpr (!ONE) x_end = load_end();
       if constexpr (FINE) {
         // q^rem h + p sum_e q^e x[rem - 1 - e], h the state in front of that chunk; lane (n, a) = (lane % 16, lane / 16) adds
         // up the exponents 16 a .. 16 a + 15 of mode n.  (Step by step the rounding of q alone costs 1e-6 over a chunk.)
         const int first = cl == 0 ? w.lo : 0, n = lane & 15, a = lane >> 4;
         const cf q1 = sm.pw[8][n];
         cf t{0.f, 0.f};
-#pragma unroll 1
+#pragma unroll(ONE ? 4 : 1)
         for (int k = 0; k < 4; ++k) {
           cf v{0.f, 0.f};
 #pragma unroll
           for (int e = 3; e >= 0; --e) {
             const int j = rem - 1 - (16 * a + 4 * k + e);
+            const float xv = __shfl(x_end, j & 63, 64);
             v = cmul(q1, v);
-            if (j >= first) v.x += Elem<DT>::load(xrow + cl * kT + j);
+            if (j >= first) v.x += xv;
           }
           t = cadd(t, cmul(sm.pw[k][n], v));
         }
@@ -757,24 +792,24 @@ __global__ __launch_bounds__(kThreads, ONE && !kFine<ROWS> ? 4 : 3) void cema_sc
         const cf h = cmul(qr, cf{prev[0], prev[1]});
         if (lane < N) h_last[w.row * N + lane] = cf{h.x + sm.pn[n] * t.x, h.y + sm.pn[n] * t.y};
       } else {
+        const int n = lane & 15;
         cf h;
         if (rem == kT) {
-          const float* lastrow = sm.H + (1 + c0 + cl) * kHP + 2 * lane;
+          const float* lastrow = sm.H + (1 + c0 + cl) * kHP + 2 * n;
           h = cf{lastrow[0], lastrow[1]};
         } else {
-          const float* prev = cl == 0 ? sm.wave_cin[wave] + 2 * lane : sm.H + (c0 + cl) * kHP + 2 * lane;
-          // the recurrence itself over the last chunk's steps (the power table has made way for
-          // the states by now): h <- q h + p x
+          const float* prev = cl == 0 ? sm.wave_cin[wave] + 2 * n : sm.H + (c0 + cl) * kHP + 2 * n;
+          // the recurrence itself over the last chunk's steps: h <- q h + p x
           h = cf{prev[0], prev[1]};
-          const cf q1 = sm.pw[8][lane];
-          const float pp = sm.pn[lane];
+          const cf q1 = sm.pw[8][n];
+          const float pp = sm.pn[n];
           for (int j = 0; j < rem; ++j) {
-            const float xv = Elem<DT>::load(xrow + cl * kT + j) * pp;
+            const float xv = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x_end), j)) * pp;
             h = cmul(q1, h);
             h.x += xv;
           }
         }
-        h_last[w.row * N + lane] = h;
+        if (lane < N) h_last[w.row * N + lane] = h;
       }
     }
   };
@@ -825,7 +860,7 @@ int launch_fwd_as(const void* x, void* y, const Coeffs& co, const cf* h0, cf* h_
 int lines_of(int64_t B, int64_t D, int64_t L, int rows, Lines* ln, int64_t* slots, bool* one) {
   int cus = 0;
   if (const int rc = compute_units(&cus); rc != MEGA_OK) return rc;
-  *slots = (rows == kWhole ? 4 : 3) * static_cast<int64_t>(cus);  // workgroups that fit the chip
+  *slots = 4 * static_cast<int64_t>(cus);  // workgroups that fit the chip
   *ln = make_lines(B, D, L, *slots, false, rows);
   *one = ln->nb * static_cast<int64_t>(ln->tpr) <= kWaves;
   if (!*one) {

@@ -4,7 +4,9 @@ the bits have to be: of the same channels in longer rows, in batches of any size
 import pytest
 import torch
 
+from conftest import rel_err
 from megalodon_amd.modules import MultiHeadComplexEMA
+from oracle import cema as ocema
 
 pytestmark = pytest.mark.gpu
 
@@ -52,3 +54,24 @@ def test_with_and_without_gradients(L, dtype, params):
         y, h = layer(x, None, True)  # the branch with a last state: coefficients from their own launch
     assert torch.equal(y, want) and torch.isfinite(torch.view_as_real(h)).all()
     assert torch.equal(layer(x.requires_grad_(True))[0].detach(), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("L", [8, 64, 72, 1984, 2040, 2048, 2056, 4088])
+def test_state_behind_the_last_step(L, dtype):
+    """The lanes hand each other the steps of the last chunk: full, of one step, and of most; the last chunk of a tile, the
+    first, and rows that leave waves without a tile.  Rows alone and in a batch: the same bits; the 16-bit rows of a length
+    that is one step shorter likewise.  Bar against float64: the operands' two bf16 pieces, 2^-16, over a sum of terms of
+    either sign, which cost some digits (1e-4, as for every state)."""
+    lengths = [L] if dtype == torch.float32 else [L, L - 1]
+    for steps in lengths:
+        layer, x = _layer(256, 16, torch.float32), _rows(20, 256, steps, dtype)
+        with torch.no_grad():
+            batch = layer(x, None, True)[1]
+            alone = torch.cat([layer(x[b:b + 1], None, True)[1] for b in range(4)])
+        assert torch.equal(torch.view_as_real(batch[:4]), torch.view_as_real(alone))
+        pick = slice(0, None, 51)
+        pr = {n: getattr(layer, n).detach().cpu().double()[pick] for n in ("alpha", "delta", "theta", "gamma")}
+        p, q, _ = ocema.calc_coeffs(pr["alpha"], pr["delta"], pr["theta"], pr["gamma"], 16)
+        want = ocema.ema_hidden_fwd(x[:4, pick].cpu().double(), p, q.log(), None)
+        assert rel_err(alone[:, pick], want) <= 1e-4
