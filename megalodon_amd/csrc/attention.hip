@@ -130,6 +130,11 @@ struct GemmParams {
   const uint16_t* bias_of[2];
   int size[2], start[2];
   int kva;      // as kvb, for a k-major A (LIN: rows behind it are not there; else they hold zeros)
+  // CUT: items full .. items - 1, fewer than there are CUs, are cut along k into `cut` parts; float32 sums of part i
+  // of item full + r at parts + (r cut + i) 256 x 256, as the waves hold them (linear_parts_kernel adds them up).
+  int full, cut;
+  float* parts;
+  int split_ok;  // (the launcher's: there is memory for the parts)
   int n_group;  // plain schedule: tiles numbered n fastest inside bands of n_group column tiles, then m,
                 // then band (0: one band) -- the 32 tiles an XCD works on at a time then share fewer
                 // distinct operand blocks (4 x 8 instead of 2 x 16 of a 16-column problem)
@@ -461,6 +466,20 @@ __device__ __forceinline__ Tile tile_of(const GemmParams& p, int z0, int z1, int
     }
   }
   return t;
+}
+
+// The plain schedule's tile number `rem`.
+__device__ __forceinline__ void plain_tile(const GemmParams& p, int rem, int* mt, int* nt) {
+  if (p.n_group > 0) {
+    const int band = p.n_group * p.mt_count;       // tiles of a full band
+    const int b0 = rem / band, r2 = rem % band;
+    const int w = min(p.n_group, p.nt_count - b0 * p.n_group);  // the last band may be narrower
+    *nt = b0 * p.n_group + r2 % w;
+    *mt = r2 / w;
+  } else {
+    *nt = rem % p.nt_count;
+    *mt = rem / p.nt_count;
+  }
 }
 
 // Epilogue of a wave: its 32 IT x 64 accumulators at row0, col0 of C through its own LDS region `stage` ([row][EP]) into
@@ -834,7 +853,7 @@ constexpr int kDma64Operand = kTile * kSlab64;  // elements of an operand slab (
 constexpr int kDma64Stage = 2 * kDma64Operand;
 static_assert(sizeof(uint16_t) * 2 * kDma64Stage <= kDmaLds, "two slab buffers fit");
 
-template <int DT, bool TA, bool TB, int T = kTile, bool LIN = false>
+template <int DT, bool TA, bool TB, int T = kTile, bool LIN = false, bool CUT = false>
 __global__ __launch_bounds__(2 * T) void gemm_dma64_kernel(const GemmParams p) {
   extern __shared__ __align__(16) uint16_t smem[];
   constexpr int JN = 2, NL = 4;
@@ -843,8 +862,15 @@ __global__ __launch_bounds__(2 * T) void gemm_dma64_kernel(const GemmParams p) {
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   const int wm = wave / (NW / 2), wn = wave % (NW / 2);
   const int G = static_cast<int>(gridDim.x), lin = static_cast<int>(blockIdx.x);
-  int it_lo, it_hi, it_step;
-  if (G % kXcds == 0) {
+  int it_lo, it_hi, it_step, part = 0;
+  if constexpr (CUT) {  // one part of one item; neighbours on an XCD
+    const int left = p.items - p.full, at = lin % kXcds * (G / kXcds) + lin / kXcds;
+    if (at >= left * p.cut) return;
+    part = at / left;
+    it_lo = p.full + at % left;
+    it_hi = it_lo + 1;
+    it_step = 1;
+  } else if (G % kXcds == 0) {
     const int xcd = lin % kXcds;
     it_lo = static_cast<int>(static_cast<int64_t>(p.items) * xcd / kXcds) + lin / kXcds;
     it_hi = static_cast<int>(static_cast<int64_t>(p.items) * (xcd + 1) / kXcds);
@@ -873,14 +899,8 @@ __global__ __launch_bounds__(2 * T) void gemm_dma64_kernel(const GemmParams p) {
     const int pr = rem / p.nt_count;
     mt_first = p.mt_count - 1 - pr;
     if (T == kTile && mt_first != pr) mt_second = pr;
-  } else if (p.n_group > 0) {  // as in gemm_dma_kernel
-    const int band = p.n_group * p.mt_count, b0 = rem / band, r2 = rem % band;
-    const int w = min(p.n_group, p.nt_count - b0 * p.n_group);
-    nt = b0 * p.n_group + r2 % w;
-    mt_first = r2 / w;
   } else {
-    nt = rem % p.nt_count;
-    mt_first = rem / p.nt_count;
+    plain_tile(p, rem, &mt_first, &nt);
   }
   const int z0 = zz / p.nh, z1 = zz % p.nh;
   for (int half = 0; half < 2; ++half) {
@@ -894,6 +914,11 @@ __global__ __launch_bounds__(2 * T) void gemm_dma64_kernel(const GemmParams p) {
   int kb = 0, ke = p.K;
   if (p.k_mode == 1) ke = min(p.K, ((mt + 1) * T + p.off + kSlab64 - 1) / kSlab64 * kSlab64);
   if (p.k_mode == 2) kb = min(p.K, max(0, mt * T - p.off) / kSlab64 * kSlab64);
+  if constexpr (CUT) {
+    const int slabs = p.K / kSlab64;
+    kb = slabs * part / p.cut * kSlab64;
+    ke = slabs * (part + 1) / p.cut * kSlab64;
+  }
   const int nslab = (ke - kb + kSlab64 - 1) / kSlab64;
 
   floatx16 acc[IT][JN];
@@ -1028,10 +1053,58 @@ __global__ __launch_bounds__(2 * T) void gemm_dma64_kernel(const GemmParams p) {
 #undef MEGA_DMA64_KSTEP
 #undef MEGA_SGB
 
-  store_tile<DT, IT, LIN>(acc, p, t, t.M, m0 + wm * 32 * IT, n0 + wn * 64, lane, smem + wave * 32 * IT * (64 + 8));
+  if constexpr (CUT) {
+    char* const dst = reinterpret_cast<char*>(p.parts + ((static_cast<int64_t>(item - p.full) * p.cut + part) * NW + wave) * (32 * IT * 64));
+    uint32_t at = 16 * lane;
+#pragma unroll
+    for (int i = 0; i < IT; ++i)
+#pragma unroll
+      for (int j = 0; j < JN; ++j) {
+        asm volatile("" : "+v"(at));  // (one address that advances, not one for each store)
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4)
+          *reinterpret_cast<float4*>(dst + at + 1024 * q4) =
+              make_float4(acc[i][j][4 * q4], acc[i][j][4 * q4 + 1], acc[i][j][4 * q4 + 2], acc[i][j][4 * q4 + 3]);
+        at += 4096;
+      }
+  } else {
+    store_tile<DT, IT, LIN>(acc, p, t, t.M, m0 + wm * 32 * IT, n0 + wn * 64, lane, smem + wave * 32 * IT * (64 + 8));
+  }
   lds_barrier();
   }  // tile of the pair
   }  // work item
+}
+
+// The parts of gemm_dma64_kernel's last tiles added up, in order: 32 x 64 values of a wave of that kernel per wave of this one,
+// 32 workgroups of one wave a tile, so that the parts of few tiles are read by many CUs.
+template <int DT>
+__global__ __launch_bounds__(kWave) void linear_parts_kernel(const GemmParams p) {
+  __shared__ __align__(16) uint16_t stage[32 * (64 + 8)];
+  constexpr int kPart = 32 * 4 * 64;  // values of a wave of the product
+  const int lane = threadIdx.x, i = blockIdx.x % 4;
+  const int tile = blockIdx.x / 32, of = blockIdx.x / 4 % 8, wm = of / 4, wn = of % 4;
+  int mt, nt;
+  plain_tile(p, p.full + tile, &mt, &nt);
+  const Tile t = tile_of<true, false, false>(p, 0, 0, mt, nt);
+  const float* src = p.parts + (static_cast<int64_t>(tile) * p.cut * 8 + of) * kPart + i * (32 * 64) + 4 * lane;
+  floatx16 acc[1][2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[0][j][r] = 0.f;
+#pragma unroll 2
+  for (int part = 0; part < p.cut; ++part)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        const float4 v = *reinterpret_cast<const float4*>(src + static_cast<int64_t>(part) * 8 * kPart + (j * 4 + q4) * 256);
+        acc[0][j][4 * q4] += v.x;
+        acc[0][j][4 * q4 + 1] += v.y;
+        acc[0][j][4 * q4 + 2] += v.z;
+        acc[0][j][4 * q4 + 3] += v.w;
+      }
+  store_tile<DT, 1, true>(acc, p, t, t.M, t.mt * kTile + wm * 128 + 32 * i, t.nt * kTile + wn * 64, lane, stage);
 }
 
 // ---- one k-contiguous and one k-major operand: A in slabs of 64 k, B in slabs of 32 k ------
@@ -1087,16 +1160,7 @@ __global__ __launch_bounds__(2 * kThreads) void gemm_dma_a64_kernel(const GemmPa
     mt_first = p.mt_count - 1 - pr;
     if (mt_first != pr) mt_second = pr;
   } else {
-    if (p.n_group > 0) {
-      const int band = p.n_group * p.mt_count;       // tiles of a full band
-      const int b0 = rem / band, r2 = rem % band;
-      const int w = min(p.n_group, p.nt_count - b0 * p.n_group);  // the last band may be narrower
-      nt = b0 * p.n_group + r2 % w;
-      mt_first = r2 / w;
-    } else {
-      nt = rem % p.nt_count;
-      mt_first = rem / p.nt_count;
-    }
+    plain_tile(p, rem, &mt_first, &nt);
   }
   const int z0 = zz / p.nh, z1 = zz % p.nh;
   for (int half = 0; half < 2; ++half) {
@@ -1922,9 +1986,28 @@ int compute_units(int* cus) {
 // Time of a launch in us by what was measured (1000 to 32768 tokens, layers of 1024 to 11008).  A tile of 256 takes longer
 // for 32 k the more of the chip works (the clock falls: forward 0.45 us alone, 0.80 with every CU busy); tiles of 128 run
 // two to a CU, each pair as long as two one after the other; every round of tiles starts and ends in a few us.
-double estimate(const GemmParams& q, int kind, int T, int cus) {
+//
+// Where the last round holds few tiles, they are cut along k, a part for a workgroup, and another launch adds up the parts (0.12
+// us for each part of 256 KB written and read, 14 us for two launches).  2 x 11008 x 4096, us whole / cut: 1531 tokens (516 tiles)
+// 278 / 235, 2100 (774) 351 / 332, 3000 (1032) 477 / 435, 9000 (3096) 1345 / 1288; the parts of few tiles are read by 32
+// workgroups of a wave each (eight of four waves: 19.6 us for 32 parts, so under 10).  Tiles that fill more than half a round stay
+// whole: there is no second workgroup for each.
+double estimate_cut(GemmParams& q, double slabs, int cus) {
+  const int grid = std::max(cus / kXcds, 1) * kXcds, left = q.items % grid, full = q.items - left;
+  const auto round = [&](double tiles, double k) { return k * (0.45 + 0.35 * tiles / grid) + 5; };
+  const double whole = full / grid * round(grid, slabs) + 3;
+  double best = whole + (left > 0 ? round(left, slabs) : 0);
+  q.full = q.items, q.cut = 0;
+  for (int cut = 2; cut <= 8 && left > 0 && left * cut <= grid && slabs >= 16 * cut; ++cut) {
+    const double t = whole + round(left * cut, slabs / cut) + 0.12 * left * cut + 14;
+    if (t < best) best = t, q.full = full, q.cut = cut;
+  }
+  return best;
+}
+double estimate(GemmParams& q, int kind, int T, int cus) {
   const double slabs = (q.K + kSlab - 1) / kSlab, rounds = (q.items + cus - 1) / cus, load = q.items / (rounds * cus);
   if (T == kTile) {
+    if (kind == kForward && q.split_ok) return estimate_cut(q, slabs, cus);
     if (kind == kWeightGrad) return rounds * (slabs * (0.40 + 0.36 * load) + 1) + 2;
     if (kind == kForward) return rounds * (slabs * (0.45 + 0.35 * load) + 5) + 3;
     return rounds * (slabs * (0.42 + 0.37 * load) + 5) + 2;
@@ -1941,7 +2024,8 @@ double plan(GemmParams& q, int kind, int count, const int64_t* sizes, int cus, b
   lay_out(q, kind, count, sizes, kSmall);
   const double tl = estimate(l, kind, kTile, cus), ts = estimate(q, kind, kSmall, cus);
   *small = ts <= tl;
-  if (!*small) q = l;
+  if (*small) q.full = q.items, q.cut = 0;
+  else q = l;
   return std::min(ts, tl);
 }
 
@@ -1993,6 +2077,16 @@ int launch_linear(GemmParams q, int kind, int count, const int64_t* sizes, hipSt
   int grid = (q.items + kXcds - 1) / kXcds * kXcds;
   if (!small) grid = std::min(grid, std::max(cus / kXcds, 1) * kXcds);
   if (kind == kForward) {
+    if (!small && q.cut > 0) {
+      const int left = q.items - q.full;
+      GemmParams whole = q;
+      whole.items = q.full;
+      if (q.full > 0)
+        if (const int rc = launch_tiles<gemm_dma64_kernel<DT, false, false, kTile, true>>(whole, grid, threads, lds, s); rc != MEGA_OK) return rc;
+      grid = (left * q.cut + kXcds - 1) / kXcds * kXcds;
+      if (const int rc = launch_tiles<gemm_dma64_kernel<DT, false, false, kTile, true, true>>(q, grid, threads, lds, s); rc != MEGA_OK) return rc;
+      return launch_tiles<linear_parts_kernel<DT>>(q, left * 32, kWave, 0, s);
+    }
     if (!small) return launch_tiles<gemm_dma64_kernel<DT, false, false, kTile, true>>(q, grid, threads, lds, s);
     if (q.items <= cus) return launch_tiles<gemm_dma_kernel<DT, false, false, false, kSmall, true>>(q, grid, threads, lds, s);
     return launch_tiles<gemm_dma64_kernel<DT, false, false, kSmall, true>>(q, grid, threads, lds, s);
@@ -2045,6 +2139,7 @@ extern "C" int mega_linear_takes(int kind, int dtype, int64_t tokens, int64_t n_
   GemmParams q{};
   bool apart;
   q.M = (int)tokens; q.N = (int)(kind == kForward ? n_out[0] : n_in); q.K = (int)(kind == kForward ? n_in : n_out[0]);
+  q.split_ok = 1;
   const double here = plan_group(q, kind, kind == kForward ? count : 1, kind == kForward ? n_out : &n_in, cus, &apart);
   // The library: at least 20 us a call (its host path), then what it reaches on products of so many terms, in PFLOP/s; widths
   // off the multiples of 1024 cost it a quarter up to some 2^39.  Forward, us (library / here): 4096 tokens, 256 + 2048 + 1024 x
@@ -2060,11 +2155,29 @@ extern "C" int mega_linear_takes(int kind, int dtype, int64_t tokens, int64_t n_
   return here <= library;
 }
 
+extern "C" int64_t mega_linear_fwd_workspace_bytes(int64_t tokens, int64_t n_in, int count, const int64_t* n_out) {
+  if (check_linear("mega_linear_fwd_workspace_bytes", kForward, MEGA_BF16, tokens, n_in, count, n_out) != MEGA_OK) return 0;
+  int cus = 0;
+  if (compute_units(&cus) != MEGA_OK) return 0;
+  GemmParams q{};
+  q.M = (int)tokens; q.N = (int)n_out[0]; q.K = (int)n_in;
+  q.split_ok = 1;
+  bool apart, small;
+  plan_group(q, kForward, count, n_out, cus, &apart);
+  int64_t parts = 0;
+  for (int i = 0; i < (apart ? count : 1); ++i) {
+    GemmParams o = apart ? one_of(q, kForward, i, n_out[i]) : q;
+    plan(o, kForward, apart ? 1 : count, apart ? n_out + i : n_out, cus, &small);
+    parts = std::max(parts, static_cast<int64_t>(o.items - o.full) * o.cut);
+  }
+  return parts * (sizeof(float) * kTile * kTile);
+}
+
 extern "C" int mega_linear_fwd(const void* x, const void* const* w, const void* const* bias, const void* add, int dtype,
-                               int64_t tokens, int64_t n_in, int count, const int64_t* n_out, void* const* y, void* stream) {
+                               int64_t tokens, int64_t n_in, int count, const int64_t* n_out, void* const* y, void* workspace, void* stream) {
   const int rc = check_linear("mega_linear_fwd", kForward, dtype, tokens, n_in, count, n_out);
   if (rc != MEGA_OK) return rc;
-  MEGA_CHECK_ARG(w && y && aligned16(x) && x && aligned16(add) && (!add || count == 1), "mega_linear_fwd: null or misaligned pointer");
+  MEGA_CHECK_ARG(w && y && aligned16(x) && x && aligned16(add) && aligned16(workspace) && (!add || count == 1), "mega_linear_fwd: null or misaligned pointer");
   for (int i = 0; i < count; ++i)
     MEGA_CHECK_ARG(w[i] && y[i] && aligned16(w[i]) && aligned16(y[i]) && (!bias || aligned16(bias[i])), "mega_linear_fwd: null or misaligned pointer");
   const auto u = [](const void* q) { return static_cast<const uint16_t*>(q); };
@@ -2073,6 +2186,7 @@ extern "C" int mega_linear_fwd(const void* x, const void* const* w, const void* 
   g.M = (int)tokens; g.N = (int)n_out[0]; g.K = (int)n_in;
   g.lda = n_in; g.ldb = n_in; g.ldc = n_out[0];
   g.bias = bias ? u(bias[0]) : nullptr; g.add = u(add);
+  g.parts = static_cast<float*>(workspace); g.split_ok = workspace != nullptr;
   for (int i = 1; i < count; ++i) g.op[i - 1] = u(w[i]), g.out[i - 1] = static_cast<uint16_t*>(y[i]), g.bias_of[i - 1] = bias ? u(bias[i]) : nullptr;
   hipStream_t s = static_cast<hipStream_t>(stream);
   return dtype == MEGA_BF16 ? launch_linear<MEGA_BF16>(g, kForward, count, n_out, s) : launch_linear<MEGA_F16>(g, kForward, count, n_out, s);

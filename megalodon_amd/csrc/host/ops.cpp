@@ -567,7 +567,9 @@ std::optional<variable_list> products(const Tensor& x, const variable_list& w, c
     bp.push_back(bias[i].has_value() ? bias[i]->data_ptr() : nullptr);
     yp.push_back(y.back().data_ptr());
   }
-  check(mega_linear_fwd(x.data_ptr(), wp.data(), bp.data(), residual.has_value() ? residual->data_ptr() : nullptr, code, tokens, n_in, count, n_out.data(), yp.data(), stream_of(x)), "mega_linear_fwd");
+  const int64_t bytes = mega_linear_fwd_workspace_bytes(tokens, n_in, count, n_out.data());
+  const Tensor ws = bytes > 0 ? at::empty({bytes}, x.options().dtype(at::kByte)) : Tensor();
+  check(mega_linear_fwd(x.data_ptr(), wp.data(), bp.data(), residual.has_value() ? residual->data_ptr() : nullptr, code, tokens, n_in, count, n_out.data(), yp.data(), ptr(ws), stream_of(x)), "mega_linear_fwd");
   return y;
 }
 // x W^T (+ bias), or x W^T + residual with the residual as the product's accumulator input
@@ -689,7 +691,20 @@ struct LinearGroupFn : Function<LinearGroupFn> {
   }
 };
 std::vector<Tensor> linear_group(const Tensor& x, const std::vector<Tensor>& params, const std::vector<bool>& has_bias) {
-  return LinearGroupFn::apply(x, at::TensorList(params), has_bias);
+  bool recorded = wants_grad({&x});
+  for (const Tensor& t : params) recorded = recorded || wants_grad({&t});
+  if (recorded) return LinearGroupFn::apply(x, at::TensorList(params), has_bias);
+  variable_list weights;
+  std::vector<Optional> biases;
+  size_t at_ = 0;
+  for (const bool b : has_bias) {
+    weights.push_back(params[at_++]);
+    biases.push_back(b ? Optional(params[at_++]) : Optional());
+  }
+  if (auto y = products(x, weights, biases, Optional()); y.has_value()) return *y;
+  variable_list out;
+  for (size_t i = 0; i < weights.size(); ++i) out.push_back(linear_raw(x, weights[i], biases[i], Optional()));
+  return out;
 }
 
 }  // namespace

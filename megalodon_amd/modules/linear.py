@@ -20,12 +20,16 @@ from .. import _lib
 
 
 def linear_group(x: torch.Tensor, layers) -> Tuple[torch.Tensor, ...]:
-    """`tuple(layer(x) for layer in layers)` for `Linear` layers that read the same input; on the
-    GPU in 16 bits with gradients enabled their backward shares one input-gradient accumulation."""
+    """`tuple(layer(x) for layer in layers)` for `Linear` layers that read the same input; on the GPU in
+    16 bits their products are one launch where that is the faster form, and with gradients their backward
+    shares one input-gradient accumulation.  Without gradients only for layers whose call is nothing but
+    `Linear.forward`: no hooks of their own or for all modules."""
     layers = list(layers)
-    fused = (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and torch.is_grad_enabled()
-             and all(l.weight.dtype == x.dtype for l in layers)
-             and (x.requires_grad or any(l.weight.requires_grad for l in layers)))
+    fused = (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16)
+             and all(l.weight.dtype == x.dtype for l in layers))
+    if fused and not (torch.is_grad_enabled() and (x.requires_grad or any(l.weight.requires_grad for l in layers))):
+        fused = all(type(l) is Linear and "forward" not in l.__dict__ and not l._forward_hooks and not l._forward_pre_hooks for l in layers) \
+            and not torch.nn.modules.module._global_forward_hooks and not torch.nn.modules.module._global_forward_pre_hooks
     if not fused or len(layers) < 2:
         return tuple(l(x) for l in layers)
     params, has_bias = [], []

@@ -54,7 +54,14 @@ def test_products_match_float64(tokens, n_in, n_out, dtype):
     dw = [torch.empty_like(t) for t in w]
     outs, s = (i64 * len(n_out))(*n_out), _lib.stream_ptr(x.device)
     call = lambda name, *a: _lib.call(name, *a, s)
-    call("mega_linear_fwd", _lib.ptr(x), _pointers(w), _pointers(bias), None, _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(len(w)), outs, _pointers(y))
+
+    def fwd(w, bias, add, n_out, y):
+        n, outs = len(w), (i64 * len(w))(*n_out)
+        size = _lib.load().mega_linear_fwd_workspace_bytes(i64(tokens), i64(n_in), n, outs)
+        ws = torch.empty(size, dtype=torch.uint8, device="cuda")
+        call("mega_linear_fwd", _lib.ptr(x), _pointers(w), bias and _pointers(bias), add, _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(n), outs, _pointers(y), _lib.ptr(ws) if size else None)
+
+    fwd(w, bias, None, n_out, y)
     call("mega_linear_weight_grads", _pointers(dy), _lib.ptr(x), _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(len(w)), outs, _pointers(dw))
     x64, w64, dy64 = x.double(), [t.double() for t in w], [t.double() for t in dy]
     for i in range(len(w)):
@@ -63,9 +70,9 @@ def test_products_match_float64(tokens, n_in, n_out, dtype):
         # one layer alone gives the same bits as in the group
         if len(w) > 1:
             alone = torch.empty_like(y[i])
-            call("mega_linear_fwd", _lib.ptr(x), _pointers([w[i]]), _pointers([bias[i]]), None, _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(1), (i64 * 1)(n_out[i]), _pointers([alone]))
+            fwd([w[i]], [bias[i]], None, [n_out[i]], [alone])
             assert torch.equal(alone, y[i])
-    call("mega_linear_fwd", _lib.ptr(x), _pointers(w[:1]), None, _lib.ptr(add), _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(1), (i64 * 1)(n_out[0]), _pointers(y[:1]))
+    fwd(w[:1], None, _lib.ptr(add), n_out[:1], y[:1])
     _close(y[0], x64 @ w64[0].t() + add.double())
     dx = torch.empty_like(x)
     for i in range(len(w)):  # added up in place
@@ -110,3 +117,60 @@ def test_layers_whose_operands_need_the_general_path(tokens, sizes):
     dx, dw = torch.autograd.grad(y, (leaf, layer.weight), many, is_grads_batched=True)
     _close(dx, many.double() @ layer.weight.double())
     _close(dw, torch.stack([g.double().t() @ x.double() for g in many]))
+
+
+@pytest.mark.parametrize("tokens,n_in,n_out,dtype", [
+    (4100, 4096, [4096], torch.bfloat16),             # 272 tiles: 16 left over, the last of four rows
+    (1531, 4096, [5504, 5568], torch.float16),        # two layers, layers and rows that end inside a tile
+    (1531, 11008, [4096], torch.bfloat16),            # fewer tiles than the chip takes
+])
+def test_last_tiles_cut_along_k(tokens, n_in, n_out, dtype):
+    """The tiles that a last round of the chip would hold alone, cut along k and added up by a second launch: against
+    float64, the same twice (the parts are added in order), and without memory for the parts, where nothing is cut."""
+    g = torch.Generator("cuda").manual_seed(tokens)
+    rows = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x = _poisoned(rows(tokens, n_in).to(dtype))
+    w = [_poisoned((rows(o, n_in) / n_in ** 0.5).to(dtype)) for o in n_out]
+    bias, add = [rows(o).to(dtype) for o in n_out], rows(tokens, n_out[0]).to(dtype)
+    i64, outs = ctypes.c_int64, (ctypes.c_int64 * len(n_out))(*n_out)
+    size = ctypes.CFUNCTYPE(i64, i64, i64, ctypes.c_int, ctypes.c_void_p)(("mega_linear_fwd_workspace_bytes", _lib.load()))
+    bytes_, summed = size(tokens, n_in, len(n_out), outs), add if len(n_out) == 1 else None
+    assert 0 < bytes_ <= 64 << 20
+
+    def run(ws):
+        y = [torch.full((tokens, o), float("nan"), dtype=dtype, device="cuda") for o in n_out]
+        _lib.call("mega_linear_fwd", _lib.ptr(x), _pointers(w), _pointers(bias), None if summed is None else _lib.ptr(summed),
+                  _lib.i32(_lib.dtype_code(dtype)), i64(tokens), i64(n_in), _lib.i32(len(w)), outs, _pointers(y), ws, _lib.stream_ptr(x.device))
+        return y
+
+    parts = torch.full((bytes_ + 4096,), 255, dtype=torch.uint8, device="cuda")  # NaN
+    once, again, whole = run(_lib.ptr(parts)), run(_lib.ptr(parts)), run(None)
+    assert (parts[bytes_:] == 255).all()
+    for i, o in enumerate(n_out):
+        want = x.double() @ w[i].double().t() + bias[i].double() + (0 if summed is None else summed.double())
+        _close(once[i], want)
+        _close(whole[i], want)
+        assert torch.equal(once[i], again[i])
+
+
+def test_group_without_gradients():
+    """One launch where no gradient is wanted: the values of the layers one by one, and their own calls where a layer's call is
+    more than its product (hooks, a subclass)."""
+    torch.manual_seed(3)
+    layers = [Linear(1024, o, bias=b).cuda().bfloat16() for o, b in ((256, True), (2048, False), (1024, True))]
+    x = torch.randn(500, 1024, device="cuda").bfloat16()
+    with torch.no_grad():
+        for y, l in zip(linear_group(x, layers), layers):
+            _close(y, x.double() @ l.weight.double().t() + (0 if l.bias is None else l.bias.double()))
+        seen = []
+        hook = layers[1].register_forward_hook(lambda m, a, y: seen.append(y) or y + 1)
+        y = linear_group(x, layers)[1]
+        assert len(seen) == 1 and torch.equal(y, seen[0] + 1)
+        hook.remove()
+
+        class Twice(Linear):
+            def forward(self, x, residual=None):
+                return 2 * super().forward(x, residual)
+
+        layers[0].__class__ = Twice
+        assert torch.equal(linear_group(x, layers)[0], layers[0](x))
