@@ -411,7 +411,7 @@ int mega_linear_weight_grad(const void* dy, const void* x, int dtype, int64_t to
  *                 null; add (tokens, n_out) with one layer only; n_in a multiple of 64.  `workspace`:
  *                 mega_linear_fwd_workspace_bytes bytes (up to 64 MiB; for many sizes 0), or null: no product is cut
  *                 along k then, which some sizes are slower without.
- *   input_grad:   dx = dy w + add; add (tokens, n_in) or null, may be dx itself; n_out a multiple of 64.
+ *   input_grad:   dx = sum_i dy_i w_i + add; add (tokens, n_in) or null, may be dx itself; n_out a multiple of 64.
  *   weight_grads: dw_i = dy_i^T x.
  * `takes` (kind 0, 1, 2 in this order; input_grad: count 1) is 1 where the launch is expected to be
  * faster than a general library's products, 0 where it is not or where the sizes are refused. */
@@ -420,8 +420,8 @@ int mega_linear_fwd(const void* x, const void* const* w, const void* const* bias
                     int dtype, int64_t tokens, int64_t n_in, int count, const int64_t* n_out,
                     void* const* y, void* workspace, void* stream);
 int64_t mega_linear_fwd_workspace_bytes(int64_t tokens, int64_t n_in, int count, const int64_t* n_out);
-int mega_linear_input_grad(const void* dy, const void* w, const void* add, int dtype, int64_t tokens,
-                           int64_t n_out, int64_t n_in, void* dx, void* stream);
+int mega_linear_input_grad(const void* const* dy, const void* const* w, const void* add, int dtype,
+                           int64_t tokens, int64_t n_in, int count, const int64_t* n_out, void* dx, void* stream);
 int mega_linear_weight_grads(const void* const* dy, const void* x, int dtype, int64_t tokens,
                              int64_t n_in, int count, const int64_t* n_out, void* const* dw,
                              void* stream);

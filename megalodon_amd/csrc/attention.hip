@@ -129,6 +129,10 @@ struct GemmParams {
   uint16_t* out[2];
   const uint16_t* bias_of[2];
   int size[2], start[2];
+  // ... and an input gradient whose layers lie behind each other along k: k slabs >= seg_start[i] (of kSlab) are those of
+  // op[i] and op_b[i], rows of A size[i] apart there
+  const uint16_t* op_b[2];
+  int seg_start[2];
   int kva;      // as kvb, for a k-major A (LIN: rows behind it are not there; else they hold zeros)
   // CUT: items full .. items - 1, fewer than there are CUs, are cut along k into `cut` parts; float32 sums of part i
   // of item full + r at parts + (r cut + i) 256 x 256, as the waves hold them (linear_parts_kernel adds them up).
@@ -591,8 +595,9 @@ __device__ __forceinline__ void load_to_lds16(u32x4 buffer, uint32_t offset, uin
 
 //
 // T: the workgroup's tile, 256 (2 x 4 waves of 128 x 64) or 128 (2 x 2 waves of 64 x 64, two workgroups per CU).
-// RAG: p.kvb and p.ms are set (B k-major)
-template <int DT, bool TA, bool TB, bool RAG = false, int T = kTile, bool LIN = false>
+// RAG: p.kvb and p.ms are set (B k-major).  SEG: p.seg_start and the operands behind it are (apart, since the choice of the
+// operands with every request costs a product of one pair 10 %: 4096 x 1024 -> 2752 21.3 us, 23.6 so)
+template <int DT, bool TA, bool TB, bool RAG = false, int T = kTile, bool LIN = false, bool SEG = false>
 __global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
   extern __shared__ __align__(16) uint16_t smem[];
   constexpr int JN = 2, NL = 2;
@@ -688,14 +693,16 @@ __global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
   // memory side: wave w sends the 1 KB pieces w and w + 8 of each operand slab; lane l
   // of piece pc fetches what belongs at position l of the piece (addresses clamped into
   // the matrix, so every lane always loads)
-  uint32_t offa[NL], offb[NL];
+  static_assert(!SEG || (LIN && !TA && TB && !RAG), "several pairs of operands along k: input gradients");
+  uint32_t offa[NL], offb[NL], row_a[NL];
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
     const int pc = wave + NW * i;
     const int krow = KR * pc + lane / CR, cm = (lane % CR) ^ ((krow & 3) << 2);  // k-major piece
     const int row = 16 * pc + (lane >> 2), ck = (lane & 3) ^ ((lane >> 4) & 3);   // k-contiguous piece
     if (TA) offa[i] = static_cast<uint32_t>(((kb + krow) * t.lda + min(m0 + cm * 8, t.M - 8)) * 2);
-    else offa[i] = static_cast<uint32_t>((static_cast<int64_t>(min(m0 + row, t.M - 1)) * t.lda + kb + ck * 8) * 2);
+    else offa[i] = static_cast<uint32_t>((SEG ? 0 : static_cast<int64_t>(min(m0 + row, t.M - 1)) * t.lda + kb + ck * 8) * 2);
+    if constexpr (SEG) row_a[i] = static_cast<uint32_t>(min(m0 + row, t.M - 1)), offa[i] = static_cast<uint32_t>(ck * 16);
     if (TB) offb[i] = static_cast<uint32_t>(((kb + krow) * p.ldb + min(n0 + cm * 8, t.N - 8)) * 2);
     else offb[i] = static_cast<uint32_t>((static_cast<int64_t>(min(n0 + row, t.N - 1)) * p.ldb + kb + ck * 8) * 2);
   }
@@ -708,8 +715,20 @@ __global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
   const u32x4 bufa = RAG && LIN && TA ? buffer_of(A, static_cast<uint32_t>(((p.kva - 1) * t.lda + t.M) * 2)) : u32x4{};
   // request number n of a slab: n = 0, 2 the two pieces of A, n = 1, 3 those of B
   auto request_one = [&](int s, int stage, int n) {
-    const uint32_t sc = static_cast<uint32_t>(min(s, nslab - 1));
+    uint32_t sc = static_cast<uint32_t>(min(s, nslab - 1));
     const uint32_t dst = lds_wave + static_cast<uint32_t>(stage * kStage + (n >> 1) * NW * 512 + (n & 1) * kOperand) * 2;
+    if constexpr (SEG) {
+      const int at = __builtin_amdgcn_readfirstlane(static_cast<int>(sc));
+      const bool past = at >= p.seg_start[0], past2 = at >= p.seg_start[1];
+      sc = static_cast<uint32_t>(at - (past2 ? p.seg_start[1] : past ? p.seg_start[0] : 0));
+      if (n & 1) {
+        load_to_lds16(past2 ? p.op_b[1] : past ? p.op_b[0] : B, offb[n >> 1] + sc * stepb, dst);
+      } else {
+        const uint32_t ld = past2 ? p.size[1] : past ? p.size[0] : static_cast<uint32_t>(t.lda);
+        load_to_lds16(past2 ? p.op[1] : past ? p.op[0] : A, (row_a[n >> 1] * ld) * 2 + offa[n >> 1] + sc * stepa, dst);
+      }
+      return;
+    }
     if (n & 1) {
       static_assert(TB || !RAG, "rows of k");
       if constexpr (RAG) load_to_lds16(bufb, offb[n >> 1] + sc * stepb, dst);
@@ -1965,6 +1984,8 @@ enum { kForward, kInputGrad, kWeightGrad };
 void lay_out(GemmParams& q, int kind, int count, const int64_t* sizes, int T) {
   const auto tiles = [&](int64_t n) { return static_cast<int>((n + T - 1) / T); };
   q.start[0] = q.start[1] = 0x7fffffff;
+  if (kind != kInputGrad || q.op_b[0] == nullptr) q.seg_start[0] = 0x7fffffff;
+  if (kind != kInputGrad || q.op_b[1] == nullptr) q.seg_start[1] = 0x7fffffff;
   int along = tiles(sizes[0]);
   for (int i = 1; i < count; ++i) {
     q.start[i - 1] = along;
@@ -2093,6 +2114,7 @@ int launch_linear(GemmParams q, int kind, int count, const int64_t* sizes, hipSt
   }
   if (kind == kInputGrad) {
     if (!small) return launch_tiles<gemm_dma_a64_kernel<DT, false, true>>(q, grid, threads, kA64Lds, s);
+    if (q.op_b[0] != nullptr) return launch_tiles<gemm_dma_kernel<DT, false, true, false, kSmall, true, true>>(q, grid, threads, lds, s);
     return launch_tiles<gemm_dma_kernel<DT, false, true, false, kSmall, true>>(q, grid, threads, lds, s);
   }
   const bool rag = q.K % kSlab != 0;
@@ -2138,7 +2160,9 @@ extern "C" int mega_linear_takes(int kind, int dtype, int64_t tokens, int64_t n_
   }
   GemmParams q{};
   bool apart;
-  q.M = (int)tokens; q.N = (int)(kind == kForward ? n_out[0] : n_in); q.K = (int)(kind == kForward ? n_in : n_out[0]);
+  q.M = (int)tokens; q.N = (int)(kind == kForward ? n_out[0] : n_in); q.K = (int)(kind == kForward ? n_in : 0);
+  if (kind == kInputGrad)
+    for (int i = 0; i < count; ++i) q.K += (int)n_out[i];
   q.split_ok = 1;
   const double here = plan_group(q, kind, kind == kForward ? count : 1, kind == kForward ? n_out : &n_in, cus, &apart);
   // The library: at least 20 us a call (its host path), then what it reaches on products of so many terms, in PFLOP/s; widths
@@ -2192,18 +2216,39 @@ extern "C" int mega_linear_fwd(const void* x, const void* const* w, const void* 
   return dtype == MEGA_BF16 ? launch_linear<MEGA_BF16>(g, kForward, count, n_out, s) : launch_linear<MEGA_F16>(g, kForward, count, n_out, s);
 }
 
-extern "C" int mega_linear_input_grad(const void* dy, const void* w, const void* add, int dtype, int64_t tokens, int64_t n_out,
-                                      int64_t n_in, void* dx, void* stream) {
-  const int rc = check_linear("mega_linear_input_grad", kInputGrad, dtype, tokens, n_in, 1, &n_out);
+extern "C" int mega_linear_input_grad(const void* const* dy, const void* const* w, const void* add, int dtype, int64_t tokens,
+                                      int64_t n_in, int count, const int64_t* n_out, void* dx, void* stream) {
+  const int rc = check_linear("mega_linear_input_grad", kInputGrad, dtype, tokens, n_in, count, n_out);
   if (rc != MEGA_OK) return rc;
-  MEGA_CHECK_ARG(dy && w && dx && aligned16(dy) && aligned16(w) && aligned16(dx) && aligned16(add), "mega_linear_input_grad: null or misaligned pointer");
-  GemmParams g{};
-  g.A = static_cast<const uint16_t*>(dy); g.B = static_cast<const uint16_t*>(w); g.C = static_cast<uint16_t*>(dx);
-  g.M = (int)tokens; g.N = (int)n_in; g.K = (int)n_out;
-  g.lda = n_out; g.ldb = n_in; g.ldc = n_in; g.tb = 1;
-  g.add = static_cast<const uint16_t*>(add);
+  MEGA_CHECK_ARG(dy && w && dx && aligned16(dx) && aligned16(add), "mega_linear_input_grad: null or misaligned pointer");
+  for (int i = 0; i < count; ++i) MEGA_CHECK_ARG(dy[i] && w[i] && aligned16(dy[i]) && aligned16(w[i]), "mega_linear_input_grad: null or misaligned pointer");
+  const auto u = [](const void* q) { return static_cast<const uint16_t*>(q); };
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return dtype == MEGA_BF16 ? launch_linear<MEGA_BF16>(g, kInputGrad, 1, &n_in, s) : launch_linear<MEGA_F16>(g, kInputGrad, 1, &n_in, s);
+  GemmParams g{};
+  g.C = static_cast<uint16_t*>(dx);
+  g.M = (int)tokens; g.N = (int)n_in;
+  g.ldb = n_in; g.ldc = n_in; g.tb = 1;
+  int cus = 0;
+  if (const int rc2 = compute_units(&cus); rc2 != MEGA_OK) return rc2;
+  // One product with the layers behind each other along k, in tiles of 128: one rounding, and dx is neither read again nor
+  // launched for again.  us, one after the other / so: 4096 tokens, 256 + 2048 + 1024 x 1024 50 / 32, 2 x 2752 x 1024 59 / 50; 4084
+  // tokens, 512 + 4096 + 2048 x 2048 140 / 114; 500 tokens of the first 41 / 26.  Where tiles of 256 are the faster ones, one
+  // after the other.
+  GemmParams all = g;
+  bool small = false;
+  for (int i = 0; i < count; ++i) all.K += (int)n_out[i];
+  plan(all, kInputGrad, 1, &n_in, cus, &small);
+  for (int i = 0, n = small ? count : 1; i < count; i += n) {
+    g.A = u(dy[i]); g.B = u(w[i]); g.K = (int)n_out[i]; g.lda = n_out[i];
+    g.add = i == 0 ? u(add) : u(dx);
+    for (int k = 1; k < n; ++k) {
+      g.op[k - 1] = u(dy[k]); g.op_b[k - 1] = u(w[k]); g.size[k - 1] = (int)n_out[k];
+      g.seg_start[k - 1] = g.K / kSlab;
+      g.K += (int)n_out[k];
+    }
+    if (const int rc2 = dtype == MEGA_BF16 ? launch_linear<MEGA_BF16>(g, kInputGrad, 1, &n_in, s) : launch_linear<MEGA_F16>(g, kInputGrad, 1, &n_in, s); rc2 != MEGA_OK) return rc2;
+  }
+  return MEGA_OK;
 }
 
 extern "C" int mega_linear_weight_grads(const void* const* dy, const void* x, int dtype, int64_t tokens, int64_t n_in, int count,

@@ -528,13 +528,39 @@ Tensor input_grad(const Tensor& g, const Tensor& w, const Tensor& sum) {
   if (w.scalar_type() == g.scalar_type() && w.size(0) == n_out && mega_linear_takes(kLinearInputGrad, code, tokens, n_in, 1, &n_out) &&
       dense16(g) && dense16(w) && (!sum.defined() || dense16(sum))) {
     const Tensor dx = sum.defined() ? sum : at::empty({tokens, n_in}, g.options());
-    check(mega_linear_input_grad(g.data_ptr(), w.data_ptr(), ptr(sum), code, tokens, n_out, n_in, dx.data_ptr(), stream_of(g)), "mega_linear_input_grad");
+    const void *gp = g.data_ptr(), *wp = w.data_ptr();
+    check(mega_linear_input_grad(&gp, &wp, ptr(sum), code, tokens, n_in, 1, &n_out, dx.data_ptr(), stream_of(g)), "mega_linear_input_grad");
     return dx;
   }
   if (!sum.defined()) return turned(g, w) ? at::linear(g, transpose_raw(w)) : at::mm(g, w);
   const Tensor wt = turned(g, w) ? transpose_raw(w).t() : w;
   Tensor dx = sum;
   at::addmm_out(dx, sum, g, wt);
+  return dx;
+}
+// sum_i g_i W_i, (tokens, out_i) x (out_i, in): one product along all of the outputs where its launch takes them
+Tensor input_grads(const variable_list& gs, const variable_list& ws) {
+  const int64_t tokens = gs[0].size(0), n_in = ws[0].size(1);
+  const int code = code_of(gs[0].scalar_type()), count = static_cast<int>(gs.size());
+  bool taken = count >= 2 && count <= 3;
+  std::vector<int64_t> n_out;
+  std::vector<const void*> gp, wp;
+  for (size_t i = 0; i < gs.size(); ++i) {
+    n_out.push_back(gs[i].size(1));
+    taken = taken && gs[i].scalar_type() == gs[0].scalar_type() && ws[i].scalar_type() == gs[0].scalar_type() && gs[i].size(0) == tokens &&
+            ws[i].size(0) == n_out[i] && ws[i].size(1) == n_in && dense16(gs[i]) && dense16(ws[i]);
+    if (taken) {
+      gp.push_back(gs[i].data_ptr());
+      wp.push_back(ws[i].data_ptr());
+    }
+  }
+  if (taken && mega_linear_takes(kLinearInputGrad, code, tokens, n_in, count, n_out.data())) {
+    const Tensor dx = at::empty({tokens, n_in}, gs[0].options());
+    check(mega_linear_input_grad(gp.data(), wp.data(), nullptr, code, tokens, n_in, count, n_out.data(), dx.data_ptr(), stream_of(gs[0])), "mega_linear_input_grad");
+    return dx;
+  }
+  Tensor dx;
+  for (size_t i = 0; i < gs.size(); ++i) dx = input_grad(gs[i], ws[i], dx);
   return dx;
 }
 // y_i = x W_i^T (+ bias_i), + residual with one layer, in one launch; nothing where the library's products are faster or
@@ -668,10 +694,12 @@ struct LinearGroupFn : Function<LinearGroupFn> {
     const Tensor x2 = flat(x);
     variable_list wanted;             // the gradients whose layers want a weight gradient,
     std::vector<size_t> place;        // and where in `grads` it goes
+    variable_list all, weights;
     for (size_t i = 0; i < has_bias.size(); ++i) {
       const Tensor& w = saved[1 + i];
       const Tensor g2 = flat(g[i]);
-      if (ctx->needs_input_grad(0)) dx = input_grad(g2, w, dx);
+      all.push_back(g2);
+      weights.push_back(w);
       if (ctx->needs_input_grad(edge++)) {
         wanted.push_back(g2);
         place.push_back(grads.size());
@@ -679,6 +707,7 @@ struct LinearGroupFn : Function<LinearGroupFn> {
       grads.push_back(Tensor());
       if (has_bias[i]) grads.push_back(ctx->needs_input_grad(edge++) ? bias_grad(g2) : Tensor());
     }
+    if (ctx->needs_input_grad(0)) dx = input_grads(all, weights);
     if (wanted.size() <= 3) {
       const variable_list dw = wanted.empty() ? variable_list() : weight_grads(wanted, x2);
       for (size_t i = 0; i < dw.size(); ++i) grads[place[i]] = dw[i];

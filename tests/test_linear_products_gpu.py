@@ -77,8 +77,13 @@ def test_products_match_float64(tokens, n_in, n_out, dtype):
     dx = torch.empty_like(x)
     for i in range(len(w)):  # added up in place
         before = dx.double()
-        call("mega_linear_input_grad", _lib.ptr(dy[i]), _lib.ptr(w[i]), _lib.ptr(dx) if i else None, _lib.i32(code), i64(tokens), i64(n_out[i]), i64(n_in), _lib.ptr(dx))
+        call("mega_linear_input_grad", _pointers(dy[i:i + 1]), _pointers(w[i:i + 1]), _lib.ptr(dx) if i else None, _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(1), (i64 * 1)(n_out[i]), _lib.ptr(dx))
         _close(dx, dy64[i] @ w64[i] + (before if i else 0))
+    # all of the layers at once, onto a summand
+    start = rows(tokens, n_in).to(dtype)
+    dx = torch.full_like(start, float("nan"))
+    call("mega_linear_input_grad", _pointers(dy), _pointers(w), _lib.ptr(start), _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(len(w)), outs, _lib.ptr(dx))
+    _close(dx, sum(a @ b for a, b in zip(dy64, w64)) + start.double())
 
 
 def test_refused_sizes():
