@@ -648,7 +648,7 @@ Tensor linear(const Tensor& x, const Tensor& weight, const Optional& bias, const
   return linear_raw(x, weight, bias, residual);
 }
 
-// several layers of one input: separate products forward, one accumulation of the input's gradient
+// several layers of one input: products, input gradient and weight gradients in one launch each where that is the faster form
 struct LinearGroupFn : Function<LinearGroupFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& x, at::TensorList params, std::vector<bool> has_bias) {
     at::AutoDispatchBelowADInplaceOrView below;

@@ -1,13 +1,12 @@
-"""`nn.Linear` whose input gradient is computed, for large products, from a transposed copy of the weight.
+"""`nn.Linear` on the attention operator's product kernels where they are ahead of the library.
 
 With model-parallel world size 1 the reference's Column/RowParallelLinear are
-`F.linear` (megalodon/modules/model_parallel/layers.py:222-235,321-341), whose
-backward forms `dx = dy @ W` with W (out, in) read along its rows.  On MI355X
-the library GEMM is 13-24 % faster when both operands run along the reduction
-axis (`dy @ Wt^T` with Wt = W^T contiguous, the same layout the forward
-`x @ W^T` uses), and the tiled transpose of W costs 5-30 us, so the backward
-makes that copy where the product is large enough to win it back; the weight gradient of the large layers runs on the attention
-operator's product kernel.  The autograd nodes are C++ (csrc/host/ops.cpp).
+`F.linear` (megalodon/modules/model_parallel/layers.py:222-235,321-341).  Weight gradients, and
+forward products and input gradients of ordinary sizes, run on the library's own kernels, layers of one input in
+one launch; the other products are library GEMMs.  Those of `dx = dy @ W` with W (out, in) read along its rows are
+13-24 % faster on MI355X when both operands run along the reduction axis (`dy @ Wt^T` with Wt = W^T contiguous, the
+layout the forward `x @ W^T` uses), and the tiled transpose of W costs 5-30 us, so the backward makes that copy where the
+product is large enough to win it back.  The autograd nodes are C++ (csrc/host/ops.cpp).
 Values are those of `F.linear`; parameters keep the names and shapes of
 `nn.Linear`, so state dicts are interchangeable."""
 from typing import Optional, Tuple
