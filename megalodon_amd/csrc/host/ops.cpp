@@ -4,6 +4,7 @@
 #include "host.hpp"
 
 #include <ATen/autocast_mode.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/autograd/custom_function.h>
 
 #include <map>
@@ -467,6 +468,8 @@ Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, double scale
 // ---- linear layers --------------------------------------------------------------------------------
 // A matrix as the library's products take it: its own memory (no vmap wrapper), whole rows, 16-byte boundary.
 bool dense16(const Tensor& t) {
+  // (a subclass or a mode that watches the operations -- fake tensors, a count of the flops -- is shown the library's)
+  if (t.key_set().has(c10::DispatchKey::Python) || c10::impl::TorchDispatchModeTLS::any_modes_set()) return false;
   return t.has_storage() && t.is_contiguous() && !lazy(t) && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
 }
 enum { kLinearForward, kLinearInputGrad, kLinearWeightGrad };

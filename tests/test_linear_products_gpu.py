@@ -179,3 +179,20 @@ def test_group_without_gradients():
 
         layers[0].__class__ = Twice
         assert torch.equal(linear_group(x, layers)[0], layers[0](x))
+
+
+def test_products_that_a_mode_watches():
+    """Fake tensors have no memory to launch on, and a mode that counts operations has to see the products."""
+    from torch._subclasses import FakeTensorMode
+    from torch.utils.flop_counter import FlopCounterMode
+    layers = [Linear(256, 128).cuda().bfloat16() for _ in range(2)]
+    x = torch.randn(64, 256, device="cuda").bfloat16().requires_grad_(True)
+    with FlopCounterMode(display=False) as counter:
+        y = layers[0](x)
+        y.backward(torch.ones_like(y))
+        with torch.no_grad():
+            linear_group(x, layers)
+    assert counter.get_total_flops() == 5 * 2 * 64 * 256 * 128
+    with FakeTensorMode(), torch.no_grad():
+        fake = Linear(256, 128, device="cuda", dtype=torch.bfloat16)
+        assert fake(torch.empty(64, 256, device="cuda", dtype=torch.bfloat16)).shape == (64, 128)
