@@ -196,3 +196,32 @@ def test_products_that_a_mode_watches():
     with FakeTensorMode(), torch.no_grad():
         fake = Linear(256, 128, device="cuda", dtype=torch.bfloat16)
         assert fake(torch.empty(64, 256, device="cuda", dtype=torch.bfloat16)).shape == (64, 128)
+
+
+def test_products_under_capture():
+    """Captured: layers of one input with last tiles cut along k (parts from the graph's pool), replayed on other inputs with
+    eager work between."""
+    torch.manual_seed(7)
+    layers = [Linear(4096, o).cuda().bfloat16() for o in (5504, 5504)]
+    i64 = ctypes.c_int64
+    tokens = 1531
+    size = ctypes.CFUNCTYPE(i64, i64, i64, ctypes.c_int, ctypes.c_void_p)(("mega_linear_fwd_workspace_bytes", _lib.load()))
+    assert size(tokens, 4096, 2, (i64 * 2)(5504, 5504)) > 0
+    x = torch.randn(tokens, 4096, device="cuda").bfloat16()
+    with torch.no_grad():
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            linear_group(x, layers)
+        torch.cuda.current_stream().wait_stream(side)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            ys = linear_group(x, layers)
+        for _ in range(3):
+            x.copy_(torch.randn(tokens, 4096, device="cuda"))
+            want = linear_group(x, layers)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(ys, want))
