@@ -408,23 +408,22 @@ int mega_linear_weight_grad(const void* dy, const void* x, int dtype, int64_t to
  * (n_out[i] each; `count`) in one launch: tensors of `dtype` (MEGA_BF16 / MEGA_F16, float32 accumulation, one
  * rounding), contiguous, on 16-byte boundaries, n_in and n_out multiples of 8, every matrix of fewer than 2^30 elements.
  *   fwd:          y_i (tokens, n_out_i) = x (tokens, n_in) w_i^T + bias_i + add; bias, an entry of it and add may be
- *                 null; add (tokens, n_out) with one layer only; n_in a multiple of 64.  `workspace`:
- *                 mega_linear_fwd_workspace_bytes bytes (up to 64 MiB; for many sizes 0), or null: no product is cut
- *                 along k then, which some sizes are slower without.
+ *                 null; add (tokens, n_out) with one layer only; n_in a multiple of 64.
  *   input_grad:   dx = sum_i dy_i w_i + add; add (tokens, n_in) or null, may be dx itself; n_out a multiple of 64.
  *   weight_grads: dw_i = dy_i^T x.
+ * `workspace` of fwd and weight_grads: mega_linear_workspace_bytes(0 or 2, ...) bytes (up to 64 MiB; for many sizes 0), or
+ * null: no product is cut along its reduction axis then, which makes some sizes slower.
  * `takes` (kind 0, 1, 2 in this order; input_grad: count 1) is 1 where the launch is expected to be
  * faster than a general library's products, 0 where it is not or where the sizes are refused. */
 int mega_linear_takes(int kind, int dtype, int64_t tokens, int64_t n_in, int count, const int64_t* n_out);
 int mega_linear_fwd(const void* x, const void* const* w, const void* const* bias, const void* add,
                     int dtype, int64_t tokens, int64_t n_in, int count, const int64_t* n_out,
                     void* const* y, void* workspace, void* stream);
-int64_t mega_linear_fwd_workspace_bytes(int64_t tokens, int64_t n_in, int count, const int64_t* n_out);
 int mega_linear_input_grad(const void* const* dy, const void* const* w, const void* add, int dtype,
                            int64_t tokens, int64_t n_in, int count, const int64_t* n_out, void* dx, void* stream);
-int mega_linear_weight_grads(const void* const* dy, const void* x, int dtype, int64_t tokens,
-                             int64_t n_in, int count, const int64_t* n_out, void* const* dw,
-                             void* stream);
+int mega_linear_weight_grads(const void* const* dy, const void* x, int dtype, int64_t tokens, int64_t n_in,
+                             int count, const int64_t* n_out, void* const* dw, void* workspace, void* stream);
+int64_t mega_linear_workspace_bytes(int kind, int64_t tokens, int64_t n_in, int count, const int64_t* n_out);
 
 /* ------------------------------------------------------------------------
  * Convolution with spectra kept between forward and backward.

@@ -135,7 +135,7 @@ struct GemmParams {
   int seg_start[2];
   int kva;      // as kvb, for a k-major A (LIN: rows behind it are not there; else they hold zeros)
   // CUT: items full .. items - 1, fewer than there are CUs, are cut along k into `cut` parts; float32 sums of part i
-  // of item full + r at parts + (r cut + i) 256 x 256, as the waves hold them (linear_parts_kernel adds them up).
+  // of item full + r at parts + (r cut + i) T T, as the waves hold them (linear_parts_kernel adds them up).
   int full, cut;
   float* parts;
   int split_ok;  // (the launcher's: there is memory for the parts)
@@ -551,6 +551,33 @@ __device__ __forceinline__ void store_tile(const floatx16 (&acc)[IT][2], const G
   }
 }
 
+// CUT: a workgroup's part of an item, neighbours on an XCD; false where there is none.
+__device__ __forceinline__ bool cut_item(const GemmParams& p, int* item, int* part) {
+  const int G = static_cast<int>(gridDim.x), lin = static_cast<int>(blockIdx.x);
+  const int left = p.items - p.full, at = lin % kXcds * (G / kXcds) + lin / kXcds;
+  if (at >= left * p.cut) return false;
+  *part = at / left;
+  *item = p.full + at % left;
+  return true;
+}
+// ... and where a wave's sums of it go (kept as they are, 16 bytes a lane and store)
+template <int IT, int NW>
+__device__ __forceinline__ void store_part(const floatx16 (&acc)[IT][2], const GemmParams& p, int item, int part, int wave, int lane) {
+  char* const dst = reinterpret_cast<char*>(p.parts + ((static_cast<int64_t>(item - p.full) * p.cut + part) * NW + wave) * (32 * IT * 64));
+  uint32_t at = 16 * lane;
+#pragma unroll
+  for (int i = 0; i < IT; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      asm volatile("" : "+v"(at));  // (one address that advances, not one for each store)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4)
+        *reinterpret_cast<float4*>(dst + at + 1024 * q4) =
+            make_float4(acc[i][j][4 * q4], acc[i][j][4 * q4 + 1], acc[i][j][4 * q4 + 2], acc[i][j][4 * q4 + 3]);
+      at += 4096;
+    }
+}
+
 // ---- the same product with the operand slabs sent from memory straight into LDS ------
 // Eight waves of 128 x 64 as above, aligned operands only.  `global_load_lds_dwordx4`
 // writes the 64 lanes' 16-byte pieces to 1 KB of consecutive LDS (base in M0), so no slab
@@ -597,7 +624,7 @@ __device__ __forceinline__ void load_to_lds16(u32x4 buffer, uint32_t offset, uin
 // T: the workgroup's tile, 256 (2 x 4 waves of 128 x 64) or 128 (2 x 2 waves of 64 x 64, two workgroups per CU).
 // RAG: p.kvb and p.ms are set (B k-major).  SEG: p.seg_start and the operands behind it are (apart, since the choice of the
 // operands with every request costs a product of one pair 10 %: 4096 x 1024 -> 2752 21.3 us, 23.6 so)
-template <int DT, bool TA, bool TB, bool RAG = false, int T = kTile, bool LIN = false, bool SEG = false>
+template <int DT, bool TA, bool TB, bool RAG = false, int T = kTile, bool LIN = false, bool SEG = false, bool CUT = false>
 __global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
   extern __shared__ __align__(16) uint16_t smem[];
   constexpr int JN = 2, NL = 2;
@@ -611,8 +638,12 @@ __global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
   const int wm = wave / (NW / 2), wn = wave % (NW / 2);
   // work items as in gemm_kernel
   const int G = static_cast<int>(gridDim.x), lin = static_cast<int>(blockIdx.x);
-  int it_lo, it_hi, it_step;
-  if (G % kXcds == 0) {
+  int it_lo, it_hi, it_step, part = 0;
+  if constexpr (CUT) {
+    if (!cut_item(p, &it_lo, &part)) return;
+    it_hi = it_lo + 1;
+    it_step = 1;
+  } else if (G % kXcds == 0) {
     const int xcd = lin % kXcds;
     it_lo = static_cast<int>(static_cast<int64_t>(p.items) * xcd / kXcds) + lin / kXcds;
     it_hi = static_cast<int>(static_cast<int64_t>(p.items) * (xcd + 1) / kXcds);
@@ -622,7 +653,7 @@ __global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
     it_hi = p.items;
     it_step = G;
   }
-  if (T != kTile && p.snake) it_lo = lin, it_hi = p.items, it_step = G;  // one item per workgroup, in order
+  if (!CUT && T != kTile && p.snake) it_lo = lin, it_hi = p.items, it_step = G;  // one item per workgroup, in order
   for (int item = it_lo; item < it_hi; item += it_step) {
   int zz = item / p.per_batch;
   const int rem = item % p.per_batch;
@@ -680,6 +711,11 @@ __global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
   int kb = 0, ke = p.K;
   if (p.k_mode == 1) ke = min(p.K, ((mt + 1) * T + p.off + kSlab - 1) / kSlab * kSlab);
   if (p.k_mode == 2) kb = min(p.K, max(0, mt * T - p.off) / kSlab * kSlab);
+  if constexpr (CUT) {
+    const int slabs = p.K / kSlab;
+    kb = slabs * part / p.cut * kSlab;
+    ke = slabs * (part + 1) / p.cut * kSlab;
+  }
   const int nslab = (ke - kb + kSlab - 1) / kSlab;
 
   floatx16 acc[IT][JN];
@@ -847,7 +883,8 @@ __global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
 #undef MEGA_DMA_STEP
 #undef MEGA_SGB
 
-  store_tile<DT, IT, LIN>(acc, p, t, RAG && !LIN ? p.ms : t.M, m0 + wm * 32 * IT, n0 + wn * 64, lane, smem + wave * 32 * IT * (64 + 8));
+  if constexpr (CUT) store_part<IT, NW>(acc, p, item, part, wave, lane);
+  else store_tile<DT, IT, LIN>(acc, p, t, RAG && !LIN ? p.ms : t.M, m0 + wm * 32 * IT, n0 + wn * 64, lane, smem + wave * 32 * IT * (64 + 8));
   // the output regions overlap the slab buffers: every read of this tile's epilogue
   // retires before the next tile's first slab is requested
   lds_barrier();
@@ -882,11 +919,8 @@ __global__ __launch_bounds__(2 * T) void gemm_dma64_kernel(const GemmParams p) {
   const int wm = wave / (NW / 2), wn = wave % (NW / 2);
   const int G = static_cast<int>(gridDim.x), lin = static_cast<int>(blockIdx.x);
   int it_lo, it_hi, it_step, part = 0;
-  if constexpr (CUT) {  // one part of one item; neighbours on an XCD
-    const int left = p.items - p.full, at = lin % kXcds * (G / kXcds) + lin / kXcds;
-    if (at >= left * p.cut) return;
-    part = at / left;
-    it_lo = p.full + at % left;
+  if constexpr (CUT) {
+    if (!cut_item(p, &it_lo, &part)) return;
     it_hi = it_lo + 1;
     it_step = 1;
   } else if (G % kXcds == 0) {
@@ -1073,19 +1107,7 @@ __global__ __launch_bounds__(2 * T) void gemm_dma64_kernel(const GemmParams p) {
 #undef MEGA_SGB
 
   if constexpr (CUT) {
-    char* const dst = reinterpret_cast<char*>(p.parts + ((static_cast<int64_t>(item - p.full) * p.cut + part) * NW + wave) * (32 * IT * 64));
-    uint32_t at = 16 * lane;
-#pragma unroll
-    for (int i = 0; i < IT; ++i)
-#pragma unroll
-      for (int j = 0; j < JN; ++j) {
-        asm volatile("" : "+v"(at));  // (one address that advances, not one for each store)
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4)
-          *reinterpret_cast<float4*>(dst + at + 1024 * q4) =
-              make_float4(acc[i][j][4 * q4], acc[i][j][4 * q4 + 1], acc[i][j][4 * q4 + 2], acc[i][j][4 * q4 + 3]);
-        at += 4096;
-      }
+    store_part<IT, NW>(acc, p, item, part, wave, lane);
   } else {
     store_tile<DT, IT, LIN>(acc, p, t, t.M, m0 + wm * 32 * IT, n0 + wn * 64, lane, smem + wave * 32 * IT * (64 + 8));
   }
@@ -1094,36 +1116,36 @@ __global__ __launch_bounds__(2 * T) void gemm_dma64_kernel(const GemmParams p) {
   }  // work item
 }
 
-// The parts of gemm_dma64_kernel's last tiles added up, in order: 32 x 64 values of a wave of that kernel per wave of this one,
-// 32 workgroups of one wave a tile, so that the parts of few tiles are read by many CUs.
-template <int DT>
+// The parts of cut tiles added up, in order: 32 x 64 values of a wave of the product per workgroup, one wave, so that the parts
+// of few tiles are read by many CUs.
+template <int DT, int T, bool TA, bool TB>
 __global__ __launch_bounds__(kWave) void linear_parts_kernel(const GemmParams p) {
   __shared__ __align__(16) uint16_t stage[32 * (64 + 8)];
-  constexpr int kPart = 32 * 4 * 64;  // values of a wave of the product
-  const int lane = threadIdx.x, i = blockIdx.x % 4;
-  const int tile = blockIdx.x / 32, of = blockIdx.x / 4 % 8, wm = of / 4, wn = of % 4;
+  constexpr int IT = T / 64, NW = T / 32, kPart = 32 * IT * 64;  // blocks of 32 rows of a wave, waves, values of a wave
+  const int lane = threadIdx.x, i = blockIdx.x % IT;
+  const int tile = blockIdx.x / (IT * NW), of = blockIdx.x / IT % NW, wm = of / (NW / 2), wn = of % (NW / 2);
   int mt, nt;
   plain_tile(p, p.full + tile, &mt, &nt);
-  const Tile t = tile_of<true, false, false>(p, 0, 0, mt, nt);
-  const float* src = p.parts + (static_cast<int64_t>(tile) * p.cut * 8 + of) * kPart + i * (32 * 64) + 4 * lane;
+  const Tile t = tile_of<true, TA, TB>(p, 0, 0, mt, nt);
+  const float* src = p.parts + (static_cast<int64_t>(tile) * p.cut * NW + of) * kPart + i * (32 * 64) + 4 * lane;
   floatx16 acc[1][2];
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[0][j][r] = 0.f;
-#pragma unroll 2
+#pragma unroll 4
   for (int part = 0; part < p.cut; ++part)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4) {
-        const float4 v = *reinterpret_cast<const float4*>(src + static_cast<int64_t>(part) * 8 * kPart + (j * 4 + q4) * 256);
+        const float4 v = *reinterpret_cast<const float4*>(src + static_cast<int64_t>(part) * NW * kPart + (j * 4 + q4) * 256);
         acc[0][j][4 * q4] += v.x;
         acc[0][j][4 * q4 + 1] += v.y;
         acc[0][j][4 * q4 + 2] += v.z;
         acc[0][j][4 * q4 + 3] += v.w;
       }
-  store_tile<DT, 1, true>(acc, p, t, t.M, t.mt * kTile + wm * 128 + 32 * i, t.nt * kTile + wn * 64, lane, stage);
+  store_tile<DT, 1, true>(acc, p, t, t.M, t.mt * T + wm * 32 * IT + 32 * i, t.nt * T + wn * 64, lane, stage);
 }
 
 // ---- one k-contiguous and one k-major operand: A in slabs of 64 k, B in slabs of 32 k ------
@@ -1995,6 +2017,7 @@ void lay_out(GemmParams& q, int kind, int count, const int64_t* sizes, int T) {
   q.mt_count = kind == kWeightGrad ? along : tiles(q.M);
   q.nt_count = kind == kForward ? along : tiles(q.N);
   q.per_batch = q.items = q.mt_count * q.nt_count;
+  q.full = q.items, q.cut = 0;
 }
 
 int compute_units(int* cus) {
@@ -2018,7 +2041,6 @@ double estimate_cut(GemmParams& q, double slabs, int cus) {
   const auto round = [&](double tiles, double k) { return k * (0.45 + 0.35 * tiles / grid) + 5; };
   const double whole = full / grid * round(grid, slabs) + 3;
   double best = whole + (left > 0 ? round(left, slabs) : 0);
-  q.full = q.items, q.cut = 0;
   for (int cut = 2; cut <= 8 && left > 0 && left * cut <= grid && slabs >= 16 * cut; ++cut) {
     const double t = whole + round(left * cut, slabs / cut) + 0.12 * left * cut + 14;
     if (t < best) best = t, q.full = full, q.cut = cut;
@@ -2033,7 +2055,17 @@ double estimate(GemmParams& q, int kind, int T, int cus) {
     if (kind == kForward) return rounds * (slabs * (0.45 + 0.35 * load) + 5) + 3;
     return rounds * (slabs * (0.42 + 0.37 * load) + 5) + 2;
   }
-  if (kind == kWeightGrad) return rounds * slabs * 0.23 + 3;
+  if (kind == kWeightGrad) {
+    // Tiles for half of the CUs or fewer are cut along the tokens, as forward products are.  us, whole / cut: 4096 tokens, 2048 x
+    // 1024 (128 tiles) 28.5 / 26.8, 1024 x 1024 28.4 / 23.9, 512 x 512 22.4 / 20.5; 8192 tokens 51 / 40 and (512 x 512)
+    // 50 / 26; 32768 tokens 187 / 127, 191 / 72, 186 / 41.
+    double best = rounds * slabs * 0.23 + 3;
+    for (int cut = 2; q.split_ok && cut <= 16 && q.items * cut <= cus && slabs >= 16 * cut; ++cut) {
+      const double t = slabs / cut * 0.23 + 0.03 * q.items * cut + 7;
+      if (t < best) best = t, q.full = 0, q.cut = cut;
+    }
+    return best;
+  }
   if (kind == kForward) return rounds * (slabs * 0.255 + 1.3) + 3;
   return rounds * (slabs * 0.27 + 1) + 3;
 }
@@ -2045,8 +2077,7 @@ double plan(GemmParams& q, int kind, int count, const int64_t* sizes, int cus, b
   lay_out(q, kind, count, sizes, kSmall);
   const double tl = estimate(l, kind, kTile, cus), ts = estimate(q, kind, kSmall, cus);
   *small = ts <= tl;
-  if (*small) q.full = q.items, q.cut = 0;
-  else q = l;
+  if (!*small) q = l;
   return std::min(ts, tl);
 }
 
@@ -2106,7 +2137,7 @@ int launch_linear(GemmParams q, int kind, int count, const int64_t* sizes, hipSt
         if (const int rc = launch_tiles<gemm_dma64_kernel<DT, false, false, kTile, true>>(whole, grid, threads, lds, s); rc != MEGA_OK) return rc;
       grid = (left * q.cut + kXcds - 1) / kXcds * kXcds;
       if (const int rc = launch_tiles<gemm_dma64_kernel<DT, false, false, kTile, true, true>>(q, grid, threads, lds, s); rc != MEGA_OK) return rc;
-      return launch_tiles<linear_parts_kernel<DT>>(q, left * 32, kWave, 0, s);
+      return launch_tiles<linear_parts_kernel<DT, kTile, false, false>>(q, left * 32, kWave, 0, s);
     }
     if (!small) return launch_tiles<gemm_dma64_kernel<DT, false, false, kTile, true>>(q, grid, threads, lds, s);
     if (q.items <= cus) return launch_tiles<gemm_dma_kernel<DT, false, false, false, kSmall, true>>(q, grid, threads, lds, s);
@@ -2121,6 +2152,13 @@ int launch_linear(GemmParams q, int kind, int count, const int64_t* sizes, hipSt
   q.kva = q.kvb = q.K;
   q.ms = q.M;
   q.K = (q.K + kSlab - 1) / kSlab * kSlab;
+  if (small && q.cut > 0) {
+    grid = (q.items * q.cut + kXcds - 1) / kXcds * kXcds;
+    const int rc = rag ? launch_tiles<gemm_dma_kernel<DT, true, true, true, kSmall, true, false, true>>(q, grid, threads, lds, s)
+                       : launch_tiles<gemm_dma_kernel<DT, true, true, false, kSmall, true, false, true>>(q, grid, threads, lds, s);
+    if (rc != MEGA_OK) return rc;
+    return launch_tiles<linear_parts_kernel<DT, kSmall, true, true>>(q, q.items * 8, kWave, 0, s);
+  }
   if (rag) {
     if (!small) return launch_tiles<gemm_dma_kernel<DT, true, true, true, kTile, true>>(q, grid, threads, lds, s);
     return launch_tiles<gemm_dma_kernel<DT, true, true, true, kSmall, true>>(q, grid, threads, lds, s);
@@ -2152,11 +2190,9 @@ extern "C" int mega_linear_takes(int kind, int dtype, int64_t tokens, int64_t n_
   if (kind == kWeightGrad) {
     // Both operands run across the reduction axis, the library's slowest layout: this kernel is ahead at every size (us,
     // library / here): 4096 tokens, 256 + 2048 + 1024 x 1024 91 / 30, 2 x 2752 x 1024 85 / 58, 2 x 5504 x 2048 174 / 166, 11008 x 4096
-    // 380 / 281; 4084 tokens, 2048 x 5504 106 / 82; 1531, 4096 x 11008 174 / 122; 32768, 3328 x 1024 595 / 280, except a long
-    // reduction over few tiles, which the library cuts up.
-    int64_t tiles = 0;
-    for (int i = 0; i < count; ++i) tiles += (n_out[i] + kSmall - 1) / kSmall * ((n_in + kSmall - 1) / kSmall);
-    return tokens <= 4096 || 4 * tiles >= cus;
+    // 380 / 281; 4084 tokens, 2048 x 5504 106 / 82; 1531, 4096 x 11008 174 / 122; 32768, 3328 x 1024 595 / 280, 1024 x 1024 198 / 72,
+    // 512 x 512 152 / 41, 64 x 64 169 / 31.
+    return 1;
   }
   GemmParams q{};
   bool apart;
@@ -2179,22 +2215,23 @@ extern "C" int mega_linear_takes(int kind, int dtype, int64_t tokens, int64_t n_
   return here <= library;
 }
 
-extern "C" int64_t mega_linear_fwd_workspace_bytes(int64_t tokens, int64_t n_in, int count, const int64_t* n_out) {
-  if (check_linear("mega_linear_fwd_workspace_bytes", kForward, MEGA_BF16, tokens, n_in, count, n_out) != MEGA_OK) return 0;
+extern "C" int64_t mega_linear_workspace_bytes(int kind, int64_t tokens, int64_t n_in, int count, const int64_t* n_out) {
+  if ((kind != kForward && kind != kWeightGrad) || check_linear("mega_linear_workspace_bytes", kind, MEGA_BF16, tokens, n_in, count, n_out) != MEGA_OK) return 0;
   int cus = 0;
   if (compute_units(&cus) != MEGA_OK) return 0;
   GemmParams q{};
-  q.M = (int)tokens; q.N = (int)n_out[0]; q.K = (int)n_in;
+  q.M = (int)(kind == kForward ? tokens : n_out[0]); q.N = (int)(kind == kForward ? n_out[0] : n_in); q.K = (int)(kind == kForward ? n_in : tokens);
   q.split_ok = 1;
   bool apart, small;
-  plan_group(q, kForward, count, n_out, cus, &apart);
-  int64_t parts = 0;
+  plan_group(q, kind, count, n_out, cus, &apart);
+  int64_t values = 0;
   for (int i = 0; i < (apart ? count : 1); ++i) {
-    GemmParams o = apart ? one_of(q, kForward, i, n_out[i]) : q;
-    plan(o, kForward, apart ? 1 : count, apart ? n_out + i : n_out, cus, &small);
-    parts = std::max(parts, static_cast<int64_t>(o.items - o.full) * o.cut);
+    GemmParams o = apart ? one_of(q, kind, i, n_out[i]) : q;
+    plan(o, kind, apart ? 1 : count, apart ? n_out + i : n_out, cus, &small);
+    const int64_t tile = small ? kSmall : kTile;
+    values = std::max(values, static_cast<int64_t>(o.items - o.full) * o.cut * tile * tile);
   }
-  return parts * (sizeof(float) * kTile * kTile);
+  return values * static_cast<int64_t>(sizeof(float));
 }
 
 extern "C" int mega_linear_fwd(const void* x, const void* const* w, const void* const* bias, const void* add, int dtype,
@@ -2252,16 +2289,17 @@ extern "C" int mega_linear_input_grad(const void* const* dy, const void* const* 
 }
 
 extern "C" int mega_linear_weight_grads(const void* const* dy, const void* x, int dtype, int64_t tokens, int64_t n_in, int count,
-                                        const int64_t* n_out, void* const* dw, void* stream) {
+                                        const int64_t* n_out, void* const* dw, void* workspace, void* stream) {
   const int rc = check_linear("mega_linear_weight_grads", kWeightGrad, dtype, tokens, n_in, count, n_out);
   if (rc != MEGA_OK) return rc;
-  MEGA_CHECK_ARG(dy && dw && x && aligned16(x), "mega_linear_weight_grads: null or misaligned pointer");
+  MEGA_CHECK_ARG(dy && dw && x && aligned16(x) && aligned16(workspace), "mega_linear_weight_grads: null or misaligned pointer");
   for (int i = 0; i < count; ++i) MEGA_CHECK_ARG(dy[i] && dw[i] && aligned16(dy[i]) && aligned16(dw[i]), "mega_linear_weight_grads: null or misaligned pointer");
   const auto u = [](const void* q) { return static_cast<const uint16_t*>(q); };
   GemmParams g{};
   g.A = u(dy[0]); g.B = u(x); g.C = static_cast<uint16_t*>(dw[0]);
   g.M = (int)n_out[0]; g.N = (int)n_in; g.K = (int)tokens;
   g.lda = n_out[0]; g.ldb = n_in; g.ldc = n_in; g.ta = 1; g.tb = 1;
+  g.parts = static_cast<float*>(workspace); g.split_ok = workspace != nullptr;
   for (int i = 1; i < count; ++i) g.op[i - 1] = u(dy[i]), g.out[i - 1] = static_cast<uint16_t*>(dw[i]);
   hipStream_t s = static_cast<hipStream_t>(stream);
   return dtype == MEGA_BF16 ? launch_linear<MEGA_BF16>(g, kWeightGrad, count, n_out, s) : launch_linear<MEGA_F16>(g, kWeightGrad, count, n_out, s);

@@ -473,6 +473,11 @@ bool dense16(const Tensor& t) {
   return t.has_storage() && t.is_contiguous() && !lazy(t) && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
 }
 enum { kLinearForward, kLinearInputGrad, kLinearWeightGrad };
+// memory for the parts of products that are cut along their reduction axis
+Tensor parts_of(int kind, const Tensor& x, int64_t tokens, int64_t n_in, const std::vector<int64_t>& n_out) {
+  const int64_t size = mega_linear_workspace_bytes(kind, tokens, n_in, static_cast<int>(n_out.size()), n_out.data());
+  return size > 0 ? at::empty({size}, x.options().dtype(at::kByte)) : Tensor();
+}
 // dW_i = g_i^T x, (out_i, in) from (tokens, out_i) and (tokens, in), for layers of one input in one launch.
 variable_list weight_grads(variable_list gs, const Tensor& x) {
   const int64_t tokens = x.size(0), n_in = x.size(1);
@@ -498,7 +503,8 @@ variable_list weight_grads(variable_list gs, const Tensor& x) {
         from.push_back(g.data_ptr());
         to.push_back(dw.back().data_ptr());
       }
-      check(mega_linear_weight_grads(from.data(), xc.data_ptr(), code, tokens, n_in, static_cast<int>(gs.size()), n_out.data(), to.data(), stream_of(x)), "mega_linear_weight_grads");
+      const Tensor ws = parts_of(kLinearWeightGrad, x, tokens, n_in, n_out);
+      check(mega_linear_weight_grads(from.data(), xc.data_ptr(), code, tokens, n_in, static_cast<int>(gs.size()), n_out.data(), to.data(), ptr(ws), stream_of(x)), "mega_linear_weight_grads");
       return dw;
     }
   }
@@ -596,8 +602,7 @@ std::optional<variable_list> products(const Tensor& x, const variable_list& w, c
     bp.push_back(bias[i].has_value() ? bias[i]->data_ptr() : nullptr);
     yp.push_back(y.back().data_ptr());
   }
-  const int64_t bytes = mega_linear_fwd_workspace_bytes(tokens, n_in, count, n_out.data());
-  const Tensor ws = bytes > 0 ? at::empty({bytes}, x.options().dtype(at::kByte)) : Tensor();
+  const Tensor ws = parts_of(kLinearForward, x, tokens, n_in, n_out);
   check(mega_linear_fwd(x.data_ptr(), wp.data(), bp.data(), residual.has_value() ? residual->data_ptr() : nullptr, code, tokens, n_in, count, n_out.data(), yp.data(), ptr(ws), stream_of(x)), "mega_linear_fwd");
   return y;
 }

@@ -17,6 +17,12 @@ def _pointers(tensors):
     return (ctypes.c_void_p * len(tensors))(*[0 if t is None else t.data_ptr() for t in tensors])
 
 
+def _parts(kind, tokens, n_in, n_out):
+    i64 = ctypes.c_int64
+    fn = ctypes.CFUNCTYPE(i64, ctypes.c_int, i64, i64, ctypes.c_int, ctypes.c_void_p)(("mega_linear_workspace_bytes", _lib.load()))
+    return fn(kind, tokens, n_in, len(n_out), (i64 * len(n_out))(*n_out))
+
+
 def _poisoned(t):  # NaN behind the last element
     buf = torch.full((t.numel() + 4096,), float("nan"), dtype=t.dtype, device="cuda")
     return buf[:t.numel()].view(t.shape).copy_(t)
@@ -57,12 +63,14 @@ def test_products_match_float64(tokens, n_in, n_out, dtype):
 
     def fwd(w, bias, add, n_out, y):
         n, outs = len(w), (i64 * len(w))(*n_out)
-        size = _lib.load().mega_linear_fwd_workspace_bytes(i64(tokens), i64(n_in), n, outs)
+        size = _parts(0, tokens, n_in, n_out)
         ws = torch.empty(size, dtype=torch.uint8, device="cuda")
         call("mega_linear_fwd", _lib.ptr(x), _pointers(w), bias and _pointers(bias), add, _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(n), outs, _pointers(y), _lib.ptr(ws) if size else None)
 
     fwd(w, bias, None, n_out, y)
-    call("mega_linear_weight_grads", _pointers(dy), _lib.ptr(x), _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(len(w)), outs, _pointers(dw))
+    size = _parts(2, tokens, n_in, n_out)
+    ws = torch.empty(size, dtype=torch.uint8, device="cuda")
+    call("mega_linear_weight_grads", _pointers(dy), _lib.ptr(x), _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(len(w)), outs, _pointers(dw), _lib.ptr(ws) if size else None)
     x64, w64, dy64 = x.double(), [t.double() for t in w], [t.double() for t in dy]
     for i in range(len(w)):
         _close(y[i], x64 @ w64[i].t() + (0 if bias[i] is None else bias[i].double()))
@@ -138,8 +146,7 @@ def test_last_tiles_cut_along_k(tokens, n_in, n_out, dtype):
     w = [_poisoned((rows(o, n_in) / n_in ** 0.5).to(dtype)) for o in n_out]
     bias, add = [rows(o).to(dtype) for o in n_out], rows(tokens, n_out[0]).to(dtype)
     i64, outs = ctypes.c_int64, (ctypes.c_int64 * len(n_out))(*n_out)
-    size = ctypes.CFUNCTYPE(i64, i64, i64, ctypes.c_int, ctypes.c_void_p)(("mega_linear_fwd_workspace_bytes", _lib.load()))
-    bytes_, summed = size(tokens, n_in, len(n_out), outs), add if len(n_out) == 1 else None
+    bytes_, summed = _parts(0, tokens, n_in, n_out), add if len(n_out) == 1 else None
     assert 0 < bytes_ <= 64 << 20
 
     def run(ws):
@@ -203,10 +210,8 @@ def test_products_under_capture():
     eager work between."""
     torch.manual_seed(7)
     layers = [Linear(4096, o).cuda().bfloat16() for o in (5504, 5504)]
-    i64 = ctypes.c_int64
     tokens = 1531
-    size = ctypes.CFUNCTYPE(i64, i64, i64, ctypes.c_int, ctypes.c_void_p)(("mega_linear_fwd_workspace_bytes", _lib.load()))
-    assert size(tokens, 4096, 2, (i64 * 2)(5504, 5504)) > 0
+    assert _parts(0, tokens, 4096, (5504, 5504)) > 0
     x = torch.randn(tokens, 4096, device="cuda").bfloat16()
     with torch.no_grad():
         side = torch.cuda.Stream()
@@ -225,3 +230,31 @@ def test_products_under_capture():
             graph.replay()
             torch.cuda.synchronize()
             assert all(torch.equal(a, b) for a, b in zip(ys, want))
+
+
+@pytest.mark.parametrize("tokens,n_in,n_out,dtype", [
+    (4096, 1024, [2048], torch.bfloat16),       # 128 tiles, two parts
+    (4093, 1024, [1000], torch.float16),        # 64 tiles that end inside, tokens off the slabs, four parts of unequal length
+    (2500, 136, [256, 72], torch.bfloat16),     # two layers, three tiles
+])
+def test_weight_gradients_cut_along_the_tokens(tokens, n_in, n_out, dtype):
+    g = torch.Generator("cuda").manual_seed(tokens)
+    rows = lambda *s: _poisoned(torch.randn(*s, generator=g, device="cuda").to(dtype))
+    x, dy, i64 = rows(tokens, n_in), [rows(tokens, o) for o in n_out], ctypes.c_int64
+    size = _parts(2, tokens, n_in, n_out)
+    assert 0 < size <= 64 << 20
+
+    def run(ws):
+        dw = [torch.full((o, n_in), float("nan"), dtype=dtype, device="cuda") for o in n_out]
+        _lib.call("mega_linear_weight_grads", _pointers(dy), _lib.ptr(x), _lib.i32(_lib.dtype_code(dtype)), i64(tokens), i64(n_in),
+                  _lib.i32(len(dy)), (i64 * len(n_out))(*n_out), _pointers(dw), ws, _lib.stream_ptr(x.device))
+        return dw
+
+    parts = torch.full((size + 4096,), 255, dtype=torch.uint8, device="cuda")  # NaN
+    once, again, whole = run(_lib.ptr(parts)), run(_lib.ptr(parts)), run(None)
+    assert (parts[size:] == 255).all()
+    for i in range(len(n_out)):
+        want = dy[i].double().t() @ x.double()
+        _close(once[i], want)
+        _close(whole[i], want)
+        assert torch.equal(once[i], again[i])
