@@ -560,13 +560,14 @@ __device__ __forceinline__ bool cut_item(const GemmParams& p, int* item, int* pa
   *item = p.full + at % left;
   return true;
 }
-// ... and where a wave's sums of it go (kept as they are, 16 bytes a lane and store)
+// ... and where a wave's sums of it go (kept as they are, 16 bytes a lane and store), those blocks of 32 that have some of its `rows`
 template <int IT, int NW>
-__device__ __forceinline__ void store_part(const floatx16 (&acc)[IT][2], const GemmParams& p, int item, int part, int wave, int lane) {
+__device__ __forceinline__ void store_part(const floatx16 (&acc)[IT][2], const GemmParams& p, int item, int part, int wave, int lane, int rows) {
   char* const dst = reinterpret_cast<char*>(p.parts + ((static_cast<int64_t>(item - p.full) * p.cut + part) * NW + wave) * (32 * IT * 64));
   uint32_t at = 16 * lane;
 #pragma unroll
-  for (int i = 0; i < IT; ++i)
+  for (int i = 0; i < IT; ++i) {
+    if (32 * i >= rows) break;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       asm volatile("" : "+v"(at));  // (one address that advances, not one for each store)
@@ -576,6 +577,7 @@ __device__ __forceinline__ void store_part(const floatx16 (&acc)[IT][2], const G
             make_float4(acc[i][j][4 * q4], acc[i][j][4 * q4 + 1], acc[i][j][4 * q4 + 2], acc[i][j][4 * q4 + 3]);
       at += 4096;
     }
+  }
 }
 
 // ---- the same product with the operand slabs sent from memory straight into LDS ------
@@ -883,7 +885,7 @@ __global__ __launch_bounds__(2 * T) void gemm_dma_kernel(const GemmParams p) {
 #undef MEGA_DMA_STEP
 #undef MEGA_SGB
 
-  if constexpr (CUT) store_part<IT, NW>(acc, p, item, part, wave, lane);
+  if constexpr (CUT) store_part<IT, NW>(acc, p, item, part, wave, lane, t.M - m0 - wm * 32 * IT);
   else store_tile<DT, IT, LIN>(acc, p, t, RAG && !LIN ? p.ms : t.M, m0 + wm * 32 * IT, n0 + wn * 64, lane, smem + wave * 32 * IT * (64 + 8));
   // the output regions overlap the slab buffers: every read of this tile's epilogue
   // retires before the next tile's first slab is requested
@@ -1107,7 +1109,7 @@ __global__ __launch_bounds__(2 * T) void gemm_dma64_kernel(const GemmParams p) {
 #undef MEGA_SGB
 
   if constexpr (CUT) {
-    store_part<IT, NW>(acc, p, item, part, wave, lane);
+    store_part<IT, NW>(acc, p, item, part, wave, lane, t.M - m0 - wm * 32 * IT);
   } else {
     store_tile<DT, IT, LIN>(acc, p, t, t.M, m0 + wm * 32 * IT, n0 + wn * 64, lane, smem + wave * 32 * IT * (64 + 8));
   }
@@ -1127,6 +1129,7 @@ __global__ __launch_bounds__(kWave) void linear_parts_kernel(const GemmParams p)
   int mt, nt;
   plain_tile(p, p.full + tile, &mt, &nt);
   const Tile t = tile_of<true, TA, TB>(p, 0, 0, mt, nt);
+  if (t.mt * T + wm * 32 * IT + 32 * i >= t.M) return;
   const float* src = p.parts + (static_cast<int64_t>(tile) * p.cut * NW + of) * kPart + i * (32 * 64) + 4 * lane;
   floatx16 acc[1][2];
 #pragma unroll
@@ -2066,7 +2069,18 @@ double estimate(GemmParams& q, int kind, int T, int cus) {
     }
     return best;
   }
-  if (kind == kForward) return rounds * (slabs * 0.255 + 1.3) + 3;
+  if (kind == kForward) {
+    // A row or two of tiles read their weights from memory, not from an L2 that others have filled: 0.40 us a slab.  As many as
+    // leave half of the CUs idle are cut along k as well, down to what streaming the weights takes.  us, library / whole / cut: 16
+    // tokens, 1024 + 8192 + 4096 x 4096 60 / 45 / 33; 100 tokens 61 / 53 / 38, 512 + 4096 + 2048 x 2048 64 / 28 / 21.
+    const double slab = q.mt_count <= 2 ? 0.40 : 0.255, stream = 2.0 * q.nt_count * T * q.K / 4.0e6;
+    double best = rounds * (slabs * slab + 1.3) + 3;
+    for (int cut = 2; q.split_ok && cut <= 8 && q.items * cut <= cus && slabs >= 16 * cut; ++cut) {
+      const double t = std::max(slabs / cut * slab, stream) + 0.03 * q.items * cut * std::min(q.M, T) / T + 9;
+      if (t < best) best = t, q.full = 0, q.cut = cut;
+    }
+    return best;
+  }
   return rounds * (slabs * 0.27 + 1) + 3;
 }
 
@@ -2140,6 +2154,11 @@ int launch_linear(GemmParams q, int kind, int count, const int64_t* sizes, hipSt
       return launch_tiles<linear_parts_kernel<DT, kTile, false, false>>(q, left * 32, kWave, 0, s);
     }
     if (!small) return launch_tiles<gemm_dma64_kernel<DT, false, false, kTile, true>>(q, grid, threads, lds, s);
+    if (q.cut > 0) {
+      grid = (q.items * q.cut + kXcds - 1) / kXcds * kXcds;
+      if (const int rc = launch_tiles<gemm_dma_kernel<DT, false, false, false, kSmall, true, false, true>>(q, grid, threads, lds, s); rc != MEGA_OK) return rc;
+      return launch_tiles<linear_parts_kernel<DT, kSmall, false, false>>(q, q.items * 8, kWave, 0, s);
+    }
     if (q.items <= cus) return launch_tiles<gemm_dma_kernel<DT, false, false, false, kSmall, true>>(q, grid, threads, lds, s);
     return launch_tiles<gemm_dma64_kernel<DT, false, false, kSmall, true>>(q, grid, threads, lds, s);
   }
@@ -2210,7 +2229,8 @@ extern "C" int mega_linear_takes(int kind, int dtype, int64_t tokens, int64_t n_
     const double products = static_cast<double>(tokens) * n_in * n_out[i];
     if (kind == kInputGrad && products > 0x1p35) return 0;  // goes through a transposed copy of W there
     const double rate = kind == kInputGrad ? 1.1 : products > 0x1p39 ? 1.5 : products < 0x1p33 ? 1.0 : n_out[i] % 1024 == 0 ? 1.4 : 1.1;
-    library += std::max(20.0, 2e-9 * products / rate + (kind == kInputGrad ? 10 : 8));
+    const double stream = kind == kForward && tokens <= 256 ? 2.0 * n_in * n_out[i] / 3.3e6 + 3 : 0;  // the weights from memory
+    library += std::max({20.0, stream, 2e-9 * products / rate + (kind == kInputGrad ? 10 : 8)});
   }
   return here <= library;
 }

@@ -61,9 +61,9 @@ def test_products_match_float64(tokens, n_in, n_out, dtype):
     outs, s = (i64 * len(n_out))(*n_out), _lib.stream_ptr(x.device)
     call = lambda name, *a: _lib.call(name, *a, s)
 
-    def fwd(w, bias, add, n_out, y):
+    def fwd(w, bias, add, n_out, y, cut=True):
         n, outs = len(w), (i64 * len(w))(*n_out)
-        size = _parts(0, tokens, n_in, n_out)
+        size = _parts(0, tokens, n_in, n_out) if cut else 0
         ws = torch.empty(size, dtype=torch.uint8, device="cuda")
         call("mega_linear_fwd", _lib.ptr(x), _pointers(w), bias and _pointers(bias), add, _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(n), outs, _pointers(y), _lib.ptr(ws) if size else None)
 
@@ -75,11 +75,13 @@ def test_products_match_float64(tokens, n_in, n_out, dtype):
     for i in range(len(w)):
         _close(y[i], x64 @ w64[i].t() + (0 if bias[i] is None else bias[i].double()))
         _close(dw[i], dy64[i].t() @ x64)
-        # one layer alone gives the same bits as in the group
+        # one layer alone gives the same bits as in the group, where neither is cut
         if len(w) > 1:
-            alone = torch.empty_like(y[i])
-            fwd([w[i]], [bias[i]], None, [n_out[i]], [alone])
-            assert torch.equal(alone, y[i])
+            alone, whole = torch.empty_like(y[i]), [torch.empty_like(t) for t in y]
+            fwd([w[i]], [bias[i]], None, [n_out[i]], [alone], cut=False)
+            fwd(w, bias, None, n_out, whole, cut=False)
+            assert torch.equal(alone, whole[i])
+            _close(alone, x64 @ w64[i].t() + (0 if bias[i] is None else bias[i].double()))
     fwd(w[:1], None, _lib.ptr(add), n_out[:1], y[:1])
     _close(y[0], x64 @ w64[0].t() + add.double())
     dx = torch.empty_like(x)
@@ -136,6 +138,8 @@ def test_layers_whose_operands_need_the_general_path(tokens, sizes):
     (4100, 4096, [4096], torch.bfloat16),             # 272 tiles: 16 left over, the last of four rows
     (1531, 4096, [5504, 5568], torch.float16),        # two layers, layers and rows that end inside a tile
     (1531, 11008, [4096], torch.bfloat16),            # fewer tiles than the chip takes
+    (16, 4096, [1024, 2048, 1000], torch.bfloat16),   # one row of tiles of 128, of whose rows most are not there
+    (129, 2048, [512, 2048], torch.float16),          # two, one row in the second
 ])
 def test_last_tiles_cut_along_k(tokens, n_in, n_out, dtype):
     """The tiles that a last round of the chip would hold alone, cut along k and added up by a second launch: against
