@@ -4,7 +4,7 @@
 #include "host.hpp"
 
 #include <ATen/autocast_mode.h>
-#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <torch/csrc/autograd/custom_function.h>
 
 #include <map>
@@ -466,10 +466,16 @@ Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, double scale
 }
 
 // ---- linear layers --------------------------------------------------------------------------------
+// Whether the thread shows its operations to something beside autograd: the TorchScript tracer, a mode that counts flops
+// or makes fake tensors, a functorch transform.  A launch is no operation -- a trace of one holds the allocation of its
+// result and nothing that fills it -- so these are given the library's products.
+bool watched() {
+  const auto tls = c10::impl::tls_local_dispatch_key_set();
+  return (tls.included_ - tls.excluded_ - c10::default_included_set).highestFunctionalityKey() != c10::DispatchKey::Undefined;
+}
 // A matrix as the library's products take it: its own memory (no vmap wrapper), whole rows, 16-byte boundary.
 bool dense16(const Tensor& t) {
-  // (a subclass or a mode that watches the operations -- fake tensors, a count of the flops -- is shown the library's)
-  if (t.key_set().has(c10::DispatchKey::Python) || c10::impl::TorchDispatchModeTLS::any_modes_set()) return false;
+  if (t.key_set().has(c10::DispatchKey::Python) || watched()) return false;  // (Python: a subclass that sees its operations)
   return t.has_storage() && t.is_contiguous() && !lazy(t) && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
 }
 enum { kLinearForward, kLinearInputGrad, kLinearWeightGrad };

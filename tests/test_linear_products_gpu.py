@@ -209,6 +209,32 @@ def test_products_that_a_mode_watches():
         assert fake(torch.empty(64, 256, device="cuda", dtype=torch.bfloat16)).shape == (64, 128)
 
 
+class _Layers(torch.nn.Module):
+    def __init__(self):
+        super().__init__()
+        self.one, self.two, self.three = Linear(256, 128), Linear(256, 128, bias=False), Linear(256, 64)
+
+    def forward(self, x, residual):
+        return self.one(x), self.two(x, residual), *linear_group(x, [self.one, self.three])
+
+
+@pytest.mark.parametrize("gradients", [False, True])
+def test_products_that_are_traced(gradients):
+    """A trace holds the products themselves: called with other inputs it gives what the layers give."""
+    torch.manual_seed(5)
+    layers = _Layers().cuda().bfloat16()
+    draw = lambda: (torch.randn(64, 256, device="cuda").bfloat16(), torch.randn(64, 128, device="cuda").bfloat16())
+    with torch.set_grad_enabled(gradients):
+        traced = torch.jit.trace(layers, draw(), check_trace=False)
+        x, residual = draw()
+        got = traced(x, residual)
+        weights = [(layers.one, None), (layers.two, residual), (layers.one, None), (layers.three, None)]
+        for y, (l, r) in zip(got, weights):
+            _close(y.detach(), x.double() @ l.weight.detach().double().t() + (0 if l.bias is None else l.bias.detach().double())
+                   + (0 if r is None else r.double()))
+        assert all(y.requires_grad == gradients for y in got)
+
+
 def test_products_under_capture():
     """Captured: layers of one input with last tiles cut along k (parts from the graph's pool), replayed on other inputs with
     eager work between."""
