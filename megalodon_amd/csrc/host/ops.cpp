@@ -473,10 +473,17 @@ bool watched() {
   const auto tls = c10::impl::tls_local_dispatch_key_set();
   return (tls.included_ - tls.excluded_ - c10::default_included_set).highestFunctionalityKey() != c10::DispatchKey::Undefined;
 }
-// A matrix as the library's products take it: its own memory (no vmap wrapper), whole rows, 16-byte boundary.
+// Whether a tensor is what its memory holds and nothing more: dispatch keys of a dense tensor, no subclass, functional
+// wrapper, zeros without memory or batch.
+bool plain(const Tensor& t) {
+  constexpr auto usual = c10::default_included_set | c10::autograd_dispatch_keyset | c10::autocast_dispatch_keyset | c10::DispatchKeySet(c10::DispatchKey::Dense);
+  return (t.key_set() - usual).highestFunctionalityKey() == c10::DispatchKey::Undefined && t.has_storage();
+}
+// A matrix as the library's products take it: its own memory, whole rows, 16-byte boundary.
 bool dense16(const Tensor& t) {
-  if (t.key_set().has(c10::DispatchKey::Python) || watched()) return false;  // (Python: a subclass that sees its operations)
-  return t.has_storage() && t.is_contiguous() && !lazy(t) && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  if (!plain(t) || watched() || !t.is_contiguous()) return false;
+  const void* memory = t.data_ptr();
+  return memory != nullptr && reinterpret_cast<uintptr_t>(memory) % 16 == 0;
 }
 enum { kLinearForward, kLinearInputGrad, kLinearWeightGrad };
 // memory for the parts of products that are cut along their reduction axis

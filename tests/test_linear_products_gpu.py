@@ -209,6 +209,24 @@ def test_products_that_a_mode_watches():
         assert fake(torch.empty(64, 256, device="cuda", dtype=torch.bfloat16)).shape == (64, 128)
 
 
+def test_products_of_tensors_without_memory():
+    """Functional wrappers and zeros that are never written have a storage, but nothing in it to launch on."""
+    torch.manual_seed(9)
+    layers = [Linear(256, o, bias=b).cuda().bfloat16() for o, b in ((128, True), (64, False))]
+    x, residual = torch.randn(64, 256, device="cuda").bfloat16(), torch.randn(64, 64, device="cuda").bfloat16()
+    with torch.no_grad():
+        for y, l in zip(torch.func.functionalize(lambda x: linear_group(x, layers))(x), layers):
+            _close(y, x.double() @ l.weight.double().t() + (0 if l.bias is None else l.bias.double()))
+        y = torch.func.functionalize(lambda x, r: layers[1](x, r))(x, residual)
+        _close(y, x.double() @ layers[1].weight.double().t() + residual.double())
+    leaf = x.clone().requires_grad_(True)
+    ys = (layers[1](leaf), *linear_group(leaf, layers))
+    zeros = [torch._efficientzerotensor(tuple(y.shape), dtype=y.dtype, device=y.device) for y in ys]
+    for wanted in ((ys[:1], zeros[:1]), (ys[1:], zeros[1:])):
+        grads = torch.autograd.grad(wanted[0], [leaf, layers[1].weight], wanted[1], retain_graph=True)
+        assert all(torch.equal(g, torch.zeros_like(t)) for g, t in zip(grads, [leaf, layers[1].weight]))
+
+
 class _Layers(torch.nn.Module):
     def __init__(self):
         super().__init__()
