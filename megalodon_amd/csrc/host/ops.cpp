@@ -529,8 +529,7 @@ Tensor flat(const Tensor& t) { return t.reshape({-1, t.size(-1)}); }
 Tensor bias_grad(const Tensor& g) {
   const int64_t rows = g.size(0), cols = g.size(1);
   const bool taken = rows >= 1 && cols >= 1 && cols % 8 == 0 && cols <= (1 << 24) &&
-                     (g.scalar_type() == at::kBFloat16 || g.scalar_type() == at::kHalf) && g.is_contiguous() &&
-                     reinterpret_cast<uintptr_t>(g.data_ptr()) % 16 == 0;
+                     (g.scalar_type() == at::kBFloat16 || g.scalar_type() == at::kHalf) && dense16(g);
   if (!taken) return g.sum(0);
   Tensor out = at::empty({cols}, g.options()), ws = bytes(mega_column_sums_workspace_bytes(rows, cols), g);
   check(mega_column_sums(g.data_ptr(), kernel_code(g), rows, cols, out.data_ptr(), ws.data_ptr(), stream_of(g)), "mega_column_sums");
@@ -541,7 +540,7 @@ Tensor bias_grad(const Tensor& g) {
 // included / without it, in us: 4096 tokens x 2048 x 1024 30 / 25, 4096 x 2752 x 1024 37 / 32, 4096 x 4096 x 2048 (2^35
 // products) 68 / 66; 8192 x 4096 x 2048 102 / 107, 32768 x 2048 x 1024 109 / 120, 8192 x 4096 x 4096 194 / 217.
 bool turned(const Tensor& g, const Tensor& w) {
-  return static_cast<double>(g.size(0)) * w.size(0) * w.size(1) > static_cast<double>(1ll << 35);
+  return static_cast<double>(g.size(0)) * w.size(0) * w.size(1) > static_cast<double>(1ll << 35) && plain(w) && !watched();
 }
 // dx = g W, added to `sum` (in place) where there is one
 Tensor input_grad(const Tensor& g, const Tensor& w, const Tensor& sum) {

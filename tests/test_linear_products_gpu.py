@@ -209,6 +209,21 @@ def test_products_that_a_mode_watches():
         assert fake(torch.empty(64, 256, device="cuda", dtype=torch.bfloat16)).shape == (64, 128)
 
 
+@pytest.mark.parametrize("size", [256, 4096])  # 4096^3: the input gradient takes a transposed copy of the weight
+def test_gradients_that_a_mode_watches(size):
+    from torch._subclasses import FakeTensorMode
+    with FakeTensorMode():
+        fake = Linear(size, size, device="cuda", dtype=torch.bfloat16)
+        x = torch.empty(size, size, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+        y = fake(x)
+        grads = torch.autograd.grad(y, (x, fake.weight, fake.bias), torch.empty_like(y))
+        assert [tuple(g.shape) for g in grads] == [(size, size), (size, size), (size,)]
+    layer = Linear(256, 128).cuda().bfloat16()
+    y = layer(torch.randn(64, 256, device="cuda").bfloat16())
+    db, = torch.autograd.grad(y, layer.bias, torch._efficientzerotensor((64, 128), dtype=y.dtype, device="cuda"))
+    assert torch.equal(db, torch.zeros_like(layer.bias))
+
+
 def test_products_of_tensors_without_memory():
     """Functional wrappers and zeros that are never written have a storage, but nothing in it to launch on."""
     torch.manual_seed(9)
