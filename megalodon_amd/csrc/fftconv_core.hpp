@@ -620,5 +620,23 @@ MEGA_HD constexpr int out_pos(int n2) {
   return H == 0 ? bitrev<5>(n2) : shifted_dit32_pos(n2);
 }
 
+// How a launch shares out its rows: how many rows of a channel a group takes, chosen for the shortest line of
+// transforms, in halves of one, that a workgroup slot gets (5 for a pair of rows, 3 for a row alone).  `bound`: a channel's sum
+// stands in its groups' slots, so that there may be no more groups than slots, unless a group has the channel to itself.
+// Of the sizes that leave as many groups to a channel the smallest is the shortest, so only these are looked at, 2 sqrt(B)
+// at most: for the three launches of a step on 10^6 rows of one channel, 24 ms of the host's time size by size, 0.08 so.
+inline int64_t group_rows(int64_t B, int64_t D, int64_t slots, int pair, bool bound) {
+  int64_t best = B, least = -1;
+  for (int64_t nb = 1;;) {
+    const int64_t shares = (B + nb - 1) / nb, groups = D * shares;
+    if (!bound || shares == 1 || groups <= slots) {
+      const int64_t cost = (groups + slots - 1) / slots * (pair == 2 ? nb / 2 * 5 + nb % 2 * 3 : nb * 3);
+      if (least < 0 || cost < least) best = nb, least = cost;
+    }
+    if (shares == 1) return best;
+    nb = (B + shares - 2) / (shares - 1);  // the smallest that leaves fewer
+  }
+}
+
 }  // namespace fftc
 }  // namespace mega

@@ -479,18 +479,9 @@ __global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict_
   dk[i] = sum;
 }
 
-// How a launch shares out its rows: the rows of a channel that a group takes are chosen for the shortest line of
-// transforms, in halves of one, that a workgroup slot gets (5 for a pair of rows, 3 for a row alone).  `bound`: a channel's sum
-// stands in its groups' slots, so that there may be no more groups than slots, unless a group has the channel to itself.
 Rows make_rows(int64_t B, int64_t D, int64_t L, int slots, int part, int pair, bool bound) {
-  int64_t best = B, least = -1;
-  for (int64_t nb = 1; nb <= B; ++nb) {
-    const int64_t groups = D * ((B + nb - 1) / nb);
-    if (bound && nb < B && groups > slots) continue;
-    const int64_t cost = (groups + slots - 1) / slots * (pair == 2 ? nb / 2 * 5 + nb % 2 * 3 : nb * 3);
-    if (least < 0 || cost < least) best = nb, least = cost;
-  }
-  return Rows{static_cast<int>(B), static_cast<int>(D), static_cast<int>(L), static_cast<int>(best), static_cast<int>(D * ((B + best - 1) / best)), part};
+  const int64_t nb = group_rows(B, D, slots, pair, bound);
+  return Rows{static_cast<int>(B), static_cast<int>(D), static_cast<int>(L), static_cast<int>(nb), static_cast<int>(D * ((B + nb - 1) / nb)), part};
 }
 
 template <int LOGM, int DT, int MODE, bool VEC, int PAIR>

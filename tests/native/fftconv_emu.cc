@@ -154,3 +154,7 @@ extern "C" int emu_fft_half(int logm, int h, const float* inr, const float* ini,
   else return 1;
   return 0;
 }
+
+extern "C" int64_t emu_group_rows(int64_t B, int64_t D, int64_t slots, int pair, int bound) {
+  return group_rows(B, D, slots, pair, bound != 0);
+}

@@ -6,6 +6,7 @@ without a GPU."""
 import ctypes
 import os
 import subprocess
+import time
 
 import numpy as np
 import pytest
@@ -58,3 +59,29 @@ def test_convolution_matches_numpy(emu, logm):
             if flip_out:
                 want = want[::-1]
             assert np.abs(y - want).max() / np.abs(want).max() < 5e-6
+
+
+def test_rows_are_shared_out_without_looking_at_every_size(emu):
+    """The rows of a channel that a workgroup takes: the best of all sizes, the smallest of equals, found in about the square
+    root of their number."""
+    emu.emu_group_rows.restype = ctypes.c_int64
+    i64 = ctypes.c_int64
+    choose = lambda B, D, slots, pair, bound: emu.emu_group_rows(i64(B), i64(D), i64(slots), pair, bound)
+
+    def all_sizes(B, D, slots, pair, bound):
+        costs = {}
+        for nb in range(1, B + 1):
+            groups = D * -(-B // nb)
+            if not bound or nb == B or groups <= slots:
+                costs[nb] = -(-groups // slots) * (nb // 2 * 5 + nb % 2 * 3 if pair == 2 else 3 * nb)
+        return min(costs, key=lambda nb: (costs[nb], nb))
+
+    for B in (*range(1, 41), 97, 128, 360, 1001):
+        for D in (1, 3, 64, 257, 1024, 4100):
+            for slots in (1, 256, 512, 2048):
+                for pair in (1, 2):
+                    for bound in (0, 1):
+                        assert choose(B, D, slots, pair, bound) == all_sizes(B, D, slots, pair, bound), (B, D, slots, pair, bound)
+    start = time.perf_counter()
+    assert 1 <= choose(10 ** 9, 1, 512, 2, 0) <= 10 ** 9
+    assert time.perf_counter() - start < 0.5  # all of them: seconds
