@@ -148,12 +148,13 @@ int mega_cema_coeffs_bwd(const float* dp, const float* dq, const float* dgamma_h
  *   a stream gets a block of its own, so launches on different streams never
  *   share slots, up to four blocks; a fifth stream takes over the block that
  *   has been idle longest and waits on the device for the last launch that
- *   used it); they are kept until process exit (96 MiB per block at every
- *   size on 256 compute units).  mega_fftconv_prepare(L, stream) makes
- *   them ahead of time (it allocates and synchronises `stream` once; not
+ *   used it); they are kept until process exit.  A block has one to three parts
+ *   of 32 MiB (at every size on 256 compute units), as many as its launches have
+ *   needed.  mega_fftconv_prepare(L, stream) makes
+ *   them ahead of time, whole (it allocates and synchronises `stream` once; not
  *   capturable); after it, the convolution entry points on that stream only
- *   enqueue.  Without it the first call for a size / stream does the same
- *   work itself.  To capture a convolution into a graph, prepare the stream
+ *   enqueue.  Without it the first calls for a size / stream do the same
+ *   work themselves.  To capture a convolution into a graph, prepare the stream
  *   the capture runs on; a block used under capture belongs to that graph's
  *   replays and is never handed to another stream.
  *   mega_fftconv_scratch_blocks(L): blocks held on the current device for the

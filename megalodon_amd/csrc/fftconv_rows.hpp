@@ -14,9 +14,13 @@ namespace mega {
 // ------------------------------ tables --------------------------------------
 constexpr int kFftDevices = 16;
 constexpr int kFftScratch = 4;  // scratch blocks per device and size before streams start taking turns
+constexpr int kSlotParts = 3;   // parts of a workgroup's scratch slot, 2 M floats each; a part of all slots is one allocation
+struct Scratch {
+  float* part[kSlotParts];  // null behind the parts that a block has
+};
 struct StreamScratch {
   hipStream_t stream;  // the stream whose launches used the block last
-  float* ptr;
+  Scratch parts;
   hipEvent_t done;     // recorded behind the last launch that used the block
   uint64_t tick;       // when that was
   bool pinned;         // used under stream capture: the graph's replays own the block from then on
@@ -70,9 +74,6 @@ using namespace fftc;
 template <int LOGM>
 constexpr int kPerCu = 1 << (14 - LOGM);
 
-constexpr int kSlotParts = 3;  // parts of a workgroup's scratch slot, 2 M floats each, a part of all slots together
-
-
 bool stream_is_capturing(hipStream_t stream) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &st) != hipSuccess) {
@@ -86,10 +87,10 @@ bool stream_is_capturing(hipStream_t stream) {
 // scratch slots live for the life of the process.  They are made on first use,
 // or ahead of time by mega_fftconv_prepare; making them allocates and, for the
 // tables, synchronises the stream once, so that call cannot be captured into a
-// graph.  Scratch is three parts of 2*M floats per resident workgroup (kPerCu of
-// them per CU: 101 MB at every size).
+// graph.  A part of scratch is 2*M floats per resident workgroup (kPerCu of
+// them per CU: 34 MB at every size); a block gets as many of the three as its launches have needed.
 template <int LOGM>
-int get_tables(hipStream_t stream, const c32** out, float** scratch, int* slots) {
+int get_tables(hipStream_t stream, const c32** out, int* slots) {
   using C = Cfg<LOGM>;
   int dev = 0;
   MEGA_CHECK_HIP(hipGetDevice(&dev));
@@ -112,7 +113,19 @@ int get_tables(hipStream_t stream, const c32** out, float** scratch, int* slots)
     }
     slot = p;
   }
-  const int nslots = fft_tables.slots[dev][LOGM - 11];
+  *out = slot;
+  *slots = fft_tables.slots[dev][LOGM - 11];
+  return MEGA_OK;
+}
+
+// The stream's scratch block, with `need` parts or more; under capture, where nothing can be allocated, with those that
+// it has (*have).
+template <int LOGM>
+int get_scratch(hipStream_t stream, int need, Scratch* scratch, int* have) {
+  using C = Cfg<LOGM>;
+  int dev = 0;
+  MEGA_CHECK_HIP(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lock(fft_tables.mu);
   std::vector<StreamScratch>& blocks = fft_tables.scratch[dev][LOGM - 11];
   StreamScratch* mine = nullptr;
   int open_blocks = 0;
@@ -128,23 +141,33 @@ int get_tables(hipStream_t stream, const c32** out, float** scratch, int* slots)
     MEGA_CHECK_HIP(hipStreamWaitEvent(stream, mine->done, 0));
     mine->stream = stream;
   }
-  if (mine == nullptr) {
-    float* sc = nullptr;
-    hipEvent_t ev = nullptr;
-    MEGA_CHECK_HIP(hipMalloc(reinterpret_cast<void**>(&sc), sizeof(float) * kSlotParts * 2 * C::M * nslots));
-    hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+  const bool fresh = mine == nullptr;
+  StreamScratch made{stream, {}, nullptr, 0, false};
+  if (fresh) mine = &made;
+  *have = 0;
+  while (*have < kSlotParts && mine->parts.part[*have] != nullptr) ++*have;
+  while (*have < need && (fresh || !capturing)) {
+    const hipError_t e = hipMalloc(reinterpret_cast<void**>(&mine->parts.part[*have]), sizeof(float) * 2 * C::M * fft_tables.slots[dev][LOGM - 11]);
     if (e != hipSuccess) {
-      (void)hipFree(sc);
+      mine->parts.part[*have] = nullptr;
+      if (fresh)
+        for (float* p : made.parts.part) (void)hipFree(p);
+      return set_error(MEGA_ERR_HIP, "fftconv scratch: %s", hipGetErrorString(e));
+    }
+    ++*have;
+  }
+  if (fresh) {
+    const hipError_t e = hipEventCreateWithFlags(&made.done, hipEventDisableTiming);
+    if (e != hipSuccess) {
+      for (float* p : made.parts.part) (void)hipFree(p);
       return set_error(MEGA_ERR_HIP, "fftconv scratch event: %s", hipGetErrorString(e));
     }
-    blocks.push_back(StreamScratch{stream, sc, ev, 0, false});
+    blocks.push_back(made);
     mine = &blocks.back();
   }
   mine->tick = ++fft_tables.tick;
   if (capturing) mine->pinned = true;
-  *out = slot;
-  *scratch = mine->ptr;
-  *slots = nslots;
+  *scratch = mine->parts;
   return MEGA_OK;
 }
 
@@ -390,7 +413,6 @@ __device__ __forceinline__ void outputs(float* re, float* im, int t, const Table
 struct Rows {
   int B, D, L;
   int nb, groups;  // group g: channel g % D, rows g / D nb ..
-  int part;        // floats from a part of a slot to its next
 };
 
 // spectrum of a row's half H; SCALED: times 1 / (4 N) (E, O halves and the inverse), as one factor of every product is
@@ -415,7 +437,7 @@ __device__ __forceinline__ void spectrum(float* re, float* im, const void* row, 
 //         shared by several workgroups, whose sums stand in their slots.
 template <int LOGM, int DT, int MODE, bool VEC, int H, int PAIR>
 __device__ __forceinline__ void conv_half(const void* a, const void* b, void* out, const Rows& rows, int d, int b0, int n, bool add,
-                                          int flip, const Tables& tb, float* lre, float* lim, float* scratch, const float* omega) {
+                                          int flip, const Tables& tb, float* lre, float* lim, const Scratch& scratch, const float* omega) {
   using C = Cfg<LOGM>;
   const int64_t pitch = static_cast<int64_t>(rows.L) * (DT == MEGA_F32 ? 4 : 2);
   float pre[32], pim[32];
@@ -433,20 +455,21 @@ __device__ __forceinline__ void conv_half(const void* a, const void* b, void* ou
     if (MODE == 1) spectrum<LOGM, DT, VEC, H, true>(pre, pim, static_cast<const char*>(b) + row * pitch, rows.L, false, t, tb, lre, lim);
     spectrum<LOGM, DT, VEC, H, false>(re, im, arow, rows.L, MODE == 1 || flip != 0, t, tb, lre, lim);
     pointwise<LOGM, H>(re, im, pre, pim, t, launder(tb));
-    // the slot's parts: half 0's outputs; of the second row, or (MODE 1) the spectrum so far; a shared channel's sum
-    if (MODE == 1) {
-      if (i > 0) fetch<LOGM, true>(scratch + rows.part, re, im, t);
+    // the slot's parts: half 0's outputs; with pairs those of the second row, or (MODE 1) the spectrum so far; last a
+    // shared channel's sum
+    if (MODE == 1 && PAIR > 1) {
+      if (i > 0) fetch<LOGM, true>(scratch.part[1], re, im, t);
       if (i + 1 < count) {
-        keep<LOGM>(scratch + rows.part, re, im, t);
+        keep<LOGM>(scratch.part[1], re, im, t);
         continue;
       }
     }
-    outputs<LOGM, H>(re, im, t, tb, lre, lim, MODE == 0 ? scratch + i * rows.part : scratch);
+    outputs<LOGM, H>(re, im, t, tb, lre, lim, MODE == 0 && PAIR > 1 && i > 0 ? scratch.part[1] : scratch.part[0]);
     if (H == 1 && MODE == 0)
       store_row<LOGM, DT, VEC, false>(re, im, static_cast<char*>(out) + row * pitch, rows.L, flip != 0, t,
                                       omega != nullptr ? arow : nullptr, omega != nullptr ? omega[d] : 0.f);
     if (H == 1 && MODE == 1) {
-      float* sum = flip ? scratch + 2 * rows.part : static_cast<float*>(out) + static_cast<int64_t>(d) * rows.L;
+      float* sum = flip ? scratch.part[PAIR] : static_cast<float*>(out) + static_cast<int64_t>(d) * rows.L;
       if (add) store_row<LOGM, MEGA_F32, VEC, true>(re, im, sum, rows.L, true, t);
       else store_row<LOGM, MEGA_F32, VEC, false>(re, im, sum, rows.L, true, t);
     }
@@ -455,11 +478,12 @@ __device__ __forceinline__ void conv_half(const void* a, const void* b, void* ou
 template <int LOGM, int DT, int MODE, bool VEC, int PAIR>
 __global__ __launch_bounds__(Cfg<LOGM>::T, 2) void fftconv_kernel(
     const void* __restrict__ a, const void* __restrict__ b, void* __restrict__ out, const Rows rows, int flip,
-    const c32* __restrict__ tab, float* __restrict__ scratch_all, const float* __restrict__ omega) {
+    const c32* __restrict__ tab, const Scratch all, const float* __restrict__ omega) {
   extern __shared__ __align__(16) float lds[];
   float *lre = lds, *lim = lds + Cfg<LOGM>::PLANE;
   const Tables tb = make_tables<LOGM>(tab);
-  float* scratch = scratch_all + blockIdx.x * 2 * Cfg<LOGM>::M;
+  const size_t slot = blockIdx.x * 2 * Cfg<LOGM>::M;  // (within a part; parts that the launch does not use are never touched)
+  const Scratch scratch{{all.part[0] + slot, all.part[1] + slot, all.part[2] + slot}};
   for (int g = blockIdx.x; g < rows.groups; g += gridDim.x) {
     const int d = g % rows.D, first = g / rows.D * rows.nb, end = min(rows.B, first + rows.nb);
     for (int b0 = first; b0 < end; b0 += PAIR) {
@@ -470,22 +494,21 @@ __global__ __launch_bounds__(Cfg<LOGM>::T, 2) void fftconv_kernel(
   }
 }
 // dk of channels whose rows several workgroups took, from their slots in order
-__global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict__ scratch, float* __restrict__ dk, const Rows rows, int slot) {
+__global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict__ sums, float* __restrict__ dk, const Rows rows, int slot) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (i >= static_cast<int64_t>(rows.D) * rows.L) return;
   const int d = static_cast<int>(i / rows.L), m = static_cast<int>(i % rows.L);
   float sum = 0.f;
-  for (int g = d; g < rows.groups; g += rows.D) sum += scratch[2 * static_cast<int64_t>(rows.part) + static_cast<int64_t>(g) * slot + m];
+  for (int g = d; g < rows.groups; g += rows.D) sum += sums[static_cast<int64_t>(g) * slot + m];
   dk[i] = sum;
 }
 
-Rows make_rows(int64_t B, int64_t D, int64_t L, int slots, int part, int pair, bool bound) {
-  const int64_t nb = group_rows(B, D, slots, pair, bound);
-  return Rows{static_cast<int>(B), static_cast<int>(D), static_cast<int>(L), static_cast<int>(nb), static_cast<int>(D * ((B + nb - 1) / nb)), part};
+Rows make_rows(int64_t B, int64_t D, int64_t L, int64_t nb) {
+  return Rows{static_cast<int>(B), static_cast<int>(D), static_cast<int>(L), static_cast<int>(nb), static_cast<int>(D * ((B + nb - 1) / nb))};
 }
 
 template <int LOGM, int DT, int MODE, bool VEC, int PAIR>
-int launch_rows(const void* a, const void* b, void* out, const Rows& rows, int flip, const float* omega, const c32* tab, float* scratch,
+int launch_rows(const void* a, const void* b, void* out, const Rows& rows, int flip, const float* omega, const c32* tab, const Scratch& scratch,
                 int slots, hipStream_t stream) {
   const size_t lds_bytes = sizeof(float) * 2 * Cfg<LOGM>::PLANE;
   MEGA_CHECK_HIP(hipFuncSetAttribute(
@@ -501,20 +524,27 @@ template <int LOGM, int DT, int MODE, bool VEC>
 int launch_fft_v(const void* a, const void* b, void* out, int64_t B, int64_t D, int64_t L, int flip, const float* omega, hipStream_t stream) {
   using C = Cfg<LOGM>;
   const c32* tab = nullptr;
-  float* scratch = nullptr;
-  int slots = 0;
-  int rc = get_tables<LOGM>(stream, &tab, &scratch, &slots);
+  Scratch scratch{};
+  int slots = 0, have = 0;
+  int rc = get_tables<LOGM>(stream, &tab, &slots);
   if (rc != MEGA_OK) return rc;
   MEGA_CHECK_ARG(B * D <= 0x7fffffff, "fftconv: too many rows");
   constexpr int kMost = MODE == 0 && (LOGM == 14 || !VEC) ? 1 : 2;
-  const Rows rows = make_rows(B, D, L, slots, slots * 2 * C::M, kMost, MODE == 1);
-  const bool split = MODE == 1 && rows.nb < B;
+  int64_t nb = group_rows(B, D, slots, kMost, MODE == 1);
+  int pair = nb == 1 ? 1 : kMost;
+  const auto parts = [&] { return pair + (MODE == 1 && nb < B ? 1 : 0); };
+  rc = get_scratch<LOGM>(stream, parts(), &scratch, &have);
+  if (rc != MEGA_OK) return rc;
+  // (fewer under capture, in a block of other launches: rows one by one then, and no channel's dk shared out)
+  if (have < parts()) pair = 1, nb = MODE == 1 ? B : group_rows(B, D, slots, 1, false);
+  const Rows rows = make_rows(B, D, L, nb);
+  const bool split = MODE == 1 && nb < B;
   const int how = MODE == 1 ? split : flip;
-  if (kMost == 1 || rows.nb == 1) rc = launch_rows<LOGM, DT, MODE, VEC, 1>(a, b, out, rows, how, omega, tab, scratch, slots, stream);
+  if (kMost == 1 || pair == 1) rc = launch_rows<LOGM, DT, MODE, VEC, 1>(a, b, out, rows, how, omega, tab, scratch, slots, stream);
   else rc = launch_rows<LOGM, DT, MODE, VEC, kMost>(a, b, out, rows, how, omega, tab, scratch, slots, stream);
   if (rc != MEGA_OK) return rc;
   if (split) {
-    split_sum_kernel<<<dim3(static_cast<unsigned>((D * L + 255) / 256)), 256, 0, stream>>>(scratch, static_cast<float*>(out), rows, 2 * C::M);
+    split_sum_kernel<<<dim3(static_cast<unsigned>((D * L + 255) / 256)), 256, 0, stream>>>(scratch.part[pair], static_cast<float*>(out), rows, 2 * C::M);
     MEGA_CHECK_LAUNCH();
   }
   return scratch_used<LOGM>(stream);
@@ -546,9 +576,10 @@ int fftconv_rows(int dtype, int mode, const void* a, const void* b, void* out, i
 template <int LOGM>
 int fftconv_tables(hipStream_t stream) {
   const c32* tab = nullptr;
-  float* scratch = nullptr;
-  int slots = 0;
-  return get_tables<LOGM>(stream, &tab, &scratch, &slots);
+  Scratch scratch{};
+  int slots = 0, have = 0;
+  if (const int rc = get_tables<LOGM>(stream, &tab, &slots); rc != MEGA_OK) return rc;
+  return get_scratch<LOGM>(stream, kSlotParts, &scratch, &have);
 }
 template int fftconv_rows<MEGA_FFTCONV_LOGM>(int, int, const void*, const void*, void*, int64_t, int64_t, int64_t, int, const float*, hipStream_t);
 template int fftconv_tables<MEGA_FFTCONV_LOGM>(hipStream_t);

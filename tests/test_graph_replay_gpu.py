@@ -141,3 +141,57 @@ def test_float32_convolution_scratch_blocks_are_bounded():
     for o in outs:
         assert torch.equal(o, want)
     assert 1 <= ops.fftconv_scratch_blocks(L) <= 4
+
+
+def test_float32_convolution_scratch_is_sized_by_use():
+    """A block holds what its stream's launches have needed: rows of a channel one at a time one part of three (32 MiB at 256
+    compute units), pairs a second, channels whose dk is shared out a third."""
+    L, part = 12000, 32 << 20
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        blocks = ops.fftconv_scratch_blocks(L)
+        if blocks >= 4:
+            pytest.skip("another stream's block would be taken over")
+        held = []
+        for B, D in ((1, 512), (2, 512), (8, 128), (1, 512)):
+            x, k = torch.randn(B, D, L, device="cuda"), torch.randn(D, L, device="cuda")
+            torch.cuda.synchronize()
+            free, torchs = torch.cuda.mem_get_info()[0], torch.cuda.memory_reserved()
+            ops.fftconv_fwd(x, k)
+            ops.fftconv_bwd(x, x, k, torch.float32)
+            torch.cuda.synchronize()
+            held.append((free - torch.cuda.mem_get_info()[0] - (torch.cuda.memory_reserved() - torchs)) / part)
+    assert ops.fftconv_scratch_blocks(L) == blocks + 1
+    assert all(1 <= h < 2 for h in held[:3]) and held[3] < 1, held  # (and what the runtime takes for a kernel's first launch)
+
+
+def test_float32_convolution_captured_in_a_block_of_smaller_launches():
+    """A stream that has run one row at a time holds one part of scratch; a capture on it, where nothing can be allocated,
+    runs rows one by one and shares no channel's dk: forward and backward of a batch against the oracle on every replay."""
+    L, D = 2100, 1024
+    g_ = torch.Generator().manual_seed(13)
+    x, dy = torch.randn(4, D, L, generator=g_).cuda(), torch.randn(4, D, L, generator=g_).cuda()
+    k = (torch.randn(D, L, generator=g_) / L ** 0.5).cuda()
+    base = [x.clone(), x.flip(-1).clone(), (2 * x).clone()]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        ops.fftconv_fwd(x[:1], k)
+        ops.fftconv_bwd(dy[:1], x[:1], k, torch.float32)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        y = ops.fftconv_fwd(x, k)
+        dx, dk = ops.fftconv_bwd(dy, x, k, torch.float32)
+    for i in (0, 1, 2, 1):
+        x.copy_(base[i])
+        ops.fftconv_fwd(x, k)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        n = 2 * L
+        rfft, irfft = (lambda t: torch.fft.rfft(t, n)), (lambda t: torch.fft.irfft(t, n)[..., :L])
+        x64, k64, r64 = x.double(), k.double(), dy.double().flip(-1)
+        for got, want in ((y, irfft(rfft(x64) * rfft(k64))), (dx, irfft(rfft(r64) * rfft(k64)).flip(-1)),
+                          (dk, irfft(rfft(r64) * rfft(x64)).sum(0).flip(-1))):
+            assert (got.double() - want).norm() <= 2e-6 * want.norm()  # the float32 transforms' error
