@@ -414,8 +414,9 @@ int mega_linear_weight_grad(const void* dy, const void* x, int dtype, int64_t to
  *   weight_grads: dw_i = dy_i^T x.
  * `workspace` of fwd and weight_grads: mega_linear_workspace_bytes(0 or 2, ...) bytes (up to 64 MiB; for many sizes 0), or
  * null: no product is cut along its reduction axis then, which makes some sizes slower.
- * `takes` (kind 0, 1, 2 in this order; input_grad: count 1) is 1 where the launch is expected to be
- * faster than a general library's products, 0 where it is not or where the sizes are refused. */
+ * `takes` (kind 0, 1, 2 in this order) is 1 where the call on these layers is expected to be
+ * faster than a general library's products, one a layer, 0 where it is not or where the sizes are refused; it and
+ * workspace_bytes leave mega_last_error as it is. */
 int mega_linear_takes(int kind, int dtype, int64_t tokens, int64_t n_in, int count, const int64_t* n_out);
 int mega_linear_fwd(const void* x, const void* const* w, const void* const* bias, const void* add,
                     int dtype, int64_t tokens, int64_t n_in, int count, const int64_t* n_out,

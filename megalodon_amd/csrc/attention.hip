@@ -2189,21 +2189,25 @@ int launch_linear(GemmParams q, int kind, int count, const int64_t* sizes, hipSt
 }  // namespace
 }  // namespace mega
 
-// (the contiguous reduction axis of forward and input gradient comes in slabs of 64)
-static int check_linear(const char* who, int kind, int dtype, int64_t tokens, int64_t n_in, int count, const int64_t* n_out) {
-  MEGA_CHECK_ARG(dtype == MEGA_BF16 || dtype == MEGA_F16, "%s: bfloat16 or float16 tensors", who);
-  MEGA_CHECK_ARG(count >= 1 && count <= 3 && n_out != nullptr, "%s: one to three layers", who);
+// What a product's launch refuses, or null.  (The contiguous reduction axis of forward and input gradient comes in slabs of 64.)
+static const char* linear_refuses(int kind, int dtype, int64_t tokens, int64_t n_in, int count, const int64_t* n_out) {
+  if (dtype != MEGA_BF16 && dtype != MEGA_F16) return "bfloat16 or float16 tensors";
+  if (count < 1 || count > 3 || n_out == nullptr) return "one to three layers";
   const int64_t in = kind == kForward ? 64 : 8, out = kind == kInputGrad ? 64 : 8;
-  MEGA_CHECK_ARG(tokens >= 1 && n_in >= in && n_in % in == 0 && tokens < (1 << 30) / n_in, "%s: bad sizes", who);
+  if (tokens < 1 || n_in < in || n_in % in != 0 || tokens >= (1 << 30) / n_in) return "bad sizes";
   for (int i = 0; i < count; ++i)
-    MEGA_CHECK_ARG(n_out[i] >= out && n_out[i] % out == 0 && tokens < (1 << 30) / n_out[i] && n_in < (1 << 30) / n_out[i], "%s: bad sizes", who);
-  return MEGA_OK;
+    if (n_out[i] < out || n_out[i] % out != 0 || tokens >= (1 << 30) / n_out[i] || n_in >= (1 << 30) / n_out[i]) return "bad sizes";
+  return nullptr;
+}
+static int check_linear(const char* who, int kind, int dtype, int64_t tokens, int64_t n_in, int count, const int64_t* n_out) {
+  const char* why = linear_refuses(kind, dtype, tokens, n_in, count, n_out);
+  return why == nullptr ? MEGA_OK : set_error(MEGA_ERR_INVALID_ARG, "%s: %s", who, why);
 }
 static bool aligned16(const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; }
 
 // Whether the launch is expected to be faster than the library's products, one call a layer.
 extern "C" int mega_linear_takes(int kind, int dtype, int64_t tokens, int64_t n_in, int count, const int64_t* n_out) {
-  if (kind < kForward || kind > kWeightGrad || check_linear("mega_linear_takes", kind, dtype, tokens, n_in, count, n_out) != MEGA_OK) return 0;
+  if (kind < kForward || kind > kWeightGrad || linear_refuses(kind, dtype, tokens, n_in, count, n_out) != nullptr) return 0;
   int cus = 0;
   if (compute_units(&cus) != MEGA_OK) return 0;
   if (kind == kWeightGrad) {
@@ -2236,7 +2240,7 @@ extern "C" int mega_linear_takes(int kind, int dtype, int64_t tokens, int64_t n_
 }
 
 extern "C" int64_t mega_linear_workspace_bytes(int kind, int64_t tokens, int64_t n_in, int count, const int64_t* n_out) {
-  if ((kind != kForward && kind != kWeightGrad) || check_linear("mega_linear_workspace_bytes", kind, MEGA_BF16, tokens, n_in, count, n_out) != MEGA_OK) return 0;
+  if ((kind != kForward && kind != kWeightGrad) || linear_refuses(kind, MEGA_BF16, tokens, n_in, count, n_out) != nullptr) return 0;
   int cus = 0;
   if (compute_units(&cus) != MEGA_OK) return 0;
   GemmParams q{};

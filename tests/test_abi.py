@@ -59,3 +59,18 @@ def test_attention_layer_pads_only_what_the_scores_kernel_writes():
     assert saved(1021, 5000, 256, 1.0) == 5000 * 1021 * 1021   # a batch entry of 2^30 elements and more
     assert saved(1021, 2, 96, 1.0) == 2 * 1021 * 1021
     assert saved(1021, 2, 256, 1.0, dtype=0) == 2 * 1021 * 1021
+
+
+def test_questions_about_linear_layers_leave_the_last_error():
+    """Whether a launch takes a size and what memory it wants are questions: no is an answer, not an error."""
+    lib = _lib.load()
+    i64, null = ctypes.c_int64, ctypes.c_void_p(0)
+    one = (i64 * 1)(77)
+    assert lib.mega_linear_fwd(null, null, null, null, ctypes.c_int(1), i64(100), i64(64), ctypes.c_int(1), one, null, null, null) == 1
+    before = lib.mega_last_error()
+    assert before == b"mega_linear_fwd: bad sizes"
+    lib.mega_linear_workspace_bytes.restype = i64
+    for kind, dtype, tokens, n_in, count in [(0, 1, 100, 64, 1), (1, 1, 100, 64, 1), (2, 1, 100, 64, 1), (2, 0, 100, 64, 1), (2, 1, 0, 64, 1), (0, 1, 100, 64, 4)]:
+        assert lib.mega_linear_takes(ctypes.c_int(kind), ctypes.c_int(dtype), i64(tokens), i64(n_in), ctypes.c_int(count), one) == 0
+        assert lib.mega_linear_workspace_bytes(ctypes.c_int(kind), i64(tokens), i64(n_in), ctypes.c_int(count), one) == 0
+    assert lib.mega_last_error() == before
