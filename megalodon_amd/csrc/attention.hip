@@ -22,6 +22,7 @@
 // diagonal by L2 - L1 columns in every one of these rules.
 #include "common.hpp"
 #include "dropkey.hpp"
+#include "linear_plan.hpp"
 
 #include <algorithm>
 
@@ -48,9 +49,6 @@ int attention_probs_fused(int dtype, const uint16_t* q, const uint16_t* k, uint1
 
 namespace {
 
-constexpr int kTile = 256;     // workgroup tile (M and N)
-constexpr int kSmall = 128;    // the same where 256 leaves compute units idle
-constexpr int kSlab = 32;      // k elements staged per iteration
 // LDS slab layout: 16-byte chunks (8 k values of one row), chunk (c, row) at
 // index c * kChunkPitch + row.  A fragment read then has consecutive lanes on
 // consecutive chunks.  16-byte LDS accesses go eight lanes at a time over 32
@@ -64,7 +62,6 @@ constexpr int kPitchT = kTile + 32;
 constexpr int kOperandElems = kSlab * kPitchT;  // elements per operand slab (either layout fits)
 static_assert((kSlab / 8) * kChunkPitch * 8 <= kOperandElems, "chunk layout must fit");
 constexpr int kThreads = 256;
-constexpr int kXcds = 8;       // accelerator dies, each with a private L2
 constexpr int kRing = 3;       // slabs in flight in registers (prefetch distance)
 constexpr int kEpiPitch = 128 + 8;  // epilogue staging pitch (elements) of a wave's 128x128 tile (4-wave form)
 constexpr size_t kGemmLds =
@@ -91,57 +88,6 @@ template <> struct Mma<MEGA_F16> {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
                                                   __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
   }
-};
-
-// C[m][n] = alpha * sum_k A(m, k) B(n, k); element (m, k) of an operand sits at
-// [m * ld + k], or at [k * ld + m] when the operand is flagged k-major
-struct GemmParams {
-  const uint16_t* A;
-  const uint16_t* B;
-  uint16_t* C;
-  int M, N, K;
-  int64_t lda, ldb, ldc;
-  int64_t sa0, sa1, sb0, sb1, sc0, sc1;  // batch z = z0 * nh + z1 -> offset z0*s0 + z1*s1
-  int nh;
-  float alpha;
-  // Causal structure with rows = queries r, columns = keys c, c <= r + off
-  // (off = L2 - L1 >= 0, the length of a key/value prefix):
-  int tri_out;  // 1: tiles wholly above that diagonal are skipped (left unwritten)
-  int k_mode;   // 0: all k; 1: m = queries, k = keys: k < (mt+1)*256 + off, rounded up to a slab;
-                // 2: m = keys, k = queries: k >= mt*256 - off, rounded down to a slab
-  int off;
-  // persistent schedule (filled in by the launcher): work items of equal weight,
-  // walked by gridDim.x workgroups
-  int mt_count, nt_count;  // tiles along m and n
-  int per_batch;           // work items per batch index
-  int items;               // per_batch * batch
-  int snake;               // 128-wide tiles of unequal length: all of them run at once
-  int ta, tb;   // operand is k-major: element (m, k) at [k * ld + m]
-  int kvb;      // rows of k that a k-major B holds when K has been rounded up behind them (0: all K); A holds
-                // zeros there, and zeros stand in for those rows of B (0 times an infinity would be NaN)
-  int ms;       // rows of C to store when M has been rounded up (0: all M)
-  // Linear layers (LIN): C = A B^T + bias + add, with up to three problems in one launch.  Side by side along n (two
-  // k-contiguous operands: layers of one input) they differ in B, C, ldc, bias and N; along m (two k-major operands: their
-  // weight gradients) in A, lda, C and M.  Tiles mt (nt) >= start[i] belong to problem i + 1.
-  const uint16_t* bias;    // N values or null
-  const uint16_t* add;     // summand of C's layout or null
-  const uint16_t* op[2];
-  uint16_t* out[2];
-  const uint16_t* bias_of[2];
-  int size[2], start[2];
-  // ... and an input gradient whose layers lie behind each other along k: k slabs >= seg_start[i] (of kSlab) are those of
-  // op[i] and op_b[i], rows of A size[i] apart there
-  const uint16_t* op_b[2];
-  int seg_start[2];
-  int kva;      // as kvb, for a k-major A (LIN: rows behind it are not there; else they hold zeros)
-  // CUT: items full .. items - 1, fewer than there are CUs, are cut along k into `cut` parts; float32 sums of part i
-  // of item full + r at parts + (r cut + i) T T, as the waves hold them (linear_parts_kernel adds them up).
-  int full, cut;
-  float* parts;
-  int split_ok;  // (the launcher's: there is memory for the parts)
-  int n_group;  // plain schedule: tiles numbered n fastest inside bands of n_group column tiles, then m,
-                // then band (0: one band) -- the 32 tiles an XCD works on at a time then share fewer
-                // distinct operand blocks (4 x 8 instead of 2 x 16 of a 16-column problem)
 };
 
 template <bool ALIGNED>
@@ -2003,126 +1949,11 @@ int launch_tiles(const GemmParams& q, int grid, int threads, size_t lds, hipStre
   return MEGA_OK;
 }
 
-enum { kForward, kInputGrad, kWeightGrad };
-
-// The tiles of the `count` problems of a launch (sizes along the axis they lie side by side on), in tiles of T.
-void lay_out(GemmParams& q, int kind, int count, const int64_t* sizes, int T) {
-  const auto tiles = [&](int64_t n) { return static_cast<int>((n + T - 1) / T); };
-  q.start[0] = q.start[1] = 0x7fffffff;
-  if (kind != kInputGrad || q.op_b[0] == nullptr) q.seg_start[0] = 0x7fffffff;
-  if (kind != kInputGrad || q.op_b[1] == nullptr) q.seg_start[1] = 0x7fffffff;
-  int along = tiles(sizes[0]);
-  for (int i = 1; i < count; ++i) {
-    q.start[i - 1] = along;
-    q.size[i - 1] = static_cast<int>(sizes[i]);
-    along += tiles(sizes[i]);
-  }
-  q.mt_count = kind == kWeightGrad ? along : tiles(q.M);
-  q.nt_count = kind == kForward ? along : tiles(q.N);
-  q.per_batch = q.items = q.mt_count * q.nt_count;
-  q.full = q.items, q.cut = 0;
-}
-
 int compute_units(int* cus) {
   int dev = 0;
   MEGA_CHECK_HIP(hipGetDevice(&dev));
   MEGA_CHECK_HIP(hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev));
   return MEGA_OK;
-}
-
-// Time of a launch in us by what was measured (1000 to 32768 tokens, layers of 1024 to 11008).  A tile of 256 takes longer
-// for 32 k the more of the chip works (the clock falls: forward 0.45 us alone, 0.80 with every CU busy); tiles of 128 run
-// two to a CU, each pair as long as two one after the other; every round of tiles starts and ends in a few us.
-//
-// Where the last round holds few tiles, they are cut along k, a part for a workgroup, and another launch adds up the parts (0.12
-// us for each part of 256 KB written and read, 14 us for two launches).  2 x 11008 x 4096, us whole / cut: 1531 tokens (516 tiles)
-// 278 / 235, 2100 (774) 351 / 332, 3000 (1032) 477 / 435, 9000 (3096) 1345 / 1288; the parts of few tiles are read by 32
-// workgroups of a wave each (eight of four waves: 19.6 us for 32 parts, so under 10).  Tiles that fill more than half a round stay
-// whole: there is no second workgroup for each.
-double estimate_cut(GemmParams& q, double slabs, int cus) {
-  const int grid = std::max(cus / kXcds, 1) * kXcds, left = q.items % grid, full = q.items - left;
-  const auto round = [&](double tiles, double k) { return k * (0.45 + 0.35 * tiles / grid) + 5; };
-  const double whole = full / grid * round(grid, slabs) + 3;
-  double best = whole + (left > 0 ? round(left, slabs) : 0);
-  for (int cut = 2; cut <= 8 && left > 0 && left * cut <= grid && slabs >= 16 * cut; ++cut) {
-    const double t = whole + round(left * cut, slabs / cut) + 0.12 * left * cut + 14;
-    if (t < best) best = t, q.full = full, q.cut = cut;
-  }
-  return best;
-}
-double estimate(GemmParams& q, int kind, int T, int cus) {
-  const double slabs = (q.K + kSlab - 1) / kSlab, rounds = (q.items + cus - 1) / cus, load = q.items / (rounds * cus);
-  if (T == kTile) {
-    if (kind == kForward && q.split_ok) return estimate_cut(q, slabs, cus);
-    if (kind == kWeightGrad) return rounds * (slabs * (0.40 + 0.36 * load) + 1) + 2;
-    if (kind == kForward) return rounds * (slabs * (0.45 + 0.35 * load) + 5) + 3;
-    return rounds * (slabs * (0.42 + 0.37 * load) + 5) + 2;
-  }
-  if (kind == kWeightGrad) {
-    // Tiles for half of the CUs or fewer are cut along the tokens, as forward products are.  us, whole / cut: 4096 tokens, 2048 x
-    // 1024 (128 tiles) 28.5 / 26.8, 1024 x 1024 28.4 / 23.9, 512 x 512 22.4 / 20.5; 8192 tokens 51 / 40 and (512 x 512)
-    // 50 / 26; 32768 tokens 187 / 127, 191 / 72, 186 / 41.
-    double best = rounds * slabs * 0.23 + 3;
-    for (int cut = 2; q.split_ok && cut <= 16 && q.items * cut <= cus && slabs >= 16 * cut; ++cut) {
-      const double t = slabs / cut * 0.23 + 0.03 * q.items * cut + 7;
-      if (t < best) best = t, q.full = 0, q.cut = cut;
-    }
-    return best;
-  }
-  if (kind == kForward) {
-    // A row or two of tiles read their weights from memory, not from an L2 that others have filled: 0.40 us a slab.  As many as
-    // leave half of the CUs idle are cut along k as well, down to what streaming the weights takes.  us, library / whole / cut: 16
-    // tokens, 1024 + 8192 + 4096 x 4096 60 / 45 / 33; 100 tokens 61 / 53 / 38, 512 + 4096 + 2048 x 2048 64 / 28 / 21.
-    const double slab = q.mt_count <= 2 ? 0.40 : 0.255, stream = 2.0 * q.nt_count * T * q.K / 4.0e6;
-    double best = rounds * (slabs * slab + 1.3) + 3;
-    for (int cut = 2; q.split_ok && cut <= 8 && q.items * cut <= cus && slabs >= 16 * cut; ++cut) {
-      const double t = std::max(slabs / cut * slab, stream) + 0.03 * q.items * cut * std::min(q.M, T) / T + 9;
-      if (t < best) best = t, q.full = 0, q.cut = cut;
-    }
-    return best;
-  }
-  return rounds * (slabs * 0.27 + 1) + 3;
-}
-
-// Lays the tiles out in the size that is expected to be faster; its time.
-double plan(GemmParams& q, int kind, int count, const int64_t* sizes, int cus, bool* small) {
-  GemmParams l = q;
-  lay_out(l, kind, count, sizes, kTile);
-  lay_out(q, kind, count, sizes, kSmall);
-  const double tl = estimate(l, kind, kTile, cus), ts = estimate(q, kind, kSmall, cus);
-  *small = ts <= tl;
-  if (!*small) q = l;
-  return std::min(ts, tl);
-}
-
-// The part of a launch's problems that is problem i alone.
-GemmParams one_of(const GemmParams& q, int kind, int i, int64_t size) {
-  GemmParams o = q;
-  if (kind == kForward) {
-    if (i > 0) o.B = q.op[i - 1], o.C = q.out[i - 1], o.bias = q.bias_of[i - 1];
-    o.N = (int)size;
-    o.ldc = size;
-  } else {
-    if (i > 0) o.A = q.op[i - 1], o.C = q.out[i - 1];
-    o.M = (int)size;
-    o.lda = size;
-  }
-  return o;
-}
-// The time of `count` problems in one launch, or one launch after the other where that is shorter (*apart).
-double plan_group(const GemmParams& q, int kind, int count, const int64_t* sizes, int cus, bool* apart) {
-  GemmParams g = q;
-  bool small;
-  const double together = plan(g, kind, count, sizes, cus, &small);
-  *apart = false;
-  if (count == 1) return together;
-  double sum = 0;
-  for (int i = 0; i < count; ++i) {
-    GemmParams o = one_of(q, kind, i, sizes[i]);
-    sum += plan(o, kind, 1, sizes + i, cus, &small);
-  }
-  *apart = sum < 1.05 * together;  // (at equal rounds of tiles: 2 x 11008 x 4096, 32768 tokens, 4280 us apart, 4384 together)
-  return std::min(sum, together);
 }
 
 template <int DT>
@@ -2189,73 +2020,24 @@ int launch_linear(GemmParams q, int kind, int count, const int64_t* sizes, hipSt
 }  // namespace
 }  // namespace mega
 
-// What a product's launch refuses, or null.  (The contiguous reduction axis of forward and input gradient comes in slabs of 64.)
-static const char* linear_refuses(int kind, int dtype, int64_t tokens, int64_t n_in, int count, const int64_t* n_out) {
-  if (dtype != MEGA_BF16 && dtype != MEGA_F16) return "bfloat16 or float16 tensors";
-  if (count < 1 || count > 3 || n_out == nullptr) return "one to three layers";
-  const int64_t in = kind == kForward ? 64 : 8, out = kind == kInputGrad ? 64 : 8;
-  if (tokens < 1 || n_in < in || n_in % in != 0 || tokens >= (1 << 30) / n_in) return "bad sizes";
-  for (int i = 0; i < count; ++i)
-    if (n_out[i] < out || n_out[i] % out != 0 || tokens >= (1 << 30) / n_out[i] || n_in >= (1 << 30) / n_out[i]) return "bad sizes";
-  return nullptr;
-}
 static int check_linear(const char* who, int kind, int dtype, int64_t tokens, int64_t n_in, int count, const int64_t* n_out) {
   const char* why = linear_refuses(kind, dtype, tokens, n_in, count, n_out);
   return why == nullptr ? MEGA_OK : set_error(MEGA_ERR_INVALID_ARG, "%s: %s", who, why);
 }
 static bool aligned16(const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; }
 
-// Whether the launch is expected to be faster than the library's products, one call a layer.
 extern "C" int mega_linear_takes(int kind, int dtype, int64_t tokens, int64_t n_in, int count, const int64_t* n_out) {
   if (kind < kForward || kind > kWeightGrad || linear_refuses(kind, dtype, tokens, n_in, count, n_out) != nullptr) return 0;
   int cus = 0;
   if (compute_units(&cus) != MEGA_OK) return 0;
-  if (kind == kWeightGrad) {
-    // Both operands run across the reduction axis, the library's slowest layout: this kernel is ahead at every size (us,
-    // library / here): 4096 tokens, 256 + 2048 + 1024 x 1024 91 / 30, 2 x 2752 x 1024 85 / 58, 2 x 5504 x 2048 174 / 166, 11008 x 4096
-    // 380 / 281; 4084 tokens, 2048 x 5504 106 / 82; 1531, 4096 x 11008 174 / 122; 32768, 3328 x 1024 595 / 280, 1024 x 1024 198 / 72,
-    // 512 x 512 152 / 41, 64 x 64 169 / 31.
-    return 1;
-  }
-  GemmParams q{};
-  bool apart;
-  q.M = (int)tokens; q.N = (int)(kind == kForward ? n_out[0] : n_in); q.K = (int)(kind == kForward ? n_in : 0);
-  if (kind == kInputGrad)
-    for (int i = 0; i < count; ++i) q.K += (int)n_out[i];
-  q.split_ok = 1;
-  const double here = plan_group(q, kind, kind == kForward ? count : 1, kind == kForward ? n_out : &n_in, cus, &apart);
-  // The library: at least 20 us a call (its host path), then what it reaches on products of so many terms, in PFLOP/s; widths
-  // off the multiples of 1024 cost it a quarter up to some 2^39.  Forward, us (library / here): 4096 tokens, 256 + 2048 + 1024 x
-  // 1024 60 / 33, 2 x 2752 x 1024 71 / 61, 2 x 5504 x 2048 181 / 165, 2 x 11008 x 4096 813 / 594, 4096 x 2048 51 / 61, 8192 x 4096
-  // 180 / 214; 1531 tokens, 2 x 11008 x 4096 262 / 283.  Input gradient: 2752 x 1024 32 / 24, 4096 x 2048 65 / 73.
-  double library = 0;
-  for (int i = 0; i < count; ++i) {
-    const double products = static_cast<double>(tokens) * n_in * n_out[i];
-    if (kind == kInputGrad && products > 0x1p35) return 0;  // goes through a transposed copy of W there
-    const double rate = kind == kInputGrad ? 1.1 : products > 0x1p39 ? 1.5 : products < 0x1p33 ? 1.0 : n_out[i] % 1024 == 0 ? 1.4 : 1.1;
-    const double stream = kind == kForward && tokens <= 256 ? 2.0 * n_in * n_out[i] / 3.3e6 + 3 : 0;  // the weights from memory
-    library += std::max({20.0, stream, 2e-9 * products / rate + (kind == kInputGrad ? 10 : 8)});
-  }
-  return here <= library;
+  return linear_takes(kind, tokens, n_in, count, n_out, cus);
 }
 
 extern "C" int64_t mega_linear_workspace_bytes(int kind, int64_t tokens, int64_t n_in, int count, const int64_t* n_out) {
   if ((kind != kForward && kind != kWeightGrad) || linear_refuses(kind, MEGA_BF16, tokens, n_in, count, n_out) != nullptr) return 0;
   int cus = 0;
   if (compute_units(&cus) != MEGA_OK) return 0;
-  GemmParams q{};
-  q.M = (int)(kind == kForward ? tokens : n_out[0]); q.N = (int)(kind == kForward ? n_out[0] : n_in); q.K = (int)(kind == kForward ? n_in : tokens);
-  q.split_ok = 1;
-  bool apart, small;
-  plan_group(q, kind, count, n_out, cus, &apart);
-  int64_t values = 0;
-  for (int i = 0; i < (apart ? count : 1); ++i) {
-    GemmParams o = apart ? one_of(q, kind, i, n_out[i]) : q;
-    plan(o, kind, apart ? 1 : count, apart ? n_out + i : n_out, cus, &small);
-    const int64_t tile = small ? kSmall : kTile;
-    values = std::max(values, static_cast<int64_t>(o.items - o.full) * o.cut * tile * tile);
-  }
-  return values * static_cast<int64_t>(sizeof(float));
+  return linear_workspace_bytes(kind, tokens, n_in, count, n_out, cus);
 }
 
 extern "C" int mega_linear_fwd(const void* x, const void* const* w, const void* const* bias, const void* add, int dtype,

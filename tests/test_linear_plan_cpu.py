@@ -1,0 +1,35 @@
+"""The choice of tiles for the linear layers' products, and whether they are taken at all (linear_plan.hpp): plain C++, built
+with g++ and asked about a chip of 256 compute units."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+SRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "linear_plan_emu.cc")
+FORWARD, INPUT_GRAD, WEIGHT_GRAD = 0, 1, 2
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    """ask(name, kind, tokens, n_in, *n_out)"""
+    out = tmp_path_factory.mktemp("emu") / "liblinear_plan_emu.so"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-o", str(out), SRC], check=True)
+    lib, i64 = ctypes.CDLL(str(out)), ctypes.c_int64
+    lib.emu_linear_time.restype = ctypes.c_double
+
+    def call(name, kind, tokens, n_in, *n_out):
+        return getattr(lib, "emu_linear_" + name)(kind, i64(tokens), i64(n_in), len(n_out), (i64 * len(n_out))(*n_out), 256)
+
+    return call
+
+
+@pytest.mark.parametrize("kind,tokens,n_in,n_out,tile", [
+    (FORWARD, 1021, 2048, [512, 4096, 2048], 128),
+    (FORWARD, 1531, 4096, [11008, 11008], 256),
+    (INPUT_GRAD, 4096, 2752, [1024], 256),                # one layer
+    (INPUT_GRAD, 4084, 2048, [512, 4096, 2048], 128),     # joined along k
+    (WEIGHT_GRAD, 4084, 2048, [512, 4096, 2048], 256),
+])
+def test_tiles(ask, kind, tokens, n_in, n_out, tile):
+    assert ask("tile", kind, tokens, n_in, *n_out) == tile
