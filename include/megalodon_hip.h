@@ -406,11 +406,13 @@ int mega_linear_weight_grad(const void* dy, const void* x, int dtype, int64_t to
                             int64_t n_out, int64_t n_in, void* dw, void* stream);
 
 /* The three products of linear layers on the same kernels, for one to three layers of one input
- * (n_out[i] each; `count`) in one launch: tensors of `dtype` (MEGA_BF16 / MEGA_F16, float32 accumulation, one
- * rounding), contiguous, on 16-byte boundaries, n_in and n_out multiples of 8, every matrix of fewer than 2^30 elements.
+ * (n_out[i] each; `count`) in as few launches as is fastest: one for all of them or one each, two or three where a product
+ * is cut along its reduction axis.  Tensors of `dtype` (MEGA_BF16 / MEGA_F16, float32 accumulation, rounded at the end),
+ * contiguous, on 16-byte boundaries, n_in and n_out multiples of 8, every matrix of fewer than 2^30 elements.
  *   fwd:          y_i (tokens, n_out_i) = x (tokens, n_in) w_i^T + bias_i + add; bias, an entry of it and add may be
  *                 null; add (tokens, n_out) with one layer only; n_in a multiple of 64.
- *   input_grad:   dx = sum_i dy_i w_i + add; add (tokens, n_in) or null, may be dx itself; n_out a multiple of 64.
+ *   input_grad:   dx = sum_i dy_i w_i + add; add (tokens, n_in) or null, may be dx itself; n_out a multiple of 64.  Rounded
+ *                 once where the layers are one product along all of their outputs, else (large ones) once for each layer.
  *   weight_grads: dw_i = dy_i^T x.
  * `workspace` of fwd and weight_grads: mega_linear_workspace_bytes(0 or 2, ...) bytes (up to 64 MiB; for many sizes 0), or
  * null: no product is cut along its reduction axis then, which makes some sizes slower.

@@ -2073,15 +2073,7 @@ extern "C" int mega_linear_input_grad(const void* const* dy, const void* const* 
   g.ldb = n_in; g.ldc = n_in; g.tb = 1;
   int cus = 0;
   if (const int rc2 = compute_units(&cus); rc2 != MEGA_OK) return rc2;
-  // One product with the layers behind each other along k, in tiles of 128: one rounding, and dx is neither read again nor
-  // launched for again.  us, one after the other / so: 4096 tokens, 256 + 2048 + 1024 x 1024 50 / 32, 2 x 2752 x 1024 59 / 50; 4084
-  // tokens, 512 + 4096 + 2048 x 2048 140 / 114; 500 tokens of the first 41 / 26.  Where tiles of 256 are the faster ones, one
-  // after the other.
-  GemmParams all = g;
-  bool small = false;
-  for (int i = 0; i < count; ++i) all.K += (int)n_out[i];
-  plan(all, kInputGrad, 1, &n_in, cus, &small);
-  for (int i = 0, n = small ? count : 1; i < count; i += n) {
+  for (int i = 0, n = joined_along_k(tokens, n_in, count, n_out, cus) ? count : 1; i < count; i += n) {
     g.A = u(dy[i]); g.B = u(w[i]); g.K = (int)n_out[i]; g.lda = n_out[i];
     g.add = i == 0 ? u(add) : u(dx);
     for (int k = 1; k < n; ++k) {

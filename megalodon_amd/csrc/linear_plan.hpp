@@ -134,11 +134,24 @@ inline GemmParams linear_sizes(int kind, int64_t tokens, int64_t n_in, int count
   q.split_ok = 1;
   return q;
 }
-// The time of a call.
+// Whether the layers of an input gradient lie behind each other along k of one product, in tiles of 128: one rounding, and dx
+// is neither read again nor launched for again.  us, one after the other / so: 4096 tokens, 256 + 2048 + 1024 x 1024 50 / 32,
+// 2 x 2752 x 1024 59 / 50; 4084 tokens, 512 + 4096 + 2048 x 2048 140 / 114; 500 tokens of the first 41 / 26.  Where tiles of
+// 256 are the faster ones, one after the other, each onto the sum so far.
+inline bool joined_along_k(int64_t tokens, int64_t n_in, int count, const int64_t* n_out, int cus) {
+  GemmParams all = linear_sizes(kInputGrad, tokens, n_in, count, n_out);
+  bool small;
+  plan(all, kInputGrad, 1, &n_in, cus, &small);
+  return small;
+}
+// The time of a call, of all of its launches.
 inline double linear_time(int kind, int64_t tokens, int64_t n_in, int count, const int64_t* n_out, int cus) {
-  const GemmParams q = linear_sizes(kind, tokens, n_in, count, n_out);
   bool apart;
-  return plan_group(q, kind, kind == kInputGrad ? 1 : count, kind == kInputGrad ? &n_in : n_out, cus, &apart);
+  if (kind != kInputGrad) return plan_group(linear_sizes(kind, tokens, n_in, count, n_out), kind, count, n_out, cus, &apart);
+  const int n = joined_along_k(tokens, n_in, count, n_out, cus) ? count : 1;
+  double time = 0;
+  for (int i = 0; i < count; i += n) time += plan_group(linear_sizes(kind, tokens, n_in, n, n_out + i), kind, 1, &n_in, cus, &apart);
+  return time;
 }
 
 // What a product's launch refuses, or null.  (The contiguous reduction axis of forward and input gradient comes in slabs of 64.)

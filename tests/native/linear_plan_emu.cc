@@ -14,19 +14,24 @@ extern "C" double emu_linear_time(int kind, int64_t tokens, int64_t n_in, int co
 
 // the tile of a call's products: 128 or 256, 0 where its layers run in tiles of either
 extern "C" int emu_linear_tile(int kind, int64_t tokens, int64_t n_in, int count, const int64_t* n_out, int cus) {
-  GemmParams q = linear_sizes(kind, tokens, n_in, count, n_out);
+  const GemmParams q = linear_sizes(kind, tokens, n_in, count, n_out);
   bool apart = false, small = false;
-  if (kind == kInputGrad) {
-    plan(q, kind, 1, &n_in, cus, &small);
-    return small ? kSmall : kTile;
-  }
-  plan_group(q, kind, count, n_out, cus, &apart);
   int tile = -1;
-  for (int i = 0; i < (apart ? count : 1); ++i) {
-    GemmParams o = apart ? one_of(q, kind, i, n_out[i]) : q;
-    plan(o, kind, apart ? 1 : count, apart ? n_out + i : n_out, cus, &small);
+  const auto with = [&](GemmParams o, int n, const int64_t* sizes) {
+    plan(o, kind, n, sizes, cus, &small);
     const int t = small ? kSmall : kTile;
     tile = tile < 0 || tile == t ? t : 0;
+  };
+  if (kind == kInputGrad) {
+    const int n = joined_along_k(tokens, n_in, count, n_out, cus) ? count : 1;
+    for (int i = 0; i < count; i += n) with(linear_sizes(kind, tokens, n_in, n, n_out + i), 1, &n_in);
+    return tile;
   }
+  plan_group(q, kind, count, n_out, cus, &apart);
+  for (int i = 0; i < (apart ? count : 1); ++i) with(apart ? one_of(q, kind, i, n_out[i]) : q, apart ? 1 : count, apart ? n_out + i : n_out);
   return tile;
+}
+
+extern "C" int emu_linear_joined(int, int64_t tokens, int64_t n_in, int count, const int64_t* n_out, int cus) {
+  return joined_along_k(tokens, n_in, count, n_out, cus);
 }

@@ -33,3 +33,18 @@ def ask(tmp_path_factory):
 ])
 def test_tiles(ask, kind, tokens, n_in, n_out, tile):
     assert ask("tile", kind, tokens, n_in, *n_out) == tile
+
+
+def test_input_gradients_one_after_the_other_are_priced_so(ask):
+    """Layers that are not joined along k cost a launch each, not one product along all of their outputs."""
+    apart = 0
+    for tokens in (500, 2100, 4096, 7000, 10000, 16384):
+        for n_in, n_out in ((1024, (2752, 2752)), (1280, (1280, 1280, 1280)), (1024, (256, 2048, 1024))):
+            alone = sum(ask("time", INPUT_GRAD, tokens, n_in, n) for n in n_out)
+            together = ask("time", INPUT_GRAD, tokens, n_in, *n_out)
+            if ask("joined", INPUT_GRAD, tokens, n_in, *n_out):
+                assert together < alone
+            else:
+                assert together == pytest.approx(alone)
+                apart += 1
+    assert apart >= 3
