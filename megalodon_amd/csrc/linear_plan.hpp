@@ -2,6 +2,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 
 #include "../../include/megalodon_hip.h"
@@ -165,29 +166,55 @@ inline const char* linear_refuses(int kind, int dtype, int64_t tokens, int64_t n
   return nullptr;
 }
 
+// The time in us of a general library's product of x (tokens, n_in) and a layer (n_out, n_in), forward or the input gradient: the
+// smaller of two estimates, and no less than its host path (20 us) or than reading the weights for few tokens takes.
+// One is the mean rate of products of so many terms, in PFLOP/s; widths off the multiples of 1024 cost it a quarter up to some 2^39.
+// The other is what the tiles allow.  The library's are up to 256 x 256, in as many rounds as they need, by as many workgroups as
+// divide them evenly; where none does, tiles are cut along k between workgroups, which costs about 1.3 tiles.  PFLOP/s of 4096
+// -> 11008: 2500 tokens (430 tiles, two rounds of 215) 1.42, 5000 (four of 215) 1.46, 4096 (688) 0.92, 3500 (602) 0.90; 6912 -> 2560:
+// 12000 (two of 235) 1.58, 16384 (640) 1.02.  For up to two rounds it looks for a tile that fits, then takes 256 x 256.  Widths off
+// 256 cost up to two rounds 20 % and more rounds 10.
+inline double library_time(int kind, int64_t tokens, int64_t n_in, int64_t n_out, int cus) {
+  const double products = static_cast<double>(tokens) * n_in * n_out;
+  const double rate = kind == kInputGrad ? 1.1 : products > 0x1p39 ? 1.5 : products < 0x1p33 ? 1.0 : n_out % 1024 == 0 ? 1.4 : 1.1;
+  const double mean = 2e-9 * products / rate + (kind == kInputGrad ? 10 : 8);
+  const int64_t cols = kind == kInputGrad ? n_in : n_out, k = kind == kInputGrad ? n_out : n_in;
+  const auto in_tiles = [&](int64_t m, int64_t n) {
+    const double tile = 1.2 / 64 * k * std::pow(m * n / 65536.0, 0.75) + 6;
+    const int64_t tiles = (tokens + m - 1) / m * ((cols + n - 1) / n), rounds = (tiles + cus - 1) / cus;
+    return (tiles % rounds == 0 ? static_cast<double>(rounds) : static_cast<double>(tiles) / cus + 1.3) * tile + 3;
+  };
+  double even = in_tiles(256, 256);
+  const bool fitted = (tokens + 255) / 256 * ((cols + 255) / 256) <= 2 * cus;
+  constexpr int kShapes[][2] = {{256, 192}, {256, 160}, {256, 128}, {192, 128}, {160, 128}, {128, 128}, {128, 64}, {64, 64}};
+  for (int i = 0; fitted && i < 8; ++i) even = std::min({even, in_tiles(kShapes[i][0], kShapes[i][1]), in_tiles(kShapes[i][1], kShapes[i][0])});
+  if (cols % 256 != 0) even *= fitted ? 1.2 : 1.1;
+  const double stream = kind == kForward && tokens <= 256 ? 2.0 * n_in * n_out / 3.3e6 + 3 : 0;
+  return std::max({20.0, stream, std::min(mean, even)});
+}
+
 // Whether the launch is expected to be faster than the library's products, one call a layer (sizes that linear_refuses lets pass).
 inline bool linear_takes(int kind, int64_t tokens, int64_t n_in, int count, const int64_t* n_out, int cus) {
   if (kind == kWeightGrad) {
-    // Both operands run across the reduction axis, the library's slowest layout: this kernel is ahead at every size (us,
+    // Both operands run across the reduction axis, the library's slowest layout: this kernel is ahead at nearly every size (us,
     // library / here): 4096 tokens, 256 + 2048 + 1024 x 1024 91 / 30, 2 x 2752 x 1024 85 / 58, 2 x 5504 x 2048 174 / 166, 11008 x 4096
     // 380 / 281; 4084 tokens, 2048 x 5504 106 / 82; 1531, 4096 x 11008 174 / 122; 32768, 3328 x 1024 595 / 280, 1024 x 1024 198 / 72,
-    // 512 x 512 152 / 41, 64 x 64 169 / 31.
+    // 512 x 512 152 / 41, 64 x 64 169 / 31.  Of 640 measured (300 to 32768 tokens, layers and groups of 768 to 13824) four are 3 to 16 %
+    // slower, all of 24000 tokens and more: 32768, 2560 x 6912 1290 / 1490.
     return true;
   }
   const double here = linear_time(kind, tokens, n_in, count, n_out, cus);
-  // The library: at least 20 us a call (its host path), then what it reaches on products of so many terms, in PFLOP/s; widths
-  // off the multiples of 1024 cost it a quarter up to some 2^39.  Forward, us (library / here): 4096 tokens, 256 + 2048 + 1024 x
-  // 1024 60 / 33, 2 x 2752 x 1024 71 / 61, 2 x 5504 x 2048 181 / 165, 2 x 11008 x 4096 813 / 594, 4096 x 2048 51 / 61, 8192 x 4096
-  // 180 / 214; 1531 tokens, 2 x 11008 x 4096 262 / 283.  Input gradient: 2752 x 1024 32 / 24, 4096 x 2048 65 / 73.
+  // Of 3128 forward products and input gradients, alone and in groups (300 to 32768 tokens, layers of 512 to 13824, widths on and
+  // off 256), this takes 806: 24 of them are more than 3 % slower than the library's calls (1.10 in the mean, the worst 1.35), the
+  // others 1.39 times as fast in the mean.  By the mean rate alone it took 1059, 193 of them slower (1.13 in the mean).  us, library /
+  // here: 4096 tokens, 256 + 2048 + 1024 x 1024 60 / 33, 2 x 2752 x 1024 71 / 61, 2 x 5504 x 2048 181 / 165, 2 x 11008 x 4096 800 / 585;
+  // left to the library: 2 x 11008 x 4096 of 1250 tokens 167 / 204, of 2500 317 / 374, of 5000 616 / 666.
   double library = 0;
   for (int i = 0; i < count; ++i) {
-    const double products = static_cast<double>(tokens) * n_in * n_out[i];
-    if (kind == kInputGrad && products > 0x1p35) return false;  // goes through a transposed copy of W there
-    const double rate = kind == kInputGrad ? 1.1 : products > 0x1p39 ? 1.5 : products < 0x1p33 ? 1.0 : n_out[i] % 1024 == 0 ? 1.4 : 1.1;
-    const double stream = kind == kForward && tokens <= 256 ? 2.0 * n_in * n_out[i] / 3.3e6 + 3 : 0;  // the weights from memory
-    library += std::max({20.0, stream, 2e-9 * products / rate + (kind == kInputGrad ? 10 : 8)});
+    if (kind == kInputGrad && static_cast<double>(tokens) * n_in * n_out[i] > 0x1p35) return false;  // goes through a transposed copy of W there
+    library += library_time(kind, tokens, n_in, n_out[i], cus);
   }
-  return here <= library;
+  return here <= 1.02 * library;  // (large tiles here take 2 to 5 % less than their estimate)
 }
 
 // The memory for the parts of cut tiles.

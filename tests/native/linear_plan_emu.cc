@@ -35,3 +35,9 @@ extern "C" int emu_linear_tile(int kind, int64_t tokens, int64_t n_in, int count
 extern "C" int emu_linear_joined(int, int64_t tokens, int64_t n_in, int count, const int64_t* n_out, int cus) {
   return joined_along_k(tokens, n_in, count, n_out, cus);
 }
+
+extern "C" double emu_linear_library(int kind, int64_t tokens, int64_t n_in, int count, const int64_t* n_out, int cus) {
+  double time = 0;
+  for (int i = 0; i < count; ++i) time += library_time(kind, tokens, n_in, n_out[i], cus);
+  return time;
+}

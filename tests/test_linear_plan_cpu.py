@@ -48,3 +48,29 @@ def test_input_gradients_one_after_the_other_are_priced_so(ask):
                 assert together == pytest.approx(alone)
                 apart += 1
     assert apart >= 3
+
+
+# us measured, (library, here): products that the library's tiles fit, which stay there, and products that they do not fit
+@pytest.mark.parametrize("kind,tokens,n_in,n_out,library,here", [
+    (FORWARD, 1250, 4096, [11008, 11008], 167, 204),
+    (FORWARD, 2500, 4096, [11008, 11008], 317, 374),
+    (FORWARD, 5000, 4096, [11008, 11008], 616, 666),
+    (FORWARD, 12000, 6912, [2560], 269, 332),
+    (FORWARD, 3500, 4608, [4608], 98, 118),
+    (FORWARD, 4096, 3584, [3584], 72, 89),
+    (FORWARD, 32768, 1536, [1536], 112, 137),
+    (FORWARD, 32768, 2048, [5504, 5504], 1025, 1149),
+    (INPUT_GRAD, 7000, 1280, [1280, 1280, 1280], 87, 117),
+    (INPUT_GRAD, 10000, 1024, [2752, 2752], 105, 128),
+    (FORWARD, 1531, 4096, [11008, 11008], 261, 244),
+    (FORWARD, 2100, 4096, [11008, 11008], 566, 335),
+    (FORWARD, 4096, 4096, [11008, 11008], 800, 585),
+    (FORWARD, 4096, 1024, [2752, 2752], 66, 55),
+    (FORWARD, 4096, 2048, [5504, 5504], 169, 151),
+    (FORWARD, 1000, 2048, [512, 4096, 2048], 46, 31),
+    (INPUT_GRAD, 4096, 1024, [256, 2048, 1024], 48, 31),
+    (INPUT_GRAD, 4096, 2752, [1024], 35, 27),
+    (WEIGHT_GRAD, 32768, 512, [512], 152, 41),
+])
+def test_products_go_where_they_are_faster(ask, kind, tokens, n_in, n_out, library, here):
+    assert ask("takes", kind, tokens, n_in, *n_out) == (here < library)
