@@ -24,10 +24,14 @@ def ask(tmp_path_factory):
     return call
 
 
-@pytest.mark.parametrize("kind,tokens,n_in,n_out,tile", [
+@pytest.mark.parametrize("kind,tokens,n_in,n_out,tile", [  # (among them the sizes that stand for a tile in test_linear_products_gpu.py)
     (FORWARD, 1021, 2048, [512, 4096, 2048], 128),
     (FORWARD, 1531, 4096, [11008, 11008], 256),
+    (FORWARD, 4084, 1024, [2752, 2752], 256),
     (INPUT_GRAD, 4096, 2752, [1024], 256),                # one layer
+    (INPUT_GRAD, 4093, 2752, [1024], 256),
+    (INPUT_GRAD, 4093, 2744, [1024, 512], 256),           # one after the other
+    (WEIGHT_GRAD, 1021, 2048, [512, 4096, 2048], 256),
     (INPUT_GRAD, 4084, 2048, [512, 4096, 2048], 128),     # joined along k
     (WEIGHT_GRAD, 4084, 2048, [512, 4096, 2048], 256),
 ])

@@ -1,7 +1,7 @@
 """The linear layers' three products on the library's own kernels (`mega_linear_*`), one to three layers of one input in a
 launch, against float64: one row, edges of tiles of 128 and 256, tokens off the slabs of 32, layers narrower than a
-tile, sizes that take either tile.  A 16-bit result of a float32 accumulation: 2^-9 of each value (bfloat16, float16
-2^-12) from its one rounding, and as much again for sums of thousands of terms in float32."""
+tile, sizes that take either tile.  A 16-bit result of a float32 accumulation: 2^-8 of each value (bfloat16, float16
+2^-11) from its one rounding, in the norm over all of them about half of that, and what the sums themselves are off by."""
 import ctypes
 
 import pytest
@@ -28,10 +28,27 @@ def _poisoned(t):  # NaN behind the last element
     return buf[:t.numel()].view(t.shape).copy_(t)
 
 
-def _close(got, want):
-    eps = 2.0 ** -8 if got.dtype == torch.bfloat16 else 2.0 ** -11
+def _eps(dtype):
+    return 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+
+
+def _sum(a, b, *more):
+    """a @ b and summands of its shape in float64, and how far a sum of these terms in float32 can be from it: roundings of
+    2^-23 at most (cut off, not to nearest) of no more than the sum of the magnitudes, one for each four terms at
+    least (a matrix instruction adds up 16 or 8), one for each summand and a few for parts that are added up."""
+    want, size = a @ b, a.abs() @ b.abs()
+    for m in more:
+        want, size = want + m, size + m.abs()
+    return want, size * ((a.shape[-1] / 4 + 16) * 2.0 ** -23)
+
+
+def _close(got, want, reach=None):
+    """In the norm, and with `reach` (the sum's own error) every value: a rounding of what is off by that much."""
+    eps = _eps(got.dtype)
     assert torch.isfinite(got.float()).all()
     assert (got.double() - want).norm() <= eps * want.norm()
+    if reach is not None:
+        assert ((got.double() - want).abs() <= eps * want.abs() + (1 + eps) * reach).all()
 
 
 @pytest.mark.parametrize("tokens,n_in,n_out,dtype", [
@@ -41,11 +58,11 @@ def _close(got, want):
     (129, 128, [64, 320, 128], torch.bfloat16),
     (256, 256, [256, 128, 64], torch.float16),
     (257, 320, [192], torch.bfloat16),
-    (1021, 2048, [512, 4096, 2048], torch.bfloat16),   # tiles of 256 forward
+    (1021, 2048, [512, 4096, 2048], torch.bfloat16),   # tiles of 256 for the weight gradients
     (1021, 5504, [2048], torch.bfloat16),
     (2048, 2048, [5504], torch.float16),
-    (4084, 1024, [2752, 2752], torch.bfloat16),
-    (4084, 2048, [512, 4096, 2048], torch.bfloat16),   # tiles of 256 for the weight gradients
+    (4084, 1024, [2752, 2752], torch.bfloat16),        # tiles of 256 forward
+    (4084, 2048, [512, 4096, 2048], torch.bfloat16),   # and for the weight gradients
     (4100, 704, [2048, 64], torch.float16),
 ])
 def test_products_match_float64(tokens, n_in, n_out, dtype):
@@ -73,27 +90,57 @@ def test_products_match_float64(tokens, n_in, n_out, dtype):
     call("mega_linear_weight_grads", _pointers(dy), _lib.ptr(x), _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(len(w)), outs, _pointers(dw), _lib.ptr(ws) if size else None)
     x64, w64, dy64 = x.double(), [t.double() for t in w], [t.double() for t in dy]
     for i in range(len(w)):
-        _close(y[i], x64 @ w64[i].t() + (0 if bias[i] is None else bias[i].double()))
-        _close(dw[i], dy64[i].t() @ x64)
+        forward = _sum(x64, w64[i].t(), *([] if bias[i] is None else [bias[i].double()]))
+        _close(y[i], *forward)
+        _close(dw[i], *_sum(dy64[i].t(), x64))
         # one layer alone gives the same bits as in the group, where neither is cut
         if len(w) > 1:
             alone, whole = torch.empty_like(y[i]), [torch.empty_like(t) for t in y]
             fwd([w[i]], [bias[i]], None, [n_out[i]], [alone], cut=False)
             fwd(w, bias, None, n_out, whole, cut=False)
             assert torch.equal(alone, whole[i])
-            _close(alone, x64 @ w64[i].t() + (0 if bias[i] is None else bias[i].double()))
+            _close(alone, *forward)
     fwd(w[:1], None, _lib.ptr(add), n_out[:1], y[:1])
-    _close(y[0], x64 @ w64[0].t() + add.double())
+    _close(y[0], *_sum(x64, w64[0].t(), add.double()))
     dx = torch.empty_like(x)
     for i in range(len(w)):  # added up in place
         before = dx.double()
         call("mega_linear_input_grad", _pointers(dy[i:i + 1]), _pointers(w[i:i + 1]), _lib.ptr(dx) if i else None, _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(1), (i64 * 1)(n_out[i]), _lib.ptr(dx))
-        _close(dx, dy64[i] @ w64[i] + (before if i else 0))
+        _close(dx, *_sum(dy64[i], w64[i], *([before] if i else [])))
     # all of the layers at once, onto a summand
     start = rows(tokens, n_in).to(dtype)
     dx = torch.full_like(start, float("nan"))
     call("mega_linear_input_grad", _pointers(dy), _pointers(w), _lib.ptr(start), _lib.i32(code), i64(tokens), i64(n_in), _lib.i32(len(w)), outs, _lib.ptr(dx))
-    _close(dx, sum(a @ b for a, b in zip(dy64, w64)) + start.double())
+    _close(dx, *_sum(torch.cat(dy64, 1), torch.cat(w64), start.double()))
+
+
+@pytest.mark.parametrize("tokens,n_in,n_out,dtype", [
+    (4096, 2752, [1024], torch.bfloat16),
+    (4093, 2752, [1024], torch.float16),           # rows that end inside a tile
+    (4093, 2744, [1024, 512], torch.bfloat16),     # columns too; two layers, one after the other
+])
+@pytest.mark.parametrize("onto", ["nothing", "summand", "itself"])
+def test_input_gradients_in_tiles_of_256(tokens, n_in, n_out, dtype, onto):
+    """Sizes whose input gradients take the large tiles, a launch and a rounding for each layer: without a summand, with one, and
+    with the result's own memory as the summand."""
+    g = torch.Generator("cuda").manual_seed(tokens + len(onto))
+    rows = lambda *s: _poisoned(torch.randn(*s, generator=g, device="cuda").to(dtype))
+    dy, w, i64 = [rows(tokens, o) for o in n_out], [rows(o, n_in) for o in n_out], ctypes.c_int64
+    start = rows(tokens, n_in)
+    behind = torch.full((tokens * n_in + 4096,), float("nan"), dtype=dtype, device="cuda")
+    dx = behind[:tokens * n_in].view(tokens, n_in)
+    if onto == "itself":
+        dx.copy_(start)
+    add = {"nothing": None, "summand": _lib.ptr(start), "itself": _lib.ptr(dx)}[onto]
+    _lib.call("mega_linear_input_grad", _pointers(dy), _pointers(w), add, _lib.i32(_lib.dtype_code(dtype)), i64(tokens), i64(n_in),
+              _lib.i32(len(w)), (i64 * len(w))(*n_out), _lib.ptr(dx), _lib.stream_ptr(dx.device))
+    want, reach = (0, 0) if onto == "nothing" else (start.double(), 0)
+    for i in range(len(w)):  # what the sum so far is off by, its rounding included, goes into the next
+        before = reach if i == 0 else reach + _eps(dtype) * (want.abs() + reach)
+        want, own = _sum(dy[i].double(), w[i].double(), *([] if onto == "nothing" and i == 0 else [want]))
+        reach = before + own
+    _close(dx, want, reach)
+    assert behind[tokens * n_in:].isnan().all()
 
 
 def test_refused_sizes():
@@ -163,9 +210,9 @@ def test_last_tiles_cut_along_k(tokens, n_in, n_out, dtype):
     once, again, whole = run(_lib.ptr(parts)), run(_lib.ptr(parts)), run(None)
     assert (parts[bytes_:] == 255).all()
     for i, o in enumerate(n_out):
-        want = x.double() @ w[i].double().t() + bias[i].double() + (0 if summed is None else summed.double())
-        _close(once[i], want)
-        _close(whole[i], want)
+        want = _sum(x.double(), w[i].double().t(), bias[i].double(), *([] if summed is None else [summed.double()]))
+        _close(once[i], *want)
+        _close(whole[i], *want)
         assert torch.equal(once[i], again[i])
 
 
@@ -317,7 +364,7 @@ def test_weight_gradients_cut_along_the_tokens(tokens, n_in, n_out, dtype):
     once, again, whole = run(_lib.ptr(parts)), run(_lib.ptr(parts)), run(None)
     assert (parts[size:] == 255).all()
     for i in range(len(n_out)):
-        want = dy[i].double().t() @ x.double()
-        _close(once[i], want)
-        _close(whole[i], want)
+        want = _sum(dy[i].double().t(), x.double())
+        _close(once[i], *want)
+        _close(whole[i], *want)
         assert torch.equal(once[i], again[i])
