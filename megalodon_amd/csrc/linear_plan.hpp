@@ -167,14 +167,14 @@ inline const char* linear_refuses(int kind, int dtype, int64_t tokens, int64_t n
 }
 
 // The time in us of a general library's product of x (tokens, n_in) and a layer (n_out, n_in), forward or the input gradient: the
-// smaller of two estimates, and no less than its host path (20 us) or than reading the weights for few tokens takes.
+// smaller of two estimates, and no less than its host path (`host`) or than reading the weights for few tokens takes.
 // One is the mean rate of products of so many terms, in PFLOP/s; widths off the multiples of 1024 cost it a quarter up to some 2^39.
 // The other is what the tiles allow.  The library's are up to 256 x 256, in as many rounds as they need, by as many workgroups as
 // divide them evenly; where none does, tiles are cut along k between workgroups, which costs about 1.3 tiles.  PFLOP/s of 4096
 // -> 11008: 2500 tokens (430 tiles, two rounds of 215) 1.42, 5000 (four of 215) 1.46, 4096 (688) 0.92, 3500 (602) 0.90; 6912 -> 2560:
 // 12000 (two of 235) 1.58, 16384 (640) 1.02.  For up to two rounds it looks for a tile that fits, then takes 256 x 256.  Widths off
 // 256 cost up to two rounds 20 % and more rounds 10.
-inline double library_time(int kind, int64_t tokens, int64_t n_in, int64_t n_out, int cus) {
+inline double library_time(int kind, int64_t tokens, int64_t n_in, int64_t n_out, int cus, double host) {
   const double products = static_cast<double>(tokens) * n_in * n_out;
   const double rate = kind == kInputGrad ? 1.1 : products > 0x1p39 ? 1.5 : products < 0x1p33 ? 1.0 : n_out % 1024 == 0 ? 1.4 : 1.1;
   const double mean = 2e-9 * products / rate + (kind == kInputGrad ? 10 : 8);
@@ -190,7 +190,7 @@ inline double library_time(int kind, int64_t tokens, int64_t n_in, int64_t n_out
   for (int i = 0; fitted && i < 8; ++i) even = std::min({even, in_tiles(kShapes[i][0], kShapes[i][1]), in_tiles(kShapes[i][1], kShapes[i][0])});
   if (cols % 256 != 0) even *= fitted ? 1.2 : 1.1;
   const double stream = kind == kForward && tokens <= 256 ? 2.0 * n_in * n_out / 3.3e6 + 3 : 0;
-  return std::max({20.0, stream, std::min(mean, even)});
+  return std::max({host, stream, std::min(mean, even)});
 }
 
 // Whether the launch is expected to be faster than the library's products, one call a layer (sizes that linear_refuses lets pass).
@@ -209,10 +209,14 @@ inline bool linear_takes(int kind, int64_t tokens, int64_t n_in, int count, cons
   // others 1.39 times as fast in the mean.  By the mean rate alone it took 1059, 193 of them slower (1.13 in the mean).  us, library /
   // here: 4096 tokens, 256 + 2048 + 1024 x 1024 60 / 33, 2 x 2752 x 1024 71 / 61, 2 x 5504 x 2048 181 / 165, 2 x 11008 x 4096 800 / 585;
   // left to the library: 2 x 11008 x 4096 of 1250 tokens 167 / 204, of 2500 317 / 374, of 5000 616 / 666.
+  // Its host path is 18 us a call, more than many small products take.  A single layer of few tokens is up to 3 us above its
+  // estimate here, so it has to be ahead by as much (us, library / here: 16 tokens, 5504 -> 2048 18.5 / 21.1, 512 tokens, 2752 ->
+  // 1024 18.4 / 20.1; 16 tokens, 1024 -> 1024 18.3 / 9.7); several take less (384 tokens, 2 x 5504 x 2048 39.3 / 29.7, estimate 38).
+  const double host = count == 1 ? 17 : 20;
   double library = 0;
   for (int i = 0; i < count; ++i) {
     if (kind == kInputGrad && static_cast<double>(tokens) * n_in * n_out[i] > 0x1p35) return false;  // goes through a transposed copy of W there
-    library += library_time(kind, tokens, n_in, n_out[i], cus);
+    library += library_time(kind, tokens, n_in, n_out[i], cus, host);
   }
   return here <= 1.02 * library;  // (large tiles here take 2 to 5 % less than their estimate)
 }

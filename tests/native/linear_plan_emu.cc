@@ -38,6 +38,6 @@ extern "C" int emu_linear_joined(int, int64_t tokens, int64_t n_in, int count, c
 
 extern "C" double emu_linear_library(int kind, int64_t tokens, int64_t n_in, int count, const int64_t* n_out, int cus) {
   double time = 0;
-  for (int i = 0; i < count; ++i) time += library_time(kind, tokens, n_in, n_out[i], cus);
+  for (int i = 0; i < count; ++i) time += library_time(kind, tokens, n_in, n_out[i], cus, 20);
   return time;
 }

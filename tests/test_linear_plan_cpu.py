@@ -66,6 +66,15 @@ def test_input_gradients_one_after_the_other_are_priced_so(ask):
     (FORWARD, 32768, 2048, [5504, 5504], 1025, 1149),
     (INPUT_GRAD, 7000, 1280, [1280, 1280, 1280], 87, 117),
     (INPUT_GRAD, 10000, 1024, [2752, 2752], 105, 128),
+    (FORWARD, 16, 5504, [2048], 18.5, 21.1),
+    (FORWARD, 64, 5504, [2048], 18.3, 23.0),
+    (FORWARD, 512, 2752, [1024], 18.4, 20.1),
+    (FORWARD, 640, 2752, [1024], 18.4, 20.8),
+    (FORWARD, 16, 1024, [1024], 18.3, 9.7),
+    (FORWARD, 16, 2048, [512, 4096, 2048], 54.0, 15.5),
+    (FORWARD, 384, 2048, [5504, 5504], 39.3, 29.7),
+    (INPUT_GRAD, 384, 2752, [1024], 17.6, 10.2),
+    (INPUT_GRAD, 100, 2048, [512, 4096, 2048], 53.4, 46.3),
     (FORWARD, 1531, 4096, [11008, 11008], 261, 244),
     (FORWARD, 2100, 4096, [11008, 11008], 566, 335),
     (FORWARD, 4096, 4096, [11008, 11008], 800, 585),
