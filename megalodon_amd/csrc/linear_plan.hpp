@@ -178,14 +178,15 @@ inline double library_time(int kind, int64_t tokens, int64_t n_in, int64_t n_out
   const double products = static_cast<double>(tokens) * n_in * n_out;
   const double rate = kind == kInputGrad ? 1.1 : products > 0x1p39 ? 1.5 : products < 0x1p33 ? 1.0 : n_out % 1024 == 0 ? 1.4 : 1.1;
   const double mean = 2e-9 * products / rate + (kind == kInputGrad ? 10 : 8);
-  const int64_t cols = kind == kInputGrad ? n_in : n_out, k = kind == kInputGrad ? n_out : n_in;
-  const auto in_tiles = [&](int64_t m, int64_t n) {
-    const double tile = 1.2 / 64 * k * std::pow(m * n / 65536.0, 0.75) + 6;
-    const int64_t tiles = (tokens + m - 1) / m * ((cols + n - 1) / n), rounds = (tiles + cus - 1) / cus;
+  const int rows = static_cast<int>(tokens), cols = static_cast<int>(kind == kInputGrad ? n_in : n_out);
+  const double k = static_cast<double>(kind == kInputGrad ? n_out : n_in);
+  const auto in_tiles = [&](int m, int n) {
+    const double root = std::sqrt(m * n / 65536.0), tile = 1.2 / 64 * k * root * std::sqrt(root) + 6;  // (area to 3/4)
+    const int tiles = (rows + m - 1) / m * ((cols + n - 1) / n), rounds = (tiles + cus - 1) / cus;
     return (tiles % rounds == 0 ? static_cast<double>(rounds) : static_cast<double>(tiles) / cus + 1.3) * tile + 3;
   };
   double even = in_tiles(256, 256);
-  const bool fitted = (tokens + 255) / 256 * ((cols + 255) / 256) <= 2 * cus;
+  const bool fitted = (rows + 255) / 256 * ((cols + 255) / 256) <= 2 * cus;
   constexpr int kShapes[][2] = {{256, 192}, {256, 160}, {256, 128}, {192, 128}, {160, 128}, {128, 128}, {128, 64}, {64, 64}};
   for (int i = 0; fitted && i < 8; ++i) even = std::min({even, in_tiles(kShapes[i][0], kShapes[i][1]), in_tiles(kShapes[i][1], kShapes[i][0])});
   if (cols % 256 != 0) even *= fitted ? 1.2 : 1.1;
@@ -203,6 +204,8 @@ inline bool linear_takes(int kind, int64_t tokens, int64_t n_in, int count, cons
     // slower, all of 24000 tokens and more: 32768, 2560 x 6912 1290 / 1490.
     return true;
   }
+  for (int i = 0; kind == kInputGrad && i < count; ++i)
+    if (static_cast<double>(tokens) * n_in * n_out[i] > 0x1p35) return false;  // goes through a transposed copy of W there
   const double here = linear_time(kind, tokens, n_in, count, n_out, cus);
   // Of 3128 forward products and input gradients, alone and in groups (300 to 32768 tokens, layers of 512 to 13824, widths on and
   // off 256), this takes 806: 24 of them are more than 3 % slower than the library's calls (1.10 in the mean, the worst 1.35), the
@@ -213,11 +216,9 @@ inline bool linear_takes(int kind, int64_t tokens, int64_t n_in, int count, cons
   // estimate here, so it has to be ahead by as much (us, library / here: 16 tokens, 5504 -> 2048 18.5 / 21.1, 512 tokens, 2752 ->
   // 1024 18.4 / 20.1; 16 tokens, 1024 -> 1024 18.3 / 9.7); several take less (384 tokens, 2 x 5504 x 2048 39.3 / 29.7, estimate 38).
   const double host = count == 1 ? 17 : 20;
+  if (here <= 1.02 * host * count) return true;  // (nothing takes it less: spares the host its estimate, up to 1 us a call)
   double library = 0;
-  for (int i = 0; i < count; ++i) {
-    if (kind == kInputGrad && static_cast<double>(tokens) * n_in * n_out[i] > 0x1p35) return false;  // goes through a transposed copy of W there
-    library += library_time(kind, tokens, n_in, n_out[i], cus, host);
-  }
+  for (int i = 0; i < count; ++i) library += library_time(kind, tokens, n_in, n_out[i], cus, host);
   return here <= 1.02 * library;  // (large tiles here take 2 to 5 % less than their estimate)
 }
 
