@@ -201,7 +201,9 @@ inline bool linear_takes(int kind, int64_t tokens, int64_t n_in, int count, cons
     // library / here): 4096 tokens, 256 + 2048 + 1024 x 1024 91 / 30, 2 x 2752 x 1024 85 / 58, 2 x 5504 x 2048 174 / 166, 11008 x 4096
     // 380 / 281; 4084 tokens, 2048 x 5504 106 / 82; 1531, 4096 x 11008 174 / 122; 32768, 3328 x 1024 595 / 280, 1024 x 1024 198 / 72,
     // 512 x 512 152 / 41, 64 x 64 169 / 31.  Of 640 measured (300 to 32768 tokens, layers and groups of 768 to 13824) four are 3 to 16 %
-    // slower, all of 24000 tokens and more: 32768, 2560 x 6912 1290 / 1490.
+    // slower, all of 24000 tokens and more: 32768, 2560 x 6912 1290 / 1490.  Of 88 of 1 to 300 tokens (512 x 512 to 13824 x 5120; from
+    // 19 / 6, the library's host path, to 92 / 70) three are 4 to 15 % slower, matrices of 64 MB and more from 64 or 128 tokens: 64,
+    // 8192 x 4096 20 / 23.
     return true;
   }
   for (int i = 0; kind == kInputGrad && i < count; ++i)

@@ -1,9 +1,9 @@
-"""`nn.Linear` on the attention operator's product kernels where they are ahead of the library.
+"""`nn.Linear` on the attention operator's product kernels where they are expected to be ahead of the library GEMMs.
 
 With model-parallel world size 1 the reference's Column/RowParallelLinear are
-`F.linear` (megalodon/modules/model_parallel/layers.py:222-235,321-341).  Weight gradients, and
-forward products and input gradients of ordinary sizes, run on the library's own kernels, layers of one input in
-one launch; the other products are library GEMMs.  Those of `dx = dy @ W` with W (out, in) read along its rows are
+`F.linear` (megalodon/modules/model_parallel/layers.py:222-235,321-341).  Weight gradients, and the
+forward products and input gradients that an estimate by sizes (csrc/linear_plan.hpp) finds faster there, run on these kernels,
+layers of one input together; the other products are library GEMMs.  Those of `dx = dy @ W` with W (out, in) read along its rows are
 13-24 % faster on MI355X when both operands run along the reduction axis (`dy @ Wt^T` with Wt = W^T contiguous, the
 layout the forward `x @ W^T` uses), and the tiled transpose of W costs 5-30 us, so the backward makes that copy where the
 product is large enough to win it back.  The autograd nodes are C++ (csrc/host/ops.cpp).
