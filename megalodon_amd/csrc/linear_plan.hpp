@@ -145,13 +145,34 @@ inline bool joined_along_k(int64_t tokens, int64_t n_in, int count, const int64_
   plan(all, kInputGrad, 1, &n_in, cus, &small);
   return small;
 }
-// The time of a call, of all of its launches.
+// The time of a call, of all of its launches: the estimate that its tiles were chosen by, put right where that is known to be off.
+// - Forward, up to 128 tokens, weights of 64 MB and more: they are read at 5.4 TB/s, 0.65 of the estimate's time in the mean; above 200
+//   MB, which the memory-side cache no longer holds, only by tiles that are cut along k (three layers of 284 MB, uncut, 99 us).
+// - Forward, a layer alone that fills one round with tiles of 128: 0.30 us a slab where the estimate has 0.255 (1344 tokens, 2560 ->
+//   2752 31 us for 25).
+// - Input gradients one after the other: each onto the sum so far, read and written again (two layers of 512: 1226 tokens, 8192
+//   inputs, 46 us for 35; 19663 tokens, 512 inputs, 45 for 35).
 inline double linear_time(int kind, int64_t tokens, int64_t n_in, int count, const int64_t* n_out, int cus) {
-  bool apart;
-  if (kind != kInputGrad) return plan_group(linear_sizes(kind, tokens, n_in, count, n_out), kind, count, n_out, cus, &apart);
-  const int n = joined_along_k(tokens, n_in, count, n_out, cus) ? count : 1;
+  bool apart, small;
   double time = 0;
-  for (int i = 0; i < count; i += n) time += plan_group(linear_sizes(kind, tokens, n_in, n, n_out + i), kind, 1, &n_in, cus, &apart);
+  if (kind != kInputGrad) {
+    GemmParams q = linear_sizes(kind, tokens, n_in, count, n_out);
+    time = plan_group(q, kind, count, n_out, cus, &apart);
+    if (kind == kForward && tokens <= 128) {
+      double weights = 0;
+      for (int i = 0; i < count; ++i) weights += 2.0 * n_in * n_out[i];
+      if (weights > 200e6) plan(q, kind, count, n_out, cus, &small);
+      return weights >= 64e6 && (weights <= 200e6 || (!apart && q.cut > 0)) ? std::min(time, weights / 5.4e6 + 5) : time;
+    }
+    if (kind == kForward && count == 1) {
+      plan(q, kind, 1, n_out, cus, &small);
+      if (small && q.cut == 0 && q.mt_count > 2 && q.items <= cus) time *= 1.13;
+    }
+    return time;
+  }
+  const int n = joined_along_k(tokens, n_in, count, n_out, cus) ? count : 1;
+  for (int i = 0; i < count; i += n)
+    time += plan_group(linear_sizes(kind, tokens, n_in, n, n_out + i), kind, 1, &n_in, cus, &apart) + (i > 0 ? 2.0 * tokens * n_in / 2.2e6 : 0);
   return time;
 }
 
@@ -190,7 +211,7 @@ inline double library_time(int kind, int64_t tokens, int64_t n_in, int64_t n_out
   constexpr int kShapes[][2] = {{256, 192}, {256, 160}, {256, 128}, {192, 128}, {160, 128}, {128, 128}, {128, 64}, {64, 64}};
   for (int i = 0; fitted && i < 8; ++i) even = std::min({even, in_tiles(kShapes[i][0], kShapes[i][1]), in_tiles(kShapes[i][1], kShapes[i][0])});
   if (cols % 256 != 0) even *= fitted ? 1.2 : 1.1;
-  const double stream = kind == kForward && tokens <= 256 ? 2.0 * n_in * n_out / 3.3e6 + 3 : 0;
+  const double stream = kind == kForward && tokens <= 256 ? 2.0 * n_in * n_out / 5.9e6 + 1 : 0;  // (64 to 380 MB, 1 to 64 tokens)
   return std::max({host, stream, std::min(mean, even)});
 }
 
@@ -214,6 +235,8 @@ inline bool linear_takes(int kind, int64_t tokens, int64_t n_in, int count, cons
   // others 1.39 times as fast in the mean.  By the mean rate alone it took 1059, 193 of them slower (1.13 in the mean).  us, library /
   // here: 4096 tokens, 256 + 2048 + 1024 x 1024 60 / 33, 2 x 2752 x 1024 71 / 61, 2 x 5504 x 2048 181 / 165, 2 x 11008 x 4096 800 / 585;
   // left to the library: 2 x 11008 x 4096 of 1250 tokens 167 / 204, of 2500 317 / 374, of 5000 616 / 666.
+  // (After what linear_time puts right, of 11556 that it takes of 44454 drawn, 1 to 32768 tokens, 146 are more than 3 % slower, 1.09 in
+  // the mean, the worst 1.26; the time of all 0.52 of the library's in the mean.  Before, 1296 of 28872 were, the worst 1.62.)
   // Its host path is 18 us a call, more than many small products take.  A single layer of few tokens is up to 3 us above its
   // estimate here, so it has to be ahead by as much (us, library / here: 16 tokens, 5504 -> 2048 18.5 / 21.1, 512 tokens, 2752 ->
   // 1024 18.4 / 20.1; 16 tokens, 1024 -> 1024 18.3 / 9.7); several take less (384 tokens, 2 x 5504 x 2048 39.3 / 29.7, estimate 38).
