@@ -14,7 +14,9 @@
 // wavefront (lane = timestep) and obtains the carry of all earlier tiles by a
 // decoupled look-back over per-tile records in device memory (aggregate /
 // inclusive-prefix words published with relaxed device-scope atomics, two
-// floats per 64-bit word, all ones meaning "not written yet").  Groups of at
+// floats per 64-bit word, all ones meaning "not written yet").  How many
+// aggregates a tile merges before it meets an inclusive prefix depends on which
+// tiles are done, so the statistics' last bits may differ from run to run.  Groups of at
 // most 16 lanes per row (128 bf16 features) give every wavefront a tile of its
 // own in the forward pass, with no workgroup barrier after the ticket.
 // The tile is then normalised from registers:
