@@ -667,25 +667,23 @@ __global__ __launch_bounds__(kThreads, ONE ? 4 : 3) void cema_scan_fwd_kernel(
     wave_sync();
     // ---- scan over the chunks: a sub-segment per 16 lanes, the wave's four sub-segments are its
     //      own chunks; one workgroup barrier hands over the waves' ends ---------------------------
-    float* const col = sm.H + kHP + 2 * sn;  // state column n of row 1 + c
+    //      (chunks behind the row's end need no mask: their X is zero, so their S is, and nothing takes
+    //      up a state behind them; what a wave without a tile passes on nobody reads)
+    float* const col = sm.H + (1 + sa * CPS) * kHP + 2 * sn;  // state column n of the sub-segment's rows
     float2 sv[CPS];                          // the sub-segment's local states, kept for the second pass
     cf h{0.f, 0.f};
     if (runs) {
 #pragma unroll
-      for (int i = 0; i < CPS; ++i) {
-        const int c = sa * CPS + i;
-        const float2 s0 = *reinterpret_cast<const float2*>(col + c * kHP);  // read, then masked
-        sv[i] = sl * CPS + i < w.nc ? s0 : make_float2(0.f, 0.f);
-      }
+      for (int i = 0; i < CPS; ++i) sv[i] = *reinterpret_cast<const float2*>(col + i * kHP);
 #pragma unroll
-      for (int i = 0; i < CPS; ++i) h = cadd(cmul(qT, h), cf{sv[i].x, sv[i].y});
+      for (int i = 0; i < CPS; ++i) h = cfma(qT, h, cf{sv[i].x, sv[i].y});
       if (sl < 3) sm.sub_end[3 * wave + sl][sn] = h;
       wave_sync();
       if (sl == 3) {
         cf e = sm.sub_end[3 * wave][sn];
-        e = cadd(cmul(qS, e), sm.sub_end[3 * wave + 1][sn]);
-        e = cadd(cmul(qS, e), sm.sub_end[3 * wave + 2][sn]);
-        sm.wave_end[par][wave][sn] = cadd(cmul(qS, e), h);
+        e = cfma(qS, e, sm.sub_end[3 * wave + 1][sn]);
+        e = cfma(qS, e, sm.sub_end[3 * wave + 2][sn]);
+        sm.wave_end[par][wave][sn] = cfma(qS, e, h);
       }
     }
     lds_barrier();
@@ -697,20 +695,19 @@ __global__ __launch_bounds__(kThreads, ONE ? 4 : 3) void cema_scan_fwd_kernel(
       if (k <= wave) cin = h0 != nullptr && w.nc > 0 && sn < N ? h0[w.row * N + sn] : cf{0.f, 0.f};
 #pragma unroll
       for (int v = 0; v < kWaves - 1; ++v)
-        if (v >= from && v < wave) cin = cadd(cmul(qW, cin), sm.wave_end[par][v][sn]);
-      if (!ONE && sa == kSubs - 1) sm.carry[cur ^ 1][sn] = cadd(cmul(qW, cin), sm.wave_end[par][kWaves - 1][sn]);
+        if (v >= from && v < wave) cin = cfma(qW, cin, sm.wave_end[par][v][sn]);
+      if (!ONE && sa == kSubs - 1) sm.carry[cur ^ 1][sn] = cfma(qW, cin, sm.wave_end[par][kWaves - 1][sn]);
       if (sl == 0) *reinterpret_cast<float2*>(sm.wave_cin[wave] + 2 * sn) = make_float2(cin.x, cin.y);
 #pragma unroll
       for (int s = 0; s < 3; ++s) {
         const cf e = sm.sub_end[3 * wave + s][sn];
-        if (s < sl) cin = cadd(cmul(qS, cin), e);
+        if (s < sl) cin = cfma(qS, cin, e);
       }
       h = cin;
 #pragma unroll
       for (int i = 0; i < CPS; ++i) {
-        const int c = sa * CPS + i;
-        h = cadd(cmul(qT, h), cf{sv[i].x, sv[i].y});
-        if (sl * CPS + i < w.nc) *reinterpret_cast<float2*>(col + c * kHP) = make_float2(h.x, h.y);
+        h = cfma(qT, h, cf{sv[i].x, sv[i].y});
+        *reinterpret_cast<float2*>(col + i * kHP) = make_float2(h.x, h.y);
       }
     }
     wave_sync();
@@ -888,13 +885,15 @@ int launch_fwd(const void* x, void* y, const Coeffs& co, const cf* h0, cf* h_las
 // fftconv.py:53-75) are dp = Re(A gamma), dq = conj(B p gamma), dgamma = conj(A p),
 // domega = sum dy x, and dx[s] = sum_{t >= s} k[t-s] dy[t] + omega dy[s].  By chunks, in
 // reverse time (DY[c][i] = dy[64 c + i], XR[c][j'] = x[64 c + 63 - j']):
-//   (G, G')[c]   = Pg DY[c],     Pg = rows (Re, Im)(q^i), then (Re, Im)(i q^(i-1)), i < 64
-//   R[c]  = G[c] + q^64 R[c+1],   R'[c] = G'[c] + 64 q^63 R[c+1] + q^64 R'[c+1]      (scan)
+//   (G, G')[c]   = Pg DY[c],     Pg = rows (Re, Im)(q^i), then (Re, Im)(i / 64 q^i), i < 64
+//   R[c]  = G[c] + q^64 R[c+1],   R'[c] = G'[c] + q^64 (R[c+1] + R'[c+1])            (scan)
 //   (X, X')[c]   = Pg XR[c]
 //   W  = sum_c X[c] R[c+1],   W' = sum_c (X'[c] R[c+1] + X[c] R'[c+1])
 //   DX[c] = K^T DY[c] + Qd R[c+1],   Qd[j][m] = (Re, -Im)(c_n q_n^(64-j)),  omega on the diagonal of K
 //   M     = sum_c DY[c]^T X[c]   (64 x 64, rows i >= columns j), dkin[l] = sum_j M[j+l][j]
-//   A = sum_l q^l dkin[l] + q W,   B = sum_l l q^(l-1) dkin[l] + W + q W'
+//   A = sum_l q^l dkin[l] + q W,   B = sum_l l q^(l-1) dkin[l] + W + 64 W'
+// Primed states are derivatives by q times q / 64, so that a step over n chunks multiplies both by one power,
+// R' <- G' + q^(64 n) (R' + n R): ten operations a chunk, mode and pass instead of eighteen.
 // Segments of 128 chunks are taken from the end of the row to its start; a
 // wave holds one chunk tile of the segment.  The chunk-contracted product M
 // needs operands with chunks along k: the wave parks its DY and X tiles in a
@@ -922,7 +921,7 @@ struct BwdSmem {
   float R[kBwdNC * kRP];
   float pn[16];
   cf gn[16];
-  cf pw[14][16];                         // powers evaluated directly (see setup_row)
+  cf pw[12][16];                         // powers evaluated directly (see setup_row)
   cf sub_end[kSubs][2][16];              // local (R, R') at the start of each sub-segment
   cf wave_end[2][kWaves][2][16];         // the same for each wave's four sub-segments, by item parity
   float wave_cin[kWaves][64];            // (R, R') behind each wave's last chunk
@@ -947,12 +946,12 @@ static_assert(sizeof(cf) * 16 * (kT + 2) + sizeof(u32x4) * 4 * kWave + sizeof(fl
               "the third pieces of the second kind pass through the state buffer, behind the power table, k behind them");
 static_assert(sizeof(BwdSmemFine) <= 80 * 1024, "two workgroups per compute unit");
 
-// (h, h') <- (g, g') + [[m, 0], [md, m]] (h, h'): one step of the reverse scan, over a chunk
-// (m = q^64, md = 64 q^63), a sub-segment or a wave's chunks (the same form with larger powers)
-__device__ __forceinline__ void rstep(cf& h, cf& hd, cf g, cf gd, cf m, cf md) {
-  const cf nd = cadd(gd, cadd(cmul(md, h), cmul(m, hd)));
-  h = cadd(g, cmul(m, h));
-  hd = nd;
+// (h, h') <- (g, g') + m (h, h' + n h): the reverse scan's step over n chunks (m = q^(64 n)): one, a
+// sub-segment or a wave's
+__device__ __forceinline__ void rstep(cf& h, cf& hd, cf g, cf gd, cf m, float n) {
+  const cf t{fmaf(n, h.x, hd.x), fmaf(n, h.y, hd.y)};
+  h = cfma(m, h, g);
+  hd = cfma(m, t, gd);
 }
 
 // DX32: dx is written in float32 (or, with a null pointer, not at all) instead of the rows'
@@ -1027,7 +1026,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
   };
 
   // scan multipliers of this thread's mode: over a chunk, a sub-segment, a wave's chunks
-  cf qT{0.f, 0.f}, qTd{0.f, 0.f}, q1{0.f, 0.f};
+  cf qT{0.f, 0.f}, q1{0.f, 0.f};
   int cur = 0, par = 0;
   RowParams rp = fetch_params(blockIdx.x);
 
@@ -1038,17 +1037,17 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
 
   auto setup_row = [&](int group) {
     MEGA_LANE_IDS;
-    // powers evaluated directly (phase reduced in float64), 14 per mode: q^(4 k), q^(16 k)
-    // (k < 4), q, q^64, q^(64 CPS), q^(64 CPS - 1), q^(256 CPS), q^(256 CPS - 1)
+    // powers evaluated directly (phase reduced in float64), 12 per mode: q^(4 k), q^(16 k)
+    // (k < 4), q, q^64, q^(64 CPS), q^(256 CPS)
     cf direct{0.f, 0.f};
-    if (tid < 14 * 16 && sn < N) {
+    if (tid < 12 * 16 && sn < N) {
       const int k = tid >> 4;
-      const int tab[6] = {1, kT, kT * CPS, kT * CPS - 1, 4 * kT * CPS, 4 * kT * CPS - 1};
+      const int tab[4] = {1, kT, kT * CPS, 4 * kT * CPS};
       const int e = k < 4 ? 4 * k : (k < 8 ? 16 * (k - 4) : tab[k - 8]);
       direct = qpow(rp.lq.x, rp.lq.y, e);
     }
     __syncthreads();  // every wave is done with the previous row's tables and reductions
-    if (tid < 14 * 16) sm.pw[tid >> 4][sn] = direct;
+    if (tid < 12 * 16) sm.pw[tid >> 4][sn] = direct;
     if (tid < 16) {
       sm.pn[tid] = rp.pv;
       sm.gn[tid] = rp.gv;
@@ -1072,8 +1071,6 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       qT = sm.pw[9][sn];
     }
     __syncthreads();
-    // 64 q^63
-    qTd = cf{kT * qp[sn][kT - 1].x, kT * qp[sn][kT - 1].y};
     for (int item = tid; item < kBwdBlocks * kWave; item += kThreads) {
       const int blk = item >> 6, ln = item & 63, rr = ln & 31, gg = ln >> 5;
       float v[8];
@@ -1082,8 +1079,8 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const int i = 16 * s + 8 * gg + e;
-          const cf w = qp[n][kind ? (i > 0 ? i - 1 : 0) : i];
-          const float sc = kind ? static_cast<float>(i) : 1.f;
+          const cf w = qp[n][i];
+          const float sc = kind ? static_cast<float>(i) / kT : 1.f;
           v[e] = sc * (part ? w.y : w.x);
         }
       } else if (blk < 12) {
@@ -1240,7 +1237,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       }
       const cf qq = sm.pw[8][n];
       const cf A = cadd(ain, cmul(qq, w));
-      const cf Bq = cadd(cadd(bin, w), cmul(qq, wd));
+      const cf Bq{fmaf(kT, wd.x, bin.x + w.x), fmaf(kT, wd.y, bin.y + w.y)};
       const cf gm = sm.gn[n];
       const float pp = sm.pn[n];
       dp[row * N + n] = A.x * gm.x - A.y * gm.y;
@@ -1250,13 +1247,14 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
         // A carried state h0 adds b[t] = Re(gamma q^(t+1) h0) to the output (ema_parameters.cc:56-77).
         // With R0 = sum_t dy[t] q^t and R0' = dR0 / dq -- what the reverse scan has carried to the
         // start of the row -- its gradients are (ema_parameters.cc:158-188, PyTorch's convention)
-        //   dgamma += conj(q h0 R0),  dq += conj(gamma h0 (R0 + q R0')),  dh0 = conj(gamma q R0).
+        //   dgamma += conj(q h0 R0),  dq += conj(gamma h0 (R0 + q R0')),  dh0 = conj(gamma q R0)
+        // (q R0' = 64 times what the scan has carried).
         const cf r0 = sm.carry[cur][0][n], r0d = sm.carry[cur][1][n];
         const cf h = h0[row * N + n];
         const cf e1 = cmul(cmul(qq, h), r0);
         dgv.x += e1.x;
         dgv.y -= e1.y;
-        const cf e2 = cmul(cmul(gm, h), cadd(r0, cmul(qq, r0d)));
+        const cf e2 = cmul(cmul(gm, h), cf{fmaf(kT, r0d.x, r0.x), fmaf(kT, r0d.y, r0.y)});
         dqv.x += e2.x;
         dqv.y -= e2.y;
         if (dh0 != nullptr) {
@@ -1364,38 +1362,38 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
     load_dy(next);
     // ---- reverse scan over the chunks of the segment; a wave's four sub-segments are its own
     //      chunks, one workgroup barrier hands over the waves' ends ---------------------------------
-    {
-      float* col = sm.R + 2 * sn;
-      float2 gv[CPS], gd[CPS];
+    //      (a wave whose tile has no steps passes on zeros: it may be its row's last, kShifted.  Chunks behind the
+    //      row's end need no mask: their DY is zero, so their G is, and the scan starts from zero behind them)
+    float* const col = sm.R + sa * CPS * kRP + 2 * sn;
+    float2 gv[CPS], gd[CPS];
+    const cf qS = sm.pw[10][sn], qW = sm.pw[11][sn];  // over a sub-segment, over a wave's chunks
+    if (on) {
 #pragma unroll
       for (int i = 0; i < CPS; ++i) {
-        const int c = sa * CPS + i;
-        const bool live = sl * CPS + i < w.nc;
-        const float2 a0 = *reinterpret_cast<const float2*>(col + c * kRP);
-        const float2 b0 = *reinterpret_cast<const float2*>(col + c * kRP + 32);
-        gv[i] = live ? a0 : make_float2(0.f, 0.f);
-        gd[i] = live ? b0 : make_float2(0.f, 0.f);
+        gv[i] = *reinterpret_cast<const float2*>(col + i * kRP);
+        gd[i] = *reinterpret_cast<const float2*>(col + i * kRP + 32);
       }
       cf e{0.f, 0.f}, ed{0.f, 0.f};
 #pragma unroll
-      for (int i = CPS - 1; i >= 0; --i) rstep(e, ed, cf{gv[i].x, gv[i].y}, cf{gd[i].x, gd[i].y}, qT, qTd);
+      for (int i = CPS - 1; i >= 0; --i) rstep(e, ed, cf{gv[i].x, gv[i].y}, cf{gd[i].x, gd[i].y}, qT, 1.f);
       sm.sub_end[sa][0][sn] = e;
       sm.sub_end[sa][1][sn] = ed;
       wave_sync();
-      // multipliers over a sub-segment and over a wave's chunks
-      const cf qS = sm.pw[10][sn], qW = sm.pw[12][sn];
-      const cf qSd{(kT * CPS) * sm.pw[11][sn].x, (kT * CPS) * sm.pw[11][sn].y};
-      const cf qWd{(4 * kT * CPS) * sm.pw[13][sn].x, (4 * kT * CPS) * sm.pw[13][sn].y};
       if (sl == 0) {
         // the wave's chunks from zero: sub-segments 3, 2, 1, then this one
         cf h = sm.sub_end[sa + 3][0][sn], hd = sm.sub_end[sa + 3][1][sn];
-        rstep(h, hd, sm.sub_end[sa + 2][0][sn], sm.sub_end[sa + 2][1][sn], qS, qSd);
-        rstep(h, hd, sm.sub_end[sa + 1][0][sn], sm.sub_end[sa + 1][1][sn], qS, qSd);
-        rstep(h, hd, e, ed, qS, qSd);
+        rstep(h, hd, sm.sub_end[sa + 2][0][sn], sm.sub_end[sa + 2][1][sn], qS, CPS);
+        rstep(h, hd, sm.sub_end[sa + 1][0][sn], sm.sub_end[sa + 1][1][sn], qS, CPS);
+        rstep(h, hd, e, ed, qS, CPS);
         sm.wave_end[par][wave][0][sn] = h;
         sm.wave_end[par][wave][1][sn] = hd;
       }
-      lds_barrier();
+    } else if (sl == 0) {
+      sm.wave_end[par][wave][0][sn] = cf{0.f, 0.f};
+      sm.wave_end[par][wave][1][sn] = cf{0.f, 0.f};
+    }
+    lds_barrier();
+    {
       cf h = sm.carry[cur][0][sn], hd = sm.carry[cur][1][sn];
       // through the tiles behind this wave's, from the last one of its row if that is among the four
       // (nothing comes from behind it)
@@ -1403,11 +1401,11 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       if (wave + k < kWaves) h = hd = cf{0.f, 0.f};
 #pragma unroll
       for (int v = kWaves - 1; v >= 1; --v)
-        if (v > wave && v <= from) rstep(h, hd, sm.wave_end[par][v][0][sn], sm.wave_end[par][v][1][sn], qW, qWd);
+        if (v > wave && v <= from) rstep(h, hd, sm.wave_end[par][v][0][sn], sm.wave_end[par][v][1][sn], qW, 4.f * CPS);
       if (sa == 0) {
         // through wave 0's chunks too: the state at the start of the segment, the next item's carry
         cf ch = h, chd = hd;
-        rstep(ch, chd, sm.wave_end[par][0][0][sn], sm.wave_end[par][0][1][sn], qW, qWd);
+        rstep(ch, chd, sm.wave_end[par][0][0][sn], sm.wave_end[par][0][1][sn], qW, 4.f * CPS);
         sm.carry[cur ^ 1][0][sn] = ch;
         sm.carry[cur ^ 1][1][sn] = chd;
       }
@@ -1415,28 +1413,25 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
         *reinterpret_cast<float2*>(sm.wave_cin[wave] + 2 * sn) = make_float2(h.x, h.y);
         *reinterpret_cast<float2*>(sm.wave_cin[wave] + 32 + 2 * sn) = make_float2(hd.x, hd.y);
       }
+      if (on) {
 #pragma unroll
-      for (int s = 3; s >= 1; --s) {
-        const cf se = sm.sub_end[4 * wave + s][0][sn], sed = sm.sub_end[4 * wave + s][1][sn];
-        if (s > sl) rstep(h, hd, se, sed, qS, qSd);
-      }
+        for (int s = 3; s >= 1; --s) {
+          const cf se = sm.sub_end[4 * wave + s][0][sn], sed = sm.sub_end[4 * wave + s][1][sn];
+          if (s > sl) rstep(h, hd, se, sed, qS, CPS);
+        }
 #pragma unroll
-      for (int i = CPS - 1; i >= 0; --i) {
-        const int c = sa * CPS + i;
-        rstep(h, hd, cf{gv[i].x, gv[i].y}, cf{gd[i].x, gd[i].y}, qT, qTd);
-        if (sl * CPS + i < w.nc) {
-          *reinterpret_cast<float2*>(col + c * kRP) = make_float2(h.x, h.y);
-          *reinterpret_cast<float2*>(col + c * kRP + 32) = make_float2(hd.x, hd.y);
+        for (int i = CPS - 1; i >= 0; --i) {
+          rstep(h, hd, cf{gv[i].x, gv[i].y}, cf{gd[i].x, gd[i].y}, qT, 1.f);
+          *reinterpret_cast<float2*>(col + i * kRP) = make_float2(h.x, h.y);
+          *reinterpret_cast<float2*>(col + i * kRP + 32) = make_float2(hd.x, hd.y);
         }
       }
     }
     wave_sync();
     if (on) {
       // (R, R')[c + 1]: the next row of the buffer, or, for the wave's last chunk, wave_cin;
-      // chunks past the end of the row have X = 0 and DY = 0, their rows may hold anything
-      const bool live = r < w.nc;
+      // behind the row's end R is zero
       const float* rnext = (r == 31) ? sm.wave_cin[wave] : myrows + (r + 1) * kRP;
-      const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
       // the stores of dX go out first: they have the (X, X') products and the next item's
       // staging to retire under before the next loads are issued behind them
       // ---- DX = K^T DY + Qd R[c+1] (omega dy included: K carries omega on its diagonal) -------------
@@ -1446,9 +1441,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
         const float* src = rnext + 16 * s2 + 8 * g;
         const float4 u0 = *reinterpret_cast<const float4*>(src);
         const float4 u1 = *reinterpret_cast<const float4*>(src + 4);
-        const float4 ua = live ? u0 : zero4;
-        const float4 ub = live ? u1 : zero4;
-        const float v[8] = {ua.x, ua.y, ua.z, ua.w, ub.x, ub.y, ub.z, ub.w};
+        const float v[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
         split8(v, hb[s2][0], hb[s2][1]);
       }
 #pragma unroll
@@ -1515,20 +1508,16 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
         }
 #pragma unroll
         for (int qd = 0; qd < 4; ++qd) {
-          // loaded whatever the row holds, then masked: a conditional load is split into
-          // single-word reads under an execution mask
-          const float4 rv0 = *reinterpret_cast<const float4*>(rnext + 4 * g + 8 * qd);
-          const float4 rd0 = *reinterpret_cast<const float4*>(rnext + 32 + 4 * g + 8 * qd);
-          const float4 rv = live ? rv0 : zero4;
-          const float4 rd = live ? rd0 : zero4;
+          const float4 rv = *reinterpret_cast<const float4*>(rnext + 4 * g + 8 * qd);
+          const float4 rd = *reinterpret_cast<const float4*>(rnext + 32 + 4 * g + 8 * qd);
 #pragma unroll
           for (int b = 0; b < 2; ++b) {
             const cf xv{xacc[0][4 * qd + 2 * b], xacc[0][4 * qd + 2 * b + 1]};
             const cf xd{xacc[1][4 * qd + 2 * b], xacc[1][4 * qd + 2 * b + 1]};
             const cf rr_ = b ? cf{rv.z, rv.w} : cf{rv.x, rv.y};
             const cf rdd = b ? cf{rd.z, rd.w} : cf{rd.x, rd.y};
-            wacc[2 * qd + b] = cadd(wacc[2 * qd + b], cmul(xv, rr_));
-            wdacc[2 * qd + b] = cadd(wdacc[2 * qd + b], cadd(cmul(xd, rr_), cmul(xv, rdd)));
+            wacc[2 * qd + b] = cfma(xv, rr_, wacc[2 * qd + b]);
+            wdacc[2 * qd + b] = cfma(xv, rdd, cfma(xd, rr_, wdacc[2 * qd + b]));
           }
         }
       }

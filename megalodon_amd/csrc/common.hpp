@@ -118,6 +118,10 @@ __device__ __forceinline__ cf cmulc(cf a, cf b) {  // a * conj(b)
   return {a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y};
 }
 __device__ __forceinline__ cf cadd(cf a, cf b) { return {a.x + b.x, a.y + b.y}; }
+// c + a b in four fused operations (a sum of products is not contracted by itself: six)
+__device__ __forceinline__ cf cfma(cf a, cf b, cf c) {
+  return {fmaf(-a.y, b.y, fmaf(a.x, b.x, c.x)), fmaf(a.y, b.x, fmaf(a.x, b.y, c.y))};
+}
 __device__ __forceinline__ cf csub(cf a, cf b) { return {a.x - b.x, a.y - b.y}; }
 
 // ---- DPP row reductions --------------------------------------------------------
