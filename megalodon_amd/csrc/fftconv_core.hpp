@@ -21,12 +21,14 @@
 // Engine.  One workgroup of T = M/32 lanes transforms one M-point half with 32
 // complex points per lane in registers: M = 32 * 32 * R3 (R3 = M/1024 in
 // {2,4,8,16}); pass 1 radix-32 over the top digit, LDS exchange, pass 2
-// radix-32, LDS exchange, pass 3 radix-R3 (32/R3 butterflies per lane).  The
+// radix-32, LDS exchange, pass 3 radix-R3 (32/R3 butterflies per lane).  All are
+// decimation in time: a pass takes its inputs' twiddles into its butterflies, six
+// fused operations each, where twiddles of its own between the passes had to be
+// formed (136 operations) and multiplied in (124) beside butterflies of four to eight.  The
 // residues handled by one lane in pass 3 are chosen in conjugate pairs
 // (c, 1024-c) / (c, 1023-c), so both Z[r] and Z[N-r] of every bin sit in the
 // same lane and the pointwise stage needs no further exchange.  The inverse is
-// the mirror image (decimation-in-time first pass, then the same radix-32
-// passes on swapped re/im).
+// the mirror image, the same transforms on swapped re/im.
 #pragma once
 
 #include <stdint.h>
@@ -72,10 +74,9 @@ constexpr int bitrev(int x) {
 }
 constexpr int ilog2(int x) { return x <= 1 ? 0 : 1 + ilog2(x >> 1); }
 
-// v *= W_R^i with W_R = exp(-2 pi i / R), i < R/2 ... general k in [0, R)
+// v *= W_R^k with W_R = exp(-2 pi i / R), k in [0, R) known at compile time after unrolling
 template <int R>
 MEGA_HD void mul_w(float& xr, float& xi, int k) {
-  // callers pass compile-time k after unrolling
   const int q = (k * (64 / R)) & 63;
   const float c = kC64[q], s = kS64[q];  // W = c - i s
   const float r = xr * c + xi * s;
@@ -84,46 +85,104 @@ MEGA_HD void mul_w(float& xr, float& xi, int k) {
   xi = i;
 }
 
-// In-place radix-2 decimation-in-frequency DFT (kernel exp(-2 pi i nk/R)) over
-// v[0], v[S], ..., v[(R-1)S]; output index k ends at position bitrev(k)*S.
-template <int R, int S>
-MEGA_HD void dif(float* re, float* im) {
-  if constexpr (R > 1) {
-    constexpr int H = R / 2;
+MEGA_HD float fma1(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+MEGA_HD c32 cmulv(c32 a, c32 b) { return c32{fma1(-a.y, b.y, a.x * b.x), fma1(a.y, b.x, a.x * b.y)}; }
+MEGA_HD c32 csqv(c32 a) { return c32{fma1(-a.y, a.y, a.x * a.x), (a.x + a.x) * a.y}; }
+
+// (a, b) <- (a + w b, a - w b): the sum in four fused operations, the difference as 2 a - sum in two.  With the
+// twiddle in front of the butterfly its product costs no instruction of its own; behind it (decimation in
+// frequency) a butterfly and its twiddle are eight.
+MEGA_HD void butterfly(float& ar, float& ai, float& br, float& bi, c32 w) {
+  const float tr = fma1(-bi, w.y, fma1(br, w.x, ar)), ti = fma1(bi, w.x, fma1(br, w.y, ai));
+  br = fma1(2.f, ar, -tr);
+  bi = fma1(2.f, ai, -ti);
+  ar = tr;
+  ai = ti;
+}
+// the same with w = 1 and w = -i
+MEGA_HD void butterfly1(float& ar, float& ai, float& br, float& bi) {
+  const float r = br, i = bi;
+  br = ar - r;
+  bi = ai - i;
+  ar += r;
+  ai += i;
+}
+MEGA_HD void butterfly_mi(float& ar, float& ai, float& br, float& bi) {
+  const float r = br, i = bi;
+  br = ar - i;
+  bi = ai + r;
+  ar += i;
+  ai -= r;
+}
+
+// Stage R of a transform of N natural-order inputs v[j] with a twiddle of its own on each, v[j] w^j: butterflies of blocks
+// of R outputs, w here the power N / R of that twiddle.  After the last stage, R = N, output k stands at position
+// bitrev(k).  The twiddles of a stage are w times roots of unity, two butterflies to a product (its quarter turn is free).
+template <int N, int R>
+MEGA_HD void stage_w(float* re, float* im, c32 w) {
+  constexpr int S = N / R, B = ilog2(R) - 1, Q = R >= 4 ? R / 4 : 1;
 #pragma unroll
-    for (int i = 0; i < H; ++i) {
-      const float ar = re[i * S], ai = im[i * S];
-      const float br = re[(i + H) * S], bi = im[(i + H) * S];
-      re[i * S] = ar + br;
-      im[i * S] = ai + bi;
-      const float dr = ar - br, di = ai - bi;
-      float orr, oi;
-      if (i == 0) {
-        orr = dr;
-        oi = di;
-      } else if (4 * i == R) {  // -i
-        orr = di;
-        oi = -dr;
-      } else if (8 * i == R) {  // (1 - i)/sqrt2
-        orr = (dr + di) * kRsqrt2;
-        oi = (di - dr) * kRsqrt2;
-      } else if (8 * i == 3 * R) {  // (-1 - i)/sqrt2
-        orr = (di - dr) * kRsqrt2;
-        oi = -(dr + di) * kRsqrt2;
-      } else {
-        orr = dr;
-        oi = di;
-        mul_w<R>(orr, oi, i);
+  for (int i = 0; i < Q; ++i) {
+    c32 t = w;
+    if (i > 0) mul_w<R>(t.x, t.y, i);
+#pragma unroll
+    for (int b = 0; b < S; ++b) {
+      const int p = b + 2 * S * bitrev<B>(i);
+      butterfly(re[p], im[p], re[p + S], im[p + S], t);
+      if (R >= 4) {
+        const int q = b + 2 * S * bitrev<B>(i + R / 4);
+        butterfly(re[q], im[q], re[q + S], im[q + S], c32{t.y, -t.x});
       }
-      re[(i + H) * S] = orr;
-      im[(i + H) * S] = oi;
     }
-    dif<H, S>(re, im);
-    dif<H, S>(re + H * S, im + H * S);
+  }
+}
+// ... with w = W_X^(N / R), known at compile time (X = 0: w = 1)
+template <int N, int R, int X = 0>
+MEGA_HD void stage(float* re, float* im) {
+  constexpr int S = N / R, B = ilog2(R) - 1;
+#pragma unroll
+  for (int i = 0; i < R / 2; ++i) {
+    const int turn = i * (64 / R) + (X ? S * (64 / (X ? X : 64)) : 0);  // in 64ths, below 32
+#pragma unroll
+    for (int b = 0; b < S; ++b) {
+      const int p = b + 2 * S * bitrev<B>(i);
+      if (turn == 0) butterfly1(re[p], im[p], re[p + S], im[p + S]);
+      else if (turn == 16) butterfly_mi(re[p], im[p], re[p + S], im[p + S]);
+      else butterfly(re[p], im[p], re[p + S], im[p + S], c32{kC64[turn], -kS64[turn]});
+    }
+  }
+}
+// sum_j v[j] W_N^(j k), or with X sum_j v[j] W_X^j W_N^(j k): output k at position bitrev(k)
+template <int N, int X = 0>
+MEGA_HD void transform(float* re, float* im) {
+  stage<N, 2, X>(re, im);
+  if constexpr (N >= 4) stage<N, 4, X>(re, im);
+  if constexpr (N >= 8) stage<N, 8, X>(re, im);
+  if constexpr (N >= 16) stage<N, 16, X>(re, im);
+  if constexpr (N >= 32) stage<N, 32, X>(re, im);
+}
+// sum_j v[j] w^j W_N^(j k), N <= 16, from w alone
+template <int N>
+MEGA_HD void transform_w(float* re, float* im, c32 w) {
+  const c32 w2 = csqv(w), w4 = csqv(w2), w8 = csqv(w4);
+  if constexpr (N == 2) {
+    stage_w<N, 2>(re, im, w);
+  } else if constexpr (N == 4) {
+    stage_w<N, 2>(re, im, w2);
+    stage_w<N, 4>(re, im, w);
+  } else if constexpr (N == 8) {
+    stage_w<N, 2>(re, im, w4);
+    stage_w<N, 4>(re, im, w2);
+    stage_w<N, 8>(re, im, w);
+  } else {
+    stage_w<N, 2>(re, im, w8);
+    stage_w<N, 4>(re, im, w4);
+    stage_w<N, 8>(re, im, w2);
+    stage_w<N, 16>(re, im, w);
   }
 }
 
-// Transpose of dif: input index k at position bitrev(k)*S, output natural order.
+// The same sums for inputs that stand at bitrev(j) * S: output k at position k * S.
 template <int R, int S>
 MEGA_HD void dit(float* re, float* im) {
   if constexpr (R > 1) {
@@ -132,73 +191,51 @@ MEGA_HD void dit(float* re, float* im) {
     dit<H, S>(re + H * S, im + H * S);
 #pragma unroll
     for (int i = 0; i < H; ++i) {
-      const float ar = re[i * S], ai = im[i * S];
-      float br = re[(i + H) * S], bi = im[(i + H) * S];
-      if (i == 0) {
-      } else if (4 * i == R) {
-        const float t = br;
-        br = bi;
-        bi = -t;
-      } else if (8 * i == R) {
-        const float t = (br + bi) * kRsqrt2;
-        bi = (bi - br) * kRsqrt2;
-        br = t;
-      } else if (8 * i == 3 * R) {
-        const float t = (bi - br) * kRsqrt2;
-        bi = -(br + bi) * kRsqrt2;
-        br = t;
-      } else {
-        mul_w<R>(br, bi, i);
-      }
-      re[i * S] = ar + br;
-      im[i * S] = ai + bi;
-      re[(i + H) * S] = ar - br;
-      im[(i + H) * S] = ai - bi;
+      float *ar = re + i * S, *ai = im + i * S, *br = ar + H * S, *bi = ai + H * S;
+      if (i == 0) butterfly1(*ar, *ai, *br, *bi);
+      else if (4 * i == R) butterfly_mi(*ar, *ai, *br, *bi);
+      else butterfly(*ar, *ai, *br, *bi, c32{kC64[i * (64 / R)], -kS64[i * (64 / R)]});
     }
   }
 }
 
-// V[a] = sum_n v[n] W_64^(n (2a+1)), n, a < 32 (odd bins of a 64-point DFT of
-// v padded with zeros).  Natural input; V[a] ends at position bitrev5(a).
-MEGA_HD void shifted_dif32(float* re, float* im) {
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const float ar = re[i], ai = im[i], br = re[i + 16], bi = im[i + 16];
-    // g = W_64^i (a - i b), h = W_64^(3i) (a + i b)
-    float gr = ar + bi, gi = ai - br;
-    float hr = ar - bi, hi = ai + br;
-    if (i != 0) {
-      mul_w<64>(gr, gi, i);
-      mul_w<64>(hr, hi, 3 * i);
-    }
-    re[i] = gr;
-    im[i] = gi;
-    re[i + 16] = hr;
-    im[i + 16] = hi;
-  }
-  dif<16, 1>(re, im);
-  dif<16, 1>(re + 16, im + 16);
+// The transform of 32 with a lane's own twiddle, sum_j v[j] w^j W_32^(j k), from w, w^4 and w^16.
+struct Powers {
+  c32 w1, w4, w16;
+};
+MEGA_HD void transform32_w(float* re, float* im, const Powers& w) {
+  stage_w<32, 2>(re, im, w.w16);
+  stage_w<32, 4>(re, im, csqv(w.w4));
+  stage_w<32, 8>(re, im, w.w4);
+  stage_w<32, 16>(re, im, csqv(w.w1));
+  stage_w<32, 32>(re, im, w.w1);
 }
-
-// P[n] = sum_a u[a] W_64^((2a+1) n), the transpose of shifted_dif32.  Natural
-// input; P[n] ends at position 2*bitrev4(n) for n < 16 and 1 + 2*bitrev4(n-16)
+// ... and over odd frequencies, P[n] = sum_a u[a] z_n^(2a+1) with z_n = z W_64^n and w = z^2: even and odd a apart, P[n] = z_n E +
+// z_n^3 O and P[n + 16] = -i (z_n E - z_n^3 O).  P[n] ends at position 2*bitrev4(n) for n < 16 and 1 + 2*bitrev4(n-16)
 // otherwise.
-MEGA_HD void shifted_dit32(float* re, float* im) {
-  dif<16, 2>(re, im);          // G over even a
-  dif<16, 2>(re + 1, im + 1);  // H over odd a
+MEGA_HD void odd_last(float& er, float& ei, float& orr, float& oi, c32 z1, c32 z3) {
+  const float pr = fma1(-ei, z1.y, er * z1.x), pi = fma1(ei, z1.x, er * z1.y);
+  const float tr = fma1(-oi, z3.y, fma1(orr, z3.x, pr)), ti = fma1(oi, z3.x, fma1(orr, z3.y, pi));
+  orr = fma1(2.f, pi, -ti);
+  oi = fma1(-2.f, pr, tr);
+  er = tr;
+  ei = ti;
+}
+MEGA_HD void odd_transform32_w(float* re, float* im, const Powers& w, c32 z) {
+  stage_w<32, 2>(re, im, w.w16);
+  stage_w<32, 4>(re, im, csqv(w.w4));
+  stage_w<32, 8>(re, im, w.w4);
+  stage_w<32, 16>(re, im, csqv(w.w1));
+  const c32 z3 = cmulv(z, w.w1);
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-    const int pg = 2 * bitrev<4>(i), ph = pg + 1;
-    float gr = re[pg], gi = im[pg], hr = re[ph], hi = im[ph];
-    if (i != 0) {
-      mul_w<64>(gr, gi, i);
-      mul_w<64>(hr, hi, 3 * i);
+    const int p = 2 * bitrev<4>(i);
+    c32 a = z, b = z3;
+    if (i > 0) {
+      mul_w<64>(a.x, a.y, i);
+      mul_w<64>(b.x, b.y, 3 * i);
     }
-    re[pg] = gr + hr;
-    im[pg] = gi + hi;
-    const float dr = gr - hr, di = gi - hi;  // P[i+16] = -i (g - h)
-    re[ph] = di;
-    im[ph] = -dr;
+    odd_last(re[p], im[p], re[p + 1], im[p + 1], a, b);
   }
 }
 MEGA_HD constexpr int shifted_dit32_pos(int n) {
@@ -219,52 +256,38 @@ struct Cfg {
   static constexpr int LD2 = R3 + (R3 >= 8 ? 2 : 0);
   static constexpr int V2 = R3 == 4 ? 4 : 2;
   static constexpr int PLANE = (32 * LD1 > 1024 * LD2) ? 32 * LD1 : 1024 * LD2;
-  static constexpr int TABLE = 4 * T + R3 + 96 + 2048;  // c32 entries
+  static constexpr int TABLE = 4 * T + 3 * R3 + 192 + 2048;  // c32 entries
   static_assert(LOGM >= 11 && LOGM <= 14, "M must be 2048..16384");
 };
 
-// Per-lane twiddle seeds for one M (device memory, W_X^k = exp(-2 pi i k / X)).
-// Every twiddle of a pass is a geometric sequence base * ratio^k whose base
-// and ratio depend only on the lane, so a pass loads two seeds and generates
-// the rest with multiplications instead of 31 dependent table loads.
-//   kr[t]   = W_M^t                      ratio, forward pass 1 (t = lane)
-//   kbo[t]  = W_N^t                      base,  forward pass 1, odd half
-//   kp2[n0] = W_T^n0                     ratio, forward pass 2
-//   ki3[a1] = W_T^a1                     ratio, inverse pass 3
-//   kbe[t]  = W_M^(n0 a2)                base,  inverse pass 2, even (t = a2*R3 + n0)
-//   kre[a2] = W_M^(R3 a2)                ratio, inverse pass 2, even
-//   kbo2[t] = W_N^(n0 (2 a2 + 1))        base,  inverse pass 2, odd
-//   kro[a2] = W_N^(R3 (2 a2 + 1))        ratio, inverse pass 2, odd
-//   pw[h*1024 + c] = W_N^(2c + h)        pointwise twiddle
+// Per-lane twiddles for one M (device memory, W_X^k = exp(-2 pi i k / X)).
+// The inputs of a pass have the twiddles w^j of one w that depends only on the lane; a transform of 32 takes
+// its first, fourth and sixteenth power.
+//   k1[t]       = W_M^t                      inverse pass 1 (t = lane)
+//   kz[t]       = W_N^t                      inverse pass 1, odd half
+//   k2e[a2]     = W_M^(R3 a2)                forward pass 2, even half
+//   k2o[a2]     = W_N^(R3 (2 a2 + 1))        forward pass 2, odd half
+//   ki2[n0]     = W_T^n0                     inverse pass 2
+//   pw[h*1024 + c] = W_N^(2c + h)            forward pass 3 (residue c), pointwise twiddle
 struct Tables {
-  const c32* kr;
-  const c32* kbo;
-  const c32* kp2;
-  const c32* ki3;
-  const c32* kbe;
-  const c32* kre;
-  const c32* kbo2;
-  const c32* kro;
-  const c32* pw;
+  const Powers *k1, *k2e, *k2o, *ki2;
+  const c32 *kz, *pw;
 };
 
 template <int LOGM>
 MEGA_HD Tables make_tables(const c32* base) {
   using C = Cfg<LOGM>;
   Tables tb;
-  tb.kr = base;
-  tb.kbo = tb.kr + C::T;
-  tb.kbe = tb.kbo + C::T;
-  tb.kbo2 = tb.kbe + C::T;
-  tb.kp2 = tb.kbo2 + C::T;
-  tb.ki3 = tb.kp2 + C::R3;
-  tb.kre = tb.ki3 + 32;
-  tb.kro = tb.kre + 32;
-  tb.pw = tb.kro + 32;
+  tb.k1 = reinterpret_cast<const Powers*>(base);
+  tb.k2e = tb.k1 + C::T;
+  tb.k2o = tb.k2e + 32;
+  tb.ki2 = tb.k2o + 32;
+  tb.kz = reinterpret_cast<const c32*>(tb.ki2 + C::R3);
+  tb.pw = tb.kz + C::T;
   return tb;
 }
 
-// Host-side fill of the seed table (float64 trigonometry, exact argument reduction).
+// Host-side fill of the table (float64 trigonometry, exact argument reduction).
 template <int LOGM>
 inline void fill_tables(c32* out) {
   using C = Cfg<LOGM>;
@@ -275,58 +298,36 @@ inline void fill_tables(c32* out) {
     return c32{static_cast<float>(__builtin_cos(a)), static_cast<float>(__builtin_sin(a))};
   };
   c32* p = out;
-  for (int t = 0; t < C::T; ++t) *p++ = w(t, C::M);
+  auto powers = [&](double num, double den) {
+    for (int e = 1; e <= 16; e *= 4) *p++ = w(e * num, den);
+  };
+  for (int t = 0; t < C::T; ++t) powers(t, C::M);
+  for (int a2 = 0; a2 < 32; ++a2) powers(static_cast<double>(C::R3) * a2, C::M);
+  for (int a2 = 0; a2 < 32; ++a2) powers(static_cast<double>(C::R3) * (2 * a2 + 1), N);
+  for (int n0 = 0; n0 < C::R3; ++n0) powers(n0, C::T);
   for (int t = 0; t < C::T; ++t) *p++ = w(t, N);
-  for (int t = 0; t < C::T; ++t) *p++ = w(static_cast<double>(t % C::R3) * (t / C::R3), C::M);
-  for (int t = 0; t < C::T; ++t) *p++ = w(static_cast<double>(t % C::R3) * (2 * (t / C::R3) + 1), N);
-  for (int n0 = 0; n0 < C::R3; ++n0) *p++ = w(n0, C::T);
-  for (int a1 = 0; a1 < 32; ++a1) *p++ = w(a1, C::T);
-  for (int a2 = 0; a2 < 32; ++a2) *p++ = w(static_cast<double>(C::R3) * a2, C::M);
-  for (int a2 = 0; a2 < 32; ++a2) *p++ = w(static_cast<double>(C::R3) * (2 * a2 + 1), N);
   for (int h = 0; h < 2; ++h)
     for (int c = 0; c < 1024; ++c) *p++ = w(2.0 * c + h, N);
 }
 
 // table[idx] addressed as uniform base + 32-bit unsigned byte offset (lets the
 // compiler use the scalar-base addressing form instead of a 64-bit lane address)
+#if defined(__HIP_DEVICE_COMPILE__)
+// (said to be global memory: of a base that came through `launder` the compiler does not know it, and a flat load counts
+// among the LDS operations too, so that every wait for one waits for the other)
+#define MEGA_FFT_GLOBAL __attribute__((address_space(1)))
+#else
+#define MEGA_FFT_GLOBAL
+#endif
 MEGA_HD c32 ldc(const c32* base, unsigned idx) {
-  return *reinterpret_cast<const c32*>(reinterpret_cast<const char*>(base) + idx * 8u);
+  const auto* const p = (const MEGA_FFT_GLOBAL char*)(base) + idx * 8u;
+  const auto* const f = (const MEGA_FFT_GLOBAL float*)(p);
+  return c32{f[0], f[1]};
 }
-
-MEGA_HD c32 cmulv(c32 a, c32 b) { return c32{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x}; }
-MEGA_HD c32 csqv(c32 a) { return c32{a.x * a.x - a.y * a.y, 2.f * a.x * a.y}; }
-MEGA_HD c32 conjv(c32 a) { return c32{a.x, -a.y}; }
-
-// Calls f(k, base * r^k) for k = 0..COUNT-1.  Powers are built in blocks of 8
-// (block seeds by r^8, then a chain of 7), so no twiddle is more than 10
-// multiplications away from a table value.
-template <int COUNT, typename F>
-MEGA_HD void geo_twiddles(c32 base, c32 r, F&& f) {
-  const c32 r8 = csqv(csqv(csqv(r)));
-  c32 blk = base;
-#pragma unroll
-  for (int a = 0; a < COUNT; a += 8) {
-    c32 s = blk;
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
-      if (a + b < COUNT) {
-        f(a + b, s);
-        if (b + 1 < 8 && a + b + 1 < COUNT) s = cmulv(s, r);
-      }
-    }
-    if (a + 8 < COUNT) blk = cmulv(blk, r8);
-  }
-}
-
-MEGA_HD void cmul_ip(float& xr, float& xi, c32 w) {
-  const float r = xr * w.x - xi * w.y;
-  xi = xr * w.y + xi * w.x;
-  xr = r;
-}
-MEGA_HD void cmulc_ip(float& xr, float& xi, c32 w) {  // times conj(w)
-  const float r = xr * w.x + xi * w.y;
-  xi = xi * w.x - xr * w.y;
-  xr = r;
+MEGA_HD Powers ldc(const Powers* base, unsigned idx) {
+  const auto* const p = (const MEGA_FFT_GLOBAL char*)(base) + idx * 24u;
+  const auto* const f = (const MEGA_FFT_GLOBAL float*)(p);
+  return Powers{c32{f[0], f[1]}, c32{f[2], f[3]}, c32{f[4], f[5]}};
 }
 
 // residues of slot s for half H
@@ -342,19 +343,11 @@ MEGA_HD void slot_residues(int s, int& c0, int& c1) {
 }
 
 // ------------------------------ forward ------------------------------------
-// F1: pass 1 on natural-order input v[j] = z[t + T j]; leaves the twiddled
-// outputs in registers (output a2 at position bitrev5(a2)).
-template <int LOGM, int H>
-MEGA_HD void fwd_pass1(float* re, float* im, int t, const Tables& tb) {
-  const c32 r = ldc(tb.kr, t);
-  const c32 base = H == 0 ? c32{1.f, 0.f} : ldc(tb.kbo, t);
-  if (H == 0) dif<32, 1>(re, im); else shifted_dif32(re, im);
-  // W_M^(t a2) (even) or W_N^(t (2 a2 + 1)) = W_N^t (W_M^t)^a2 (odd)
-  geo_twiddles<32>(base, r, [&](int a2, c32 w) {
-    if (H == 0 && a2 == 0) return;
-    const int pos = bitrev<5>(a2);
-    cmul_ip(re[pos], im[pos], w);
-  });
+// Every pass takes its inputs' twiddles with it (transform32_w); pass 1's are known at compile time.
+// Pass 1 on natural-order input v[j] = z[t + T j]; output a2 at position bitrev5(a2).
+template <int H>
+MEGA_HD void fwd_first(float* re, float* im) {
+  transform<32, H == 0 ? 0 : 64>(re, im);
 }
 template <int LOGM>
 MEGA_HD void x1_write(const float* re, const float* im, int t, float* lre, float* lim) {
@@ -377,17 +370,13 @@ MEGA_HD void x1_read(float* re, float* im, int t, const float* lre, const float*
     im[n1] = lim[a2p * C::LD1 + n1 * C::R3 + n0p];
   }
 }
-template <int LOGM>
-MEGA_HD void fwd_pass2(float* re, float* im, int t, const Tables& tb) {
-  using C = Cfg<LOGM>;
-  const c32 r = ldc(tb.kp2, t % C::R3);  // W_T^n0'
-  dif<32, 1>(re, im);
-  geo_twiddles<32>(c32{1.f, 0.f}, r, [&](int a1, c32 w) {
-    if (a1 == 0) return;
-    const int pos = bitrev<5>(a1);
-    cmul_ip(re[pos], im[pos], w);
-  });
+// Pass 2 behind the twiddles W_M^(R3 n1 a2') (even) or W_N^(R3 n1 (2 a2' + 1)); what their share of n0' is goes to pass 3.
+// A pass needs its twiddles with its first butterfly, so the kernels ask for them a pass ahead.
+template <int LOGM, int H>
+MEGA_HD Powers second_twiddles(int t, const Tables& tb) {
+  return ldc(H == 0 ? tb.k2e : tb.k2o, t / Cfg<LOGM>::R3);
 }
+MEGA_HD void fwd_second(float* re, float* im, const Powers& w) { transform32_w(re, im, w); }
 // element (a2', a1, n0') goes to residue c = a2' + 32 a1
 template <int LOGM>
 MEGA_HD void x2_write(const float* re, const float* im, int t, float* lre, float* lim) {
@@ -430,12 +419,35 @@ MEGA_HD void x2_read(float* re, float* im, int t, const float* lre, const float*
     }
   }
 }
-// pass 3: bin a0 of (u, w) ends at register sidx(u, w, bitrev(a0))
+// pass 3: bin a0 of (u, w) ends at register sidx(u, w, bitrev(a0)); the twiddles of residue c are W_M^(n0 c) (even) or
+// W_N^(n0 (2 c + 1))
 template <int LOGM>
-MEGA_HD void fwd_pass3(float* re, float* im) {
-  using C = Cfg<LOGM>;
+struct Thirds {
+  c32 w[Cfg<LOGM>::NSLOT];  // of c0 of the lane's slots
+};
+template <int LOGM, int H>
+MEGA_HD Thirds<LOGM> third_twiddles(int t, const Tables& tb) {
+  Thirds<LOGM> th;
 #pragma unroll
-  for (int g = 0; g < 2 * C::NSLOT; ++g) dif<C::R3, 1>(re + g * C::R3, im + g * C::R3);
+  for (int u = 0; u < Cfg<LOGM>::NSLOT; ++u) th.w[u] = ldc(tb.pw, H * 1024 + t + Cfg<LOGM>::T * u);
+  return th;
+}
+template <int LOGM, int H>
+MEGA_HD void fwd_third(float* re, float* im, int t, const Thirds<LOGM>& th) {
+  constexpr int R3 = Cfg<LOGM>::R3, q = 64 / R3;
+#pragma unroll
+  for (int u = 0; u < Cfg<LOGM>::NSLOT; ++u) {
+    const c32 w0 = th.w[u];
+    // the partner's: c1 = 1024 - c0 or (2 c1 + 1) = 2048 - (2 c0 + 1), W_M^1024 = W_R3; 512 beside 0
+    c32 w1{fma1(-kS64[q], w0.y, kC64[q] * w0.x), fma1(-kC64[q], w0.y, -kS64[q] * w0.x)};
+    if (H == 0 && u == 0) {
+      const bool self = t == 0;
+      w1.x = self ? kC64[q / 2] : w1.x;
+      w1.y = self ? -kS64[q / 2] : w1.y;
+    }
+    transform_w<R3>(re + sidx<LOGM>(u, 0, 0), im + sidx<LOGM>(u, 0, 0), w0);
+    transform_w<R3>(re + sidx<LOGM>(u, 1, 0), im + sidx<LOGM>(u, 1, 0), w1);
+  }
 }
 
 // ------------------------------ pointwise ----------------------------------
@@ -515,29 +527,12 @@ MEGA_HD void pointwise(float* re, float* im, const float* bre, const float* bim,
 }
 
 // ------------------------------ inverse ------------------------------------
-// pass 3': inverse radix-R3 over a0 (swapped re/im), then conj pass-2 twiddle
-template <int LOGM, int H>
-MEGA_HD void inv_pass3(float* re, float* im, int t, const Tables& tb) {
+// pass 3': inverse radix-R3 over a0 (swapped re/im: a conjugated twiddle is a plain one there)
+template <int LOGM>
+MEGA_HD void inv_third(float* re, float* im) {
   using C = Cfg<LOGM>;
-  c32 rr[2 * C::NSLOT];
-#pragma unroll
-  for (int u = 0; u < C::NSLOT; ++u) {
-    int c[2];
-    slot_residues<H>(t + C::T * u, c[0], c[1]);
-    rr[2 * u] = conjv(ldc(tb.ki3, c[0] >> 5));
-    rr[2 * u + 1] = conjv(ldc(tb.ki3, c[1] >> 5));
-  }
 #pragma unroll
   for (int g = 0; g < 2 * C::NSLOT; ++g) dit<C::R3, 1>(im + g * C::R3, re + g * C::R3);
-#pragma unroll
-  for (int g = 0; g < 2 * C::NSLOT; ++g) {
-    // conj(W_T^(n0 a1)), a1 = residue >> 5
-    geo_twiddles<C::R3>(c32{1.f, 0.f}, rr[g], [&](int n0, c32 w) {
-      if (n0 == 0) return;
-      const int i = g * C::R3 + n0;
-      cmul_ip(re[i], im[i], w);
-    });
-  }
 }
 template <int LOGM, int H>
 MEGA_HD void ix2_write(const float* re, const float* im, int t, float* lre, float* lim) {
@@ -576,20 +571,12 @@ MEGA_HD void ix2_read(float* re, float* im, int t, const float* lre, const float
     im[a1] = lim[c * C::LD2 + n0p];
   }
 }
-// pass 2': inverse radix-32 over a1 -> n1 at bitrev5(n1); conj pass-1 twiddle
-// conj(W^((n1 R3 + n0') ...)) = conj(base) conj(ratio)^n1
-template <int LOGM, int H>
-MEGA_HD void inv_pass2(float* re, float* im, int t, const Tables& tb) {
-  using C = Cfg<LOGM>;
-  const int a2p = t / C::R3;
-  const c32 base = conjv(ldc(H == 0 ? tb.kbe : tb.kbo2, t));
-  const c32 r = conjv(ldc(H == 0 ? tb.kre : tb.kro, a2p));
-  dif<32, 1>(im, re);
-  geo_twiddles<32>(base, r, [&](int n1, c32 w) {
-    const int pos = bitrev<5>(n1);
-    cmul_ip(re[pos], im[pos], w);
-  });
+// pass 2': inverse radix-32 over a1 -> n1 at bitrev5(n1), behind the twiddles conj W_T^(n0' a1)
+template <int LOGM>
+MEGA_HD Powers inv_second_twiddles(int t, const Tables& tb) {
+  return ldc(tb.ki2, t % Cfg<LOGM>::R3);
 }
+MEGA_HD void inv_second(float* re, float* im, const Powers& w) { transform32_w(im, re, w); }
 template <int LOGM>
 MEGA_HD void ix1_write(const float* re, const float* im, int t, float* lre, float* lim) {
   using C = Cfg<LOGM>;
@@ -610,15 +597,74 @@ MEGA_HD void ix1_read(float* re, float* im, int t, const float* lre, const float
     im[a2] = lim[a2 * C::LD1 + t];
   }
 }
-// pass 1': inverse radix-32 over a2; zy[t + T n2] ends at register out_pos<H>(n2)
+// pass 1': inverse radix-32 over a2, behind the twiddles conj W_M^(t a2) or conj W_N^(t (2 a2 + 1)); zy[t + T n2] ends at
+// register out_pos<H>(n2)
+struct Firsts {
+  Powers w;
+  c32 z;
+};
 template <int H>
-MEGA_HD void inv_pass1(float* re, float* im) {
-  if (H == 0) dif<32, 1>(im, re); else shifted_dit32(im, re);
+MEGA_HD Firsts inv_first_twiddles(int t, const Tables& tb) {
+  return Firsts{ldc(tb.k1, t), H == 0 ? c32{1.f, 0.f} : ldc(tb.kz, t)};
+}
+template <int H>
+MEGA_HD void inv_first(float* re, float* im, const Firsts& f) {
+  if (H == 0) transform32_w(im, re, f.w);
+  else odd_transform32_w(im, re, f.w, f.z);
 }
 template <int H>
 MEGA_HD constexpr int out_pos(int n2) {
   return H == 0 ? bitrev<5>(n2) : shifted_dit32_pos(n2);
 }
+
+#if !defined(__HIPCC__)
+// On the CPU also the passes one by one as textbooks have them, each leaving its outputs with the twiddles that the next
+// one's inputs take: a pass above with those of its inputs moved.
+MEGA_HD void turn(float& xr, float& xi, double num, double den) {  // times exp(-2 pi i num / den)
+  const double a = -6.283185307179586476925286766559 * (__builtin_fmod(num, den) / den);
+  const c32 v = cmulv(c32{xr, xi}, c32{static_cast<float>(__builtin_cos(a)), static_cast<float>(__builtin_sin(a))});
+  xr = v.x;
+  xi = v.y;
+}
+template <int LOGM, int H>
+MEGA_HD void fwd_pass1(float* re, float* im, int t, const Tables&) {
+  fwd_first<H>(re, im);
+  for (int j = 0; j < 32; ++j) turn(re[j], im[j], H * t, 2.0 * Cfg<LOGM>::M);
+}
+template <int LOGM>
+MEGA_HD void fwd_pass2(float* re, float* im, int t, const Tables& tb) {
+  using C = Cfg<LOGM>;
+  fwd_second(re, im, second_twiddles<LOGM, 0>(t, tb));
+  for (int a1 = 0; a1 < 32; ++a1) {
+    const int at = bitrev<5>(a1);
+    turn(re[at], im[at], static_cast<double>(t % C::R3) * (t / C::R3 + 32 * a1), C::M);
+  }
+}
+template <int LOGM>
+MEGA_HD void fwd_pass3(float* re, float* im) {
+  constexpr int R3 = Cfg<LOGM>::R3;
+  for (int g = 0; g < 32; g += R3) transform<R3>(re + g, im + g);
+}
+template <int LOGM, int H>
+MEGA_HD void inv_pass3(float* re, float* im, int, const Tables&) {
+  inv_third<LOGM>(re, im);
+}
+template <int LOGM, int H>
+MEGA_HD void inv_pass2(float* re, float* im, int t, const Tables& tb) {
+  using C = Cfg<LOGM>;
+  inv_second(re, im, inv_second_twiddles<LOGM>(t, tb));
+  for (int n1 = 0; n1 < 32; ++n1) {
+    const int at = bitrev<5>(n1);
+    turn(re[at], im[at], -static_cast<double>(n1 * C::R3 + t % C::R3) * (2 * (t / C::R3) + H), 2.0 * C::M);
+  }
+}
+template <int H>
+MEGA_HD void inv_pass1(float* re, float* im) {
+  const c32 one{1.f, 0.f};
+  if (H == 0) transform<32>(im, re);
+  else odd_transform32_w(im, re, Powers{one, one, one}, one);
+}
+#endif
 
 // How a launch shares out its rows: how many rows of a channel a group takes, chosen for the shortest line of
 // transforms, in halves of one, that a workgroup slot gets (5 for a pair of rows, 3 for a row alone).  `bound`: a channel's sum

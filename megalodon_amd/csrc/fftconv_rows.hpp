@@ -196,13 +196,22 @@ __device__ __forceinline__ void gst(void* base, unsigned byte_off, V v) {
 
 // A pair of adjacent elements as one 32/64-bit access.
 template <int DT> struct Pair;
+typedef float float2_any __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t u32_any __attribute__((aligned(2)));
 template <> struct Pair<MEGA_F32> {
   using type = float2;
+  static __device__ __forceinline__ type load_any(const void* base, unsigned off) {
+    const float2_any v = gld<float2_any>(base, off);
+    return make_float2(v.x, v.y);
+  }
+  static __device__ __forceinline__ void store_any(void* base, unsigned off, type v) { gst<float2_any>(base, off, float2_any{v.x, v.y}); }
   static __device__ __forceinline__ void unpack(type v, float& lo, float& hi) { lo = v.x; hi = v.y; }
   static __device__ __forceinline__ type pack(float lo, float hi) { return make_float2(lo, hi); }
 };
 template <> struct Pair<MEGA_BF16> {
   using type = uint32_t;
+  static __device__ __forceinline__ type load_any(const void* base, unsigned off) { return gld<u32_any>(base, off); }
+  static __device__ __forceinline__ void store_any(void* base, unsigned off, type v) { gst<u32_any>(base, off, v); }
   static __device__ __forceinline__ void unpack(type v, float& lo, float& hi) {
     lo = __uint_as_float(v << 16);
     hi = __uint_as_float(v & 0xffff0000u);
@@ -211,6 +220,8 @@ template <> struct Pair<MEGA_BF16> {
 };
 template <> struct Pair<MEGA_F16> {
   using type = uint32_t;
+  static __device__ __forceinline__ type load_any(const void* base, unsigned off) { return gld<u32_any>(base, off); }
+  static __device__ __forceinline__ void store_any(void* base, unsigned off, type v) { gst<u32_any>(base, off, v); }
   static __device__ __forceinline__ void unpack(type v, float& lo, float& hi) {
     lo = f16_bits_to_float(static_cast<uint16_t>(v & 0xffffu));
     hi = f16_bits_to_float(static_cast<uint16_t>(v >> 16));
@@ -230,8 +241,10 @@ __device__ __forceinline__ int own_lane(int t) {
 
 // z[n] = s[2n] + i s[2n+1] of the zero-padded (optionally reversed) row.  Every lane reads inside the
 // row and takes zero for what lies behind it, so that the 32 loads stand in one piece without branches.
-// VEC: L is even and the row is pair-aligned, so (s[2n], s[2n+1]) is one access
-// addressed with a 32-bit offset from the wave-uniform row base.
+// A pair (s[2n], s[2n+1]) is one access addressed with a 32-bit offset from the wave-uniform row base.
+// VEC: L is even and the row is pair-aligned.  Otherwise the pairs lie at any element, and of an odd L the last value is
+// taken with the one in front of it (L >= 2).  (Element by element the loads had no registers to stand in together and were
+// waited for one by one: 2 x 512 rows of 10001 bfloat16 forward and backward 403 us, 8 x 1024 of 2049 691.)
 template <int LOGM, int DT, bool VEC>
 __device__ __forceinline__ void load_row(float* re, float* im, const void* row, int L, bool flip,
                                          int lane) {
@@ -256,13 +269,22 @@ __device__ __forceinline__ void load_row(float* re, float* im, const void* row, 
       im[j] = in ? (flip ? lo : hi) : 0.f;
     }
   } else {
+    using P = typename Pair<DT>::type;
+    constexpr int kSize = sizeof(P) / 2;
+    P raw[32];
 #pragma unroll
     for (int j = 0; j < 32; ++j) {
-      const unsigned m0 = 2u * (t + C::T * j), m1 = m0 + 1u;
-      const float a = ld<DT>(row, static_cast<int64_t>(((m0 < last ? m0 : last) ^ turn) + from));
-      const float b = ld<DT>(row, static_cast<int64_t>(((m1 < last ? m1 : last) ^ turn) + from));
-      re[j] = m0 < count ? a : 0.f;
-      im[j] = m1 < count ? b : 0.f;
+      const int m = 2 * static_cast<int>(t + C::T * j), at = flip ? L - 2 - m : m;
+      raw[j] = Pair<DT>::load_any(row, static_cast<unsigned>(max(0, min(at, L - 2)) * kSize));
+    }
+#pragma unroll
+    for (int j = 0; j < 32; ++j) {
+      const int m = 2 * static_cast<int>(t + C::T * j);
+      float lo, hi;
+      Pair<DT>::unpack(raw[j], lo, hi);
+      const bool alone = m + 1 == L;
+      re[j] = m < L ? (flip != alone ? hi : lo) : 0.f;
+      im[j] = m + 1 < L ? (flip ? lo : hi) : 0.f;
     }
   }
 }
@@ -301,18 +323,31 @@ __device__ __forceinline__ void store_row(const float* re, const float* im, void
       }
     }
   } else {
+    using P = typename Pair<DT>::type;
+    constexpr int kSize = sizeof(P) / 2;
 #pragma unroll
     for (int j = 0; j < 32; ++j) {
-      const int m0 = 2 * (t + C::T * j), m1 = m0 + 1;
-      if (m0 < L) {
-        const int o = flip ? L - 1 - m0 : m0;
-        const float r = res != nullptr ? w * ld<DT>(res, o) : 0.f;
-        st<DT>(row, o, (ACC ? ld<DT>(row, o) + re[j] : re[j]) + r);
-      }
-      if (m1 < L) {
-        const int o = flip ? L - 1 - m1 : m1;
-        const float r = res != nullptr ? w * ld<DT>(res, o) : 0.f;
-        st<DT>(row, o, (ACC ? ld<DT>(row, o) + im[j] : im[j]) + r);
+      const int m = 2 * (t + C::T * j);
+      if (m + 1 < L) {
+        const unsigned off = static_cast<unsigned>(flip ? L - 2 - m : m) * kSize;
+        float lo = flip ? im[j] : re[j], hi = flip ? re[j] : im[j];
+        if (ACC) {
+          float plo, phi;
+          Pair<DT>::unpack(Pair<DT>::load_any(row, off), plo, phi);
+          lo += plo;
+          hi += phi;
+        }
+        if (res != nullptr) {
+          float rlo, rhi;
+          Pair<DT>::unpack(Pair<DT>::load_any(res, off), rlo, rhi);
+          lo = fmaf(w, rlo, lo);
+          hi = fmaf(w, rhi, hi);
+        }
+        Pair<DT>::store_any(row, off, Pair<DT>::pack(lo, hi));
+      } else if (m < L) {
+        const int o = flip ? 0 : m;
+        const float r = ACC ? ld<DT>(row, o) + re[j] : re[j];
+        st<DT>(row, o, res != nullptr ? fmaf(w, ld<DT>(res, o), r) : r);
       }
     }
   }
@@ -322,8 +357,7 @@ __device__ __forceinline__ void store_row(const float* re, const float* im, void
 // twiddles are re-read from L1/L2 at each use instead of being kept live in
 // registers across transforms (which would spill).
 __device__ __forceinline__ Tables launder(Tables tb) {
-  asm volatile("" : "+s"(tb.kr), "+s"(tb.kbo), "+s"(tb.kbe), "+s"(tb.kbo2));
-  asm volatile("" : "+s"(tb.kp2), "+s"(tb.ki3), "+s"(tb.kre), "+s"(tb.kro), "+s"(tb.pw));
+  asm volatile("" : "+s"(tb.k1), "+s"(tb.k2e), "+s"(tb.k2o), "+s"(tb.ki2), "+s"(tb.kz), "+s"(tb.pw));
   return tb;
 }
 
@@ -331,34 +365,38 @@ template <int LOGM, int H>
 __device__ __forceinline__ void forward_half(float* re, float* im, int t, const Tables& tb0,
                                              float* lre, float* lim) {
   const Tables tb = launder(tb0);
-  fwd_pass1<LOGM, H>(re, im, t, tb);
+  const Powers second = second_twiddles<LOGM, H>(t, tb);
+  fwd_first<H>(re, im);
   __syncthreads();
   x1_write<LOGM>(re, im, t, lre, lim);
   __syncthreads();
   x1_read<LOGM>(re, im, t, lre, lim);
-  fwd_pass2<LOGM>(re, im, t, tb);
+  const Thirds<LOGM> third = third_twiddles<LOGM, H>(t, tb);
+  fwd_second(re, im, second);
   __syncthreads();
   x2_write<LOGM>(re, im, t, lre, lim);
   __syncthreads();
   x2_read<LOGM, H>(re, im, t, lre, lim);
-  fwd_pass3<LOGM>(re, im);
+  fwd_third<LOGM, H>(re, im, t, third);
 }
 
 template <int LOGM, int H>
 __device__ __forceinline__ void inverse_half(float* re, float* im, int t, const Tables& tb0,
                                              float* lre, float* lim) {
   const Tables tb = launder(tb0);
-  inv_pass3<LOGM, H>(re, im, t, tb);
+  const Powers second = inv_second_twiddles<LOGM>(t, tb);
+  inv_third<LOGM>(re, im);
   __syncthreads();
   ix2_write<LOGM, H>(re, im, t, lre, lim);
   __syncthreads();
   ix2_read<LOGM>(re, im, t, lre, lim);
-  inv_pass2<LOGM, H>(re, im, t, tb);
+  const Firsts first = inv_first_twiddles<H>(t, tb);
+  inv_second(re, im, second);
   __syncthreads();
   ix1_write<LOGM>(re, im, t, lre, lim);
   __syncthreads();
   ix1_read<LOGM>(re, im, t, lre, lim);
-  inv_pass1<H>(re, im);
+  inv_first<H>(re, im, first);
 }
 
 // The lane's 32 values as they stand in its registers, to and from a part of the workgroup's scratch slot (2 M floats a part).
@@ -529,7 +567,7 @@ int launch_fft_v(const void* a, const void* b, void* out, int64_t B, int64_t D, 
   int rc = get_tables<LOGM>(stream, &tab, &slots);
   if (rc != MEGA_OK) return rc;
   MEGA_CHECK_ARG(B * D <= 0x7fffffff, "fftconv: too many rows");
-  constexpr int kMost = MODE == 0 && (LOGM == 14 || !VEC) ? 1 : 2;
+  constexpr int kMost = MODE == 0 && LOGM == 14 ? 1 : 2;
   int64_t nb = group_rows(B, D, slots, kMost, MODE == 1);
   int pair = nb == 1 ? 1 : kMost;
   const auto parts = [&] { return pair + (MODE == 1 && nb < B ? 1 : 0); };
