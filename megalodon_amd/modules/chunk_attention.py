@@ -62,8 +62,19 @@ class _InnerAttention(nn.Module):
             return t
         return t.reshape(-1, self.chunk_size, *t.shape[2:])
 
+    @staticmethod
+    def _joined(old: Tensor, new: Tensor, fresh: bool) -> Tensor:
+        """`torch.cat((old, new), dim=1)`; behind an empty cache a tensor that is nobody else's is that already."""
+        if (fresh and old.dim() == 4 and old.shape[1] == 0 and old.shape[::2] == new.shape[::2] and old.shape[3] == new.shape[3]
+                and old.dtype == new.dtype and old.device == new.device and not old.requires_grad
+                and type(old) is Tensor and type(new) is Tensor
+                and new.is_contiguous()):
+            return new
+        return torch.cat((old, new), dim=1)
+
     def forward(self, xq: Tensor, xk: Tensor, xv: Tensor, mask: Optional[Tensor], freqs_cis: Optional[Tensor],
-                cache: Optional[Tuple[Tensor, Tensor, int]] = None):
+                cache: Optional[Tuple[Tensor, Tensor, int]] = None, *, fresh: bool = False):
+        """`fresh`: the caller has made xk and xv for this call alone, so that they may become the cache themselves."""
         batch, new_len = xq.shape[:2]
         q = xq.unflatten(-1, (self.n_heads, self.z_head_dim))
         k = xk.unflatten(-1, (self.n_heads, self.z_head_dim))
@@ -80,7 +91,7 @@ class _InnerAttention(nn.Module):
             old_k, old_v, old_len = cache
             total = old_len + new_len
             tail = total % self.chunk_size  # steps of the chunk still open after this call
-            k, v = torch.cat((old_k, k), dim=1), torch.cat((old_v, v), dim=1)
+            k, v = self._joined(old_k, k, fresh), self._joined(old_v, v, fresh)
             carried = (k.detach()[:, total - tail:], v.detach()[:, total - tail:], tail)
 
         q, k, v = self._chunks(q), self._chunks(k), self._chunks(v)

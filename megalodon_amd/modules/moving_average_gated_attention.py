@@ -111,7 +111,9 @@ class MovingAverageGatedAttention(nn.Module):
         # B x L x E
         v = F.silu(self.wv(out_tsn))
 
-        attn, cache_attn = self.inner_attention(q.contiguous(), k.contiguous(), v, mask, freqs_cis, cache_attn)
+        # (k and v are made here, and nobody else holds them: a new cache may keep them as they are)
+        fresh = {"fresh": True} if type(self.inner_attention) is _InnerAttention and not v.requires_grad and not k.requires_grad else {}
+        attn, cache_attn = self.inner_attention(q.contiguous(), k.contiguous(), v, mask, freqs_cis, cache_attn, **fresh)
         # attn * silu(r) in one pass
         attn = memory_efficient_dropout(silu_mul(r, attn), self.hidden_dropout, self.training)
 
