@@ -1337,19 +1337,26 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       wave_sync();  // the tile has been read: its place takes the wave's rows of (G, G')
     }
     load_x(next);
+    floatx16 xacc[2];  // (X, X') of the lane's chunk, until R is there
     if (on) {
-      // ---- (G, G') = Pg DY, into this wave's own rows of the state buffer ----------------
+      // ---- (G, G') = Pg DY, into this wave's own rows of the state buffer, and (X, X') = Pg XR with
+      //      the same operands ---------------------------------------------------------------------
 #pragma unroll
       for (int kind = 0; kind < 2; ++kind) {
         floatx16 acc;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+        for (int i = 0; i < 16; ++i) acc[i] = xacc[kind][i] = 0.f;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
           u32x4 a[2];
           load_block(kind * 4 + s, a, lane);
           acc = mma_split<1>(a, db[s].pc, acc);
-          if constexpr (FINE) acc = mfma_bf16(kind ? third1[s] : sm.third[s][lane], db[s].pc[0], acc);
+          xacc[kind] = mma_split<1>(a, &xr[s], xacc[kind]);
+          if constexpr (FINE) {
+            const u32x4 third = kind ? third1[s] : sm.third[s][lane];
+            acc = mfma_bf16(third, db[s].pc[0], acc);
+            xacc[kind] = mfma_bf16(third, xr[s], xacc[kind]);
+          }
         }
         float* dst = myrows + r * kRP + 32 * kind + 4 * g;
 #pragma unroll
@@ -1491,21 +1498,8 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
           }
         }
       }
-      // ---- (X, X') = Pg XR;  W += X R[c+1], W' += X' R[c+1] + X R'[c+1] ---------------------------
+      // ---- W += X R[c+1], W' += X' R[c+1] + X R'[c+1] -----------------------------------------------
       {
-        floatx16 xacc[2];
-#pragma unroll
-        for (int kind = 0; kind < 2; ++kind) {
-#pragma unroll
-          for (int i = 0; i < 16; ++i) xacc[kind][i] = 0.f;
-#pragma unroll
-          for (int s = 0; s < 4; ++s) {
-            u32x4 a[2];
-            load_block(kind * 4 + s, a, lane);
-            xacc[kind] = mma_split<1>(a, &xr[s], xacc[kind]);
-            if constexpr (FINE) xacc[kind] = mfma_bf16(kind ? third1[s] : sm.third[s][lane], xr[s], xacc[kind]);
-          }
-        }
 #pragma unroll
         for (int qd = 0; qd < 4; ++qd) {
           const float4 rv = *reinterpret_cast<const float4*>(rnext + 4 * g + 8 * qd);

@@ -67,7 +67,7 @@ using namespace fftc;
 
 // Workgroups of a transform size that share a compute unit: the kernel's time is the latency of its
 // exchanges and barriers, so two waves per SIMD at every size, which is what the registers (32 complex
-// points per lane and operand: 219-256 of 256, none spilled) and the planes in LDS allow.  With one wave
+// points per lane and operand: 229-256 of 256, with rows one by one none spilled) and the planes in LDS allow.  With one wave
 // per SIMD below M = 16384 (and 330 registers) and the loads in branches, forward / backward in
 // bfloat16 took 2 x 1024 rows of 3000: 152 / 348 us, now 51 / 138; of 8192: 226 / 479, now 95 / 198;
 // 1024 rows of 16384: 236 / 485, now 115 / 219; of 32768: 440 / 891, now 246 / 502 (the last by the loads alone).
@@ -441,13 +441,15 @@ __device__ __forceinline__ void outputs(float* re, float* im, int t, const Table
 }
 
 // The rows of a channel that a workgroup takes: two at a time, which then share the transform of k (MODE 0) or the
-// inverse transform of dk, whose spectrum is summed over them (MODE 1).  The kernels' time is the transforms' arithmetic
-// (87 % of the vector issue slots), so what counts is their number: 2.5 per row instead of 3.  In MODE 0 k's spectrum then has
-// to stay in registers to the row's end: 8 to 12 of them spill, at M = 16384 72 and with odd lengths' loads 26, where the
-// rows go one by one (PAIR 1), as a channel's only row does.  One kernel for dx and dk, with dy's spectrum formed once (4
+// inverse transform of dk, whose spectrum is summed over them (MODE 1).  The kernels' time is mostly the transforms'
+// arithmetic (76 % of the vector issue slots at M = 4096), so what counts is their number: 2.5 per row instead of 3.  In MODE 0
+// k's spectrum then has to stay in registers to the row's end: 15 to 49 of them spill (written once, read once a row), at
+// M = 16384 72, where the rows go one by one (PAIR 1), as a channel's only row does.  Odd lengths in pairs / one by one: 8 x 1024
+// rows of 2049 forward 146 / 156 us, 8 x 512 of 3001 80 / 82, 2 x 512 of 10001 96 / 99, but 3 x 1024 of 4097 128 / 122.  One kernel for dx and dk, with dy's spectrum formed once (4
 // transforms per row), spills 54 to 139 registers and takes 269 us where these two take 168.
 // bfloat16, forward / backward in us: 2 x 1024 rows of 8192 97 / 194 -> 86 / 168, 4 x 1024 of 8190 181 / 385 -> 158 / 325; of
-// channels whose rows now share out the chip for dk too: 8 x 256 of 8192 89 / 377 -> 82 / 169, 8 x 512 of 3001 120 / 541 -> 119 / 271.
+// channels whose rows now share out the chip for dk too: 8 x 256 of 8192 89 / 377 -> 82 / 169, 8 x 512 of 3001 120 / 541 -> 119 / 271
+// (since, with twiddles inside the butterflies and odd rows' loads in pairs: forward alone 88, 148, 76, 80).
 struct Rows {
   int B, D, L;
   int nb, groups;  // group g: channel g % D, rows g / D nb ..
