@@ -50,6 +50,12 @@ __device__ __forceinline__ floatx16 mfma_bf16(u32x4 a, u32x4 b, floatx16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
                                                  __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+template <int DT>
+__device__ __forceinline__ floatx16 mfma16(u32x4 a, u32x4 b, floatx16 c) {
+  if constexpr (DT == MEGA_BF16) return mfma_bf16(a, b, c);
+  else return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
 // 8 floats -> packed bf16 high parts and packed bf16 residuals
 __device__ __forceinline__ void split8(const float* v, u32x4& hi, u32x4& lo) {
 #pragma unroll
@@ -59,6 +65,28 @@ __device__ __forceinline__ void split8(const float* v, u32x4& hi, u32x4& lo) {
     const float r1 = v[2 * e + 1] - __uint_as_float(h & 0xffff0000u);
     hi[e] = h;
     lo[e] = pack_bf16x2(r0, r1);
+  }
+}
+// the same in float16: 22 significant bits of values of some 2^12 (far below them the residuals end), with `third` 33
+// Each piece is taken off as it stands in the packed word, hidden from the optimiser: left alone it packs by one
+// instruction and takes the residual from another's result, and the two round ties apart.
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t take_f16(float& a, float& b) {
+  uint32_t w = __builtin_bit_cast(uint32_t, f16x2{static_cast<_Float16>(a), static_cast<_Float16>(b)});
+  asm volatile("" : "+v"(w));
+  const f16x2 h = __builtin_bit_cast(f16x2, w);
+  a -= static_cast<float>(h[0]);
+  b -= static_cast<float>(h[1]);
+  return w;
+}
+template <bool THIRD>
+__device__ __forceinline__ void split8_f16(const float* v, u32x4& hi, u32x4& lo, u32x4& third) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float a = v[2 * e], b = v[2 * e + 1];
+    hi[e] = take_f16(a, b);
+    lo[e] = take_f16(a, b);
+    if (THIRD) third[e] = take_f16(a, b);
   }
 }
 // ... and what is left of them behind that: 24 significant bits in three pieces
@@ -913,6 +941,13 @@ __device__ __forceinline__ uint2 lds_read_tr(const uint16_t* q) {
   return __builtin_bit_cast(uint2, v);
 }
 
+// Float16 rows are taken as they are: dy and x are matrix operands of their own type, the power matrix and the lags of
+// k two float16 pieces each (the power matrix three where the bfloat16 form has three), the largest value at 2^12, so that what
+// a float16 cannot hold is 2^-25 of it; the state part stays in bfloat16 pieces, whose range a state needs.  R and X are 2^12 times
+// themselves, a scale that Qd and the row's reductions take back; dx is scaled with k's largest lag, undone where it is
+// rounded.  With rows as bfloat16 pieces three launches (four where third pieces are) added up what one gives now:
+// backward of 1024 x 35840 385 / 77 us, 4096 x 32768 1315 / 275, 4 x 2048 x 5001 649 / 120, 2 x 512 x 759 100 / 37.
+constexpr float kPowScale = 4096.f;
 struct BwdSmem {
   u32x4 aop[kBwdBlocks][2][kWave];       // operand blocks, two pieces
   // row c: (R, R') at the start of chunk c of the segment.  A wave's own 32 rows double as its
@@ -963,7 +998,10 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
     const float* __restrict__ p, const cf* __restrict__ log_q, const cf* __restrict__ gamma,
     const float* __restrict__ omega, const cf* __restrict__ h0, float* __restrict__ dp, cf* __restrict__ dq,
     cf* __restrict__ dgamma, float* __restrict__ domega, cf* __restrict__ dh0, const Lines ln, int N) {
-  static_assert(XOp<DT>::XP == 1, "the backward kernel takes bfloat16 rows");
+  static_assert(DT == MEGA_BF16 || (DT == MEGA_F16 && DX32 == 0), "bfloat16 rows, or float16 rows with dx of their type");
+  constexpr bool H16 = DT == MEGA_F16;
+  constexpr float kScale = H16 ? kPowScale : 1.f;  // of Pg
+  using Op = XOp<MEGA_BF16>;                       // eight 16-bit steps as they are
   constexpr int CPS = kBwdCPS;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   constexpr bool FINE = kFine<ROWS>;
@@ -987,7 +1025,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
   // the last four tiles of a group's line, where its walk starts
   auto tail_of = [&](int group) { return group < ln.groups ? (ln.tiles(group) - 1) / kWaves * kWaves : 0; };
 
-  XOp<DT> db[4], xb[4], dn[4];  // dn: the next item's dy tile on its way
+  Op db[4], xb[4], dn[4];  // dn: the next item's dy tile on its way
   auto load_dy = [&](const Tile& w) {
     MEGA_LANE_IDS;
     const uint16_t* row = static_cast<const uint16_t*>(dy) + w.base;
@@ -1027,6 +1065,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
 
   // scan multipliers of this thread's mode: over a chunk, a sub-segment, a wave's chunks
   cf qT{0.f, 0.f}, q1{0.f, 0.f};
+  float unscale = 1.f;  // H16: of dx
   int cur = 0, par = 0;
   RowParams rp = fetch_params(blockIdx.x);
 
@@ -1071,6 +1110,13 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       qT = sm.pw[9][sn];
     }
     __syncthreads();
+    float kscale = 1.f;  // of K and with it of dx
+    if constexpr (H16) {
+      const float most = wave_max(fabsf(klocal[lane]));
+      const int up = most > 0.f && most < INFINITY ? min(100, max(-100, 13 - __builtin_amdgcn_frexp_expf(most))) : 0;
+      kscale = ldexpf(1.f, up);
+      unscale = ldexpf(1.f, -up);
+    }
     for (int item = tid; item < kBwdBlocks * kWave; item += kThreads) {
       const int blk = item >> 6, ln = item & 63, rr = ln & 31, gg = ln >> 5;
       float v[8];
@@ -1080,7 +1126,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
         for (int e = 0; e < 8; ++e) {
           const int i = 16 * s + 8 * gg + e;
           const cf w = qp[n][i];
-          const float sc = kind ? static_cast<float>(i) / kT : 1.f;
+          const float sc = kScale * (kind ? static_cast<float>(i) / kT : 1.f);
           v[e] = sc * (part ? w.y : w.x);
         }
       } else if (blk < 12) {
@@ -1089,7 +1135,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
         for (int e = 0; e < 8; ++e) {
           const int lag = o - rr + 8 * gg + e;
           const float kv = klocal[lag >= 0 ? lag : 0];  // read, then masked: no branch around the load
-          v[e] = lag >= 0 ? kv : 0.f;
+          v[e] = lag >= 0 ? (H16 ? kscale * kv : kv) : 0.f;
         }
       } else {
         const int jt = (blk - 12) >> 1, s2 = (blk - 12) & 1, j = 32 * jt + rr;
@@ -1099,16 +1145,19 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
           const cf c = cf{sm.pn[n] * sm.gn[n].x, sm.pn[n] * sm.gn[n].y};
           const cf w = cmul(c, qp[n][kT - j]);
           v[e] = (m & 1) ? -w.y : w.x;
+          if (H16) v[e] *= kscale / kPowScale;
         }
       }
-      u32x4 hi, lo;
-      split8(v, hi, lo);
+      u32x4 hi, lo, third;
+      if (H16 && blk < 12) split8_f16<FINE>(v, hi, lo, third);
+      else split8(v, hi, lo);
+      if (FINE && !H16) third = split8_third(v, hi, lo);
       sm.aop[blk][0][ln] = hi;
       sm.aop[blk][1][ln] = lo;
       if constexpr (FINE)
-        if (blk < 8) (blk < 4 ? sm.third[blk] : passed[blk - 4])[ln] = split8_third(v, hi, lo);
+        if (blk < 8) (blk < 4 ? sm.third[blk] : passed[blk - 4])[ln] = third;
     }
-    if constexpr (FINE) fill_thirds<false>(sm.kthird, klocal, tid);
+    if constexpr (FINE && !H16) fill_thirds<false>(sm.kthird, klocal, tid);
 #pragma unroll
     for (int t = 0; t < 3; ++t)
 #pragma unroll
@@ -1235,6 +1284,11 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
         wd.x += part[2];
         wd.y += part[3];
       }
+      if (H16) {  // (X and R each)
+        constexpr float back = 1.f / (kPowScale * kPowScale);
+        w = cf{back * w.x, back * w.y};
+        wd = cf{back * wd.x, back * wd.y};
+      }
       const cf qq = sm.pw[8][n];
       const cf A = cadd(ain, cmul(qq, w));
       const cf Bq{fmaf(kT, wd.x, bin.x + w.x), fmaf(kT, wd.y, bin.y + w.y)};
@@ -1249,7 +1303,11 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
         // start of the row -- its gradients are (ema_parameters.cc:158-188, PyTorch's convention)
         //   dgamma += conj(q h0 R0),  dq += conj(gamma h0 (R0 + q R0')),  dh0 = conj(gamma q R0)
         // (q R0' = 64 times what the scan has carried).
-        const cf r0 = sm.carry[cur][0][n], r0d = sm.carry[cur][1][n];
+        cf r0 = sm.carry[cur][0][n], r0d = sm.carry[cur][1][n];
+        if (H16) {
+          r0 = cf{r0.x / kPowScale, r0.y / kPowScale};
+          r0d = cf{r0d.x / kPowScale, r0d.y / kPowScale};
+        }
         const cf h = h0[row * N + n];
         const cf e1 = cmul(cmul(qq, h), r0);
         dgv.x += e1.x;
@@ -1328,10 +1386,10 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
           const u32x4 dyt = read_tr(it, ks);
-          if (it == 0) macc[0] = mfma_bf16(dyt, xt[0][ks], macc[0]);
+          if (it == 0) macc[0] = mfma16<DT>(dyt, xt[0][ks], macc[0]);
           if (it == 1) {
-            macc[1] = mfma_bf16(dyt, xt[0][ks], macc[1]);
-            macc[2] = mfma_bf16(dyt, xt[1][ks], macc[2]);
+            macc[1] = mfma16<DT>(dyt, xt[0][ks], macc[1]);
+            macc[2] = mfma16<DT>(dyt, xt[1][ks], macc[2]);
           }
         }
       wave_sync();  // the tile has been read: its place takes the wave's rows of (G, G')
@@ -1350,12 +1408,12 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
         for (int s = 0; s < 4; ++s) {
           u32x4 a[2];
           load_block(kind * 4 + s, a, lane);
-          acc = mma_split<1>(a, db[s].pc, acc);
-          xacc[kind] = mma_split<1>(a, &xr[s], xacc[kind]);
+          acc = mfma16<DT>(a[1], db[s].pc[0], mfma16<DT>(a[0], db[s].pc[0], acc));
+          xacc[kind] = mfma16<DT>(a[1], xr[s], mfma16<DT>(a[0], xr[s], xacc[kind]));
           if constexpr (FINE) {
             const u32x4 third = kind ? third1[s] : sm.third[s][lane];
-            acc = mfma_bf16(third, db[s].pc[0], acc);
-            xacc[kind] = mfma_bf16(third, xr[s], xacc[kind]);
+            acc = mfma16<DT>(third, db[s].pc[0], acc);
+            xacc[kind] = mfma16<DT>(third, xr[s], xacc[kind]);
           }
         }
         float* dst = myrows + r * kRP + 32 * kind + 4 * g;
@@ -1442,59 +1500,64 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       // the stores of dX go out first: they have the (X, X') products and the next item's
       // staging to retire under before the next loads are issued behind them
       // ---- DX = K^T DY + Qd R[c+1] (omega dy included: K carries omega on its diagonal) -------------
-      u32x4 hb[2][2];
-#pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
-        const float* src = rnext + 16 * s2 + 8 * g;
-        const float4 u0 = *reinterpret_cast<const float4*>(src);
-        const float4 u1 = *reinterpret_cast<const float4*>(src + 4);
-        const float v[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
-        split8(v, hb[s2][0], hb[s2][1]);
-      }
-#pragma unroll
-      for (int jt = 0; jt < 2; ++jt) {
-        floatx16 acc;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-#pragma unroll
-        for (int s = 2 * jt; s < 4; ++s) {
-          u32x4 a[2];
-          load_block(8 + s - 2 * jt, a, lane);
-          acc = mma_split<1>(a, db[s].pc, acc);
-          // (block b: lags 16 b - r + 8 g + e)
-          if constexpr (FINE) acc = mfma_bf16(read_thirds(sm.kthird, 16 * (s - 2 * jt) - r + 8 * g + 31), db[s].pc[0], acc);
-        }
+      if (DX32 != 1 || dx != nullptr) {
+        u32x4 hb[2][2];
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
-          u32x4 a[2];
-          load_block(12 + 2 * jt + s2, a, lane);
-          acc = mma_split<2, FINE>(a, hb[s2], acc);
+          const float* src = rnext + 16 * s2 + 8 * g;
+          const float4 u0 = *reinterpret_cast<const float4*>(src);
+          const float4 u1 = *reinterpret_cast<const float4*>(src + 4);
+          const float v[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+          split8(v, hb[s2][0], hb[s2][1]);
         }
 #pragma unroll
-        for (int pr = 0; pr < 2; ++pr) {
-          if constexpr (DX32) {
-            // registers 8 pr + 4 h + e hold the steps 16 pr + 8 h + 4 g + e
+        for (int jt = 0; jt < 2; ++jt) {
+          floatx16 acc;
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              const int elem = r * kT + 16 * (2 * jt + pr) + 8 * h + 4 * g;
-              if (dx != nullptr && ROWS != kAny && (ROWS == kWhole || elem >= w.lo) && elem + 4 <= w.hi) {
-                float4 v = make_float4(acc[8 * pr + 4 * h], acc[8 * pr + 4 * h + 1], acc[8 * pr + 4 * h + 2],
-                                       acc[8 * pr + 4 * h + 3]);
-                if constexpr (DX32 == 2) {
-                  const float4 o = *reinterpret_cast<const float4*>(dxrow + elem);
-                  v = make_float4(v.x + o.x, v.y + o.y, v.z + o.z, v.w + o.w);
+          for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+#pragma unroll
+          for (int s = 2 * jt; s < 4; ++s) {
+            u32x4 a[2];
+            load_block(8 + s - 2 * jt, a, lane);
+            acc = mfma16<DT>(a[1], db[s].pc[0], mfma16<DT>(a[0], db[s].pc[0], acc));
+            // (block b: lags 16 b - r + 8 g + e)
+            if constexpr (FINE && !H16) acc = mfma_bf16(read_thirds(sm.kthird, 16 * (s - 2 * jt) - r + 8 * g + 31), db[s].pc[0], acc);
+          }
+#pragma unroll
+          for (int s2 = 0; s2 < 2; ++s2) {
+            u32x4 a[2];
+            load_block(12 + 2 * jt + s2, a, lane);
+            acc = mma_split<2, FINE>(a, hb[s2], acc);
+          }
+          if constexpr (H16)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[i] *= unscale;
+#pragma unroll
+          for (int pr = 0; pr < 2; ++pr) {
+            if constexpr (DX32) {
+              // registers 8 pr + 4 h + e hold the steps 16 pr + 8 h + 4 g + e
+#pragma unroll
+              for (int h = 0; h < 2; ++h) {
+                const int elem = r * kT + 16 * (2 * jt + pr) + 8 * h + 4 * g;
+                if (dx != nullptr && ROWS != kAny && (ROWS == kWhole || elem >= w.lo) && elem + 4 <= w.hi) {
+                  float4 v = make_float4(acc[8 * pr + 4 * h], acc[8 * pr + 4 * h + 1], acc[8 * pr + 4 * h + 2],
+                                         acc[8 * pr + 4 * h + 3]);
+                  if constexpr (DX32 == 2) {
+                    const float4 o = *reinterpret_cast<const float4*>(dxrow + elem);
+                    v = make_float4(v.x + o.x, v.y + o.y, v.z + o.z, v.w + o.w);
+                  }
+                  *reinterpret_cast<float4*>(dxrow + elem) = v;
+                } else if (ROWS != kWhole && dx != nullptr) {
+#pragma unroll
+                  for (int e = 0; e < 4; ++e)
+                    if (elem + e >= w.lo && elem + e < w.hi)
+                      dxrow[elem + e] = acc[8 * pr + 4 * h + e] + (DX32 == 2 ? static_cast<float>(dxrow[elem + e]) : 0.f);
                 }
-                *reinterpret_cast<float4*>(dxrow + elem) = v;
-              } else if (ROWS != kWhole && dx != nullptr) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                  if (elem + e >= w.lo && elem + e < w.hi)
-                    dxrow[elem + e] = acc[8 * pr + 4 * h + e] + (DX32 == 2 ? static_cast<float>(dxrow[elem + e]) : 0.f);
               }
+            } else {
+              const uint4 oct = octet_of<DT>(acc, pr);
+              store8_16<ROWS>(dxrow, r * kT + 16 * (2 * jt + pr) + 8 * g, w.lo, w.hi, oct);
             }
-          } else {
-            const uint4 oct = octet_of<DT>(acc, pr);
-            store8_16<ROWS>(dxrow, r * kT + 16 * (2 * jt + pr) + 8 * g, w.lo, w.hi, oct);
           }
         }
       }
@@ -1546,19 +1609,19 @@ int bwd_lines(int64_t B, int64_t D, int64_t L, bool single, int rows, Lines* ln,
 }
 
 // single: gradients per row (B, D, N) as the operator returns them; else per group of rows
-template <int DX32, int ROWS>
+template <int DX32, int ROWS, int DT = MEGA_BF16>
 int launch_bwd(const void* dy, const void* x, void* dx, const float* p, const cf* log_q,
                const cf* gamma, const float* omega, const cf* h0, float* dp, cf* dq, cf* dgamma, float* domega,
                cf* dh0, int64_t B, int64_t D, int64_t N, int64_t L, bool single, hipStream_t stream) {
   const int lds = static_cast<int>(kFine<ROWS> ? sizeof(BwdSmemFine) : sizeof(BwdSmem));
-  MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cema_scan_bwd_kernel<MEGA_BF16, DX32, ROWS>),
+  MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cema_scan_bwd_kernel<DT, DX32, ROWS>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds));
   Lines ln;
   int64_t slots = 0;
   const int rc = bwd_lines(B, D, L, single || h0 != nullptr, ROWS, &ln, &slots);
   if (rc != MEGA_OK) return rc;
   const unsigned grid = static_cast<unsigned>(ln.groups < slots ? ln.groups : slots);
-  cema_scan_bwd_kernel<MEGA_BF16, DX32, ROWS><<<dim3(grid), kThreads, lds, stream>>>(
+  cema_scan_bwd_kernel<DT, DX32, ROWS><<<dim3(grid), kThreads, lds, stream>>>(
       dy, x, dx, p, log_q, gamma, omega, h0, dp, dq, dgamma, domega, dh0, ln, static_cast<int>(N));
   MEGA_CHECK_LAUNCH();
   return MEGA_OK;
@@ -1566,9 +1629,10 @@ int launch_bwd(const void* dy, const void* x, void* dx, const float* p, const cf
 
 using BwdLaunch = decltype(&launch_bwd<0, kWhole>);
 BwdLaunch bwd_for(int dx_mode, int rows) {
-  static const BwdLaunch table[3][3] = {{launch_bwd<0, kWhole>, launch_bwd<0, kShifted>, launch_bwd<0, kAny>},
+  static const BwdLaunch table[4][3] = {{launch_bwd<0, kWhole>, launch_bwd<0, kShifted>, launch_bwd<0, kAny>},
                                         {launch_bwd<1, kWhole>, launch_bwd<1, kShifted>, launch_bwd<1, kAny>},
-                                        {launch_bwd<2, kWhole>, launch_bwd<2, kShifted>, launch_bwd<2, kAny>}};
+                                        {launch_bwd<2, kWhole>, launch_bwd<2, kShifted>, launch_bwd<2, kAny>},
+                                        {launch_bwd<0, kWhole, MEGA_F16>, launch_bwd<0, kShifted, MEGA_F16>, launch_bwd<0, kAny, MEGA_F16>}};
   return table[dx_mode][rows];
 }
 
@@ -1726,7 +1790,7 @@ extern "C" int mega_cema_layer_scan_bwd(const void* dy, const void* x, const flo
   const char* who = "mega_cema_layer_scan_bwd";
   MEGA_CHECK_ARG(dy && x && p && log_q && gamma && dp && dq && dgamma && domega, "%s: null pointer", who);
   MEGA_CHECK_ARG(B >= 1 && D >= 1 && B * D <= 0x7fffffff, "%s: bad sizes", who);
-  MEGA_CHECK_ARG(dx_mode >= 0 && dx_mode <= 2 && (dx != nullptr || dx_mode == 1), "%s: bad dx", who);
+  MEGA_CHECK_ARG(dx_mode >= 0 && dx_mode <= 3 && (dx != nullptr || dx_mode == 1), "%s: bad dx", who);
   if (!mega_cema_scan_bwd_supported(MEGA_BF16, N, L))
     return set_error(MEGA_ERR_UNSUPPORTED, "%s: needs N <= 16 (N %lld, L %lld)", who, (long long)N, (long long)L);
   return bwd_for(dx_mode, rows_of(B * D, L, false, {dy, x, dx}))(dy, x, dx, p, reinterpret_cast<const cf*>(log_q), reinterpret_cast<const cf*>(gamma), omega, nullptr, dp,

@@ -322,10 +322,6 @@ Tensor rows_of(const Tensor& x) {
 }
 std::tuple<Tensor, Tensor> split(const Tensor& t) {
   const int64_t n = t.numel();
-  if (n % 8 != 0 || reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0) {
-    Tensor hi = t.to(at::kBFloat16);
-    return {hi, (t.to(at::kFloat) - hi.to(at::kFloat)).to(at::kBFloat16)};
-  }
   Tensor hi = at::empty(t.sizes(), t.options().dtype(at::kBFloat16)), lo = at::empty_like(hi);
   check(mega_split_bf16(t.data_ptr(), kernel_code(t), n, hi.data_ptr(), lo.data_ptr(), stream_of(t)), "mega_split_bf16");
   return {hi, lo};
@@ -352,26 +348,26 @@ struct CemaFn : Function<CemaFn> {
     void* s = stream_of(x);
     // gradients of the launches' groups of rows, stacked: (dp, dq, dgamma_hat, domega); the coefficients'
     // backward adds the stack up
-    const bool whole = L % 8 == 0;
-    const int64_t per = mega_cema_layer_scan_sets(B, D, L), pieces = x.scalar_type() == at::kBFloat16 ? 1 : whole ? 3 : 4, sets = pieces * per;
+    const bool wide = x.scalar_type() == at::kFloat;
+    const int64_t per = mega_cema_layer_scan_sets(B, D, L), pieces = wide ? 3 : 1, sets = pieces * per;
     const Tensor stack = floats({sets * (5 * DN + D)}, x);
     float *dp = stack.data_ptr<float>(), *dq = dp + sets * DN, *dg = dq + 2 * sets * DN, *dw = dg + 2 * sets * DN;
     Tensor dx;
-    if (x.scalar_type() == at::kBFloat16) {
+    if (!wide) {
       dx = at::empty_like(x);
-      check(mega_cema_layer_scan_bwd(dy.data_ptr(), x.data_ptr(), p, lq, gh, fptr(w), B, D, N, L, dx.data_ptr(), 0, dp, dq, dg, dw, s), "mega_cema_layer_scan_bwd");
+      const int mode = x.scalar_type() == at::kHalf ? 3 : 0;
+      check(mega_cema_layer_scan_bwd(dy.data_ptr(), x.data_ptr(), p, lq, gh, fptr(w), B, D, N, L, dx.data_ptr(), mode, dp, dq, dg, dw, s), "mega_cema_layer_scan_bwd");
     } else {
       // linear in dy and, for the parameter gradients, in x: the bfloat16 pieces (dy_hi, x_hi), (dy_lo, x_hi),
       // (dy_hi, x_lo); dx is linear in dy alone and is added up in float32.  What is left out, (dy_lo, x_lo), is 2e-6 of
-      // the parameter gradients; lengths that are no multiple of 8 had them from a float32 convolution at 1e-6, so
-      // there it is added too (float16 rows, whose two pieces are exact).
+      // the parameter gradients.
       auto [g_hi, g_lo] = split(dy);
       auto [x_hi, x_lo] = split(x);
       Tensor dx32 = floats(x.sizes(), x);
-      const Tensor* pairs[4][2] = {{&g_hi, &x_hi}, {&g_lo, &x_hi}, {&g_hi, &x_lo}, {&g_lo, &x_lo}};
+      const Tensor* pairs[3][2] = {{&g_hi, &x_hi}, {&g_lo, &x_hi}, {&g_hi, &x_lo}};
       for (int i = 0; i < pieces; ++i)
         check(mega_cema_layer_scan_bwd(pairs[i][0]->data_ptr(), pairs[i][1]->data_ptr(), p, lq, gh, fptr(w), B, D, N, L, i < 2 ? dx32.data_ptr() : nullptr, i == 1 ? 2 : 1, dp + i * per * DN, dq + 2 * i * per * DN, dg + 2 * i * per * DN, dw + i * per * D, s), "mega_cema_layer_scan_bwd");
-      dx = dx32.to(x.scalar_type());
+      dx = dx32;
     }
     Tensor da = at::empty_like(alpha), dd = at::empty_like(delta), dt = at::empty_like(theta), dga = at::empty_like(gamma), dom = at::empty_like(omega);
     check(mega_cema_layer_coeffs_bwd(kernel_code(alpha), dp, dq, dg, dw, sets, alpha.data_ptr(), delta.data_ptr(), theta.data_ptr(), D, N, da.data_ptr(), dd.data_ptr(), dt.data_ptr(), dga.data_ptr(), dom.data_ptr(), s), "mega_cema_layer_coeffs_bwd");
