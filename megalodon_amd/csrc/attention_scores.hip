@@ -598,15 +598,29 @@ int launch_probs_short(ProbsParams p, hipStream_t s) {
   return MEGA_OK;
 }
 
+// How many blocks of 32 rows a CU, in eighths, the short-row kernel takes.  It reads a block's keys anew for every block, so
+// its time grows with the blocks and with the head's width, while the other one's is its longest row block's until the chip
+// is full.  The operator's forward with a value head of 64, in us, the short-row kernel / the other, at blocks a CU:
+//   width 64:  256 keys 4.0 21 / 26, 5.0 27 / 26; 512 keys 5.0 33 / 37, 6.0 36 / 35; 1500 keys 5.0 70 / 81, 6.1 84 / 83; 4096 keys 5.0
+//              142 / 165, 6.0 173 / 172
+//   width 128: 256 keys 3.0 22 / 26, 3.4 28 / 24; 512 keys 4.0 35 / 37, 5.0 43 / 38; 1500 keys 4.0 77 / 87, 5.0 91 / 90; 4096 keys 4.0
+//              156 / 171, 5.0 200 / 183
+//   width 256: 256 keys 1.5 26 / 28, 2.5 35 / 30; 512 keys 2.0 34 / 43, 2.5 44 / 43; 1024 keys 2.9 64 / 66, 3.4 78 / 68; 2048 keys 3.5
+//              108 / 117, 5.0 147 / 123; 4096 keys 3.0 198 / 214, 3.5 228 / 218
+// (three blocks a CU for all of them before.)
+constexpr int short_rows(int H1, int keys) {
+  if (H1 == 64) return keys <= 384 ? 32 : 44;
+  if (H1 == 128) return keys <= 384 ? 24 : 32;
+  return keys <= 384 ? 12 : keys <= 768 ? 17 : keys <= 1280 ? 24 : 26;
+}
+
 template <int DT, int H1>
 int launch_probs(const ProbsParams& p, hipStream_t s) {
-  // Few row blocks, both kernels in us (us of this one / of the short-row kernel, head width 256): 1024 keys, 64 row
-  // blocks of 32 55 / 24, 512 56 / 37, 768 60 / 57, 1024 58 / 72; 2048 keys, 128 row blocks 99 / 41, 512 101 / 53, 768 103 / 83,
-  // 1024 104 / 106; 4096 keys, 128 185 / 98, 512 187 / 114, 1024 201 / 235.  Head width 64, 1500 keys, 752: 60 / 29.
+  // few row blocks: see short_rows
   int dev = 0, cus = 0;
   MEGA_CHECK_HIP(hipGetDevice(&dev));
   MEGA_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  if (static_cast<int64_t>(p.Z) * ((p.L1 + 31) / 32) <= 3 * cus) return launch_probs_short<DT, H1>(p, s);
+  if (8 * static_cast<int64_t>(p.Z) * ((p.L1 + 31) / 32) <= static_cast<int64_t>(short_rows(H1, p.L2)) * cus) return launch_probs_short<DT, H1>(p, s);
   constexpr int KW = H1 >= 128 ? 128 : 64;
   const size_t lds = sizeof(uint16_t) * kRing * kKeys * KW;
   MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_probs_kernel<DT, H1>),
