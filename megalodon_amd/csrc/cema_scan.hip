@@ -941,13 +941,32 @@ __device__ __forceinline__ uint2 lds_read_tr(const uint16_t* q) {
   return __builtin_bit_cast(uint2, v);
 }
 
-// Float16 rows are taken as they are: dy and x are matrix operands of their own type, the power matrix and the lags of
-// k two float16 pieces each (the power matrix three where the bfloat16 form has three), the largest value at 2^12, so that what
-// a float16 cannot hold is 2^-25 of it; the state part stays in bfloat16 pieces, whose range a state needs.  R and X are 2^12 times
-// themselves, a scale that Qd and the row's reductions take back; dx is scaled with k's largest lag, undone where it is
-// rounded.  With rows as bfloat16 pieces three launches (four where third pieces are) added up what one gives now:
-// backward of 1024 x 35840 385 / 77 us, 4096 x 32768 1315 / 275, 4 x 2048 x 5001 649 / 120, 2 x 512 x 759 100 / 37.
-constexpr float kPowScale = 4096.f;
+// Float16 rows are taken as they are: dy and x are matrix operands of their own type, the power matrix two float16 pieces
+// (three where the bfloat16 form has three).  Powers are at most 1; brought to 2^15 they have 22 (33) bits there and lose
+// nothing above 2^-40, which a float16 dx does not resolve (dy c 2^-40 is its last place where dy c is its largest).  The
+// lags of k and the state part stay in bfloat16 pieces, whose range they need: omega stands on the lag at zero and may be any
+// multiple of the others.  So the product K^T DY takes dy in two bfloat16 pieces too, split where it is multiplied.  R
+// and X are 2^15 times themselves, a scale that Qd and the row's reductions take back.  With rows as bfloat16 pieces three
+// launches (four where third pieces are) added up what one gives now: backward of 1024 x 35840 400 / 87 us, 4096 x 32768
+// 1334 / 296, 4 x 2048 x 5001 667 / 141, 2 x 512 x 759 82 / 20.  (The lags as two float16 pieces too, scaled with the largest: 84,
+// 281, 133, 19.5, but a lag at 2^-20 of omega had 17 bits and one at 2^-26 11.)
+constexpr float kPowScale = 32768.f;
+// eight 16-bit steps as bfloat16 pieces, whose sum they are exactly
+template <int DT>
+struct DyPieces {
+  static constexpr int XP = DT == MEGA_F16 ? 2 : 1;
+  u32x4 pc[XP];
+  __device__ __forceinline__ explicit DyPieces(const XOp<MEGA_BF16>& steps) {
+    const u32x4 raw = steps.pc[0];
+    if constexpr (DT == MEGA_F16) {
+      float v[8];
+      unpack8<MEGA_F16>(make_uint4(raw[0], raw[1], raw[2], raw[3]), v);
+      split8(v, pc[0], pc[1]);
+    } else {
+      pc[0] = raw;
+    }
+  }
+};
 struct BwdSmem {
   u32x4 aop[kBwdBlocks][2][kWave];       // operand blocks, two pieces
   // row c: (R, R') at the start of chunk c of the segment.  A wave's own 32 rows double as its
@@ -1065,7 +1084,6 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
 
   // scan multipliers of this thread's mode: over a chunk, a sub-segment, a wave's chunks
   cf qT{0.f, 0.f}, q1{0.f, 0.f};
-  float unscale = 1.f;  // H16: of dx
   int cur = 0, par = 0;
   RowParams rp = fetch_params(blockIdx.x);
 
@@ -1110,13 +1128,6 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       qT = sm.pw[9][sn];
     }
     __syncthreads();
-    float kscale = 1.f;  // of K and with it of dx
-    if constexpr (H16) {
-      const float most = wave_max(fabsf(klocal[lane]));
-      const int up = most > 0.f && most < INFINITY ? min(100, max(-100, 13 - __builtin_amdgcn_frexp_expf(most))) : 0;
-      kscale = ldexpf(1.f, up);
-      unscale = ldexpf(1.f, -up);
-    }
     for (int item = tid; item < kBwdBlocks * kWave; item += kThreads) {
       const int blk = item >> 6, ln = item & 63, rr = ln & 31, gg = ln >> 5;
       float v[8];
@@ -1135,7 +1146,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
         for (int e = 0; e < 8; ++e) {
           const int lag = o - rr + 8 * gg + e;
           const float kv = klocal[lag >= 0 ? lag : 0];  // read, then masked: no branch around the load
-          v[e] = lag >= 0 ? (H16 ? kscale * kv : kv) : 0.f;
+          v[e] = lag >= 0 ? kv : 0.f;
         }
       } else {
         const int jt = (blk - 12) >> 1, s2 = (blk - 12) & 1, j = 32 * jt + rr;
@@ -1145,11 +1156,11 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
           const cf c = cf{sm.pn[n] * sm.gn[n].x, sm.pn[n] * sm.gn[n].y};
           const cf w = cmul(c, qp[n][kT - j]);
           v[e] = (m & 1) ? -w.y : w.x;
-          if (H16) v[e] *= kscale / kPowScale;
+          if (H16) v[e] *= 1.f / kPowScale;
         }
       }
       u32x4 hi, lo, third;
-      if (H16 && blk < 12) split8_f16<FINE>(v, hi, lo, third);
+      if (H16 && blk < 8) split8_f16<FINE>(v, hi, lo, third);
       else split8(v, hi, lo);
       if (FINE && !H16) third = split8_third(v, hi, lo);
       sm.aop[blk][0][ln] = hi;
@@ -1157,7 +1168,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       if constexpr (FINE)
         if (blk < 8) (blk < 4 ? sm.third[blk] : passed[blk - 4])[ln] = third;
     }
-    if constexpr (FINE && !H16) fill_thirds<false>(sm.kthird, klocal, tid);
+    if constexpr (FINE) fill_thirds<false>(sm.kthird, klocal, tid);
 #pragma unroll
     for (int t = 0; t < 3; ++t)
 #pragma unroll
@@ -1519,9 +1530,10 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
           for (int s = 2 * jt; s < 4; ++s) {
             u32x4 a[2];
             load_block(8 + s - 2 * jt, a, lane);
-            acc = mfma16<DT>(a[1], db[s].pc[0], mfma16<DT>(a[0], db[s].pc[0], acc));
-            // (block b: lags 16 b - r + 8 g + e)
-            if constexpr (FINE && !H16) acc = mfma_bf16(read_thirds(sm.kthird, 16 * (s - 2 * jt) - r + 8 * g + 31), db[s].pc[0], acc);
+            const DyPieces<DT> d(db[s]);
+            acc = mma_split<DyPieces<DT>::XP, true>(a, d.pc, acc);
+            // (block b: lags 16 b - r + 8 g + e; of two-piece steps the third pieces' product with the second, 2^-26, is left out)
+            if constexpr (FINE) acc = mfma_bf16(read_thirds(sm.kthird, 16 * (s - 2 * jt) - r + 8 * g + 31), d.pc[0], acc);
           }
 #pragma unroll
           for (int s2 = 0; s2 < 2; ++s2) {
@@ -1529,9 +1541,6 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
             load_block(12 + 2 * jt + s2, a, lane);
             acc = mma_split<2, FINE>(a, hb[s2], acc);
           }
-          if constexpr (H16)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[i] *= unscale;
 #pragma unroll
           for (int pr = 0; pr < 2; ++pr) {
             if constexpr (DX32) {
