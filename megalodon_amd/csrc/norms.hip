@@ -226,8 +226,8 @@ __global__ __launch_bounds__(kThreads) void norm_bwd_vec_kernel(NormParams p) {
 // D = 512 W: a workgroup of W waves takes kRowsAtOnce rows at a time, a lane the same eight columns of each.  The column sums
 // stay in its registers from the first row to the last (16 instead of D / 32 of a wave that owns a row, which at D = 4096
 // left one wave per SIMD) and need no reduction over the workgroup; the row sums meet in LDS, one barrier for the rows at
-// once, while the next rows are on their way.  LayerNorm backward, with a wave to a row / so: 32768 x 4096 237 / 176 us,
-// 4084 x 2048 34.7 / 14.9, 4096 x 1024 15.1 / 12.0; RMSNorm 165 / 161, 16.3 / 13.5, 10.2 / 10.9.
+// once, while the next rows are on their way.  LayerNorm backward, with a wave to a row / so: 32768 x 4096 239 / 175 us,
+// 4096 x 2048 38.9 / 19.2, 4096 x 1024 20.9 / 15.2; RMSNorm 165 / 161, 21.1 / 16.5, 13.8 / 11.9 (see by_columns).
 constexpr int kRowsAtOnce = 4;
 template <int DT, int W, bool RMS>
 __global__ __launch_bounds__(W * kWave) void norm_bwd_columns_kernel(NormParams p) {
@@ -730,6 +730,20 @@ int groups_for(int64_t rows, int rows_per_group) {
   return static_cast<int>(g < 1 ? 1 : (g > kMaxGroups ? kMaxGroups : g));
 }
 
+// Where the backward by columns is ahead of a row to a wave: with parameter gradients, whose sums over a workgroup's waves
+// it does without.  Without them it only waits at its barriers (8192 x 1024 16.2 us / 9.1, 1500 x 512 4.5 / 2.5).  Its rows
+// come in passes of 2048, which cost the same half full.  By columns / a row to a wave:
+//   LayerNorm, 512   100 rows 6.4 / 6.7, 2048 9.0 / 9.4, 3000 11.3 / 11.0, 4096 11.9 / 13.1, 4500 14.1 / 13.2, 8192 17.6 / 14.6
+//   RMSNorm, 512     100 5.9 / 4.8, 4096 10.1 / 9.4, 16384 19.0 / 14.6
+//   RMSNorm, 1024    1000 8.0 / 7.2, 2300 11.0 / 10.3, 3000 11.1 / 11.5, 4096 11.9 / 13.8, 5000 14.3 / 14.8, 5500 14.9 / 14.6, 7000 17.6 / 15.4
+//   RMSNorm, 2048    1531 11.0 / 13.1, 6000 19.7 / 24.3, 12000 30.3 / 32.0, 14000 36.9 / 35.3, 32768 86.3 / 83.3
+constexpr bool by_columns(bool rms, bool affine, int nch, int64_t rows) {
+  if (!affine) return false;
+  if (nch == 1) return !rms && (rows <= 2048 || (rows > 3200 && rows <= 4096));
+  if (!rms || nch == 8) return true;
+  return nch == 2 ? rows > 2800 && rows <= 5200 : rows <= 12288;
+}
+
 // Workgroups of the kernel by columns: each adds a row of partial sums that is written and read again, so more than 512 only
 // where each has sixteen rows.
 int column_groups(int64_t rows) {
@@ -738,15 +752,16 @@ int column_groups(int64_t rows) {
 }
 
 template <int DT, bool RMS, bool BWD>
-int launch_vec(const NormParams& p, Shape sh, int groups, hipStream_t s) {
+int launch_vec(const NormParams& p, Shape sh, bool columns, int groups, hipStream_t s) {
   const size_t lds = BWD && p.part_w ? static_cast<size_t>(p.D) * (RMS ? 1 : 2) * sizeof(float) : 0;
 #define MEGA_NORM(LPR, NCH)                                                                  \
   if (sh.lpr == LPR && sh.nch == NCH) {                                                      \
-    if constexpr (BWD && LPR == kWave)                                                       \
-      norm_bwd_columns_kernel<DT, NCH, RMS><<<groups, NCH * kWave, 0, s>>>(p);               \
-    else if constexpr (BWD)                                                                  \
-      norm_bwd_vec_kernel<DT, LPR, NCH, RMS><<<groups, kThreads, lds, s>>>(p);               \
-    else                                                                                     \
+    if constexpr (BWD) {                                                                     \
+      if (LPR == kWave && columns)                                                           \
+        norm_bwd_columns_kernel<DT, NCH, RMS><<<groups, NCH * kWave, 0, s>>>(p);             \
+      else                                                                                   \
+        norm_bwd_vec_kernel<DT, LPR, NCH, RMS><<<groups, kThreads, lds, s>>>(p);             \
+    } else                                                                                   \
       norm_fwd_vec_kernel<DT, LPR, NCH, RMS><<<groups, kThreads, 0, s>>>(p);                 \
   }
   MEGA_NORM(64, 1) MEGA_NORM(64, 2) MEGA_NORM(64, 4) MEGA_NORM(64, 8)
@@ -763,7 +778,7 @@ int run_fwd(const NormParams& p, int dtype, hipStream_t s) {
     if (sh.lpr) {
       const int rpg = kWaves * (kWave / sh.lpr);
       const int64_t g = (p.rows + rpg - 1) / rpg;
-      return launch_vec<DT, RMS, false>(p, sh, static_cast<int>(g > 16384 ? 16384 : g), s);
+      return launch_vec<DT, RMS, false>(p, sh, false, static_cast<int>(g > 16384 ? 16384 : g), s);
     }
   }
   const int64_t g = (p.rows + kWaves - 1) / kWaves;
@@ -813,13 +828,14 @@ static int run_bwd(NormParams p, int dtype, void* dweight, void* dbias, float* w
   const bool affine = dweight != nullptr;
   const Shape sh = vec_shape(dtype, p.D, p);
   const int rpg = sh.lpr ? kWaves * (kWave / sh.lpr) : kWaves;
-  const int groups = sh.lpr == kWave ? column_groups(p.rows) : groups_for(p.rows, rpg);
+  const bool columns = sh.lpr == kWave && by_columns(RMS, affine, sh.nch, p.rows);
+  const int groups = columns ? column_groups(p.rows) : groups_for(p.rows, rpg);
   p.part_w = affine ? ws : nullptr;
   p.part_b = (affine && !RMS && dbias) ? ws + static_cast<int64_t>(kMaxGroups) * p.D : nullptr;
   bool done = false;
   if constexpr (DT != MEGA_F32) {
     if (sh.lpr) {
-      int rc = launch_vec<DT, RMS, true>(p, sh, groups, s);
+      int rc = launch_vec<DT, RMS, true>(p, sh, columns, groups, s);
       if (rc != MEGA_OK) return rc;
       done = true;
     }

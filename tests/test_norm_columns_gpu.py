@@ -1,5 +1,6 @@
 """The norms' backward by columns (widths 512, 1024, 2048, 4096 in 16 bits): row counts around the four rows of a pass, the
-workgroups of a launch and its limits, with and without affine parameters.
+workgroups of a launch and its limits, with and without affine parameters, and both sides of the lines to the kernel that takes
+a row to a wave.
 
 Bounds: dx is rounded once to the element type (2^-9 in bfloat16, 2^-12 in float16, of the largest values: 4e-3 / 5e-4 of
 the 2-norm); the parameters' gradients are float32 sums rounded once."""
@@ -15,7 +16,10 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("rms", [False, True])
 @pytest.mark.parametrize("rows,D,affine", [(1, 512, "both"), (3, 1024, "both"), (4, 2048, "weight"), (5, 4096, "both"),
                                            (2047, 512, "none"), (2049, 1024, "both"), (2053, 2048, "both"),
-                                           (8193, 512, "both"), (16389, 1024, "weight"), (4101, 4096, "none")])
+                                           (8193, 512, "both"), (16389, 1024, "weight"), (4101, 4096, "none"),
+                                           (2048, 512, "both"), (2049, 512, "both"), (3201, 512, "both"), (4097, 512, "weight"),
+                                           (2800, 1024, "both"), (2801, 1024, "weight"), (5201, 1024, "both"),
+                                           (12288, 2048, "both"), (12289, 2048, "both"), (5, 1024, "none"), (7, 2048, "none")])
 def test_backward_matches_float64(rows, D, affine, rms, dtype, bar):
     gen = torch.Generator("cuda").manual_seed(rows + D)
     rand = lambda *s: torch.randn(*s, generator=gen, device="cuda").to(dtype)
