@@ -49,17 +49,21 @@ __global__ __launch_bounds__(kThreads) void norm_fwd_vec_kernel(NormParams p) {
   uint16_t* y = static_cast<uint16_t*>(p.y);
   const float inv_d = 1.f / static_cast<float>(p.D);
   // weight and bias stay packed (one register per element pair)
-  // the row's pieces are requested a row ahead, the first before the weights (32768 x 4096 100 us, 94 so; 4084 x 2048
-  // LayerNorm 7.7, 7.1)
+  // A wave has one row up to 65536 rows of them, so what counts beside its chain of loads is how many waves there are: the
+  // next row is not asked for before this one has left its registers (LayerNorm at width 4096 200 of them so, two waves per
+  // SIMD, now 166: 4096 rows 15.1 us, now 13.4).  Wide rows are asked for in front of the weights, narrow ones
+  // behind them, in us: RMSNorm 4096 x 4096 11.3 / 11.6, 32768 x 4096 92.9 / 96.0 (99.7 with a wait for each piece of the
+  // weights), 16384 x 1024 11.2 / 11.8, but 16384 x 512 6.2 / 5.8; LayerNorm 4096 x 2048 7.1 / 7.3, but 16384 x 1024 12.9 / 12.1.
+  constexpr bool kRowFirst = NCH >= 4 || (RMS && NCH == 2);
   const int64_t step = static_cast<int64_t>(gridDim.x) * kWaves * RPW;
   int64_t row = (static_cast<int64_t>(blockIdx.x) * kWaves + wave) * RPW + slot;
-  uint4 next[NCH];
+  uint4 piece[NCH];
   auto request = [&](int64_t at) {  // rows behind the last: the last one again, unused
     const uint16_t* src = x + (at < p.rows ? at : p.rows - 1) * p.D;
 #pragma unroll
-    for (int i = 0; i < NCH; ++i) next[i] = *reinterpret_cast<const uint4*>(src + (lr + LPR * i) * 8);
+    for (int i = 0; i < NCH; ++i) piece[i] = *reinterpret_cast<const uint4*>(src + (lr + LPR * i) * 8);
   };
-  request(row);
+  if (kRowFirst) request(row);
   uint4 gq[NCH], bq[NCH];
 #pragma unroll
   for (int i = 0; i < NCH; ++i) gq[i] = bq[i] = make_uint4(0, 0, 0, 0);
@@ -72,15 +76,15 @@ __global__ __launch_bounds__(kThreads) void norm_fwd_vec_kernel(NormParams p) {
     for (int i = 0; i < NCH; ++i) bq[i] = reinterpret_cast<const uint4*>(p.bias)[lr + LPR * i];
   for (; row - slot < p.rows; row += step) {
     const bool live = row < p.rows;
+    if (!kRowFirst) request(row);
     float v[NCH][8];
     float s = 0.f;
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
-      unpack8<DT>(next[i], v[i]);
+      unpack8<DT>(piece[i], v[i]);
 #pragma unroll
       for (int e = 0; e < 8; ++e) s += RMS ? v[i][e] * v[i][e] : v[i][e];
     }
-    if (row - slot + step < p.rows) request(row + step);
     s = group_sum<LPR>(s) * inv_d;
     float mu = 0.f, var = s;
     if (!RMS) {
@@ -115,6 +119,7 @@ __global__ __launch_bounds__(kThreads) void norm_fwd_vec_kernel(NormParams p) {
         if (!RMS) p.mean[row] = mu;
       }
     }
+    if (kRowFirst && row - slot + step < p.rows) request(row + step);
   }
 }
 
