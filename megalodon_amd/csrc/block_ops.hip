@@ -62,13 +62,15 @@ __global__ __launch_bounds__(kThreads) void transpose16_kernel(const uint16_t* i
         v[pass] = make_uint4(p[0], p[1], p[2], p[3]);
       }
     }
-  } else {
+  } else if (!WHOLE && c < C) {
+    // (columns behind the last: the last one again, never stored.  A branch and a wait to each of these, one workgroup
+    // in 32 held up the rest: 3001 x 4095 16.5 us, 11.5 so)
 #pragma unroll
     for (int pass = 0; pass < 8; ++pass) {
-      const uint16_t* from = src + static_cast<int64_t>(min(r0 + q + 16 * pass, R - 1)) * C + c;
+      const uint16_t* from = src + static_cast<int64_t>(min(r0 + q + 16 * pass, R - 1)) * C;
       uint32_t e[8];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) e[k] = !WHOLE && c + k < C ? from[k] : 0u;
+      for (int k = 0; k < 8; ++k) e[k] = from[min(c + k, C - 1)];
       v[pass] = make_uint4(e[0] | e[1] << 16, e[2] | e[3] << 16, e[4] | e[5] << 16, e[6] | e[7] << 16);
     }
   }
@@ -77,9 +79,10 @@ __global__ __launch_bounds__(kThreads) void transpose16_kernel(const uint16_t* i
     const int rl = q + 16 * pass;
     const uint32_t u[4] = {v[pass].x, v[pass].y, v[pass].z, v[pass].w};
     const int w = ((rl >> 1) ^ (m << 2)) * 2 + (rl & 1);
+    if (c < C)
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-      t16[(8 * m + k) * kTT + w] = static_cast<uint16_t>(k & 1 ? u[k >> 1] >> 16 : u[k >> 1] & 0xffffu);
+      for (int k = 0; k < 8; ++k)
+        t16[(8 * m + k) * kTT + w] = static_cast<uint16_t>(k & 1 ? u[k >> 1] >> 16 : u[k >> 1] & 0xffffu);
   }
   __syncthreads();
   // store: thread (q, m) writes rows r0 + 8m .. +7 of output row c0 + q + 16 * pass
