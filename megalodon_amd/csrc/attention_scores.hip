@@ -600,18 +600,36 @@ int launch_probs_short(ProbsParams p, hipStream_t s) {
 
 // How many blocks of 32 rows a CU, in eighths, the short-row kernel takes.  It reads a block's keys anew for every block, so
 // its time grows with the blocks and with the head's width, while the other one's is its longest row block's until the chip
-// is full.  The operator's forward with a value head of 64, in us, the short-row kernel / the other, at blocks a CU:
-//   width 64:  256 keys 4.0 21 / 26, 5.0 27 / 26; 512 keys 5.0 33 / 37, 6.0 36 / 35; 1500 keys 5.0 70 / 81, 6.1 84 / 83; 4096 keys 5.0
-//              142 / 165, 6.0 173 / 172
-//   width 128: 256 keys 3.0 22 / 26, 3.4 28 / 24; 512 keys 4.0 35 / 37, 5.0 43 / 38; 1500 keys 4.0 77 / 87, 5.0 91 / 90; 4096 keys 4.0
-//              156 / 171, 5.0 200 / 183
-//   width 256: 256 keys 1.5 26 / 28, 2.5 35 / 30; 512 keys 2.0 34 / 43, 2.5 44 / 43; 1024 keys 2.9 64 / 66, 3.4 78 / 68; 2048 keys 3.5
-//              108 / 117, 5.0 147 / 123; 4096 keys 3.0 198 / 214, 3.5 228 / 218
-// (three blocks a CU for all of them before.)
-constexpr int short_rows(int H1, int keys) {
-  if (H1 == 64) return keys <= 384 ? 32 : 44;
-  if (H1 == 128) return keys <= 384 ? 24 : 32;
-  return keys <= 384 ? 12 : keys <= 768 ? 17 : keys <= 1280 ? 24 : 26;
+// is full; keys that a causal block does not see are left out by both, but only the other one waits for its longest.  The
+// operator's forward with a value head of 64, time of the other kernel over the short-row kernel's, at blocks a CU:
+//   causal squares  width 64:  256 keys 4.0 1.19, 5.0 0.96; 512 keys 5.0 1.13, 6.0 1.02; 1500 keys 5.0 1.15, 5.9 1.11; 4096 keys 5.5 1.07, 6.0 0.98
+//                   width 128: 256 keys 3.0 1.13, 3.3 0.96; 512 keys 4.0 1.07, 4.5 0.93; 1500 keys 3.9 1.20, 5.0 0.99; 4096 keys 4.0 1.08, 4.5 0.99
+//                   width 256: 100 keys 1.3 1.04, 1.5 0.94; 256 keys 2.0 1.08, 2.3 0.83; 512 keys 2.0 1.27, 2.3 0.96; 700 keys 3.0 1.02, 3.2 0.84; 2048
+//                              keys 3.3 1.14, 4.5 0.89; 4096 keys 3.0 1.08, 3.5 0.95
+//   causal, more keys than rows (the first rows see most of them)
+//                   width 64:  256 x 1024 5.0 1.02, 5.5 0.93; 1024 x 1536 4.0 1.10, 5.0 0.97; 100 x 1500 5.5 1.24; 1024 x 2048 4.0 1.12, 4.5 0.97
+//                   width 128: 256 x 384 3.0 1.12, 3.3 0.95; 1024 x 2048 3.0 1.11, 3.3 0.95
+//                   width 256: 256 x 1024 2.0 1.16, 2.3 0.90; 1024 x 1280 3.0 1.03, 3.3 0.90
+//   without a mask  width 64:  256 keys 2.0 1.08, 3.0 0.91; 384 keys 4.0 1.08, 4.5 0.87; 512 keys 3.3 1.05, 3.5 0.94; 1024 keys 4.0 1.09, 5.5 0.92; 1500
+//                              keys 3.5 1.06, 4.0 0.99; 4096 keys 3.0 1.10, 3.5 0.89
+//                   width 128: 256 keys 2.0 1.00, 2.3 0.86; 1024 keys 3.0 1.05, 3.3 0.92; 4096 keys 2.0 1.18, 2.5 0.87
+//                   width 256: 256 keys 1.0 1.31, 1.3 0.89; 512 keys 2.0 0.99, 2.3 0.79; 1024 keys 2.0 1.09, 2.3 0.84; 4096 keys 1.0 1.61, 1.5 0.96
+// (three blocks a CU for all of them before; with the lines of causal squares for all of them, 3.5 blocks of 256 keys without
+// a mask at width 64 took 24.4 us instead of 19.9, 4 of 4096 at width 128 322 instead of 257.)
+constexpr int short_rows(int H1, int rows, int keys, bool causal) {
+  if (causal && rows == keys) {
+    if (H1 == 64) return keys <= 384 ? 32 : 44;
+    if (H1 == 128) return keys <= 384 ? 24 : 32;
+    return keys <= 128 ? 10 : keys <= 544 ? 16 : keys <= 1280 ? 24 : 26;
+  }
+  if (causal) {
+    if (H1 == 64) return rows <= 128 ? 44 : keys <= 1536 ? 40 : 32;
+    if (H1 == 128) return 24;
+    return keys > 1024 && 2 * rows >= keys ? 24 : 16;
+  }
+  if (H1 == 64) return keys <= 288 ? 24 : keys <= 384 ? 32 : keys <= 544 ? 26 : keys <= 1152 ? 40 : keys <= 1536 ? 28 : 24;
+  if (H1 == 128) return keys <= 288 || keys > 3072 ? 16 : 24;
+  return keys <= 288 || keys > 3072 ? 8 : 16;
 }
 
 template <int DT, int H1>
@@ -620,7 +638,8 @@ int launch_probs(const ProbsParams& p, hipStream_t s) {
   int dev = 0, cus = 0;
   MEGA_CHECK_HIP(hipGetDevice(&dev));
   MEGA_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  if (8 * static_cast<int64_t>(p.Z) * ((p.L1 + 31) / 32) <= static_cast<int64_t>(short_rows(H1, p.L2)) * cus) return launch_probs_short<DT, H1>(p, s);
+  if (8 * static_cast<int64_t>(p.Z) * ((p.L1 + 31) / 32) <= static_cast<int64_t>(short_rows(H1, p.L1, p.L2, p.causal)) * cus)
+    return launch_probs_short<DT, H1>(p, s);
   constexpr int KW = H1 >= 128 ? 128 : 64;
   const size_t lds = sizeof(uint16_t) * kRing * kKeys * KW;
   MEGA_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_probs_kernel<DT, H1>),
