@@ -58,6 +58,63 @@ template <int DT>
 __device__ __forceinline__ void st(void* base, int64_t i, float v) {
   Elem<DT>::store(static_cast<typename Elem<DT>::type*>(base) + i, v);
 }
+// uniform base + 32-bit unsigned byte offset (scalar-base addressing form)
+template <typename V>
+__device__ __forceinline__ V gld(const void* base, unsigned byte_off) {
+  return *reinterpret_cast<const V*>(static_cast<const char*>(base) + byte_off);
+}
+template <typename V>
+__device__ __forceinline__ void gst(void* base, unsigned byte_off, V v) {
+  *reinterpret_cast<V*>(static_cast<char*>(base) + byte_off) = v;
+}
+
+// A pair of adjacent elements as one 32/64-bit access.
+template <int DT> struct Pair;
+typedef float float2_any __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t u32_any __attribute__((aligned(2)));
+// at any element (by a cast to the typedef itself: as a template's argument, of gld, it would lose its alignment)
+__device__ __forceinline__ uint32_t load_u32_any(const void* base, unsigned off) {
+  return *reinterpret_cast<const u32_any*>(static_cast<const char*>(base) + off);
+}
+__device__ __forceinline__ void store_u32_any(void* base, unsigned off, uint32_t v) {
+  *reinterpret_cast<u32_any*>(static_cast<char*>(base) + off) = v;
+}
+template <> struct Pair<MEGA_F32> {
+  using type = float2;
+  static __device__ __forceinline__ type load_any(const void* base, unsigned off) {
+    const float2_any v = *reinterpret_cast<const float2_any*>(static_cast<const char*>(base) + off);
+    return make_float2(v.x, v.y);
+  }
+  static __device__ __forceinline__ void store_any(void* base, unsigned off, type v) {
+    *reinterpret_cast<float2_any*>(static_cast<char*>(base) + off) = float2_any{v.x, v.y};
+  }
+  static __device__ __forceinline__ void unpack(type v, float& lo, float& hi) { lo = v.x; hi = v.y; }
+  static __device__ __forceinline__ type pack(float lo, float hi) { return make_float2(lo, hi); }
+};
+template <> struct Pair<MEGA_BF16> {
+  using type = uint32_t;
+  static __device__ __forceinline__ type load_any(const void* base, unsigned off) { return load_u32_any(base, off); }
+  static __device__ __forceinline__ void store_any(void* base, unsigned off, type v) { store_u32_any(base, off, v); }
+  static __device__ __forceinline__ void unpack(type v, float& lo, float& hi) {
+    lo = __uint_as_float(v << 16);
+    hi = __uint_as_float(v & 0xffff0000u);
+  }
+  static __device__ __forceinline__ type pack(float lo, float hi) { return pack_bf16x2(lo, hi); }
+};
+template <> struct Pair<MEGA_F16> {
+  using type = uint32_t;
+  static __device__ __forceinline__ type load_any(const void* base, unsigned off) { return load_u32_any(base, off); }
+  static __device__ __forceinline__ void store_any(void* base, unsigned off, type v) { store_u32_any(base, off, v); }
+  static __device__ __forceinline__ void unpack(type v, float& lo, float& hi) {
+    lo = f16_bits_to_float(static_cast<uint16_t>(v & 0xffffu));
+    hi = f16_bits_to_float(static_cast<uint16_t>(v >> 16));
+  }
+  static __device__ __forceinline__ type pack(float lo, float hi) {
+    return static_cast<uint32_t>(float_to_f16_bits(lo)) |
+           (static_cast<uint32_t>(float_to_f16_bits(hi)) << 16);
+  }
+};
+
 }  // namespace
 
 #ifdef MEGA_FFTCONV_LOGM
@@ -183,54 +240,6 @@ int scratch_used(hipStream_t stream) {
     if (s.stream == stream && !s.pinned) MEGA_CHECK_HIP(hipEventRecord(s.done, stream));
   return MEGA_OK;
 }
-
-// uniform base + 32-bit unsigned byte offset (scalar-base addressing form)
-template <typename V>
-__device__ __forceinline__ V gld(const void* base, unsigned byte_off) {
-  return *reinterpret_cast<const V*>(static_cast<const char*>(base) + byte_off);
-}
-template <typename V>
-__device__ __forceinline__ void gst(void* base, unsigned byte_off, V v) {
-  *reinterpret_cast<V*>(static_cast<char*>(base) + byte_off) = v;
-}
-
-// A pair of adjacent elements as one 32/64-bit access.
-template <int DT> struct Pair;
-typedef float float2_any __attribute__((ext_vector_type(2), aligned(4)));
-typedef uint32_t u32_any __attribute__((aligned(2)));
-template <> struct Pair<MEGA_F32> {
-  using type = float2;
-  static __device__ __forceinline__ type load_any(const void* base, unsigned off) {
-    const float2_any v = gld<float2_any>(base, off);
-    return make_float2(v.x, v.y);
-  }
-  static __device__ __forceinline__ void store_any(void* base, unsigned off, type v) { gst<float2_any>(base, off, float2_any{v.x, v.y}); }
-  static __device__ __forceinline__ void unpack(type v, float& lo, float& hi) { lo = v.x; hi = v.y; }
-  static __device__ __forceinline__ type pack(float lo, float hi) { return make_float2(lo, hi); }
-};
-template <> struct Pair<MEGA_BF16> {
-  using type = uint32_t;
-  static __device__ __forceinline__ type load_any(const void* base, unsigned off) { return gld<u32_any>(base, off); }
-  static __device__ __forceinline__ void store_any(void* base, unsigned off, type v) { gst<u32_any>(base, off, v); }
-  static __device__ __forceinline__ void unpack(type v, float& lo, float& hi) {
-    lo = __uint_as_float(v << 16);
-    hi = __uint_as_float(v & 0xffff0000u);
-  }
-  static __device__ __forceinline__ type pack(float lo, float hi) { return pack_bf16x2(lo, hi); }
-};
-template <> struct Pair<MEGA_F16> {
-  using type = uint32_t;
-  static __device__ __forceinline__ type load_any(const void* base, unsigned off) { return gld<u32_any>(base, off); }
-  static __device__ __forceinline__ void store_any(void* base, unsigned off, type v) { gst<u32_any>(base, off, v); }
-  static __device__ __forceinline__ void unpack(type v, float& lo, float& hi) {
-    lo = f16_bits_to_float(static_cast<uint16_t>(v & 0xffffu));
-    hi = f16_bits_to_float(static_cast<uint16_t>(v >> 16));
-  }
-  static __device__ __forceinline__ type pack(float lo, float hi) {
-    return static_cast<uint32_t>(float_to_f16_bits(lo)) |
-           (static_cast<uint32_t>(float_to_f16_bits(hi)) << 16);
-  }
-};
 
 // The lane id, hidden from the optimiser: left alone it keeps the offsets of a row's 32 accesses in
 // registers from its load to its store, across both halves (with two waves per SIMD: 74 spilled).
