@@ -234,6 +234,7 @@ __global__ __launch_bounds__(kThreads) void norm_bwd_vec_kernel(NormParams p) {
 // once, while the next rows are on their way.  LayerNorm backward, with a wave to a row / so: 32768 x 4096 239 / 175 us,
 // 4096 x 2048 38.9 / 19.2, 4096 x 1024 20.9 / 15.2; RMSNorm 165 / 161, 21.1 / 16.5, 13.8 / 11.9 (see by_columns).
 constexpr int kRowsAtOnce = 4;
+typedef float float4_any __attribute__((ext_vector_type(4), aligned(4)));  // (a workspace is a caller's, at any float)
 template <int DT, int W, bool RMS>
 __global__ __launch_bounds__(W * kWave) void norm_bwd_columns_kernel(NormParams p) {
   constexpr int R = kRowsAtOnce;
@@ -317,9 +318,9 @@ __global__ __launch_bounds__(W * kWave) void norm_bwd_columns_kernel(NormParams 
   }
   if (p.part_w == nullptr) return;  // no affine parameters
   auto put = [&](float* part, const float (&a)[8]) {
-    float4* const to = reinterpret_cast<float4*>(part + static_cast<int64_t>(blockIdx.x) * p.D + col);
-    to[0] = make_float4(a[0], a[1], a[2], a[3]);
-    to[1] = make_float4(a[4], a[5], a[6], a[7]);
+    float4_any* const to = reinterpret_cast<float4_any*>(part + static_cast<int64_t>(blockIdx.x) * p.D + col);
+    to[0] = float4_any{a[0], a[1], a[2], a[3]};
+    to[1] = float4_any{a[4], a[5], a[6], a[7]};
   };
   put(p.part_w, aw);
   if (!RMS && p.part_b) put(p.part_b, ab);

@@ -7,6 +7,7 @@ the 2-norm); the parameters' gradients are float32 sums rounded once."""
 import pytest
 import torch
 
+from megalodon_amd import _lib
 from megalodon_amd import extension as ext
 
 pytestmark = pytest.mark.gpu
@@ -41,3 +42,19 @@ def test_backward_matches_float64(rows, D, affine, rms, dtype, bar):
         assert err(dw, wd.grad) <= bar
     if b is not None:
         assert err(db, dy.double().sum(0)) <= bar
+
+
+def test_a_workspace_at_any_float():
+    rows, D = 100, 2048
+    gen = torch.Generator("cuda").manual_seed(7)
+    x, dy, w = (torch.randn(*s, generator=gen, device="cuda").bfloat16() for s in ((rows, D), (rows, D), (D,)))
+    _, mean, rstd = ext.layer_norm_fwd(x, w, w, 1e-5, False)
+    want = ext.layer_norm_bwd(dy, x, w, mean, rstd, False, True)
+    size = _lib.load().mega_layer_norm_workspace_bytes
+    size.restype = _lib.ctypes.c_int64
+    ws = torch.zeros(size(_lib.i64(rows), _lib.i64(D)) // 4 + 3, device="cuda")
+    got = [torch.empty_like(t) for t in want]
+    _lib.call("mega_layer_norm_bwd", *map(_lib.ptr, (dy, x, w, mean, rstd)), _lib.i32(_lib.dtype_code(x.dtype)), _lib.i64(rows), _lib.i64(D),
+              _lib.i32(0), *map(_lib.ptr, got), _lib.ptr(ws[1:]), _lib.stream_ptr(x.device))
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
