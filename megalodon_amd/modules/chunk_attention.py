@@ -17,6 +17,7 @@ from typing import Optional, Tuple
 import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
+from torch.nn.modules import module as nn_module
 
 from ..fused_ops import memory_efficient_dropout, swift_efficient_attention
 
@@ -109,6 +110,16 @@ class _InnerAttention(nn.Module):
             out = (prob @ vh).transpose(1, 2).contiguous()
         return out.reshape(batch, new_len, -1), carried
 
+    _own_forward = forward
+
     def extra_repr(self) -> str:
         return (f"heads={self.n_heads}, z_head_dim={self.z_head_dim}, v_head_dim={self.v_head_dim}, "
                 f"chunk={self.chunk_size}")
+
+
+def takes_fresh(module) -> bool:
+    """Whether `module(..., fresh=True)` hands its tensors to `_InnerAttention`'s own forward and to nobody else: a hook may keep
+    them, and a forward in its place need not know of the argument."""
+    return (type(module) is _InnerAttention and _InnerAttention.forward is _InnerAttention._own_forward
+            and "forward" not in module.__dict__ and not module._forward_hooks and not module._forward_pre_hooks
+            and not nn_module._global_forward_hooks and not nn_module._global_forward_pre_hooks)

@@ -20,7 +20,7 @@ from torch.nn import Parameter
 from .. import extension as megalodon_ops
 from ..fused_ops import memory_efficient_dropout, qk_norm_rotary, silu_mul, transpose_last2
 from .block_decode import decode_step
-from .chunk_attention import _InnerAttention
+from .chunk_attention import _InnerAttention, takes_fresh
 from .complex_exponential_moving_average import MultiHeadComplexEMA
 from .linear import Linear, linear_group
 from .layer_norm import FusedRMSNorm
@@ -111,8 +111,8 @@ class MovingAverageGatedAttention(nn.Module):
         # B x L x E
         v = F.silu(self.wv(out_tsn))
 
-        # (k and v are made here, and nobody else holds them: a new cache may keep them as they are)
-        fresh = {"fresh": True} if type(self.inner_attention) is _InnerAttention and not v.requires_grad and not k.requires_grad else {}
+        # (k and v are made here: where nobody is shown them on the way, nobody else holds them and a new cache may keep them)
+        fresh = {"fresh": True} if cache_attn is not None and not v.requires_grad and not k.requires_grad and takes_fresh(self.inner_attention) else {}
         attn, cache_attn = self.inner_attention(q.contiguous(), k.contiguous(), v, mask, freqs_cis, cache_attn, **fresh)
         # attn * silu(r) in one pass
         attn = memory_efficient_dropout(silu_mul(r, attn), self.hidden_dropout, self.training)

@@ -3,7 +3,7 @@ a tensor that the caller has made for the call is taken as it is."""
 import pytest
 import torch
 
-from megalodon_amd.modules.chunk_attention import _InnerAttention
+from megalodon_amd.modules.chunk_attention import _InnerAttention, takes_fresh
 
 
 def _empty(*shape, dtype=torch.float32):
@@ -38,3 +38,34 @@ def test_other_shapes_are_refused_as_before(shape):
         torch.cat((_empty(*shape), NEW), dim=1)
     with pytest.raises(RuntimeError):
         _InnerAttention._joined(_empty(*shape), NEW, True)
+
+
+def _inner():
+    return _InnerAttention(4, 8, 2, 16, 0.0, None)
+
+
+class _Sub(_InnerAttention):
+    pass
+
+
+def test_who_is_told():
+    assert takes_fresh(_inner())
+    assert not takes_fresh(_Sub(4, 8, 2, 16, 0.0, None)) and not takes_fresh(torch.nn.Identity())
+    m = _inner()
+    m.forward = lambda q, k, v, mask, freqs, cache=None: (v, None)
+    assert not takes_fresh(m)
+    for listen in ("register_forward_hook", "register_forward_pre_hook"):
+        m = _inner()
+        handle = getattr(m, listen)(lambda *a: None)
+        assert not takes_fresh(m)
+        handle.remove()
+        assert takes_fresh(m)
+        handle = getattr(torch.nn.modules.module, listen.replace("register", "register_module"))(lambda *a: None)
+        assert not takes_fresh(m)
+        handle.remove()
+        assert takes_fresh(m)
+
+
+def test_a_forward_in_the_class_place_is_not_told(monkeypatch):
+    monkeypatch.setattr(_InnerAttention, "forward", lambda self, q, k, v, mask, freqs, cache=None: (v, None))
+    assert not takes_fresh(_inner())
