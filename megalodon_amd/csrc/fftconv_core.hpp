@@ -38,8 +38,6 @@
 #else
 #define MEGA_HD inline
 #endif
-// keeps the compiler from issuing every table load of a pass at once
-#define MEGA_MEM_FENCE() asm volatile("" ::: "memory")
 
 namespace mega {
 namespace fftc {
@@ -616,55 +614,6 @@ template <int H>
 MEGA_HD constexpr int out_pos(int n2) {
   return H == 0 ? bitrev<5>(n2) : shifted_dit32_pos(n2);
 }
-
-#if !defined(__HIPCC__)
-// On the CPU also the passes one by one as textbooks have them, each leaving its outputs with the twiddles that the next
-// one's inputs take: a pass above with those of its inputs moved.
-MEGA_HD void turn(float& xr, float& xi, double num, double den) {  // times exp(-2 pi i num / den)
-  const double a = -6.283185307179586476925286766559 * (__builtin_fmod(num, den) / den);
-  const c32 v = cmulv(c32{xr, xi}, c32{static_cast<float>(__builtin_cos(a)), static_cast<float>(__builtin_sin(a))});
-  xr = v.x;
-  xi = v.y;
-}
-template <int LOGM, int H>
-MEGA_HD void fwd_pass1(float* re, float* im, int t, const Tables&) {
-  fwd_first<H>(re, im);
-  for (int j = 0; j < 32; ++j) turn(re[j], im[j], H * t, 2.0 * Cfg<LOGM>::M);
-}
-template <int LOGM>
-MEGA_HD void fwd_pass2(float* re, float* im, int t, const Tables& tb) {
-  using C = Cfg<LOGM>;
-  fwd_second(re, im, second_twiddles<LOGM, 0>(t, tb));
-  for (int a1 = 0; a1 < 32; ++a1) {
-    const int at = bitrev<5>(a1);
-    turn(re[at], im[at], static_cast<double>(t % C::R3) * (t / C::R3 + 32 * a1), C::M);
-  }
-}
-template <int LOGM>
-MEGA_HD void fwd_pass3(float* re, float* im) {
-  constexpr int R3 = Cfg<LOGM>::R3;
-  for (int g = 0; g < 32; g += R3) transform<R3>(re + g, im + g);
-}
-template <int LOGM, int H>
-MEGA_HD void inv_pass3(float* re, float* im, int, const Tables&) {
-  inv_third<LOGM>(re, im);
-}
-template <int LOGM, int H>
-MEGA_HD void inv_pass2(float* re, float* im, int t, const Tables& tb) {
-  using C = Cfg<LOGM>;
-  inv_second(re, im, inv_second_twiddles<LOGM>(t, tb));
-  for (int n1 = 0; n1 < 32; ++n1) {
-    const int at = bitrev<5>(n1);
-    turn(re[at], im[at], -static_cast<double>(n1 * C::R3 + t % C::R3) * (2 * (t / C::R3) + H), 2.0 * C::M);
-  }
-}
-template <int H>
-MEGA_HD void inv_pass1(float* re, float* im) {
-  const c32 one{1.f, 0.f};
-  if (H == 0) transform<32>(im, re);
-  else odd_transform32_w(im, re, Powers{one, one, one}, one);
-}
-#endif
 
 // How a launch shares out its rows: how many rows of a channel a group takes, chosen for the shortest line of
 // transforms, in halves of one, that a workgroup slot gets (5 for a pair of rows, 3 for a row alone).  `bound`: a channel's sum

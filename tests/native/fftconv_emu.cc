@@ -1,6 +1,7 @@
-// CPU emulation of the register-FFT convolution engine (fftconv_core.hpp):
-// the lanes of one workgroup are run one after another, phase by phase, with
-// LDS as a plain array.  Built by tests/test_fftconv_engine_cpu.py with g++.
+// CPU emulation of the convolution engine with the passes as the kernels run them (twiddles asked for a pass
+// ahead, taken into the butterflies): the lanes of one workgroup one after another, LDS as a plain
+// array.  Built by tests/test_fftconv_engine_cpu.py and
+// tests/test_fftconv_engine_passes_cpu.py with g++.
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -24,26 +25,26 @@ template <int LOGM, int H>
 static void forward(std::vector<float>& re, std::vector<float>& im, std::vector<float>& lre,
                     std::vector<float>& lim, const Tables& tb) {
   using C = Cfg<LOGM>;
-  for (int t = 0; t < C::T; ++t) fwd_pass1<LOGM, H>(&re[t * 32], &im[t * 32], t, tb);
+  for (int t = 0; t < C::T; ++t) fwd_first<H>(&re[t * 32], &im[t * 32]);
   for (int t = 0; t < C::T; ++t) x1_write<LOGM>(&re[t * 32], &im[t * 32], t, lre.data(), lim.data());
   for (int t = 0; t < C::T; ++t) x1_read<LOGM>(&re[t * 32], &im[t * 32], t, lre.data(), lim.data());
-  for (int t = 0; t < C::T; ++t) fwd_pass2<LOGM>(&re[t * 32], &im[t * 32], t, tb);
+  for (int t = 0; t < C::T; ++t) fwd_second(&re[t * 32], &im[t * 32], second_twiddles<LOGM, H>(t, tb));
   for (int t = 0; t < C::T; ++t) x2_write<LOGM>(&re[t * 32], &im[t * 32], t, lre.data(), lim.data());
   for (int t = 0; t < C::T; ++t) x2_read<LOGM, H>(&re[t * 32], &im[t * 32], t, lre.data(), lim.data());
-  for (int t = 0; t < C::T; ++t) fwd_pass3<LOGM>(&re[t * 32], &im[t * 32]);
+  for (int t = 0; t < C::T; ++t) fwd_third<LOGM, H>(&re[t * 32], &im[t * 32], t, third_twiddles<LOGM, H>(t, tb));
 }
 
 template <int LOGM, int H>
 static void inverse(std::vector<float>& re, std::vector<float>& im, std::vector<float>& lre,
                     std::vector<float>& lim, const Tables& tb) {
   using C = Cfg<LOGM>;
-  for (int t = 0; t < C::T; ++t) inv_pass3<LOGM, H>(&re[t * 32], &im[t * 32], t, tb);
+  for (int t = 0; t < C::T; ++t) inv_third<LOGM>(&re[t * 32], &im[t * 32]);
   for (int t = 0; t < C::T; ++t) ix2_write<LOGM, H>(&re[t * 32], &im[t * 32], t, lre.data(), lim.data());
   for (int t = 0; t < C::T; ++t) ix2_read<LOGM>(&re[t * 32], &im[t * 32], t, lre.data(), lim.data());
-  for (int t = 0; t < C::T; ++t) inv_pass2<LOGM, H>(&re[t * 32], &im[t * 32], t, tb);
+  for (int t = 0; t < C::T; ++t) inv_second(&re[t * 32], &im[t * 32], inv_second_twiddles<LOGM>(t, tb));
   for (int t = 0; t < C::T; ++t) ix1_write<LOGM>(&re[t * 32], &im[t * 32], t, lre.data(), lim.data());
   for (int t = 0; t < C::T; ++t) ix1_read<LOGM>(&re[t * 32], &im[t * 32], t, lre.data(), lim.data());
-  for (int t = 0; t < C::T; ++t) inv_pass1<H>(&re[t * 32], &im[t * 32]);
+  for (int t = 0; t < C::T; ++t) inv_first<H>(&re[t * 32], &im[t * 32], inv_first_twiddles<H>(t, tb));
 }
 
 template <int LOGM>

@@ -1,4 +1,4 @@
-"""The convolution engine's passes as the kernels run them, on the CPU (tests/native/fftconv_passes_emu.cc), against
+"""The convolution engine's passes as the kernels run them, on the CPU (tests/native/fftconv_emu.cc), against
 numpy's float64 FFT.
 
 Bounds: a transform is log2 M <= 14 butterflies deep, each a rounding or two of 2^-24 beside a twiddle that is at most three
@@ -11,12 +11,12 @@ import subprocess
 import numpy as np
 import pytest
 
-SRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "fftconv_passes_emu.cc")
+SRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "fftconv_emu.cc")
 
 
 @pytest.fixture(scope="module")
 def emu(tmp_path_factory):
-    out = tmp_path_factory.mktemp("emu") / "libfftconv_passes_emu.so"
+    out = tmp_path_factory.mktemp("emu") / "libfftconv_emu.so"
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-o", str(out), SRC], check=True)
     return ctypes.CDLL(str(out))
 
