@@ -730,7 +730,8 @@ int mega_bench_stream_copy(const void* a, const void* b, void* out, int64_t byte
 /* mega_cema_scan_bwd / _wide for a caller that adds the parameter gradients up anyway (the layer): several
  * rows of a channel share a workgroup and leave one set of gradients.  dp (sets, D, N), dq and dgamma
  * likewise, domega (sets, D) with sets = mega_cema_layer_scan_sets(B, D, L).  bfloat16 dy and x; dx_mode 0: dx
- * bfloat16; 1: float32, or not written when NULL; 2: added to float32 dx.  dx_mode 3: dy, x and dx float16. */
+ * bfloat16; 1: float32, or not written when NULL; 2: added to float32 dx.  dx_mode 3: dy, x and dx float16, and
+ * |q| <= 1 (of larger ones the powers leave a float16). */
 int64_t mega_cema_layer_scan_sets(int64_t B, int64_t D, int64_t L);
 int mega_cema_layer_scan_bwd(const void* dy, const void* x, const float* p, const float* log_q,
                              const float* gamma, const float* omega, int64_t B, int64_t D,

@@ -1317,17 +1317,13 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       dp[row * N + n] = A.x * gm.x - A.y * gm.y;
       const cf t = cmul(Bq, cf{pp * gm.x, pp * gm.y});
       cf dqv{t.x, -t.y}, dgv{A.x * pp, -A.y * pp};
-      if (h0 != nullptr) {
+      if (!H16 && h0 != nullptr) {  // (float16 rows with a carried state go in pieces)
         // A carried state h0 adds b[t] = Re(gamma q^(t+1) h0) to the output (ema_parameters.cc:56-77).
         // With R0 = sum_t dy[t] q^t and R0' = dR0 / dq -- what the reverse scan has carried to the
         // start of the row -- its gradients are (ema_parameters.cc:158-188, PyTorch's convention)
         //   dgamma += conj(q h0 R0),  dq += conj(gamma h0 (R0 + q R0')),  dh0 = conj(gamma q R0)
         // (q R0' = 64 times what the scan has carried).
-        cf r0 = sm.carry[cur][0][n], r0d = sm.carry[cur][1][n];
-        if (H16) {
-          r0 = cf{r0.x / kPowScale, r0.y / kPowScale};
-          r0d = cf{r0d.x / kPowScale, r0d.y / kPowScale};
-        }
+        const cf r0 = sm.carry[cur][0][n], r0d = sm.carry[cur][1][n];
         const cf h = h0[row * N + n];
         const cf e1 = cmul(cmul(qq, h), r0);
         dgv.x += e1.x;
