@@ -51,10 +51,12 @@ __global__ __launch_bounds__(kThreads) void norm_fwd_vec_kernel(NormParams p) {
   // weight and bias stay packed (one register per element pair)
   // A wave has one row up to 65536 rows of them, so what counts beside its chain of loads is how many waves there are: the
   // next row is not asked for before this one has left its registers (LayerNorm at width 4096 200 of them so, two waves per
-  // SIMD, now 166: 4096 rows 15.1 us, now 13.4).  Wide rows are asked for in front of the weights, narrow ones
+  // SIMD, now a third: 4096 rows 15.1 us, now 13.5).  Wide rows are asked for in front of the weights, narrow ones
   // behind them, in us: RMSNorm 4096 x 4096 11.3 / 11.6, 32768 x 4096 92.9 / 96.0 (99.7 with a wait for each piece of the
-  // weights), 16384 x 1024 11.2 / 11.8, but 16384 x 512 6.2 / 5.8; LayerNorm 4096 x 2048 7.1 / 7.3, but 16384 x 1024 12.9 / 12.1.
+  // weights), 16384 x 1024 11.2 / 11.8, but 16384 x 512 6.2 / 5.8; LayerNorm 4096 x 2048 7.1 / 7.3, but 16384 x 1024 12.9 / 12.1 and, of few rows,
+  // 1531 x 4096 6.7 / 6.4, 2048 7.6 / 7.4, 8192 23.0 / 23.2, 32768 93.9 / 97.3.
   constexpr bool kRowFirst = NCH >= 4 || (RMS && NCH == 2);
+  const bool row_first = kRowFirst && (RMS || NCH < 8 || p.rows > 8192);
   const int64_t step = static_cast<int64_t>(gridDim.x) * kWaves * RPW;
   int64_t row = (static_cast<int64_t>(blockIdx.x) * kWaves + wave) * RPW + slot;
   uint4 piece[NCH];
@@ -63,7 +65,7 @@ __global__ __launch_bounds__(kThreads) void norm_fwd_vec_kernel(NormParams p) {
 #pragma unroll
     for (int i = 0; i < NCH; ++i) piece[i] = *reinterpret_cast<const uint4*>(src + (lr + LPR * i) * 8);
   };
-  if (kRowFirst) request(row);
+  if (row_first) request(row);
   uint4 gq[NCH], bq[NCH];
 #pragma unroll
   for (int i = 0; i < NCH; ++i) gq[i] = bq[i] = make_uint4(0, 0, 0, 0);
@@ -76,7 +78,7 @@ __global__ __launch_bounds__(kThreads) void norm_fwd_vec_kernel(NormParams p) {
     for (int i = 0; i < NCH; ++i) bq[i] = reinterpret_cast<const uint4*>(p.bias)[lr + LPR * i];
   for (; row - slot < p.rows; row += step) {
     const bool live = row < p.rows;
-    if (!kRowFirst) request(row);
+    if (!row_first) request(row);
     float v[NCH][8];
     float s = 0.f;
 #pragma unroll
@@ -119,7 +121,7 @@ __global__ __launch_bounds__(kThreads) void norm_fwd_vec_kernel(NormParams p) {
         if (!RMS) p.mean[row] = mu;
       }
     }
-    if (kRowFirst && row - slot + step < p.rows) request(row + step);
+    if (row_first && row - slot + step < p.rows) request(row + step);
   }
 }
 
