@@ -5,15 +5,19 @@
 // The step is bound by reading the block's weights once and moving the cached keys and
 // values once: at width 4096 the weights are 514 MB, and operator by operator a
 // step was 59 launches, 0.84 ms for one sequence and 4.1 ms for sixteen (1531 and
-// 3000 cached tokens).  Here it is seven launches, 0.151 and 0.50 ms, cut where a whole row is needed by everybody:
-//   1. step_kernel    TimestepNorm step, EMA state step, partial square sums of the row
-//   2. skinny_kernel  RMSNorm folded into z, r, h1; v = silu(...) straight into the new cache
+// 3000 cached tokens).  Here it is seven launches, nine above eight sequences, 0.123 and 0.49 ms, cut where a whole row is
+// needed by everybody:
+//   1. step_kernel    TimestepNorm step, EMA state step
+//   2. products       RMSNorm folded into z, r, h1; v = silu(...) straight into the new cache
 //   3. attend_kernel  q, k (norm, affine maps, rotary), one softmax part per split; the old keys and values
 //                     pass into the new cache as they are read, the new key joins them
 //   4. combine_kernel the parts put together, gate silu(r)
-//   5. skinny_kernel  wh2 + h1 + residual, partial moments of the row
-//   6. skinny_kernel  LayerNorm folded into fc1, fc3; silu(a) b
-//   7. skinny_kernel  fc2 + residual
+//   5. products       wh2 + h1 + residual
+//   6. products       LayerNorm folded into fc1, fc3; silu(a) b
+//   7. products       fc2 + residual
+// The products are rows_kernel's for few sequences, which normalises on the way, else rows_norm_kernel's and skinny_kernel's.
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace mega {
@@ -57,7 +61,6 @@ struct StepParams {
   uint16_t *tsn, *cema, *mean, *var;
   int64_t* count;
   float4* h_out;
-  float* squares;  // (B, D / 32): sum of squares of the stored EMA outputs
   int D, G, Dg;
   float eps;
 };
@@ -65,8 +68,7 @@ struct StepParams {
 template <int DT>
 __global__ __launch_bounds__(256) void step_kernel(const StepParams a) {
   using E = Elem<DT>;
-  __shared__ float part[4];
-  const int b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int b = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
   const int d0 = blockIdx.x * kStepChannels, g = d0 / a.Dg;
   const int d = d0 + (tid >> 3), m2 = tid & 7;  // modes 2 m2, 2 m2 + 1
   const int64_t hidx = (static_cast<int64_t>(b) * a.D + d) * (kModes / 2) + m2;
@@ -113,10 +115,6 @@ __global__ __launch_bounds__(256) void step_kernel(const StepParams a) {
     E::store(a.tsn + static_cast<int64_t>(b) * a.D + d, xn);
     E::store(a.cema + static_cast<int64_t>(b) * a.D + d, out);
   }
-  const float sq = wave_sum(m2 == 0 ? out * out : 0.f);
-  if (lane == 0) part[wave] = sq;
-  __syncthreads();
-  if (tid == 0) a.squares[static_cast<int64_t>(b) * gridDim.x + blockIdx.x] = part[0] + part[1] + part[2] + part[3];
 }
 
 // ---- 2, 5, 6, 7: products of a weight matrix with at most 32 rows --------------
@@ -125,9 +123,11 @@ __global__ __launch_bounds__(256) void step_kernel(const StepParams a) {
 // 16x16x32 product (16 weight rows by 16 or 32 tokens; the matrix pipe is idle otherwise,
 // so columns without a token cost nothing).  A workgroup of NW waves takes a strip of 16
 // rows (RT strips), its waves equal runs of the reduction; two batches of
-// loads are kept in flight per wave, 128 or 256 contiguous bytes of every row, and the first is requested
-// before the row statistics are put together.  x comes through the caches (at most 700 KB for all).
-// A normalisation in front of the product is applied to the operand on its way in.
+// loads are kept in flight per wave, 128 contiguous bytes of every row.  x comes through the caches (at most 700 KB for
+// all) and holds up the weights: loads come back in order, so its share of what is in flight is lost to them
+// (16 sequences: one strip per load of x 60 us for 176 MB, two 48, four 56 on too few workgroups).  That is why
+// it comes normalised: on its way in the norm took 60.2 / 51.7 us where the products alone take 47.8 / 48.0 and
+// rows_norm_kernel 4.6.
 // Waves per strip.  Two-strip products have 672 and 688 workgroups at width 4096: four waves each
 // are all resident at once (eight ran 45.9 / 50.0 us, four 40.6 / 45.6, two 41.5 / 44.4 for 176 / 180 MB).
 // One-strip products have one workgroup per compute unit there: eight (16.2 / 20.6 us for 67 / 90 MB;
@@ -151,22 +151,17 @@ struct SkinnyParams {
   Segment seg[kMaxSegs];
   int segs, K, tokens;
   const uint16_t *norm_weight, *norm_bias;  // stored weight = gamma - 1; may be null
-  const float* stats;      // RMS: (tokens, stat_parts) square sums; layer: (stat_parts, tokens) x (mean, M2) of 16 values
-  int stat_parts, stat_count;  // partial results per token, values behind one
   float eps;
   const uint16_t *add1, *add2;  // (tokens, rows), added to the result
-  float2* moments;         // (workgroups, tokens): mean and M2 of this workgroup's 16 stored values, or null
 };
 
 // PAIR: the two strips are the same rows of two matrices and silu(a) b is stored;
 // otherwise RT consecutive strips of one.
-template <int DT, int MT, int RT, bool PAIR, int NORM, int NW>
+template <int DT, int MT, int RT, bool PAIR, int NW>
 __global__ __launch_bounds__(NW * kWave, MT == 1 ? 4 : 2) void skinny_kernel(const SkinnyParams a) {
   using E = Elem<DT>;
   constexpr int T = NW * kWave;
   __shared__ float red[NW][RT * MT][4][kWave];
-  __shared__ float st_mean[kMaxTokens], st_rstd[kMaxTokens];
-  extern __shared__ __align__(16) uint16_t norm_lds[];  // K values of the norm's weight, K of its bias
   // (uniform to the compiler: a matrix instruction ignores the lane mask, so a step past the wave's
   // end has to be skipped by a branch)
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -195,7 +190,8 @@ __global__ __launch_bounds__(NW * kWave, MT == 1 ? 4 : 2) void skinny_kernel(con
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[t][m] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  constexpr int kSteps = 4 / RT;  // steps of 32 per batch
+  // steps of 32 per batch (one strip and sixteen tokens: four 26.5 us, two 24.9, one 29.3 for 67 / 90 MB)
+  constexpr int kSteps = 2;
   // weights and x of a batch of steps are requested together, in the order in which they are waited
   // for: a wait for x would otherwise also wait for the weights requested ahead
   struct Batch {
@@ -214,70 +210,10 @@ __global__ __launch_bounds__(NW * kWave, MT == 1 ? 4 : 2) void skinny_kernel(con
   };
   request(b0, s_lo);
 
-  float mean[MT], rstd[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t) mean[t] = 0.f, rstd[t] = 1.f;
-  const bool normed = NORM != kNormNone && sg.norm != kNormNone;
-  if (NORM != kNormNone) {
-    // the norm's weight and bias, read from LDS in the loop
-    for (int k = tid * 8; k < a.K; k += T * 8) {
-      const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
-      *reinterpret_cast<uint4*>(norm_lds + k) =
-          a.norm_weight ? *reinterpret_cast<const uint4*>(a.norm_weight + k) : zero;
-      if (NORM == kNormLayer)
-        *reinterpret_cast<uint4*>(norm_lds + a.K + k) =
-            a.norm_bias ? *reinterpret_cast<const uint4*>(a.norm_bias + k) : zero;
-    }
-    // 16 threads per token put its partial results together
-    const int j = tid & 15;
-    for (int m = tid >> 4; m < a.tokens; m += T / 16) {
-      const float inv = 1.f / static_cast<float>(a.K);
-      if (NORM == kNormRms) {
-        float s = 0.f;
-        for (int i = j; i < a.stat_parts; i += 16) s += a.stats[static_cast<int64_t>(m) * a.stat_parts + i];
-        s = group_sum<16>(s);
-        if (j == 0) st_mean[m] = 0.f, st_rstd[m] = rsqrtf(s * inv + a.eps);
-      } else {
-        const float2* st = reinterpret_cast<const float2*>(a.stats);
-        float s = 0.f, q = 0.f;
-        for (int i = j; i < a.stat_parts; i += 16) s += st[static_cast<int64_t>(i) * a.tokens + m].x;
-        const float mu = group_sum<16>(s) / static_cast<float>(a.stat_parts);  // equal counts behind every part
-        for (int i = j; i < a.stat_parts; i += 16) {
-          const float2 v = st[static_cast<int64_t>(i) * a.tokens + m];
-          q += v.y + static_cast<float>(a.stat_count) * (v.x - mu) * (v.x - mu);
-        }
-        q = group_sum<16>(q);
-        if (j == 0) st_mean[m] = mu, st_rstd[m] = rsqrtf(q * inv + a.eps);
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      const int m = 16 * t + r < a.tokens ? 16 * t + r : 0;
-      mean[t] = st_mean[m];
-      rstd[t] = st_rstd[m];
-    }
-  }
-
   auto consume = [&](Batch& t, int s) {
 #pragma unroll
     for (int i = 0; i < kSteps; ++i) {
       if (s + i < s_hi) {
-        if (NORM != kNormNone && normed) {
-          const int k = 32 * (s + i) + 8 * kg;
-          float g[8], c[8], v[8];
-          unpack8<DT>(*reinterpret_cast<const uint4*>(norm_lds + k), g);
-          if (NORM == kNormLayer) unpack8<DT>(*reinterpret_cast<const uint4*>(norm_lds + a.K + k), c);
-#pragma unroll
-          for (int j = 0; j < MT; ++j) {
-            unpack8<DT>(make_uint4(t.x[j][i][0], t.x[j][i][1], t.x[j][i][2], t.x[j][i][3]), v);
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-              v[e] = NORM == kNormLayer ? (v[e] - mean[j]) * rstd[j] * (g[e] + 1.f) + c[e] : v[e] * rstd[j] * (g[e] + 1.f);
-            const uint4 pk = pack8<DT>(v);
-            t.x[j][i] = u32x4{pk.x, pk.y, pk.z, pk.w};
-          }
-        }
 #pragma unroll
         for (int j = 0; j < RT; ++j)
 #pragma unroll
@@ -319,43 +255,331 @@ __global__ __launch_bounds__(NW * kWave, MT == 1 ? 4 : 2) void skinny_kernel(con
       if (sg.bias) v += E::load(sg.bias + row);
       if (sg.act) v = silu(round_to<DT>(v));
     }
-    const bool on = m < a.tokens;
-    if (on) {
+    if (m < a.tokens) {
       const int64_t at = static_cast<int64_t>(m) * sg.out_stride + row;
       if (a.add1) v += E::load(a.add1 + at);
       if (a.add2) v += E::load(a.add2 + at);
       E::store(sg.out + at, v);
     }
-    if (RT == 1 && a.moments) {
-      // mean and M2 of the strip's 16 values per token: four of them in this wave's lanes ...
-      v = round_to<DT>(v);
-      float s1 = v;
-      s1 += __shfl_xor(s1, 16, 64);
-      s1 += __shfl_xor(s1, 32, 64);
-      const float mu4 = 0.25f * s1;
-      float q = (v - mu4) * (v - mu4);
-      q += __shfl_xor(q, 16, 64);
-      q += __shfl_xor(q, 32, 64);
-      if (ln < 16) {  // the slots of (tile, i) have been read by this very wave only
-        red[0][tile][i][ln] = mu4;
-        red[1][tile][i][ln] = q;
-      }
+  }
+}
+
+// Rows normalised as the layer would, for the products that take them as they are: a workgroup per row, 16 values a thread
+// (bound by its launch: 2.8-4.7 us for 9-28 rows of 1024-4096 values).
+constexpr int kNormThreads = 512;
+template <int DT, int NORM>
+__global__ __launch_bounds__(kNormThreads) void rows_norm_kernel(const uint16_t* x, const uint16_t* weight, const uint16_t* bias,
+                                                                 uint16_t* out, int K, float eps) {
+  constexpr int NW = kNormThreads / kWave;
+  __shared__ float sums[NW], squares[NW];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * K;
+  float v[2][8], g[2][8], b[2][8];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int k = 8 * (tid + i * kNormThreads);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[i][e] = g[i][e] = b[i][e] = 0.f;
+    if (k < K) {
+      unpack8<DT>(*reinterpret_cast<const uint4*>(x + row + k), v[i]);
+      if (weight) unpack8<DT>(*reinterpret_cast<const uint4*>(weight + k), g[i]);
+      if (NORM == kNormLayer && bias) unpack8<DT>(*reinterpret_cast<const uint4*>(bias + k), b[i]);
     }
   }
-  if (RT == 1 && a.moments) {
+  const float inv = 1.f / static_cast<float>(K);
+  float mean = 0.f, s = 0.f;
+  if (NORM == kNormLayer) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s += v[i][e];
+    s = wave_sum(s);
+    if (lane == 0) sums[wave] = s;
     __syncthreads();
-    if (tid < a.tokens) {
-      const int tile = tid >> 4, ln = tid & 15;
-      float mu = 0.f, q = 0.f;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) mu += 0.25f * red[0][tile][i][ln];
+    for (int w = 0; w < NW; ++w) mean += sums[w];
+    mean *= inv;
+  }
+  s = 0.f;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float dm = red[0][tile][i][ln] - mu;
-        q += red[1][tile][i][ln] + 4.f * dm * dm;
-      }
-      a.moments[static_cast<int64_t>(blockIdx.x) * a.tokens + tid] = make_float2(mu, q);
+  for (int i = 0; i < 2; ++i)
+    if (8 * (tid + i * kNormThreads) < K)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s += (v[i][e] - mean) * (v[i][e] - mean);
+  s = wave_sum(s);
+  if (lane == 0) squares[wave] = s;
+  __syncthreads();
+  s = 0.f;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) s += squares[w];
+  const float rstd = rsqrtf(s * inv + eps);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int k = 8 * (tid + i * kNormThreads);
+    if (k >= K) continue;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[i][e] = fmaf((v[i][e] - mean) * rstd, g[i][e] + 1.f, b[i][e]);
+    *reinterpret_cast<uint4*>(out + row + k) = pack8<DT>(v[i]);
+  }
+}
+
+// ---- 2, 5, 6, 7 for few tokens: a workgroup per few weight rows ------------------
+// out[m][n] = sum_k x[m][k] W[n][k] again, for at most 4 TT tokens.  A wave's load is four rows by 128 values (256
+// contiguous bytes of each), the operand of two 4x4x4 products in sixteen blocks: lane l holds row l % 4, values
+// 8 (l / 4) .. + 7, and x in the same arrangement, token l % 4.  The eight waves of a workgroup share its G groups of four rows along k,
+// 128 values each in turn, and ask for four pieces at once.
+// What the layout is for: 256 bytes of a row in one request with the non-temporal hint, and many small workgroups, which the
+// hardware hands out as others end.  Reading alone, 176 MB in four rows a workgroup take 26.5 us (6.6 TB/s; without the hint
+// 28.5), in sixteen rows by 64 bytes 33, and by one workgroup per compute unit with an equal share each 52.  With that and x
+// through the caches the products of one row take 14.5 us for 67 / 90 MB (skinny_kernel 18.7).  A norm in front costs vector
+// work per workgroup, so those take 16 rows: 32.3 and 36.5 us for 176 / 180 MB (in 8 rows 36.4 and 40.5, skinny_kernel 41.5 and
+// 45).  Their weights come in two pieces at a time, one with two token tiles: all four would leave one workgroup per unit
+// (41.6 us) or spill (84).
+template <int DT>
+__device__ __forceinline__ floatx4 mma4(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1, floatx4 c) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  if constexpr (DT == MEGA_BF16)
+    return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4, u32x2{a0, a1}), __builtin_bit_cast(s16x4, u32x2{b0, b1}), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, u32x2{a0, a1}), __builtin_bit_cast(f16x4, u32x2{b0, b1}), c, 0, 0, 0);
+}
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// Row q of 16 lanes of the result holds a[q] summed over the four rows of lanes.
+__device__ __forceinline__ float rows_sum(floatx4 a) {
+  auto half = [](float x, float y) {
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+  };
+  const float even = half(a[0], a[2]), odd = half(a[1], a[3]);
+  const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(even), __float_as_uint(odd), false, false);
+  return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+// Sum over the lanes of one token (l % 4), in all of them.
+__device__ __forceinline__ float token_sum(float v) {
+  v = dpp_add<0x124>(v);  // row_ror:4
+  v = dpp_add<0x128>(v);  // row_ror:8
+  v += __shfl_xor(v, 16, 64);
+  return v + __shfl_xor(v, 32, 64);
+}
+__device__ __forceinline__ u32x4 load_weights(const uint16_t* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+}
+
+constexpr int kRowsWaves = 8, kRowsPieces = 4;
+constexpr int kRowsNormK = kRowsWaves * kRowsPieces * 128;  // longest row that is normalised on the way: one round of pieces
+
+template <int DT, int TT, int G, bool PAIR, int NORM>
+__global__ __launch_bounds__(kRowsWaves * kWave, 4) void rows_kernel(const SkinnyParams a) {
+  using E = Elem<DT>;
+  constexpr int NW = kRowsWaves, U = kRowsPieces;
+  constexpr int kRed = TT * G * 16;
+  __shared__ float red[NW][kRed];
+  __shared__ float2 moment[NW][4 * TT];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int blk = blockIdx.x, si = 0;
+  while (blk >= a.seg[si].blocks) blk -= a.seg[si++].blocks;
+  const Segment& sg = a.seg[si];
+  const int K = a.K, chunks = (K + 127) / 128;
+  const int per = (chunks - wave + NW - 1) / NW;  // pieces of this wave: wave, wave + NW, ...
+  const int l_row = lane & 3, l_k = (lane >> 2) * 8;
+  const int row0 = blk * (PAIR ? 2 * G : 4 * G);
+
+  floatx4 acc[G][TT];
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int j = 0; j < TT; ++j) acc[g][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const uint16_t* wp[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+    wp[g] = (PAIR && (g & 1) ? sg.W2 : sg.W) + static_cast<int64_t>(row0 + 4 * (PAIR ? g >> 1 : g) + l_row) * K;
+  const uint16_t* xp[TT];
+#pragma unroll
+  for (int j = 0; j < TT; ++j) xp[j] = sg.x + static_cast<int64_t>(4 * j + l_row < a.tokens ? 4 * j + l_row : 0) * K;
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  // value of this lane's piece c (behind the row's end: its last one, which is not used)
+  auto at = [&](int c) {
+    const int k = 128 * (wave + NW * c) + l_k;
+    return k < K ? k : K - 8;
+  };
+  auto inside = [&](int c) { return 128 * (wave + NW * c) + l_k < K; };
+
+  // n pieces from c0 on
+  auto round = [&](int c0, auto count) {
+    constexpr int n = decltype(count)::value;
+    constexpr int kHeld = NORM == kNormNone ? n : n < 2 || TT > 1 ? 1 : 2;  // pieces of weights in registers
+    u32x4 x[n][TT], w[kHeld][G];
+    u32x4 gw[NORM != kNormNone ? n : 1], gb[NORM == kNormLayer ? n : 1];
+#pragma unroll
+    for (int i = 0; i < n; ++i) {
+      const int k = at(c0 + i);
+#pragma unroll
+      for (int j = 0; j < TT; ++j) x[i][j] = *reinterpret_cast<const u32x4*>(xp[j] + k);
     }
+    if (NORM != kNormNone) {
+#pragma unroll
+      for (int i = 0; i < n; ++i) {
+        const int k = at(c0 + i);
+        gw[i] = a.norm_weight ? *reinterpret_cast<const u32x4*>(a.norm_weight + k) : zero;
+        if (NORM == kNormLayer) gb[i] = a.norm_bias ? *reinterpret_cast<const u32x4*>(a.norm_bias + k) : zero;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kHeld; ++i) {
+      const int k = at(c0 + i);
+#pragma unroll
+      for (int g = 0; g < G; ++g) w[i][g] = load_weights(wp[g] + k);
+    }
+    if (NORM != kNormNone && sg.norm != kNormNone) {
+      // a row's moments: of a wave's values in two passes, of the waves' together
+      float mean[TT], rstd[TT];
+#pragma unroll
+      for (int j = 0; j < TT; ++j) {
+        float s = 0.f, q = 0.f, mine = 0.f, v[8];
+        if (NORM == kNormLayer) {
+          int full = 0;
+#pragma unroll
+          for (int i = 0; i < n; ++i) {
+            full += inside(c0 + i) ? 8 : 0;
+            unpack8<DT>(__builtin_bit_cast(uint4, x[i][j]), v);
+            float t = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) t += v[e];
+            s += inside(c0 + i) ? t : 0.f;
+          }
+          mine = token_sum(s) / token_sum(static_cast<float>(full));
+        }
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+          unpack8<DT>(__builtin_bit_cast(uint4, x[i][j]), v);
+          float t = 0.f;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float d = NORM == kNormLayer ? v[e] - mine : v[e];
+            t += d * d;
+          }
+          q += inside(c0 + i) ? t : 0.f;
+        }
+        q = token_sum(q);
+        if (lane < 4) moment[wave][4 * j + lane] = make_float2(mine, q);
+      }
+      lds_barrier();
+      const float inv = 1.f / static_cast<float>(K);
+#pragma unroll
+      for (int j = 0; j < TT; ++j) {
+        float mu = 0.f, q = 0.f;
+        auto count = [&](int w) {  // values of wave w
+          const int last = chunks - 1, all = (chunks - w + NW - 1) / NW * 128;
+          return static_cast<float>(last % NW == w ? all - (128 * chunks - K) : all);
+        };
+        if (NORM == kNormLayer) {
+#pragma unroll
+          for (int w = 0; w < NW; ++w) mu += w < chunks ? count(w) * moment[w][4 * j + l_row].x : 0.f;
+          mu *= inv;
+        }
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+          if (w >= chunks) continue;
+          const float2 m = moment[w][4 * j + l_row];
+          q += m.y;
+          if (NORM == kNormLayer) q += count(w) * (m.x - mu) * (m.x - mu);
+        }
+        mean[j] = mu;
+        rstd[j] = rsqrtf(q * inv + a.eps);
+      }
+#pragma unroll
+      for (int i = 0; i < n; ++i) {
+        float g[8], b[8], v[8];
+        unpack8<DT>(__builtin_bit_cast(uint4, gw[i]), g);
+        if (NORM == kNormLayer) unpack8<DT>(__builtin_bit_cast(uint4, gb[i]), b);
+#pragma unroll
+        for (int j = 0; j < TT; ++j) {
+          unpack8<DT>(__builtin_bit_cast(uint4, x[i][j]), v);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float scale = fmaf(g[e], rstd[j], rstd[j]);
+            v[e] = NORM == kNormLayer ? fmaf(v[e] - mean[j], scale, b[e]) : v[e] * scale;
+          }
+          x[i][j] = __builtin_bit_cast(u32x4, pack8<DT>(v));
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < n; ++i) {
+      const int h = i % kHeld;
+      if (128 * (wave + NW * (c0 + i)) + 128 > K) {  // lanes behind the row's end
+        const bool in = inside(c0 + i);
+#pragma unroll
+        for (int j = 0; j < TT; ++j) x[i][j] = in ? x[i][j] : zero;
+#pragma unroll
+        for (int g = 0; g < G; ++g) w[h][g] = in ? w[h][g] : zero;
+      }
+#pragma unroll
+      for (int j = 0; j < TT; ++j) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) acc[g][j] = mma4<DT>(w[h][g][0], w[h][g][1], x[i][j][0], x[i][j][1], acc[g][j]);
+#pragma unroll
+        for (int g = 0; g < G; ++g) acc[g][j] = mma4<DT>(w[h][g][2], w[h][g][3], x[i][j][2], x[i][j][3], acc[g][j]);
+      }
+      if (i + kHeld < n) {
+        const int k = at(c0 + i + kHeld);
+#pragma unroll
+        for (int g = 0; g < G; ++g) w[h][g] = load_weights(wp[g] + k);
+      }
+    }
+  };
+  if (NORM == kNormNone) {
+    int c = 0;
+    for (; c + U <= per; c += U) round(c, std::integral_constant<int, U>());
+    if (per - c == 3) round(c, std::integral_constant<int, 3>());
+    else if (per - c == 2) round(c, std::integral_constant<int, 2>());
+    else if (per - c == 1) round(c, std::integral_constant<int, 1>());
+  } else if (per == 4) {  // (at most kRowsNormK values a row)
+    round(0, std::integral_constant<int, 4>());
+  } else if (per == 3) {
+    round(0, std::integral_constant<int, 3>());
+  } else if (per == 2) {
+    round(0, std::integral_constant<int, 2>());
+  } else if (per == 1) {
+    round(0, std::integral_constant<int, 1>());
+  } else if (sg.norm != kNormNone) {
+    lds_barrier();  // (a row of fewer pieces than waves)
+  }
+
+#pragma unroll
+  for (int j = 0; j < TT; ++j)
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      float v = rows_sum(acc[g][j]);
+      v = dpp_add<0x124>(v);
+      v = dpp_add<0x128>(v);
+      if ((lane & 12) == 0) red[wave][(j * G + g) * 16 + (lane >> 4) * 4 + l_row] = v;
+    }
+  lds_barrier();
+  // 16 results of each (token tile, row group): row (o / 4) % 4, token o % 4
+  for (int o = tid; o < (PAIR ? kRed / 2 : kRed); o += NW * kWave) {
+    const int q = o >> 4, e = o & 15, j = q / (PAIR ? G / 2 : G), g = q % (PAIR ? G / 2 : G);
+    const int m = 4 * j + (e & 3), row = row0 + 4 * g + (e >> 2);
+    const int src = (j * G + (PAIR ? 2 * g : g)) * 16 + e;
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) v += red[w][src];
+    if (m >= a.tokens) continue;
+    if (PAIR) {
+      float c = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) c += red[w][src + 16];
+      v = silu(round_to<DT>(v)) * round_to<DT>(c);
+    } else {
+      if (sg.bias) v += E::load(sg.bias + row);
+      if (sg.act) v = silu(round_to<DT>(v));
+    }
+    const int64_t to = static_cast<int64_t>(m) * sg.out_stride + row;
+    if (a.add1) v += E::load(a.add1 + to);
+    if (a.add2) v += E::load(a.add2 + to);
+    E::store(sg.out + to, v);
   }
 }
 
@@ -412,14 +636,30 @@ __global__ __launch_bounds__(kAttendThreads) void attend_kernel(const AttendPara
       ahead[i] = load_once((at < old_hi ? vp : vq) + at * vstep);
     }
   };
+  // The first keys and z are asked for in front of the first value rows: loads come back in order.
+  const uint16_t* kp = a.k_old + (static_cast<int64_t>(b) * (a.total - 1) + k_lo) * S + h * zh + c;
+  uint16_t* kq = a.k + (static_cast<int64_t>(b) * a.total + k_lo) * S + h * zh + c;
+  constexpr int kU = 4;
+  uint4 raw[kU];
+  auto request_keys = [&](int j0) {
+#pragma unroll
+    for (int i = 0; i < kU; ++i) {
+      const int j = j0 + i * 4 * KPW;
+      raw[i] = old_hi > 0 ? load_once(kp + static_cast<int64_t>(j < old_hi ? j : old_hi - 1) * S)
+                          : make_uint4(0u, 0u, 0u, 0u);
+    }
+  };
+  const int at = h * zh + c;
+  const uint4 z_raw = *reinterpret_cast<const uint4*>(a.z + static_cast<int64_t>(b) * S + at);
+  request_keys(wave * KPW + lane / LPK);
+  const uint4 g_raw = *reinterpret_cast<const uint4*>(a.gamma + at), b_raw = *reinterpret_cast<const uint4*>(a.beta + at);
   request(kg);
 
   // q, and for the run with the new token also k: every wave works them out for itself
   float q[8], kn[8];
   {
     float zv[8], g[8], bt[8];
-    const int at = h * zh + c;
-    unpack8<DT>(*reinterpret_cast<const uint4*>(a.z + static_cast<int64_t>(b) * S + at), zv);
+    unpack8<DT>(z_raw, zv);
     float ss = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) ss += zv[e] * zv[e];
@@ -429,9 +669,9 @@ __global__ __launch_bounds__(kAttendThreads) void attend_kernel(const AttendPara
 #pragma unroll
       for (int e = 0; e < 8; ++e) f[e] = a.freqs[c + e];
     }
-    auto finish = [&](const uint16_t* gp, const uint16_t* bp, float* o) {
-      unpack8<DT>(*reinterpret_cast<const uint4*>(gp + at), g);
-      unpack8<DT>(*reinterpret_cast<const uint4*>(bp + at), bt);
+    auto finish = [&](const uint4& gp, const uint4& bp, float* o) {
+      unpack8<DT>(gp, g);
+      unpack8<DT>(bp, bt);
 #pragma unroll
       for (int e = 0; e < 8; ++e) o[e] = zv[e] * rs * ((g[e] + 1.f) * a.inv_sqrt) + bt[e];
       if (a.freqs) {
@@ -443,28 +683,19 @@ __global__ __launch_bounds__(kAttendThreads) void attend_kernel(const AttendPara
         }
       }
     };
-    finish(a.gamma, a.beta, q);
+    finish(g_raw, b_raw, q);
 #pragma unroll
     for (int e = 0; e < 8; ++e) q[e] = round_to<DT>(q[e]);
     if (newest) {
-      finish(a.gamma + S, a.beta + S, kn);
+      finish(*reinterpret_cast<const uint4*>(a.gamma + S + at), *reinterpret_cast<const uint4*>(a.beta + S + at), kn);
       const uint4 packed = pack8<DT>(kn);
       if (tid < LPK)
         *reinterpret_cast<uint4*>(a.k + (static_cast<int64_t>(b) * a.total + a.total - 1) * S + at) = packed;
       unpack8<DT>(packed, kn);
     }
   }
-  const uint16_t* kp = a.k_old + (static_cast<int64_t>(b) * (a.total - 1) + k_lo) * S + h * zh + c;
-  uint16_t* kq = a.k + (static_cast<int64_t>(b) * a.total + k_lo) * S + h * zh + c;
-  constexpr int kU = 4;
-  for (int j0 = wave * KPW + lane / LPK; j0 - lane / LPK < old_hi; j0 += 4 * KPW * kU) {
-    uint4 raw[kU];
-#pragma unroll
-    for (int i = 0; i < kU; ++i) {
-      const int j = j0 + i * 4 * KPW;
-      raw[i] = old_hi > 0 ? load_once(kp + static_cast<int64_t>(j < old_hi ? j : old_hi - 1) * S)
-                          : make_uint4(0u, 0u, 0u, 0u);
-    }
+  for (int j0 = wave * KPW + lane / LPK, first = 1; j0 - lane / LPK < old_hi; j0 += 4 * KPW * kU, first = 0) {
+    if (!first) request_keys(j0);
 #pragma unroll
     for (int i = 0; i < kU; ++i) {
       const int j = j0 + i * 4 * KPW;
@@ -604,7 +835,7 @@ void key_runs(int64_t pairs, int64_t total, int* splits, int* per) {
 }
 
 struct Layout {
-  int64_t tsn, cema, z, r, h1, attn, y1, hidden, squares, moments, ml, part, bytes;
+  int64_t tsn, cema, normed, z, r, h1, attn, y1, hidden, ml, part, bytes;
 };
 Layout layout_of(const mega_block_decode_args& a) {
   int splits, per;
@@ -618,26 +849,34 @@ Layout layout_of(const mega_block_decode_args& a) {
   Layout l;
   l.tsn = take(2 * a.B * a.D);
   l.cema = take(2 * a.B * a.D);
+  l.normed = take(2 * a.B * a.D);
   l.z = take(2 * a.B * a.S);
   l.r = take(2 * a.B * a.E);
   l.h1 = take(2 * a.B * a.D);
   l.attn = take(2 * a.B * a.E);
   l.y1 = take(2 * a.B * a.D);
   l.hidden = take(2 * a.B * a.F);
-  l.squares = take(4 * a.B * (a.D / kStepChannels));
-  l.moments = take(8 * a.B * (a.D / 16));
   l.ml = take(8 * a.B * a.heads * splits);
   l.part = take(4 * a.B * a.E * splits);
   l.bytes = at;
   return l;
 }
 
-template <int DT, int MT, int RT, bool PAIR, int NORM, int NW>
+template <int DT, int MT, int RT, bool PAIR, int NW>
 void skinny(const SkinnyParams& p, hipStream_t s) {
   int blocks = 0;
   for (int i = 0; i < p.segs; ++i) blocks += p.seg[i].blocks;
-  const size_t lds = NORM == kNormNone ? 0 : sizeof(uint16_t) * p.K * (NORM == kNormLayer ? 2 : 1);
-  skinny_kernel<DT, MT, RT, PAIR, NORM, NW><<<blocks, NW * kWave, lds, s>>>(p);
+  skinny_kernel<DT, MT, RT, PAIR, NW><<<blocks, NW * kWave, 0, s>>>(p);
+}
+
+// Tokens that rows_kernel takes: at eight it is still ahead at every width (4 heads of 1024 features 1603 -> 1565 us for
+// eight tokens, 1 head 361 -> 326); sixteen would need 64 accumulators a row group and spill (2 heads 646 -> 905).
+constexpr int kRowsTokens = 8;
+template <int DT, int TT, int G, bool PAIR, int NORM>
+void rows(SkinnyParams p, hipStream_t s) {
+  int blocks = 0;
+  for (int i = 0; i < p.segs; ++i) blocks += p.seg[i].blocks;
+  rows_kernel<DT, TT, G, PAIR, NORM><<<blocks, kRowsWaves * kWave, 0, s>>>(p);
 }
 
 template <int DT, int MT>
@@ -652,27 +891,34 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
     StepParams p{u16(a.x), u16(a.prev_mean), u16(a.prev_var), u16(a.tsn_weight), u16(a.tsn_bias), u16(a.omega),
                  a.prev_count, a.p, a.q, a.gamma_hat, reinterpret_cast<const float4*>(a.h_in), at16(l.tsn),
                  at16(l.cema), static_cast<uint16_t*>(a.mean), static_cast<uint16_t*>(a.var), a.count,
-                 reinterpret_cast<float4*>(a.h_out), reinterpret_cast<float*>(ws + l.squares), D,
+                 reinterpret_cast<float4*>(a.h_out), D,
                  static_cast<int>(a.G), static_cast<int>(a.D / a.G), a.tsn_eps};
     step_kernel<DT><<<dim3(D / kStepChannels, B), 256, 0, s>>>(p);
   }
   const uint16_t* none = nullptr;
+  const bool few = B <= kRowsTokens && D <= kRowsNormK;  // by rows_kernel
+  const int wide = 4, narrow = B <= 4 ? 1 : 2;  // row groups of a workgroup
   auto seg = [&](const void* W, const void* W2, const void* bias, const uint16_t* x, uint16_t* out, int64_t stride,
                  int rows, int strip, int norm, int act) {
-    return Segment{u16(W), u16(W2), u16(bias), x, out, stride, rows / strip, norm, act};
+    return Segment{u16(W), u16(W2), u16(bias), x, out, stride, rows / (few ? (W2 ? 2 * wide : strip == 32 ? 4 * wide : 4 * narrow) : strip), norm, act};
   };
   {
+    if (!few)
+      rows_norm_kernel<DT, kNormRms><<<B, kNormThreads, 0, s>>>(at16(l.cema), u16(a.rms_weight), none, at16(l.normed), D, a.rms_eps);
+    const uint16_t* row = at16(few ? l.cema : l.normed);
     SkinnyParams p{};
     // the wide layers first: the narrow one fills the gaps at the end
     p.seg[0] = seg(a.wv, none, a.bv, at16(l.tsn), static_cast<uint16_t*>(a.v_out) + a.length * a.E,
                    (a.length + 1) * a.E, E, 32, kNormNone, 1);
-    p.seg[1] = seg(a.wr, none, a.br, at16(l.cema), at16(l.r), E, E, 32, kNormRms, 0);
-    p.seg[2] = seg(a.wh1, none, a.bh1, at16(l.cema), at16(l.h1), D, D, 32, kNormRms, 0);
-    p.seg[3] = seg(a.wz, none, a.bz, at16(l.cema), at16(l.z), S, S, 32, kNormRms, 0);
+    p.seg[1] = seg(a.wr, none, a.br, row, at16(l.r), E, E, 32, kNormRms, 0);
+    p.seg[2] = seg(a.wh1, none, a.bh1, row, at16(l.h1), D, D, 32, kNormRms, 0);
+    p.seg[3] = seg(a.wz, none, a.bz, row, at16(l.z), S, S, 32, kNormRms, 0);
     p.segs = 4, p.K = D, p.tokens = B;
     p.norm_weight = u16(a.rms_weight);
-    p.stats = reinterpret_cast<const float*>(ws + l.squares), p.stat_parts = D / kStepChannels, p.eps = a.rms_eps;
-    skinny<DT, MT, 2, false, kNormRms, kWavesWide>(p, s);
+    p.eps = a.rms_eps;
+    if (!few) skinny<DT, MT, 2, false, kWavesWide>(p, s);
+    else if (B <= 4) rows<DT, 1, 4, false, kNormRms>(p, s);
+    else rows<DT, 2, 4, false, kNormRms>(p, s);
   }
   const int zh = S / H, H2 = E / H;
   int splits, per;
@@ -697,24 +943,30 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
     p.seg[0] = seg(a.wh2, none, none, at16(l.attn), at16(l.y1), D, D, 16, kNormNone, 0);
     p.segs = 1, p.K = E, p.tokens = B;
     p.add1 = at16(l.h1), p.add2 = u16(a.x);
-    p.moments = reinterpret_cast<float2*>(ws + l.moments);
-    skinny<DT, MT, 1, false, kNormNone, kWavesNarrow>(p, s);
+    if (!few) skinny<DT, MT, 1, false, kWavesNarrow>(p, s);
+    else if (B <= 4) rows<DT, 1, 1, false, kNormNone>(p, s);
+    else rows<DT, 2, 2, false, kNormNone>(p, s);
   }
   {
+    if (!few)
+      rows_norm_kernel<DT, kNormLayer><<<B, kNormThreads, 0, s>>>(at16(l.y1), u16(a.ln_weight), u16(a.ln_bias), at16(l.normed), D, a.ln_eps);
     SkinnyParams p{};
-    p.seg[0] = seg(a.fc1, a.fc3, none, at16(l.y1), at16(l.hidden), F, F, 16, kNormLayer, 0);
+    p.seg[0] = seg(a.fc1, a.fc3, none, at16(few ? l.y1 : l.normed), at16(l.hidden), F, F, 16, kNormLayer, 0);
     p.segs = 1, p.K = D, p.tokens = B;
     p.norm_weight = u16(a.ln_weight), p.norm_bias = u16(a.ln_bias);
-    p.stats = reinterpret_cast<const float*>(ws + l.moments), p.stat_parts = D / 16, p.stat_count = 16;
     p.eps = a.ln_eps;
-    skinny<DT, MT, 2, true, kNormLayer, kWavesWide>(p, s);
+    if (!few) skinny<DT, MT, 2, true, kWavesWide>(p, s);
+    else if (B <= 4) rows<DT, 1, 4, true, kNormLayer>(p, s);
+    else rows<DT, 2, 4, true, kNormLayer>(p, s);
   }
   {
     SkinnyParams p{};
     p.seg[0] = seg(a.fc2, none, none, at16(l.hidden), static_cast<uint16_t*>(a.y), D, D, 16, kNormNone, 0);
     p.segs = 1, p.K = F, p.tokens = B;
     p.add1 = u16(a.x);
-    skinny<DT, MT, 1, false, kNormNone, kWavesNarrow>(p, s);
+    if (!few) skinny<DT, MT, 1, false, kWavesNarrow>(p, s);
+    else if (B <= 4) rows<DT, 1, 1, false, kNormNone>(p, s);
+    else rows<DT, 2, 2, false, kNormNone>(p, s);
   }
   MEGA_CHECK_LAUNCH();
   return MEGA_OK;
