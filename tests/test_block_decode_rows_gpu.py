@@ -56,3 +56,24 @@ def test_infinite_weight_stays_in_its_row():
         wanted = blk.nffn(wanted, x)
     assert torch.equal(y.isfinite(), wanted.isfinite()) and torch.equal(y.isinf(), wanted.isinf())
     assert not y[..., 7].isfinite().any() and y.isfinite().sum() == B * (D - 1)
+
+
+def test_streams_step_at_once():
+    """Six sequences, two token tiles, on eight streams at once: each its own workspace, each the step's own bits."""
+    B, D, S, E, F, n = 6, 512, 128, 256, 416, 30
+    blk = _block(D, S, E, F, 1, 4, 64)
+    rotary = RotaryEmbedding(S, 64).cuda()
+    with torch.no_grad():
+        cache = _prompt(blk, B, n, D, S, E, 1, torch.bfloat16, rotary)
+        xs = [torch.randn(B, 1, D, generator=torch.Generator().manual_seed(i)).bfloat16().cuda() for i in range(8)]
+        freqs = rotary.get_freqs_cis(n, n + 1)
+        wanted = [decode_step(blk, x, freqs, cache) for x in xs]
+        torch.cuda.synchronize()
+        streams, got = [torch.cuda.Stream() for _ in xs], []
+        for stream, x in zip(streams, xs):
+            with torch.cuda.stream(stream):
+                got.append(decode_step(blk, x, freqs, cache))
+        torch.cuda.synchronize()
+    for g, w in zip(got, wanted):
+        assert torch.equal(g[0], w[0])
+        assert all(torch.equal(a, b) for a, b in zip(_tensors(g[1]), _tensors(w[1])))
