@@ -666,6 +666,12 @@ int mega_cema_scan_fwd(const void* x, int dtype, const float* p, const float* lo
                        const float* gamma, const float* omega, const float* h0, int64_t B,
                        int64_t D, int64_t N, int64_t L, void* y, float* h_last, void* stream);
 
+/* mega_cema_scan_fwd for the layer: float32 rows (16-byte aligned) of any L >= 1 too.  Those whose length is no multiple of
+ * 8 enter the products with all their bits and come out as the matrices' 24 give them (mega_cema_layer_fwd the same). */
+int mega_cema_layer_scan_fwd(const void* x, int dtype, const float* p, const float* log_q,
+                             const float* gamma, const float* omega, const float* h0, int64_t B,
+                             int64_t D, int64_t N, int64_t L, void* y, float* h_last, void* stream);
+
 /* Backward of mega_cema_scan_fwd without a carried state (the training path):
  * replaces the chain fftconv_bwd -> (dx, dk), ema_parameters_bwd(dk, ...) ->
  * (dp, dq, dgamma) and the two elementwise passes of the skip term
@@ -714,6 +720,8 @@ int mega_cema_scan_bwd_wide(const void* dy, const void* x, const float* p, const
  * bfloat16 tensors: hi = bf16(src), lo = bf16(src - hi) -- 16 significant bits of a float32
  * value, every bit of a float16 one.  The pieces mega_cema_scan_bwd_wide runs on. */
 int mega_split_bf16(const void* src, int dtype, int64_t n, void* hi, void* lo, void* stream);
+/* ... of three, third = bf16(src - hi - lo): 24 significant bits. */
+int mega_split_bf16_three(const float* src, int64_t n, void* hi, void* lo, void* third, void* stream);
 
 /* ------------------------------------------------------------------------
  * Streaming reference kernel for measurements (no counterpart in the

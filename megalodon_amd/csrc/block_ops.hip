@@ -254,11 +254,11 @@ int launch_silu_mul(const void* dout, const void* a, const void* b, void* o0, vo
 
 // ---- a float32 / float16 tensor as the sum of two bfloat16 tensors ------------------------
 // hi = bf16(v), lo = bf16(v - hi): 16 significant bits of a float32 value, all 11 of a float16
-// one.  The backward of the CEMA recurrence is linear in dy and, for the parameter gradients,
+// one; with a third, bf16(v - hi - lo), 24.  The backward of the CEMA recurrence is linear in dy and, for the parameter gradients,
 // in x, and runs on such pieces (mega_cema_scan_bwd_wide).  8 elements per lane and pass.
-template <int DT>
+template <int DT, bool THIRD>
 __global__ __launch_bounds__(kThreads) void split_bf16_kernel(const void* __restrict__ src, uint16_t* __restrict__ hi,
-                                                             uint16_t* __restrict__ lo, int64_t n8) {
+                                                             uint16_t* __restrict__ lo, uint16_t* __restrict__ third, int64_t n8) {
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < n8;
        i += static_cast<int64_t>(gridDim.x) * kThreads) {
     float v[8];
@@ -268,14 +268,17 @@ __global__ __launch_bounds__(kThreads) void split_bf16_kernel(const void* __rest
     } else {
       unpack8<MEGA_F16>(reinterpret_cast<const uint4*>(src)[i], v);
     }
-    uint32_t h[4], l[4];
+    uint32_t h[4], l[4], t[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       h[e] = pack_bf16x2(v[2 * e], v[2 * e + 1]);
-      l[e] = pack_bf16x2(v[2 * e] - __uint_as_float(h[e] << 16), v[2 * e + 1] - __uint_as_float(h[e] & 0xffff0000u));
+      const float r0 = v[2 * e] - __uint_as_float(h[e] << 16), r1 = v[2 * e + 1] - __uint_as_float(h[e] & 0xffff0000u);
+      l[e] = pack_bf16x2(r0, r1);
+      if (THIRD) t[e] = pack_bf16x2(r0 - __uint_as_float(l[e] << 16), r1 - __uint_as_float(l[e] & 0xffff0000u));
     }
     reinterpret_cast<uint4*>(hi)[i] = make_uint4(h[0], h[1], h[2], h[3]);
     reinterpret_cast<uint4*>(lo)[i] = make_uint4(l[0], l[1], l[2], l[3]);
+    if (THIRD) reinterpret_cast<uint4*>(third)[i] = make_uint4(t[0], t[1], t[2], t[3]);
   }
 }
 
@@ -342,20 +345,28 @@ extern "C" int mega_silu_mul_bwd(const void* dout, const void* a, const void* b,
   return launch_silu_mul<MEGA_F16>(dout, a, b, da, db, n, s);
 }
 
-extern "C" int mega_split_bf16(const void* src, int dtype, int64_t n, void* hi, void* lo, void* stream) {
-  MEGA_CHECK_ARG(dtype == MEGA_F32 || dtype == MEGA_F16, "mega_split_bf16: float32 or float16 input");
-  MEGA_CHECK_ARG(n >= 0 && n % 8 == 0, "mega_split_bf16: the element count must be a multiple of 8");
+static int split_entry(const char* who, const void* src, int dtype, int64_t n, void* hi, void* lo, void* third, bool three, void* stream) {
+  MEGA_CHECK_ARG(dtype == MEGA_F32 || (dtype == MEGA_F16 && !three), "%s: float32 or float16 input", who);
+  MEGA_CHECK_ARG(n >= 0 && n % 8 == 0, "%s: the element count must be a multiple of 8", who);
   if (n == 0) return MEGA_OK;
-  MEGA_CHECK_ARG(src && hi && lo, "mega_split_bf16: null pointer");
+  MEGA_CHECK_ARG(src && hi && lo && (third || !three), "%s: null pointer", who);
   const auto al = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
-  MEGA_CHECK_ARG(al(src) && al(hi) && al(lo), "mega_split_bf16: operands must be 16-byte aligned");
+  MEGA_CHECK_ARG(al(src) && al(hi) && al(lo) && al(third), "%s: operands must be 16-byte aligned", who);
   const int64_t n8 = n / 8;
   const unsigned grid = static_cast<unsigned>(std::min<int64_t>((n8 + kThreads - 1) / kThreads, 16384));
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (dtype == MEGA_F32)
-    split_bf16_kernel<MEGA_F32><<<grid, kThreads, 0, s>>>(src, static_cast<uint16_t*>(hi), static_cast<uint16_t*>(lo), n8);
-  else
-    split_bf16_kernel<MEGA_F16><<<grid, kThreads, 0, s>>>(src, static_cast<uint16_t*>(hi), static_cast<uint16_t*>(lo), n8);
+  uint16_t *h = static_cast<uint16_t*>(hi), *l = static_cast<uint16_t*>(lo), *t = static_cast<uint16_t*>(third);
+  if (three) split_bf16_kernel<MEGA_F32, true><<<grid, kThreads, 0, s>>>(src, h, l, t, n8);
+  else if (dtype == MEGA_F32) split_bf16_kernel<MEGA_F32, false><<<grid, kThreads, 0, s>>>(src, h, l, t, n8);
+  else split_bf16_kernel<MEGA_F16, false><<<grid, kThreads, 0, s>>>(src, h, l, t, n8);
   MEGA_CHECK_LAUNCH();
   return MEGA_OK;
+}
+
+extern "C" int mega_split_bf16(const void* src, int dtype, int64_t n, void* hi, void* lo, void* stream) {
+  return split_entry("mega_split_bf16", src, dtype, n, hi, lo, nullptr, false, stream);
+}
+
+extern "C" int mega_split_bf16_three(const float* src, int64_t n, void* hi, void* lo, void* third, void* stream) {
+  return split_entry("mega_split_bf16_three", src, MEGA_F32, n, hi, lo, third, true, stream);
 }

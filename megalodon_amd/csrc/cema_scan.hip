@@ -318,13 +318,47 @@ template <> struct XOp<MEGA_F32> {
   }
 };
 
+// float32 rows of the other layouts: all three pieces, 24 significant bits, as their matrices carry.  (They went through a
+// float32 kernel row and float32 transforms: y 2.8e-6 - 3.4e-6 from 64 bits in the 2-norm, now 4.2e-7 - 6.0e-7, gradients nowhere
+// further off than they were.  1024 rows of 51151 steps forward 1974 -> 124 us, 4096 of 201 50.6 -> 16.3.)
+struct XOpWide {
+  static constexpr int XP = 3;
+  u32x4 pc[3];
+  template <int ROWS>
+  __device__ __forceinline__ void load(const void* tile, int elem, int lo, int hi) {
+    (void)lo;
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    typedef f32x4 f32x4_any __attribute__((aligned(4)));
+    const float* src = static_cast<const float*>(tile) + elem;
+    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (ROWS == kShifted ? elem < hi : elem + 8 <= hi) {  // (kShifted: a piece with one of the steps is inside the tensor)
+      const f32x4 a = *reinterpret_cast<const f32x4_any*>(src), b = *reinterpret_cast<const f32x4_any*>(src + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = a[e], v[4 + e] = b[e];
+    } else if (elem < hi) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (elem + e < hi) v[e] = src[e];
+    }
+    split8(v, pc[0], pc[1]);
+    pc[2] = split8_third(v, pc[0], pc[1]);
+  }
+  __device__ __forceinline__ void keep(int elem, int lo, int hi) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) pc[i] = keep_steps(pc[i], elem, lo, hi);
+  }
+};
+template <int DT, bool FINE>
+using XRow = typename std::conditional<DT == MEGA_F32 && FINE, XOpWide, XOp<DT>>::type;
+
 // acc += (A_hi + A_lo) * x, without FINE the lo * lo term of a two-piece x left out
 template <int XP, bool FINE = false>
 __device__ __forceinline__ floatx16 mma_split(const u32x4* a, const u32x4* x, floatx16 acc) {
   acc = mfma_bf16(a[0], x[0], acc);
   acc = mfma_bf16(a[1], x[0], acc);
-  if (XP == 2) acc = mfma_bf16(a[0], x[1], acc);
-  if (XP == 2 && FINE) acc = mfma_bf16(a[1], x[1], acc);
+  if (XP >= 2) acc = mfma_bf16(a[0], x[1], acc);
+  if (XP >= 2 && FINE) acc = mfma_bf16(a[1], x[1], acc);
+  if (XP == 3) acc = mfma_bf16(a[0], x[2], acc);
   return acc;
 }
 
@@ -463,7 +497,8 @@ __global__ __launch_bounds__(kThreads, ONE ? 4 : 3) void cema_scan_fwd_kernel(
   constexpr bool FINE = kFine<ROWS>;
   using Smem = typename std::conditional<ONE, typename std::conditional<FINE, FwdSmemOneFine, FwdSmemOne>::type,
                                          typename std::conditional<FINE, FwdSmemFine, FwdSmem>::type>::type;
-  constexpr int NC = Smem::NC, CPS = NC / kSubs, XP = XOp<DT>::XP;
+  using Op = XRow<DT, FINE>;
+  constexpr int NC = Smem::NC, CPS = NC / kSubs, XP = Op::XP;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Smem& sm = *reinterpret_cast<Smem*>(smem_raw);
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -474,7 +509,7 @@ __global__ __launch_bounds__(kThreads, ONE ? 4 : 3) void cema_scan_fwd_kernel(
   // The workgroup walks (group, four tiles) items: groups blockIdx.x, + gridDim.x, ..., the tiles
   // of a group in line.  The x tile of the next item and the parameters of the next group are
   // requested ahead.
-  auto load_tile = [&](XOp<DT> (&t)[4], const Tile& w) {
+  auto load_tile = [&](Op (&t)[4], const Tile& w) {
     const typename Elem<DT>::type* xrow = static_cast<const typename Elem<DT>::type*>(x) + w.base;
     const int id = opaque(lane), at = (id & 31) * kT + 8 * (id >> 5);
 #pragma unroll
@@ -616,7 +651,7 @@ __global__ __launch_bounds__(kThreads, ONE ? 4 : 3) void cema_scan_fwd_kernel(
   // reads it -- the local states and the K X part of the outputs -- comes first, then the
   // same registers are reloaded with the next item's tile while the scan and the state part of
   // the outputs run.
-  XOp<DT> xb[4];
+  Op xb[4];
   Tile cur_tile = tile_at<ROWS>(ln, blockIdx.x, wave);  // this wave's tile of the item
   auto item = [&](int group, int t0, int tiles) {
     if (t0 == 0) setup_row(group);
@@ -780,9 +815,14 @@ __global__ __launch_bounds__(kThreads, ONE ? 4 : 3) void cema_scan_fwd_kernel(
 #pragma unroll
               for (int h = 0; h < 2; ++h) {
                 const int elem = at + 16 * (2 * it + pr) + 8 * h + 4 * ag;
-                if (elem < w.hi)
+                if (ROWS == kWhole ? elem < w.hi : ROWS == kShifted && elem >= w.lo && elem + 4 <= w.hi) {
                   *reinterpret_cast<float4*>(yrow + elem) = make_float4(acc[8 * pr + 4 * h], acc[8 * pr + 4 * h + 1],
                                                                         acc[8 * pr + 4 * h + 2], acc[8 * pr + 4 * h + 3]);
+                } else if (ROWS != kWhole) {
+#pragma unroll
+                  for (int e = 0; e < 4; ++e)
+                    if (elem + e >= w.lo && elem + e < w.hi) yrow[elem + e] = acc[8 * pr + 4 * h + e];
+                }
               }
             } else {
               const uint4 oct = octet_of<DT>(acc, pr);
@@ -1664,25 +1704,29 @@ int rows_of(int64_t count, int64_t L, bool carried, std::initializer_list<const 
 using namespace mega;
 
 extern "C" int mega_cema_scan_supported(int dtype, int64_t N, int64_t L) {
-  // float32 rows of other lengths stay with the convolution, whose float32 transforms are the finer of the two
+  // (float32 rows of other lengths: mega_cema_layer_scan_fwd)
   return valid_dtype(dtype) && N >= 1 && N <= 16 && L >= 1 && (dtype != MEGA_F32 || L % 8 == 0);
 }
 
+// any_length: float32 rows of every length, as the layer takes them
 static int scan_fwd_entry(const char* who, const void* x, int dtype, const Coeffs& co, const float* h0, int64_t B, int64_t D,
-                          int64_t N, int64_t L, void* y, float* h_last, void* stream) {
+                          int64_t N, int64_t L, void* y, float* h_last, bool any_length, void* stream) {
   MEGA_CHECK_ARG(B >= 0 && D >= 0 && L >= 0, "%s: negative size", who);
   MEGA_CHECK_ARG(B * D <= 0x7fffffff, "%s: too many rows", who);
-  if (!mega_cema_scan_supported(dtype, N, L))
+  if (!mega_cema_scan_supported(any_length && dtype == MEGA_F32 ? MEGA_BF16 : dtype, N, L))
     return set_error(MEGA_ERR_UNSUPPORTED,
                      "%s: needs N <= 16 and, for float32 rows, L a multiple of 8 (dtype %d, N %lld, L %lld)",
                      who, dtype, (long long)N, (long long)L);
   const int rows = rows_of(B * D, L, h0 != nullptr, {x, y});
-  MEGA_CHECK_ARG(rows == kWhole || dtype != MEGA_F32, "%s: float32 rows must be 16-byte aligned", who);
+  for (const void* t : {x, static_cast<const void*>(y)})
+    MEGA_CHECK_ARG(dtype != MEGA_F32 || reinterpret_cast<uintptr_t>(t) % 16 == 0, "%s: float32 rows must be 16-byte aligned", who);
   if (B == 0 || D == 0) return MEGA_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const cf* h0c = reinterpret_cast<const cf*>(h0);
   cf* hl = reinterpret_cast<cf*>(h_last);
-  auto go = dtype == MEGA_F32     ? launch_fwd<MEGA_F32, kWhole>
+  auto go = dtype == MEGA_F32    ? (rows == kWhole     ? launch_fwd<MEGA_F32, kWhole>
+                                    : rows == kShifted ? launch_fwd<MEGA_F32, kShifted>
+                                                       : launch_fwd<MEGA_F32, kAny>)
             : dtype == MEGA_BF16 ? (rows == kWhole     ? launch_fwd<MEGA_BF16, kWhole>
                                     : rows == kShifted ? launch_fwd<MEGA_BF16, kShifted>
                                                        : launch_fwd<MEGA_BF16, kAny>)
@@ -1692,18 +1736,30 @@ static int scan_fwd_entry(const char* who, const void* x, int dtype, const Coeff
   return go(x, y, co, h0c, hl, B, D, N, L, s);
 }
 
-extern "C" int mega_cema_scan_fwd(const void* x, int dtype, const float* p, const float* log_q,
-                                  const float* gamma, const float* omega, const float* h0, int64_t B,
-                                  int64_t D, int64_t N, int64_t L, void* y, float* h_last,
-                                  void* stream) {
-  const char* who = "mega_cema_scan_fwd";
+static int scan_fwd(const char* who, bool any_length, const void* x, int dtype, const float* p, const float* log_q, const float* gamma,
+                    const float* omega, const float* h0, int64_t B, int64_t D, int64_t N, int64_t L, void* y, float* h_last,
+                    void* stream) {
   MEGA_CHECK_ARG(x && p && log_q && gamma && y, "%s: null pointer", who);
   Coeffs co{};
   co.p = p;
   co.log_q = reinterpret_cast<const cf*>(log_q);
   co.gamma = reinterpret_cast<const cf*>(gamma);
   co.omega = omega;
-  return scan_fwd_entry(who, x, dtype, co, h0, B, D, N, L, y, h_last, stream);
+  return scan_fwd_entry(who, x, dtype, co, h0, B, D, N, L, y, h_last, any_length, stream);
+}
+
+extern "C" int mega_cema_scan_fwd(const void* x, int dtype, const float* p, const float* log_q,
+                                  const float* gamma, const float* omega, const float* h0, int64_t B,
+                                  int64_t D, int64_t N, int64_t L, void* y, float* h_last,
+                                  void* stream) {
+  return scan_fwd("mega_cema_scan_fwd", false, x, dtype, p, log_q, gamma, omega, h0, B, D, N, L, y, h_last, stream);
+}
+
+extern "C" int mega_cema_layer_scan_fwd(const void* x, int dtype, const float* p, const float* log_q,
+                                        const float* gamma, const float* omega, const float* h0, int64_t B,
+                                        int64_t D, int64_t N, int64_t L, void* y, float* h_last,
+                                        void* stream) {
+  return scan_fwd("mega_cema_layer_scan_fwd", true, x, dtype, p, log_q, gamma, omega, h0, B, D, N, L, y, h_last, stream);
 }
 
 extern "C" int mega_cema_layer_fwd(const void* x, int dtype, int param_dtype, const void* alpha, const void* delta, const void* theta,
@@ -1730,7 +1786,7 @@ extern "C" int mega_cema_layer_fwd(const void* x, int dtype, int param_dtype, co
     co.log_q = reinterpret_cast<const cf*>(w + D * N);
     co.gamma = reinterpret_cast<const cf*>(w + 3 * D * N);
   }
-  return scan_fwd_entry(who, x, dtype, co, nullptr, B, D, N, L, y, nullptr, stream);
+  return scan_fwd_entry(who, x, dtype, co, nullptr, B, D, N, L, y, nullptr, true, stream);
 }
 
 extern "C" int mega_cema_scan_bwd_supported(int dtype, int64_t N, int64_t L) {

@@ -309,7 +309,7 @@ Tensor cema_coeffs(const Tensor& alpha, const Tensor& delta, const Tensor& theta
 }
 Tensor scan_raw(const Tensor& x, const float* p, const float* log_q, const float* gamma_hat, const float* omega, const float* h0, float* h_last, int64_t N) {
   Tensor y = at::empty_like(x);
-  check(mega_cema_scan_fwd(x.data_ptr(), kernel_code(x), p, log_q, gamma_hat, omega, h0, x.size(0), x.size(1), N, x.size(2), y.data_ptr(), h_last, stream_of(x)), "mega_cema_scan_fwd");
+  check(mega_cema_layer_scan_fwd(x.data_ptr(), kernel_code(x), p, log_q, gamma_hat, omega, h0, x.size(0), x.size(1), N, x.size(2), y.data_ptr(), h_last, stream_of(x)), "mega_cema_layer_scan_fwd");
   return y;
 }
 // float32 (contiguous) form of the skip weight
@@ -320,11 +320,16 @@ Tensor rows_of(const Tensor& x) {
   if (c.scalar_type() == at::kFloat && reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 != 0) c = c.clone(at::MemoryFormat::Contiguous);
   return c;
 }
-std::tuple<Tensor, Tensor> split(const Tensor& t) {
-  const int64_t n = t.numel();
-  Tensor hi = at::empty(t.sizes(), t.options().dtype(at::kBFloat16)), lo = at::empty_like(hi);
-  check(mega_split_bf16(t.data_ptr(), kernel_code(t), n, hi.data_ptr(), lo.data_ptr(), stream_of(t)), "mega_split_bf16");
-  return {hi, lo};
+// a float32 tensor in two bfloat16 pieces, or in three; all in one tensor, each on a 16-byte boundary
+Tensor split(const Tensor& t, int pieces) {
+  const int64_t n = t.numel(), n8 = (n + 7) / 8 * 8;
+  Tensor out = at::empty({pieces, n8}, t.options().dtype(at::kBFloat16));
+  uint16_t* p = static_cast<uint16_t*>(out.data_ptr());
+  Tensor whole = t;
+  if (n != n8) whole = at::constant_pad_nd(t.reshape({-1}), {0, n8 - n});
+  if (pieces == 2) check(mega_split_bf16(whole.data_ptr(), kernel_code(t), n8, p, p + n8, stream_of(t)), "mega_split_bf16");
+  else check(mega_split_bf16_three(whole.data_ptr<float>(), n8, p, p + n8, p + 2 * n8, stream_of(t)), "mega_split_bf16_three");
+  return out;
 }
 struct CemaFn : Function<CemaFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& alpha, const Tensor& delta, const Tensor& theta, const Tensor& gamma, const Tensor& omega) {
@@ -349,25 +354,27 @@ struct CemaFn : Function<CemaFn> {
     // gradients of the launches' groups of rows, stacked: (dp, dq, dgamma_hat, domega); the coefficients'
     // backward adds the stack up
     const bool wide = x.scalar_type() == at::kFloat;
-    const int64_t per = mega_cema_layer_scan_sets(B, D, L), pieces = wide ? 3 : 1, sets = pieces * per;
+    const bool thirds = wide && L % 8 != 0;
+    const int64_t per = mega_cema_layer_scan_sets(B, D, L), launches = thirds ? 6 : wide ? 3 : 1, sets = launches * per;
     const Tensor stack = floats({sets * (5 * DN + D)}, x);
     float *dp = stack.data_ptr<float>(), *dq = dp + sets * DN, *dg = dq + 2 * sets * DN, *dw = dg + 2 * sets * DN;
-    Tensor dx;
+    Tensor dx = wide ? floats(x.sizes(), x) : at::empty_like(x);
     if (!wide) {
-      dx = at::empty_like(x);
       const int mode = x.scalar_type() == at::kHalf ? 3 : 0;
       check(mega_cema_layer_scan_bwd(dy.data_ptr(), x.data_ptr(), p, lq, gh, fptr(w), B, D, N, L, dx.data_ptr(), mode, dp, dq, dg, dw, s), "mega_cema_layer_scan_bwd");
     } else {
-      // linear in dy and, for the parameter gradients, in x: the bfloat16 pieces (dy_hi, x_hi), (dy_lo, x_hi),
-      // (dy_hi, x_lo); dx is linear in dy alone and is added up in float32.  What is left out, (dy_lo, x_lo), is 2e-6 of
-      // the parameter gradients.
-      auto [g_hi, g_lo] = split(dy);
-      auto [x_hi, x_lo] = split(x);
-      Tensor dx32 = floats(x.sizes(), x);
-      const Tensor* pairs[3][2] = {{&g_hi, &x_hi}, {&g_lo, &x_hi}, {&g_hi, &x_lo}};
-      for (int i = 0; i < pieces; ++i)
-        check(mega_cema_layer_scan_bwd(pairs[i][0]->data_ptr(), pairs[i][1]->data_ptr(), p, lq, gh, fptr(w), B, D, N, L, i < 2 ? dx32.data_ptr() : nullptr, i == 1 ? 2 : 1, dp + i * per * DN, dq + 2 * i * per * DN, dg + 2 * i * per * DN, dw + i * per * D, s), "mega_cema_layer_scan_bwd");
-      dx = dx32;
+      // linear in dy and, for the parameter gradients, in x: pairs of bfloat16 pieces.  dx is linear in dy alone and is
+      // added up in float32 over the pairs with x's first piece.  Lengths that are a multiple of 8 take two pieces and leave out
+      // (dy_lo, x_lo), 2e-6 of the parameter gradients; the others, which came from a float32 convolution, three and leave
+      // out what is below 2^-25 (forward and backward of 2048 x 52327 12.2 -> 2.1 ms, 2048 x 22185 1.72 -> 1.01).
+      static constexpr int pairs[6][2] = {{0, 0}, {1, 0}, {0, 1}, {2, 0}, {1, 1}, {0, 2}};
+      const Tensor gp = split(dy, thirds ? 3 : 2), xp = split(x, thirds ? 3 : 2);
+      const int64_t n8 = gp.size(1);
+      const uint16_t *g0 = static_cast<const uint16_t*>(gp.data_ptr()), *x0 = static_cast<const uint16_t*>(xp.data_ptr());
+      for (int i = 0; i < launches; ++i) {
+        const bool to_dx = pairs[i][1] == 0;
+        check(mega_cema_layer_scan_bwd(g0 + pairs[i][0] * n8, x0 + pairs[i][1] * n8, p, lq, gh, fptr(w), B, D, N, L, to_dx ? dx.data_ptr() : nullptr, to_dx && i > 0 ? 2 : 1, dp + i * per * DN, dq + 2 * i * per * DN, dg + 2 * i * per * DN, dw + i * per * D, s), "mega_cema_layer_scan_bwd");
+      }
     }
     Tensor da = at::empty_like(alpha), dd = at::empty_like(delta), dt = at::empty_like(theta), dga = at::empty_like(gamma), dom = at::empty_like(omega);
     check(mega_cema_layer_coeffs_bwd(kernel_code(alpha), dp, dq, dg, dw, sets, alpha.data_ptr(), delta.data_ptr(), theta.data_ptr(), D, N, da.data_ptr(), dd.data_ptr(), dt.data_ptr(), dga.data_ptr(), dom.data_ptr(), s), "mega_cema_layer_coeffs_bwd");
@@ -376,7 +383,7 @@ struct CemaFn : Function<CemaFn> {
 };
 // rows of this shape and type run on the recurrence kernels in one launch per piece
 bool cema_takes(const Tensor& x, int64_t N) {
-  return x.is_cuda() && x.dim() == 3 && N >= 1 && N <= 16 && code_of(x.scalar_type()) >= 0 && x.size(2) >= 1 && (x.scalar_type() != at::kFloat || x.size(2) % 8 == 0) && x.size(0) * x.size(1) <= 0x7fffffff;
+  return x.is_cuda() && x.dim() == 3 && N >= 1 && N <= 16 && code_of(x.scalar_type()) >= 0 && x.size(2) >= 1 && x.size(0) * x.size(1) <= 0x7fffffff;
 }
 Optional cema(const Tensor& x, const Tensor& alpha, const Tensor& delta, const Tensor& theta, const Tensor& gamma, const Tensor& omega) {
   if (alpha.dim() != 3 || !cema_takes(x, alpha.size(1))) return std::nullopt;
@@ -395,6 +402,9 @@ Optional cema(const Tensor& x, const Tensor& alpha, const Tensor& delta, const T
 std::optional<std::tuple<Tensor, Optional>> cema_state(const Tensor& x, const Tensor& p, const Tensor& log_q, const Tensor& gamma_hat, const Tensor& omega, const Optional& h0, bool last) {
   const int64_t N = p.size(1);
   if (!cema_takes(x, N)) return std::nullopt;
+  // (the state's share of the outputs is a product of two-piece factors, 2^-18: 3.9e-6 of one step's outputs, where these
+  // lengths add it in float32)
+  if (h0.has_value() && x.scalar_type() == at::kFloat && x.size(2) % 8 != 0) return std::nullopt;
   const int64_t B = x.size(0), D = x.size(1);
   require(p.numel() == D * N && log_q.numel() == D * N && gamma_hat.numel() == D * N && omega.numel() == D, "cema: x and the parameters must have the same number of channels");
   if (h0.has_value()) require(h0->scalar_type() == at::kComplexFloat && h0->numel() == B * D * N && h0->device() == x.device(), "cema: the carried state must be complex64 (B, D, N)");

@@ -1,0 +1,76 @@
+"""The EMA layer on float32 rows whose length no piece of the kernels divides, against the float64 oracle: outputs, gradients,
+last state.  Rows and matrices enter with 24 bits, sums are float32, powers come from float32 coefficients: y, dx and
+the state 5e-7 in the 2-norm at the initial decays (longest chains 6e-7), gradients up to 2e-6 (theta, a sum of cancelling
+terms).  Bars: three times that."""
+import pytest
+import torch
+
+from megalodon_amd.modules import MultiHeadComplexEMA
+from oracle import cema as ocema, fftconv as offt
+from test_cema_any_length_gpu import NAMES, _picked, _rows
+
+pytestmark = pytest.mark.gpu
+
+
+def _err(got, ref):
+    got, ref = (torch.view_as_real(t) if t.is_complex() else t for t in (got.detach().cpu(), ref.detach()))
+    return ((got.double() - ref).norm() / ref.norm()).item()
+
+
+# rows taken from the boundary in front where B D L is a multiple of 8, by accesses at any element elsewhere; one item and several,
+# several rows of a channel in one workgroup; one step, a piece, a chunk and a tile cut on either side
+@pytest.mark.parametrize("B,D,L,offset", [(1, 8, 1, 0), (2, 8, 7, 0), (1, 3, 9, 0), (1, 8, 63, 1), (3, 8, 65, 0), (1, 5, 1021, 0),
+                                          (2, 16, 2047, 0), (1, 16, 2049, 2), (1, 3, 8191, 0), (2, 8, 8195, 0), (1, 8, 20003, 0),
+                                          (5, 304, 130, 0), (5, 520, 2049, 0)])
+def test_layer_matches_oracle(B, D, L, offset):
+    torch.manual_seed(L)
+    layer = MultiHeadComplexEMA(D, 16).cuda().train()
+    x0, x = _rows(B, D, L, torch.float32, L, offset)
+    dy0, dy = _rows(B, D, L, torch.float32, L + 1, offset)
+    x.requires_grad_(True)
+    out, _ = layer(x)
+    out.backward(dy)
+    with torch.no_grad():
+        layer.eval()
+        again = layer(x)[0]
+    grads = {n: getattr(layer, n).grad for n in NAMES}
+    dx = x.grad
+    if D > 64:  # every 50th channel is checked
+        pick = slice(0, None, 50)
+        out, again, dx, x0, dy0 = (t[:, pick] for t in (out, again, dx, x0, dy0))
+        grads = {n: g[pick] for n, g in grads.items()}
+        layer = _picked(layer, pick)
+    pr = {n: getattr(layer, n).detach().cpu().double().requires_grad_(True) for n in NAMES}
+    xo = x0.double().requires_grad_(True)
+    p, q, g = ocema.calc_coeffs(pr["alpha"], pr["delta"], pr["theta"], pr["gamma"], 16)
+    want = offt.fftconv_fwd(xo, ocema.ema_weight_fwd(p, q.log(), g, L)) + xo * pr["omega"]
+    want.backward(dy0.double())
+    assert out.dtype == dx.dtype == torch.float32
+    assert max(_err(out, want), _err(again, want), _err(dx, xo.grad)) <= 2e-6
+    for n in NAMES:
+        if L > 1 or n in ("alpha", "gamma", "omega"):  # (one step: no power of q, those gradients are rounding alone)
+            assert _err(grads[n], pr[n].grad) <= 6e-6, n
+
+
+@pytest.mark.parametrize("carried", [False, True])
+@pytest.mark.parametrize("B,D,L", [(2, 8, 1), (1, 3, 5), (2, 8, 63), (2, 8, 1531), (1, 3, 8201), (7, 400, 2113)])
+def test_last_state(B, D, L, carried):
+    """With a carried state these lengths stay with the float32 convolution, whose outputs are 3e-6 off: bar three times that."""
+    N = 16
+    torch.manual_seed(L)
+    layer = MultiHeadComplexEMA(D, N).cuda().eval()
+    x0, x = _rows(B, D, L, torch.float32, L, 0)
+    h0 = torch.randn(B, D, N, dtype=torch.complex64, generator=torch.Generator().manual_seed(2)) if carried else None
+    with torch.no_grad():
+        out, last = layer(x, h0.cuda() if carried else None, True)
+    if D > 64:
+        pick = slice(0, None, 50)
+        out, last, x0, h0 = out[:, pick], last[:, pick], x0[:, pick], h0[:, pick] if carried else None
+        layer = _picked(layer, pick)
+    pr = {n: getattr(layer, n).detach().cpu().double() for n in NAMES}
+    p, q, g = ocema.calc_coeffs(pr["alpha"], pr["delta"], pr["theta"], pr["gamma"], N)
+    want = offt.fftconv_fwd(x0.double(), ocema.ema_weight_fwd(p, q.log(), g, L)) + x0.double() * pr["omega"]
+    if carried:
+        want = want + ocema.ema_bias_fwd(q.log(), g, h0, L)
+    assert _err(out, want) <= (9e-6 if carried else 2e-6)
+    assert last.dtype == torch.complex64 and _err(last, ocema.ema_hidden_fwd(x0, p, q.log(), h0)) <= 2e-6
