@@ -16,6 +16,7 @@
 //   6. products       LayerNorm folded into fc1, fc3; silu(a) b
 //   7. products       fc2 + residual
 // The products are rows_kernel's for few sequences, which normalises on the way, else rows_norm_kernel's and skinny_kernel's.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -593,9 +594,12 @@ __global__ __launch_bounds__(kRowsWaves * kWave, 4) void rows_kernel(const Skinn
 // handed out is never written again, and the one that continues it is contiguous.  (Appended in place to storage
 // with room the steps took 0.144 and 0.32 ms, but then a cache shares memory with the one it continues; with
 // stores that stay in the caches 0.156 and 0.52.)
+// The memory bounds it, old keys and values in and out, and how much of its rate is had depends on how many streams there
+// are: a workgroup a CU, all of equal runs (key_runs).  AHEAD value rows and KU pieces of keys are in flight per thread:
+// long runs twice as many as short ones, whose requests past the end are for nothing.
 constexpr int kAttendThreads = 256;
-constexpr int kMaxKeys = 1024;  // keys of a run
-constexpr int kAhead = 8;       // value rows in flight per thread
+constexpr int kMaxKeys = 4096;  // keys of a run
+constexpr int kLongRun = 300;
 
 struct AttendParams {
   const uint16_t *z, *gamma, *beta;  // (B, S); (2, S)
@@ -608,7 +612,7 @@ struct AttendParams {
   float eps, inv_sqrt;
 };
 
-template <int DT, int LPK>
+template <int DT, int LPK, int AHEAD, int KU>
 __global__ __launch_bounds__(kAttendThreads) void attend_kernel(const AttendParams a) {
   using E = Elem<DT>;
   __shared__ float score[kMaxKeys];
@@ -628,10 +632,10 @@ __global__ __launch_bounds__(kAttendThreads) void attend_kernel(const AttendPara
   const int old_hi = newest ? nk - 1 : nk;  // keys of the run that the old cache holds
   const uint16_t* vp = a.v_old + (static_cast<int64_t>(b) * (a.total - 1) + k_lo) * vstep + vcol;
   uint16_t* vq = a.v + (static_cast<int64_t>(b) * a.total + k_lo) * vstep + vcol;
-  uint4 ahead[kAhead];
+  uint4 ahead[AHEAD];
   auto request = [&](int i0) {  // rows past the run's end: the last one again, unused
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) {
+    for (int i = 0; i < AHEAD; ++i) {
       const int j = i0 + i * kgroups, at = j < nk ? j : nk - 1;
       ahead[i] = load_once((at < old_hi ? vp : vq) + at * vstep);
     }
@@ -639,11 +643,10 @@ __global__ __launch_bounds__(kAttendThreads) void attend_kernel(const AttendPara
   // The first keys and z are asked for in front of the first value rows: loads come back in order.
   const uint16_t* kp = a.k_old + (static_cast<int64_t>(b) * (a.total - 1) + k_lo) * S + h * zh + c;
   uint16_t* kq = a.k + (static_cast<int64_t>(b) * a.total + k_lo) * S + h * zh + c;
-  constexpr int kU = 4;
-  uint4 raw[kU];
+  uint4 raw[KU];
   auto request_keys = [&](int j0) {
 #pragma unroll
-    for (int i = 0; i < kU; ++i) {
+    for (int i = 0; i < KU; ++i) {
       const int j = j0 + i * 4 * KPW;
       raw[i] = old_hi > 0 ? load_once(kp + static_cast<int64_t>(j < old_hi ? j : old_hi - 1) * S)
                           : make_uint4(0u, 0u, 0u, 0u);
@@ -694,10 +697,10 @@ __global__ __launch_bounds__(kAttendThreads) void attend_kernel(const AttendPara
       unpack8<DT>(packed, kn);
     }
   }
-  for (int j0 = wave * KPW + lane / LPK, first = 1; j0 - lane / LPK < old_hi; j0 += 4 * KPW * kU, first = 0) {
+  for (int j0 = wave * KPW + lane / LPK, first = 1; j0 - lane / LPK < old_hi; j0 += 4 * KPW * KU, first = 0) {
     if (!first) request_keys(j0);
 #pragma unroll
-    for (int i = 0; i < kU; ++i) {
+    for (int i = 0; i < KU; ++i) {
       const int j = j0 + i * 4 * KPW;
       float kv[8], s = 0.f;
       if (j < old_hi) store_streaming(kq + static_cast<int64_t>(j) * S, raw[i]);
@@ -737,13 +740,13 @@ __global__ __launch_bounds__(kAttendThreads) void attend_kernel(const AttendPara
   float o[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] = 0.f;
-  for (int j0 = kg; j0 < nk; j0 += kAhead * kgroups) {
-    uint4 now[kAhead];
+  for (int j0 = kg; j0 < nk; j0 += AHEAD * kgroups) {
+    uint4 now[AHEAD];
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) now[i] = ahead[i];
-    request(j0 + kAhead * kgroups);
+    for (int i = 0; i < AHEAD; ++i) now[i] = ahead[i];
+    request(j0 + AHEAD * kgroups);
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) {
+    for (int i = 0; i < AHEAD; ++i) {
       const int j = j0 + i * kgroups;
       const float w = j < nk ? score[j] : 0.f;
       if (j < old_hi) store_streaming(vq + j * vstep, now[i]);
@@ -823,10 +826,17 @@ __global__ __launch_bounds__(256) void combine_kernel(const CombineParams a) {
 }
 
 // ---- host ----------------------------------------------------------------------
-// Runs of keys: enough workgroups to fill the chip twice over, at least 16 keys each (a run's
-// partial result is 4 bytes per value column, a key 2), at most what the score buffer holds.
+// Runs of keys: a workgroup for every CU, or for as many as equal shares of the pairs leave, where that is two thirds of them;
+// else two.  At least 16 keys each (a run's partial result is 4 bytes per value column, a key 2), at most what the score
+// buffer holds.  With at least 512 workgroups, most of them resident two to a CU and a few left for the end, the step of
+// four heads on 8 tokens took, us before / now: 1 x 1531 keys 986 / 968, 5 x 3900 2350 / 2144, 9 x 3000 2868 / 2577, 13 x 3000 3700 / 3260, 16 x
+// 3000 3903 / 3738, 22 x 3000 (69 % of the CUs) 5692 / 4983, 32 x 3500 7822 / 7434; of eight heads 24 x 1000 (75 %) 8279 / 8083, 20 x
+// 1000 (62 %, so two a CU) 7337 / 7239 where one a CU takes 7457.  With long requests for all 1 x 1531 took 982, with short ones
+// 32 x 3500 7531.
 void key_runs(int64_t pairs, int64_t total, int* splits, int* per) {
-  int64_t want = (512 + pairs - 1) / pairs;
+  constexpr int64_t kCus = 256;
+  int64_t want = kCus / pairs;
+  if (3 * want * pairs < 2 * kCus) want = std::max<int64_t>(2 * kCus / pairs, 1);
   int64_t n = (total + want - 1) / want;
   if (n < 16) n = 16;
   if (n > kMaxKeys) n = kMaxKeys;
@@ -879,6 +889,13 @@ void rows(SkinnyParams p, hipStream_t s) {
   rows_kernel<DT, TT, G, PAIR, NORM><<<blocks, kRowsWaves * kWave, 0, s>>>(p);
 }
 
+template <int DT, int AHEAD, int KU>
+void attend(const AttendParams& p, int zh, dim3 grid, hipStream_t s) {
+  if (zh == 64) attend_kernel<DT, 8, AHEAD, KU><<<grid, kAttendThreads, 0, s>>>(p);
+  else if (zh == 128) attend_kernel<DT, 16, AHEAD, KU><<<grid, kAttendThreads, 0, s>>>(p);
+  else attend_kernel<DT, 32, AHEAD, KU><<<grid, kAttendThreads, 0, s>>>(p);
+}
+
 template <int DT, int MT>
 int run(const mega_block_decode_args& a, hipStream_t s) {
   const Layout l = layout_of(a);
@@ -929,9 +946,8 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
                    reinterpret_cast<float2*>(ws + l.ml), H, H2, static_cast<int>(a.length + 1), splits, per, a.z_eps,
                    1.f / sqrtf(static_cast<float>(zh))};
     const dim3 grid(splits, B * H);
-    if (zh == 64) attend_kernel<DT, 8><<<grid, kAttendThreads, 0, s>>>(p);
-    else if (zh == 128) attend_kernel<DT, 16><<<grid, kAttendThreads, 0, s>>>(p);
-    else attend_kernel<DT, 32><<<grid, kAttendThreads, 0, s>>>(p);
+    if (per >= kLongRun) attend<DT, 16, 8>(p, zh, grid, s);
+    else attend<DT, 8, 4>(p, zh, grid, s);
   }
   {
     CombineParams p{reinterpret_cast<const float*>(ws + l.part), reinterpret_cast<const float2*>(ws + l.ml),
