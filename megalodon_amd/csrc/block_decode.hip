@@ -15,7 +15,7 @@
 //   5. products       wh2 + h1 + residual
 //   6. products       LayerNorm folded into fc1, fc3; silu(a) b
 //   7. products       fc2 + residual
-// The products are rows_kernel's for few sequences, which normalises on the way, else rows_norm_kernel's and skinny_kernel's.
+// The products are rows_kernel's for few sequences, which normalises on the way, else rows_norm_kernel's and tiles_kernel's.
 #include <algorithm>
 #include <type_traits>
 
@@ -119,21 +119,7 @@ __global__ __launch_bounds__(256) void step_kernel(const StepParams a) {
 }
 
 // ---- 2, 5, 6, 7: products of a weight matrix with at most 32 rows --------------
-// out[m][n] = sum_k x[m][k] W[n][k].  What counts is that the weights stream in at the
-// memory's rate: each is read once, 16 bytes per lane straight into the operand of a
-// 16x16x32 product (16 weight rows by 16 or 32 tokens; the matrix pipe is idle otherwise,
-// so columns without a token cost nothing).  A workgroup of NW waves takes a strip of 16
-// rows (RT strips), its waves equal runs of the reduction; two batches of
-// loads are kept in flight per wave, 128 contiguous bytes of every row.  x comes through the caches (at most 700 KB for
-// all) and holds up the weights: loads come back in order, so its share of what is in flight is lost to them
-// (16 sequences: one strip per load of x 60 us for 176 MB, two 48, four 56 on too few workgroups).  That is why
-// it comes normalised: on its way in the norm took 60.2 / 51.7 us where the products alone take 47.8 / 48.0 and
-// rows_norm_kernel 4.6.
-// Waves per strip.  Two-strip products have 672 and 688 workgroups at width 4096: four waves each
-// are all resident at once (eight ran 45.9 / 50.0 us, four 40.6 / 45.6, two 41.5 / 44.4 for 176 / 180 MB).
-// One-strip products have one workgroup per compute unit there: eight (16.2 / 20.6 us for 67 / 90 MB;
-// sixteen 18.9 / 23.8).
-constexpr int kWavesWide = 4, kWavesNarrow = 8;
+// out[m][n] = sum_k x[m][k] W[n][k].  What counts is that the weights, each read once, stream in at the memory's rate.
 enum { kNormNone = 0, kNormRms = 1, kNormLayer = 2 };
 constexpr int kMaxSegs = 4;
 
@@ -148,122 +134,13 @@ struct Segment {       // rows of one weight matrix
   int norm;
   int act;             // silu on the result
 };
-struct SkinnyParams {
+struct ProductParams {
   Segment seg[kMaxSegs];
   int segs, K, tokens;
   const uint16_t *norm_weight, *norm_bias;  // stored weight = gamma - 1; may be null
   float eps;
   const uint16_t *add1, *add2;  // (tokens, rows), added to the result
 };
-
-// PAIR: the two strips are the same rows of two matrices and silu(a) b is stored;
-// otherwise RT consecutive strips of one.
-template <int DT, int MT, int RT, bool PAIR, int NW>
-__global__ __launch_bounds__(NW * kWave, MT == 1 ? 4 : 2) void skinny_kernel(const SkinnyParams a) {
-  using E = Elem<DT>;
-  constexpr int T = NW * kWave;
-  __shared__ float red[NW][RT * MT][4][kWave];
-  // (uniform to the compiler: a matrix instruction ignores the lane mask, so a step past the wave's
-  // end has to be skipped by a branch)
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int blk = blockIdx.x, si = 0;
-  while (blk >= a.seg[si].blocks) blk -= a.seg[si++].blocks;
-  const Segment& sg = a.seg[si];
-  constexpr int kRows = PAIR ? 16 : 16 * RT;
-  const int row0 = blk * kRows;
-  const int r = lane & 15, kg = lane >> 4;
-  const int steps = a.K / 32, per = (steps + NW - 1) / NW;
-  const int s_lo = wave * per < steps ? wave * per : steps, s_hi = s_lo + per < steps ? s_lo + per : steps;
-
-  const uint16_t* wp[RT];
-#pragma unroll
-  for (int t = 0; t < RT; ++t)
-    wp[t] = (PAIR && t == 1 ? sg.W2 : sg.W) + static_cast<int64_t>(row0 + (PAIR ? 0 : 16 * t) + r) * a.K + 8 * kg;
-  const uint16_t* xp[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    const int m = 16 * t + r;
-    xp[t] = sg.x + static_cast<int64_t>(m < a.tokens ? m : 0) * a.K + 8 * kg;
-  }
-  floatx4 acc[RT][MT];
-#pragma unroll
-  for (int t = 0; t < RT; ++t)
-#pragma unroll
-    for (int m = 0; m < MT; ++m) acc[t][m] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-  // steps of 32 per batch (one strip and sixteen tokens: four 26.5 us, two 24.9, one 29.3 for 67 / 90 MB)
-  constexpr int kSteps = 2;
-  // weights and x of a batch of steps are requested together, in the order in which they are waited
-  // for: a wait for x would otherwise also wait for the weights requested ahead
-  struct Batch {
-    u32x4 w[RT][kSteps], x[MT][kSteps];
-  };
-  Batch b0, b1;
-  auto request = [&](Batch& t, int s) {  // steps past the wave's end: the last one again, unused
-#pragma unroll
-    for (int i = 0; i < kSteps; ++i) {
-      const int64_t k = 32 * static_cast<int64_t>(s + i < s_hi ? s + i : (s_hi > 0 ? s_hi - 1 : 0));
-#pragma unroll
-      for (int j = 0; j < RT; ++j) t.w[j][i] = *reinterpret_cast<const u32x4*>(wp[j] + k);
-#pragma unroll
-      for (int j = 0; j < MT; ++j) t.x[j][i] = *reinterpret_cast<const u32x4*>(xp[j] + k);
-    }
-  };
-  request(b0, s_lo);
-
-  auto consume = [&](Batch& t, int s) {
-#pragma unroll
-    for (int i = 0; i < kSteps; ++i) {
-      if (s + i < s_hi) {
-#pragma unroll
-        for (int j = 0; j < RT; ++j)
-#pragma unroll
-          for (int m = 0; m < MT; ++m) acc[j][m] = mma16<DT>(t.w[j][i], t.x[m][i], acc[j][m]);
-      }
-    }
-  };
-  for (int s = s_lo; s < s_hi; s += 2 * kSteps) {
-    request(b1, s + kSteps);
-    consume(b0, s);
-    if (s + kSteps < s_hi) {
-      request(b0, s + 2 * kSteps);
-      consume(b1, s + kSteps);
-    }
-  }
-
-#pragma unroll
-  for (int t = 0; t < RT; ++t)
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) red[wave][t * MT + m][i][lane] = acc[t][m][i];
-  __syncthreads();
-  // value (i, lane) of a tile: weight row 4 (lane / 16) + i, token lane % 16
-  constexpr int kOuts = (PAIR ? 1 : RT) * MT * 256;
-  for (int o = tid; o < kOuts; o += T) {
-    const int tile = o >> 8, i = (o >> 6) & 3, ln = o & 63;
-    const int rt = tile / MT, m = 16 * (tile % MT) + (ln & 15);
-    const int row = row0 + 16 * rt + 4 * (ln >> 4) + i;
-    float v = 0.f;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) v += red[w][tile][i][ln];
-    if (PAIR) {
-      float c = 0.f;
-#pragma unroll
-      for (int w = 0; w < NW; ++w) c += red[w][MT + tile][i][ln];
-      v = silu(round_to<DT>(v)) * round_to<DT>(c);
-    } else {
-      if (sg.bias) v += E::load(sg.bias + row);
-      if (sg.act) v = silu(round_to<DT>(v));
-    }
-    if (m < a.tokens) {
-      const int64_t at = static_cast<int64_t>(m) * sg.out_stride + row;
-      if (a.add1) v += E::load(a.add1 + at);
-      if (a.add2) v += E::load(a.add2 + at);
-      E::store(sg.out + at, v);
-    }
-  }
-}
 
 // Rows normalised as the layer would, for the products that take them as they are: a workgroup per row, 16 values a thread
 // (bound by its launch: 2.8-4.7 us for 9-28 rows of 1024-4096 values).
@@ -332,9 +209,9 @@ __global__ __launch_bounds__(kNormThreads) void rows_norm_kernel(const uint16_t*
 // What the layout is for: 256 bytes of a row in one request with the non-temporal hint, and many small workgroups, which the
 // hardware hands out as others end.  Reading alone, 176 MB in four rows a workgroup take 26.5 us (6.6 TB/s; without the hint
 // 28.5), in sixteen rows by 64 bytes 33, and by one workgroup per compute unit with an equal share each 52.  With that and x
-// through the caches the products of one row take 14.5 us for 67 / 90 MB (skinny_kernel 18.7).  A norm in front costs vector
-// work per workgroup, so those take 16 rows: 32.3 and 36.5 us for 176 / 180 MB (in 8 rows 36.4 and 40.5, skinny_kernel 41.5 and
-// 45).  Their weights come in two pieces at a time, one with two token tiles: all four would leave one workgroup per unit
+// through the caches the products of one row take 14.5 us for 67 / 90 MB (in sixteen rows by 64 bytes 18.7).  A norm in front costs vector
+// work per workgroup, so those take 16 rows: 32.3 and 36.5 us for 176 / 180 MB (in 8 rows 36.4 and 40.5, in sixteen by 64 bytes
+// 41.5 and 45).  Their weights come in two pieces at a time, one with two token tiles: all four would leave one workgroup per unit
 // (41.6 us) or spill (84).
 template <int DT>
 __device__ __forceinline__ floatx4 mma4(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1, floatx4 c) {
@@ -372,7 +249,7 @@ constexpr int kRowsWaves = 8, kRowsPieces = 4;
 constexpr int kRowsNormK = kRowsWaves * kRowsPieces * 128;  // longest row that is normalised on the way: one round of pieces
 
 template <int DT, int TT, int G, bool PAIR, int NORM>
-__global__ __launch_bounds__(kRowsWaves * kWave, 4) void rows_kernel(const SkinnyParams a) {
+__global__ __launch_bounds__(kRowsWaves * kWave, 4) void rows_kernel(const ProductParams a) {
   using E = Elem<DT>;
   constexpr int NW = kRowsWaves, U = kRowsPieces;
   constexpr int kRed = TT * G * 16;
@@ -581,6 +458,136 @@ __global__ __launch_bounds__(kRowsWaves * kWave, 4) void rows_kernel(const Skinn
     if (a.add1) v += E::load(a.add1 + to);
     if (a.add2) v += E::load(a.add2 + to);
     E::store(sg.out + to, v);
+  }
+}
+
+// ---- 2, 5, 6, 7 for more tokens: strips of 16 weight rows ----------------------
+// A wave asks for four rows by 128 values (256 contiguous bytes of each, with the non-temporal hint) at a time, as
+// rows_kernel does, but turns four such pieces, 16 rows by 128 values, through LDS of its own into the operands of
+// 16x16x32 products with 16 MT tokens: four accumulators a tile, where the 4x4x4 products of rows_kernel would take sixteen
+// (with 16 tokens 64 registers for 16 rows, 41 / 42 us for 176 / 180 MB).  A strip's registers take its next piece while
+// the products run.  x comes through the caches and holds up the weights (loads come back in order), so it comes
+// normalised and serves two strips (one: 1204 -> 1249 us for the step of four heads on 8 tokens of 16 sequences; four 1293).
+// In sixteen rows by 64 bytes straight into the operands, as this was before, that step took 1447 us, 16 sequences of two heads
+// 620 (577), of one 396 (374), 32 of four 1977 (1567); eight of four by rows_kernel 1259 (1093), five 1175 (1058).
+// Waves: few to a workgroup, so that there is little to add up (that step with 8 / 4 / 2 / 1 waves 1332 / 1256 / 1204 / 1199, 32
+// sequences 1781 / 1654 / 1567 / 1804, 16 of two heads 637 / 597 / 577 / 633), but four where fewer than 256 workgroups come
+// about (16 of one head 384 / 374 / 387 / 427).  One-strip products of 64 to 256 workgroups: eight (sixteen 1368 for 1332).
+// PAIR: the two strips are the same rows of two matrices and silu(a) b is stored; otherwise RT consecutive strips of one.
+constexpr int kTileNarrow = 8, kTileFull = 256;
+template <int DT, int MT, int RT, bool PAIR, int NW>
+__global__ __launch_bounds__(NW * kWave, MT == 1 ? 4 : 3) void tiles_kernel(const ProductParams a) {
+  using E = Elem<DT>;
+  constexpr int T = NW * kWave, kPitch = 128 + 8;
+  constexpr int kStage = NW * 16 * kPitch * 2, kRedBytes = NW * RT * MT * 1024;
+  __shared__ __align__(16) unsigned char raw[kStage > kRedBytes ? kStage : kRedBytes];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int blk = blockIdx.x, si = 0;
+  while (blk >= a.seg[si].blocks) blk -= a.seg[si++].blocks;
+  const Segment& sg = a.seg[si];
+  const int K = a.K, chunks = (K + 127) / 128;
+  const int per = (chunks - wave + NW - 1) / NW;
+  const int row0 = blk * (PAIR ? 16 : 16 * RT);
+  const int lq = lane >> 4, lc = (lane & 15) * 8;   // memory side: row of four, values of the piece
+  const int r = lane & 15, kg = lane >> 4;          // operand side: row (token), group of eight values
+  uint16_t* const stage = reinterpret_cast<uint16_t*>(raw) + wave * 16 * kPitch;
+  uint16_t* const put = stage + lq * kPitch + lc;
+  const uint16_t* const get = stage + r * kPitch + 8 * kg;
+
+  const uint16_t* wp[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+    wp[t] = (PAIR && t == 1 ? sg.W2 : sg.W) + static_cast<int64_t>(row0 + (PAIR ? 0 : 16 * t) + lq) * K;
+  const uint16_t* xp[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    const int m = 16 * t + r;
+    xp[t] = sg.x + static_cast<int64_t>(m < a.tokens ? m : 0) * K;
+  }
+  floatx4 acc[RT][MT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[t][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  u32x4 w[RT][4], x[MT][4], xn[MT][4];
+  auto first = [&](int c) { return 128 * (wave + NW * (c < per ? c : per - 1)); };  // (behind the end the last piece again, unused)
+  auto load_w = [&](int c, int t) {
+    const int k = first(c) + lc;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[t][i] = load_weights(wp[t] + static_cast<int64_t>(4 * i) * K + (k < K ? k : K - 8));
+  };
+  auto load_x = [&](int c, u32x4 (&to)[MT][4]) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int k = first(c) + 32 * s + 8 * kg;
+#pragma unroll
+      for (int m = 0; m < MT; ++m) to[m][s] = *reinterpret_cast<const u32x4*>(xp[m] + (k < K ? k : K - 8));
+    }
+  };
+  if (per > 0) {
+    load_x(0, xn);
+#pragma unroll
+    for (int t = 0; t < RT; ++t) load_w(0, t);
+  }
+  for (int c = 0; c < per; ++c) {
+    const int k0 = first(c);
+    const bool cut = k0 + 128 > K;
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) x[m][s] = cut && k0 + 32 * s + 8 * kg >= K ? zero : xn[m][s];
+    load_x(c + 1, xn);
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(put + 4 * i * kPitch) = cut && k0 + lc >= K ? zero : w[t][i];
+      load_w(c + 1, t);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_wave_barrier();
+      u32x4 f[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) f[s] = *reinterpret_cast<const u32x4*>(get + 32 * s);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[t][m] = mma16<DT>(f[s], x[m][s], acc[t][m]);
+      asm volatile("" ::: "memory");
+    }
+  }
+  __syncthreads();
+  float (*red)[RT * MT][4][kWave] = reinterpret_cast<float (*)[RT * MT][4][kWave]>(raw);
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) red[wave][t * MT + m][i][lane] = acc[t][m][i];
+  __syncthreads();
+  constexpr int kOuts = (PAIR ? 1 : RT) * MT * 256;
+  for (int o = tid; o < kOuts; o += T) {
+    const int tile = o >> 8, i = (o >> 6) & 3, ln = o & 63;
+    const int rt = tile / MT, m = 16 * (tile % MT) + (ln & 15);
+    const int row = row0 + 16 * rt + 4 * (ln >> 4) + i;
+    float v = 0.f;
+#pragma unroll
+    for (int q = 0; q < NW; ++q) v += red[q][tile][i][ln];
+    if (PAIR) {
+      float c = 0.f;
+#pragma unroll
+      for (int q = 0; q < NW; ++q) c += red[q][MT + tile][i][ln];
+      v = silu(round_to<DT>(v)) * round_to<DT>(c);
+    } else {
+      if (sg.bias) v += E::load(sg.bias + row);
+      if (sg.act) v = silu(round_to<DT>(v));
+    }
+    if (m < a.tokens) {
+      const int64_t at = static_cast<int64_t>(m) * sg.out_stride + row;
+      if (a.add1) v += E::load(a.add1 + at);
+      if (a.add2) v += E::load(a.add2 + at);
+      E::store(sg.out + at, v);
+    }
   }
 }
 
@@ -873,17 +880,23 @@ Layout layout_of(const mega_block_decode_args& a) {
 }
 
 template <int DT, int MT, int RT, bool PAIR, int NW>
-void skinny(const SkinnyParams& p, hipStream_t s) {
+void tiles_as(const ProductParams& p, int blocks, hipStream_t s) {
+  tiles_kernel<DT, MT, RT, PAIR, NW><<<blocks, NW * kWave, 0, s>>>(p);
+}
+template <int DT, int MT, int RT, bool PAIR>
+void tiles(const ProductParams& p, hipStream_t s) {
   int blocks = 0;
   for (int i = 0; i < p.segs; ++i) blocks += p.seg[i].blocks;
-  skinny_kernel<DT, MT, RT, PAIR, NW><<<blocks, NW * kWave, 0, s>>>(p);
+  if constexpr (RT == 1) tiles_as<DT, MT, RT, PAIR, kTileNarrow>(p, blocks, s);
+  else if (blocks < kTileFull) tiles_as<DT, MT, RT, PAIR, 4>(p, blocks, s);
+  else tiles_as<DT, MT, RT, PAIR, 2>(p, blocks, s);
 }
 
-// Tokens that rows_kernel takes: at eight it is still ahead at every width (4 heads of 1024 features 1603 -> 1565 us for
-// eight tokens, 1 head 361 -> 326); sixteen would need 64 accumulators a row group and spill (2 heads 646 -> 905).
-constexpr int kRowsTokens = 8;
+// Whether the products are rows_kernel's: up to four tokens, and up to eight in narrow blocks (us, rows_kernel / tiles_kernel: eight
+// sequences of one head of 1024 features 324 / 363, of two 522 / 506, of four 1259 / 1093; one of four 974 / 1090).
+bool few_rows(int B, int D) { return D <= kRowsNormK && B <= (D < 2048 ? 8 : 4); }
 template <int DT, int TT, int G, bool PAIR, int NORM>
-void rows(SkinnyParams p, hipStream_t s) {
+void rows(ProductParams p, hipStream_t s) {
   int blocks = 0;
   for (int i = 0; i < p.segs; ++i) blocks += p.seg[i].blocks;
   rows_kernel<DT, TT, G, PAIR, NORM><<<blocks, kRowsWaves * kWave, 0, s>>>(p);
@@ -913,7 +926,7 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
     step_kernel<DT><<<dim3(D / kStepChannels, B), 256, 0, s>>>(p);
   }
   const uint16_t* none = nullptr;
-  const bool few = B <= kRowsTokens && D <= kRowsNormK;  // by rows_kernel
+  const bool few = few_rows(B, D);
   const int wide = 4, narrow = B <= 4 ? 1 : 2;  // row groups of a workgroup
   auto seg = [&](const void* W, const void* W2, const void* bias, const uint16_t* x, uint16_t* out, int64_t stride,
                  int rows, int strip, int norm, int act) {
@@ -923,7 +936,7 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
     if (!few)
       rows_norm_kernel<DT, kNormRms><<<B, kNormThreads, 0, s>>>(at16(l.cema), u16(a.rms_weight), none, at16(l.normed), D, a.rms_eps);
     const uint16_t* row = at16(few ? l.cema : l.normed);
-    SkinnyParams p{};
+    ProductParams p{};
     // the wide layers first: the narrow one fills the gaps at the end
     p.seg[0] = seg(a.wv, none, a.bv, at16(l.tsn), static_cast<uint16_t*>(a.v_out) + a.length * a.E,
                    (a.length + 1) * a.E, E, 32, kNormNone, 1);
@@ -933,7 +946,7 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
     p.segs = 4, p.K = D, p.tokens = B;
     p.norm_weight = u16(a.rms_weight);
     p.eps = a.rms_eps;
-    if (!few) skinny<DT, MT, 2, false, kWavesWide>(p, s);
+    if (!few) tiles<DT, MT, 2, false>(p, s);
     else if (B <= 4) rows<DT, 1, 4, false, kNormRms>(p, s);
     else rows<DT, 2, 4, false, kNormRms>(p, s);
   }
@@ -955,32 +968,32 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
     combine_kernel<DT><<<dim3(H2 / 64, B * H), 256, 0, s>>>(p);
   }
   {
-    SkinnyParams p{};
+    ProductParams p{};
     p.seg[0] = seg(a.wh2, none, none, at16(l.attn), at16(l.y1), D, D, 16, kNormNone, 0);
     p.segs = 1, p.K = E, p.tokens = B;
     p.add1 = at16(l.h1), p.add2 = u16(a.x);
-    if (!few) skinny<DT, MT, 1, false, kWavesNarrow>(p, s);
+    if (!few) tiles<DT, MT, 1, false>(p, s);
     else if (B <= 4) rows<DT, 1, 1, false, kNormNone>(p, s);
     else rows<DT, 2, 2, false, kNormNone>(p, s);
   }
   {
     if (!few)
       rows_norm_kernel<DT, kNormLayer><<<B, kNormThreads, 0, s>>>(at16(l.y1), u16(a.ln_weight), u16(a.ln_bias), at16(l.normed), D, a.ln_eps);
-    SkinnyParams p{};
+    ProductParams p{};
     p.seg[0] = seg(a.fc1, a.fc3, none, at16(few ? l.y1 : l.normed), at16(l.hidden), F, F, 16, kNormLayer, 0);
     p.segs = 1, p.K = D, p.tokens = B;
     p.norm_weight = u16(a.ln_weight), p.norm_bias = u16(a.ln_bias);
     p.eps = a.ln_eps;
-    if (!few) skinny<DT, MT, 2, true, kWavesWide>(p, s);
+    if (!few) tiles<DT, MT, 2, true>(p, s);
     else if (B <= 4) rows<DT, 1, 4, true, kNormLayer>(p, s);
     else rows<DT, 2, 4, true, kNormLayer>(p, s);
   }
   {
-    SkinnyParams p{};
+    ProductParams p{};
     p.seg[0] = seg(a.fc2, none, none, at16(l.hidden), static_cast<uint16_t*>(a.y), D, D, 16, kNormNone, 0);
     p.segs = 1, p.K = F, p.tokens = B;
     p.add1 = u16(a.x);
-    if (!few) skinny<DT, MT, 1, false, kWavesNarrow>(p, s);
+    if (!few) tiles<DT, MT, 1, false>(p, s);
     else if (B <= 4) rows<DT, 1, 1, false, kNormNone>(p, s);
     else rows<DT, 2, 2, false, kNormNone>(p, s);
   }
