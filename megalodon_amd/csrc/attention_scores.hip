@@ -424,20 +424,28 @@ __global__ __launch_bounds__(64 * kWaves) void attn_probs_kernel(const ProbsPara
 // Row blocks of 256 leave the chip idle at ordinary sizes (four heads and 1531 steps: 24 workgroups walk their keys
 // twice, 83 us).  Here a workgroup owns 32 query rows and its eight waves share out the keys, 32-key block
 // b to wave b % 8, so every wave holds all of its scores (KB blocks of 16 registers) at once: one pass, the row
-// maximum and the row sum combined over the waves through LDS (33 us).  A wave's keys are its own, so their
-// fragments come from memory straight into registers, a ring of RING fragments ahead of the products.
+// maximum and the row sum combined over the waves through LDS.  A wave's keys are its own: pieces of 32 keys by 64 values come in
+// whole cache lines, RING of them ahead of the products, and are turned into operands through LDS of the wave's own.  Straight into the
+// operands, 32 bytes of 32 rows a request, a line was asked for four times and had left the cache in between: the layer's forward
+// with a value head of 64, us before / now: 1531 keys, four heads of 256 46.0 / 32.8; 4 x 1024, one head 32.7 / 24.1; 4000, two heads
+// 125 / 77; 2 x 2048, four heads of 128 50 / 39; 4 x 1024, four of 64 23.3 / 19.8; 300 keys 16.7 / 13.8.  (Without the piece behind the
+// last block, which is asked for again, +- 0.)
 // Rows of more than 256 KB keys (SEGMENTS) pass in pieces of that many keys: running maxima and sums, then the
-// probabilities of the last piece, whose scores are still there, and of the others from products formed again.
+// probabilities of the last piece, whose scores are still there, and of the others from products formed again.  (At
+// width 256 with one piece on its way: two spilled 18 registers, 300 x 4000 at two blocks a CU 329 us for 304.)
 // Every row block reads its keys from the L2 anew, which is what bounds full grids: those take the kernel above.
 template <int DT, int H1, int KB, bool SEGMENTS>
 __global__ __launch_bounds__(64 * kWaves) void attn_probs_short_kernel(const ProbsParams p) {
   constexpr int QF = H1 / 16;
-  constexpr int RING = KB > 4 && QF > 8 ? 8 : QF;
+  constexpr int PIECES = QF / 4, RING = KB > 4 && PIECES > 2 ? (SEGMENTS ? 1 : 2) : PIECES, kPitch = 64 + 8;
   constexpr int STEP = KB * kWaves;  // 32-key blocks of a piece
   __shared__ float red[2][kWaves][32];
+  __shared__ __align__(16) uint16_t stage[kWaves][32 * kPitch];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
   const int r = lane & 31, h = lane >> 5;
+  uint16_t* const put = stage[wave] + (lane >> 3) * kPitch + (lane & 7) * 8;
+  const uint16_t* const get = stage[wave] + r * kPitch + 8 * h;
   const int idx = static_cast<int>(blockIdx.x);
   const int mt = p.MT - 1 - idx / p.Z, z = idx % p.Z;  // long rows first
   const int b = z / p.NH, hd = z % p.NH;
@@ -450,10 +458,15 @@ __global__ __launch_bounds__(64 * kWaves) void attn_probs_short_kernel(const Pro
   const int nblk = (kend + 31) / 32;
   const int lim = p.causal ? min(row + p.off, p.L2 - 1) : p.L2 - 1;  // last key of this lane's row
 
-  // lane (r, h) holds k = 16 f + 8 h .. + 7 of fragment f, of its query row and of key r of a block
-  const uint16_t* kbase = K + 8 * h;
-  const auto key_row = [&](int blk) { return kbase + static_cast<int64_t>(min(32 * blk + r, p.L2 - 1)) * ld; };
-  u32x4 kf[RING], qf[QF];
+  // Operands: lane (r, h) holds k = 16 f + 8 h .. + 7 of fragment f, of its query row and of key r of a block.
+  // Memory side: request i of a piece of 32 keys by 64 values takes key 8 i + lane / 8, whole cache lines
+  const int key = lane >> 3, col = (lane & 7) * 8;
+  const auto load_piece = [&](int blk, int piece, u32x4* to) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      to[i] = *reinterpret_cast<const u32x4*>(K + static_cast<int64_t>(min(32 * blk + 8 * i + key, p.L2 - 1)) * ld + 64 * piece + col);
+  };
+  u32x4 kf[4 * RING], qf[QF];
   {
     const uint16_t* qr = Q + static_cast<int64_t>(min(row, p.L1 - 1)) * ld + 8 * h;
 #pragma unroll
@@ -463,21 +476,28 @@ __global__ __launch_bounds__(64 * kWaves) void attn_probs_short_kernel(const Pro
   // 32 (b0 + wave + 8 i) + 8 (e / 4) + 4 h + e % 4
   floatx16 acc[KB];
   const auto scores = [&](int b0) {
-    const uint16_t* first = key_row(b0 + wave);
 #pragma unroll
-    for (int f = 0; f < RING; ++f) kf[f] = *reinterpret_cast<const u32x4*>(first + 16 * f);
+    for (int n = 0; n < RING; ++n) load_piece(b0 + wave, n, kf + 4 * n);
 #pragma unroll
     for (int i = 0; i < KB; ++i) {
       const int blk = b0 + wave + kWaves * i;
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
       if (blk < nblk) {
-        const uint16_t* here = key_row(blk);
-        const uint16_t* next = key_row(blk + kWaves);  // (clamped into the keys)
 #pragma unroll
-        for (int f = 0; f < QF; ++f) {
-          acc[i] = mma16<DT>(kf[f % RING], qf[f], acc[i]);
-          kf[f % RING] = *reinterpret_cast<const u32x4*>(f + RING < QF ? here + 16 * (f + RING) : next + 16 * (f + RING - QF));
+        for (int n = 0; n < PIECES; ++n) {
+          u32x4* const here = kf + 4 * (n % RING);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4*>(put + 8 * j * kPitch) = here[j];
+          if (n + RING < PIECES) load_piece(blk, n + RING, here);
+          else load_piece(blk + kWaves, n + RING - PIECES, here);  // (clamped into the keys)
+          asm volatile("" ::: "memory");
+          u32x4 f[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) f[j] = *reinterpret_cast<const u32x4*>(get + 16 * j);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[i] = mma16<DT>(f[j], qf[4 * n + j], acc[i]);
+          asm volatile("" ::: "memory");
         }
         const int x0 = 32 * blk + 4 * h;
 #pragma unroll
@@ -602,34 +622,37 @@ int launch_probs_short(ProbsParams p, hipStream_t s) {
 // its time grows with the blocks and with the head's width, while the other one's is its longest row block's until the chip
 // is full; keys that a causal block does not see are left out by both, but only the other one waits for its longest.  The
 // operator's forward with a value head of 64, time of the other kernel over the short-row kernel's, at blocks a CU:
-//   causal squares  width 64:  256 keys 4.0 1.19, 5.0 0.96; 512 keys 5.0 1.13, 6.0 1.02; 1500 keys 5.0 1.15, 5.9 1.11; 4096 keys 5.5 1.07, 6.0 0.98
-//                   width 128: 256 keys 3.0 1.13, 3.3 0.96; 512 keys 4.0 1.07, 4.5 0.93; 1500 keys 3.9 1.20, 5.0 0.99; 4096 keys 4.0 1.08, 4.5 0.99
-//                   width 256: 100 keys 1.3 1.04, 1.5 0.94; 256 keys 2.0 1.08, 2.3 0.83; 512 keys 2.0 1.27, 2.3 0.96; 700 keys 3.0 1.02, 3.2 0.84; 2048
-//                              keys 3.3 1.14, 4.5 0.89; 4096 keys 3.0 1.08, 3.5 0.95
-//   causal, more keys than rows (the first rows see most of them)
-//                   width 64:  256 x 1024 5.0 1.02, 5.5 0.93; 1024 x 1536 4.0 1.10, 5.0 0.97; 100 x 1500 5.5 1.24; 1024 x 2048 4.0 1.12, 4.5 0.97
-//                   width 128: 256 x 384 3.0 1.12, 3.3 0.95; 1024 x 2048 3.0 1.11, 3.3 0.95
-//                   width 256: 256 x 1024 2.0 1.16, 2.3 0.90; 1024 x 1280 3.0 1.03, 3.3 0.90
-//   without a mask  width 64:  256 keys 2.0 1.08, 3.0 0.91; 384 keys 4.0 1.08, 4.5 0.87; 512 keys 3.3 1.05, 3.5 0.94; 1024 keys 4.0 1.09, 5.5 0.92; 1500
-//                              keys 3.5 1.06, 4.0 0.99; 4096 keys 3.0 1.10, 3.5 0.89
-//                   width 128: 256 keys 2.0 1.00, 2.3 0.86; 1024 keys 3.0 1.05, 3.3 0.92; 4096 keys 2.0 1.18, 2.5 0.87
-//                   width 256: 256 keys 1.0 1.31, 1.3 0.89; 512 keys 2.0 0.99, 2.3 0.79; 1024 keys 2.0 1.09, 2.3 0.84; 4096 keys 1.0 1.61, 1.5 0.96
-// (three blocks a CU for all of them before; with the lines of causal squares for all of them, 3.5 blocks of 256 keys without
-// a mask at width 64 took 24.4 us instead of 19.9, 4 of 4096 at width 128 322 instead of 257.)
+//   causal squares  width 64:  200 keys 5.9 1.06; 256 keys 5.0 1.10, 7.0 0.94; 512 keys 6.0 1.18; 1024 keys 6.0 1.30; 1500 keys 5.7 1.07, 6.1 1.00; 4096 keys 6.0
+//                              1.14, 8.0 0.96
+//                   width 128: 64 keys 1.8 0.84, 2.3 1.00; 256 keys 3.0 1.13, 4.0 0.93; 512 keys 4.0 1.19, 5.0 0.98; 700 keys 3.0 1.13, 4.0 0.95; 850 keys 4.2
+//                              1.27; 1024 keys 4.3 1.12, 4.6 0.90; 4096 keys 4.5 1.28
+//                   width 256: 64 keys 1.3 0.75; 100 keys 2.0 1.04, 2.5 0.86; 256 keys 2.0 1.28, 2.5 1.01; 384 keys 2.3 1.19, 2.5 0.95; 700 keys 2.5 1.18, 3.0
+//                              0.94; 850 keys 3.2 1.29, 3.5 0.97; 1500 keys 4.0 1.32, 4.6 0.98; 4096 keys 4.0 1.37, 4.5 1.08
+//   causal, more keys than rows (the first rows see most of them; more than 2048 go in pieces)
+//                   width 64:  100 x 400 5.9 1.40; 256 x 1024 5.0 1.06, 6.0 0.98; 1024 x 1280 4.8 1.02, 5.3 0.93; 600 x 3000 3.3 1.16, 3.7 0.91
+//                   width 128: 100 x 400 2.7 1.12, 3.2 0.94; 300 x 600 2.7 1.13, 3.2 0.97; 1024 x 1280 3.8 1.09, 4.3 0.96; 600 x 3000 2.7 1.30, 3.2 0.72
+//                   width 256: 100 x 400 2.8 1.07; 300 x 600 2.5 1.28, 2.7 0.98; 1024 x 1280 4.0 1.10, 4.5 0.97; 600 x 3000 1.8 1.56, 2.5 0.88
+//   without a mask  width 64:  100 x 1000 5.9 1.43; 256 keys 2.0 1.14, 3.0 0.97; 384 keys 3.7 1.16, 4.3 0.99; 1024 keys 5.0 1.10, 6.0 0.98; 4096 keys 4.0 1.07, 5.0 0.94
+//                   width 128: 256 keys 2.0 1.04, 3.0 0.86; 384 keys 2.7 1.15, 3.2 0.92; 1300 keys 3.2 1.18, 3.7 0.96; 4096 keys 3.0 1.19, 4.0 1.02
+//                   width 256: 256 keys 2.0 1.04, 2.5 0.85; 384 keys 1.7 1.17, 2.3 0.95; 1024 keys 3.0 1.19, 4.0 0.97; 2500 keys 2.5 1.10, 2.8 0.97
+// (While the keys came by 32 bytes of a row the lines lay at 1.3 to 5.5 blocks; over 900 sizes of 64 to 4096 keys at up to 12 blocks
+// the better of the two kernels at every one would be 1.6 % ahead of these lines, 3.8 % of those.)
 constexpr int short_rows(int H1, int rows, int keys, bool causal) {
   if (causal && rows == keys) {
-    if (H1 == 64) return keys <= 384 ? 32 : 44;
-    if (H1 == 128) return keys <= 384 ? 24 : 32;
-    return keys <= 128 ? 10 : keys <= 544 ? 16 : keys <= 1280 ? 24 : 26;
+    if (H1 == 64) return keys <= 384 ? 42 : 48;
+    if (H1 == 128) return keys <= 72 ? 14 : keys <= 384 ? 24 : keys <= 544 ? 32 : keys <= 768 ? 28 : 36;
+    return keys <= 72 ? 8 : keys <= 128 ? 16 : keys <= 384 ? 19 : keys <= 768 ? 22 : keys <= 1152 ? 28 : 34;
   }
   if (causal) {
-    if (H1 == 64) return rows <= 128 ? 44 : keys <= 1536 ? 40 : 32;
-    if (H1 == 128) return 24;
-    return keys > 1024 && 2 * rows >= keys ? 24 : 16;
+    const bool half = keys > 1024 && 2 * rows >= keys;
+    if (keys > 2048 && !half) return H1 == 64 ? 27 : H1 == 128 ? 24 : 16;
+    if (H1 == 64) return rows <= 128 ? 47 : 40;
+    if (H1 == 128) return half ? 32 : 25;
+    return half ? 33 : 22;
   }
-  if (H1 == 64) return keys <= 288 ? 24 : keys <= 384 ? 32 : keys <= 544 ? 26 : keys <= 1152 ? 40 : keys <= 1536 ? 28 : 24;
-  if (H1 == 128) return keys <= 288 || keys > 3072 ? 16 : 24;
-  return keys <= 288 || keys > 3072 ? 8 : 16;
+  if (H1 == 64) return rows <= 128 && keys >= 512 ? 47 : keys <= 288 ? 22 : keys <= 768 ? 33 : keys <= 1152 ? 41 : 32;
+  if (H1 == 128) return keys <= 288 ? 16 : keys <= 768 ? 22 : 27;
+  return keys <= 384 ? 16 : keys <= 768 ? 20 : keys <= 1536 ? 24 : 20;
 }
 
 template <int DT, int H1>
