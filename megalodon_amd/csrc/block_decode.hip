@@ -466,7 +466,9 @@ __global__ __launch_bounds__(kRowsWaves * kWave, 4) void rows_kernel(const Produ
 // rows_kernel does, but turns four such pieces, 16 rows by 128 values, through LDS of its own into the operands of
 // 16x16x32 products with 16 MT tokens: four accumulators a tile, where the 4x4x4 products of rows_kernel would take sixteen
 // (with 16 tokens 64 registers for 16 rows, 41 / 42 us for 176 / 180 MB).  A strip's registers take its next piece while
-// the products run.  x comes through the caches and holds up the weights (loads come back in order), so it comes
+// the products run, and x's its next one behind them: a second set for x and a piece behind the last one asked for again cost 1 to 8 %
+// (eight tokens of 16 sequences of four, two, one heads 1151, 575, 375 -> 1113, 567, 365 us; of 32, 24, 24 1528, 700, 449 -> 1490, 679, 416),
+// two pieces of everything on their way +- 0.  x comes through the caches and holds up the weights (loads come back in order), so it comes
 // normalised and serves two strips (one: 1204 -> 1249 us for the step of four heads on 8 tokens of 16 sequences; four 1293).
 // In sixteen rows by 64 bytes straight into the operands, as this was before, that step took 1447 us, 16 sequences of two heads
 // 620 (577), of one 396 (374), 32 of four 1977 (1567); eight of four by rows_kernel 1259 (1093), five 1175 (1058).
@@ -510,42 +512,35 @@ __global__ __launch_bounds__(NW * kWave, MT == 1 ? 4 : 3) void tiles_kernel(cons
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[t][m] = floatx4{0.f, 0.f, 0.f, 0.f};
   const u32x4 zero = {0u, 0u, 0u, 0u};
-  u32x4 w[RT][4], x[MT][4], xn[MT][4];
-  auto first = [&](int c) { return 128 * (wave + NW * (c < per ? c : per - 1)); };  // (behind the end the last piece again, unused)
+  u32x4 w[RT][4], x[MT][4];
   auto load_w = [&](int c, int t) {
-    const int k = first(c) + lc;
+    const int k = 128 * (wave + NW * c) + lc;
 #pragma unroll
     for (int i = 0; i < 4; ++i) w[t][i] = load_weights(wp[t] + static_cast<int64_t>(4 * i) * K + (k < K ? k : K - 8));
   };
-  auto load_x = [&](int c, u32x4 (&to)[MT][4]) {
+  auto load_x = [&](int c) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      const int k = first(c) + 32 * s + 8 * kg;
+      const int k = 128 * (wave + NW * c) + 32 * s + 8 * kg;
 #pragma unroll
-      for (int m = 0; m < MT; ++m) to[m][s] = *reinterpret_cast<const u32x4*>(xp[m] + (k < K ? k : K - 8));
+      for (int m = 0; m < MT; ++m) x[m][s] = *reinterpret_cast<const u32x4*>(xp[m] + (k < K ? k : K - 8));
     }
   };
-  if (per > 0) {
-    load_x(0, xn);
+  // piece c; its registers take the next one as they are read
+  auto piece = [&](int c, bool more) {
+    const int k0 = 128 * (wave + NW * c);
+    const bool cut = k0 + 128 > K;  // lanes behind the row's end
+    if (cut)
 #pragma unroll
-    for (int t = 0; t < RT; ++t) load_w(0, t);
-  }
-  for (int c = 0; c < per; ++c) {
-    const int k0 = first(c);
-    const bool cut = k0 + 128 > K;
+      for (int s = 0; s < 4; ++s)
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-      for (int s = 0; s < 4; ++s) x[m][s] = cut && k0 + 32 * s + 8 * kg >= K ? zero : xn[m][s];
-    load_x(c + 1, xn);
+        for (int m = 0; m < MT; ++m) x[m][s] = k0 + 32 * s + 8 * kg >= K ? zero : x[m][s];
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
-      __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(put + 4 * i * kPitch) = cut && k0 + lc >= K ? zero : w[t][i];
-      load_w(c + 1, t);
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_wave_barrier();
+      if (more) load_w(c + 1, t);
+      asm volatile("" ::: "memory");  // (a wave's LDS accesses are served in order)
       u32x4 f[4];
 #pragma unroll
       for (int s = 0; s < 4; ++s) f[s] = *reinterpret_cast<const u32x4*>(get + 32 * s);
@@ -555,6 +550,14 @@ __global__ __launch_bounds__(NW * kWave, MT == 1 ? 4 : 3) void tiles_kernel(cons
         for (int m = 0; m < MT; ++m) acc[t][m] = mma16<DT>(f[s], x[m][s], acc[t][m]);
       asm volatile("" ::: "memory");
     }
+    if (more) load_x(c + 1);
+  };
+  if (per > 0) {
+    load_x(0);
+#pragma unroll
+    for (int t = 0; t < RT; ++t) load_w(0, t);
+    for (int c = 0; c + 1 < per; ++c) piece(c, true);
+    piece(per - 1, false);
   }
   __syncthreads();
   float (*red)[RT * MT][4][kWave] = reinterpret_cast<float (*)[RT * MT][4][kWave]>(raw);
