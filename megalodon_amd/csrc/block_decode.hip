@@ -209,7 +209,7 @@ __global__ __launch_bounds__(kNormThreads) void rows_norm_kernel(const uint16_t*
 // What the layout is for: 256 bytes of a row in one request with the non-temporal hint, and many small workgroups, which the
 // hardware hands out as others end.  Reading alone, 176 MB in four rows a workgroup take 26.5 us (6.6 TB/s; without the hint
 // 28.5), in sixteen rows by 64 bytes 33, and by one workgroup per compute unit with an equal share each 52.  With that and x
-// through the caches the products of one row take 14.5 us for 67 / 90 MB (in sixteen rows by 64 bytes 18.7).  A norm in front costs vector
+// through the caches the products of one row take 14.5 us for 67 / 90 MB (in sixteen rows by 64 bytes 18.7).  A norm on the way costs vector
 // work per workgroup, so those take 16 rows: 32.3 and 36.5 us for 176 / 180 MB (in 8 rows 36.4 and 40.5, in sixteen by 64 bytes
 // 41.5 and 45).  Their weights come in two pieces at a time, one with two token tiles: all four would leave one workgroup per unit
 // (41.6 us) or spill (84).
@@ -897,6 +897,9 @@ void tiles(const ProductParams& p, hipStream_t s) {
 
 // Whether the products are rows_kernel's: up to four tokens, and up to eight in narrow blocks (us, rows_kernel / tiles_kernel: eight
 // sequences of one head of 1024 features 324 / 363, of two 522 / 506, of four 1259 / 1093; one of four 974 / 1090).
+// Their norms come on the way, each workgroup's for itself, while that costs less than a launch: in front of fc1 and fc3 up to 2048
+// features (us, on the way / ahead, four rows of each a workgroup: one sequence of two heads 417 / 417, four 424 / 432; of three 628 / 605, 816 / 807;
+// of four 970 / 928, 1604 / 1586), in front of z, r and h1 but for one sequence of 4096 (928 / 908; two 877 / 883, one of three heads 605 / 610).
 bool few_rows(int B, int D) { return D <= kRowsNormK && B <= (D < 2048 ? 8 : 4); }
 template <int DT, int TT, int G, bool PAIR, int NORM>
 void rows(ProductParams p, hipStream_t s) {
@@ -930,26 +933,29 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
   }
   const uint16_t* none = nullptr;
   const bool few = few_rows(B, D);
-  const int wide = 4, narrow = B <= 4 ? 1 : 2;  // row groups of a workgroup
+  const bool front = !few || (B == 1 && D >= 4096), behind = !few || D > 2048;  // whether the norms have launches of their own
+  // rows of a workgroup: of z, r, h1 and v, of fc1 and fc3 (a pair), of wh2 and fc2
+  const int wide = !few ? 32 : front ? 4 : 16, pair = !few ? 16 : behind ? 4 : 8, narrow = !few ? 16 : B <= 4 ? 4 : 8;
   auto seg = [&](const void* W, const void* W2, const void* bias, const uint16_t* x, uint16_t* out, int64_t stride,
                  int rows, int strip, int norm, int act) {
-    return Segment{u16(W), u16(W2), u16(bias), x, out, stride, rows / (few ? (W2 ? 2 * wide : strip == 32 ? 4 * wide : 4 * narrow) : strip), norm, act};
+    return Segment{u16(W), u16(W2), u16(bias), x, out, stride, rows / strip, norm, act};
   };
   {
-    if (!few)
+    if (front)
       rows_norm_kernel<DT, kNormRms><<<B, kNormThreads, 0, s>>>(at16(l.cema), u16(a.rms_weight), none, at16(l.normed), D, a.rms_eps);
-    const uint16_t* row = at16(few ? l.cema : l.normed);
+    const uint16_t* row = at16(front ? l.normed : l.cema);
     ProductParams p{};
     // the wide layers first: the narrow one fills the gaps at the end
     p.seg[0] = seg(a.wv, none, a.bv, at16(l.tsn), static_cast<uint16_t*>(a.v_out) + a.length * a.E,
-                   (a.length + 1) * a.E, E, 32, kNormNone, 1);
-    p.seg[1] = seg(a.wr, none, a.br, row, at16(l.r), E, E, 32, kNormRms, 0);
-    p.seg[2] = seg(a.wh1, none, a.bh1, row, at16(l.h1), D, D, 32, kNormRms, 0);
-    p.seg[3] = seg(a.wz, none, a.bz, row, at16(l.z), S, S, 32, kNormRms, 0);
+                   (a.length + 1) * a.E, E, wide, kNormNone, 1);
+    p.seg[1] = seg(a.wr, none, a.br, row, at16(l.r), E, E, wide, kNormRms, 0);
+    p.seg[2] = seg(a.wh1, none, a.bh1, row, at16(l.h1), D, D, wide, kNormRms, 0);
+    p.seg[3] = seg(a.wz, none, a.bz, row, at16(l.z), S, S, wide, kNormRms, 0);
     p.segs = 4, p.K = D, p.tokens = B;
     p.norm_weight = u16(a.rms_weight);
     p.eps = a.rms_eps;
     if (!few) tiles<DT, MT, 2, false>(p, s);
+    else if (front) rows<DT, 1, 1, false, kNormNone>(p, s);
     else if (B <= 4) rows<DT, 1, 4, false, kNormRms>(p, s);
     else rows<DT, 2, 4, false, kNormRms>(p, s);
   }
@@ -972,7 +978,7 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
   }
   {
     ProductParams p{};
-    p.seg[0] = seg(a.wh2, none, none, at16(l.attn), at16(l.y1), D, D, 16, kNormNone, 0);
+    p.seg[0] = seg(a.wh2, none, none, at16(l.attn), at16(l.y1), D, D, narrow, kNormNone, 0);
     p.segs = 1, p.K = E, p.tokens = B;
     p.add1 = at16(l.h1), p.add2 = u16(a.x);
     if (!few) tiles<DT, MT, 1, false>(p, s);
@@ -980,20 +986,21 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
     else rows<DT, 2, 2, false, kNormNone>(p, s);
   }
   {
-    if (!few)
+    if (behind)
       rows_norm_kernel<DT, kNormLayer><<<B, kNormThreads, 0, s>>>(at16(l.y1), u16(a.ln_weight), u16(a.ln_bias), at16(l.normed), D, a.ln_eps);
     ProductParams p{};
-    p.seg[0] = seg(a.fc1, a.fc3, none, at16(few ? l.y1 : l.normed), at16(l.hidden), F, F, 16, kNormLayer, 0);
+    p.seg[0] = seg(a.fc1, a.fc3, none, at16(behind ? l.normed : l.y1), at16(l.hidden), F, F, pair, kNormLayer, 0);
     p.segs = 1, p.K = D, p.tokens = B;
     p.norm_weight = u16(a.ln_weight), p.norm_bias = u16(a.ln_bias);
     p.eps = a.ln_eps;
     if (!few) tiles<DT, MT, 2, true>(p, s);
+    else if (behind) rows<DT, 1, 2, true, kNormNone>(p, s);
     else if (B <= 4) rows<DT, 1, 4, true, kNormLayer>(p, s);
     else rows<DT, 2, 4, true, kNormLayer>(p, s);
   }
   {
     ProductParams p{};
-    p.seg[0] = seg(a.fc2, none, none, at16(l.hidden), static_cast<uint16_t*>(a.y), D, D, 16, kNormNone, 0);
+    p.seg[0] = seg(a.fc2, none, none, at16(l.hidden), static_cast<uint16_t*>(a.y), D, D, narrow, kNormNone, 0);
     p.segs = 1, p.K = F, p.tokens = B;
     p.add1 = u16(a.x);
     if (!few) tiles<DT, MT, 1, false>(p, s);
