@@ -667,7 +667,8 @@ int mega_cema_scan_fwd(const void* x, int dtype, const float* p, const float* lo
                        int64_t D, int64_t N, int64_t L, void* y, float* h_last, void* stream);
 
 /* mega_cema_scan_fwd for the layer: float32 rows (16-byte aligned) of any L >= 1 too.  Those whose length is no multiple of
- * 8 enter the products with all their bits and come out as the matrices' 24 give them (mega_cema_layer_fwd the same). */
+ * 8 enter the products with all their 24 bits, as do the matrices and the state between chunks (mega_cema_layer_fwd and, for
+ * a float32 dx, mega_cema_layer_scan_bwd the same). */
 int mega_cema_layer_scan_fwd(const void* x, int dtype, const float* p, const float* log_q,
                              const float* gamma, const float* omega, const float* h0, int64_t B,
                              int64_t D, int64_t N, int64_t L, void* y, float* h_last, void* stream);

@@ -18,7 +18,8 @@
 // chunk), and y is written once from the accumulators.  Parameter matrices are
 // float32 values split into two bf16 pieces (hi + lo, 16 significant bits; some have a third, see kFine); x in
 // bf16 is exact, fp16 x is split into two exact bf16 pieces; the states are
-// float32 and split the same way; accumulation is float32.
+// float32 and split the same way (where float32 rows need more, the state's products are float32 ones, see XOpWide);
+// accumulation is float32.
 //
 // One workgroup of four waves owns a channel's rows: one of them, or, where the batch has several,
 // as many as still leave a workgroup for every slot of the chip.  Setting up the channel's parameter
@@ -122,6 +123,17 @@ __device__ __forceinline__ void put_pair(u32x4 (*blocks)[2][kWave], int n, int i
   const uint32_t h = pack_bf16x2(a, b);
   reinterpret_cast<uint32_t*>(&blocks[blk][0][ln])[n & 3] = h;
   reinterpret_cast<uint32_t*>(&blocks[blk][1][ln])[n & 3] = pack_bf16x2(a - __uint_as_float(h << 16), b - __uint_as_float(h & 0xffff0000u));
+}
+// ... as they are, two words of four floats a lane where put_pair has two pieces of eight
+__device__ __forceinline__ void put_pair_f32(u32x4 (*blocks)[2][kWave], int n, int i, float a, float b) {
+  const int blk = 2 * (i >> 5) + (n >> 3), ln = (i & 31) + 32 * ((n >> 2) & 1);
+  reinterpret_cast<float2*>(&blocks[blk][(n >> 1) & 1][ln])[n & 1] = make_float2(a, b);
+}
+// acc += A B over 16 columns: lane (r, g) holds row (column) r and the values 8 g .. + 7 of both
+__device__ __forceinline__ floatx16 mma_f32(const u32x4* a, const float* b, floatx16 acc) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[e >> 2][e & 3]), b[e], acc, 0, 0, 0);
+  return acc;
 }
 // Third pieces of k[0 .. 63] for the Toeplitz blocks, whose lanes read eight consecutive lags each: one table of the
 // lags in the blocks' order, zeros at negative ones, and a second one that starts an element later, so that every
@@ -318,9 +330,16 @@ template <> struct XOp<MEGA_F32> {
   }
 };
 
-// float32 rows of the other layouts: all three pieces, 24 significant bits, as their matrices carry.  (They went through a
-// float32 kernel row and float32 transforms: y 2.8e-6 - 3.4e-6 from 64 bits in the 2-norm, now 4.2e-7 - 6.0e-7, gradients nowhere
-// further off than they were.  1024 rows of 51151 steps forward 1974 -> 124 us, 4096 of 201 50.6 -> 16.3.)
+// float32 rows of the other layouts: all three pieces, 24 significant bits, as P and K carry.  The state's share of the outputs (Q H, and
+// in the backward Qd R) is a product of float32 matrix instructions, whose operands lie where the others' two pieces do: in two
+// pieces each it was good to 2^-18, which is most of what y and dx are off where memories are long.  Against 64 bits on the same
+// float32 coefficients, all of 64 channels in the 2-norm / the channel that is furthest off, 121 and 4097 steps with and without a mean: at the
+// initial decays 1.7e-7 / 2.9e-6 (in pieces 4.8e-7 / 3.1e-5), at ten times slower ones 2.1e-7 / 6.6e-7 (1.8e-6 / 1.2e-5), at a hundred times
+// slower 4.6e-7 / 7.2e-7 (4.1e-6 / 6.2e-6).  It costs 3 to 16 %: forward, 1024 rows of 51151 steps 123 -> 128 us, 4096 of 1531 45 -> 51, of 201 41 -> 48;
+// forward and backward, 2048 of 22185 956 -> 985, 4 x 2048 of 5001 948 -> 987.  (Through a float32 kernel row and float32 transforms, as
+// these lengths went before, 2181, 204, 66, 1717 and 1184; y and dx 2.6e-6 - 3.4e-6 and 2e-5 - 1.4e-4 at the initial decays, in no channel more
+// than a tenth nearer at slower ones; gradients of the parameters that are sums of terms of one sign, as rows with a mean have, 0.8e-7 - 4.3e-7 there and
+// 1.1e-7 - 5.2e-7 here, the others nowhere nearer.)  The forward of kShifted keeps two registers of ONE in scratch, the others' long walk one.
 struct XOpWide {
   static constexpr int XP = 3;
   u32x4 pc[3];
@@ -362,7 +381,7 @@ __device__ __forceinline__ floatx16 mma_split(const u32x4* a, const u32x4* x, fl
   return acc;
 }
 
-// Operand blocks of the forward kernel (each 64 lanes x 8 values, two pieces):
+// Operand blocks of the forward kernel (each 64 lanes x 8 values, two pieces; Q of WIDE kernels: 64 lanes x 8 floats):
 //   0..3   P, k-step s:            rows m, steps j = 16 s + 8 g + e
 //   4..7   K by offset o = 16 (b - 5): rows r, lag = o + r - 8 g - e (zero where negative)
 //   8..11  Q, (row tile it, k-step s2): rows i = 32 it + r, state columns m = 16 s2 + 8 g + e
@@ -497,6 +516,7 @@ __global__ __launch_bounds__(kThreads, ONE ? 4 : 3) void cema_scan_fwd_kernel(
   constexpr bool FINE = kFine<ROWS>;
   using Smem = typename std::conditional<ONE, typename std::conditional<FINE, FwdSmemOneFine, FwdSmemOne>::type,
                                          typename std::conditional<FINE, FwdSmemFine, FwdSmem>::type>::type;
+  constexpr bool WIDE = FINE && DT == MEGA_F32;  // Q and the states as float32 operands
   using Op = XRow<DT, FINE>;
   constexpr int NC = Smem::NC, CPS = NC / kSubs, XP = Op::XP;
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -608,7 +628,8 @@ __global__ __launch_bounds__(kThreads, ONE ? 4 : 3) void cema_scan_fwd_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const cf w = cmul(rp.gv, v[e + 1]);
-        put_pair(sm.aop + Smem::kQ, n, 4 * quad + e, w.x, -w.y);
+        if constexpr (WIDE) put_pair_f32(sm.aop + Smem::kQ, n, 4 * quad + e, w.x, -w.y);
+        else put_pair(sm.aop + Smem::kQ, n, 4 * quad + e, w.x, -w.y);
       }
       qT = sm.pw[9][sn];
       qS = sm.pw[10][sn];
@@ -786,10 +807,12 @@ __global__ __launch_bounds__(kThreads, ONE ? 4 : 3) void cema_scan_fwd_kernel(
     // ---- the state part of the outputs, Q H[c-1], and the stores ------------------------------
     if (runs) {
       u32x4 Q[4][2];
+      if constexpr (!WIDE)
 #pragma unroll
-      for (int b = 0; b < 4; ++b) load_block(Smem::kQ + b, Q[b]);
+        for (int b = 0; b < 4; ++b) load_block(Smem::kQ + b, Q[b]);
       if (on) {
-        u32x4 hb[2][2];
+        u32x4 hb[WIDE ? 1 : 2][2];
+        float hv[2][8];
         // the state in front of chunk c0 + r: the previous row of the buffer, or, for the
         // wave's first chunk, what the scan left in wave_cin
         const float* hrow = r == 0 ? sm.wave_cin[wave] : sm.H + (c0 + r) * kHP;
@@ -799,14 +822,26 @@ __global__ __launch_bounds__(kThreads, ONE ? 4 : 3) void cema_scan_fwd_kernel(
           const float4 u = *reinterpret_cast<const float4*>(src);
           const float4 u1 = *reinterpret_cast<const float4*>(src + 4);
           const float v[8] = {u.x, u.y, u.z, u.w, u1.x, u1.y, u1.z, u1.w};
-          split8(v, hb[s2][0], hb[s2][1]);
+          if constexpr (WIDE) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) hv[s2][e] = v[e];
+          } else {
+            split8(v, hb[s2][0], hb[s2][1]);
+          }
         }
         const int id = opaque(lane), at = (id & 31) * kT, ag = id >> 5;
 #pragma unroll
         for (int it = 0; it < 2; ++it) {
           floatx16 acc = yacc[it];
 #pragma unroll
-          for (int s2 = 0; s2 < 2; ++s2) acc = mma_split<2, FINE>(Q[2 * it + s2], hb[s2], acc);
+          for (int s2 = 0; s2 < 2; ++s2) {
+            if constexpr (WIDE) {
+              load_block(Smem::kQ + 2 * it + s2, Q[0]);
+              acc = mma_f32(Q[0], hv[s2], acc);
+            } else {
+              acc = mma_split<2, FINE>(Q[2 * it + s2], hb[s2], acc);
+            }
+          }
 #pragma unroll
           for (int pr = 0; pr < 2; ++pr) {
             if constexpr (DT == MEGA_F32) {
@@ -1073,6 +1108,7 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
   constexpr int CPS = kBwdCPS;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   constexpr bool FINE = kFine<ROWS>;
+  constexpr bool WIDE = FINE && DX32 != 0;  // Qd and the states as float32 operands
   using Smem = typename std::conditional<FINE, BwdSmemFine, BwdSmem>::type;
   Smem& sm = *reinterpret_cast<Smem*>(smem_raw);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -1209,6 +1245,14 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
         }
       }
       u32x4 hi, lo, third;
+      if (WIDE && blk >= 12) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          sm.aop[blk][0][ln][e] = __float_as_uint(v[e]);
+          sm.aop[blk][1][ln][e] = __float_as_uint(v[4 + e]);
+        }
+        continue;
+      }
       if (H16 && blk < 8) split8_f16<FINE>(v, hi, lo, third);
       else split8(v, hi, lo);
       if (FINE && !H16) third = split8_third(v, hi, lo);
@@ -1557,14 +1601,20 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
       // staging to retire under before the next loads are issued behind them
       // ---- DX = K^T DY + Qd R[c+1] (omega dy included: K carries omega on its diagonal) -------------
       if (DX32 != 1 || dx != nullptr) {
-        u32x4 hb[2][2];
+        u32x4 hb[WIDE ? 1 : 2][2];
+        float hv[2][8];
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
           const float* src = rnext + 16 * s2 + 8 * g;
           const float4 u0 = *reinterpret_cast<const float4*>(src);
           const float4 u1 = *reinterpret_cast<const float4*>(src + 4);
           const float v[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
-          split8(v, hb[s2][0], hb[s2][1]);
+          if constexpr (WIDE) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) hv[s2][e] = v[e];
+          } else {
+            split8(v, hb[s2][0], hb[s2][1]);
+          }
         }
 #pragma unroll
         for (int jt = 0; jt < 2; ++jt) {
@@ -1584,7 +1634,8 @@ __global__ __launch_bounds__(kThreads, 2) void cema_scan_bwd_kernel(
           for (int s2 = 0; s2 < 2; ++s2) {
             u32x4 a[2];
             load_block(12 + 2 * jt + s2, a, lane);
-            acc = mma_split<2, FINE>(a, hb[s2], acc);
+            if constexpr (WIDE) acc = mma_f32(a, hv[s2], acc);
+            else acc = mma_split<2, FINE>(a, hb[s2], acc);
           }
 #pragma unroll
           for (int pr = 0; pr < 2; ++pr) {

@@ -402,8 +402,7 @@ Optional cema(const Tensor& x, const Tensor& alpha, const Tensor& delta, const T
 std::optional<std::tuple<Tensor, Optional>> cema_state(const Tensor& x, const Tensor& p, const Tensor& log_q, const Tensor& gamma_hat, const Tensor& omega, const Optional& h0, bool last) {
   const int64_t N = p.size(1);
   if (!cema_takes(x, N)) return std::nullopt;
-  // (the state's share of the outputs is a product of two-piece factors, 2^-18: 3.9e-6 of one step's outputs, where these
-  // lengths add it in float32)
+  // (with a carried state these lengths take the convolution)
   if (h0.has_value() && x.scalar_type() == at::kFloat && x.size(2) % 8 != 0) return std::nullopt;
   const int64_t B = x.size(0), D = x.size(1);
   require(p.numel() == D * N && log_q.numel() == D * N && gamma_hat.numel() == D * N && omega.numel() == D, "cema: x and the parameters must have the same number of channels");

@@ -1,10 +1,13 @@
 """The EMA layer on float32 rows whose length no piece of the kernels divides, against the float64 oracle: outputs, gradients,
-last state.  Rows and matrices enter with 24 bits, sums are float32, powers come from float32 coefficients: y, dx and
-the state 5e-7 in the 2-norm at the initial decays (longest chains 6e-7), gradients up to 2e-6 (theta, a sum of cancelling
+last state.  Rows, matrices and the state between chunks enter with 24 bits, sums are float32, powers come from float32
+coefficients: y, dx and the state up to 6e-7 in the 2-norm at the initial decays, gradients up to 2e-6 (theta, a sum of cancelling
 terms).  Bars: three times that."""
+import math
+
 import pytest
 import torch
 
+from megalodon_amd import extension as megalodon_ops
 from megalodon_amd.modules import MultiHeadComplexEMA
 from oracle import cema as ocema, fftconv as offt
 from test_cema_any_length_gpu import NAMES, _picked, _rows
@@ -74,3 +77,53 @@ def test_last_state(B, D, L, carried):
         want = want + ocema.ema_bias_fwd(q.log(), g, h0, L)
     assert _err(out, want) <= (9e-6 if carried else 2e-6)
     assert last.dtype == torch.complex64 and _err(last, ocema.ema_hidden_fwd(x0, p, q.log(), h0)) <= 2e-6
+
+
+def _worst(got, ref):
+    """The largest over channels of a channel's error in the 2-norm."""
+    got, ref = (t.detach().cpu().double().transpose(0, 1).flatten(1) for t in (got, ref))
+    return ((got - ref).norm(dim=1) / ref.norm(dim=1)).max().item()
+
+
+@pytest.mark.parametrize("L", [121, 4097])
+@pytest.mark.parametrize("mean", [0.0, 1.0])
+@pytest.mark.parametrize("slower", [1, 10, 100])
+def test_long_memories(monkeypatch, slower, mean, L):
+    """Decays 1 - |q| ten and a hundred times slower than the initial ones, rows with a mean, the channel that is furthest off.
+    Against 64 bits on the layer's own float32 coefficients: float32 operands and sums leave some 10 * 2^-24 of a channel whose modes
+    do not cancel, up to ten times that where they do (a state of 16 bits: 3e-5).  Against 64 bits throughout: no
+    further off than the convolution, where the coefficients decide for both up to a tenth."""
+    D, N = 64, 16
+    torch.manual_seed(L)
+    layer = MultiHeadComplexEMA(D, N)
+    with torch.no_grad():
+        layer.delta.copy_(torch.logit(torch.sigmoid(layer.delta.double()) / slower))
+    layer = layer.cuda().train()
+    gen = torch.Generator().manual_seed(L + 1)
+    x0, dy = torch.randn(2, D, L, generator=gen) + mean, torch.randn(2, D, L, generator=gen) + mean
+
+    def both():
+        x = x0.cuda().requires_grad_(True)
+        out, _ = layer(x)
+        out.backward(dy.cuda())
+        return out, x.grad
+
+    def oracle(p, log_q, g):
+        xo = x0.double().requires_grad_(True)
+        want = offt.fftconv_fwd(xo, ocema.ema_weight_fwd(p, log_q, g, L)) + xo * layer.omega.detach().cpu().double()
+        want.backward(dy.double())
+        return want, xo.grad
+
+    got = both()
+    monkeypatch.setenv("MEGA_CEMA_FFT", "1")
+    convolved = both()
+    pr = {n: getattr(layer, n).detach() for n in NAMES}
+    p, log_q, g = (t.cpu() for t in megalodon_ops.cema_coeffs_fwd(pr["alpha"], pr["delta"], pr["theta"], pr["gamma"]))
+    for a, b in zip(got, oracle(p.double(), log_q.to(torch.complex128), g.to(torch.complex128))):
+        assert _err(a, b) <= 1e-6 and _worst(a, b) <= 6e-6
+    pr = {n: t.cpu().double() for n, t in pr.items()}
+    a, angle = torch.sigmoid(pr["alpha"]), torch.sigmoid(pr["theta"]) * (2 * math.pi / N) * torch.arange(1, N + 1, dtype=torch.float64).view(1, N, 1)
+    exact = oracle(a, torch.complex(torch.log1p(-a * torch.sigmoid(pr["delta"])), angle.expand_as(a)),
+                   torch.view_as_complex(pr["gamma"].contiguous()) * math.sqrt(1.0 / N))
+    for ours, theirs, b in zip(got, convolved, exact):
+        assert _err(ours, b) <= 1.1 * _err(theirs, b) and _worst(ours, b) <= 1.1 * _worst(theirs, b)
