@@ -7,7 +7,7 @@ import math
 import pytest
 import torch
 
-from megalodon_amd import extension as megalodon_ops
+from megalodon_amd import _lib, extension as megalodon_ops
 from megalodon_amd.modules import MultiHeadComplexEMA
 from oracle import cema as ocema, fftconv as offt
 from test_cema_any_length_gpu import NAMES, _picked, _rows
@@ -127,3 +127,27 @@ def test_long_memories(monkeypatch, slower, mean, L):
                    torch.view_as_complex(pr["gamma"].contiguous()) * math.sqrt(1.0 / N))
     for ours, theirs, b in zip(got, convolved, exact):
         assert _err(ours, b) <= 1.1 * _err(theirs, b) and _worst(ours, b) <= 1.1 * _worst(theirs, b)
+
+
+@pytest.mark.parametrize("B,D,L", [(2, 8, 1), (1, 3, 5), (2, 8, 63), (1, 3, 65), (2, 8, 1531), (1, 3, 8201), (7, 400, 130), (7, 400, 2113)])
+def test_entry_point_takes_a_carried_state(B, D, L):
+    """mega_cema_layer_scan_fwd with a state in front of such rows (the layer itself takes the convolution there): outputs and
+    last state to the bars of rows without one, on the float32 coefficients that the call is given."""
+    N = 16
+    torch.manual_seed(L)
+    layer = MultiHeadComplexEMA(D, N).cuda()
+    x0, x = _rows(B, D, L, torch.float32, L, 0)
+    h0 = torch.randn(B, D, N, dtype=torch.complex64, generator=torch.Generator().manual_seed(2))
+    with torch.no_grad():
+        p, log_q, g = megalodon_ops.cema_coeffs_fwd(layer.alpha, layer.delta, layer.theta, layer.gamma)
+        omega, h = layer.omega.reshape(-1).contiguous(), h0.cuda()
+        out, last = torch.empty_like(x), torch.empty(B, D, N, dtype=torch.complex64, device="cuda")
+        _lib.call("mega_cema_layer_scan_fwd", _lib.ptr(x), _lib.i32(_lib.dtype_code(x.dtype)), _lib.ptr(p), _lib.ptr(log_q), _lib.ptr(g),
+                  _lib.ptr(omega), _lib.ptr(h), _lib.i64(B), _lib.i64(D), _lib.i64(N), _lib.i64(L), _lib.ptr(out), _lib.ptr(last),
+                  _lib.stream_ptr(x.device))
+    pick = slice(0, None, 50 if D > 64 else 1)
+    p, log_q, g, omega = p[pick].cpu().double(), log_q[pick].cpu().to(torch.complex128), g[pick].cpu().to(torch.complex128), omega[pick].cpu().double()
+    x0, h0 = x0[:, pick].double(), h0[:, pick]
+    want = offt.fftconv_fwd(x0, ocema.ema_weight_fwd(p, log_q, g, L)) + x0 * omega.view(-1, 1) + ocema.ema_bias_fwd(log_q, g, h0, L)
+    assert _err(out[:, pick], want) <= 2e-6
+    assert _err(last[:, pick], ocema.ema_hidden_fwd(x0, p.view(-1, N, 1), log_q.view(-1, N, 1), h0)) <= 2e-6
