@@ -246,7 +246,11 @@ __device__ __forceinline__ u32x4 load_weights(const uint16_t* p) {
 }
 
 constexpr int kRowsWaves = 8, kRowsPieces = 4;
-constexpr int kRowsNormK = kRowsWaves * kRowsPieces * 128;  // longest row that is normalised on the way: one round of pieces
+// Longest row that is normalised on the way with `tt` token tiles: one round of pieces.  Only the RMSNorm of one tile goes up to four a
+// wave; the others end at two (see few_rows), and rounds of three and four that nothing reaches took their kernels from 78, 82 and 90 registers
+// to 119, 116 and 128, with ten more in scratch (eight tokens of one sequence of two heads of 1024 features 415 -> 410 us, of four 518 -> 513,
+// of one head +- 0).
+constexpr int norm_row(int norm, int tt) { return kRowsWaves * 128 * (norm == kNormRms && tt == 1 ? kRowsPieces : 2); }
 
 template <int DT, int TT, int G, bool PAIR, int NORM>
 __global__ __launch_bounds__(kRowsWaves * kWave, 4) void rows_kernel(const ProductParams a) {
@@ -414,16 +418,14 @@ __global__ __launch_bounds__(kRowsWaves * kWave, 4) void rows_kernel(const Produ
     if (per - c == 3) round(c, std::integral_constant<int, 3>());
     else if (per - c == 2) round(c, std::integral_constant<int, 2>());
     else if (per - c == 1) round(c, std::integral_constant<int, 1>());
-  } else if (per == 4) {  // (at most kRowsNormK values a row)
-    round(0, std::integral_constant<int, 4>());
-  } else if (per == 3) {
-    round(0, std::integral_constant<int, 3>());
-  } else if (per == 2) {
-    round(0, std::integral_constant<int, 2>());
-  } else if (per == 1) {
-    round(0, std::integral_constant<int, 1>());
-  } else if (sg.norm != kNormNone) {
-    lds_barrier();  // (a row of fewer pieces than waves)
+  } else {  // (at most norm_row values)
+    if constexpr (norm_row(NORM, TT) > 2 * NW * 128) {
+      if (per == 4) round(0, std::integral_constant<int, 4>());
+      else if (per == 3) round(0, std::integral_constant<int, 3>());
+    }
+    if (per == 2) round(0, std::integral_constant<int, 2>());
+    else if (per == 1) round(0, std::integral_constant<int, 1>());
+    else if (per == 0 && sg.norm != kNormNone) lds_barrier();  // (a row of fewer pieces than waves)
   }
 
 #pragma unroll
@@ -900,7 +902,7 @@ void tiles(const ProductParams& p, hipStream_t s) {
 // Their norms come on the way, each workgroup's for itself, while that costs less than a launch: in front of fc1 and fc3 up to 2048
 // features (us, on the way / ahead, four rows of each a workgroup: one sequence of two heads 417 / 417, four 424 / 432; of three 628 / 605, 816 / 807;
 // of four 970 / 928, 1604 / 1586), in front of z, r and h1 but for one sequence of 4096 (928 / 908; two 877 / 883, one of three heads 605 / 610).
-bool few_rows(int B, int D) { return D <= kRowsNormK && B <= (D < 2048 ? 8 : 4); }
+bool few_rows(int B, int D) { return D <= norm_row(kNormRms, 1) && B <= (D < norm_row(kNormRms, 2) ? 8 : 4); }
 template <int DT, int TT, int G, bool PAIR, int NORM>
 void rows(ProductParams p, hipStream_t s) {
   int blocks = 0;
@@ -933,7 +935,7 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
   }
   const uint16_t* none = nullptr;
   const bool few = few_rows(B, D);
-  const bool front = !few || (B == 1 && D >= 4096), behind = !few || D > 2048;  // whether the norms have launches of their own
+  const bool front = !few || (B == 1 && D >= 4096), behind = !few || D > norm_row(kNormLayer, 1);  // whether the norms have launches of their own
   // rows of a workgroup: of z, r, h1 and v, of fc1 and fc3 (a pair), of wh2 and fc2
   const int wide = !few ? 32 : front ? 4 : 16, pair = !few ? 16 : behind ? 4 : 8, narrow = !few ? 16 : B <= 4 ? 4 : 8;
   auto seg = [&](const void* W, const void* W2, const void* bias, const uint16_t* x, uint16_t* out, int64_t stride,
