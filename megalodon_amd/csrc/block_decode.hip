@@ -901,7 +901,9 @@ void tiles(const ProductParams& p, hipStream_t s) {
 // sequences of one head of 1024 features 324 / 363, of two 522 / 506, of four 1259 / 1093; one of four 974 / 1090).
 // Their norms come on the way, each workgroup's for itself, while that costs less than a launch: in front of fc1 and fc3 up to 2048
 // features (us, on the way / ahead, four rows of each a workgroup: one sequence of two heads 417 / 417, four 424 / 432; of three 628 / 605, 816 / 807;
-// of four 970 / 928, 1604 / 1586), in front of z, r and h1 but for one sequence of 4096 (928 / 908; two 877 / 883, one of three heads 605 / 610).
+// of four 970 / 928, 1604 / 1586), in front of z, r and h1 but for one sequence of rows that give a wave a fourth piece (a token of one sequence
+// of 100 keys, us, on the way / ahead: 2304 features 53.7 / 54.9, 2560 60.0 / 59.7, 2816 65.5 / 65.3, 3072 70.0 / 70.8, 3328 82.0 / 80.6, 3584 88.2 / 87.1, 3840
+// 95.6 / 94.5, 4096 105.7 / 102.5; eight of two sequences of 4096 877 / 883).
 bool few_rows(int B, int D) { return D <= norm_row(kNormRms, 1) && B <= (D < norm_row(kNormRms, 2) ? 8 : 4); }
 template <int DT, int TT, int G, bool PAIR, int NORM>
 void rows(ProductParams p, hipStream_t s) {
@@ -935,7 +937,7 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
   }
   const uint16_t* none = nullptr;
   const bool few = few_rows(B, D);
-  const bool front = !few || (B == 1 && D >= 4096), behind = !few || D > norm_row(kNormLayer, 1);  // whether the norms have launches of their own
+  const bool front = !few || (B == 1 && D > 3 * kRowsWaves * 128), behind = !few || D > norm_row(kNormLayer, 1);  // whether the norms have launches of their own
   // rows of a workgroup: of z, r, h1 and v, of fc1 and fc3 (a pair), of wh2 and fc2
   const int wide = !few ? 32 : front ? 4 : 16, pair = !few ? 16 : behind ? 4 : 8, narrow = !few ? 16 : B <= 4 ? 4 : 8;
   auto seg = [&](const void* W, const void* W2, const void* bias, const uint16_t* x, uint16_t* out, int64_t stride,
