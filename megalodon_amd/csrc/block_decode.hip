@@ -839,19 +839,25 @@ __global__ __launch_bounds__(256) void combine_kernel(const CombineParams a) {
 
 // ---- host ----------------------------------------------------------------------
 // Runs of keys: a workgroup for every CU, or for as many as equal shares of the pairs leave, where that is two thirds of them;
-// else two.  At least 16 keys each (a run's partial result is 4 bytes per value column, a key 2), at most what the score
-// buffer holds.  With at least 512 workgroups, most of them resident two to a CU and a few left for the end, the step of
+// else two.  At least 16 keys each (a run's partial result is 4 bytes per value column, a key 2).  Where the score buffer holds fewer, equal
+// shares of as many more runs as that takes (us of a step, cut at the buffer's end with the rest in a run of its own / so: 32 sequences of
+// eight heads of 512 value columns and 4101 keys 557 / 457, 5001 625 / 556, 24 of 4501 530 / 404, 32 of twenty heads of 128 and 4201 549 / 444).
+// The number of CUs is a constant: the workspace is asked for apart from the launch, and both have to come to the same runs whatever
+// device is current then.  With at least 512 workgroups, most of them resident two to a CU and a few left for the end, the step of
 // four heads on 8 tokens took, us before / now: 1 x 1531 keys 986 / 968, 5 x 3900 2350 / 2144, 9 x 3000 2868 / 2577, 13 x 3000 3700 / 3260, 16 x
 // 3000 3903 / 3738, 22 x 3000 (69 % of the CUs) 5692 / 4983, 32 x 3500 7822 / 7434; of eight heads 24 x 1000 (75 %) 8279 / 8083, 20 x
 // 1000 (62 %, so two a CU) 7337 / 7239 where one a CU takes 7457.  With long requests for all 1 x 1531 took 982, with short ones
 // 32 x 3500 7531.
+constexpr int64_t kCus = 256;
 void key_runs(int64_t pairs, int64_t total, int* splits, int* per) {
-  constexpr int64_t kCus = 256;
   int64_t want = kCus / pairs;
   if (3 * want * pairs < 2 * kCus) want = std::max<int64_t>(2 * kCus / pairs, 1);
   int64_t n = (total + want - 1) / want;
   if (n < 16) n = 16;
-  if (n > kMaxKeys) n = kMaxKeys;
+  if (n > kMaxKeys) {
+    const int64_t runs = (total + kMaxKeys - 1) / kMaxKeys;
+    n = (total + runs - 1) / runs;
+  }
   *per = static_cast<int>(n);
   *splits = static_cast<int>((total + n - 1) / n);
 }

@@ -17,7 +17,8 @@ pytestmark = pytest.mark.gpu
     (16, 4, 1195, 64, 64),    # four runs of 299 keys
     (16, 4, 1196, 64, 128),   # four of 300, the last of 297
     (32, 8, 40, 64, 64),      # a run each
-    (32, 8, 4100, 64, 64),    # 4101 keys: more than a run holds, the last run shorter
+    (32, 8, 4100, 64, 64),    # 4101 keys: more than a run holds, two of 2051 and 2050
+    (32, 8, 8192, 64, 64),    # 8193: three of 2731
     (32, 4, 2200, 128, 64),   # two runs of more than 1024
     (20, 8, 301, 64, 64),     # pairs that a workgroup a CU does not fit: three runs of two workgroups a CU
     (5, 4, 176, 256, 256),    # eleven runs of 16 keys and one of the new key alone
