@@ -842,6 +842,10 @@ __global__ __launch_bounds__(256) void combine_kernel(const CombineParams a) {
 // else two.  At least 16 keys each (a run's partial result is 4 bytes per value column, a key 2).  Where the score buffer holds fewer, equal
 // shares of as many more runs as that takes (us of a step, cut at the buffer's end with the rest in a run of its own / so: 32 sequences of
 // eight heads of 512 value columns and 4101 keys 557 / 457, 5001 625 / 556, 24 of 4501 530 / 404, 32 of twenty heads of 128 and 4201 549 / 444).
+// More pairs than CUs take two runs each up to half as many again and one above, of at most 1024 keys; a run each, up to the score buffer,
+// left CUs with one workgroup where others had two (us, so cut / now, value columns of 256: 261 pairs of 700 keys 95 / 89, of 4090 364 / 320, 300 of
+// 2000 221 / 198, of 4090 407 / 339, 341 of 2000 227 / 211, 384 234 / 223, 576 357 / 329; with two runs each 403 of 2000 would take 245 for 238, 480 of
+// 64 columns and 700 keys 69 for 66).
 // The number of CUs is a constant: the workspace is asked for apart from the launch, and both have to come to the same runs whatever
 // device is current then.  With at least 512 workgroups, most of them resident two to a CU and a few left for the end, the step of
 // four heads on 8 tokens took, us before / now: 1 x 1531 keys 986 / 968, 5 x 3900 2350 / 2144, 9 x 3000 2868 / 2577, 13 x 3000 3700 / 3260, 16 x
@@ -850,12 +854,13 @@ __global__ __launch_bounds__(256) void combine_kernel(const CombineParams a) {
 // 32 x 3500 7531.
 constexpr int64_t kCus = 256;
 void key_runs(int64_t pairs, int64_t total, int* splits, int* per) {
-  int64_t want = kCus / pairs;
-  if (3 * want * pairs < 2 * kCus) want = std::max<int64_t>(2 * kCus / pairs, 1);
+  int64_t want = kCus / pairs, most = kMaxKeys;
+  if (pairs > kCus) want = 2 * pairs <= 3 * kCus ? 2 : 1, most = kMaxKeys / 4;
+  else if (3 * want * pairs < 2 * kCus) want = 2 * kCus / pairs;
   int64_t n = (total + want - 1) / want;
   if (n < 16) n = 16;
-  if (n > kMaxKeys) {
-    const int64_t runs = (total + kMaxKeys - 1) / kMaxKeys;
+  if (n > most) {
+    const int64_t runs = (total + most - 1) / most;
     n = (total + runs - 1) / runs;
   }
   *per = static_cast<int>(n);

@@ -20,6 +20,9 @@ pytestmark = pytest.mark.gpu
     (32, 8, 4100, 64, 64),    # 4101 keys: more than a run holds, two of 2051 and 2050
     (32, 8, 8192, 64, 64),    # 8193: three of 2731
     (32, 4, 2200, 128, 64),   # two runs of more than 1024
+    (29, 9, 2100, 64, 64),    # more pairs than CUs: three runs of 701, 701 and 699
+    (32, 12, 40, 64, 64),     # two runs, of 21 and 20
+    (31, 13, 1024, 64, 64),   # one run each, were it not for the last key: 513 and 512
     (20, 8, 301, 64, 64),     # pairs that a workgroup a CU does not fit: three runs of two workgroups a CU
     (5, 4, 176, 256, 256),    # eleven runs of 16 keys and one of the new key alone
     (32, 2, 1, 64, 2048),     # two keys
