@@ -908,14 +908,16 @@ void tiles(const ProductParams& p, hipStream_t s) {
   else tiles_as<DT, MT, RT, PAIR, 2>(p, blocks, s);
 }
 
-// Whether the products are rows_kernel's: up to four tokens, and up to eight in narrow blocks (us, rows_kernel / tiles_kernel: eight
-// sequences of one head of 1024 features 324 / 363, of two 522 / 506, of four 1259 / 1093; one of four 974 / 1090).
+// Whether the products are rows_kernel's: up to four tokens, up to eight in narrow blocks (us, rows_kernel / tiles_kernel: eight
+// sequences of one head of 1024 features 324 / 363, of two 522 / 506, of four 1259 / 1093; one of four 974 / 1090), and up to sixteen where
+// the step is its launches, two fewer so (a token of nine / sixteen sequences: 128 features 33.3 / 33.5 and 36.5 / 37.7, 256 33.7 / 34.0 and 37.6 / 39.0,
+// 384 34.6 / 34.7 and 38.4 / 39.2; at 480 40.1 / 40.2 and 39.0 / 38.5.  From 17 on those two launches cost 64 features 3 to 4 us of 34).
 // Their norms come on the way, each workgroup's for itself, while that costs less than a launch: in front of fc1 and fc3 up to 2048
 // features (us, on the way / ahead, four rows of each a workgroup: one sequence of two heads 417 / 417, four 424 / 432; of three 628 / 605, 816 / 807;
 // of four 970 / 928, 1604 / 1586), in front of z, r and h1 but for one sequence of rows that give a wave a fourth piece (a token of one sequence
 // of 100 keys, us, on the way / ahead: 2304 features 53.7 / 54.9, 2560 60.0 / 59.7, 2816 65.5 / 65.3, 3072 70.0 / 70.8, 3328 82.0 / 80.6, 3584 88.2 / 87.1, 3840
 // 95.6 / 94.5, 4096 105.7 / 102.5; eight of two sequences of 4096 877 / 883).
-bool few_rows(int B, int D) { return D <= norm_row(kNormRms, 1) && B <= (D < norm_row(kNormRms, 2) ? 8 : 4); }
+bool few_rows(int B, int D) { return D <= norm_row(kNormRms, 1) && B <= (D <= 384 ? 16 : D < norm_row(kNormRms, 2) ? 8 : 4); }
 template <int DT, int TT, int G, bool PAIR, int NORM>
 void rows(ProductParams p, hipStream_t s) {
   int blocks = 0;
@@ -950,7 +952,7 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
   const bool few = few_rows(B, D);
   const bool front = !few || (B == 1 && D > 3 * kRowsWaves * 128), behind = !few || D > norm_row(kNormLayer, 1);  // whether the norms have launches of their own
   // rows of a workgroup: of z, r, h1 and v, of fc1 and fc3 (a pair), of wh2 and fc2
-  const int wide = !few ? 32 : front ? 4 : 16, pair = !few ? 16 : behind ? 4 : 8, narrow = !few ? 16 : B <= 4 ? 4 : 8;
+  const int wide = !few ? 32 : front ? 4 : 16, pair = !few ? 16 : behind ? 4 : 8, narrow = !few ? 16 : B <= 4 || B > 8 ? 4 : 8;
   auto seg = [&](const void* W, const void* W2, const void* bias, const uint16_t* x, uint16_t* out, int64_t stride,
                  int rows, int strip, int norm, int act) {
     return Segment{u16(W), u16(W2), u16(bias), x, out, stride, rows / strip, norm, act};
@@ -972,7 +974,8 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
     if (!few) tiles<DT, MT, 2, false>(p, s);
     else if (front) rows<DT, 1, 1, false, kNormNone>(p, s);
     else if (B <= 4) rows<DT, 1, 4, false, kNormRms>(p, s);
-    else rows<DT, 2, 4, false, kNormRms>(p, s);
+    else if (B <= 8) rows<DT, 2, 4, false, kNormRms>(p, s);
+    else rows<DT, 4, 4, false, kNormRms>(p, s);
   }
   const int zh = S / H, H2 = E / H;
   int splits, per;
@@ -998,7 +1001,8 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
     p.add1 = at16(l.h1), p.add2 = u16(a.x);
     if (!few) tiles<DT, MT, 1, false>(p, s);
     else if (B <= 4) rows<DT, 1, 1, false, kNormNone>(p, s);
-    else rows<DT, 2, 2, false, kNormNone>(p, s);
+    else if (B <= 8) rows<DT, 2, 2, false, kNormNone>(p, s);
+    else rows<DT, 4, 1, false, kNormNone>(p, s);
   }
   {
     if (behind)
@@ -1011,7 +1015,8 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
     if (!few) tiles<DT, MT, 2, true>(p, s);
     else if (behind) rows<DT, 1, 2, true, kNormNone>(p, s);
     else if (B <= 4) rows<DT, 1, 4, true, kNormLayer>(p, s);
-    else rows<DT, 2, 4, true, kNormLayer>(p, s);
+    else if (B <= 8) rows<DT, 2, 4, true, kNormLayer>(p, s);
+    else rows<DT, 4, 4, true, kNormLayer>(p, s);
   }
   {
     ProductParams p{};
@@ -1020,7 +1025,8 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
     p.add1 = u16(a.x);
     if (!few) tiles<DT, MT, 1, false>(p, s);
     else if (B <= 4) rows<DT, 1, 1, false, kNormNone>(p, s);
-    else rows<DT, 2, 2, false, kNormNone>(p, s);
+    else if (B <= 8) rows<DT, 2, 2, false, kNormNone>(p, s);
+    else rows<DT, 4, 1, false, kNormNone>(p, s);
   }
   MEGA_CHECK_LAUNCH();
   return MEGA_OK;

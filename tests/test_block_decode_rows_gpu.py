@@ -20,6 +20,9 @@ pytestmark = pytest.mark.gpu
     (2, 4128, 64, 128, 64, 1, 3, torch.bfloat16),       # one that is not
     (9, 1024, 256, 512, 416, 2, 8, torch.float16),      # more tokens than two tiles
     (1, 8192, 64, 64, 64, 1, 8, torch.bfloat16),
+    (9, 32, 64, 64, 32, 1, 1, torch.bfloat16),          # four token tiles, the third of one token; one piece of 32 values
+    (16, 384, 128, 1024, 1056, 2, 12, torch.float16),   # all full, the widest rows
+    (13, 352, 64, 256, 160, 1, 11, torch.bfloat16),     # three pieces, the last of 96
 ])
 def test_step_against_float64(B, D, S, E, F, heads, groups, dtype):
     n, chunk = 20, 64

@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("B,D,S,E,F,heads,groups,dtype", [
     (5, 2048, 256, 512, 416, 1, 8, torch.bfloat16),     # the fewest tokens
     (8, 2048, 256, 8192, 4128, 4, 8, torch.float16),    # two waves a workgroup, else four; the last piece of F 32 values
-    (9, 32, 64, 64, 32, 1, 1, torch.bfloat16),          # one piece of 32 values
+    (17, 32, 64, 64, 32, 1, 1, torch.bfloat16),         # one piece of 32 values
+    (9, 416, 64, 64, 32, 1, 13, torch.bfloat16),        # the first width of nine tokens
     (16, 1024, 256, 512, 2784, 2, 8, torch.float16),    # a full tile; F cut at 96
     (17, 352, 128, 1024, 160, 2, 11, torch.bfloat16),   # a second tile of one token, three pieces of D, the last of 96
     (32, 1088, 128, 4096, 4192, 2, 2, torch.bfloat16),  # two full tiles, D cut at half a piece
