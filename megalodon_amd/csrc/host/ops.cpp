@@ -385,13 +385,33 @@ struct CemaFn : Function<CemaFn> {
 bool cema_takes(const Tensor& x, int64_t N) {
   return x.is_cuda() && x.dim() == 3 && N >= 1 && N <= 16 && code_of(x.scalar_type()) >= 0 && x.size(2) >= 1 && x.size(0) * x.size(1) <= 0x7fffffff;
 }
+// float32 rows whose length is no multiple of 8: whether the recurrence is ahead of the convolution (kernel row, float32 transforms).
+// A row of one chunk costs the recurrence a tile like one of 24 of them, and the backward six launches, each of which sets
+// up its channels; the transforms' cost follows the power of two above 2 L.  us, recurrence / convolution: forward 64 x 1024 rows of 9
+// steps 220 / 46, 16 x 4096 of 193 225 / 151, of 385 228 / 309; 4 x 2048 of 9 35 / 47.  Forward and backward 64 x 1024 of 9 1669 / 152, of 513
+// 1912 / 1588, of 1021 2145 / 3276; 16 x 1024 of 65 520 / 255, of 700 611 / 593, of 850 628 / 829; 2048 of 1100 357 / 271, 2 x 1024 220 / 253; 4 x 2048
+// of 3001 741 / 674, of 5001 987 / 1184, of 8191 1503 / 1415, 1024 x 16383 485 / 490, x 20001 523 / 900.  Few rows take the host longer than the
+// device, four launches and Python where the recurrence is one call: 4 x 64 rows of 65 108 / 150 - 260.  Batches of narrow layers
+// add the convolution's weight gradient up slowly: 256 x 64 of 129 steps 544 / 675, 64 x 16 of 257 178 / 347.
+bool recurrence_ahead(int64_t B, int64_t D, int64_t L, bool train) {
+  const int64_t rows = B * D;
+  if (!train) return L > 288 || B <= 4 || rows <= 6144;
+  if (L <= 512) return (B <= 8 && D <= 512 && rows <= 2048) || (B >= 16 && D <= 128 && L > 128);
+  if (L <= 1024) return (D <= 512 && (B >= 8 || rows <= 2048)) || (B >= 4 && L > 736);
+  if (L <= 2048) return B >= 2 || D <= 512 || L > 1400;
+  if (L <= 4096) return (B <= 8 && D <= 512 && rows <= 1024) || (B >= 4 && L <= 2304);
+  if (L <= 6144) return B >= 2 || D <= 512;
+  return L > 8192 || rows <= 512;
+}
 Optional cema(const Tensor& x, const Tensor& alpha, const Tensor& delta, const Tensor& theta, const Tensor& gamma, const Tensor& omega) {
   if (alpha.dim() != 3 || !cema_takes(x, alpha.size(1))) return std::nullopt;
   const int64_t D = x.size(1), N = alpha.size(1);
   const auto is = [&](const Tensor& t, int64_t n) { return t.scalar_type() == alpha.scalar_type() && t.device() == x.device() && t.numel() == n && t.is_contiguous(); };
   if (code_of(alpha.scalar_type()) < 0 || !is(alpha, D * N) || !is(delta, D * N) || !is(theta, D) || !is(gamma, 2 * D * N) || !is(omega, D)) return std::nullopt;
+  const bool train = wants_grad({&x, &alpha, &delta, &theta, &gamma, &omega});
+  if (x.scalar_type() == at::kFloat && x.size(2) % 8 != 0 && !recurrence_ahead(x.size(0), D, x.size(2), train)) return std::nullopt;
   c10::DeviceGuard guard(x.device());
-  if (wants_grad({&x, &alpha, &delta, &theta, &gamma, &omega})) return CemaFn::apply(x, alpha, delta, theta, gamma, omega);
+  if (train) return CemaFn::apply(x, alpha, delta, theta, gamma, omega);
   const Tensor xc = rows_of(x), ws = floats({5 * D * N}, x);
   Tensor y = at::empty_like(xc);
   if (y.numel() == 0) return y;

@@ -6,7 +6,8 @@ instead of being broadcast (:21-26).  On the GPU the layer runs as a chunked
 recurrence (csrc/host/ops.cpp, fused_ops/cema_scan.py) wherever its kernels take
 the case -- at most 32 modes, with or without gradients, carried state and last
 state, at lengths that are a multiple of 8; rows of any length with at most
-16 modes and either gradients or a state (float32 ones: but for a carried state); MEGA_CEMA_FFT=1 in the environment keeps everything on the
+16 modes and either gradients or a state (float32 ones: but for a carried state,
+and without one or the last state where the recurrence is ahead); MEGA_CEMA_FFT=1 in the environment keeps everything on the
 kernel-row + FFT-convolution operators that the remaining cases use."""
 from typing import Optional, Tuple
 import math

@@ -151,3 +151,29 @@ def test_entry_point_takes_a_carried_state(B, D, L):
     want = offt.fftconv_fwd(x0, ocema.ema_weight_fwd(p, log_q, g, L)) + x0 * omega.view(-1, 1) + ocema.ema_bias_fwd(log_q, g, h0, L)
     assert _err(out[:, pick], want) <= 2e-6
     assert _err(last[:, pick], ocema.ema_hidden_fwd(x0, p.view(-1, N, 1), log_q.view(-1, N, 1), h0)) <= 2e-6
+
+
+@pytest.mark.parametrize("B,D,L,forward,backward", [
+    (8, 256, 9, True, True), (9, 256, 9, True, False), (1, 520, 9, True, False), (16, 64, 129, True, True), (16, 64, 127, True, False),
+    (64, 104, 9, False, False), (64, 96, 9, True, False), (4, 1664, 289, True, False), (5, 1232, 287, False, False),
+    (4, 520, 737, True, True), (4, 520, 735, True, False), (1, 520, 1025, True, False), (1, 520, 1401, True, True),
+    (4, 264, 2303, True, True), (3, 512, 2051, True, False), (1, 513, 5001, True, False), (1, 520, 8191, True, False), (1, 520, 8193, True, True),
+])
+def test_shorter_way(monkeypatch, B, D, L, forward, backward):
+    """Rows for which the convolution is ahead of the recurrence (many short ones: up to seventeen times) take it, bit for bit;
+    the others do not."""
+    torch.manual_seed(L)
+    layer = MultiHeadComplexEMA(D, 16).cuda().train()
+    x = _rows(B, D, L, torch.float32, L, 0)[1]
+
+    def both():
+        with torch.no_grad():
+            y = layer(x)[0]
+        xg = x.detach().requires_grad_(True)
+        return y, torch.autograd.grad(layer(xg)[0].square().sum(), xg)[0]
+
+    got = both()
+    monkeypatch.setenv("MEGA_CEMA_FFT", "1")
+    convolved = both()
+    assert [torch.equal(a, b) for a, b in zip(got, convolved)] == [not forward, not backward]
+    assert all(_err(a, b.double().cpu()) <= 1e-5 for a, b in zip(got, convolved))
