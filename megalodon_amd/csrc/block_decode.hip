@@ -846,6 +846,10 @@ __global__ __launch_bounds__(256) void combine_kernel(const CombineParams a) {
 // left CUs with one workgroup where others had two (us, so cut / now, value columns of 256: 261 pairs of 700 keys 95 / 89, of 4090 364 / 320, 300 of
 // 2000 221 / 198, of 4090 407 / 339, 341 of 2000 227 / 211, 384 234 / 223, 576 357 / 329; with two runs each 403 of 2000 would take 245 for 238, 480 of
 // 64 columns and 700 keys 69 for 66).
+// So do more than two thirds of the CUs' number where the keys are more than a fifth of what is read: while a lone workgroup is at its keys or
+// between the two, nothing of its CU's is on the way (us, one run / so, key by value columns: 172 pairs of 256 x 64 and 4000 keys 226 / 193, of 1000
+// 79 / 70, of 64 x 128 and 4000 132 / 120, 180 of 64 x 64 and 4000 107 / 101, 228 of 128 x 256 and 300 56.1 / 53.5, 256 of 64 x 64 and 2000 78.7 / 80.1; of 64 x
+// 512 and 1000, where it does not hold, 180 115 / 119, of 256 x 1024 225 / 233).
 // The number of CUs is a constant: the workspace is asked for apart from the launch, and both have to come to the same runs whatever
 // device is current then.  With at least 512 workgroups, most of them resident two to a CU and a few left for the end, the step of
 // four heads on 8 tokens took, us before / now: 1 x 1531 keys 986 / 968, 5 x 3900 2350 / 2144, 9 x 3000 2868 / 2577, 13 x 3000 3700 / 3260, 16 x
@@ -853,9 +857,9 @@ __global__ __launch_bounds__(256) void combine_kernel(const CombineParams a) {
 // 1000 (62 %, so two a CU) 7337 / 7239 where one a CU takes 7457.  With long requests for all 1 x 1531 took 982, with short ones
 // 32 x 3500 7531.
 constexpr int64_t kCus = 256;
-void key_runs(int64_t pairs, int64_t total, int* splits, int* per) {
+void key_runs(int64_t pairs, int64_t total, int64_t zh, int64_t H2, int* splits, int* per) {
   int64_t want = kCus / pairs, most = kMaxKeys;
-  if (pairs > kCus) want = 2 * pairs <= 3 * kCus ? 2 : 1, most = kMaxKeys / 4;
+  if (pairs > kCus || (3 * pairs > 2 * kCus && H2 < 4 * zh)) want = 2 * pairs <= 3 * kCus ? 2 : 1, most = kMaxKeys / 4;
   else if (3 * want * pairs < 2 * kCus) want = 2 * kCus / pairs;
   int64_t n = (total + want - 1) / want;
   if (n < 16) n = 16;
@@ -872,7 +876,7 @@ struct Layout {
 };
 Layout layout_of(const mega_block_decode_args& a) {
   int splits, per;
-  key_runs(a.B * a.heads, a.length + 1, &splits, &per);
+  key_runs(a.B * a.heads, a.length + 1, a.S / a.heads, a.E / a.heads, &splits, &per);
   int64_t at = 0;
   auto take = [&](int64_t bytes) {
     const int64_t here = at;
@@ -979,7 +983,7 @@ int run(const mega_block_decode_args& a, hipStream_t s) {
   }
   const int zh = S / H, H2 = E / H;
   int splits, per;
-  key_runs(static_cast<int64_t>(B) * H, a.length + 1, &splits, &per);
+  key_runs(static_cast<int64_t>(B) * H, a.length + 1, zh, H2, &splits, &per);
   {
     AttendParams p{at16(l.z), u16(a.qk_gamma), u16(a.qk_beta), a.freqs, u16(a.k_in), u16(a.v_in),
                    static_cast<uint16_t*>(a.k_out), static_cast<uint16_t*>(a.v_out), reinterpret_cast<float*>(ws + l.part),

@@ -16,9 +16,14 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("B,heads,n,zh,H2", [
     (16, 4, 1195, 64, 64),    # four runs of 299 keys
     (16, 4, 1196, 64, 128),   # four of 300, the last of 297
-    (32, 8, 40, 64, 64),      # a run each
-    (32, 8, 4100, 64, 64),    # 4101 keys: more than a run holds, two of 2051 and 2050
-    (32, 8, 8192, 64, 64),    # 8193: three of 2731
+    (32, 8, 40, 64, 64),      # two runs, of 21 and 20
+    (32, 8, 40, 64, 256),     # a run each
+    (32, 8, 4100, 64, 64),    # five runs of at most 1024 keys
+    (32, 8, 8192, 64, 64),    # nine
+    (16, 16, 4100, 64, 256),  # 4101 keys: more than a run holds, two of 2051 and 2050
+    (19, 9, 1030, 64, 64),    # the fewest pairs of two runs each for their narrow values
+    (17, 10, 1030, 64, 64),   # one pair fewer: three runs of two workgroups a CU
+    (19, 9, 1030, 64, 256),   # wide values: one run
     (32, 4, 2200, 128, 64),   # two runs of more than 1024
     (29, 9, 2100, 64, 64),    # more pairs than CUs: three runs of 701, 701 and 699
     (32, 12, 40, 64, 64),     # two runs, of 21 and 20
