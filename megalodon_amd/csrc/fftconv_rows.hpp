@@ -124,7 +124,7 @@ using namespace fftc;
 
 // Workgroups of a transform size that share a compute unit: the kernel's time is the latency of its
 // exchanges and barriers, so two waves per SIMD at every size, which is what the registers (32 complex
-// points per lane and operand: 229-256 of 256, with rows one by one none spilled) and the planes in LDS allow.  With one wave
+// points per lane and operand: 229-256 of 256) and the planes in LDS allow.  With one wave
 // per SIMD below M = 16384 (and 330 registers) and the loads in branches, forward / backward in
 // bfloat16 took 2 x 1024 rows of 3000: 152 / 348 us, now 51 / 138; of 8192: 226 / 479, now 95 / 198;
 // 1024 rows of 16384: 236 / 485, now 115 / 219; of 32768: 440 / 891, now 246 / 502 (the last by the loads alone).
@@ -429,9 +429,19 @@ __device__ __forceinline__ void fetch(const float* part, float* re, float* im, i
   }
 }
 
+// Has the lane's values worked out here.  Where branches follow (the product of spectra with its lane of self-paired residues, the
+// stores at a row's end) the last butterflies are otherwise sunk into them, and both their operands stay in registers until then: pairs
+// of rows spilled 15 to 49 beside k's spectrum (80 bytes a lane: 40 MiB that the runtime took at a first launch).  Forward, us, before / now: bfloat16
+// 3 x 1024 rows of 4095 86 / 73, 4 x 1024 of 5001 166 / 145, 2 x 1024 of 8192 89 / 84, of 10001 190 / 169, of 12000 173 / 163, 2 x 512 of 16384 97 / 92;
+// float32 86 / 72, 163 / 138, 94 / 81, 192 / 169, 179 / 175, 101 / 97.
+__device__ __forceinline__ void settle(float* re, float* im) {
+#pragma unroll
+  for (int j = 0; j < 32; ++j) asm volatile("" : "+v"(re[j]), "+v"(im[j]));
+}
+
 // Back from a product of spectra.  Half 0 leaves its M outputs zy[t + T j] in `part`; half 1 adds them and has the
-// sum in (re, im), zy[t + T j] at register j.
-template <int LOGM, int H>
+// sum in (re, im), zy[t + T j] at register j.  FULL: the registers hold k's spectrum too.
+template <int LOGM, int H, bool FULL>
 __device__ __forceinline__ void outputs(float* re, float* im, int t, const Tables& tb, float* lre, float* lim, float* part) {
   inverse_half<LOGM, H>(re, im, t, tb, lre, lim);
   float ore[32], oim[32];
@@ -440,6 +450,7 @@ __device__ __forceinline__ void outputs(float* re, float* im, int t, const Table
     ore[j] = re[out_pos<H>(j)];
     oim[j] = im[out_pos<H>(j)];
   }
+  if (H == 1 && FULL) settle(ore, oim);
   if (H == 0) keep<LOGM>(part, ore, oim, t);
   else fetch<LOGM, true>(part, ore, oim, t);
 #pragma unroll
@@ -452,8 +463,8 @@ __device__ __forceinline__ void outputs(float* re, float* im, int t, const Table
 // The rows of a channel that a workgroup takes: two at a time, which then share the transform of k (MODE 0) or the
 // inverse transform of dk, whose spectrum is summed over them (MODE 1).  The kernels' time is mostly the transforms'
 // arithmetic (72 to 75 % of the vector issue slots at M = 4096), so what counts is their number: 2.5 per row instead of 3.  In MODE 0
-// k's spectrum then has to stay in registers to the row's end: 15 to 49 of them spill (written once, read once a row), at
-// M = 16384 72, where the rows go one by one (PAIR 1), as a channel's only row does (odd lengths: see launch_fft_v).  One kernel for dx and dk, with dy's spectrum formed once (4
+// k's spectrum then has to stay in registers to the row's end, which none of them leaves (one, of odd rows at M = 8192) since `settle`; at M = 16384 67
+// to 76 would, and the rows go one by one (PAIR 1), as a channel's only row does (odd lengths: see launch_fft_v).  One kernel for dx and dk, with dy's spectrum formed once (4
 // transforms per row), spills 54 to 139 registers and takes 269 us where these two take 168.
 // bfloat16, forward / backward in us: 2 x 1024 rows of 8192 97 / 194 -> 86 / 168, 4 x 1024 of 8190 181 / 385 -> 158 / 325; of
 // channels whose rows now share out the chip for dk too: 8 x 256 of 8192 89 / 377 -> 82 / 169, 8 x 512 of 3001 120 / 541 -> 119 / 271
@@ -490,6 +501,7 @@ __device__ __forceinline__ void conv_half(const void* a, const void* b, void* ou
   const int64_t pitch = static_cast<int64_t>(rows.L) * (DT == MEGA_F32 ? 4 : 2);
   float pre[32], pim[32];
   const int count = PAIR == 1 ? 1 : n;
+  constexpr bool FULL = MODE == 0 && PAIR > 1;
   if (MODE == 0) {
     const int t = own_lane(threadIdx.x) & (C::T - 1);  // (restores the range so that offsets stay 32-bit)
     spectrum<LOGM, MEGA_F32, VEC, H, true>(pre, pim, static_cast<const float*>(b) + static_cast<int64_t>(d) * rows.L, rows.L, false, t, tb, lre, lim);
@@ -502,6 +514,7 @@ __device__ __forceinline__ void conv_half(const void* a, const void* b, void* ou
     float re[32], im[32];
     if (MODE == 1) spectrum<LOGM, DT, VEC, H, true>(pre, pim, static_cast<const char*>(b) + row * pitch, rows.L, false, t, tb, lre, lim);
     spectrum<LOGM, DT, VEC, H, false>(re, im, arow, rows.L, MODE == 1 || flip != 0, t, tb, lre, lim);
+    if (H == 0 && FULL) settle(re, im);
     pointwise<LOGM, H>(re, im, pre, pim, t, launder(tb));
     // the slot's parts: half 0's outputs; with pairs those of the second row, or (MODE 1) the spectrum so far; last a
     // shared channel's sum
@@ -512,7 +525,7 @@ __device__ __forceinline__ void conv_half(const void* a, const void* b, void* ou
         continue;
       }
     }
-    outputs<LOGM, H>(re, im, t, tb, lre, lim, MODE == 0 && PAIR > 1 && i > 0 ? scratch.part[1] : scratch.part[0]);
+    outputs<LOGM, H, FULL>(re, im, t, tb, lre, lim, MODE == 0 && PAIR > 1 && i > 0 ? scratch.part[1] : scratch.part[0]);
     if (H == 1 && MODE == 0)
       store_row<LOGM, DT, VEC, false>(re, im, static_cast<char*>(out) + row * pitch, rows.L, flip != 0, t,
                                       omega != nullptr ? arow : nullptr, omega != nullptr ? omega[d] : 0.f);
