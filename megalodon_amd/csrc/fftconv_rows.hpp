@@ -464,7 +464,7 @@ __device__ __forceinline__ void outputs(float* re, float* im, int t, const Table
 // inverse transform of dk, whose spectrum is summed over them (MODE 1).  The kernels' time is mostly the transforms'
 // arithmetic (72 to 75 % of the vector issue slots at M = 4096), so what counts is their number: 2.5 per row instead of 3.  In MODE 0
 // k's spectrum then has to stay in registers to the row's end, which none of them leaves (one, of odd rows at M = 8192) since `settle`; at M = 16384 67
-// to 76 would, and the rows go one by one (PAIR 1), as a channel's only row does (odd lengths: see launch_fft_v).  One kernel for dx and dk, with dy's spectrum formed once (4
+// to 76 would, and the rows go one by one (PAIR 1), as a channel's only row does.  One kernel for dx and dk, with dy's spectrum formed once (4
 // transforms per row), spills 54 to 139 registers and takes 269 us where these two take 168.
 // bfloat16, forward / backward in us: 2 x 1024 rows of 8192 97 / 194 -> 86 / 168, 4 x 1024 of 8190 181 / 385 -> 158 / 325; of
 // channels whose rows now share out the chip for dk too: 8 x 256 of 8192 89 / 377 -> 82 / 169, 8 x 512 of 3001 120 / 541 -> 119 / 271
@@ -591,12 +591,8 @@ int launch_fft_v(const void* a, const void* b, void* out, int64_t B, int64_t D, 
   if (rc != MEGA_OK) return rc;
   MEGA_CHECK_ARG(B * D <= 0x7fffffff, "fftconv: too many rows");
   constexpr int kMost = MODE == 0 && LOGM == 14 ? 1 : 2;
-  // Odd rows of an odd batch at M = 4096, where the pair spills most beside what it saves, go one by one (bfloat16, pairs /
-  // so: 3 x 1024 rows of 4097 131 / 123 us, 5 x 512 of 5001 122 / 109, 3 x 1024 of 8191 141 / 128; but 4 x 1024 of 5001 161 / 165, and of other
-  // sizes 3 x 1024 of 3001 76 / 80, 5 x 512 of 10001 237 / 243).
-  const int most = MODE == 0 && !VEC && LOGM == 12 && B % 2 ? 1 : kMost;
-  int64_t nb = group_rows(B, D, slots, most, MODE == 1);
-  int pair = nb == 1 ? 1 : most;
+  int64_t nb = group_rows(B, D, slots, kMost, MODE == 1);
+  int pair = nb == 1 ? 1 : kMost;
   const auto parts = [&] { return pair + (MODE == 1 && nb < B ? 1 : 0); };
   rc = get_scratch<LOGM>(stream, parts(), &scratch, &have);
   if (rc != MEGA_OK) return rc;

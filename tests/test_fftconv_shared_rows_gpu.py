@@ -18,7 +18,7 @@ def _conv(a, b):
     (1, 3, 2049, torch.float32), (2, 5, 4096, torch.float32), (3, 1100, 2050, torch.bfloat16),
     (7, 130, 4097, torch.float32), (5, 400, 6000, torch.float16), (9, 256, 8192, torch.bfloat16),
     (4, 1030, 5001, torch.bfloat16), (6, 100, 16384, torch.float32), (3, 300, 9999, torch.bfloat16),
-    (5, 64, 32768, torch.float32), (2, 257, 20001, torch.bfloat16),
+    (5, 64, 32768, torch.float32), (2, 257, 20001, torch.bfloat16), (3, 700, 5001, torch.float16), (5, 420, 8191, torch.float32),
 ])
 def test_against_64_bits(B, D, L, dtype):
     g = torch.Generator("cuda").manual_seed(B * D + L)
