@@ -5,17 +5,18 @@
 // The step is bound by reading the block's weights once and moving the cached keys and
 // values once: at width 4096 the weights are 514 MB, and operator by operator a
 // step was 59 launches, 0.84 ms for one sequence and 4.1 ms for sixteen (1531 and
-// 3000 cached tokens).  Here it is seven launches, nine above eight sequences, 0.123 and 0.49 ms, cut where a whole row is
-// needed by everybody:
+// 3000 cached tokens).  Here it is seven launches, and one for each norm that does not come on the products' way: two there, 0.114 and
+// 0.43 ms.  They are cut where a whole row is needed by everybody:
 //   1. step_kernel    TimestepNorm step, EMA state step
-//   2. products       RMSNorm folded into z, r, h1; v = silu(...) straight into the new cache
+//   2. products       z, r, h1 of the RMSNorm; v = silu(...) straight into the new cache
 //   3. attend_kernel  q, k (norm, affine maps, rotary), one softmax part per split; the old keys and values
 //                     pass into the new cache as they are read, the new key joins them
 //   4. combine_kernel the parts put together, gate silu(r)
 //   5. products       wh2 + h1 + residual
-//   6. products       LayerNorm folded into fc1, fc3; silu(a) b
+//   6. products       fc1, fc3 of the LayerNorm; silu(a) b
 //   7. products       fc2 + residual
-// The products are rows_kernel's for few sequences, which normalises on the way, else rows_norm_kernel's and tiles_kernel's.
+// The products are rows_kernel's for few sequences, else tiles_kernel's (few_rows).  rows_kernel can normalise on the way, which it does
+// for the RMSNorm but with one sequence of more than 3072 features, for the LayerNorm up to 2048; rows_norm_kernel has the others'.
 #include <algorithm>
 #include <type_traits>
 
@@ -210,8 +211,8 @@ __global__ __launch_bounds__(kNormThreads) void rows_norm_kernel(const uint16_t*
 // hardware hands out as others end.  Reading alone, 176 MB in four rows a workgroup take 26.5 us (6.6 TB/s; without the hint
 // 28.5), in sixteen rows by 64 bytes 33, and by one workgroup per compute unit with an equal share each 52.  With that and x
 // through the caches the products of one row take 14.5 us for 67 / 90 MB (in sixteen rows by 64 bytes 18.7).  A norm on the way costs vector
-// work per workgroup, so those take 16 rows: 32.3 and 36.5 us for 176 / 180 MB (in 8 rows 36.4 and 40.5, in sixteen by 64 bytes
-// 41.5 and 45).  Their weights come in two pieces at a time, one with two token tiles: all four would leave one workgroup per unit
+// work per workgroup, so those take 16 rows (while both came so at width 4096, 176 / 180 MB: 32.3 and 36.5 us; in 8 rows 36.4 and 40.5, in sixteen
+// by 64 bytes 41.5 and 45).  Their weights come in two pieces at a time, one with more than one token tile: all four would leave one workgroup per unit
 // (41.6 us) or spill (84).
 template <int DT>
 __device__ __forceinline__ floatx4 mma4(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1, floatx4 c) {

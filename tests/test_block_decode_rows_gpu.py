@@ -1,4 +1,4 @@
-"""The weight products of the one-token step (csrc/block_decode.hip: rows_kernel, skinny_kernel behind rows_norm_kernel) where
+"""The weight products of the one-token step (csrc/block_decode.hip: rows_kernel, tiles_kernel behind rows_norm_kernel) where
 they can go wrong: one and two token tiles full and not, reductions of fewer pieces of 128 than waves, pieces cut by a row's
 end, rows longer than are normalised on the way.  Against the step in 64 bits; bars as in test_block_decode_gpu."""
 import pytest
@@ -16,9 +16,9 @@ pytestmark = pytest.mark.gpu
     (4, 1024, 256, 2048, 2752, 1, 8, torch.bfloat16),   # a full tile, F cut at half a piece
     (5, 1120, 128, 512, 1056, 2, 5, torch.bfloat16),    # nine pieces of D, the last of 96: waves of one and of two
     (8, 640, 64, 64, 160, 1, 4, torch.float16),         # five pieces for eight waves, an E of half a piece
-    (7, 4096, 128, 256, 96, 2, 8, torch.bfloat16),      # the longest row that is normalised on the way
-    (2, 4128, 64, 128, 64, 1, 3, torch.bfloat16),       # one that is not
-    (9, 1024, 256, 512, 416, 2, 8, torch.float16),      # more tokens than two tiles
+    (7, 4096, 128, 256, 96, 2, 8, torch.bfloat16),      # the longest row that rows_kernel would take, of more tokens
+    (2, 4128, 64, 128, 64, 1, 3, torch.bfloat16),       # one that is longer
+    (9, 1024, 256, 512, 416, 2, 8, torch.float16),      # more tokens than two tiles of its width
     (1, 8192, 64, 64, 64, 1, 8, torch.bfloat16),
     (9, 32, 64, 64, 32, 1, 1, torch.bfloat16),          # four token tiles, the third of one token; one piece of 32 values
     (16, 384, 128, 1024, 1056, 2, 12, torch.float16),   # all full, the widest rows

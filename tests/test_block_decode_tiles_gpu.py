@@ -15,6 +15,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("B,D,S,E,F,heads,groups,dtype", [
     (5, 2048, 256, 512, 416, 1, 8, torch.bfloat16),     # the fewest tokens
     (8, 2048, 256, 8192, 4128, 4, 8, torch.float16),    # two waves a workgroup, else four; the last piece of F 32 values
+    (9, 32, 64, 64, 32, 1, 1, torch.bfloat16),          # (rows_kernel's, four token tiles)
     (17, 32, 64, 64, 32, 1, 1, torch.bfloat16),         # one piece of 32 values
     (9, 416, 64, 64, 32, 1, 13, torch.bfloat16),        # the first width of nine tokens
     (16, 1024, 256, 512, 2784, 2, 8, torch.float16),    # a full tile; F cut at 96
