@@ -462,7 +462,7 @@ __device__ __forceinline__ void outputs(float* re, float* im, int t, const Table
 
 // The rows of a channel that a workgroup takes: two at a time, which then share the transform of k (MODE 0) or the
 // inverse transform of dk, whose spectrum is summed over them (MODE 1).  The kernels' time is mostly the transforms'
-// arithmetic (72 to 75 % of the vector issue slots at M = 4096), so what counts is their number: 2.5 per row instead of 3.  In MODE 0
+// arithmetic (75 to 77 % of the vector issue slots at M = 4096), so what counts is their number: 2.5 per row instead of 3.  In MODE 0
 // k's spectrum then has to stay in registers to the row's end, which none of them leaves (one, of odd rows at M = 8192) since `settle`; at M = 16384 67
 // to 76 would, and the rows go one by one (PAIR 1), as a channel's only row does.  One kernel for dx and dk, with dy's spectrum formed once (4
 // transforms per row), spills 54 to 139 registers and takes 269 us where these two take 168.
