@@ -428,16 +428,19 @@ __global__ __launch_bounds__(64 * kWaves) void attn_probs_kernel(const ProbsPara
 // whole cache lines, RING of them ahead of the products, and are turned into operands through LDS of the wave's own.  Straight into the
 // operands, 32 bytes of 32 rows a request, a line was asked for four times and had left the cache in between: the layer's forward
 // with a value head of 64, us before / now: 1531 keys, four heads of 256 46.0 / 32.8; 4 x 1024, one head 32.7 / 24.1; 4000, two heads
-// 125 / 77; 2 x 2048, four heads of 128 50 / 39; 4 x 1024, four of 64 23.3 / 19.8; 300 keys 16.7 / 13.8.  (Without the piece behind the
-// last block, which is asked for again, +- 0.)
+// 125 / 77; 2 x 2048, four heads of 128 50 / 39; 4 x 1024, four of 64 23.3 / 19.8; 300 keys 16.7 / 13.8.  Up to
+// 1024 keys a wave asks for nothing behind its last block, nor without one (up to 128 keys 1.02, 1.04 and 1.09 of the speed at widths 64, 128, 256,
+// where such requests had made short rows slower than before); beyond, where that costs 2 %, for its last piece again.
 // Rows of more than 256 KB keys (SEGMENTS) pass in pieces of that many keys: running maxima and sums, then the
 // probabilities of the last piece, whose scores are still there, and of the others from products formed again.  (At
 // width 256 with one piece on its way: two spilled 18 registers, 300 x 4000 at two blocks a CU 329 us for 304.)
+// Up to 1024 keys at width 128 one piece is on its way too, which is what lets two workgroups share a CU (124 registers; with two 133,
+// and rows of up to 1024 keys at more than a block a CU took 1.05 to 1.2 times as long, up to 128 keys longer than with keys straight into the operands).
 // Every row block reads its keys from the L2 anew, which is what bounds full grids: those take the kernel above.
 template <int DT, int H1, int KB, bool SEGMENTS>
-__global__ __launch_bounds__(64 * kWaves) void attn_probs_short_kernel(const ProbsParams p) {
+__global__ __launch_bounds__(64 * kWaves, KB > 4 || H1 > 128 ? 2 : 4) void attn_probs_short_kernel(const ProbsParams p) {
   constexpr int QF = H1 / 16;
-  constexpr int PIECES = QF / 4, RING = KB > 4 && PIECES > 2 ? (SEGMENTS ? 1 : 2) : PIECES, kPitch = 64 + 8;
+  constexpr int PIECES = QF / 4, RING = KB > 4 ? (PIECES > 2 ? (SEGMENTS ? 1 : 2) : PIECES) : H1 == 128 ? 1 : PIECES, kPitch = 64 + 8;
   constexpr int STEP = KB * kWaves;  // 32-key blocks of a piece
   __shared__ float red[2][kWaves][32];
   __shared__ __align__(16) uint16_t stage[kWaves][32 * kPitch];
@@ -476,6 +479,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_probs_short_kernel(const Pro
   // 32 (b0 + wave + 8 i) + 8 (e / 4) + 4 h + e % 4
   floatx16 acc[KB];
   const auto scores = [&](int b0) {
+    if (KB > 4 || b0 + wave < nblk)
 #pragma unroll
     for (int n = 0; n < RING; ++n) load_piece(b0 + wave, n, kf + 4 * n);
 #pragma unroll
@@ -490,7 +494,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_probs_short_kernel(const Pro
 #pragma unroll
           for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4*>(put + 8 * j * kPitch) = here[j];
           if (n + RING < PIECES) load_piece(blk, n + RING, here);
-          else load_piece(blk + kWaves, n + RING - PIECES, here);  // (clamped into the keys)
+          else if (KB > 4 || blk + kWaves < nblk) load_piece(blk + kWaves, n + RING - PIECES, here);  // (beyond the keys: the last one)
           asm volatile("" ::: "memory");
           u32x4 f[4];
 #pragma unroll
@@ -657,7 +661,6 @@ constexpr int short_rows(int H1, int rows, int keys, bool causal) {
 
 template <int DT, int H1>
 int launch_probs(const ProbsParams& p, hipStream_t s) {
-  // few row blocks: see short_rows
   int dev = 0, cus = 0;
   MEGA_CHECK_HIP(hipGetDevice(&dev));
   MEGA_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
