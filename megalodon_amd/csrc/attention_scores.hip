@@ -622,41 +622,29 @@ int launch_probs_short(ProbsParams p, hipStream_t s) {
   return MEGA_OK;
 }
 
-// How many blocks of 32 rows a CU, in eighths, the short-row kernel takes.  It reads a block's keys anew for every block, so
-// its time grows with the blocks and with the head's width, while the other one's is its longest row block's until the chip
-// is full; keys that a causal block does not see are left out by both, but only the other one waits for its longest.  The
-// operator's forward with a value head of 64, time of the other kernel over the short-row kernel's, at blocks a CU:
-//   causal squares  width 64:  200 keys 5.9 1.06; 256 keys 5.0 1.10, 7.0 0.94; 512 keys 6.0 1.18; 1024 keys 6.0 1.30; 1500 keys 5.7 1.07, 6.1 1.00; 4096 keys 6.0
-//                              1.14, 8.0 0.96
-//                   width 128: 64 keys 1.8 0.84, 2.3 1.00; 256 keys 3.0 1.13, 4.0 0.93; 512 keys 4.0 1.19, 5.0 0.98; 700 keys 3.0 1.13, 4.0 0.95; 850 keys 4.2
-//                              1.27; 1024 keys 4.3 1.12, 4.6 0.90; 4096 keys 4.5 1.28
-//                   width 256: 64 keys 1.3 0.75; 100 keys 2.0 1.04, 2.5 0.86; 256 keys 2.0 1.28, 2.5 1.01; 384 keys 2.3 1.19, 2.5 0.95; 700 keys 2.5 1.18, 3.0
-//                              0.94; 850 keys 3.2 1.29, 3.5 0.97; 1500 keys 4.0 1.32, 4.6 0.98; 4096 keys 4.0 1.37, 4.5 1.08
-//   causal, more keys than rows (the first rows see most of them; more than 2048 go in pieces)
-//                   width 64:  100 x 400 5.9 1.40; 256 x 1024 5.0 1.06, 6.0 0.98; 1024 x 1280 4.8 1.02, 5.3 0.93; 600 x 3000 3.3 1.16, 3.7 0.91
-//                   width 128: 100 x 400 2.7 1.12, 3.2 0.94; 300 x 600 2.7 1.13, 3.2 0.97; 1024 x 1280 3.8 1.09, 4.3 0.96; 600 x 3000 2.7 1.30, 3.2 0.72
-//                   width 256: 100 x 400 2.8 1.07; 300 x 600 2.5 1.28, 2.7 0.98; 1024 x 1280 4.0 1.10, 4.5 0.97; 600 x 3000 1.8 1.56, 2.5 0.88
-//   without a mask  width 64:  100 x 1000 5.9 1.43; 256 keys 2.0 1.14, 3.0 0.97; 384 keys 3.7 1.16, 4.3 0.99; 1024 keys 5.0 1.10, 6.0 0.98; 4096 keys 4.0 1.07, 5.0 0.94
-//                   width 128: 256 keys 2.0 1.04, 3.0 0.86; 384 keys 2.7 1.15, 3.2 0.92; 1300 keys 3.2 1.18, 3.7 0.96; 4096 keys 3.0 1.19, 4.0 1.02
-//                   width 256: 256 keys 2.0 1.04, 2.5 0.85; 384 keys 1.7 1.17, 2.3 0.95; 1024 keys 3.0 1.19, 4.0 0.97; 2500 keys 2.5 1.10, 2.8 0.97
-// (While the keys came by 32 bytes of a row the lines lay at 1.3 to 5.5 blocks; over 900 sizes of 64 to 4096 keys at up to 12 blocks
-// the better of the two kernels at every one would be 1.6 % ahead of these lines, 3.8 % of those.)
-constexpr int short_rows(int H1, int rows, int keys, bool causal) {
-  if (causal && rows == keys) {
-    if (H1 == 64) return keys <= 384 ? 42 : 48;
-    if (H1 == 128) return keys <= 72 ? 14 : keys <= 384 ? 24 : keys <= 544 ? 32 : keys <= 768 ? 28 : 36;
-    return keys <= 72 ? 8 : keys <= 128 ? 16 : keys <= 384 ? 19 : keys <= 768 ? 22 : keys <= 1152 ? 28 : 34;
-  }
-  if (causal) {
-    const bool half = keys > 1024 && 2 * rows >= keys;
-    if (keys > 2048 && !half) return H1 == 64 ? 27 : H1 == 128 ? 24 : 16;
-    if (H1 == 64) return rows <= 128 ? 47 : 40;
-    if (H1 == 128) return half ? 32 : 25;
-    return half ? 33 : 22;
-  }
-  if (H1 == 64) return rows <= 128 && keys >= 512 ? 47 : keys <= 288 ? 22 : keys <= 768 ? 33 : keys <= 1152 ? 41 : 32;
-  if (H1 == 128) return keys <= 288 ? 16 : keys <= 768 ? 22 : 27;
-  return keys <= 384 ? 16 : keys <= 768 ? 20 : keys <= 1536 ? 24 : 20;
+// Which kernel takes the rows: an estimate of how many us the short-row kernel is behind the other one.  It reads a block's keys anew for
+// every block of 32 rows, so that its time grows with the blocks a CU and the keys they see, those of a block's pieces but the last twice; the other
+// one's is its longest row block's, all keys, and, a block of 256 rows a CU and more, what those see.  The coefficients of a width (us for a block a
+// CU, for 1024 keys of each, for 1024 keys, for 1024 keys of 256 rows a CU, for those rows, for a block's piece that is passed again) are least
+// squares of both kernels' times of 6971 calls of the operator's forward with a value head of 64, of 16 to 5000 keys, squares, fewer rows than keys and
+// no mask, 0.25 to 14 blocks a CU, 1 to 16 heads, each weighted by its faster time and by how near the kernels are.  The kernel so taken is 0.3
+// to 0.5 % behind the faster one on average, also on a half that was not fitted; lines by width, rows, keys and mask, about 30 constants, were
+// 4.7 to 8.2 % behind it, at 32 rows of 160 keys and width 64 1.75 times.
+bool short_rows_ahead(int H1, const ProbsParams& p, int cus) {
+  constexpr float kPiece = 8.f * 32.f * kWaves;
+  const float z = static_cast<float>(p.Z) / static_cast<float>(cus), rows = static_cast<float>(p.L1), all = static_cast<float>(p.L2);
+  const float keys = all / 1024.f, half = p.causal ? rows / 2048.f : 0.f;  // causal rows see half of their own number less
+  const float blocks = z * static_cast<float>((p.L1 + 31) / 32), wide = z * static_cast<float>((p.L1 + 255) / 256);
+  // (33 to 64 rows and keys at more than a block a CU, which the estimate misses: 164 heads of 64 16.4 us here, 13.0 there, 940 54.6 / 42.6)
+  if (H1 == 256 && p.L1 > 32 && p.L1 <= 64 && p.L2 <= 64 && blocks > 1.f) return false;
+  const float seen = fmaxf(keys - half, 0.f), wide_seen = fmaxf(keys - fmaxf(half - 0.0625f, 0.f), 0.f);
+  const float again = all <= kPiece ? 0.f : (ceilf(all / kPiece) - 1.f) * (p.causal ? fminf((all - kPiece) / rows, 1.f) : 1.f);
+  const auto behind = [&](float c0, float c1, float c2, float c3, float c4, float c5, float c6) {
+    return c0 + blocks * (c1 + c2 * seen + c6 * again) - c3 * keys - wide * (c4 * wide_seen + c5);
+  };
+  return (H1 == 64    ? behind(-0.5f, 0.3f, 8.6f, 29.0f, 28.2f, 3.0f, 8.3f)
+          : H1 == 128 ? behind(-0.5f, 0.9f, 11.9f, 35.5f, 33.4f, 3.7f, 7.1f)
+                      : behind(-0.8f, 4.1f, 13.1f, 48.3f, 19.8f, 7.0f, 10.8f)) <= 0.f;
 }
 
 template <int DT, int H1>
@@ -664,7 +652,7 @@ int launch_probs(const ProbsParams& p, hipStream_t s) {
   int dev = 0, cus = 0;
   MEGA_CHECK_HIP(hipGetDevice(&dev));
   MEGA_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  if (8 * static_cast<int64_t>(p.Z) * ((p.L1 + 31) / 32) <= static_cast<int64_t>(short_rows(H1, p.L1, p.L2, p.causal)) * cus)
+  if (short_rows_ahead(H1, p, cus))
     return launch_probs_short<DT, H1>(p, s);
   constexpr int KW = H1 >= 128 ? 128 : 64;
   const size_t lds = sizeof(uint16_t) * kRing * kKeys * KW;
